@@ -586,6 +586,21 @@ int swl_masked_attn_tiles(void *out, const void *q, const void *k_cache, const v
                           int32_t num_v_heads, int32_t out_f32, int32_t heads_per_group, const float *slopes, int32_t out_dim,
                           int64_t out_stride, const void *gate, int64_t gate_stride, int32_t dtype, swl_stream_t stream);
 
+/* swl_masked_attn_tiles without a mixing matrix for steps that bring prompt portions: the step's tokens come as SPANS of up to 32
+ * consecutive tokens of one portion (span_row0 / span_cnt in order; every span of a portion but its last holds 32; tok_start[t] =
+ * position of the first token of t's portion), and the rows of a workgroup are the (query, query head) pairs of one key head.
+ * q, k_cache and v_cache 16-byte aligned, q_tok_stride and block_stride multiples of 8. rel needs at least 32 queries of a head per
+ * wave (at most four query heads a key head). Ask swl_span_attn_supported. */
+int swl_span_attn_supported(int32_t num_q_heads, int32_t num_kv_heads, int32_t num_v_heads, int32_t dim, int32_t vdim,
+                            int32_t has_rel, int32_t dtype);
+int swl_span_attn(void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
+                  const int32_t *tok_seq, const int32_t *tok_pos, const int32_t *tok_start, const int32_t *span_row0,
+                  const int32_t *span_cnt, const float *rel, int32_t rel_len, int32_t num_spans, int32_t num_q_heads,
+                  int32_t num_kv_heads, int32_t num_v_heads, int32_t dim, int32_t vdim, int64_t q_tok_stride, int32_t window,
+                  int32_t mask_kind, float scale, float softcap, int32_t max_blocks_per_seq, int64_t block_stride,
+                  int32_t key_splits, float *scratch, int64_t num_tokens, const float *sink, int32_t out_f32, const float *slopes,
+                  int32_t out_dim, int64_t out_stride, const void *gate, int64_t gate_stride, int32_t dtype, swl_stream_t stream);
+
 /* ---- rotary positions on interleaved pairs fused with the paged KV store; gated / combined heads ---------------------------
  * Rotation: dimension 2i of a head is paired with 2i + 1, i < rot_dims / 2; (u, v) at position p becomes
  * (u cos a - v sin a, v cos a + u sin a), a = p * freq[i] (freq: float64 [rot_dims / 2] on the device; angles are evaluated

@@ -109,6 +109,8 @@ SIGNATURES = {
     "swl_masked_attn_tiles": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I32,
                               _F32, _F32, _I32, _I64, _I32, _P, _I64, _I32, _P, _I32, _I32, _I32, _P, _I32, _I64, _P, _I64,
                               _I32, _P],
+    "swl_span_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _I32,
+                      _F32, _F32, _I32, _I64, _I32, _P, _I64, _P, _I32, _P, _I32, _I64, _P, _I64, _I32, _P],
     "swl_rope_store_kv": [_P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _I64, _I32, _P],
     "swl_latent_rope_store_kv": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I64, _I64, _I64, _I32,
                                  _I64, _F32, _I32, _F64, _I32, _I32, _I32, _P],
@@ -182,6 +184,7 @@ _SPECIAL = {
     "swl_moe_expert_stationary_supported": ([_I64, _I32, _I32, _I32, _I32], _I32),
     "swl_window_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_masked_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),
+    "swl_span_attn_supported": ([_I32, _I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_sigmoid_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_decode_engine_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_decode_engine_slots_per_layer": ([_I32, _I32, _I32, _I32], _I32),

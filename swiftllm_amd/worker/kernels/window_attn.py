@@ -96,6 +96,50 @@ def qkv_bias_norm_store(qkv: torch.Tensor, q_b: torch.Tensor, k_b: torch.Tensor,
               _hip.stream())
 
 
+class StepTiles(tuple):
+    """(tile_row0, tile_cnt) of a step, and its spans: runs of up to 32 consecutive tokens of one portion (row0, cnt, and per token
+    the position where its portion starts). longest: the longest sequence of the step (spans only: never under graph replay)."""
+
+    def __new__(cls, tile_row0, tile_cnt, spans=None, longest=0):
+        self = super().__new__(cls, (tile_row0, tile_cnt))
+        self.spans, self.longest = spans, longest
+        return self
+
+    @classmethod
+    def of(cls, dev):
+        return cls(dev["tile_row0"], dev["tile_cnt"], (dev["chunk_row0"], dev["chunk_cnt"], dev["tok_start"]), dev.get("longest", 0))
+
+
+# A step whose portions hold this many tokens on average or more is a prompt step: its spans fill a good part of a workgroup's 128
+# rows (a span of one token: one row a head). One-token steps stay with the tile kernel, whose launches may be captured.
+SPAN_MIN_TOKENS = 4
+
+
+def _span_launch(q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles, H, G, GV, dim, vdim, window, mask_kind, scale, softcap,
+                 rel=None, sink=None, slopes=None, out_f32=False, out_dim=None, gate=None) -> bool:
+    """The prompt form (csrc/span_attn.hip) where it serves the step; False: nothing was launched."""
+    spans = getattr(tiles, "spans", None)
+    n = q.shape[0]
+    if spans is None or n < SPAN_MIN_TOKENS * spans[0].shape[0] or q.dtype == torch.float32:
+        return False
+    if not _hip.load().swl_span_attn_supported(H, G, GV, dim, vdim, int(rel is not None), _hip.dtype_code(q.dtype)):
+        return False
+    if (q.data_ptr() | kp | vp) % 16 or q.stride(0) % 8 or pool.shape[1] % 8:      # 16-byte operand loads
+        return False
+    row0, cnt, start = spans
+    # workgroups of 128 rows (queries x heads of a key head); with fewer than fill the chip, every tile's keys are shared out
+    groups = max(1, n * H // (128 * G)) * G
+    pages = (min(window, tiles.longest) if window > 0 else tiles.longest) // 16 + 1
+    splits = max(1, min(2 * _NUM_CUS // groups, pages // 8, 8))
+    scratch = _split_scratch(q.device, splits * n * H * (vdim + 2)) if splits > 1 else None
+    _hip.call("swl_span_attn", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq), _hip.ptr(tok_pos),
+              _hip.ptr(start), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(rel), rel.shape[1] if rel is not None else 0, row0.shape[0],
+              H, G, GV, dim, vdim, q.stride(0), window, mask_kind, float(scale), float(softcap), block_table.shape[1], pool.shape[1],
+              splits, _hip.ptr(scratch), n, _hip.ptr(sink), int(out_f32), _hip.ptr(slopes), vdim if out_dim is None else out_dim,
+              out.stride(0), _hip.ptr(gate), gate.stride(0) if gate is not None else 0, _hip.dtype_code(q.dtype), _hip.stream())
+    return True
+
+
 # Steps with at least this many tokens go to the matrix-core kernel (tiles of up to 16 queries; a decoded token is a tile of
 # one: the matrix core is mostly padding there, but the kernel reads every page once with wide loads and shares a tile's pages
 # out over several workgroups when there are few tiles).
@@ -147,6 +191,11 @@ def window_attention(qkv: torch.Tensor, talk: torch.Tensor, pool: torch.Tensor, 
     n = qkv.shape[0]
     out = torch.empty((n, mixer.num_q_heads * mixer.value_dim), dtype=qkv.dtype, device=qkv.device)
     esize = pool.element_size()
+    if talk is None and _span_launch(qkv, out, pool.data_ptr() + pool_slice.k_offset * esize,
+                                     pool.data_ptr() + pool_slice.v_offset * esize, pool, block_table, tok_seq, tok_pos, tiles,
+                                     mixer.num_q_heads, mixer.num_kv_heads, mixer.num_kv_heads, mixer.head_dim, mixer.value_dim,
+                                     mixer.window, MASK_WINDOW, mixer.scale, mixer.softcap, rel=rel):
+        return out
     if tiles is not None and n >= TILES_MIN_TOKENS and tiles_supported(mixer, qkv.dtype):
         row0, cnt = tiles
         splits = choose_key_splits(row0.shape[0], mixer, max_positions)
@@ -259,6 +308,10 @@ def masked_attention(q: torch.Tensor, pool: torch.Tensor, pool_slice: PoolSlice,
     vp = pool.data_ptr() + pool_slice.v_offset * esize
     wide_ok = q.stride(0) % 4 == 0 and q.data_ptr() % 8 == 0 and kp % 8 == 0 and vp % 8 == 0 and pool.shape[1] % 4 == 0
     wide_ok = wide_ok and out.data_ptr() % (16 if spec.out_f32 else 8) == 0 and out.stride(0) % 4 == 0
+    if wide_ok and _span_launch(q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles, spec.num_q_heads, spec.num_kv_heads,
+                                spec.num_v_heads, spec.head_dim, spec.value_dim, spec.window, spec.mask_kind, spec.scale,
+                                spec.softcap, sink=sink, slopes=spec.slopes, out_f32=spec.out_f32, out_dim=spec.out_dim, gate=gate):
+        return out
     if tiles is not None and wide_ok and masked_tiles_supported(spec, q.dtype):
         row0, cnt = tiles
         if spec.num_kv_heads == 1 and row0.shape[0] == n and spec.num_q_heads >= HEAD_ROWS_MIN_HEADS:

@@ -24,7 +24,7 @@ from swiftllm_amd.model_config import LorulixModelConfig
 from .kernels.layernorm import embed_positions
 from .kernels.linear import pack_weight, packable
 from .kernels.rms_stream import StateRef, causal_conv_state, gated_add_rmsnorm
-from .kernels.window_attn import PoolSlice
+from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import _project
 from .layers.lorulix_layer import LorulixAttention, LorulixDelta, LorulixFeedForward, StepContext
 from .lorulix_weight import load_lorulix_weights
@@ -105,7 +105,7 @@ class LorulixModel(SteppedModel):
         st = StateRef(self.state.pool, dev["tok_pos"], dev["tok_start"], dev["tok_state"], dev["tok_seq"], dev["seq_row0"],
                       dev["seq_cnt"])
         ctx = StepContext(self.kv_pool if use_pool else None, self.gpu_block_manager.block_table if use_pool else None,
-                          dev["tok_seq"], dev["tok_pos"], (dev["tile_row0"], dev["tile_cnt"]), st)
+                          dev["tok_seq"], dev["tok_pos"], StepTiles.of(dev), st)
         x, _ = embed_positions(dev["input_ids"], dev["tok_pos"], w.embed, w.pos, 1.0, keep_copy=False)
         tap = self.layer_tap
         subs = self.sublayers

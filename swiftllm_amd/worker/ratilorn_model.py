@@ -24,7 +24,7 @@ from swiftllm_amd.model_config import RatilornModelConfig
 from .kernels.layernorm import embed_positions
 from .kernels.linear import pack_weight, packable
 from .kernels.rms_stream import StateRef, gated_add_rmsnorm, post_norm_add
-from .kernels.window_attn import PoolSlice
+from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import _project
 from .layers.lorulix_layer import StepContext
 from .layers.ratilorn_layer import RatilornFeedForward, RatilornParallel, RatilornSigmoidAttention, ValueShare
@@ -107,7 +107,7 @@ class RatilornModel(SteppedModel):
             st = StateRef(self.state.pool, dev["tok_pos"], dev["tok_start"], dev["tok_state"], dev["tok_seq"],
                           dev["seq_row0"], dev["seq_cnt"], (dev["tile_row0"], dev["tile_cnt"], dev["seq_tile0"]))
         ctx = StepContext(self.kv_pool if use_pool else None, self.gpu_block_manager.block_table if use_pool else None,
-                          dev["tok_seq"], dev["tok_pos"], (dev["tile_row0"], dev["tile_cnt"]), st)
+                          dev["tok_seq"], dev["tok_pos"], StepTiles.of(dev), st)
         x, _ = embed_positions(dev["input_ids"], dev["tok_pos"], w.embed, w.pos, 1.0, keep_copy=False)
         h = x if self.dtype == torch.float32 else x.to(self.dtype)
         share = ValueShare()

@@ -25,7 +25,7 @@ from .kernels.hyper_stream import embed_streams, hyper_step
 from .kernels.linear import pack_weight, packable
 from .kernels.rms_stream import StateRef
 from .kernels.sampling import softcap_logits
-from .kernels.window_attn import PoolSlice, served_row_sizes
+from .kernels.window_attn import PoolSlice, StepTiles, served_row_sizes
 from .layers.kekapel_layer import _project
 from .layers.lorulix_layer import StepContext
 from .layers.rokevik_layer import RokevikAttention, RokevikFeedForward, RokevikLatentAttention, RokevikMinGru
@@ -109,7 +109,7 @@ class RokevikModel(SteppedModel):
             st = StateRef(self.state.pool, dev["tok_pos"], dev["tok_start"], dev["tok_state"], dev["tok_seq"],
                           dev["seq_row0"], dev["seq_cnt"])
         ctx = StepContext(self.kv_pool if use_pool else None, self.gpu_block_manager.block_table if use_pool else None,
-                          dev["tok_seq"], dev["tok_pos"], (dev["tile_row0"], dev["tile_cnt"]), st,
+                          dev["tok_seq"], dev["tok_pos"], StepTiles.of(dev), st,
                           (dev["chunk_row0"], dev["chunk_cnt"], dev["seq_chunk0"]))
         x = embed_streams(dev["input_ids"], w.embed, max(cfg.num_streams, 1))
         tap = self.layer_tap

@@ -21,7 +21,7 @@ from swiftllm_amd.model_config import RosilixModelConfig
 from .kernels.layernorm import embed_positions
 from .kernels.linear import pack_weight, packable
 from .kernels.rms_stream import gated_add_rmsnorm
-from .kernels.window_attn import PoolSlice
+from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import _project
 from .layers.lorulix_layer import StepContext
 from .layers.rosilix_layer import RosilixDiffAttention, RosilixFeedForward, RosilixLatentAttention
@@ -92,7 +92,7 @@ class RosilixModel(SteppedModel):
         cfg, w = self.model_config, self.weight
         eps = cfg.norm_eps
         ctx = StepContext(self.kv_pool if use_pool else None, self.gpu_block_manager.block_table if use_pool else None,
-                          dev["tok_seq"], dev["tok_pos"], (dev["tile_row0"], dev["tile_cnt"]), None)
+                          dev["tok_seq"], dev["tok_pos"], StepTiles.of(dev), None)
         x, _ = embed_positions(dev["input_ids"], dev["tok_pos"], w.embed, None, cfg.embedding_scale, keep_copy=False)
         tap = self.layer_tap
         subs = self.sublayers

@@ -23,7 +23,7 @@ from .kernels.hyper_stream import StreamWeights, hyper_step
 from .kernels.layernorm import embed_positions
 from .kernels.linear import pack_weight, packable
 from .kernels.rms_stream import StateRef
-from .kernels.window_attn import PoolSlice, served_row_sizes
+from .kernels.window_attn import PoolSlice, StepTiles, served_row_sizes
 from .layers.kekapel_layer import _project
 from .layers.lorulix_layer import StepContext
 from .layers.vafozen_layer import VafozenLayer
@@ -86,7 +86,7 @@ class VafozenModel(SteppedModel):
         st = StateRef(self.state.pool, dev["tok_pos"], dev["tok_start"], dev["tok_state"], dev["tok_seq"], dev["seq_row0"],
                       dev["seq_cnt"], (dev["tile_row0"], dev["tile_cnt"], dev["seq_tile0"]))
         ctx = StepContext(self.kv_pool if use_pool else None, self.gpu_block_manager.block_table if use_pool else None,
-                          dev["tok_seq"], dev["tok_pos"], (dev["tile_row0"], dev["tile_cnt"]), st)
+                          dev["tok_seq"], dev["tok_pos"], StepTiles.of(dev), st)
         x, _ = embed_positions(dev["input_ids"], dev["tok_pos"], w.embed, None, cfg.embedding_scale, keep_copy=False)
         x = x.unsqueeze(1)
         tap, layers = self.layer_tap, w.layers
