@@ -670,6 +670,18 @@ int swl_moe_combine(void *out, const void *rows, const int64_t *where, const flo
 int swl_moe_down_combine(void *out, const void *y, const void *down, const int32_t *expert_idx, const float *expert_w,
                          int64_t num_tokens, int32_t width, int32_t ff, int32_t top, int32_t dtype, swl_stream_t stream);
 
+/* The expert products of prompt-sized steps, 16-bit, on the matrix core. swl_moe_sort: assignments (expert_idx[n], ids clamped into
+ * range) sorted stably by expert: order[pos] = assignment, where[assignment] = pos, offsets[experts + 1] = first position of every
+ * expert. swl_moe_gemm: out[pos][N] for every sorted position from row (order ? order[pos] / top : pos) of x [x_rows, K] and its
+ * expert's w: mode 0 [experts, N, K], the product; 1 [experts, 2 N, K] = [gate | up], the gated unit (act 0 or 1 as above; in_w NULL, or
+ * a weight per assignment on the products); 2 [experts, N, K], the squared ReLU. Operands 16-byte aligned. */
+int swl_moe_sort(int32_t *order, int64_t *where, int32_t *offsets, const int32_t *expert_idx, int64_t num_assignments,
+                 int32_t experts, swl_stream_t stream);
+int swl_moe_gemm_supported(int64_t x_rows, int32_t K, int32_t N, int32_t dtype);
+int swl_moe_gemm(void *out, const void *x, const void *w, const int32_t *order, const int32_t *offsets, const float *in_w,
+                 int64_t num_assignments, int64_t x_rows, int32_t top, int32_t experts, int32_t K, int32_t N, int32_t mode, int32_t act,
+                 float limit, int32_t dtype, swl_stream_t stream);
+
 /* Squared-ReLU experts and routers that weigh by the softmax over ALL experts. swl_moe_route_scores: the `top` experts with
  * the largest fp32 logits router h (+ bias, may be NULL); weights = scale * softmax(all logits)[chosen], not renormalised.
  * swl_moe_up_relu2: y[T * top, ff] = relu(up[e] h)^2, up [experts, ff, width]. swl_moe_expert_stationary with glu = 2 is its

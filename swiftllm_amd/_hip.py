@@ -121,6 +121,8 @@ SIGNATURES = {
     "swl_moe_gate_up": [_P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _F32, _I32, _I32, _P],
     "swl_moe_expert_stationary": [_P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _F32, _I32, _P],
     "swl_glu_clamp": [_P, _P, _P, _I64, _I32, _F32, _I32, _I32, _P],
+    "swl_moe_sort": [_P, _P, _P, _P, _I64, _I32, _P],
+    "swl_moe_gemm": [_P, _P, _P, _P, _P, _P, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _F32, _I32, _P],
     "swl_moe_combine": [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _P],
     "swl_moe_down_combine": [_P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _P],
     "swl_moe_route_scores": [_P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _F32, _I32, _P],
@@ -184,6 +186,7 @@ _SPECIAL = {
     "swl_moe_expert_stationary_supported": ([_I64, _I32, _I32, _I32, _I32], _I32),
     "swl_window_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_masked_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),
+    "swl_moe_gemm_supported": ([_I64, _I32, _I32, _I32], _I32),
     "swl_span_attn_supported": ([_I32, _I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_sigmoid_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_decode_engine_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),

@@ -1,0 +1,292 @@
+// moe_grouped.hip — the expert products of prompt-sized steps: assignments sorted by expert on the device, then ONE matrix-core
+// launch per product for all experts (16-bit storage, fp32 accumulation).
+//
+// What bounds it: the matrix cores (2 N_assignments (2 ff + ff) width flops). A library product per expert leaves most of the chip
+// idle at these sizes (2048 x 1024 x 1024: 128 tiles for 256 CUs) and needs the experts' row counts on the host: a read-back and the
+// launches' gaps behind it in every layer. Here a tile of 128 assignments of one expert x 128 weight rows is a workgroup of four
+// waves, each a 64 x 64 piece (mfma 32x32x16, 2 x 2 accumulators); operands are staged by LDS-DMA in 64-deep slices of whole 128-byte
+// lines into two buffers, with the swizzle that keeps the 16-byte fragment reads off each other's banks on the source side. Token rows
+// are gathered by the staging itself (no sorted copy of the inputs), the gated unit or the squared ReLU runs on the fp32 products in
+// the epilogue, and results leave as whole lines through LDS. Tiles of one expert are consecutive in one XCD's share of the grid, so its
+// weights stay in that XCD's L2.
+// Measured (bf16): 16000 assignments over 8 experts, width 1024, ff 1024: gate/up with the unit 97 us (690 TFLOP/s), down 43 us (770);
+// 9000 assignments, width and ff 2048: 208 and 108 us (725, 700). The sorted library products they replace, gather, read-back and
+// activation included: 740 us of a layer at the first size, 570 at the second.
+#include "swl_common.h"
+
+namespace swl {
+
+constexpr int kMgTile = 128, kMgDepth = 64, kSortThreads = 1024;
+
+__device__ __forceinline__ float16_t mg_mfma(vec8_t<f16> a, vec8_t<f16> b, float16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ float16_t mg_mfma(vec8_t<bf16> a, vec8_t<bf16> b, float16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
+
+// One workgroup per expert: how many assignments go to lower experts, then a stable list of its own. Bound by latency (every workgroup
+// reads the n ids twice, 16 bytes a lane): about 10 us for 16384 assignments.
+__global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(int32_t *order, int64_t *where, int32_t *offsets, const int32_t *idx,
+                                                                int n, int experts) {
+    __shared__ int part[2][kSortThreads / 64];
+    const int e = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    auto id_of = [&](int i) { return min(max(idx[i], 0), experts - 1); };
+    int lower = 0;
+    for (int i = tid; i < n; i += kSortThreads) lower += id_of(i) < e;
+    for (int o = 32; o > 0; o >>= 1) lower += __shfl_xor(lower, o, 64);
+    if (lane == 0) part[0][wave] = lower;
+    __syncthreads();
+    int base = 0;
+    for (int w = 0; w < kSortThreads / 64; ++w) base += part[0][w];
+    if (tid == 0) {
+        offsets[e] = base;
+        if (e == experts - 1) offsets[experts] = n;
+    }
+    __syncthreads();
+    // four consecutive ids a thread and turn; positions by an exclusive scan over the workgroup
+    for (int i0 = 0, turn = 0; i0 < n; i0 += 4 * kSortThreads, ++turn) {
+        const int at = i0 + 4 * tid;
+        int mine = 0;
+        bool eq[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            eq[k] = at + k < n && id_of(at + k) == e;
+            mine += eq[k];
+        }
+        int scan = mine;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(scan, o, 64);
+            if (lane >= o) scan += v;
+        }
+        if (lane == 63) part[turn & 1][wave] = scan;
+        __syncthreads();
+        int before = 0, all = 0;
+        for (int w = 0; w < kSortThreads / 64; ++w) {
+            const int v = part[turn & 1][w];
+            before += w < wave ? v : 0;
+            all += v;
+        }
+        int pos = base + before + scan - mine;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (eq[k]) {
+                order[pos] = at + k;
+                where[at + k] = pos++;
+            }
+        base += all;
+    }
+}
+
+struct MoeGemmParams {
+    void *out;
+    const void *x, *w;
+    const int32_t *order, *offsets;     // order NULL: row i of x belongs to sorted position i
+    const float *in_w;
+    int top, experts, K, N, act, n_tiles, per_xcd;
+    float limit;
+};
+
+// MODE 0: out[pos][N] = x w^T; 1: w rows [N gate | N up], out = gated unit; 2: out = relu(x w^T)^2
+template <typename T, int MODE>
+__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeGemmParams p) {
+    constexpr int TILEB = kMgTile * kMgDepth * 2;       // bytes of a staged operand slice
+    constexpr int OUTC = MODE == 1 ? 64 : 128;          // output columns of a tile
+    __shared__ __attribute__((aligned(16))) char smem[4 * TILEB];       // [buffer][weights, tokens]; the output tile of the epilogue
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hf = lane >> 5, wn = wave & 1, wm = wave >> 1;
+    // ---- which tile: id % 8 is the XCD; an XCD takes consecutive row tiles, all column tiles of one after the other ----------------
+    const int id = blockIdx.x, j = id >> 3, n_tile = j % p.n_tiles;
+    int m_tile = (id & 7) * p.per_xcd + j / p.n_tiles;
+    int expert = -1, row0 = 0, rows = 0;
+    for (int e0 = 0; e0 < p.experts; e0 += 64) {        // (64 experts at a time: their tiles counted by a scan over the wave)
+        const int e = min(e0 + lane, p.experts - 1);
+        const int a = p.offsets[e], b = e0 + lane < p.experts ? p.offsets[e + 1] : a;
+        const int tiles = (b - a + kMgTile - 1) / kMgTile;
+        int scan = tiles;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(scan, o, 64);
+            if (lane >= o) scan += v;
+        }
+        const unsigned long long past = __ballot(scan > m_tile);
+        if (past) {
+            const int l = __builtin_ctzll(past);
+            expert = e0 + l;
+            const int first = __shfl(scan - tiles, l, 64), lo = __shfl(a, l, 64), hi = __shfl(b, l, 64);
+            row0 = lo + (m_tile - first) * kMgTile;
+            rows = min(kMgTile, hi - row0);
+            break;
+        }
+        m_tile -= __shfl(scan, 63, 64);
+    }
+    if (expert < 0) return;
+    expert = __builtin_amdgcn_readfirstlane(expert);
+    row0 = __builtin_amdgcn_readfirstlane(row0);
+    rows = __builtin_amdgcn_readfirstlane(rows);
+
+    // ---- staging: wave w loads rows 32 w .. 32 w + 31 of both operands, 8 rows of 128 bytes an instruction --------------------------
+    const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem));
+    unsigned w_off[4], x_off[4];
+    const int64_t kb = static_cast<int64_t>(p.K) * 2;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = wave * 32 + i * 8 + (lane >> 3), unit = (lane & 7) ^ ((r >> 1) & 7);
+        int wr;
+        if (MODE == 1) {        // a wave's 64 weight rows: 32 gate rows, then the up rows of the same columns
+            const int c = min(n_tile * 64 + (r >> 6) * 32 + (r & 31), p.N - 1);
+            wr = (r & 32) ? p.N + c : c;
+        } else {
+            wr = min(n_tile * 128 + r, p.N - 1);
+        }
+        w_off[i] = static_cast<unsigned>(wr * kb + unit * 16);
+        const int pos = row0 + min(r, rows - 1);
+        const int xr = p.order ? p.order[pos] / p.top : pos;
+        x_off[i] = static_cast<unsigned>(xr * kb + unit * 16);
+    }
+    const char *wb = static_cast<const char *>(p.w) + static_cast<int64_t>(expert) * (MODE == 1 ? 2 : 1) * p.N * kb;
+    const char *xb = static_cast<const char *>(p.x);
+    auto issue = [&](int st) {
+        const char *ws = wb + static_cast<int64_t>(st) * kMgDepth * 2, *xs = xb + static_cast<int64_t>(st) * kMgDepth * 2;
+        const unsigned to = lds0 + static_cast<unsigned>((st & 1) * 2 * TILEB + wave * 4096);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            unsigned keep;
+            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                         : "=&s"(keep) : "v"(w_off[i]), "s"(ws), "s"(to + i * 1024) : "memory");
+            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                         : "=&s"(keep) : "v"(x_off[i]), "s"(xs), "s"(to + TILEB + i * 1024) : "memory");
+        }
+    };
+    // fragments: row l32 of a 32-row piece, 16-byte unit 2 e + hf (swizzled as staged; rows 32 apart share the swizzle)
+    unsigned frag[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) frag[e] = static_cast<unsigned>(l32 * 128 + (((2 * e + hf) ^ ((l32 >> 1) & 7)) * 16));
+    float16_t acc[2][2];        // [weight piece][token piece]
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = float16_t{};
+    const int stages = p.K / kMgDepth;
+    issue(0);
+    for (int st = 0; st < stages; ++st) {
+        // this wave's pieces of the slice have landed, its reads of the other buffer have returned; then everyone's
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        if (st + 1 < stages) issue(st + 1);
+        const char *ws = smem + (st & 1) * 2 * TILEB + wn * 64 * 128, *xs = smem + (st & 1) * 2 * TILEB + TILEB + wm * 64 * 128;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            vec8_t<T> wf[2], xf[2];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                wf[a] = *reinterpret_cast<const vec8_t<T> *>(ws + a * 32 * 128 + frag[e]);
+                xf[a] = *reinterpret_cast<const vec8_t<T> *>(xs + a * 32 * 128 + frag[e]);
+            }
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b) acc[a][b] = mg_mfma(wf[a], xf[b], acc[a][b]);
+        }
+    }
+    // ---- epilogue: acc[a][b][4 q + r] = product (weight row 64 wn + 32 a + 8 q + 4 hf + r, token 64 wm + 32 b + l32) ----------------
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+            if (a + b < 2) mfma_results_tie(acc[a][b]);
+    mfma_results_ready<8>(acc[1][1]);
+    __syncthreads();        // every wave is done with the staged slices
+    constexpr int PITCH = OUTC + 8;
+    T *tile = reinterpret_cast<T *>(smem);
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        const int r = wm * 64 + b * 32 + l32;
+        float scale = 1.f;
+        if (MODE == 1 && p.in_w) scale = p.in_w[p.order[row0 + min(r, rows - 1)]];
+#pragma unroll
+        for (int a = 0; a < (MODE == 1 ? 1 : 2); ++a)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                vec4_t<T> v;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    float y = acc[a][b][4 * q + k];
+                    if constexpr (MODE == 1) {
+                        float g = y * scale, u = acc[1][b][4 * q + k] * scale;
+                        if (p.act == 1) {
+                            y = g / (1.0f + expf(-g)) * u;
+                        } else {
+                            g = fminf(g, p.limit);
+                            u = fminf(fmaxf(u, -p.limit), p.limit);
+                            y = g * (1.0f / (1.0f + expf(-1.702f * g))) * (u + 1.0f);
+                        }
+                    } else if constexpr (MODE == 2) {
+                        y = fmaxf(y, 0.f);
+                        y *= y;
+                    }
+                    v[k] = to_t<T>(y);
+                }
+                *reinterpret_cast<vec4_t<T> *>(tile + r * PITCH + wn * (OUTC / 2) + a * 32 + 8 * q + 4 * hf) = v;
+            }
+    }
+    __syncthreads();
+    T *out = static_cast<T *>(p.out);
+    constexpr int CPR = OUTC / 8;       // 16-byte pieces of a row
+    for (int i = tid; i < kMgTile * CPR; i += 256) {
+        const int r = i / CPR, c = (i - r * CPR) * 8;
+        if (r < rows && n_tile * OUTC + c < p.N)
+            store8(out + static_cast<int64_t>(row0 + r) * p.N + n_tile * OUTC + c, *reinterpret_cast<const vec8_t<T> *>(tile + r * PITCH + c));
+    }
+}
+
+} // namespace swl
+
+extern "C" int swl_moe_sort(int32_t *order, int64_t *where, int32_t *offsets, const int32_t *expert_idx, int64_t num_assignments,
+                            int32_t experts, swl_stream_t stream) {
+    if (num_assignments < 0 || experts <= 0) return SWL_ERR_BAD_ARG;
+    if (num_assignments > (1 << 30)) return SWL_ERR_UNSUPPORTED;
+    if (!order || !where || !offsets || !expert_idx) return SWL_ERR_BAD_ARG;
+    hipLaunchKernelGGL(swl::moe_sort_kernel, dim3(static_cast<unsigned>(experts)), dim3(swl::kSortThreads), 0,
+                       static_cast<hipStream_t>(stream), order, where, offsets, expert_idx, static_cast<int>(num_assignments), experts);
+    return swl::check_launch();
+}
+
+/* 1 when swl_moe_gemm serves products of these sizes: 16-bit, a reduction of whole 64-deep slices, rows of whole 16-byte pieces, and
+ * operand rows within 4 GiB of their matrix's start. */
+extern "C" int swl_moe_gemm_supported(int64_t x_rows, int32_t K, int32_t N, int32_t dtype) {
+    if (dtype != SWL_F16 && dtype != SWL_BF16) return 0;
+    if (x_rows <= 0 || K <= 0 || N <= 0 || K % swl::kMgDepth || N % 8) return 0;
+    const int64_t row = static_cast<int64_t>(K) * 2;
+    return x_rows * row < (1LL << 32) && 2LL * N * row < (1LL << 32);
+}
+
+extern "C" int swl_moe_gemm(void *out, const void *x, const void *w, const int32_t *order, const int32_t *offsets, const float *in_w,
+                            int64_t num_assignments, int64_t x_rows, int32_t top, int32_t experts, int32_t K, int32_t N, int32_t mode,
+                            int32_t act, float limit, int32_t dtype, swl_stream_t stream) {
+    if (num_assignments < 0 || experts <= 0 || top <= 0 || mode < 0 || mode > 2 || act < 0 || act > 1) return SWL_ERR_BAD_ARG;
+    if (in_w && (mode != 1 || !order)) return SWL_ERR_BAD_ARG;
+    if (num_assignments == 0) return SWL_OK;
+    if (!swl_moe_gemm_supported(x_rows, K, N, dtype)) return SWL_ERR_UNSUPPORTED;
+    // (rows of x: assignments when sorted, else tokens)
+    if (order ? x_rows * top < num_assignments : x_rows < num_assignments) return SWL_ERR_BAD_ARG;
+    if (!out || !x || !w || !offsets || !swl::aligned16(out) || !swl::aligned16(x) || !swl::aligned16(w)) return SWL_ERR_BAD_ARG;
+    swl::MoeGemmParams p;
+    p.out = out; p.x = x; p.w = w; p.order = order; p.offsets = offsets; p.in_w = in_w;
+    p.top = top; p.experts = experts; p.K = K; p.N = N; p.act = act; p.limit = limit;
+    const int cols = mode == 1 ? 64 : 128;
+    p.n_tiles = (N + cols - 1) / cols;
+    // as many row tiles as there can be (every expert may end in a part of one); surplus workgroups leave at once
+    const int64_t m_tiles = (num_assignments + swl::kMgTile - 1) / swl::kMgTile + (experts < num_assignments ? experts : num_assignments);
+    p.per_xcd = static_cast<int>((m_tiles + 7) / 8);
+    const int64_t grid = 8LL * p.per_xcd * p.n_tiles;
+    if (grid > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+#define SWL_MG(MODE) hipLaunchKernelGGL((swl::moe_gemm_kernel<T, MODE>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, p)
+    SWL_DISPATCH_DTYPE(dtype, T, {
+        if (mode == 0) SWL_MG(0);
+        else if (mode == 1) SWL_MG(1);
+        else SWL_MG(2);
+    });
+#undef SWL_MG
+    return swl::check_launch();
+}

@@ -54,6 +54,8 @@ def moe_experts_relu2(h: torch.Tensor, idx: torch.Tensor, wts: torch.Tensor, up:
     code, stream = _hip.dtype_code3(h.dtype), _hip.stream()
     out = torch.empty((n, width), dtype=h.dtype, device=h.device)
     if n * top_k >= GROUPED_MIN_ROWS_PER_EXPERT * experts and not torch.cuda.is_current_stream_capturing():
+        if _sorted_served(h, up, down, ff):
+            return _moe_sorted(h, idx, wts, up, down, ff, 2, 0, 0.0, False)
         flat = idx.reshape(-1).long()
         order = torch.argsort(flat, stable=True)
         counts = torch.bincount(flat, minlength=experts).tolist()
@@ -92,9 +94,43 @@ def moe_experts_relu2(h: torch.Tensor, idx: torch.Tensor, wts: torch.Tensor, up:
     return out
 
 
-# From this many assignments per expert on (on average), a step's expert products are library GEMMs over the assignments
-# sorted by expert; below, every assignment streams its expert's rows (decode batches: capturable, no host read-back).
+# From this many assignments per expert on (on average), a step's expert products run over the assignments sorted by expert: in one
+# matrix-core launch each (csrc/moe_grouped.hip) where the sizes allow it, else (fp32, odd sizes) as a library GEMM per expert; below,
+# every assignment streams its expert's rows (decode batches: capturable).
 GROUPED_MIN_ROWS_PER_EXPERT = 16
+
+
+def _sorted_served(h: torch.Tensor, up: torch.Tensor, down: torch.Tensor, ff: int) -> bool:
+    if h.dtype not in (torch.float16, torch.bfloat16):
+        return False
+    lib, code, (n, width) = _hip.load(), _hip.dtype_code(h.dtype), h.shape
+    return bool(h.is_contiguous() and (h.data_ptr() | up.data_ptr() | down.data_ptr()) % 16 == 0
+                and lib.swl_moe_gemm_supported(n, width, ff, code)
+                # (the activations of a token's experts are at most `experts` rows a token)
+                and lib.swl_moe_gemm_supported(n * up.shape[0], ff, width, code))
+
+
+def _moe_sorted(h, idx, wts, up, down, ff, mode, act, limit, weigh_inputs):
+    """Sort on the device, first product with its activation, second product, weighted combination: no read-back. Positions, products
+    and weights are fp32 until the results of each launch are rounded once."""
+    n, width = h.shape
+    experts, top_k = up.shape[0], idx.shape[1]
+    total, dev, code, stream = n * top_k, h.device, _hip.dtype_code(h.dtype), _hip.stream()
+    order = torch.empty(total, dtype=torch.int32, device=dev)
+    where = torch.empty(total, dtype=torch.int64, device=dev)
+    offsets = torch.empty(experts + 1, dtype=torch.int32, device=dev)
+    idx = idx.contiguous()
+    _hip.call("swl_moe_sort", _hip.ptr(order), _hip.ptr(where), _hip.ptr(offsets), _hip.ptr(idx), total, experts, stream)
+    y = torch.empty((total, ff), dtype=h.dtype, device=dev)
+    _hip.call("swl_moe_gemm", _hip.ptr(y), _hip.ptr(h), _hip.ptr(up), _hip.ptr(order), _hip.ptr(offsets),
+              _hip.ptr(wts) if weigh_inputs else 0, total, n, top_k, experts, width, ff, mode, act, float(limit), code, stream)
+    rows = torch.empty((total, width), dtype=h.dtype, device=dev)
+    _hip.call("swl_moe_gemm", _hip.ptr(rows), _hip.ptr(y), _hip.ptr(down), 0, _hip.ptr(offsets), 0, total, total, top_k, experts, ff,
+              width, 0, 0, 0.0, code, stream)
+    out = torch.empty((n, width), dtype=h.dtype, device=dev)
+    _hip.call("swl_moe_combine", _hip.ptr(out), _hip.ptr(rows), _hip.ptr(where), 0 if weigh_inputs else _hip.ptr(wts), n, width,
+              top_k, code, stream)
+    return out
 
 
 _identities = {}
@@ -201,6 +237,8 @@ def moe_experts(h: torch.Tensor, idx: torch.Tensor, wts: torch.Tensor, gate_up: 
     assert gate_up.is_contiguous() and down.is_contiguous() and down.shape == (experts, width, ff)
     assert gate_up.dtype == down.dtype == h.dtype and idx.dtype == torch.int32 and wts.dtype == torch.float32
     if n * top_k >= GROUPED_MIN_ROWS_PER_EXPERT * experts and not torch.cuda.is_current_stream_capturing():
+        if act in (ACT_CLAMPED, ACT_SILU) and _sorted_served(h, gate_up, down, ff):
+            return _moe_sorted(h, idx, wts, gate_up, down, ff, 1, act, limit, weigh_inputs)
         return moe_experts_grouped(h, idx, wts, gate_up, down, limit, act, weigh_inputs)
     code, stream = _hip.dtype_code3(h.dtype), _hip.stream()
     in_w, out_w = (_hip.ptr(wts), 0) if weigh_inputs else (0, _hip.ptr(wts))
