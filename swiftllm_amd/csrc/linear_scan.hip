@@ -16,7 +16,12 @@
 //                      the accumulators of the fp32 matrix core (16x16x4: exact fp32 operands): the rows are shared out over the
 //                      waves, and an accumulator tile is, register by register, the B operand of the read-out when the reduction
 //                      index is taken in the order 4 (lane / 16) + r — so the state never moves. The waves' partial outputs meet
-//                      in LDS, one barrier per tile; the next tile's operands are requested a tile ahead.
+//                      in LDS, one barrier per tile; the next tiles' operands are requested ahead, as whole 1 KiB blocks. A head's
+//                      column shares read the same operands: they run on one XCD (whose L2 holds them), neighbouring heads on the
+//                      next, so that the long portions of a step that mixes prompts and decoded tokens spread over the chip: with
+//                      the portion as the fastest grid index the two prompts beside 30 decoded tokens met on 16 CUs of two XCDs.
+//                      2 x 1000 + 30 tokens, 8 heads of 128 x 128: 360 -> 85 us. 32 columns a workgroup (half the operand reads)
+//                      took 136 us there and 106 instead of 99 us at 11 x 333 tokens, 16 heads.
 //   swl_linear_step:   steps whose portions are single tokens (decode): one workgroup per (sequence, head) streams the state once
 //                      and finishes the head — read-out, RMS norm over the head, weight, gate — in the same launch.
 // Everything after the loads of q, k, v is fp32.
@@ -60,16 +65,16 @@ __global__ __launch_bounds__(kLsThreads) void linear_chunks_kernel(
     __syncthreads();
     for (int e = threadIdx.x; e < dp; e += kLsThreads) {
         float p = 1.f;
-        float *qo = qd + at * kLsTile * dp + e;
+        float *qo = qd + at * kLsTile * dp + (e >> 4) * 256 + (e & 15);     // 16 x 16 blocks [channels / 16][token][channel]
 #pragma unroll
         for (int t = 0; t < kLsTile; ++t) {
             const float a = as[t * dp + e];
             if constexpr (BONUS) {
-                qo[t * dp] = qs[t * dp + e] * p;
+                qo[t * 16] = qs[t * dp + e] * p;
                 p *= a;
             } else {
                 p *= a;
-                qo[t * dp] = qs[t * dp + e] * p;
+                qo[t * 16] = qs[t * dp + e] * p;
             }
         }
         total[at * dp + e] = p;
@@ -136,9 +141,11 @@ __global__ __launch_bounds__(kLsThreads) void linear_scan_kernel(
     float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra, const T *v,
     int64_t v_stride, const float *dskip, float *state, int64_t slot_stride, int64_t s_off, const int32_t *seq_row0,
     const int32_t *seq_cnt, const int32_t *seq_tile0, const int32_t *tok_pos, const int32_t *tok_state, int H, int d, int dp,
-    int dv) {
+    int dv, int shares, int units) {
     __shared__ float red[2][kLsWaves][256];
-    const int seq = blockIdx.x, h = blockIdx.y, col0 = blockIdx.z * 16;
+    const int id = blockIdx.x, unit = (id & 7) + 8 * ((id >> 3) / shares);      // (portion, head); id % 8 is the XCD
+    if (unit >= units) return;
+    const int seq = unit / H, h = unit - seq * H, col0 = ((id >> 3) % shares) * 16;
     const int row0 = seq_row0[seq], cnt = seq_cnt[seq], tile0 = seq_tile0[seq];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, lq = lane >> 4;
@@ -165,7 +172,7 @@ __global__ __launch_bounds__(kLsThreads) void linear_scan_kernel(
 #pragma unroll
         for (int j = 0; j < TW; ++j) {
             const int tl = min(wave * TW + j, ntiles - 1);
-            f.q[j] = *reinterpret_cast<const float4_t *>(qd + (at * kLsTile + li) * dp + 16 * tl + 4 * lq);
+            f.q[j] = *reinterpret_cast<const float4_t *>(qd + at * kLsTile * dp + tl * 256 + li * 16 + 4 * lq);
             f.k[j] = *reinterpret_cast<const float4_t *>(kd + (at * dp + 16 * tl + li) * kLsTile + 4 * lq);
             f.a[j] = *reinterpret_cast<const float4_t *>(total + at * dp + 16 * tl + 4 * lq);
         }
@@ -396,15 +403,17 @@ extern "C" int swl_linear_scan(float *o, int64_t o_stride, const float *qd, cons
         return SWL_ERR_BAD_ARG;
     if (!swl::aligned16(qd) || !swl::aligned16(kd) || !swl::aligned16(total)) return SWL_ERR_BAD_ARG;
     const int dp = (dim + 15) / 16 * 16, shares = (vdim + 15) / 16;
-    if (dp > swl::kLsMaxDim || num_heads > 65535 || shares > 65535) return SWL_ERR_UNSUPPORTED;
+    const int64_t units = static_cast<int64_t>(num_seqs) * num_heads, blocks = 8 * ((units + 7) / 8) * shares;
+    if (dp > swl::kLsMaxDim || num_heads > 65535 || shares > 65535 || blocks > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
     const int tw = (dp / 16 + swl::kLsWaves - 1) / swl::kLsWaves;       // 1 .. 5
-    const dim3 grid(static_cast<unsigned>(num_seqs), static_cast<unsigned>(num_heads), static_cast<unsigned>(shares));
+    const dim3 grid(static_cast<unsigned>(blocks));
 #define SWL_LS(N)                                                                                                             \
     case N:                                                                                                                   \
         hipLaunchKernelGGL((swl::linear_scan_kernel<T, N, (N <= 2 ? 2 : 1)>), grid, dim3(swl::kLsThreads), 0,                 \
                            static_cast<hipStream_t>(stream), o, o_stride, qd, kd, total, intra,                         \
                            static_cast<const T *>(v), v_stride, dskip, state, slot_stride, s_off,                             \
-                           seq_row0, seq_cnt, seq_tile0, tok_pos, tok_state, num_heads, dim, dp, vdim);                       \
+                           seq_row0, seq_cnt, seq_tile0, tok_pos, tok_state, num_heads, dim, dp, vdim, shares,                \
+                           static_cast<int>(units));                                                                          \
         break
     SWL_DISPATCH_DTYPE3(dtype, T, {
         switch (tw) {
