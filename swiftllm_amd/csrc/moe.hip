@@ -27,40 +27,39 @@ __device__ __forceinline__ bool aligned16_dev(const void *p) { return (reinterpr
 constexpr int kMoeThreads = 256;
 constexpr int kMoeWaves = kMoeThreads / 64;
 
-// Per-lane share of sum_i x[i] * w[i] over a row of n elements (x fp32 in LDS, w in global memory); the caller reduces
-// over the wave. 16-bit rows whose length is a multiple of 8 are read 16 bytes per lane.
-template <typename T>
-__device__ __forceinline__ float lane_dot(const float *x, const T *w, int n, int lane) {
-    float a = 0.f;
-    if constexpr (sizeof(T) == 2) {
-        if ((n & 7) == 0 && aligned16_dev(w)) {
-            for (int i = lane * 8; i < n; i += 64 * 8) {
-                const vec8_t<T> v = load8(w + i);
+// Per-lane shares of sum_i x[i] * w[r][i] over N rows of n elements (x: fp32 in LDS or a row in global memory; the caller reduces over
+// the wave): 16 bytes per lane and row where the rows allow it, all rows' loads of a turn in flight together.
+template <int N, typename X, typename T>
+__device__ __forceinline__ void lane_dots(float (&a)[N], const X *x, const T *const (&w)[N], int n, int lane) {
+    constexpr int V = 16 / sizeof(T);
+    bool wide = n % V == 0 && (sizeof(X) != 2 || aligned16_dev(x));
 #pragma unroll
-                for (int j = 0; j < 8; ++j) a += x[i + j] * to_f(v[j]);
-            }
-            return a;
-        }
+    for (int r = 0; r < N; ++r) {
+        a[r] = 0.f;
+        wide = wide && aligned16_dev(w[r]);
     }
-    for (int i = lane; i < n; i += 64) a += x[i] * to_f(w[i]);
-    return a;
-}
-// The same with both rows in global memory.
-template <typename T>
-__device__ __forceinline__ float lane_dot2(const T *x, const T *w, int n, int lane) {
-    float a = 0.f;
-    if constexpr (sizeof(T) == 2) {
-        if ((n & 7) == 0 && aligned16_dev(w) && aligned16_dev(x)) {
-            for (int i = lane * 8; i < n; i += 64 * 8) {
-                const vec8_t<T> v = load8(w + i), u = load8(x + i);
+    if (wide) {
+#pragma unroll 2
+        for (int i = lane * V; i < n; i += 64 * V) {
+            typedef T vec __attribute__((ext_vector_type(V)));
+            vec v[N];
+            float xv[V];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) a += to_f(u[j]) * to_f(v[j]);
-            }
-            return a;
+            for (int r = 0; r < N; ++r) v[r] = *reinterpret_cast<const vec *>(w[r] + i);
+#pragma unroll
+            for (int k = 0; k < V; ++k) xv[k] = to_f(x[i + k]);
+#pragma unroll
+            for (int r = 0; r < N; ++r)
+#pragma unroll
+                for (int k = 0; k < V; ++k) a[r] += xv[k] * to_f(v[r][k]);
         }
+        return;
     }
-    for (int i = lane; i < n; i += 64) a += to_f(x[i]) * to_f(w[i]);
-    return a;
+    for (int i = lane; i < n; i += 64) {
+        const float xv = to_f(x[i]);
+#pragma unroll
+        for (int r = 0; r < N; ++r) a[r] += xv * to_f(w[r][i]);
+    }
 }
 
 // The token's row as fp32 in LDS, for the whole workgroup (the caller synchronises).
@@ -269,12 +268,19 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_grouped_kernel(int32_t 
     }
 }
 
-// grid (assignments, ceil(ff / 64)): wave w of the workgroup computes ff rows f0 + w, f0 + w + 4, ...
+// The per-assignment kernels: every (token, chosen expert) streams its expert's rows. Bound by latency at decode sizes (3 tokens, two
+// experts of 1024 x 1024, fp32: 25 MB), so a workgroup owns sixteen outputs and a wave four rows at a time, whose loads are in flight
+// together. That shape: up 115 and down 228 us with 64 outputs a workgroup and one row
+// of 4-byte loads at a time, 7.5 and 8 us.
+constexpr int kMoeRows = 16;        // outputs of a workgroup
+inline int moe_rows(int n) { return (n + kMoeRows - 1) / kMoeRows <= 65535 ? kMoeRows : 64; }
+
+// grid (assignments, ceil(ff / rows))
 template <typename T>
 __global__ __launch_bounds__(kMoeThreads) void moe_gate_up_kernel(T *y, const T *h, const T *gate_up,
                                                                   const int32_t *expert_idx, const float *in_w, int width,
-                                                                  int ff, int top, float limit, int act) {
-    extern __shared__ float lds[];
+                                                                  int ff, int top, float limit, int act, int rows) {
+    extern __shared__ __align__(16) float lds[];
     float *hf = lds;    // [width]
     const int64_t a = blockIdx.x;           // assignment = token * top + j
     const int64_t t = a / top;
@@ -284,25 +290,27 @@ __global__ __launch_bounds__(kMoeThreads) void moe_gate_up_kernel(T *y, const T 
     __syncthreads();
     const T *wg = gate_up + static_cast<int64_t>(e) * 2 * ff * width;
     const T *wu = wg + static_cast<int64_t>(ff) * width;
-    const int f0 = blockIdx.y * 64;
-    for (int f = f0 + wave; f < min(ff, f0 + 64); f += kMoeWaves) {
-        const T *rg = wg + static_cast<int64_t>(f) * width, *ru = wu + static_cast<int64_t>(f) * width;
-        float g = lane_dot(hf, rg, width, lane), u = lane_dot(hf, ru, width, lane);
-        g = wave_allreduce_sum(g);
-        u = wave_allreduce_sum(u);
-        if (in_w) {
-            g *= in_w[a];
-            u *= in_w[a];
+    const int f0 = blockIdx.y * rows, f1 = min(ff, f0 + rows);
+    for (int f = f0 + 2 * wave; f < f1; f += 2 * kMoeWaves) {
+        const int64_t at0 = static_cast<int64_t>(f) * width, at1 = static_cast<int64_t>(min(f + 1, f1 - 1)) * width;
+        const T *const w[4] = {wg + at0, wu + at0, wg + at1, wu + at1};
+        float v[4];
+        lane_dots(v, hf, w, width, lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            v[r] = wave_allreduce_sum(v[r]);
+            if (in_w) v[r] *= in_w[a];
         }
-        if (lane == 0) y[a * ff + f] = to_t<T>(gated_unit(g, u, limit, act));
+        if (lane == 0) y[a * ff + f] = to_t<T>(gated_unit(v[0], v[1], limit, act));
+        if (lane == 0 && f + 1 < f1) y[a * ff + f + 1] = to_t<T>(gated_unit(v[2], v[3], limit, act));
     }
 }
 
 // Experts without a gate: y = relu(W_up h)^2 for every (token, chosen expert); up [experts, ff, width]. Same grid.
 template <typename T>
 __global__ __launch_bounds__(kMoeThreads) void moe_up_relu2_kernel(T *y, const T *h, const T *up, const int32_t *expert_idx,
-                                                                   int width, int ff, int top) {
-    extern __shared__ float lds[];
+                                                                   int width, int ff, int top, int rows) {
+    extern __shared__ __align__(16) float lds[];
     float *hf = lds;    // [width]
     const int64_t a = blockIdx.x;
     const int64_t t = a / top;
@@ -311,12 +319,17 @@ __global__ __launch_bounds__(kMoeThreads) void moe_up_relu2_kernel(T *y, const T
     for (int i = threadIdx.x; i < width; i += kMoeThreads) hf[i] = to_f(h[t * width + i]);
     __syncthreads();
     const T *wu = up + static_cast<int64_t>(e) * ff * width;
-    const int f0 = blockIdx.y * 64;
-    for (int f = f0 + wave; f < min(ff, f0 + 64); f += kMoeWaves) {
-        float u = wave_allreduce_sum(lane_dot(hf, wu + static_cast<int64_t>(f) * width, width, lane));
-        if (lane == 0) {
-            u = fmaxf(u, 0.f);
-            y[a * ff + f] = to_t<T>(u * u);
+    const int f0 = blockIdx.y * rows, f1 = min(ff, f0 + rows);
+    for (int f = f0 + 4 * wave; f < f1; f += 4 * kMoeWaves) {
+        const T *w[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) w[r] = wu + static_cast<int64_t>(min(f + r, f1 - 1)) * width;
+        float v[4];
+        lane_dots(v, hf, w, width, lane);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float u = fmaxf(wave_allreduce_sum(v[r]), 0.f);
+            if (lane == 0 && f + r < f1) y[a * ff + f + r] = to_t<T>(u * u);
         }
     }
 }
@@ -349,24 +362,32 @@ __global__ __launch_bounds__(kMoeThreads) void relu_sq_wide_kernel(T *y, const T
     store8(y + r * static_cast<int64_t>(ff8) * 8 + c, o);
 }
 
-// grid (tokens, ceil(width / 64)): wave w computes output columns c0 + w, c0 + w + 4, ...
+// grid (tokens, ceil(width / rows)): out[t][c] = sum_j w[t][j] y[t * top + j] . down[e_j][c]
 template <typename T>
 __global__ __launch_bounds__(kMoeThreads) void moe_down_combine_kernel(T *out, const T *y, const T *down,
                                                                        const int32_t *expert_idx, const float *expert_w,
-                                                                       int width, int ff, int top) {
+                                                                       int width, int ff, int top, int rows) {
     const int64_t t = blockIdx.x;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int c0 = blockIdx.y * 64;
-    for (int c = c0 + wave; c < min(width, c0 + 64); c += kMoeWaves) {
-        float total = 0.f;
+    const int c0 = blockIdx.y * rows, c1 = min(width, c0 + rows);
+    for (int c = c0 + 4 * wave; c < c1; c += 4 * kMoeWaves) {
+        float total[4] = {0.f, 0.f, 0.f, 0.f};
         for (int j = 0; j < top; ++j) {
-            const int e = expert_idx[t * top + j];
-            const T *wr = down + (static_cast<int64_t>(e) * width + c) * ff;
-            const T *yr = y + (t * top + j) * ff;
-            float a = wave_allreduce_sum(lane_dot2(yr, wr, ff, lane));
-            total += expert_w ? expert_w[t * top + j] * a : a;
+            const T *wd = down + static_cast<int64_t>(expert_idx[t * top + j]) * width * ff;
+            const T *w[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) w[r] = wd + static_cast<int64_t>(min(c + r, c1 - 1)) * ff;
+            float v[4];
+            lane_dots(v, y + (t * top + j) * ff, w, ff, lane);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float a = wave_allreduce_sum(v[r]);
+                total[r] += expert_w ? expert_w[t * top + j] * a : a;
+            }
         }
-        if (lane == 0) out[t * width + c] = to_t<T>(total);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (lane == 0 && c + r < c1) out[t * width + c + r] = to_t<T>(total[r]);
     }
 }
 
@@ -565,9 +586,8 @@ __global__ __launch_bounds__(kMoeThreads) void moe_combine_kernel(T *out, const 
     }
 }
 
-// The same for 16-bit rows of whole 16-byte pieces: 8 columns a lane, flat over (token, piece). Bound by HBM: 2 `top` + 1 rows a token;
-// 8000 tokens of 1024, two
-// rows each: 20 us with one 2-byte access a lane and row, 10 us.
+// The same for 16-bit rows of whole 16-byte pieces: 8 columns a lane, flat over (token, piece). Bound by HBM: `top` + 1 rows a token;
+// 8000 tokens of 1024, two rows each: 20 us with one 2-byte access a lane and row, 10 us.
 template <typename T>
 __global__ __launch_bounds__(kMoeThreads) void moe_combine_wide_kernel(T *out, const T *rows, const int64_t *where, const float *w,
                                                                        int64_t pieces, int width8, int top) {
@@ -733,11 +753,12 @@ extern "C" int swl_moe_gate_up(void *y, const void *h, const void *gate_up, cons
     const size_t lds = static_cast<size_t>(width) * 4;
     const int64_t assignments = num_tokens * top;
     if (assignments > 0x7fffffffLL || lds > 64 * 1024 || (ff + 63) / 64 > 65535) return SWL_ERR_UNSUPPORTED;
-    const dim3 grid(static_cast<unsigned>(assignments), static_cast<unsigned>((ff + 63) / 64));
+    const int rows = swl::moe_rows(ff);
+    const dim3 grid(static_cast<unsigned>(assignments), static_cast<unsigned>((ff + rows - 1) / rows));
     SWL_DISPATCH_DTYPE3(dtype, T, {
         hipLaunchKernelGGL((swl::moe_gate_up_kernel<T>), grid, dim3(swl::kMoeThreads), lds,
                            static_cast<hipStream_t>(stream), static_cast<T *>(y), static_cast<const T *>(h),
-                           static_cast<const T *>(gate_up), expert_idx, in_w, width, ff, top, limit, act);
+                           static_cast<const T *>(gate_up), expert_idx, in_w, width, ff, top, limit, act, rows);
     });
     return swl::check_launch();
 }
@@ -749,11 +770,12 @@ extern "C" int swl_moe_down_combine(void *out, const void *y, const void *down, 
     if (num_tokens == 0) return SWL_OK;
     if (!out || !y || !down || !expert_idx) return SWL_ERR_BAD_ARG;
     if (num_tokens > 0x7fffffffLL || (width + 63) / 64 > 65535) return SWL_ERR_UNSUPPORTED;
-    const dim3 grid(static_cast<unsigned>(num_tokens), static_cast<unsigned>((width + 63) / 64));
+    const int rows = swl::moe_rows(width);
+    const dim3 grid(static_cast<unsigned>(num_tokens), static_cast<unsigned>((width + rows - 1) / rows));
     SWL_DISPATCH_DTYPE3(dtype, T, {
         hipLaunchKernelGGL((swl::moe_down_combine_kernel<T>), grid, dim3(swl::kMoeThreads), 0,
                            static_cast<hipStream_t>(stream), static_cast<T *>(out), static_cast<const T *>(y),
-                           static_cast<const T *>(down), expert_idx, expert_w, width, ff, top);
+                           static_cast<const T *>(down), expert_idx, expert_w, width, ff, top, rows);
     });
     return swl::check_launch();
 }
@@ -766,11 +788,12 @@ extern "C" int swl_moe_up_relu2(void *y, const void *h, const void *up, const in
     const size_t lds = static_cast<size_t>(width) * 4;
     const int64_t assignments = num_tokens * top;
     if (assignments > 0x7fffffffLL || lds > 64 * 1024 || (ff + 63) / 64 > 65535) return SWL_ERR_UNSUPPORTED;
-    const dim3 grid(static_cast<unsigned>(assignments), static_cast<unsigned>((ff + 63) / 64));
+    const int rows = swl::moe_rows(ff);
+    const dim3 grid(static_cast<unsigned>(assignments), static_cast<unsigned>((ff + rows - 1) / rows));
     SWL_DISPATCH_DTYPE3(dtype, T, {
         hipLaunchKernelGGL((swl::moe_up_relu2_kernel<T>), grid, dim3(swl::kMoeThreads), lds,
                            static_cast<hipStream_t>(stream), static_cast<T *>(y), static_cast<const T *>(h),
-                           static_cast<const T *>(up), expert_idx, width, ff, top);
+                           static_cast<const T *>(up), expert_idx, width, ff, top, rows);
     });
     return swl::check_launch();
 }
