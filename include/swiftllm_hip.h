@@ -575,6 +575,15 @@ int swl_masked_attn(void *out, const void *q, const void *k_cache, const void *v
                     int64_t block_stride, int32_t mask_kind, const float *sink, int32_t num_v_heads, int32_t out_f32,
                     const float *slopes, int32_t out_dim, int64_t out_stride, const void *gate, int64_t gate_stride,
                     int32_t dtype, swl_stream_t stream);
+/* swl_masked_attn with every token's pages shared out over key_splits (at most 64) workgroups, whose partial results (scratch:
+ * key_splits * num_tokens * num_q_heads * (vdim + 2) floats, 16-byte aligned) a second launch combines. */
+int swl_masked_attn_shares(void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
+                           const int32_t *tok_seq, const int32_t *tok_pos, const float *talk, const float *rel, int32_t rel_len,
+                           int64_t num_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t dim, int32_t vdim,
+                           int64_t q_tok_stride, int32_t window, float scale, float softcap, int32_t max_blocks_per_seq,
+                           int64_t block_stride, int32_t mask_kind, const float *sink, int32_t num_v_heads, int32_t out_f32,
+                           const float *slopes, int32_t out_dim, int64_t out_stride, const void *gate, int64_t gate_stride,
+                           int32_t key_splits, float *scratch, int32_t dtype, swl_stream_t stream);
 int swl_masked_attn_tiles_supported(int32_t num_q_heads, int32_t num_kv_heads, int32_t num_v_heads, int32_t dim,
                                     int32_t vdim, int32_t dtype);
 int swl_masked_attn_tiles(void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
@@ -773,6 +782,13 @@ int swl_sigmoid_attn(void *out, const void *q, const void *k_cache, const void *
                      const float *pb, int64_t num_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t dim,
                      int32_t vdim, int64_t q_tok_stride, int32_t window, float scale, int32_t max_blocks_per_seq,
                      int64_t block_stride, int32_t dtype, swl_stream_t stream);
+/* The same with every token's pages shared out over key_splits (at most 64) workgroups, whose partial sums (scratch: key_splits *
+ * num_tokens * heads * vdim floats, 16-byte aligned) a second launch adds up. */
+int swl_sigmoid_attn_shares(void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
+                            const int32_t *tok_seq, const int32_t *tok_pos, const float *talk, const float *r1, const float *r2,
+                            const float *pb, int64_t num_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t dim,
+                            int32_t vdim, int64_t q_tok_stride, int32_t window, float scale, int32_t max_blocks_per_seq,
+                            int64_t block_stride, int32_t key_splits, float *scratch, int32_t dtype, swl_stream_t stream);
 /* The matrix-core form (16-bit storage): tiles of up to 16 consecutive queries of one sequence (tile_row0, tile_cnt) against
  * 16-key pages; key_splits > 1: every tile's pages are shared out over that many workgroups, whose fp32 partial sums
  * (scratch: key_splits * num_tokens * heads * vdim floats) a second launch adds up. */

@@ -106,6 +106,8 @@ SIGNATURES = {
                               _I32, _I64, _I32, _P, _I64, _I32, _P],
     "swl_masked_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I64, _I32, _I32, _I32, _I32, _I64, _I32, _F32, _F32, _I32,
                         _I64, _I32, _P, _I32, _I32, _P, _I32, _I64, _P, _I64, _I32, _P],
+    "swl_masked_attn_shares": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I64, _I32, _I32, _I32, _I32, _I64, _I32, _F32, _F32, _I32,
+                        _I64, _I32, _P, _I32, _I32, _P, _I32, _I64, _P, _I64, _I32, _P, _I32, _P],
     "swl_masked_attn_tiles": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I32,
                               _F32, _F32, _I32, _I64, _I32, _P, _I64, _I32, _P, _I32, _I32, _I32, _P, _I32, _I64, _P, _I64,
                               _I32, _P],
@@ -141,6 +143,8 @@ SIGNATURES = {
                                 _I64, _I32, _I64, _F32, _I32, _P],
     "swl_sigmoid_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I64, _I32, _F32, _I32,
                          _I64, _I32, _P],
+    "swl_sigmoid_attn_shares": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I64, _I32, _F32, _I32,
+                         _I64, _I32, _P, _I32, _P],
     "swl_sigmoid_attn_tiles": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I64, _I32,
                                _F32, _I32, _I64, _I32, _P, _I64, _I32, _P],
     "swl_ssd_prep": [_P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32,

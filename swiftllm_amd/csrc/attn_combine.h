@@ -8,7 +8,8 @@ namespace swl {
 
 // out[t][h][:] = sum_s e^{m_s - M} O_s / sum_s e^{m_s - M} l_s over the key shares s (a share without keys has l = 0).
 // The first wave evaluates the shares' weights once (one share per lane, at most 64) and leaves them in LDS.
-template <typename T>
+// NATURAL: the maxima are in natural units (the per-token kernel, whose arithmetic is full-precision throughout).
+template <typename T, bool NATURAL = false>
 __global__ __launch_bounds__(256) void window_attn_combine_kernel(T *out, const float *part_o, const float *part_ml,
                                                                   int64_t rows, int dv, int nsplit, const float *sink, int H,
                                                                   int out_f32, int out_dim, int64_t out_stride, const T *gate,
@@ -24,11 +25,11 @@ __global__ __launch_bounds__(256) void window_attn_combine_kernel(T *out, const 
         float mx = wave_allreduce_max(m);
         float extra = 0.f;
         if (sink) {
-            const float sk = sink[row % H] * 1.4426950408889634f;
+            const float sk = sink[row % H] * (NATURAL ? 1.0f : 1.4426950408889634f);
             mx = fmaxf(mx, sk);
-            extra = exp2f(sk - mx);
+            extra = NATURAL ? expf(sk - mx) : exp2f(sk - mx);
         }
-        const float w = live ? exp2f(m - mx) : 0.f;
+        const float w = live ? (NATURAL ? expf(m - mx) : exp2f(m - mx)) : 0.f;
         const float den = wave_allreduce_sum(w * l) + extra;
         wgt[sp] = w;
         if (sp == 0) inv_den = 1.0f / den;

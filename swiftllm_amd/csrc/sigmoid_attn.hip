@@ -8,83 +8,81 @@
 // portion that continues a cached prefix, a whole prompt and a decoded token are the same case. Pool layout as in
 // qknorm_kv.hip: keys [kv_heads, 16, dim], values transposed [kv_heads, vdim, 16] per 16-token block.
 //
-//   swl_sigmoid_attn:        one workgroup per query token, keys in chunks of 64, everything after the loads in fp32 and
-//                            any storage dtype (fp32 included): the reference-grade kernel.
+//   swl_sigmoid_attn:        one workgroup per query token (and share of its pages: swl_sigmoid_attn_shares), keys in chunks of four
+//                            pages read as token_attn.h does, everything after the loads in fp32 and any storage dtype (fp32
+//                            included): the reference-grade kernel.
 //   swl_sigmoid_attn_tiles:  the matrix-core form for 16-bit storage: tiles of up to 16 consecutive queries of one sequence
 //                            against 16-key pages (see below).
 // Without a running maximum or denominator the sum over keys is a plain sum: key shares of one query (a split over
 // workgroups) are added up, no rescaling.
 #include "swl_common.h"
+#include "token_attn.h"
 
 namespace swl {
 
-constexpr int kSgThreads = 256;
-constexpr int kSgChunk = 64;        // keys per chunk
-constexpr int kSgBlock = 16;        // tokens per KV block
-constexpr int kSgMaxAcc = 32;       // (head, value column) accumulators per thread: H * vdim <= 8192
-
+// fp32 words ahead of the page table (offsets of four blocks)
 __host__ __device__ inline size_t sg_float_count(int H, int d, int mixed) {
-    size_t n = static_cast<size_t>(H) * d + (mixed ? static_cast<size_t>(H) * H : 0) +
-               (mixed ? 2 : 1) * static_cast<size_t>(H) * kSgChunk;
-    return n + (n & 1);
+    const size_t n = static_cast<size_t>(H) * d + (mixed ? static_cast<size_t>(H) * H : 0) +
+                     (mixed ? 2 : 1) * static_cast<size_t>(H) * kTaChunk;
+    return (n + 3) / 4 * 4 + 4;     // (the rows of weights start on 16-byte boundaries)
 }
 
 __device__ __forceinline__ float sg_sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
 
-template <typename T>
-__global__ __launch_bounds__(kSgThreads) void sigmoid_attn_kernel(
+template <typename T, int R>
+__global__ __launch_bounds__(kTaThreads, 2) void sigmoid_attn_kernel(
     T *out, const T *q, const T *k_cache, const T *v_cache, const int32_t *block_table, const int32_t *tok_seq,
     const int32_t *tok_pos, const float *talk, const float *r1, const float *r2, const float *pb, int H, int G, int d, int dv,
-    int64_t q_tok_stride, int window, float scale, int max_blocks_per_seq, int64_t block_stride, int Hall) {
+    int64_t q_tok_stride, int window, float scale, int max_blocks_per_seq, int64_t block_stride, int Hall, float *part_o, int k_wide,
+    int v_wide) {
     // H: heads of this workgroup, starting at head hb of the token's Hall heads (all of them when the heads are mixed)
-    extern __shared__ float lds[];
-    float *qf = lds;                                    // [H * d]
-    float *tk = qf + H * d;                             // [H * H] (mixed only)
-    float *a = tk + (talk ? H * H : 0);                 // [H][64] weights
-    float *p = talk ? a + H * kSgChunk : a;             // [H][64] mixed weights (the weights themselves without a matrix)
-    int64_t *kbase = reinterpret_cast<int64_t *>(lds + sg_float_count(H, d, talk != nullptr));   // [64] block of each key
-    int *koff = reinterpret_cast<int *>(kbase + kSgChunk);                                        // [64] slot in its block
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    float *a = lds;                                     // [H][64] weights
+    float *p = talk ? a + H * kTaChunk : a;             // [H][64] mixed weights (the weights themselves without a matrix)
+    float *qf = p + H * kTaChunk;                       // [H * d]
+    float *tk = qf + (H * d + 3) / 4 * 4;               // [H * H] (mixed only)
+    int64_t *pages = reinterpret_cast<int64_t *>(lds + sg_float_count(H, d, talk != nullptr));   // [4] element offset of each page's block
 
     const int64_t t = blockIdx.x;
     const int tid = threadIdx.x;
     const int pos = tok_pos[t];
     const int32_t *bt = block_table + static_cast<int64_t>(tok_seq[t]) * max_blocks_per_seq;
     const int lo = window <= 0 ? 0 : (pos - window + 1 > 0 ? pos - window + 1 : 0);
-    const int nkeys = pos - lo + 1;
+    int kb0 = lo / kTaPage, kb1 = pos / kTaPage;
+    if (gridDim.z > 1) {        // key split: a contiguous share of the pages (possibly none)
+        const int per = (kb1 - kb0 + static_cast<int>(gridDim.z)) / static_cast<int>(gridDim.z);
+        kb0 += per * static_cast<int>(blockIdx.z);
+        kb1 = min(kb1, kb0 + per - 1);
+    }
     const int rep = Hall / G;
     const int hb = static_cast<int>(blockIdx.y) * H;
     if (hb + H > Hall) H = Hall - hb;
 
     const T *qrow = q + t * q_tok_stride + static_cast<int64_t>(hb) * d;
-    for (int i = tid; i < H * d; i += kSgThreads) qf[i] = to_f(qrow[i]);
+    for (int i = tid; i < H * d; i += kTaThreads) qf[i] = to_f(qrow[i]);
     if (talk)
-        for (int i = tid; i < H * H; i += kSgThreads) tk[i] = talk[i];
+        for (int i = tid; i < H * H; i += kTaThreads) tk[i] = talk[i];
 
-    float acc[kSgMaxAcc];
+    float acc[kTaMaxAcc / R][R];
 #pragma unroll
-    for (int i = 0; i < kSgMaxAcc; ++i) acc[i] = 0.f;
-    const int nacc = (H * dv + kSgThreads - 1) / kSgThreads;
+    for (int i = 0; i < kTaMaxAcc / R; ++i)
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[i][r] = 0.f;
 
-    for (int c0 = 0; c0 < nkeys; c0 += kSgChunk) {
-        const int cn = min(kSgChunk, nkeys - c0);
+    for (int kb = kb0; kb <= kb1; kb += 4) {
+        const int first = max(lo - kb * kTaPage, 0), last = min(min(pos, kb1 * kTaPage + kTaPage - 1) - kb * kTaPage, kTaChunk - 1);
         __syncthreads();    // the previous chunk's weights are consumed (and qf / tk written, the first time)
-        if (tid < cn) {
-            const int kp = lo + c0 + tid;
-            kbase[tid] = bt[kp / kSgBlock];
-            koff[tid] = kp % kSgBlock;
-        }
+        if (tid < 4) pages[tid] = bt[min(kb + tid, kb1)] * block_stride;
         __syncthreads();
         // 1. weights of every head of this workgroup
-        for (int idx = tid; idx < H * kSgChunk; idx += kSgThreads) {
-            const int g = idx / kSgChunk, j = idx - g * kSgChunk;
+        ta_scores(a, qf, k_cache, pages, first, last, H, hb, rep, d, k_wide != 0);
+        __syncthreads();
+        for (int idx = tid; idx < H * kTaChunk; idx += kTaThreads) {
+            const int g = idx / kTaChunk, j = idx - g * kTaChunk;
             float w = 0.f;
-            if (j < cn) {
-                const T *kr = k_cache + kbase[j] * block_stride + (static_cast<int64_t>((hb + g) / rep) * kSgBlock + koff[j]) * d;
-                const float *qh = qf + g * d;
-                float s = 0.f;
-                for (int e = 0; e < d; ++e) s += qh[e] * to_f(kr[e]);
-                s *= scale;
-                if (r1) s -= r1[hb + g] * logf(1.0f + r2[hb + g] * static_cast<float>(pos - (lo + c0 + j)));
+            if (j >= first && j <= last) {
+                float s = a[idx] * scale;
+                if (r1) s -= r1[hb + g] * logf(1.0f + r2[hb + g] * static_cast<float>(pos - (kb * kTaPage + j)));
                 if (pb) s += pb[hb + g];
                 w = sg_sigmoid(s);
             }
@@ -93,38 +91,30 @@ __global__ __launch_bounds__(kSgThreads) void sigmoid_attn_kernel(
         __syncthreads();
         // 2. mix the heads
         if (talk) {
-            for (int idx = tid; idx < H * kSgChunk; idx += kSgThreads) {
-                const int h = idx / kSgChunk, j = idx - h * kSgChunk;
+            for (int idx = tid; idx < H * kTaChunk; idx += kTaThreads) {
+                const int h = idx / kTaChunk, j = idx - h * kTaChunk;
                 float m = 0.f;
-                for (int g = 0; g < H; ++g) m += tk[h * H + g] * a[g * kSgChunk + j];
+                for (int g = 0; g < H; ++g) m += tk[h * H + g] * a[g * kTaChunk + j];
                 p[idx] = m;
             }
             __syncthreads();
         }
         // 3. weighted values
-#pragma unroll
-        for (int i = 0; i < kSgMaxAcc; ++i) {
-            if (i >= nacc) break;
-            const int idx = tid + i * kSgThreads;
-            if (idx < H * dv) {
-                const int h = idx / dv, col = idx - h * dv;
-                const int g = (hb + h) / rep;
-                float s = acc[i];
-                const float *ph = p + h * kSgChunk;
-                for (int j = 0; j < cn; ++j) {
-                    const T *vr = v_cache + kbase[j] * block_stride + (static_cast<int64_t>(g) * dv + col) * kSgBlock;
-                    s += ph[j] * to_f(vr[koff[j]]);
-                }
-                acc[i] = s;
-            }
-        }
+        ta_values<T, R>(acc, p, v_cache, pages, first, last, H, hb, rep, G, dv, v_wide != 0);
     }
-    const int64_t obase = (t * static_cast<int64_t>(Hall) + hb) * dv;
+    // (key shares: plain sums, added up by a second launch)
+    const int64_t obase = ((gridDim.z > 1 ? static_cast<int64_t>(blockIdx.z) * gridDim.x : 0) + t) * Hall * dv + static_cast<int64_t>(hb) * dv;
 #pragma unroll
-    for (int i = 0; i < kSgMaxAcc; ++i) {
-        if (i >= nacc) break;
-        const int idx = tid + i * kSgThreads;
-        if (idx < H * dv) out[obase + idx] = to_t<T>(acc[i]);
+    for (int i = 0; i < kTaMaxAcc / R; ++i) {
+        const int idx = tid + i * kTaThreads;
+        if (i * kTaThreads >= H / R * dv) break;
+        if (idx >= H / R * dv) continue;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int64_t at = obase + static_cast<int64_t>(idx / dv * R + r) * dv + idx % dv;
+            if (gridDim.z > 1) part_o[at] = acc[i][r];
+            else out[at] = to_t<T>(acc[i][r]);
+        }
     }
 }
 
@@ -314,6 +304,14 @@ template <typename T>
 __global__ __launch_bounds__(256) void sigmoid_attn_sum_kernel(T *out, const float *part, int64_t total, int nsplit) {
     const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
     if (i >= total) return;
+    if (total & 3) {        // (uniform) odd rows: element by element
+        for (int64_t k = i; k < min(i + 4, total); ++k) {
+            float a = part[k];
+            for (int s = 1; s < nsplit; ++s) a += part[s * total + k];
+            out[k] = to_t<T>(a);
+        }
+        return;
+    }
     float4_t a = *reinterpret_cast<const float4_t *>(part + i);
     for (int s = 1; s < nsplit; ++s) a += *reinterpret_cast<const float4_t *>(part + s * total + i);
     typedef T vec4 __attribute__((ext_vector_type(4)));
@@ -355,9 +353,61 @@ int launch_sm(int hpw, dim3 grid, size_t lds, hipStream_t s, T *out, const T *q,
     return check_launch();
 }
 
-inline size_t sg_lds_bytes(int H, int d, int mixed) { return sg_float_count(H, d, mixed) * 4 + kSgChunk * (8 + 4); }
+inline size_t sg_lds_bytes(int H, int d, int mixed) { return sg_float_count(H, d, mixed) * 4 + 4 * sizeof(int64_t); }
 
 } // namespace swl
+
+extern "C" int swl_sigmoid_attn_shares(void *out, const void *q, const void *k_cache, const void *v_cache,
+                                const int32_t *block_table, const int32_t *tok_seq, const int32_t *tok_pos, const float *talk,
+                                const float *r1, const float *r2, const float *pb, int64_t num_tokens, int32_t num_q_heads,
+                                int32_t num_kv_heads, int32_t dim, int32_t vdim, int64_t q_tok_stride, int32_t window,
+                                float scale, int32_t max_blocks_per_seq, int64_t block_stride, int32_t key_splits,
+                                float *scratch, int32_t dtype, swl_stream_t stream) {
+    if (num_tokens < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || dim <= 0 || vdim <= 0 || window < 0) return SWL_ERR_BAD_ARG;
+    if (num_q_heads % num_kv_heads || (r1 == nullptr) != (r2 == nullptr)) return SWL_ERR_BAD_ARG;
+    if (key_splits < 1 || key_splits > 64 || (key_splits > 1 && (!scratch || !swl::aligned16(scratch)))) return SWL_ERR_BAD_ARG;
+    if (num_tokens == 0) return SWL_OK;
+    if (!out || !q || !k_cache || !v_cache || !block_table || !tok_seq || !tok_pos) return SWL_ERR_BAD_ARG;
+    // heads per workgroup: all of them when they are mixed, else as many as its accumulators and LDS hold
+    int hpg = num_q_heads;
+    if (!talk)
+        while (hpg > 1 && (static_cast<int64_t>(hpg) * vdim > swl::kTaMaxAcc * swl::kTaThreads ||
+                           swl::sg_lds_bytes(hpg, dim, 0) > 64 * 1024))
+            --hpg;
+    const size_t lds = swl::sg_lds_bytes(hpg, dim, talk != nullptr);
+    if (num_tokens > 0x7fffffffLL || static_cast<int64_t>(hpg) * vdim > swl::kTaMaxAcc * swl::kTaThreads || lds > 64 * 1024)
+        return SWL_ERR_UNSUPPORTED;
+    const unsigned groups = static_cast<unsigned>((num_q_heads + hpg - 1) / hpg);
+    const size_t esize = dtype == SWL_F32 ? 4 : 2;
+    auto whole = [&](const void *c, size_t piece, int elems) {     // rows of whole pieces on their boundaries
+        return elems * esize % piece == 0 && block_stride * static_cast<int64_t>(esize) % static_cast<int64_t>(piece) == 0 &&
+               reinterpret_cast<uintptr_t>(c) % piece == 0;
+    };
+    const int k_wide = whole(k_cache, 4 * esize, dim), v_wide = whole(v_cache, 16, 16);
+    // scratch: [splits][tokens][H][vdim] fp32 partial sums for the second launch
+    const int64_t total = num_tokens * num_q_heads * vdim;
+    if (key_splits > 1 && (total / 4 + 256) / 256 > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
+    const dim3 grid(static_cast<unsigned>(num_tokens), groups, static_cast<unsigned>(key_splits));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    SWL_DISPATCH_DTYPE3(dtype, T, {
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(swl::kTaThreads), lds, st, static_cast<T *>(out), static_cast<const T *>(q),
+                               static_cast<const T *>(k_cache), static_cast<const T *>(v_cache), block_table, tok_seq, tok_pos, talk, r1,
+                               r2, pb, hpg, num_kv_heads, dim, vdim, q_tok_stride, window, scale, max_blocks_per_seq, block_stride,
+                               num_q_heads, scratch, k_wide, v_wide);
+        };
+        switch (swl::ta_share(num_q_heads / num_kv_heads, hpg)) {
+        case 8: go(&swl::sigmoid_attn_kernel<T, 8>); break;
+        case 4: go(&swl::sigmoid_attn_kernel<T, 4>); break;
+        case 2: go(&swl::sigmoid_attn_kernel<T, 2>); break;
+        default: go(&swl::sigmoid_attn_kernel<T, 1>); break;
+        }
+        if (key_splits > 1)
+            hipLaunchKernelGGL((swl::sigmoid_attn_sum_kernel<T>), dim3(static_cast<unsigned>((total + 1023) / 1024)), dim3(256), 0, st,
+                               static_cast<T *>(out), scratch, total, key_splits);
+    });
+    return swl::check_launch();
+}
 
 extern "C" int swl_sigmoid_attn(void *out, const void *q, const void *k_cache, const void *v_cache,
                                 const int32_t *block_table, const int32_t *tok_seq, const int32_t *tok_pos, const float *talk,
@@ -365,28 +415,9 @@ extern "C" int swl_sigmoid_attn(void *out, const void *q, const void *k_cache, c
                                 int32_t num_kv_heads, int32_t dim, int32_t vdim, int64_t q_tok_stride, int32_t window,
                                 float scale, int32_t max_blocks_per_seq, int64_t block_stride, int32_t dtype,
                                 swl_stream_t stream) {
-    if (num_tokens < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || dim <= 0 || vdim <= 0 || window < 0) return SWL_ERR_BAD_ARG;
-    if (num_q_heads % num_kv_heads || (r1 == nullptr) != (r2 == nullptr)) return SWL_ERR_BAD_ARG;
-    if (num_tokens == 0) return SWL_OK;
-    if (!out || !q || !k_cache || !v_cache || !block_table || !tok_seq || !tok_pos) return SWL_ERR_BAD_ARG;
-    // heads per workgroup: all of them when they are mixed, else as many as its accumulators and LDS hold
-    int hpg = num_q_heads;
-    if (!talk)
-        while (hpg > 1 && (static_cast<int64_t>(hpg) * vdim > swl::kSgMaxAcc * swl::kSgThreads ||
-                           swl::sg_lds_bytes(hpg, dim, 0) > 64 * 1024))
-            --hpg;
-    const size_t lds = swl::sg_lds_bytes(hpg, dim, talk != nullptr);
-    if (num_tokens > 0x7fffffffLL || static_cast<int64_t>(hpg) * vdim > swl::kSgMaxAcc * swl::kSgThreads || lds > 64 * 1024)
-        return SWL_ERR_UNSUPPORTED;
-    const unsigned groups = static_cast<unsigned>((num_q_heads + hpg - 1) / hpg);
-    SWL_DISPATCH_DTYPE3(dtype, T, {
-        hipLaunchKernelGGL((swl::sigmoid_attn_kernel<T>), dim3(static_cast<unsigned>(num_tokens), groups),
-                           dim3(swl::kSgThreads), lds, static_cast<hipStream_t>(stream), static_cast<T *>(out),
-                           static_cast<const T *>(q), static_cast<const T *>(k_cache), static_cast<const T *>(v_cache),
-                           block_table, tok_seq, tok_pos, talk, r1, r2, pb, hpg, num_kv_heads, dim, vdim, q_tok_stride, window,
-                           scale, max_blocks_per_seq, block_stride, num_q_heads);
-    });
-    return swl::check_launch();
+    return swl_sigmoid_attn_shares(out, q, k_cache, v_cache, block_table, tok_seq, tok_pos, talk, r1, r2, pb, num_tokens, num_q_heads,
+                                   num_kv_heads, dim, vdim, q_tok_stride, window, scale, max_blocks_per_seq, block_stride, 1, nullptr,
+                                   dtype, stream);
 }
 
 // (dim, vdim) pairs with a compiled matrix-core kernel

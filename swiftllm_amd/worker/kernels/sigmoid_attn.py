@@ -4,7 +4,7 @@ import torch
 
 from swiftllm_amd import _hip
 
-from .window_attn import PoolSlice, _split_scratch, choose_key_splits
+from .window_attn import PoolSlice, _split_scratch, choose_key_splits, token_key_splits
 
 
 def tiles_supported(mixer, dtype: torch.dtype) -> bool:
@@ -44,8 +44,9 @@ def sigmoid_attention(q: torch.Tensor, pool: torch.Tensor, pool_slice: PoolSlice
                   float(mixer.scale), block_table.shape[1], pool.shape[1], splits, _hip.ptr(scratch), n,
                   _hip.dtype_code(q.dtype), _hip.stream())
         return out
-    _hip.call("swl_sigmoid_attn", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq),
+    splits, scratch = token_key_splits(n, H, mixer.value_dim, mixer, max_positions, q.device)
+    _hip.call("swl_sigmoid_attn_shares", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq),
               _hip.ptr(tok_pos), _hip.ptr(talk), _hip.ptr(r1), _hip.ptr(r2), _hip.ptr(pb), n, H, mixer.num_kv_heads,
               mixer.head_dim, mixer.value_dim, q.stride(0), mixer.window, float(mixer.scale), block_table.shape[1],
-              pool.shape[1], _hip.dtype_code3(q.dtype), _hip.stream())
+              pool.shape[1], splits, _hip.ptr(scratch), _hip.dtype_code3(q.dtype), _hip.stream())
     return out

@@ -168,6 +168,13 @@ def choose_key_splits(num_tiles: int, mixer, max_positions: int, slots: int = _N
     return max(1, min(slots // max(num_tiles, 1), pages // 4, 16))
 
 
+def token_key_splits(n: int, heads: int, vdim: int, mixer, max_positions: int, device):
+    """Key shares of the per-token kernels (and their scratch): up to 16 while they leave at most four workgroups a CU — a chunk of 64
+    keys is a chain of some microseconds, and a step of few tokens has nothing else to fill the chip with."""
+    splits = choose_key_splits(n, mixer, max_positions, slots=4 * _NUM_CUS)
+    return splits, _split_scratch(device, splits * n * heads * (vdim + 2)) if splits > 1 else None
+
+
 def tiles_supported(mixer, dtype: torch.dtype) -> bool:
     if dtype not in (torch.float16, torch.bfloat16):
         return False
@@ -210,12 +217,13 @@ def window_attention(qkv: torch.Tensor, talk: torch.Tensor, pool: torch.Tensor, 
                   float(mixer.softcap), block_table.shape[1], pool.shape[1], splits, _hip.ptr(scratch), n,
                   _hip.dtype_code(qkv.dtype), _hip.stream())
         return out
-    _hip.call("swl_window_attn", _hip.ptr(out), _hip.ptr(qkv), pool.data_ptr() + pool_slice.k_offset * esize,
+    splits, scratch = token_key_splits(n, mixer.num_q_heads, mixer.value_dim, mixer, max_positions, qkv.device)
+    _hip.call("swl_masked_attn_shares", _hip.ptr(out), _hip.ptr(qkv), pool.data_ptr() + pool_slice.k_offset * esize,
               pool.data_ptr() + pool_slice.v_offset * esize, _hip.ptr(block_table), _hip.ptr(tok_seq), _hip.ptr(tok_pos),
               _hip.ptr(talk), _hip.ptr(rel), rel_len, n, mixer.num_q_heads, mixer.num_kv_heads, mixer.head_dim,
-              mixer.value_dim, qkv.stride(0),
-              mixer.window, float(mixer.scale), float(mixer.softcap), block_table.shape[1], pool.shape[1],
-              _hip.dtype_code3(qkv.dtype), _hip.stream())
+              mixer.value_dim, qkv.stride(0), mixer.window, float(mixer.scale), float(mixer.softcap), block_table.shape[1],
+              pool.shape[1], MASK_WINDOW, 0, mixer.num_kv_heads, 0, 0, mixer.value_dim, out.stride(0), 0, 0, splits,
+              _hip.ptr(scratch), _hip.dtype_code3(qkv.dtype), _hip.stream())
     return out
 
 
@@ -332,9 +340,10 @@ def masked_attention(q: torch.Tensor, pool: torch.Tensor, pool_slice: PoolSlice,
                   _hip.ptr(sink), spec.num_v_heads, 1 if spec.out_f32 else 0, hpg, _hip.ptr(spec.slopes), spec.out_dim,
                   out.stride(0), _hip.ptr(gate), gate_stride, _hip.dtype_code(q.dtype), _hip.stream())
         return out
-    _hip.call("swl_masked_attn", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq),
+    splits, scratch = token_key_splits(n, spec.num_q_heads, spec.value_dim, spec, max_positions, q.device)
+    _hip.call("swl_masked_attn_shares", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq),
               _hip.ptr(tok_pos), 0, 0, 0, n, spec.num_q_heads, spec.num_kv_heads, spec.head_dim, spec.value_dim, q.stride(0),
               spec.window, float(spec.scale), float(spec.softcap), block_table.shape[1], pool.shape[1], spec.mask_kind,
               _hip.ptr(sink), spec.num_v_heads, 1 if spec.out_f32 else 0, _hip.ptr(spec.slopes), spec.out_dim, out.stride(0),
-              _hip.ptr(gate), gate_stride, _hip.dtype_code3(q.dtype), _hip.stream())
+              _hip.ptr(gate), gate_stride, splits, _hip.ptr(scratch), _hip.dtype_code3(q.dtype), _hip.stream())
     return out

@@ -1,0 +1,107 @@
+"""The per-token attention and expert kernels (csrc/window_attn.hip, sigmoid_attn.hip, moe.hip) against float64: rows that are and are
+not whole 16-byte pieces, windows that begin inside a page, contexts at page and chunk borders, key shares with and without keys."""
+import pytest
+import torch
+
+from test_gpu_span_attn import _pool, _spans, _want
+
+pytestmark = pytest.mark.gpu
+
+PARTS = [(1, 0, 3), (2, 62, 4), (3, 300, 2), (4, 15, 1), (5, 128, 1)]
+
+
+def _bound(want, dtype):
+    """fp32: rounding of sums of some hundred terms of order one; 16 bits: the result's own rounding (the inputs are the same)."""
+    eps = {torch.float32: 2.0 ** -18, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    return 1.1 * eps * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,d,dv,window,kind", [(8, 2, 128, 128, 0, "rel"), (8, 1, 576, 512, 70, "sink"), (6, 2, 36, 33, 37, "slopes"),
+                                                  (5, 5, 10, 7, 0, "plain"), (16, 1, 64, 64, 48, "gate"), (40, 20, 24, 100, 0, "plain")])
+def test_softmax_attention(H, G, d, dv, window, kind, dtype):
+    from swiftllm_amd.worker.kernels import window_attn as wa
+    g = torch.Generator().manual_seed(d)
+    pool, sl, table, ks, vs = _pool([a + n for _, a, n in PARTS], G, G, d, dv, dtype, g)
+    seq, pos, _ = _spans(PARTS)
+    n = seq.shape[0]
+    q = torch.randn(n, H * d, generator=g).to(dtype)
+    rel = torch.randn(H, 90, generator=g) if kind == "rel" else None
+    gate = torch.randn(n, H * dv, generator=g).to(dtype) if kind == "gate" else None
+    spec = wa.AttentionSpec(H, G, d, dv, d ** -0.5, window=window, sink=torch.randn(H, generator=g).cuda() if kind == "sink" else None,
+                            slopes=(torch.rand(H, generator=g) * 0.1).cuda() if kind == "slopes" else None)
+    for reach in (4096, 64):        # (sixteen key shares; one)
+        if kind == "rel":
+            mixer = type("Mixer", (), dict(num_q_heads=H, num_kv_heads=G, head_dim=d, value_dim=dv, window=0, scale=d ** -0.5, softcap=0.0))
+            o = wa.window_attention(q.cuda(), None, pool, sl, table, seq, pos, mixer, None, reach, rel=rel.cuda())
+        else:
+            o = wa.masked_attention(q.cuda(), pool, sl, table, seq, pos, spec, None, reach, gate=gate.cuda() if gate is not None else None)
+        at = 0
+        for b, (_, a, m) in enumerate(PARTS):
+            want = _want(q[at:at + m].double().view(m, H, d), ks[b], vs[b], a, spec, rel.double() if rel is not None else None,
+                         gate[at:at + m].double() if gate is not None else None)
+            assert (o[at:at + m].double().cpu() - want).abs().max() <= _bound(want, dtype), (reach, b)
+            at += m
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("H,G,d,dv,window,mixed", [(8, 2, 128, 128, 0, True), (6, 3, 18, 5, 37, True), (40, 20, 24, 100, 0, False)])
+def test_sigmoid_attention(H, G, d, dv, window, mixed, dtype):
+    from swiftllm_amd.worker.kernels.sigmoid_attn import sigmoid_attention
+    g = torch.Generator().manual_seed(d)
+    pool, sl, table, ks, vs = _pool([a + n for _, a, n in PARTS], G, G, d, dv, dtype, g)
+    seq, pos, _ = _spans(PARTS)
+    n = seq.shape[0]
+    q = torch.randn(n, H * d, generator=g).to(dtype)
+    talk = torch.eye(H) + 0.2 * torch.randn(H, H, generator=g)
+    r1, r2, pb = torch.rand(H, generator=g), torch.rand(H, generator=g), torch.randn(H, generator=g) - 2
+    mixer = type("Mixer", (), dict(num_q_heads=H, num_kv_heads=G, head_dim=d, value_dim=dv, window=window, scale=d ** -0.5))
+    for reach in (4096, 64):
+        o = sigmoid_attention(q.cuda(), pool, sl, table, seq, pos, mixer, talk.cuda() if mixed else None, r1.cuda(), r2.cuda(), pb.cuda(),
+                              None, reach)
+        at = 0
+        for b, (_, a, m) in enumerate(PARTS):
+            i, j = torch.arange(a, a + m)[:, None], torch.arange(a + m)[None]
+            see = (j <= i) & ((i - j < window) if window else torch.ones(m, a + m, dtype=torch.bool))
+            w = []
+            for h in range(H):
+                s = q[at:at + m, h * d:(h + 1) * d].double() @ ks[b][:, h // (H // G)].T * d ** -0.5
+                s = s - float(r1[h]) * torch.log1p(float(r2[h]) * (i - j).clamp(min=0)) + float(pb[h])
+                w.append(torch.sigmoid(s) * see)
+            w = torch.stack(w)
+            w = torch.einsum("hg,gij->hij", talk.double(), w) if mixed else w
+            want = torch.stack([w[h] @ vs[b][:, h // (H // G)] for h in range(H)], 1).reshape(m, -1)
+            # (nothing is normalised: errors of the weights add up over the keys)
+            size = float((w.abs().sum(-1)).max()) * 4
+            eps = 2.0 ** -20 if dtype == torch.float32 else 2.0 ** -20 + 2.0 ** -11 / size * max(1.0, float(want.abs().max()))
+            assert (o[at:at + m].double().cpu() - want).abs().max() <= 1.1 * eps * size, (reach, b)
+            at += m
+
+
+@pytest.mark.parametrize("width,ff,top", [(64, 48, 2), (37, 18, 3), (1024, 20, 2), (130, 257, 1)])
+@pytest.mark.parametrize("form", ["relu2", "silu", "clamped_in"])
+def test_experts_by_assignment(width, ff, top, form):
+    from swiftllm_amd.worker.kernels import moe
+    g = torch.Generator().manual_seed(width)
+    n, experts = 5, 6
+    h = torch.randn(n, width, generator=g)
+    up = torch.randn(experts, ff * (1 if form == "relu2" else 2), width, generator=g) / width ** 0.5
+    down = torch.randn(experts, width, ff, generator=g) / ff ** 0.5
+    idx = torch.stack([torch.randperm(experts, generator=g)[:top] for _ in range(n)])
+    wts = torch.rand(n, top, generator=g) + 0.1
+    args = (h.cuda(), idx.to(torch.int32).cuda(), wts.cuda(), up.cuda(), down.cuda())
+    if form == "relu2":
+        got = moe.moe_experts_relu2(*args)
+    else:
+        got = moe.moe_experts(*args, 1.5, moe.ACT_SILU if form == "silu" else moe.ACT_CLAMPED, weigh_inputs=form == "clamped_in")
+    want = torch.zeros(n, width, dtype=torch.float64)
+    for j in range(top):
+        z = torch.einsum("tk,tfk->tf", h.double() * (wts[:, j:j + 1] if form == "clamped_in" else 1.0), up.double()[idx[:, j]])
+        if form == "relu2":
+            y = torch.relu(z) ** 2
+        else:
+            a, u = z[:, :ff], z[:, ff:]
+            y = a * torch.sigmoid(a) * u if form == "silu" else a.clamp(max=1.5) * torch.sigmoid(1.702 * a.clamp(max=1.5)) * (u.clamp(-1.5, 1.5) + 1)
+        want += (1.0 if form == "clamped_in" else wts[:, j:j + 1].double()) * torch.einsum("tf,twf->tw", y, down.double()[idx[:, j]])
+    # two fp32 sums of up to 1024 terms of order one, one behind the other
+    assert (got.double().cpu() - want).abs().max() <= 2.0 ** -17 * max(1.0, float(want.abs().max()))
