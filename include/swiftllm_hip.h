@@ -610,6 +610,24 @@ int swl_span_attn(void *out, const void *q, const void *k_cache, const void *v_c
                   int32_t key_splits, float *scratch, int64_t num_tokens, const float *sink, int32_t out_f32, const float *slopes,
                   int32_t out_dim, int64_t out_stride, const void *gate, int64_t gate_stride, int32_t dtype, swl_stream_t stream);
 
+/* swl_window_attn_tiles / swl_sigmoid_attn_tiles with a mixing matrix (csrc/mix_attn.hip) for steps that bring prompt portions: at most
+ * 16 query heads; the same tiles, masks and scratch ([splits][tokens][heads] x (vdim + 2) floats, sigmoid: x vdim). q, k_cache and
+ * v_cache 16-byte aligned, out 8-byte aligned, q_tok_stride and block_stride multiples of 8. r1 / r2 both or neither; pb may be NULL. Ask
+ * swl_mix_attn_supported. */
+int swl_mix_attn_supported(int32_t num_q_heads, int32_t num_kv_heads, int32_t dim, int32_t vdim, int32_t dtype);
+int swl_mix_attn(void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
+                 const int32_t *tok_seq, const int32_t *tok_pos, const int32_t *tile_row0, const int32_t *tile_cnt,
+                 const float *talk, int32_t num_tiles, int32_t num_q_heads, int32_t num_kv_heads, int32_t dim, int32_t vdim,
+                 int64_t q_tok_stride, int32_t window, float scale, float softcap, int32_t max_blocks_per_seq,
+                 int64_t block_stride, int32_t key_splits, float *scratch, int64_t num_tokens, int32_t dtype,
+                 swl_stream_t stream);
+int swl_mix_sigmoid_attn(void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
+                         const int32_t *tok_seq, const int32_t *tok_pos, const int32_t *tile_row0, const int32_t *tile_cnt,
+                         const float *talk, const float *r1, const float *r2, const float *pb, int32_t num_tiles,
+                         int32_t num_q_heads, int32_t num_kv_heads, int32_t dim, int32_t vdim, int64_t q_tok_stride,
+                         int32_t window, float scale, int32_t max_blocks_per_seq, int64_t block_stride, int32_t key_splits,
+                         float *scratch, int64_t num_tokens, int32_t dtype, swl_stream_t stream);
+
 /* ---- rotary positions on interleaved pairs fused with the paged KV store; gated / combined heads ---------------------------
  * Rotation: dimension 2i of a head is paired with 2i + 1, i < rot_dims / 2; (u, v) at position p becomes
  * (u cos a - v sin a, v cos a + u sin a), a = p * freq[i] (freq: float64 [rot_dims / 2] on the device; angles are evaluated

@@ -113,6 +113,10 @@ SIGNATURES = {
                               _I32, _P],
     "swl_span_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _I32,
                       _F32, _F32, _I32, _I64, _I32, _P, _I64, _P, _I32, _P, _I32, _I64, _P, _I64, _I32, _P],
+    "swl_mix_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _F32, _F32, _I32, _I64, _I32,
+                     _P, _I64, _I32, _P],
+    "swl_mix_sigmoid_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _F32, _I32,
+                             _I64, _I32, _P, _I64, _I32, _P],
     "swl_rope_store_kv": [_P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _I64, _I32, _P],
     "swl_latent_rope_store_kv": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I64, _I64, _I64, _I32,
                                  _I64, _F32, _I32, _F64, _I32, _I32, _I32, _P],
@@ -192,6 +196,7 @@ _SPECIAL = {
     "swl_masked_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_moe_gemm_supported": ([_I64, _I32, _I32, _I32], _I32),
     "swl_span_attn_supported": ([_I32, _I32, _I32, _I32, _I32, _I32, _I32], _I32),
+    "swl_mix_attn_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_sigmoid_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_decode_engine_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_decode_engine_slots_per_layer": ([_I32, _I32, _I32, _I32], _I32),

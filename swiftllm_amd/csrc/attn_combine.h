@@ -1,5 +1,5 @@
-// attn_combine.h — the second launch of attention over key shares: what window_attn_mfma.hip and span_attn.hip leave per share
-// (unnormalised fp32 result, running maximum in base-2 exponent units, sum) becomes one row per (token, head).
+// attn_combine.h — the second launch of attention over key shares: what a share leaves (unnormalised fp32 result, running maximum in
+// base-2 exponent units, sum) becomes one row per (token, head); plain sums of sigmoid attention are added up.
 #pragma once
 
 #include "swl_common.h"
@@ -45,6 +45,28 @@ __global__ __launch_bounds__(256) void window_attn_combine_kernel(T *out, const 
         if (out_f32) reinterpret_cast<float *>(out)[tok * out_stride + hc0 + c] = a;
         else out[tok * out_stride + hc0 + c] = to_t<T>(a);
     }
+}
+
+// out[i] = sum over the key shares s of part[s][i]
+template <typename T>
+__global__ __launch_bounds__(256) void sigmoid_attn_sum_kernel(T *out, const float *part, int64_t total, int nsplit) {
+    const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+    if (i >= total) return;
+    if (total & 3) {        // (uniform) odd rows: element by element
+        for (int64_t k = i; k < min(i + 4, total); ++k) {
+            float a = part[k];
+            for (int s = 1; s < nsplit; ++s) a += part[s * total + k];
+            out[k] = to_t<T>(a);
+        }
+        return;
+    }
+    float4_t a = *reinterpret_cast<const float4_t *>(part + i);
+    for (int s = 1; s < nsplit; ++s) a += *reinterpret_cast<const float4_t *>(part + s * total + i);
+    typedef T vec4 __attribute__((ext_vector_type(4)));
+    vec4 w;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w[r] = to_t<T>(a[r]);
+    *reinterpret_cast<vec4 *>(out + i) = w;
 }
 
 } // namespace swl

@@ -48,6 +48,7 @@ SOURCES = [
     "low_rank_decay.hip",
     "span_attn.hip",
     "moe_grouped.hip",
+    "mix_attn.hip",
 ]
 # What a model family's worker calls (the shared pieces included): `build(only=MODEL_SOURCES[...])` compiles just these, so
 # that the first use from a fresh checkout does not pay for kernels the model never launches. A later full build compiles
@@ -56,13 +57,13 @@ _SHARED = ["swap_blocks.hip", "block_table.hip", "argmax.hip", "gemm_skinny.hip"
 MODEL_SOURCES = {
     "llama": list(SOURCES[:14]),
     "Kekapel": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip",
-                          "polynorm.hip", "moe.hip", "moe_grouped.hip"],
+                          "mix_attn.hip", "polynorm.hip", "moe.hip", "moe_grouped.hip"],
     "Lorulix": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip",
                           "rms_stream.hip", "delta_rule.hip"],
     "Rosilix": _SHARED + ["layernorm.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rms_stream.hip",
                           "rope_kv.hip"],
     "Ratilorn": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip",
-                           "rms_stream.hip", "sigmoid_attn.hip", "ssd.hip", "linear_scan.hip", "delta_rule.hip"],
+                           "rms_stream.hip", "sigmoid_attn.hip", "mix_attn.hip", "ssd.hip", "linear_scan.hip", "delta_rule.hip"],
     "Rokevik": _SHARED + ["window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rope_kv.hip", "hyper_stream.hip", "min_gru.hip"],
     "Vafozen": _SHARED + ["layernorm.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rms_stream.hip", "rope_kv.hip",
                           "hyper_stream.hip", "delta_rule.hip", "ssd.hip", "linear_scan.hip", "low_rank_decay.hip"],

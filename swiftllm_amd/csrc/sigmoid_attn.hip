@@ -15,6 +15,7 @@
 //                            against 16-key pages (see below).
 // Without a running maximum or denominator the sum over keys is a plain sum: key shares of one query (a split over
 // workgroups) are added up, no rescaling.
+#include "attn_combine.h"
 #include "swl_common.h"
 #include "token_attn.h"
 
@@ -297,28 +298,6 @@ __global__ __launch_bounds__(NW * 64) void sigmoid_attn_mfma_kernel(
             }
         }
     }
-}
-
-// out[i] = sum over the key shares s of part[s][i]
-template <typename T>
-__global__ __launch_bounds__(256) void sigmoid_attn_sum_kernel(T *out, const float *part, int64_t total, int nsplit) {
-    const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
-    if (i >= total) return;
-    if (total & 3) {        // (uniform) odd rows: element by element
-        for (int64_t k = i; k < min(i + 4, total); ++k) {
-            float a = part[k];
-            for (int s = 1; s < nsplit; ++s) a += part[s * total + k];
-            out[k] = to_t<T>(a);
-        }
-        return;
-    }
-    float4_t a = *reinterpret_cast<const float4_t *>(part + i);
-    for (int s = 1; s < nsplit; ++s) a += *reinterpret_cast<const float4_t *>(part + s * total + i);
-    typedef T vec4 __attribute__((ext_vector_type(4)));
-    vec4 w;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) w[r] = to_t<T>(a[r]);
-    *reinterpret_cast<vec4 *>(out + i) = w;
 }
 
 template <typename T, int D, int DV>

@@ -17,7 +17,7 @@ from swiftllm_amd.model_config import KekapelModelConfig
 from .kekapel_weight import load_kekapel_weights
 from .kernels.layernorm import add_layernorm, embed_positions, layernorm
 from .kernels.linear import pack_weight, packable
-from .kernels.window_attn import PoolSlice
+from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import KekapelAttention, KekapelFeedForward, _project
 from .stepped_model import SteppedModel
 
@@ -96,7 +96,7 @@ class KekapelModel(SteppedModel):
         for i, s in enumerate(subs):
             if s.kind == "mixer":
                 y = s.op.forward(h, pool, self.pool_slices[s.run] if use_pool else None, block_table, dev["tok_seq"],
-                                 dev["tok_pos"], (dev["tile_row0"], dev["tile_cnt"]))
+                                 dev["tok_pos"], StepTiles.of(dev))
             else:
                 y = s.op.forward(h)
             nxt = subs[i + 1] if i + 1 < len(subs) else None

@@ -4,7 +4,7 @@ import torch
 
 from swiftllm_amd import _hip
 
-from .window_attn import PoolSlice, _split_scratch, choose_key_splits, token_key_splits
+from .window_attn import PoolSlice, _split_scratch, choose_key_splits, mix_launch, token_key_splits
 
 
 def tiles_supported(mixer, dtype: torch.dtype) -> bool:
@@ -34,6 +34,9 @@ def sigmoid_attention(q: torch.Tensor, pool: torch.Tensor, pool_slice: PoolSlice
     kp = pool.data_ptr() + pool_slice.k_offset * esize
     vp = pool.data_ptr() + pool_slice.v_offset * esize
     wide_ok = q.stride(0) % 4 == 0 and q.data_ptr() % 8 == 0 and kp % 8 == 0 and vp % 8 == 0 and pool.shape[1] % 4 == 0
+    if talk is not None and mix_launch("swl_mix_sigmoid_attn", q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles, mixer,
+                                       (talk, r1, r2, pb), (), mixer.value_dim):
+        return out
     if tiles is not None and wide_ok and tiles_supported(mixer, q.dtype):
         row0, cnt = tiles
         splits = choose_key_splits(row0.shape[0], mixer, max_positions)

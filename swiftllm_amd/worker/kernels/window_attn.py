@@ -175,6 +175,29 @@ def token_key_splits(n: int, heads: int, vdim: int, mixer, max_positions: int, d
     return splits, _split_scratch(device, splits * n * heads * (vdim + 2)) if splits > 1 else None
 
 
+def mix_launch(entry, q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles, mixer, vectors, extra, floats) -> bool:
+    """The prompt form of attention with mixed heads (csrc/mix_attn.hip) where it serves the step; False: nothing was launched.
+    vectors: the fp32 arguments of `entry`, extra: its constants after the scale, floats: fp32 a share leaves per (token, head)."""
+    spans = getattr(tiles, "spans", None)
+    n, H = q.shape[0], mixer.num_q_heads
+    if spans is None or n < SPAN_MIN_TOKENS * spans[0].shape[0] or q.dtype == torch.float32:
+        return False
+    if not _hip.load().swl_mix_attn_supported(H, mixer.num_kv_heads, mixer.head_dim, mixer.value_dim, _hip.dtype_code(q.dtype)):
+        return False
+    if (q.data_ptr() | kp | vp) % 16 or q.stride(0) % 8 or pool.shape[1] % 8:      # 16-byte operand loads
+        return False
+    row0, cnt = tiles
+    # the registers allow one workgroup a CU: with fewer tiles than CUs, every tile's keys are shared out (at 2 and 4 workgroups a CU a
+    # step of 1.4 thousand tokens at 16 heads of 128 gets no faster and 9 % slower: each has its own prologue and partial results)
+    splits = choose_key_splits(row0.shape[0], mixer, tiles.longest)
+    scratch = _split_scratch(q.device, splits * n * H * floats) if splits > 1 else None
+    _hip.call(entry, _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq), _hip.ptr(tok_pos),
+              _hip.ptr(row0), _hip.ptr(cnt), *[_hip.ptr(t) for t in vectors], row0.shape[0], H, mixer.num_kv_heads, mixer.head_dim,
+              mixer.value_dim, q.stride(0), mixer.window, float(mixer.scale), *extra, block_table.shape[1], pool.shape[1], splits,
+              _hip.ptr(scratch), n, _hip.dtype_code(q.dtype), _hip.stream())
+    return True
+
+
 def tiles_supported(mixer, dtype: torch.dtype) -> bool:
     if dtype not in (torch.float16, torch.bfloat16):
         return False
@@ -202,6 +225,10 @@ def window_attention(qkv: torch.Tensor, talk: torch.Tensor, pool: torch.Tensor, 
                                      pool.data_ptr() + pool_slice.v_offset * esize, pool, block_table, tok_seq, tok_pos, tiles,
                                      mixer.num_q_heads, mixer.num_kv_heads, mixer.num_kv_heads, mixer.head_dim, mixer.value_dim,
                                      mixer.window, MASK_WINDOW, mixer.scale, mixer.softcap, rel=rel):
+        return out
+    if talk is not None and rel is None and mix_launch(
+            "swl_mix_attn", qkv, out, pool.data_ptr() + pool_slice.k_offset * esize, pool.data_ptr() + pool_slice.v_offset * esize,
+            pool, block_table, tok_seq, tok_pos, tiles, mixer, (talk,), (float(mixer.softcap),), mixer.value_dim + 2):
         return out
     if tiles is not None and n >= TILES_MIN_TOKENS and tiles_supported(mixer, qkv.dtype):
         row0, cnt = tiles
