@@ -767,6 +767,16 @@ int swl_delta_rule(float *o, const float *qn, const float *kn, const float *kq, 
                    float *state, int64_t slot_stride, int64_t s_off, const int32_t *seq_row0, const int32_t *seq_cnt,
                    const int32_t *tok_pos, const int32_t *tok_state, int32_t num_seqs, int32_t num_heads,
                    int32_t num_qk_heads, int32_t dim, int32_t vdim, swl_stream_t stream);
+/* swl_delta_rule by tiles (csrc/delta_chunks.hip) for steps that bring prompt portions: the portions also come cut into runs of 16 tokens
+ * (tile_row0 / tile_cnt in order; every tile of a portion but its last holds 16; seq_tile0: first tile of a portion). scratch:
+ * swl_delta_rule_tiles_floats floats; qn, kn and scratch 16-byte aligned. Ask swl_delta_rule_tiles_supported. */
+int swl_delta_rule_tiles_supported(int32_t num_heads, int32_t num_qk_heads, int32_t dim, int32_t vdim);
+int64_t swl_delta_rule_tiles_floats(int64_t num_tiles, int32_t num_heads, int32_t dim, int32_t vdim);
+int swl_delta_rule_tiles(float *o, const float *qn, const float *kn, const float *vv, const float *beta, const float *decay, float *state,
+                         int64_t slot_stride, int64_t s_off, const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0,
+                         const int32_t *tile_row0, const int32_t *tile_cnt, const int32_t *tok_pos, const int32_t *tok_state,
+                         int32_t num_seqs, int32_t num_tiles, int32_t num_heads, int32_t num_qk_heads, int32_t dim, int32_t vdim,
+                         float *scratch, swl_stream_t stream);
 int swl_gated_head_rmsnorm(void *out, int64_t out_stride, const float *o, const void *gate, int64_t gate_stride, const float *w,
                            int32_t w_head_stride, float mult, float eps, int64_t num_tokens, int32_t num_heads, int32_t vdim,
                            int32_t dtype, swl_stream_t stream);

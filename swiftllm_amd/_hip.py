@@ -141,6 +141,7 @@ SIGNATURES = {
     "swl_delta_prep": [_P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _I64, _I32, _I32, _I32,
                        _I32, _I32, _I32, _P],
     "swl_delta_rule": [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _P],
+    "swl_delta_rule_tiles": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _P, _P],
     "swl_gated_head_rmsnorm": [_P, _I64, _P, _P, _I64, _P, _I32, _F32, _F32, _I64, _I32, _I32, _I32, _P],
     "swl_moe_route_grouped": [_P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _P],
     "swl_qkv_bias_norm_store": [_P, _P, _P, _P, _P, _P, _P, _I64, _F32, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32,
@@ -196,6 +197,8 @@ _SPECIAL = {
     "swl_masked_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_moe_gemm_supported": ([_I64, _I32, _I32, _I32], _I32),
     "swl_span_attn_supported": ([_I32, _I32, _I32, _I32, _I32, _I32, _I32], _I32),
+    "swl_delta_rule_tiles_supported": ([_I32, _I32, _I32, _I32], _I32),
+    "swl_delta_rule_tiles_floats": ([_I64, _I32, _I32, _I32], _I64),
     "swl_mix_attn_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_sigmoid_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_decode_engine_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),

@@ -49,6 +49,7 @@ SOURCES = [
     "span_attn.hip",
     "moe_grouped.hip",
     "mix_attn.hip",
+    "delta_chunks.hip",
 ]
 # What a model family's worker calls (the shared pieces included): `build(only=MODEL_SOURCES[...])` compiles just these, so
 # that the first use from a fresh checkout does not pay for kernels the model never launches. A later full build compiles
@@ -59,7 +60,7 @@ MODEL_SOURCES = {
     "Kekapel": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip",
                           "mix_attn.hip", "polynorm.hip", "moe.hip", "moe_grouped.hip"],
     "Lorulix": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip",
-                          "rms_stream.hip", "delta_rule.hip"],
+                          "rms_stream.hip", "delta_rule.hip", "delta_chunks.hip"],
     "Rosilix": _SHARED + ["layernorm.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rms_stream.hip",
                           "rope_kv.hip"],
     "Ratilorn": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip",

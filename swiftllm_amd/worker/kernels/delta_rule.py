@@ -6,6 +6,15 @@ from swiftllm_amd import _hip
 from .rms_stream import StateRef
 
 
+# A step whose longest portion holds this many tokens walks by tiles. Walked token by token a portion costs 10 us and 0.3 to 0.37 us a token;
+# by tiles (heads of 128, 8 heads, the step's launches together): 1 portion of 24 / 64 / 1000 tokens 13 / 16 / 70 us against 16 / 29 / 390;
+# 16 of 32 / 64: 27 / 35 against 25 / 40; 30 decoded tokens beside one of 32 / 64 / 200: 31 / 32 / 36 against 33 / 44 / 88. Shorter portions
+# leave the tiles mostly empty: 64 of 8 tokens 60 us against 29.
+TILES_MIN_PORTION = 48
+# Steps that would need more scratch than this (1.6 KiB a token and head of 128) walk token by token.
+TILES_MAX_SCRATCH_FLOATS = 1 << 28
+
+
 def delta_rule_mixer(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
                      norm_w: torch.Tensor, st: StateRef, tail_off: int, state_off: int, mixer, eps: float) -> torch.Tensor:
     """proj [T, q | k | v | gate | b | a] (one fused projection) -> [T, heads * vdim] in proj's dtype: short convolutions
@@ -32,13 +41,30 @@ def delta_rule_mixer(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tens
               int(tail_off), _hip.ptr(st.tok_pos), _hip.ptr(st.tok_start), _hip.ptr(st.tok_state), _hip.ptr(st.tok_seq), n,
               H, G, d, dv, mixer.conv_taps, code, stream)
     o = torch.empty((n, H * dv), dtype=f32, device=dev)
-    _hip.call("swl_delta_rule", _hip.ptr(o), _hip.ptr(qn), _hip.ptr(kn), _hip.ptr(kq), _hip.ptr(vv), _hip.ptr(beta), _hip.ptr(decay),
-              _hip.ptr(st.pool), st.pool.stride(0), int(state_off), _hip.ptr(st.seq_row0), _hip.ptr(st.seq_cnt),
-              _hip.ptr(st.tok_pos), _hip.ptr(st.tok_state), st.seq_row0.shape[0], H, G, d, dv, stream)
+    delta_rule_scan(o, qn, kn, kq, vv, beta, decay, st, state_off, H, G, d, dv)
     out = torch.empty((n, H * dv), dtype=proj.dtype, device=dev)
     gate = proj[:, mixer.conv_channels:mixer.conv_channels + H * dv]
     gated_head_rmsnorm(out, o, gate, norm_w, H, dv, eps)
     return out
+
+
+def delta_rule_scan(o, qn, kn, kq, vv, beta, decay, st: StateRef, state_off: int, H: int, G: int, d: int, dv: int):
+    """o [T, H * dv] and the states from what the prep left (all fp32)."""
+    num_seqs = st.seq_row0.shape[0]
+    floats = 0
+    if st.tiles is not None and st.longest >= TILES_MIN_PORTION and _hip.load().swl_delta_rule_tiles_supported(H, G, d, dv):
+        floats = _hip.load().swl_delta_rule_tiles_floats(st.tiles[0].shape[0], H, d, dv)
+    if 0 < floats <= TILES_MAX_SCRATCH_FLOATS:
+        row0, cnt, seq_tile0 = st.tiles
+        scratch = torch.empty(floats, dtype=torch.float32, device=o.device)
+        _hip.call("swl_delta_rule_tiles", _hip.ptr(o), _hip.ptr(qn), _hip.ptr(kn), _hip.ptr(vv), _hip.ptr(beta), _hip.ptr(decay),
+                  _hip.ptr(st.pool), st.pool.stride(0), int(state_off), _hip.ptr(st.seq_row0), _hip.ptr(st.seq_cnt),
+                  _hip.ptr(seq_tile0), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(st.tok_pos), _hip.ptr(st.tok_state), num_seqs,
+                  row0.shape[0], H, G, d, dv, _hip.ptr(scratch), _hip.stream())
+        return
+    _hip.call("swl_delta_rule", _hip.ptr(o), _hip.ptr(qn), _hip.ptr(kn), _hip.ptr(kq), _hip.ptr(vv), _hip.ptr(beta), _hip.ptr(decay),
+              _hip.ptr(st.pool), st.pool.stride(0), int(state_off), _hip.ptr(st.seq_row0), _hip.ptr(st.seq_cnt),
+              _hip.ptr(st.tok_pos), _hip.ptr(st.tok_state), num_seqs, H, G, d, dv, _hip.stream())
 
 
 def gated_head_rmsnorm(out: torch.Tensor, o: torch.Tensor, gate: torch.Tensor, norm_w: torch.Tensor, num_heads: int, vdim: int,
