@@ -769,9 +769,9 @@ int swl_delta_rule(float *o, const float *qn, const float *kn, const float *kq, 
                    int32_t num_qk_heads, int32_t dim, int32_t vdim, swl_stream_t stream);
 /* swl_delta_rule by tiles (csrc/delta_chunks.hip) for steps that bring prompt portions: the portions also come cut into runs of 16 tokens
  * (tile_row0 / tile_cnt in order; every tile of a portion but its last holds 16; seq_tile0: first tile of a portion). scratch:
- * swl_delta_rule_tiles_floats floats; qn, kn and scratch 16-byte aligned. Ask swl_delta_rule_tiles_supported. */
+ * swl_delta_rule_tiles_scratch_bytes; qn, kn and scratch 16-byte aligned. Ask swl_delta_rule_tiles_supported. */
 int swl_delta_rule_tiles_supported(int32_t num_heads, int32_t num_qk_heads, int32_t dim, int32_t vdim);
-int64_t swl_delta_rule_tiles_floats(int64_t num_tiles, int32_t num_heads, int32_t dim, int32_t vdim);
+size_t swl_delta_rule_tiles_scratch_bytes(int64_t num_tiles, int32_t num_heads, int32_t dim, int32_t vdim);
 int swl_delta_rule_tiles(float *o, const float *qn, const float *kn, const float *vv, const float *beta, const float *decay, float *state,
                          int64_t slot_stride, int64_t s_off, const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0,
                          const int32_t *tile_row0, const int32_t *tile_cnt, const int32_t *tok_pos, const int32_t *tok_state,

@@ -198,7 +198,7 @@ _SPECIAL = {
     "swl_moe_gemm_supported": ([_I64, _I32, _I32, _I32], _I32),
     "swl_span_attn_supported": ([_I32, _I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_delta_rule_tiles_supported": ([_I32, _I32, _I32, _I32], _I32),
-    "swl_delta_rule_tiles_floats": ([_I64, _I32, _I32, _I32], _I64),
+    "swl_delta_rule_tiles_scratch_bytes": ([_I64, _I32, _I32, _I32], ctypes.c_size_t),
     "swl_mix_attn_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_sigmoid_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_decode_engine_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),

@@ -357,8 +357,8 @@ extern "C" int swl_delta_rule_tiles_supported(int32_t num_heads, int32_t num_qk_
            vdim % 16 == 0 && vdim <= 1024;
 }
 
-extern "C" int64_t swl_delta_rule_tiles_floats(int64_t num_tiles, int32_t num_heads, int32_t dim, int32_t vdim) {
-    return num_tiles * num_heads * swl::dc_floats(dim, vdim);
+extern "C" size_t swl_delta_rule_tiles_scratch_bytes(int64_t num_tiles, int32_t num_heads, int32_t dim, int32_t vdim) {
+    return sizeof(float) * static_cast<size_t>(num_tiles * num_heads * swl::dc_floats(dim, vdim));
 }
 
 extern "C" int swl_delta_rule_tiles(float *o, const float *qn, const float *kn, const float *vv, const float *beta, const float *decay,

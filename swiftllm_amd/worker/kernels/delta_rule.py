@@ -12,7 +12,7 @@ from .rms_stream import StateRef
 # leave the tiles mostly empty: 64 of 8 tokens 60 us against 29.
 TILES_MIN_PORTION = 48
 # Steps that would need more scratch than this (1.6 KiB a token and head of 128) walk token by token.
-TILES_MAX_SCRATCH_FLOATS = 1 << 28
+TILES_MAX_SCRATCH = 1 << 30
 
 
 def delta_rule_mixer(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
@@ -51,12 +51,12 @@ def delta_rule_mixer(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tens
 def delta_rule_scan(o, qn, kn, kq, vv, beta, decay, st: StateRef, state_off: int, H: int, G: int, d: int, dv: int):
     """o [T, H * dv] and the states from what the prep left (all fp32)."""
     num_seqs = st.seq_row0.shape[0]
-    floats = 0
+    scratch_bytes = 0
     if st.tiles is not None and st.longest >= TILES_MIN_PORTION and _hip.load().swl_delta_rule_tiles_supported(H, G, d, dv):
-        floats = _hip.load().swl_delta_rule_tiles_floats(st.tiles[0].shape[0], H, d, dv)
-    if 0 < floats <= TILES_MAX_SCRATCH_FLOATS:
+        scratch_bytes = _hip.load().swl_delta_rule_tiles_scratch_bytes(st.tiles[0].shape[0], H, d, dv)
+    if 0 < scratch_bytes <= TILES_MAX_SCRATCH:
         row0, cnt, seq_tile0 = st.tiles
-        scratch = torch.empty(floats, dtype=torch.float32, device=o.device)
+        scratch = torch.empty(scratch_bytes // 4, dtype=torch.float32, device=o.device)
         _hip.call("swl_delta_rule_tiles", _hip.ptr(o), _hip.ptr(qn), _hip.ptr(kn), _hip.ptr(vv), _hip.ptr(beta), _hip.ptr(decay),
                   _hip.ptr(st.pool), st.pool.stride(0), int(state_off), _hip.ptr(st.seq_row0), _hip.ptr(st.seq_cnt),
                   _hip.ptr(seq_tile0), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(st.tok_pos), _hip.ptr(st.tok_state), num_seqs,
