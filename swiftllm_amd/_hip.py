@@ -174,6 +174,8 @@ SIGNATURES = {
                           _I32, _P],
     "swl_linear_scan": [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _I64, _I64, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32,
                         _I32, _P],
+    "swl_linear_scan_segments": [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _I64, _I64,
+                                 _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _P, _I32, _P],
     "swl_linear_step": [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _I64, _I32, _P, _P, _F32, _P, _P, _I64, _I64,
                         _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _P, _I32, _P, _I64, _F32, _F32, _I32, _P],
     "swl_low_rank_decay": [_P, _P, _I64, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _F32, _I32, _P],
@@ -199,6 +201,7 @@ _SPECIAL = {
     "swl_span_attn_supported": ([_I32, _I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_delta_rule_tiles_supported": ([_I32, _I32, _I32, _I32], _I32),
     "swl_delta_rule_tiles_scratch_bytes": ([_I64, _I32, _I32, _I32], ctypes.c_size_t),
+    "swl_linear_scan_scratch_bytes": ([_I64, _I32, _I32, _I32, _I32], ctypes.c_size_t),
     "swl_mix_attn_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_sigmoid_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_decode_engine_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),

@@ -22,6 +22,11 @@
 //                      the portion as the fastest grid index the two prompts beside 30 decoded tokens met on 16 CUs of two XCDs.
 //                      2 x 1000 + 30 tokens, 8 heads of 128 x 128: 360 -> 85 us. 32 columns a workgroup (half the operand reads)
 //                      took 136 us there and 106 instead of 99 us at 11 x 333 tokens, 16 heads.
+//                      A step of few portions leaves the chip idle behind a chain of 1.3 us a tile. Its portions are cut into segments of
+//                      several tiles: linear_segments_kernel walks every segment's state alone (from zero; the first from the portion's),
+//                      without queries or outputs, and the scan's workgroup of a segment starts from those states, each taken on by
+//                      the decays of the segments after it. 1 x 2000 tokens, 8 heads of 128 x
+//                      128: 169 -> 45 us; 2 x 1000 + 30: 81 -> 52 us (both launches).
 //   swl_linear_step:   steps whose portions are single tokens (decode): one workgroup per (sequence, head) streams the state once
 //                      and finishes the head — read-out, RMS norm over the head, weight, gate — in the same launch.
 // Everything after the loads of q, k, v is fp32.
@@ -141,26 +146,48 @@ __global__ __launch_bounds__(kLsThreads) void linear_scan_kernel(
     float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra, const T *v,
     int64_t v_stride, const float *dskip, float *state, int64_t slot_stride, int64_t s_off, const int32_t *seq_row0,
     const int32_t *seq_cnt, const int32_t *seq_tile0, const int32_t *tok_pos, const int32_t *tok_state, int H, int d, int dp,
-    int dv, int shares, int units) {
+    int dv, int shares, int units, int segments, int seg_tiles, const float *seg_states, const float *seg_decays) {
     __shared__ float red[2][kLsWaves][256];
-    const int id = blockIdx.x, unit = (id & 7) + 8 * ((id >> 3) / shares);      // (portion, head); id % 8 is the XCD
+    const int id = blockIdx.x, unit = (id & 7) + 8 * ((id >> 3) / (shares * segments));     // (portion, head); id % 8 is the XCD
     if (unit >= units) return;
-    const int seq = unit / H, h = unit - seq * H, col0 = ((id >> 3) % shares) * 16;
-    const int row0 = seq_row0[seq], cnt = seq_cnt[seq], tile0 = seq_tile0[seq];
+    const int seq = unit / H, h = unit - seq * H, col0 = ((id >> 3) % shares) * 16, seg = (id >> 3) / shares % segments;
+    // this workgroup's segment of the portion (the whole portion without segments)
+    const int first = seg * seg_tiles * kLsTile, all = seq_cnt[seq];
+    if (first >= all) return;
+    const bool last = all - first <= seg_tiles * kLsTile;
+    const int start = seq_row0[seq], row0 = start + first, cnt = last ? all - first : seg_tiles * kLsTile;
+    const int tile0 = seq_tile0[seq] + seg * seg_tiles;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int li = lane & 15, lq = lane >> 4;
     const int col = col0 + li;
     const bool okc = col < dv;
     const int ntiles = dp >> 4;
-    float *S = state + static_cast<int64_t>(tok_state[row0] >> 1) * slot_stride + s_off + static_cast<int64_t>(h) * d * dv;
-    const bool fresh = tok_pos[row0] == 0;      // a sequence starts from the zero state whatever the slot held
+    float *S = state + static_cast<int64_t>(tok_state[start] >> 1) * slot_stride + s_off + static_cast<int64_t>(h) * d * dv;
+    const bool fresh = tok_pos[start] == 0;     // a sequence starts from the zero state whatever the slot held
+    // a portion of several segments: its own state is in the scratch too (the last segment may be done with the slot by now)
+    const int64_t states = static_cast<int64_t>(d) * dv;
+    const float *from_seg = seg_states + static_cast<int64_t>(unit) * (segments + 1) * states;
+    const bool cut = !(last && seg == 0);
+    const float *begin = !cut ? S : seg == 0 ? from_seg : from_seg + states;
     float4_t st[TW];        // st[j][r] = S[16 (wave TW + j) + 4 lq + r][col]
 #pragma unroll
     for (int j = 0; j < TW; ++j) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int row = 16 * (wave * TW + j) + 4 * lq + r;
-            st[j][r] = (!fresh && okc && row < d) ? S[static_cast<int64_t>(row) * dv + col] : 0.f;
+            st[j][r] = ((cut || !fresh) && okc && row < d) ? begin[static_cast<int64_t>(row) * dv + col] : 0.f;
+        }
+    }
+    for (int g = 1; g < seg; ++g) {
+#pragma unroll
+        for (int j = 0; j < TW; ++j) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * (wave * TW + j) + 4 * lq + r;
+                if (okc && row < d)
+                    st[j][r] = fmaf(st[j][r], seg_decays[(static_cast<int64_t>(unit) * segments + g) * dp + row],
+                                    from_seg[(g + 1) * states + static_cast<int64_t>(row) * dv + col]);
+            }
         }
     }
     const float dh = dskip ? dskip[h] : 0.f;
@@ -241,6 +268,7 @@ __global__ __launch_bounds__(kLsThreads) void linear_scan_kernel(
 #pragma unroll
     for (int a = 0; a < AHEAD; ++a)
         if (i + a < nt) compute(i + a, f[a]);       // (uniform)
+    if (!last) return;
 #pragma unroll
     for (int j = 0; j < TW; ++j) {
         float4_t s = st[j];
@@ -249,6 +277,93 @@ __global__ __launch_bounds__(kLsThreads) void linear_scan_kernel(
         for (int r = 0; r < 4; ++r) {
             const int row = 16 * (wave * TW + j) + 4 * lq + r;
             if (okc && row < d) S[static_cast<int64_t>(row) * dv + col] = s[r];
+        }
+    }
+}
+
+// The states that the segments of cut portions leave when each starts from zero (segment 0: from the portion's state): of unit u
+// seg_states[u][0] the portion's state, [1 + g] segment g's, seg_decays[u][g] the segment's total decay per row. Waves don't meet.
+template <typename T, int TW>
+__global__ __launch_bounds__(kLsThreads) void linear_segments_kernel(
+    float *seg_states, float *seg_decays, const float *kd, const float *total, const T *v, int64_t v_stride, const float *state,
+    int64_t slot_stride, int64_t s_off, const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0,
+    const int32_t *tok_pos, const int32_t *tok_state, int H, int d, int dp, int dv, int shares, int units, int segments, int seg_tiles) {
+    constexpr int AHEAD = 4;
+    const int id = blockIdx.x, unit = (id & 7) + 8 * ((id >> 3) / (shares * segments));
+    if (unit >= units) return;
+    const int seq = unit / H, h = unit - seq * H, col0 = ((id >> 3) % shares) * 16, seg = (id >> 3) / shares % segments;
+    const int first = seg * seg_tiles * kLsTile, all = seq_cnt[seq];
+    if (all - first <= seg_tiles * kLsTile) return;     // a portion's last segment (an only one too) leaves its state to the scan
+    const int start = seq_row0[seq], tile0 = seq_tile0[seq] + seg * seg_tiles;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int li = lane & 15, lq = lane >> 4, col = col0 + li, ntiles = dp >> 4;
+    const bool okc = col < dv;
+    const int64_t states = static_cast<int64_t>(d) * dv;
+    const float *S = state + static_cast<int64_t>(tok_state[start] >> 1) * slot_stride + s_off + static_cast<int64_t>(h) * states;
+    const bool fresh = tok_pos[start] == 0;
+    float *out = seg_states + (static_cast<int64_t>(unit) * (segments + 1) + seg + 1) * states;
+    float4_t st[TW], decay[TW];
+#pragma unroll
+    for (int j = 0; j < TW; ++j) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * (wave * TW + j) + 4 * lq + r;
+            const bool ok = okc && row < d;
+            st[j][r] = seg == 0 && !fresh && ok ? S[static_cast<int64_t>(row) * dv + col] : 0.f;
+            if (seg == 0 && ok) (out - states)[static_cast<int64_t>(row) * dv + col] = st[j][r];
+            decay[j][r] = 1.f;
+        }
+    }
+    struct Operands {
+        float4_t k[TW], a[TW];
+        T v[4];
+    };
+    const T *vcol = v + static_cast<int64_t>(start + first) * v_stride + static_cast<int64_t>(h) * dv + (okc ? col : dv - 1);
+    auto load = [&](int i, Operands &f) {
+        i = min(i, seg_tiles - 1);
+        const int64_t at = static_cast<int64_t>(tile0 + i) * H + h;
+#pragma unroll
+        for (int j = 0; j < TW; ++j) {
+            const int tl = min(wave * TW + j, ntiles - 1);
+            f.k[j] = *reinterpret_cast<const float4_t *>(kd + (at * dp + 16 * tl + li) * kLsTile + 4 * lq);
+            f.a[j] = *reinterpret_cast<const float4_t *>(total + at * dp + 16 * tl + 4 * lq);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) f.v[r] = vcol[static_cast<int64_t>(i * kLsTile + 4 * lq + r) * v_stride];
+    };
+    Operands f[AHEAD];
+#pragma unroll
+    for (int a = 0; a < AHEAD; ++a) load(a, f[a]);
+    for (int i = 0; i < seg_tiles; i += AHEAD) {
+#pragma unroll
+        for (int a = 0; a < AHEAD; ++a) {
+            if (i + a < seg_tiles) {
+#pragma unroll
+                for (int j = 0; j < TW; ++j) {
+                    mfma_results_ready<8>(st[j]);
+                    st[j] *= f[a].a[j];
+                    decay[j] *= f[a].a[j];
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float vv = okc ? to_f(f[a].v[r]) : 0.f;       // (every tile of these segments is full)
+#pragma unroll
+                    for (int j = 0; j < TW; ++j) st[j] = mfma_f32_16x16x4(f[a].k[j][r], vv, st[j]);
+                }
+                load(i + a + AHEAD, f[a]);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < TW; ++j) {
+        float4_t s = st[j];
+        mfma_results_ready<8>(s);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = 16 * (wave * TW + j) + 4 * lq + r;
+            if (row >= d) continue;
+            if (okc) out[static_cast<int64_t>(row) * dv + col] = s[r];
+            if (col == 0) seg_decays[(static_cast<int64_t>(unit) * segments + seg) * dp + row] = decay[j][r];
         }
     }
 }
@@ -390,12 +505,22 @@ extern "C" int swl_linear_chunks(float *qd, float *kd, float *total, float *intr
     return swl::check_launch();
 }
 
-extern "C" int swl_linear_scan(float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra,
+/* Bytes of scratch that swl_linear_scan_segments needs. */
+extern "C" size_t swl_linear_scan_scratch_bytes(int64_t num_seqs, int32_t num_heads, int32_t dim, int32_t vdim, int32_t segments) {
+    if (segments <= 1) return 0;
+    const size_t states = static_cast<size_t>(segments + 1) * dim * vdim, decays = static_cast<size_t>(segments) * ((dim + 15) / 16 * 16);
+    return sizeof(float) * static_cast<size_t>(num_seqs) * num_heads * (states + decays);
+}
+
+extern "C" int swl_linear_scan_segments(float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra,
                                const void *v, int64_t v_stride, const float *dskip, float *state, int64_t slot_stride,
                                int64_t s_off, const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0,
                                const int32_t *tok_pos, const int32_t *tok_state, int32_t num_seqs, int32_t num_heads, int32_t dim,
-                               int32_t vdim, int32_t dtype, swl_stream_t stream) {
-    if (num_seqs < 0 || num_heads <= 0 || dim <= 0 || vdim <= 0) return SWL_ERR_BAD_ARG;
+                               int32_t vdim, int32_t segments, int32_t seg_tiles, float *scratch, int32_t dtype,
+                                        swl_stream_t stream) {
+    if (num_seqs < 0 || num_heads <= 0 || dim <= 0 || vdim <= 0 || segments < 1 || segments > 64) return SWL_ERR_BAD_ARG;
+    if (segments > 1 && (seg_tiles < 1 || !scratch)) return SWL_ERR_BAD_ARG;
+    if (segments == 1) seg_tiles = 1 << 26;     // (one segment holds every portion)
     const int64_t width = static_cast<int64_t>(num_heads) * vdim;
     if (o_stride < width || v_stride < width) return SWL_ERR_BAD_ARG;
     if (num_seqs == 0) return SWL_OK;
@@ -403,17 +528,24 @@ extern "C" int swl_linear_scan(float *o, int64_t o_stride, const float *qd, cons
         return SWL_ERR_BAD_ARG;
     if (!swl::aligned16(qd) || !swl::aligned16(kd) || !swl::aligned16(total)) return SWL_ERR_BAD_ARG;
     const int dp = (dim + 15) / 16 * 16, shares = (vdim + 15) / 16;
-    const int64_t units = static_cast<int64_t>(num_seqs) * num_heads, blocks = 8 * ((units + 7) / 8) * shares;
+    const int64_t units = static_cast<int64_t>(num_seqs) * num_heads, blocks = 8 * ((units + 7) / 8) * shares * segments;
     if (dp > swl::kLsMaxDim || num_heads > 65535 || shares > 65535 || blocks > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
     const int tw = (dp / 16 + swl::kLsWaves - 1) / swl::kLsWaves;       // 1 .. 5
     const dim3 grid(static_cast<unsigned>(blocks));
+    float *seg_states = scratch, *seg_decays = scratch ? scratch + units * (segments + 1) * dim * vdim : nullptr;
 #define SWL_LS(N)                                                                                                             \
     case N:                                                                                                                   \
+        if (segments > 1)                                                                                                     \
+            hipLaunchKernelGGL((swl::linear_segments_kernel<T, N>), grid, dim3(swl::kLsThreads), 0,                           \
+                               static_cast<hipStream_t>(stream), seg_states, seg_decays, kd, total,                           \
+                               static_cast<const T *>(v), v_stride, state, slot_stride, s_off, seq_row0, seq_cnt, seq_tile0,  \
+                               tok_pos, tok_state, num_heads, dim, dp, vdim, shares, static_cast<int>(units), segments,       \
+                               seg_tiles);                                                                                    \
         hipLaunchKernelGGL((swl::linear_scan_kernel<T, N, (N <= 2 ? 2 : 1)>), grid, dim3(swl::kLsThreads), 0,                 \
-                           static_cast<hipStream_t>(stream), o, o_stride, qd, kd, total, intra,                         \
+                           static_cast<hipStream_t>(stream), o, o_stride, qd, kd, total, intra,                               \
                            static_cast<const T *>(v), v_stride, dskip, state, slot_stride, s_off,                             \
                            seq_row0, seq_cnt, seq_tile0, tok_pos, tok_state, num_heads, dim, dp, vdim, shares,                \
-                           static_cast<int>(units));                                                                          \
+                           static_cast<int>(units), segments, seg_tiles, seg_states, seg_decays);                             \
         break
     SWL_DISPATCH_DTYPE3(dtype, T, {
         switch (tw) {
@@ -427,6 +559,15 @@ extern "C" int swl_linear_scan(float *o, int64_t o_stride, const float *qd, cons
     });
 #undef SWL_LS
     return swl::check_launch();
+}
+
+extern "C" int swl_linear_scan(float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra,
+                               const void *v, int64_t v_stride, const float *dskip, float *state, int64_t slot_stride,
+                               int64_t s_off, const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0,
+                               const int32_t *tok_pos, const int32_t *tok_state, int32_t num_seqs, int32_t num_heads, int32_t dim,
+                               int32_t vdim, int32_t dtype, swl_stream_t stream) {
+    return swl_linear_scan_segments(o, o_stride, qd, kd, total, intra, v, v_stride, dskip, state, slot_stride, s_off, seq_row0, seq_cnt,
+                                    seq_tile0, tok_pos, tok_state, num_seqs, num_heads, dim, vdim, 1, 0, nullptr, dtype, stream);
 }
 
 extern "C" int swl_linear_step(void *out, int64_t out_stride, float *y, int64_t y_stride, const void *q, int64_t q_stride,

@@ -29,6 +29,29 @@ def low_rank_decay(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, bias: to
     return out
 
 
+# Segments of a portion: as many as leave SEGMENT_MIN_TILES tiles each and SEGMENT_SLOTS workgroups on the chip, and three at least (two run
+# the first half's keys twice for little). A pass of 4 layers, 8 heads of 128, against whole portions: 1 prompt of 2000 tokens 1555 -> 1257 us (12
+# segments), 2 of 1000 beside 30 decoded tokens 1450 -> 1352 us (4), 4 of 1000 1870 -> 1854 us (3; 1893 with 2, 1900 with 4).
+SEGMENT_MIN_TILES, SEGMENT_SLOTS, SEGMENT_MAX_SCRATCH = 8, 768, 1 << 28
+
+
+def scan_segments(st: StateRef, heads: int, dim: int, vdim: int):
+    """(segments, tiles of one, scratch) of a step's scan; (1, 0, None): portions run whole."""
+    tiles = -(-st.longest // 16)
+    if tiles < 3 * SEGMENT_MIN_TILES:
+        return 1, 0, None
+    long_portions = -(-st.tiles[0].shape[0] // tiles)       # (as if every tile belonged to a portion of the longest's length)
+    segments = min(SEGMENT_SLOTS // (long_portions * heads * -(-vdim // 16)), tiles // SEGMENT_MIN_TILES, 64)
+    if segments < 3:
+        return 1, 0, None
+    seg_tiles = -(-tiles // segments)
+    segments = -(-tiles // seg_tiles)
+    scratch_bytes = _hip.load().swl_linear_scan_scratch_bytes(st.seq_row0.shape[0], heads, dim, vdim, segments)
+    if scratch_bytes > SEGMENT_MAX_SCRATCH:
+        return 1, 0, None
+    return segments, seg_tiles, torch.empty(scratch_bytes // 4, dtype=torch.float32, device=st.pool.device)
+
+
 def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, st: StateRef, state_off: int,
                       num_heads: int, dim: int, vdim: int, q_scale: float = 1.0, bonus: torch.Tensor = None,
                       k_scale: torch.Tensor = None, dskip: torch.Tensor = None, num_qk_heads: int = 0, finish=None) -> torch.Tensor:
@@ -74,10 +97,11 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
               _hip.ptr(k), k.stride(0), _hip.ptr(decay), decay.stride(0), 1 if per_channel else 0, _hip.ptr(k_scale),
               _hip.ptr(bonus), float(q_scale), _hip.ptr(row0), _hip.ptr(cnt), num_tiles, H, G, dim, code, stream)
     o = torch.empty((n, H * vdim), dtype=f32, device=dev)
-    _hip.call("swl_linear_scan", _hip.ptr(o), o.stride(0), _hip.ptr(qd), _hip.ptr(kd), _hip.ptr(total), _hip.ptr(intra),
+    segments, seg_tiles, scratch = scan_segments(st, H, dim, vdim)
+    _hip.call("swl_linear_scan_segments", _hip.ptr(o), o.stride(0), _hip.ptr(qd), _hip.ptr(kd), _hip.ptr(total), _hip.ptr(intra),
               _hip.ptr(v), v.stride(0), _hip.ptr(dskip), _hip.ptr(st.pool), st.pool.stride(0), int(state_off),
               _hip.ptr(st.seq_row0), _hip.ptr(st.seq_cnt), _hip.ptr(seq_tile0), _hip.ptr(st.tok_pos), _hip.ptr(st.tok_state),
-              num_seqs, H, dim, vdim, code, stream)
+              num_seqs, H, dim, vdim, segments, seg_tiles, _hip.ptr(scratch), code, stream)
     if finish is None:
         return o
     out, norm_w, gate, eps, mult = finish

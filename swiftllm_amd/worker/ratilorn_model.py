@@ -105,7 +105,8 @@ class RatilornModel(SteppedModel):
         st = None
         if self.state is not None:
             st = StateRef(self.state.pool, dev["tok_pos"], dev["tok_start"], dev["tok_state"], dev["tok_seq"],
-                          dev["seq_row0"], dev["seq_cnt"], (dev["tile_row0"], dev["tile_cnt"], dev["seq_tile0"]))
+                          dev["seq_row0"], dev["seq_cnt"], (dev["tile_row0"], dev["tile_cnt"], dev["seq_tile0"]),
+                          dev.get("longest_portion", 0))
         ctx = StepContext(self.kv_pool if use_pool else None, self.gpu_block_manager.block_table if use_pool else None,
                           dev["tok_seq"], dev["tok_pos"], StepTiles.of(dev), st)
         x, _ = embed_positions(dev["input_ids"], dev["tok_pos"], w.embed, w.pos, 1.0, keep_copy=False)
