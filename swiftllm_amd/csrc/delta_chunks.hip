@@ -17,8 +17,8 @@
 // What bounds the walk: the chain of tiles (two products of 16 x 16 x dim on four SIMDs and an exchange through LDS a tile: about 1400
 // cycles, 512 of them matrix core). Splitting off the outputs and reading blocks took a tile from 3100 to 2100 cycles.
 // The column shares of a (portion, head) pair read the same operands: consecutive numbers on one XCD.
-// Measured against the walk token by token (8 heads of 128 x 128): 4 prompts of 2048 tokens 746 -> 149 us (both launches, back to back), 2 of 1000
-// beside 30 decoded tokens 899 -> 79 us. Error of o against 64 bits: 1 to 2e-7 of the largest value (0.6 to 1.3e-7 token by token); of
+// Measured against the walk token by token (8 heads of 128 x 128): 4 prompts of 2048 tokens 746 -> 146 us (both launches, back to back), 2 of 1000
+// beside 30 decoded tokens 899 -> 73 us. Error of o against 64 bits: 1 to 2e-7 of the largest value (0.6 to 1.3e-7 token by token); of
 // a model's logits in fp32: 0.98e-6 against 1.0e-6.
 #include "swl_common.h"
 
@@ -30,7 +30,7 @@ __device__ __forceinline__ float4_t dc_mfma(float a, float b, float4_t c) { retu
 
 // scratch of one (tile, head), in whole blocks of the order in which the walk's lanes read them:
 //   W [D / 16][16 tokens][16 dims] | K^T diag(r) [D / 16][16 dims][16 tokens] | U0 [dv / 16][token % 4][token / 4][16 columns] |
-//   A [16][16] | b [16] | b_15 [16] (once a lane: a scalar load would be waited for together with the exchange through LDS)
+//   A [key % 4][key / 4][query] | b [16] | b_15 [16] (once a lane: a scalar load would be waited for together with the exchange through LDS)
 __host__ __device__ inline int64_t dc_floats(int D, int dv) { return 16LL * (2 * D + dv) + 256 + 32; }
 
 template <int D>
@@ -95,13 +95,14 @@ __global__ __launch_bounds__(64, 3) void delta_chunk_kernel(float *scratch, cons
     }
     float *out = scratch + (static_cast<int64_t>(tile) * H + h) * dc_floats(D, dv);
     float *w_out = out, *k_out = w_out + 16 * D, *u_out = k_out + 16 * D, *a_out = u_out + 16 * dv, *b_out = a_out + 256;
-    float4_t lcol;
+    float4_t lcol, acol;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int i = 4 * g + e;
         lcol[e] = li < i ? su[e] * rr[e] * m[e] : 0.f;
-        a_out[i * 16 + li] = li <= i ? rr[e] * p[e] : 0.f;
+        acol[e] = li <= i ? rr[e] * p[e] : 0.f;
     }
+    *reinterpret_cast<float4_t *>(a_out + (li & 3) * 64 + (li >> 2) * 16 + 4 * g) = acol;
     if (g == 0) {
         b_out[li] = b;
         b_out[16 + li] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(b), 15));
@@ -283,16 +284,16 @@ __global__ __launch_bounds__(512, 4) void delta_walk_kernel(float *o, const floa
     }
     // ---- the outputs, one barrier behind: diag(b) Q S over D / 4 rows of S, and step `wave` of A U ----------------------------------
     struct Ops {
-        float4_t q[NT], b;
-        float a;
+        float4_t q[NT];
+        float a, b;
     };
-    const uint32_t a_off = 4 * (32 * D + 16 * dv + li * 16 + 4 * g + wave), b_off = 4 * (32 * D + 16 * dv + 256 + 4 * g);
+    const uint32_t a_off = 4 * (32 * D + 16 * dv + wave * 64 + lane), b_off = 4 * (32 * D + 16 * dv + 256 + 4 * g + (li & 3));
     uint32_t q_off = 4 * (li * qk + base + 4 * g);
     auto fetch = [&](Ops &f) {
         if (next == ntiles - 1) q_off = 4 * (min(li, (cnt - 1) & 15) * qk + base + 4 * g);
 #pragma unroll
         for (int t = 0; t < NT; ++t) f.q[t] = dc_load4(rows, q_off + 64 * t);
-        f.b = dc_load4(pre, b_off);
+        f.b = dc_load(pre, b_off);
         f.a = dc_load(pre, a_off);
         advance();
     };
@@ -329,8 +330,9 @@ __global__ __launch_bounds__(512, 4) void delta_walk_kernel(float *o, const floa
         mfma_results_ready<8>(own);
 #pragma unroll
         for (int t = 1; t < NT; ++t) ot[0] += ot[t];
+        const float4_t b = quad_values(f.b);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) own[e] = fmaf(ot[0][e], f.b[e], own[e]);
+        for (int e = 0; e < 4; ++e) own[e] = fmaf(ot[0][e], b[e], own[e]);
         s_o[c & 1][wave][lane] = own;
     };
     Ops ops[DEPTH];

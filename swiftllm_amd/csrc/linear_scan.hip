@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kLsThreads) void linear_chunks_kernel(
         const float v = group_allreduce_sum<16>(acc[t]);
         if (g == t) mine = v;
     }
-    intra[at * 256 + g * kLsTile + s] = mine;       // [t][s]
+    intra[at * 256 + (s & 3) * 64 + (s >> 2) * 16 + g] = mine;      // (t = g) as the scan's waves read it: wave s % 4, lane 16 (s / 4) + t
 }
 
 __device__ __forceinline__ float4_t mfma_f32_16x16x4(float a, float b, float4_t c) {
@@ -135,8 +135,8 @@ __device__ __forceinline__ float4_t mfma_f32_16x16x4(float a, float b, float4_t 
 // predicated load would be waited for on the spot, and the point is to have a tile's loads in flight while others are computed.
 template <typename T, int TW>
 struct LsOperands {
-    float4_t q[TW], k[TW], a[TW];
-    float m;
+    float4_t q[TW], k[TW];
+    float a[TW], m;
     T v[4];
 };
 
@@ -201,9 +201,9 @@ __global__ __launch_bounds__(kLsThreads) void linear_scan_kernel(
             const int tl = min(wave * TW + j, ntiles - 1);
             f.q[j] = *reinterpret_cast<const float4_t *>(qd + at * kLsTile * dp + tl * 256 + li * 16 + 4 * lq);
             f.k[j] = *reinterpret_cast<const float4_t *>(kd + (at * dp + 16 * tl + li) * kLsTile + 4 * lq);
-            f.a[j] = *reinterpret_cast<const float4_t *>(total + at * dp + 16 * tl + 4 * lq);
+            f.a[j] = total[at * dp + 16 * tl + 4 * lq + (li & 3)];
         }
-        f.m = intra[at * 256 + li * kLsTile + 4 * lq + wave];
+        f.m = intra[at * 256 + wave * 64 + lane];
 #pragma unroll
         for (int r = 0; r < 4; ++r) f.v[r] = vcol[static_cast<int64_t>(min(i * kLsTile + 4 * lq + r, cnt - 1)) * v_stride];
     };
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(kLsThreads) void linear_scan_kernel(
 #pragma unroll
         for (int j = 0; j < TW; ++j) {
             mfma_results_ready<8>(st[j]);
-            st[j] *= f.a[j];
+            st[j] *= quad_values(f.a[j]);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -315,7 +315,8 @@ __global__ __launch_bounds__(kLsThreads) void linear_segments_kernel(
         }
     }
     struct Operands {
-        float4_t k[TW], a[TW];
+        float4_t k[TW];
+        float a[TW];
         T v[4];
     };
     const T *vcol = v + static_cast<int64_t>(start + first) * v_stride + static_cast<int64_t>(h) * dv + (okc ? col : dv - 1);
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(kLsThreads) void linear_segments_kernel(
         for (int j = 0; j < TW; ++j) {
             const int tl = min(wave * TW + j, ntiles - 1);
             f.k[j] = *reinterpret_cast<const float4_t *>(kd + (at * dp + 16 * tl + li) * kLsTile + 4 * lq);
-            f.a[j] = *reinterpret_cast<const float4_t *>(total + at * dp + 16 * tl + 4 * lq);
+            f.a[j] = total[at * dp + 16 * tl + 4 * lq + (li & 3)];
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) f.v[r] = vcol[static_cast<int64_t>(i * kLsTile + 4 * lq + r) * v_stride];
@@ -341,8 +342,9 @@ __global__ __launch_bounds__(kLsThreads) void linear_segments_kernel(
 #pragma unroll
                 for (int j = 0; j < TW; ++j) {
                     mfma_results_ready<8>(st[j]);
-                    st[j] *= f[a].a[j];
-                    decay[j] *= f[a].a[j];
+                    const float4_t by = quad_values(f[a].a[j]);
+                    st[j] *= by;
+                    decay[j] *= by;
                 }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {

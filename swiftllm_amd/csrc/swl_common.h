@@ -115,6 +115,12 @@ __device__ __forceinline__ float group_allreduce_sum(float v) {
     return v;
 }
 
+// The values of the four lanes of a lane's quad. (A wave that needs the same four floats in 16 lanes loads one a lane, 4 L1 accesses, and
+// spreads them here: a 16-byte load that 16 lanes share takes 16.)
+__device__ __forceinline__ float4_t quad_values(float v) {
+    return float4_t{dpp_mov<0x00>(v), dpp_mov<0x55>(v), dpp_mov<0xAA>(v), dpp_mov<0xFF>(v)};    // quad_perm: lane 0, 1, 2, 3 to all
+}
+
 // Full-wave (64-lane) all-reduce: DPP inside rows of 16, then two cross-row exchanges.
 __device__ __forceinline__ float wave_allreduce_sum(float v) {
     v = group_allreduce_sum<16>(v);

@@ -92,7 +92,7 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
     qd = torch.empty((num_tiles, H, 16, dp), dtype=f32, device=dev)
     kd = torch.empty((num_tiles, H, dp, 16), dtype=f32, device=dev)
     total = torch.empty((num_tiles, H, dp), dtype=f32, device=dev)
-    intra = torch.empty((num_tiles, H, 16, 16), dtype=f32, device=dev)
+    intra = torch.empty((num_tiles, H, 4, 4, 16), dtype=f32, device=dev)
     _hip.call("swl_linear_chunks", _hip.ptr(qd), _hip.ptr(kd), _hip.ptr(total), _hip.ptr(intra), _hip.ptr(q), q.stride(0),
               _hip.ptr(k), k.stride(0), _hip.ptr(decay), decay.stride(0), 1 if per_channel else 0, _hip.ptr(k_scale),
               _hip.ptr(bonus), float(q_scale), _hip.ptr(row0), _hip.ptr(cnt), num_tiles, H, G, dim, code, stream)
