@@ -2,6 +2,7 @@
 // fused "normalised sublayer output into the residual, then the next sublayer's input norm" step of sandwich-norm
 // models. The residual x is fp32 [tokens, width]; sublayer inputs/outputs are the compute dtype (bf16 / f16 / f32);
 // every statistic (mean, mean of squared deviations) is taken in fp32 with two passes over the row.
+#include "row_wide.h"
 #include "swl_common.h"
 
 namespace swl {
@@ -99,6 +100,88 @@ __global__ __launch_bounds__(kLnThreads) void add_layernorm_kernel(float *x, con
         out[t * width + i] = to_t<T>((row[i] - mean) * rstd * w2[i] + b2[i]);
 }
 
+// The same with the row in registers (row_wide.h): rows of a multiple of four columns, up to 8192, on aligned addresses. Bound by memory: y and
+// out in the compute dtype, x in and out in fp32 (and x0). bf16, 4500 x 2048: 47 -> 27 us (4.1 TB/s),
+// 32 x 2048 7.7 -> 4.6 us.
+template <int TPR, int NV>
+__device__ __forceinline__ void wide_stats(const float (&v)[NV][4], int c0, int width, float eps, float *red, float &mean, float &rstd) {
+    float s = 0.f, q = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += v[j][e];       // (columns past the row are 0)
+    mean = row_sum<TPR>(s, red) / static_cast<float>(width);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        if (c0 + 4 * TPR * j < width) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float d = v[j][e] - mean;
+                q += d * d;
+            }
+        }
+    }
+    rstd = 1.0f / sqrtf(row_sum<TPR>(q, red + kRowThreads / 64) / static_cast<float>(width) + eps);
+}
+
+template <typename T, int TPR, int NV>
+__global__ __launch_bounds__(kRowThreads) void add_layernorm_wide_kernel(float *x, const T *y, float mult, const float *w1, const float *b1,
+                                                                         const float *x0, const float *step, T *out, const float *w2,
+                                                                         const float *b2, float eps, int64_t rows, int width) {
+    __shared__ float red[4][kRowThreads / 64];
+    const int64_t id = static_cast<int64_t>(blockIdx.x) * (kRowThreads / TPR) + threadIdx.x / TPR, t = min(id, rows - 1);
+    const bool live = id < rows;
+    const int c0 = (threadIdx.x % TPR) * 4;
+    float v[NV][4], s[NV][4], extra[NV][4], mean, rstd;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = c0 + 4 * TPR * j;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][e] = s[j][e] = extra[j][e] = 0.f;
+        if (c < width) {
+            if (y) row_load<T>(s[j], y + t * width + c);
+            row_load<float>(v[j], x + t * width + c);
+            if (x0) row_load<float>(extra[j], x0 + t * width + c);
+        }
+    }
+    if (y) wide_stats<TPR, NV>(s, c0, width, eps, red[0], mean, rstd);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = c0 + 4 * TPR * j;
+        if (c < width) {
+            if (y) {
+                float w[4], b[4];
+                row_load<float>(w, w1 + c);
+                row_load<float>(b, b1 + c);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[j][e] += mult * ((s[j][e] - mean) * rstd * w[e] + b[e]);
+            }
+            float add[4] = {0.f, 0.f, 0.f, 0.f};
+            if (step) row_load<float>(add, step + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (x0) v[j][e] += extra[j][e];
+                if (step) v[j][e] += add[e];
+            }
+            if (live) row_store<float>(x + t * width + c, v[j]);
+        }
+    }
+    if (!out) return;
+    wide_stats<TPR, NV>(v, c0, width, eps, red[2], mean, rstd);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = c0 + 4 * TPR * j;
+        if (live && c < width) {
+            float w[4], b[4];
+            row_load<float>(w, w2 + c);
+            row_load<float>(b, b2 + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = (v[j][e] - mean) * rstd * w[e] + b[e];
+            row_store<T>(out + t * width + c, w);
+        }
+    }
+}
+
 inline size_t ln_lds_bytes(int width) { return (static_cast<size_t>(width) + kLnThreads / 64) * sizeof(float); }
 
 } // namespace swl
@@ -139,10 +222,23 @@ extern "C" int swl_add_layernorm(float *x, const void *y, float mult, const floa
     if (num_tokens == 0) return SWL_OK;
     if (!x || (y && (!w1 || !b1)) || (out && (!w2 || !b2))) return SWL_ERR_BAD_ARG;
     if (num_tokens > 0x7fffffffLL || swl::ln_lds_bytes(width) > 64 * 1024) return SWL_ERR_UNSUPPORTED;
+#define SWL_GO(TPR, NV)                                                                                                                \
+    hipLaunchKernelGGL((swl::add_layernorm_wide_kernel<T, TPR, NV>), dim3(static_cast<unsigned>((num_tokens * TPR + 255) / 256)),      \
+                       dim3(swl::kRowThreads), 0, static_cast<hipStream_t>(stream), x, static_cast<const T *>(y), mult, w1, b1, x0,    \
+                       step, static_cast<T *>(out), w2, b2, eps, num_tokens, width)
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        const bool wide = width % 4 == 0 && width <= swl::kRowMaxWidth && swl::row_aligned<float>(x) && swl::row_aligned<T>(y) &&
+                          swl::row_aligned<T>(out) && swl::row_aligned<float>(w1) && swl::row_aligned<float>(b1) &&
+                          swl::row_aligned<float>(w2) && swl::row_aligned<float>(b2) && swl::row_aligned<float>(x0) &&
+                          swl::row_aligned<float>(step);
+        if (wide) {
+            SWL_ROW_SHAPE(num_tokens, width, SWL_GO);
+            return swl::check_launch();
+        }
         hipLaunchKernelGGL((swl::add_layernorm_kernel<T>), dim3(static_cast<unsigned>(num_tokens)), dim3(swl::kLnThreads),
                            swl::ln_lds_bytes(width), static_cast<hipStream_t>(stream), x, static_cast<const T *>(y), mult,
                            w1, b1, x0, step, static_cast<T *>(out), w2, b2, eps, width);
     });
+#undef SWL_GO
     return swl::check_launch();
 }

@@ -14,6 +14,9 @@
 //       out = x in the compute dtype, or x / rms(x) * w2 when w2 is given
 //     Two results normed separately and averaged (mixers side by side: c = 0.5), or two addends summed as they are (routed
 //     experts + a shared expert: c = 1), or one result alone.
+//   Both are bound by memory: x in and out in fp32, the results, the gate and out once each. Rows of a multiple of four columns, up to 8192,
+//   on aligned addresses are held in registers (row_wide.h); other rows go through LDS column by column. bf16, gated step:
+//   8192 x 1024 48 -> 32 us, 4500 x 2048 56 -> 37 us, 32 x 2048 7.7 -> 4.9 us; two normed results 3663 x 2048 49 -> 26 us (4 TB/s).
 //   swl_causal_conv_state: out[t] = (h[t] if add_input) + sum_j w[j][c] * h[t - taps + 1 + j] per channel (w tap-major) over the tokens of
 //     one sequence, for any cut of the sequence into steps: inputs of earlier steps come from the sequence's state slot,
 //     which keeps the last taps - 1 inputs. The tail is double-buffered: a step reads buffer `parity` and the workgroup of
@@ -22,6 +25,7 @@
 //     of every sequence is carried like a two-tap convolution's.
 #include "swl_common.h"
 #include "conv_tail.h"
+#include "row_wide.h"
 
 namespace swl {
 
@@ -74,6 +78,171 @@ __global__ __launch_bounds__(kRsThreads) void gated_add_rmsnorm_kernel(
     for (int i = threadIdx.x; i < width; i += kRsThreads) ss += row[i] * row[i];
     const float rstd = 1.0f / sqrtf(rs_block_sum(ss, red) / static_cast<float>(width) + eps);
     for (int i = threadIdx.x; i < width; i += kRsThreads) out[o * width + i] = to_t<T>(row[i] * rstd * w2[i]);
+}
+
+template <typename T, int TPR, int NV>
+__global__ __launch_bounds__(kRowThreads) void gated_add_rmsnorm_wide_kernel(
+    float *x, const T *m, const T *m2, const T *m2_gate, int64_t m2_gate_stride, const T *r, int64_t r_stride,
+    const float *r_bias, const float *w1, T *out, const float *w2, const int32_t *row_idx, float eps, int64_t rows, int width) {
+    __shared__ float red[2][kRowThreads / 64];
+    const int64_t id = static_cast<int64_t>(blockIdx.x) * (kRowThreads / TPR) + threadIdx.x / TPR, o = min(id, rows - 1);
+    const bool live = id < rows;
+    const int64_t t = row_idx ? row_idx[o] : o;
+    const int c0 = (threadIdx.x % TPR) * 4;
+    float *xr = x + t * width;
+    float v[NV][4];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[j][e] = 0.f;
+        if (c0 + 4 * TPR * j < width) row_load<float>(v[j], xr + c0 + 4 * TPR * j);
+    }
+    if (m) {
+        float y[NV][4], a2[NV][4], rv[NV][4];
+        const float s2 = m2 ? sigmoidf_(to_f(m2_gate[t * m2_gate_stride])) : 0.f;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int c = c0 + 4 * TPR * j;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[j][e] = a2[j][e] = rv[j][e] = 0.f;
+            if (c < width) {
+                row_load<T>(y[j], m + t * width + c);
+                if (m2) row_load<T>(a2[j], m2 + t * width + c);
+                if (r) row_load<T>(rv[j], r + t * r_stride + c);
+            }
+        }
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int c = c0 + 4 * TPR * j;
+            float bias[4] = {0.f, 0.f, 0.f, 0.f};
+            if (r && c < width) row_load<float>(bias, r_bias + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (m2) y[j][e] += s2 * a2[j][e];
+                if (r) y[j][e] *= sigmoidf_(rv[j][e] + bias[e]);
+                ss += y[j][e] * y[j][e];
+            }
+        }
+        const float rstd = 1.0f / sqrtf(row_sum<TPR>(ss, red[0]) / static_cast<float>(width) + eps);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int c = c0 + 4 * TPR * j;
+            if (c < width) {
+                float w[4];
+                row_load<float>(w, w1 + c);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[j][e] = v[j][e] + y[j][e] * rstd * w[e];
+                if (live) row_store<float>(xr + c, v[j]);
+            }
+        }
+    }
+    if (!out) return;
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss += v[j][e] * v[j][e];
+    const float rstd = 1.0f / sqrtf(row_sum<TPR>(ss, red[1]) / static_cast<float>(width) + eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = c0 + 4 * TPR * j;
+        if (live && c < width) {
+            float w[4];
+            row_load<float>(w, w2 + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = v[j][e] * rstd * w[e];
+            row_store<T>(out + o * width + c, w);
+        }
+    }
+}
+
+template <typename T, int TPR, int NV>
+__global__ __launch_bounds__(kRowThreads) void post_norm_add_wide_kernel(float *x, const T *a, const float *wa, const T *b, const float *wb,
+                                                                         float coef, const float *w1, T *out, const float *w2, float eps,
+                                                                         int64_t rows, int width) {
+    __shared__ float red[4][kRowThreads / 64];
+    const int64_t id = static_cast<int64_t>(blockIdx.x) * (kRowThreads / TPR) + threadIdx.x / TPR, t = min(id, rows - 1);
+    const bool live = id < rows;
+    const int c0 = (threadIdx.x % TPR) * 4;
+    float *xr = x + t * width;
+    float y[NV][4], z[NV][4], v[NV][4];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = c0 + 4 * TPR * j;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[j][e] = z[j][e] = v[j][e] = 0.f;
+        if (c < width) {
+            row_load<T>(y[j], a + t * width + c);
+            if (b) row_load<T>(z[j], b + t * width + c);
+            row_load<float>(v[j], xr + c);
+        }
+    }
+    float na = 1.f, nb = 1.f;
+    if (wa) {
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s += y[j][e] * y[j][e];
+        na = 1.0f / sqrtf(row_sum<TPR>(s, red[0]) / static_cast<float>(width) + eps);
+    }
+    if (b && wb) {
+        float s = 0.f;
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s += z[j][e] * z[j][e];
+        nb = 1.0f / sqrtf(row_sum<TPR>(s, red[1]) / static_cast<float>(width) + eps);
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = c0 + 4 * TPR * j;
+        float w[4] = {1.f, 1.f, 1.f, 1.f}, u[4] = {1.f, 1.f, 1.f, 1.f};
+        if (wa && c < width) row_load<float>(w, wa + c);
+        if (b && wb && c < width) row_load<float>(u, wb + c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float s = wa ? y[j][e] * na * w[e] : y[j][e];
+            if (b) s += wb ? z[j][e] * nb * u[e] : z[j][e];
+            s *= coef;
+            y[j][e] = s;
+            ss += s * s;
+        }
+    }
+    const float rstd = 1.0f / sqrtf(row_sum<TPR>(ss, red[2]) / static_cast<float>(width) + eps);
+    float sx = 0.f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = c0 + 4 * TPR * j;
+        if (c < width) {
+            float w[4];
+            row_load<float>(w, w1 + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[j][e] = v[j][e] + y[j][e] * rstd * w[e];
+                sx += v[j][e] * v[j][e];
+            }
+            if (live) {
+                row_store<float>(xr + c, v[j]);
+                if (out && !w2) row_store<T>(out + t * width + c, v[j]);
+            }
+        }
+    }
+    if (!out || !w2) return;
+    const float rx = 1.0f / sqrtf(row_sum<TPR>(sx, red[3]) / static_cast<float>(width) + eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = c0 + 4 * TPR * j;
+        if (live && c < width) {
+            float w[4];
+            row_load<float>(w, w2 + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = v[j][e] * rx * w[e];
+            row_store<T>(out + t * width + c, w);
+        }
+    }
 }
 
 template <typename T>
@@ -208,12 +377,25 @@ extern "C" int swl_gated_add_rmsnorm(float *x, const void *m, const void *m2, co
         return SWL_ERR_BAD_ARG;
     if (!m && !out) return SWL_OK;
     if (num_rows > 0x7fffffffLL || swl::rs_lds_bytes(width) > 64 * 1024) return SWL_ERR_UNSUPPORTED;
+#define SWL_GO(TPR, NV)                                                                                                                \
+    hipLaunchKernelGGL((swl::gated_add_rmsnorm_wide_kernel<T, TPR, NV>), dim3(static_cast<unsigned>((num_rows * TPR + 255) / 256)),    \
+                       dim3(swl::kRowThreads), 0, static_cast<hipStream_t>(stream), x, static_cast<const T *>(m),                      \
+                       static_cast<const T *>(m2), static_cast<const T *>(m2_gate), m2_gate_stride, static_cast<const T *>(r),         \
+                       r_stride, r_bias, w1, static_cast<T *>(out), w2, row_idx, eps, num_rows, width)
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        const bool wide = width % 4 == 0 && width <= swl::kRowMaxWidth && r_stride % 4 == 0 && swl::row_aligned<float>(x) &&
+                          swl::row_aligned<T>(m) && swl::row_aligned<T>(m2) && swl::row_aligned<T>(r) && swl::row_aligned<T>(out) &&
+                          swl::row_aligned<float>(r_bias) && swl::row_aligned<float>(w1) && swl::row_aligned<float>(w2);
+        if (wide) {
+            SWL_ROW_SHAPE(num_rows, width, SWL_GO);
+            return swl::check_launch();
+        }
         hipLaunchKernelGGL((swl::gated_add_rmsnorm_kernel<T>), dim3(static_cast<unsigned>(num_rows)), dim3(swl::kRsThreads),
                            swl::rs_lds_bytes(width), static_cast<hipStream_t>(stream), x, static_cast<const T *>(m),
                            static_cast<const T *>(m2), static_cast<const T *>(m2_gate), m2_gate_stride,
                            static_cast<const T *>(r), r_stride, r_bias, w1, static_cast<T *>(out), w2, row_idx, eps, width);
     });
+#undef SWL_GO
     return swl::check_launch();
 }
 
@@ -261,10 +443,22 @@ extern "C" int swl_post_norm_add(float *x, const void *a, const float *wa, const
     if (!x || !a || !w1 || (wb && !b) || (w2 && !out)) return SWL_ERR_BAD_ARG;
     const size_t lds = (2 * static_cast<size_t>(width) + swl::kRsThreads / 64) * sizeof(float);
     if (num_rows > 0x7fffffffLL || lds > 64 * 1024) return SWL_ERR_UNSUPPORTED;
+#define SWL_GO(TPR, NV)                                                                                                                \
+    hipLaunchKernelGGL((swl::post_norm_add_wide_kernel<T, TPR, NV>), dim3(static_cast<unsigned>((num_rows * TPR + 255) / 256)),        \
+                       dim3(swl::kRowThreads), 0, static_cast<hipStream_t>(stream), x, static_cast<const T *>(a), wa,                  \
+                       static_cast<const T *>(b), wb, coef, w1, static_cast<T *>(out), w2, eps, num_rows, width)
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        const bool wide = width % 4 == 0 && width <= swl::kRowMaxWidth && swl::row_aligned<float>(x) && swl::row_aligned<T>(a) &&
+                          swl::row_aligned<T>(b) && swl::row_aligned<T>(out) && swl::row_aligned<float>(wa) &&
+                          swl::row_aligned<float>(wb) && swl::row_aligned<float>(w1) && swl::row_aligned<float>(w2);
+        if (wide) {
+            SWL_ROW_SHAPE(num_rows, width, SWL_GO);
+            return swl::check_launch();
+        }
         hipLaunchKernelGGL((swl::post_norm_add_kernel<T>), dim3(static_cast<unsigned>(num_rows)), dim3(swl::kRsThreads), lds,
                            static_cast<hipStream_t>(stream), x, static_cast<const T *>(a), wa, static_cast<const T *>(b), wb,
                            coef, w1, static_cast<T *>(out), w2, eps, width);
     });
+#undef SWL_GO
     return swl::check_launch();
 }

@@ -1,0 +1,62 @@
+"""Residual steps with rows in registers (csrc/row_wide.h: rms_stream.hip, layernorm.hip) against float64, at the edges of every split of a
+row: one wave, two or four a row, the last columns of a row and the last rows of a launch, and rows that stay with the other kernels."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = 1e-5
+# (1024 rows: a wave a row up to 1024 columns, two up to 2048; 2050 and 8196 columns: column by column)
+SHAPES = [(3, 4), (33, 260), (5, 1024), (1025, 1024), (1023, 1024), (1027, 60), (2, 1028), (1026, 1028), (1025, 2048), (7, 2048), (3, 2050),
+          (1024, 3000), (2, 4096), (3, 4100), (2, 8188), (1, 8196)]
+
+
+def _rms(x):
+    return x / torch.sqrt((x * x).mean(1, keepdim=True) + EPS)
+
+
+def _ln(x, wb):
+    d = x - x.mean(1, keepdim=True)
+    return d / torch.sqrt((d * d).mean(1, keepdim=True) + EPS) * wb[0].double() + wb[1].double()
+
+
+def _close(x, out, want, out_want, dtype):
+    # the stream: a few fp32 roundings of the row's values and of a sum of up to 8196 squares; the result: one rounding to its type on top
+    scale = max(1.0, float(want.abs().max()))
+    assert (x.double().cpu() - want).abs().max() <= 4e-6 * scale
+    eps = {torch.float32: 4e-6, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10}[dtype]
+    assert ((out.double().cpu() - out_want).abs() <= eps * out_want.abs() + 4e-6 * float(out_want.abs().max())).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,width", SHAPES)
+def test_rows(rows, width, dtype):
+    from swiftllm_amd.worker.kernels.layernorm import add_layernorm
+    from swiftllm_amd.worker.kernels.rms_stream import gated_add_rmsnorm, post_norm_add
+    g = torch.Generator().manual_seed(rows + width)
+    x, x0 = torch.randn(rows, width, generator=g) * 2, torch.randn(rows, width, generator=g)
+    a, b, r, s = (torch.randn(rows, n, generator=g).to(dtype) for n in (width, width, width + 8, 3))
+    w = [1 + 0.2 * torch.randn(width, generator=g) for _ in range(4)]
+    bias = torch.randn(width, generator=g)
+    xd, ad, bd, rd = x.double(), a.double(), b.double(), r.double()
+    wd, wc = [v.double() for v in w], [v.cuda() for v in w]
+
+    for shift in (4, 2):        # (2: a gate that is not aligned goes column by column)
+        gpu = x.cuda()
+        out = gated_add_rmsnorm(gpu, a.cuda(), wc[0], r.cuda()[:, shift:shift + width], bias.cuda(), b.cuda(), s.cuda()[:, 1:2], wc[1], EPS)
+        y = (ad + torch.sigmoid(s.double()[:, 1:2]) * bd) * torch.sigmoid(rd[:, shift:shift + width] + bias.double())
+        want = xd + _rms(y) * wd[0]
+        _close(gpu, out, want, _rms(want) * wd[1], dtype)
+
+    for norms in (True, False):
+        if 2 * width + 4 > 16384:
+            break
+        gpu = x.cuda()
+        out = post_norm_add(gpu, a.cuda(), wc[0], b.cuda(), wc[1] if norms else None, wc[2] if norms else None, 0.5, wc[3] if norms else None, EPS)
+        y = 0.5 * (_rms(ad) * wd[1] + _rms(bd) * wd[2] if norms else ad + bd)
+        want = xd + _rms(y) * wd[0]
+        _close(gpu, out, want, _rms(want) * wd[3] if norms else want, dtype)
+
+    gpu = x.cuda()
+    out = add_layernorm(gpu, a.cuda(), 0.3, (wc[0], wc[1]), x0.cuda(), bias.cuda(), (wc[2], wc[3]), EPS)
+    want = xd + 0.3 * _ln(ad, w[:2]) + x0.double() + bias.double()
+    _close(gpu, out, want, _ln(want, w[2:]), dtype)
