@@ -149,6 +149,10 @@ class SteppedModel:
             self._meta_host_np = self._meta_host.numpy()
             self._meta_dev = torch.empty(cap, dtype=torch.int32, device=self.device)
             self._meta_done = torch.cuda.Event()
+            # captured graphs read the old buffer; their shared memory pool goes with them (a capture into a pool whose last graph is
+            # gone is refused by the caching allocator)
+            self._decode_graphs.clear()
+            self._graph_pool = None
         plan.pack_into(self._meta_host_np)
         self._meta_dev[:total].copy_(self._meta_host[:total], non_blocking=True)
         self._meta_done.record()
@@ -196,8 +200,6 @@ class SteppedModel:
         the next replay of the same graph."""
         key = plan.num_tokens
         entry = self._decode_graphs.pop(key, None)
-        if entry is not None and entry[2] != self._meta_dev.data_ptr():
-            entry = None        # the metadata buffer was re-allocated: the capture points at the old one
         if entry is None:
             self.graph_captures += 1
             # one eager run first: nothing may be lazily initialised under capture. The replay below runs the step once more:
@@ -217,7 +219,7 @@ class SteppedModel:
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph, pool=self._graph_pool):
                 out = self._logits(self._run_stack(dev, True), dev["want_rows"])
-            entry = (graph, out, self._meta_dev.data_ptr())
+            entry = (graph, out)
         self._decode_graphs[key] = entry
         entry[0].replay()
         return entry[1]
