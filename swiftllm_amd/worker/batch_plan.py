@@ -193,11 +193,9 @@ class StepPlan:
         return total
 
 
-def plan_step(entries: Sequence[StepEntry], vocab_size: int = None, max_positions: int = None) -> StepPlan:
-    """Flatten the entries in order. Checked here, on the host, so that nothing out of range reaches a kernel: token ids
-    against the vocabulary, positions against the position table, one entry per sequence."""
-    ids, pos, seq, want, seq_ids, targets = [], [], [], [], [], []
-    base = 0
+def _check_entries(entries: Sequence[StepEntry], vocab_size, max_positions):
+    """Raises what is wrong with the first entry that has anything wrong."""
+    seen = set()
     for e in entries:
         n = len(e.tokens)
         if n == 0:
@@ -207,43 +205,59 @@ def plan_step(entries: Sequence[StepEntry], vocab_size: int = None, max_position
         if max_positions is not None and e.start + n > max_positions:
             raise RuntimeError(f"sequence {e.seq_id} would reach position {e.start + n - 1}, the model has "
                                f"{max_positions} positions")
-        if e.seq_id in seq_ids:
+        if e.seq_id in seen:
             raise ValueError(f"sequence {e.seq_id} appears twice in one step")
         toks = np.asarray(e.tokens, dtype=np.int64)
         if vocab_size is not None and (toks.min() < 0 or toks.max() >= vocab_size):
             raise ValueError(f"sequence {e.seq_id}: token ids must be in [0, {vocab_size})")
-        ids.append(toks.astype(np.int32))
-        pos.append(np.arange(e.start, e.start + n, dtype=np.int32))
-        seq.append(np.full(n, e.seq_id, dtype=np.int32))
         for w in e.want:
             if not 0 <= w < n:
                 raise ValueError(f"sequence {e.seq_id}: wanted offset {w} outside its {n} tokens")
-            want.append(base + w)
-        seq_ids.append(int(e.seq_id))
-        targets.append(int(e.start + n))
-        base += n
-    cat = (lambda xs: np.concatenate(xs) if xs else np.empty(0, dtype=np.int32))
+        seen.add(e.seq_id)
+
+
+def plan_step(entries: Sequence[StepEntry], vocab_size: int = None, max_positions: int = None) -> StepPlan:
+    """Flatten the entries in order. Checked here, on the host, so that nothing out of range reaches a kernel: token ids
+    against the vocabulary, positions against the position table, one entry per sequence.
+    The device waits for this between two decode steps, so the arrays are made whole, not entry by entry: 32 decoded tokens
+    480 -> 50 us, 3 70 -> 24 us."""
+    i32 = np.int32
+    seq_ids = [int(e.seq_id) for e in entries]
+    lens = [len(e.tokens) for e in entries]
+    starts_list = [int(e.start) for e in entries]
+    targets = [a + n for a, n in zip(starts_list, lens)]
+    base = sum(lens)
+    counts, starts = np.asarray(lens, dtype=i32), np.asarray(starts_list, dtype=i32)
+    row0 = (np.cumsum(counts) - counts).astype(i32)
+    if base == len(lens):       # one token each
+        toks = np.asarray([t for e in entries for t in e.tokens], dtype=np.int64)
+    else:
+        toks = np.concatenate([np.asarray(e.tokens, dtype=np.int64) for e in entries])
+    want, wants_ok, at = [], True, 0
+    for e, n in zip(entries, lens):
+        for w in e.want:
+            wants_ok = wants_ok and 0 <= w < n
+            want.append(at + w)
+        at += n
+    if entries and not (wants_ok and min(lens) > 0 and min(starts_list) >= 0 and len(set(seq_ids)) == len(seq_ids)
+                        and (max_positions is None or max(targets) <= max_positions)
+                        and (vocab_size is None or (toks.min() >= 0 and toks.max() < vocab_size))):
+        _check_entries(entries, vocab_size, max_positions)
 
     def runs_of(size):
-        """(first rows, counts) of the portions cut into runs of up to `size` tokens"""
-        row0, cnt, at = [], [], 0
-        for e in entries:
-            n = len(e.tokens)
-            starts = np.arange(0, n, size, dtype=np.int32)
-            row0.append(at + starts)
-            cnt.append(np.minimum(size, n - starts).astype(np.int32))
-            at += n
-        return cat(row0), cat(cnt)
-    tile_row0, tile_cnt = runs_of(StepPlan.TILE)
-    chunk_row0, chunk_cnt = runs_of(StepPlan.CHUNK)
-    counts = np.asarray([len(e.tokens) for e in entries], dtype=np.int32)
-    starts = np.asarray([e.start for e in entries], dtype=np.int32)
-    chunks = -(-counts // StepPlan.CHUNK)
-    seq_tiles = -(-counts // StepPlan.TILE)
+        """-> (first rows, counts, first run of each portion) of the portions cut into runs of up to `size` tokens"""
+        if base == len(lens):
+            return row0, counts, row0
+        runs = -(-counts // size)
+        first = np.cumsum(runs) - runs
+        off = size * (np.arange(int(runs.sum())) - np.repeat(first, runs))      # of a run inside its portion
+        return ((np.repeat(row0, runs) + off).astype(i32), np.minimum(size, np.repeat(counts, runs) - off).astype(i32), first.astype(i32))
+    tile_row0, tile_cnt, seq_tile0 = runs_of(StepPlan.TILE)
+    chunk_row0, chunk_cnt, seq_chunk0 = runs_of(StepPlan.CHUNK)
+    tok_start = np.repeat(starts, counts)
     return StepPlan(tile_row0=tile_row0, tile_cnt=tile_cnt, seq_cnt=counts, chunk_row0=chunk_row0, chunk_cnt=chunk_cnt,
-                    seq_chunk0=(np.cumsum(chunks) - chunks).astype(np.int32),
-                    seq_tile0=(np.cumsum(seq_tiles) - seq_tiles).astype(np.int32),
-                    seq_row0=(np.cumsum(counts) - counts).astype(np.int32), tok_start=np.repeat(starts, counts),
-                    tok_state=np.zeros(base, dtype=np.int32),
+                    seq_chunk0=seq_chunk0, seq_tile0=seq_tile0, seq_row0=row0, tok_start=tok_start,
+                    tok_state=np.zeros(base, dtype=i32),
                     num_tokens=base, num_seqs=len(seq_ids), seq_ids_list=seq_ids, target_lens_list=targets,
-                    input_ids=cat(ids), tok_pos=cat(pos), tok_seq=cat(seq), want_rows=np.asarray(want, dtype=np.int32))
+                    input_ids=toks.astype(i32), tok_pos=(np.repeat(starts - row0, counts) + np.arange(base)).astype(i32),
+                    tok_seq=np.repeat(np.asarray(seq_ids, dtype=i32), counts), want_rows=np.asarray(want, dtype=i32))

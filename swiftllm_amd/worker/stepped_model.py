@@ -33,6 +33,19 @@ from .kernels.sampling import argmax_rows
 DTYPES = {"float16": torch.float16, "bfloat16": torch.bfloat16, "float32": torch.float32}
 
 
+class _PlanViews(dict):
+    """The plan's arrays inside the metadata buffer, made when one is asked for (a replayed step asks for none)."""
+
+    def __init__(self, buf: torch.Tensor, layout):
+        super().__init__()
+        self._buf, self._layout = buf, {name: (off, n) for name, off, n in layout}
+
+    def __missing__(self, name):
+        off, n = self._layout[name]
+        self[name] = view = self._buf[off:off + n]
+        return view
+
+
 class SteppedModel:
     SUPPORTED_DTYPES = tuple(DTYPES)
     CONFIG_CLASS = None         # the design's configuration class (model_config.py)
@@ -156,7 +169,7 @@ class SteppedModel:
         plan.pack_into(self._meta_host_np)
         self._meta_dev[:total].copy_(self._meta_host[:total], non_blocking=True)
         self._meta_done.record()
-        return {name: self._meta_dev[off:off + n] for name, off, n in layout}
+        return _PlanViews(self._meta_dev, layout)
 
     def _begin_state_step(self, plan: StepPlan):
         """Per-sequence state: slots for the sequences of this step, their codes into the plan."""

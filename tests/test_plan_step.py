@@ -1,0 +1,53 @@
+"""plan_step's arrays against the same arrays made entry by entry."""
+import random
+
+import numpy as np
+import pytest
+
+from swiftllm_amd.worker.batch_plan import StepEntry, StepPlan, plan_step
+
+
+def _by_entry(entries):
+    out = {name: [] for name in StepPlan.SEGMENTS}
+    at = tiles = chunks = 0
+    for e in entries:
+        n = len(e.tokens)
+        out["input_ids"] += list(e.tokens)
+        out["tok_pos"] += range(e.start, e.start + n)
+        out["tok_seq"] += [e.seq_id] * n
+        out["tok_start"] += [e.start] * n
+        out["tok_state"] += [0] * n
+        out["want_rows"] += [at + w for w in e.want]
+        out["seq_row0"].append(at)
+        out["seq_cnt"].append(n)
+        out["seq_tile0"].append(tiles)
+        out["seq_chunk0"].append(chunks)
+        for what, size in (("tile", StepPlan.TILE), ("chunk", StepPlan.CHUNK)):
+            out[what + "_row0"] += range(at, at + n, size)
+            out[what + "_cnt"] += [min(size, n - i) for i in range(0, n, size)]
+        at, tiles, chunks = at + n, tiles + -(-n // StepPlan.TILE), chunks + -(-n // StepPlan.CHUNK)
+    return out
+
+
+@pytest.mark.parametrize("lens", [[], [1], [1, 1, 1], [2, 1], [16, 17, 15, 1], [31, 32, 33, 64, 100, 1, 1]])
+def test_arrays(lens):
+    rng = random.Random(len(lens))
+    entries = [StepEntry(3 * i + 1, [rng.randrange(50) for _ in range(n)], rng.choice([0, 7, 130]), tuple(rng.sample(range(n), rng.randint(0, min(2, n)))))
+               for i, n in enumerate(lens)]
+    entries = [StepEntry(e.seq_id, np.asarray(e.tokens), e.start, e.want) if rng.random() < 0.3 else e for e in entries]
+    plan = plan_step(entries, 50, 300)
+    for name, want in _by_entry(entries).items():
+        got = getattr(plan, name)
+        assert got.dtype == np.int32 and got.tolist() == want, name
+    assert plan.num_tokens == sum(lens) and plan.num_seqs == len(lens)
+    assert plan.seq_ids_list == [e.seq_id for e in entries] and plan.target_lens_list == [e.start + len(e.tokens) for e in entries]
+
+
+def test_the_first_bad_entry_is_reported():
+    good = StepEntry(1, [3, 4], 0, (1,))
+    for bad, kind, text in ((StepEntry(2, [], 0), ValueError, "brings no tokens"), (StepEntry(2, [1], -1), ValueError, "negative start"),
+                            (StepEntry(2, [1, 2], 9), RuntimeError, "would reach position 10"), (StepEntry(1, [5], 0), ValueError, "appears twice"),
+                            (StepEntry(2, [50], 0), ValueError, r"must be in \[0, 50\)"), (StepEntry(2, [-1, 3], 0), ValueError, "must be in"),
+                            (StepEntry(2, [1], 0, (1,)), ValueError, "wanted offset 1"), (StepEntry(2, [1], 0, (-1,)), ValueError, "wanted offset -1")):
+        with pytest.raises(kind, match=text):
+            plan_step([good, bad, StepEntry(5, [], -1)], 50, 10)
