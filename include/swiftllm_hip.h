@@ -561,9 +561,9 @@ int swl_window_attn_tiles(void *out, const void *q, const void *k_cache, const v
  *                 maps over the same values: lay the maps out map-major, [map][head].
  *   out_f32       1: out is fp32 whatever dtype says of the operands.
  *   heads_per_group (tiles only; 0: all) heads handled by one workgroup when the heads are not mixed: the heads of a tile
- *                 are shared out over ceil(H / heads_per_group) workgroups. -1: the rows of a matrix-core tile are sixteen
- *                 HEADS of one token instead of sixteen tokens (requires num_tiles == num_tokens, i.e. every tile is one
- *                 token, num_kv_heads == 1, no talk, no rel): the form for decode steps of heads that share one key head.
+ *                 are shared out over ceil(H / heads_per_group) workgroups. -1: the rows of a matrix-core tile are up to
+ *                 sixteen HEADS of one token and key head instead of sixteen tokens (requires num_tiles == num_tokens, i.e.
+ *                 every tile is one token, and no talk): the form for decode steps of heads that share key heads.
  *   slopes        NULL, or fp32 [num_q_heads]: slopes[h] * (query position - key position) is taken off the (capped) score.
  *   out_dim       value columns that count (<= vdim, the row size in the pages); out rows are [num_q_heads * out_dim],
  *   out_stride    elements apart. gate (NULL: none): the result times sigmoid(gate[t * gate_stride + h * out_dim + c]).

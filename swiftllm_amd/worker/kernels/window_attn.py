@@ -232,16 +232,17 @@ def window_attention(qkv: torch.Tensor, talk: torch.Tensor, pool: torch.Tensor, 
         return out
     if tiles is not None and n >= TILES_MIN_TOKENS and tiles_supported(mixer, qkv.dtype):
         row0, cnt = tiles
-        splits = choose_key_splits(row0.shape[0], mixer, max_positions)
+        heads = talk is None and head_rows(mixer, row0, n)
+        splits = head_rows_splits(mixer, n, max_positions) if heads else choose_key_splits(row0.shape[0], mixer, max_positions)
         scratch = None
         if splits > 1:
             scratch = _split_scratch(qkv.device, splits * n * mixer.num_q_heads * (mixer.value_dim + 2))
-        _hip.call("swl_window_attn_tiles", _hip.ptr(out), _hip.ptr(qkv), pool.data_ptr() + pool_slice.k_offset * esize,
+        _hip.call("swl_masked_attn_tiles", _hip.ptr(out), _hip.ptr(qkv), pool.data_ptr() + pool_slice.k_offset * esize,
                   pool.data_ptr() + pool_slice.v_offset * esize, _hip.ptr(block_table), _hip.ptr(tok_seq),
                   _hip.ptr(tok_pos), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(talk), _hip.ptr(rel), rel_len, row0.shape[0],
-                  mixer.num_q_heads,
-                  mixer.num_kv_heads, mixer.head_dim, mixer.value_dim, qkv.stride(0), mixer.window, float(mixer.scale),
-                  float(mixer.softcap), block_table.shape[1], pool.shape[1], splits, _hip.ptr(scratch), n,
+                  mixer.num_q_heads, mixer.num_kv_heads, mixer.head_dim, mixer.value_dim, qkv.stride(0), mixer.window,
+                  float(mixer.scale), float(mixer.softcap), block_table.shape[1], pool.shape[1], splits, _hip.ptr(scratch), n,
+                  MASK_WINDOW, 0, mixer.num_kv_heads, 0, -1 if heads else 0, 0, mixer.value_dim, out.stride(0), 0, 0,
                   _hip.dtype_code(qkv.dtype), _hip.stream())
         return out
     splits, scratch = token_key_splits(n, mixer.num_q_heads, mixer.value_dim, mixer, max_positions, qkv.device)
@@ -307,8 +308,21 @@ def served_row_sizes(dim: int, vdim: int, dtype: torch.dtype):
     return _row_sizes[key]
 
 
-# From this many heads over one shared key head on, a step of single tokens runs with the heads on the matrix-core tile's rows
+# From this many heads over a key head on, a step of single tokens runs with the heads on the matrix-core tile's rows
 HEAD_ROWS_MIN_HEADS = 2
+# One-wave workgroups: eight a CU. 32 requests at 1k keys, 4 layers: 636 us a step with tokens as rows (four-wave workgroups), 608, 575, 565,
+# 580 us at 2, 4, 8, 16 a CU; 2 requests at 1.9k keys 546 against 495 to 504 us.
+HEAD_ROWS_SLOTS = 8 * _NUM_CUS
+
+
+def head_rows(spec, row0: torch.Tensor, n: int) -> bool:
+    """Whether every tile is one token (a decode step) and enough heads read a key head: the tile's rows are then the heads."""
+    return row0.shape[0] == n and spec.num_q_heads >= HEAD_ROWS_MIN_HEADS * spec.num_kv_heads
+
+
+def head_rows_splits(spec, n: int, max_positions: int) -> int:
+    groups = spec.num_kv_heads * -(-spec.num_q_heads // spec.num_kv_heads // 16)
+    return choose_key_splits(n * groups, spec, max_positions, slots=HEAD_ROWS_SLOTS)
 
 
 def choose_heads_per_group(spec: AttentionSpec) -> int:
@@ -349,10 +363,8 @@ def masked_attention(q: torch.Tensor, pool: torch.Tensor, pool_slice: PoolSlice,
         return out
     if tiles is not None and wide_ok and masked_tiles_supported(spec, q.dtype):
         row0, cnt = tiles
-        if spec.num_kv_heads == 1 and row0.shape[0] == n and spec.num_q_heads >= HEAD_ROWS_MIN_HEADS:
-            # every tile is one token (a decode step) and all heads read one key head: the tile's rows are the heads
-            hpg, groups = -1, -(-spec.num_q_heads // 16)
-            splits = choose_key_splits(row0.shape[0] * groups, spec, max_positions, slots=4 * _NUM_CUS)   # (one-wave workgroups)
+        if head_rows(spec, row0, n):
+            hpg, splits = -1, head_rows_splits(spec, n, max_positions)
         else:
             hpg = choose_heads_per_group(spec)
             groups = -(-spec.num_q_heads // hpg)
