@@ -741,6 +741,10 @@ int swl_gated_add_rmsnorm(float *x, const void *m, const void *m2, const void *m
                           const void *r, int64_t r_stride, const float *r_bias, const float *w1, void *out, const float *w2,
                           const int32_t *row_idx, float eps, int64_t num_rows, int32_t width, int32_t dtype,
                           swl_stream_t stream);
+/* The same with m as `parts` fp32 slabs [num_rows, width] that are summed in order (16-byte aligned; width % 4 == 0, at most 8192). */
+int swl_gated_add_rmsnorm_parts(float *x, const float *slabs, int32_t parts, const void *m2, const void *m2_gate, int64_t m2_gate_stride,
+                                const void *r, int64_t r_stride, const float *r_bias, const float *w1, void *out, const float *w2,
+                                float eps, int64_t num_rows, int32_t width, int32_t dtype, swl_stream_t stream);
 int swl_causal_conv_state(void *out, int64_t out_stride, const void *h, int64_t h_stride, const float *w, float *state,
                           int64_t slot_stride, int64_t tail_off, const int32_t *tok_pos, const int32_t *tok_start,
                           const int32_t *tok_state, const int32_t *tok_seq, int64_t num_tokens, int32_t channels,

@@ -513,10 +513,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(T *__restrict__ out,
         const int m = static_cast<int>(it / n4);
         const int c = static_cast<int>(it - static_cast<int64_t>(m) * n4);
         float4_t s = {0.f, 0.f, 0.f, 0.f};
-        for (int k = 0; k < KS; ++k) {
-            const float4_t v = *reinterpret_cast<const float4_t *>(
-                slabs + (static_cast<int64_t>(k) * M + m) * N + 4 * c);
-            s += v;
+        const float *p = slabs + static_cast<int64_t>(m) * N + 4 * c;
+        for (int k = 0; k < KS; k += 4) {       // (four slabs requested together: one behind the other's sum is a memory latency each)
+            float4_t v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const float4_t *>(p + static_cast<int64_t>(min(k + u, KS - 1)) * M * N);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (k + u < KS) s += v[u];
         }
         typedef T vec4 __attribute__((ext_vector_type(4)));
         vec4 o;

@@ -6,6 +6,8 @@
 //       y  *= sigmoid(r + r_bias)              element-wise gate on the result
 //       x  += y / rms(y) * w1                  into the fp32 stream
 //       out = x / rms(x) * w2                  the next sublayer's input (or, with row_idx, the norm of selected rows only)
+//     m may come as the fp32 slabs of a product whose K was split over workgroups (swl_gated_add_rmsnorm_parts): the launch that would
+//     add them up is saved, and their rounding to the compute dtype with it.
 //     Statistics, gates and the sum are fp32; m, m2, s, r and out are the compute dtype. Weights arrive as the factor itself
 //     (a loader that stores "weight around zero" adds the one).
 //   swl_post_norm_add: the same step for models whose sublayers read the stream itself (norm on the sublayer's RESULT only):
@@ -82,7 +84,7 @@ __global__ __launch_bounds__(kRsThreads) void gated_add_rmsnorm_kernel(
 
 template <typename T, int TPR, int NV>
 __global__ __launch_bounds__(kRowThreads) void gated_add_rmsnorm_wide_kernel(
-    float *x, const T *m, const T *m2, const T *m2_gate, int64_t m2_gate_stride, const T *r, int64_t r_stride,
+    float *x, const T *m, const float *slabs, int parts, int64_t slab_stride, const T *m2, const T *m2_gate, int64_t m2_gate_stride, const T *r, int64_t r_stride,
     const float *r_bias, const float *w1, T *out, const float *w2, const int32_t *row_idx, float eps, int64_t rows, int width) {
     __shared__ float red[2][kRowThreads / 64];
     const int64_t id = static_cast<int64_t>(blockIdx.x) * (kRowThreads / TPR) + threadIdx.x / TPR, o = min(id, rows - 1);
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(kRowThreads) void gated_add_rmsnorm_wide_kernel(
         for (int e = 0; e < 4; ++e) v[j][e] = 0.f;
         if (c0 + 4 * TPR * j < width) row_load<float>(v[j], xr + c0 + 4 * TPR * j);
     }
-    if (m) {
+    if (m || slabs) {
         float y[NV][4], a2[NV][4], rv[NV][4];
         const float s2 = m2 ? sigmoidf_(to_f(m2_gate[t * m2_gate_stride])) : 0.f;
 #pragma unroll
@@ -106,11 +108,12 @@ __global__ __launch_bounds__(kRowThreads) void gated_add_rmsnorm_wide_kernel(
 #pragma unroll
             for (int e = 0; e < 4; ++e) y[j][e] = a2[j][e] = rv[j][e] = 0.f;
             if (c < width) {
-                row_load<T>(y[j], m + t * width + c);
+                if (m) row_load<T>(y[j], m + t * width + c);
                 if (m2) row_load<T>(a2[j], m2 + t * width + c);
                 if (r) row_load<T>(rv[j], r + t * r_stride + c);
             }
         }
+        if (slabs) row_load_parts<TPR, NV>(y, slabs + t * width, c0, width, parts, slab_stride);
         float ss = 0.f;
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
@@ -367,25 +370,27 @@ inline size_t rs_lds_bytes(int width) { return (static_cast<size_t>(width) + kRs
 
 } // namespace swl
 
-extern "C" int swl_gated_add_rmsnorm(float *x, const void *m, const void *m2, const void *m2_gate, int64_t m2_gate_stride,
+static int gated_add_rmsnorm(float *x, const void *m, const float *slabs, int parts, const void *m2, const void *m2_gate, int64_t m2_gate_stride,
                                      const void *r, int64_t r_stride, const float *r_bias, const float *w1, void *out,
                                      const float *w2, const int32_t *row_idx, float eps, int64_t num_rows, int32_t width,
                                      int32_t dtype, swl_stream_t stream) {
     if (num_rows < 0 || width <= 0) return SWL_ERR_BAD_ARG;
     if (num_rows == 0) return SWL_OK;
-    if (!x || (m && !w1) || (m2 && (!m || !m2_gate)) || (r && (!m || !r_bias)) || (out && !w2) || (row_idx && m))
+    if (!x || ((m || slabs) && !w1) || (m2 && ((!m && !slabs) || !m2_gate)) || (r && ((!m && !slabs) || !r_bias)) || (out && !w2) ||
+        (row_idx && (m || slabs)))
         return SWL_ERR_BAD_ARG;
-    if (!m && !out) return SWL_OK;
+    if (!m && !slabs && !out) return SWL_OK;
     if (num_rows > 0x7fffffffLL || swl::rs_lds_bytes(width) > 64 * 1024) return SWL_ERR_UNSUPPORTED;
 #define SWL_GO(TPR, NV)                                                                                                                \
     hipLaunchKernelGGL((swl::gated_add_rmsnorm_wide_kernel<T, TPR, NV>), dim3(static_cast<unsigned>((num_rows * TPR + 255) / 256)),    \
-                       dim3(swl::kRowThreads), 0, static_cast<hipStream_t>(stream), x, static_cast<const T *>(m),                      \
-                       static_cast<const T *>(m2), static_cast<const T *>(m2_gate), m2_gate_stride, static_cast<const T *>(r),         \
+                       dim3(swl::kRowThreads), 0, static_cast<hipStream_t>(stream), x, static_cast<const T *>(m), slabs, parts,        \
+                       num_rows * width, static_cast<const T *>(m2), static_cast<const T *>(m2_gate), m2_gate_stride, static_cast<const T *>(r),         \
                        r_stride, r_bias, w1, static_cast<T *>(out), w2, row_idx, eps, num_rows, width)
     SWL_DISPATCH_DTYPE3(dtype, T, {
         const bool wide = width % 4 == 0 && width <= swl::kRowMaxWidth && r_stride % 4 == 0 && swl::row_aligned<float>(x) &&
                           swl::row_aligned<T>(m) && swl::row_aligned<T>(m2) && swl::row_aligned<T>(r) && swl::row_aligned<T>(out) &&
-                          swl::row_aligned<float>(r_bias) && swl::row_aligned<float>(w1) && swl::row_aligned<float>(w2);
+                          swl::row_aligned<float>(r_bias) && swl::row_aligned<float>(w1) && swl::row_aligned<float>(w2) && swl::row_aligned<float>(slabs);
+        if (slabs && !wide) return SWL_ERR_UNSUPPORTED;
         if (wide) {
             SWL_ROW_SHAPE(num_rows, width, SWL_GO);
             return swl::check_launch();
@@ -397,6 +402,23 @@ extern "C" int swl_gated_add_rmsnorm(float *x, const void *m, const void *m2, co
     });
 #undef SWL_GO
     return swl::check_launch();
+}
+
+extern "C" int swl_gated_add_rmsnorm(float *x, const void *m, const void *m2, const void *m2_gate, int64_t m2_gate_stride,
+                                     const void *r, int64_t r_stride, const float *r_bias, const float *w1, void *out,
+                                     const float *w2, const int32_t *row_idx, float eps, int64_t num_rows, int32_t width,
+                                     int32_t dtype, swl_stream_t stream) {
+    return gated_add_rmsnorm(x, m, nullptr, 0, m2, m2_gate, m2_gate_stride, r, r_stride, r_bias, w1, out, w2, row_idx, eps, num_rows, width,
+                             dtype, stream);
+}
+
+extern "C" int swl_gated_add_rmsnorm_parts(float *x, const float *slabs, int32_t parts, const void *m2, const void *m2_gate,
+                                           int64_t m2_gate_stride, const void *r, int64_t r_stride, const float *r_bias,
+                                           const float *w1, void *out, const float *w2, float eps, int64_t num_rows, int32_t width,
+                                           int32_t dtype, swl_stream_t stream) {
+    if (!slabs || parts < 1) return SWL_ERR_BAD_ARG;
+    return gated_add_rmsnorm(x, nullptr, slabs, parts, m2, m2_gate, m2_gate_stride, r, r_stride, r_bias, w1, out, w2, nullptr, eps, num_rows,
+                             width, dtype, stream);
 }
 
 extern "C" int swl_causal_conv_state(void *out, int64_t out_stride, const void *h, int64_t h_stride, const float *w,

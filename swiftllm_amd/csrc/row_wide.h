@@ -28,6 +28,32 @@ __device__ __forceinline__ void row_store(T *p, const float (&v)[4]) {
     *reinterpret_cast<vec4_t<T> *>(p) = x;
 }
 
+// The same columns of `parts` fp32 slabs `stride` floats apart (a product whose K was split over workgroups), added in order: the slabs of
+// a thread's columns are requested four (two, where a thread holds many columns) at a time, not one behind the other's sum.
+template <int TPR, int NV>
+__device__ __forceinline__ void row_load_parts(float (&v)[NV][4], const float *p, int c0, int width, int parts, int64_t stride) {
+    constexpr int DEEP = NV <= 2 ? 4 : 2;
+    for (int k = 0; k < parts; k += DEEP) {
+        float4_t b[DEEP][NV];
+#pragma unroll
+        for (int u = 0; u < DEEP; ++u)
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                b[u][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+                if (c0 + 4 * TPR * j < width) b[u][j] = *reinterpret_cast<const float4_t *>(p + min(k + u, parts - 1) * stride + c0 + 4 * TPR * j);
+            }
+#pragma unroll
+        for (int u = 0; u < DEEP; ++u) {
+            if (k + u < parts) {
+#pragma unroll
+                for (int j = 0; j < NV; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[j][e] = k + u ? v[j][e] + b[u][j][e] : b[u][j][e];
+            }
+        }
+    }
+}
+
 // Sum over the threads of a row; `red`: one float per wave, its own for every sum of a kernel.
 template <int TPR>
 __device__ __forceinline__ float row_sum(float v, float *red) {

@@ -4,6 +4,8 @@ import torch
 
 from swiftllm_amd import _hip
 
+from .linear import SplitKPartials
+
 
 def gated_add_rmsnorm(x: torch.Tensor, m: torch.Tensor = None, post: torch.Tensor = None, gate: torch.Tensor = None,
                       gate_bias: torch.Tensor = None, m2: torch.Tensor = None, m2_gate: torch.Tensor = None,
@@ -12,13 +14,21 @@ def gated_add_rmsnorm(x: torch.Tensor, m: torch.Tensor = None, post: torch.Tenso
     """In place on the fp32 stream x [T, width]:
         y = m (+ sigmoid(m2_gate[t]) * m2);  y *= sigmoid(gate + gate_bias);  x += y / rms(y) * post
     and returns x / rms(x) * pre in out_dtype when `pre` is given (of rows row_idx only, when given; then m must be None).
-    `gate` and `m2_gate` may be column slices of wider matrices (row stride taken from the tensor)."""
+    `gate` and `m2_gate` may be column slices of wider matrices (row stride taken from the tensor). m may be a product's SplitKPartials, whose
+    fp32 slabs are summed here."""
     _hip.require_gpu_tensor(x, "x")
     n, width = x.shape
     assert x.dtype == torch.float32 and x.is_contiguous()
     dtype = m.dtype if m is not None else out_dtype
+    if isinstance(m, SplitKPartials):
+        assert m.shape == (n, width)
+        quads = all(t is None or t.data_ptr() % (4 * t.element_size()) == 0 for t in (x, m.slabs, m2, gate, gate_bias, post, pre))
+        if width % 4 or width > 8192 or not quads or (gate is not None and gate.stride(0) % 4):
+            m = m.materialize()
+    parts = m if isinstance(m, SplitKPartials) else None
     if m is not None:
-        assert m.shape == x.shape and m.is_contiguous() and post is not None and post.dtype == torch.float32
+        assert parts is not None or (m.shape == x.shape and m.is_contiguous())
+        assert post is not None and post.dtype == torch.float32
         assert gate is None or (gate.shape == x.shape and gate.stride(1) == 1 and gate.dtype == dtype
                                 and gate_bias.dtype == torch.float32 and gate_bias.numel() == width)
         assert m2 is None or (m2.shape == x.shape and m2.is_contiguous() and m2.dtype == dtype
@@ -27,10 +37,14 @@ def gated_add_rmsnorm(x: torch.Tensor, m: torch.Tensor = None, post: torch.Tenso
     out = torch.empty((rows, width), dtype=dtype, device=x.device) if pre is not None else None
     if m is None and pre is None:
         return None
-    _hip.call("swl_gated_add_rmsnorm", _hip.ptr(x), _hip.ptr(m), _hip.ptr(m2), _hip.ptr(m2_gate),
-              m2_gate.stride(0) if m2_gate is not None else 0, _hip.ptr(gate), gate.stride(0) if gate is not None else 0,
-              _hip.ptr(gate_bias), _hip.ptr(post), _hip.ptr(out), _hip.ptr(pre), _hip.ptr(row_idx), float(eps), rows, width,
-              _hip.dtype_code3(dtype), _hip.stream())
+    rest = (_hip.ptr(m2), _hip.ptr(m2_gate), m2_gate.stride(0) if m2_gate is not None else 0, _hip.ptr(gate),
+            gate.stride(0) if gate is not None else 0, _hip.ptr(gate_bias), _hip.ptr(post), _hip.ptr(out), _hip.ptr(pre))
+    tail = (float(eps), rows, width, _hip.dtype_code3(dtype), _hip.stream())
+    if parts is not None:
+        assert row_idx is None
+        _hip.call("swl_gated_add_rmsnorm_parts", _hip.ptr(x), _hip.ptr(parts.slabs), parts.k_splits, *rest, *tail)
+    else:
+        _hip.call("swl_gated_add_rmsnorm", _hip.ptr(x), _hip.ptr(m), *rest, _hip.ptr(row_idx), *tail)
     return out
 
 

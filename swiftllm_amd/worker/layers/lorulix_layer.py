@@ -5,7 +5,7 @@ import torch
 from ..kernels.delta_rule import delta_rule_mixer
 from ..kernels.moe import moe_experts_relu2, moe_route_scores, relu_squared
 from ..kernels.window_attn import qknorm_full_and_store_kv, window_attention
-from .kekapel_layer import _project
+from .kekapel_layer import _project, _project_partials
 from swiftllm_amd import _hip
 
 
@@ -39,7 +39,7 @@ class LorulixAttention:
         else:
             attn = window_attention(qkv, None, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq, ctx.tok_pos, mx,
                                     ctx.tiles, self.max_positions, rel=self.w.rel)
-        return _project(attn, self.w.o, self.skinny), None, None
+        return _project_partials(attn, self.w.o, self.skinny), None, None
 
 
 class LorulixDelta:
@@ -54,7 +54,7 @@ class LorulixDelta:
         proj = _project(h, self.w.proj, self.skinny)
         y = delta_rule_mixer(proj, self.w.conv, self.w.a_log, self.w.dt_bias, self.w.out_norm, ctx.state, self.tail_off,
                              self.state_off, self.mixer, self.eps)
-        return _project(y, self.w.o, self.skinny), None, None
+        return _project_partials(y, self.w.o, self.skinny), None, None
 
 
 class LorulixFeedForward:
@@ -71,7 +71,7 @@ class LorulixFeedForward:
             y = torch.empty((h.shape[0], mlp.ffn_inter_dim), dtype=h.dtype, device=h.device)
             _hip.call("swl_glu_clamp", _hip.ptr(y), _hip.ptr(gu), 0, h.shape[0], mlp.ffn_inter_dim, float(mlp.limit), 0,
                       _hip.dtype_code3(h.dtype), _hip.stream())
-            return _project(y, w.down, self.skinny), None, None
+            return _project_partials(y, w.down, self.skinny), None, None
         idx, wts = moe_route_scores(h, w.router, mlp.top_k, mlp.router_scale)
         out = moe_experts_relu2(h, idx, wts, w.up, w.down)
         if w.shared_up is None:

@@ -5,7 +5,7 @@ import torch
 from ..kernels.moe import relu_squared
 from ..kernels.rope_kv import diff_head_combine, head_gate_, latent_rope_and_store_kv, rope_and_store_kv
 from ..kernels.window_attn import MASK_CHUNK, MASK_WINDOW, AttentionSpec, masked_attention
-from .kekapel_layer import _project
+from .kekapel_layer import _project, _project_partials
 from .lorulix_layer import StepContext
 
 
@@ -32,7 +32,7 @@ class RosilixDiffAttention:
                                     ctx.tiles, self.max_positions)
         gate = proj[:, w.gate_col:w.gate_col + mx.num_q_heads]
         y = diff_head_combine(maps, gate, w.lam, 1.0 - mx.diff, self.eps, mx.num_q_heads, mx.value_dim, h.dtype)
-        return _project(y, w.o, self.skinny)
+        return _project_partials(y, w.o, self.skinny)
 
 
 class RosilixLatentAttention:
@@ -65,7 +65,7 @@ class RosilixLatentAttention:
         y = torch.empty((n, H * e), dtype=h.dtype, device=h.device)
         torch.bmm(att.view(n, H, r).transpose(0, 1), w.uv_t, out=y.view(n, H, e).transpose(0, 1))
         head_gate_(y, proj[:, w.gate_col:w.gate_col + H], H, e)
-        return _project(y, w.o, self.skinny)
+        return _project_partials(y, w.o, self.skinny)
 
 
 class RosilixFeedForward:
@@ -76,4 +76,4 @@ class RosilixFeedForward:
 
     def forward(self, h: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         z = _project(h, self.w.up, self.skinny)
-        return _project(relu_squared(z, self.mlp.ffn_inter_dim), self.w.down, self.skinny)
+        return _project_partials(relu_squared(z, self.mlp.ffn_inter_dim), self.w.down, self.skinny)

@@ -60,3 +60,28 @@ def test_rows(rows, width, dtype):
     out = add_layernorm(gpu, a.cuda(), 0.3, (wc[0], wc[1]), x0.cuda(), bias.cuda(), (wc[2], wc[3]), EPS)
     want = xd + 0.3 * _ln(ad, w[:2]) + x0.double() + bias.double()
     _close(gpu, out, want, _ln(want, w[2:]), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,width,parts", [(1, 1024, 1), (5, 1028, 3), (33, 2048, 4), (7, 4096, 8), (3, 8192, 16), (200, 3000, 5), (1025, 64, 2)])
+def test_slabs_of_a_split_product(rows, width, parts, dtype):
+    """The sublayer's result as the fp32 slabs of a product whose K was split, added up here, or before where the gate is not aligned."""
+    from swiftllm_amd.worker.kernels.linear import SplitKPartials
+    from swiftllm_amd.worker.kernels.rms_stream import gated_add_rmsnorm
+    g = torch.Generator().manual_seed(rows + width)
+    slabs = torch.randn(parts, rows, width, generator=g) * parts ** -0.5
+    x, b, r, s = (torch.randn(rows, n, generator=g) for n in (width, width, width + 8, 1))
+    b, r, s = b.to(dtype), r.to(dtype), s.to(dtype)
+    w, w2, bias = 1 + 0.2 * torch.randn(width, generator=g), 1 + 0.2 * torch.randn(width, generator=g), torch.randn(width, generator=g)
+    for shift in (4, 2):
+        gpu = x.cuda()
+        out = gated_add_rmsnorm(gpu, SplitKPartials(slabs.cuda(), parts, rows, width, dtype), w.cuda(), r.cuda()[:, shift:shift + width],
+                                bias.cuda(), b.cuda(), s.cuda(), w2.cuda(), EPS)
+        m = slabs.double().sum(0)
+        y = (m + torch.sigmoid(s.double()) * b.double()) * torch.sigmoid(r.double()[:, shift:shift + width] + bias.double())
+        want = x.double() + _rms(y) * w.double()
+        if shift == 4:
+            _close(gpu, out, want, _rms(want) * w2.double(), dtype)
+        else:       # one rounding of m to its type first
+            eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+            assert (gpu.double().cpu() - want).abs().max() <= 4 * eps * max(1.0, float(want.abs().max()))
