@@ -60,24 +60,43 @@ struct ConvTail {
         }
     }
 
-    // ---- the same for 8 consecutive channels of 16-bit rows (16-byte loads; c a multiple of 8, rows 16-byte aligned) ----
+    // ---- the same for 8 consecutive channels (16-byte loads; c a multiple of 8, rows 16-byte aligned) ----
     template <typename T>
-    __device__ __forceinline__ void at8(const T *h, int64_t h_stride, int c, int q, float (&v)[8]) const {
-        if (q < 0) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = 0.f;
-        } else if (q >= start) {
-            const vec8_t<T> x = load8(h + (t - (pos - q)) * h_stride + c);
+    static __device__ __forceinline__ void row8(const T *p, float (&v)[8]) {
+        if constexpr (sizeof(T) == 2) {
+            const vec8_t<T> x = load8(p);
 #pragma unroll
             for (int j = 0; j < 8; ++j) v[j] = to_f(x[j]);
         } else {
-            const float *p = old_tail + static_cast<int64_t>(R - (start - q)) * C + c;
             const float4_t a = *reinterpret_cast<const float4_t *>(p), b = *reinterpret_cast<const float4_t *>(p + 4);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 v[j] = a[j];
                 v[4 + j] = b[j];
             }
+        }
+    }
+    template <typename T>
+    static __device__ __forceinline__ void put8(T *p, const float (&v)[8]) {
+        if constexpr (sizeof(T) == 2) {
+            vec8_t<T> x;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = to_t<T>(v[j]);
+            store8(p, x);
+        } else {
+            *reinterpret_cast<float4_t *>(p) = float4_t{v[0], v[1], v[2], v[3]};
+            *reinterpret_cast<float4_t *>(p + 4) = float4_t{v[4], v[5], v[6], v[7]};
+        }
+    }
+    template <typename T>
+    __device__ __forceinline__ void at8(const T *h, int64_t h_stride, int c, int q, float (&v)[8]) const {
+        if (q < 0) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = 0.f;
+        } else if (q >= start) {
+            row8(h + (t - (pos - q)) * h_stride + c, v);
+        } else {
+            row8(old_tail + static_cast<int64_t>(R - (start - q)) * C + c, v);
         }
     }
 
@@ -126,12 +145,49 @@ struct ConvTail {
         }
     }
 
+    // conv8 and save8 in one: up to three earlier inputs (four taps) and their weights are requested together and serve both; one behind
+    // the other's sum they are a memory latency each, and the tail's as many again. 3 tokens in fp32: 1024
+    // channels of 3 taps 8.5 -> 4.4 us (column by column before), the delta rule's 1536 of 4 taps with their norms 25 -> 8.2 us.
+    template <typename T>
+    __device__ __forceinline__ void conv_save8(const T *h, int64_t h_stride, const float *w, int c, const float (&cur)[8],
+                                               float (&a)[8]) const {
+        constexpr int MOST = 3;
+        if (R > MOST) {
+            conv8(h, h_stride, w, c, cur, a);
+            save8(h, h_stride, c, cur);
+            return;
+        }
+        float v[MOST][8], wk[MOST + 1][8];      // v[k - 1], wk[k]: the input k tokens back and its weights
+#pragma unroll
+        for (int k = 0; k <= MOST; ++k) {
+            if (k <= R) {       // (uniform, as everything but c)
+                row8(w + static_cast<int64_t>(R - k) * C + c, wk[k]);
+                if (k > 0) at8(h, h_stride, c, pos - k, v[k > 0 ? k - 1 : 0]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] = 0.f;
+#pragma unroll
+        for (int k = MOST; k >= 1; --k) {
+            if (k <= R) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) a[j] += wk[k][j] * v[k - 1][j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] += wk[0][j] * cur[j];
+        if (!last) return;
+#pragma unroll
+        for (int k = 0; k < MOST; ++k) {        // (the input k tokens back becomes entry R - 1 - k)
+            if (k < R && pos - k >= 0) put8<float>(new_tail + static_cast<int64_t>(R - 1 - k) * C + c, k == 0 ? cur : v[k > 0 ? k - 1 : 0]);
+        }
+    }
+
     // whether the 8-channel forms may be used for rows of h (and a state region) laid out like this
     template <typename T>
-    static __device__ __forceinline__ bool wide_ok(const T *h, int64_t h_stride, const float *w, const float *state,
+    static __host__ __device__ __forceinline__ bool wide_ok(const T *h, int64_t h_stride, const float *w, const float *state,
                                                    int64_t slot_stride, int64_t tail_off, int channels) {
-        if constexpr (sizeof(T) != 2) return false;
-        return (channels & 7) == 0 && (h_stride & 7) == 0 && (reinterpret_cast<uintptr_t>(h) & 15) == 0 &&
+        return (channels & 7) == 0 && (h_stride & (16 / sizeof(T) - 1)) == 0 && (reinterpret_cast<uintptr_t>(h) & 15) == 0 &&
                (reinterpret_cast<uintptr_t>(w) & 15) == 0 && (reinterpret_cast<uintptr_t>(state) & 15) == 0 &&
                (slot_stride & 3) == 0 && (tail_off & 3) == 0;
     }

@@ -36,20 +36,13 @@ __global__ __launch_bounds__(kDpThreads) void delta_prep_kernel(
     const int qk = G * d, C = 2 * qk + H * dv;
     const T *row = proj + t * proj_stride;
     const ConvTail tail(state, slot_stride, tail_off, tok_pos, tok_start, tok_state, tok_seq, num_tokens, C, taps, t);
-    bool wide = false;
-    if constexpr (sizeof(T) == 2) wide = ConvTail::wide_ok(proj, proj_stride, conv_w, state, slot_stride, tail_off, C);
-    if (wide) {
-        if constexpr (sizeof(T) == 2) {
-            for (int c = threadIdx.x * 8; c < C; c += kDpThreads * 8) {
-                const vec8_t<T> x = load8(row + c);
-                float cur[8], a[8];
+    if (ConvTail::wide_ok(proj, proj_stride, conv_w, state, slot_stride, tail_off, C)) {
+        for (int c = threadIdx.x * 8; c < C; c += kDpThreads * 8) {
+            float cur[8], a[8];
+            ConvTail::row8(row + c, cur);
+            tail.conv_save8(proj, proj_stride, conv_w, c, cur, a);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) cur[j] = to_f(x[j]);
-                tail.conv8(proj, proj_stride, conv_w, c, cur, a);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) act[c + j] = a[j] * dr_sigmoid(a[j]);
-                tail.save8(proj, proj_stride, c, cur);
-            }
+            for (int j = 0; j < 8; ++j) act[c + j] = a[j] * dr_sigmoid(a[j]);
         }
     } else {
         for (int c = threadIdx.x; c < C; c += kDpThreads) {

@@ -302,25 +302,21 @@ __global__ __launch_bounds__(kRsThreads) void causal_conv_state_kernel(
     int64_t num_tokens, int C, int taps, int add_input) {
     const int64_t t = blockIdx.x;
     const ConvTail tail(state, slot_stride, tail_off, tok_pos, tok_start, tok_state, tok_seq, num_tokens, C, taps, t);
-    if constexpr (sizeof(T) == 2) {
-        if (ConvTail::wide_ok(h, h_stride, w, state, slot_stride, tail_off, C) && (out_stride & 7) == 0 &&
-            (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-            for (int c = threadIdx.x * 8; c < C; c += kRsThreads * 8) {
-                const vec8_t<T> x = load8(h + t * h_stride + c);
-                float cur[8], a[8];
+    if (ConvTail::wide_ok(h, h_stride, w, state, slot_stride, tail_off, C) && (out_stride & (16 / sizeof(T) - 1)) == 0 &&
+        (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+        for (int c = threadIdx.x * 8; c < C; c += blockDim.x * 8) {
+            float cur[8], a[8];
+            ConvTail::row8(h + t * h_stride + c, cur);
+            tail.conv_save8(h, h_stride, w, c, cur, a);
+            if (add_input) {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) cur[j] = to_f(x[j]);
-                tail.conv8(h, h_stride, w, c, cur, a);
-                vec8_t<T> o;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) o[j] = to_t<T>(add_input ? a[j] + cur[j] : a[j]);
-                store8(out + t * out_stride + c, o);
-                tail.save8(h, h_stride, c, cur);
+                for (int j = 0; j < 8; ++j) a[j] += cur[j];
             }
-            return;
+            ConvTail::put8(out + t * out_stride + c, a);
         }
+        return;
     }
-    for (int c = threadIdx.x; c < C; c += kRsThreads) {
+    for (int c = threadIdx.x; c < C; c += blockDim.x) {
         const float cur = to_f(h[t * h_stride + c]);
         float a = tail.conv(h, h_stride, w, c, cur);
         if (add_input) a += cur;
@@ -432,8 +428,11 @@ extern "C" int swl_causal_conv_state(void *out, int64_t out_stride, const void *
     if (taps > 1 && (!state || !tok_state)) return SWL_ERR_BAD_ARG;
     if (num_tokens > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        // (a thread takes eight channels: no more waves than have some)
+        const bool wide = swl::ConvTail::wide_ok(static_cast<const T *>(h), h_stride, w, state, slot_stride, tail_off, channels);
+        const int threads = wide && channels < 8 * swl::kRsThreads ? (channels / 8 + 63) / 64 * 64 : swl::kRsThreads;
         hipLaunchKernelGGL((swl::causal_conv_state_kernel<T>), dim3(static_cast<unsigned>(num_tokens)),
-                           dim3(swl::kRsThreads), 0, static_cast<hipStream_t>(stream), static_cast<T *>(out), out_stride,
+                           dim3(static_cast<unsigned>(threads)), 0, static_cast<hipStream_t>(stream), static_cast<T *>(out), out_stride,
                            static_cast<const T *>(h), h_stride, w, state, slot_stride, tail_off, tok_pos, tok_start,
                            tok_state, tok_seq, num_tokens, channels, taps, add_input);
     });

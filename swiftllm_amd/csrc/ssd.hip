@@ -36,27 +36,17 @@ __global__ __launch_bounds__(kSsThreads) void ssd_prep_kernel(
     const T *conv_in = proj + inner;        // the convolved channels follow the gate columns
     const T *row = conv_in + t * proj_stride;
     const ConvTail tail(state, slot_stride, tail_off, tok_pos, tok_start, tok_state, tok_seq, num_tokens, C, taps, t);
-    bool wide = false;
-    if constexpr (sizeof(T) == 2) wide = ConvTail::wide_ok(conv_in, proj_stride, conv_w, state, slot_stride, tail_off, C);
-    if (wide) {
-        if constexpr (sizeof(T) == 2) {
-            for (int c = threadIdx.x * 8; c < C; c += kSsThreads * 8) {
-                const vec8_t<T> x = load8(row + c);
-                float cur[8], a[8];
+    if (ConvTail::wide_ok(conv_in, proj_stride, conv_w, state, slot_stride, tail_off, C)) {
+        for (int c = threadIdx.x * 8; c < C; c += kSsThreads * 8) {
+            float cur[8], a[8];
+            ConvTail::row8(row + c, cur);
+            tail.conv_save8(conv_in, proj_stride, conv_w, c, cur, a);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) cur[j] = to_f(x[j]);
-                tail.conv8(conv_in, proj_stride, conv_w, c, cur, a);
-                float o[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const float v = a[j] + conv_b[c + j];
-                    o[j] = v * ss_sigmoid(v);
-                }
-                float *dst = xbc + t * C + c;       // (C and c are multiples of 8: 32-byte aligned)
-                *reinterpret_cast<float4_t *>(dst) = float4_t{o[0], o[1], o[2], o[3]};
-                *reinterpret_cast<float4_t *>(dst + 4) = float4_t{o[4], o[5], o[6], o[7]};
-                tail.save8(conv_in, proj_stride, c, cur);
+            for (int j = 0; j < 8; ++j) {
+                const float v = a[j] + conv_b[c + j];
+                a[j] = v * ss_sigmoid(v);
             }
+            ConvTail::put8<float>(xbc + t * C + c, a);       // (C and c are multiples of 8: 32-byte aligned)
         }
     } else {
         for (int c = threadIdx.x; c < C; c += kSsThreads) {
