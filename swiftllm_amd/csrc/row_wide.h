@@ -71,7 +71,7 @@ __device__ __forceinline__ float row_sum(float v, float *red) {
 }
 
 template <typename T>
-inline bool row_aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & (4 * sizeof(T) - 1)) == 0; }
+__host__ __device__ inline bool row_aligned(const void *p) { return (reinterpret_cast<uintptr_t>(p) & (4 * sizeof(T) - 1)) == 0; }
 
 // Runs GO(TPR, NV) for a launch of `rows` rows: a wave (two) a row for many rows of up to 1024 (2048) columns, else a workgroup a row, which
 // ends a step of few rows sooner.
