@@ -92,6 +92,36 @@ __device__ __forceinline__ float router_dot(const float *x, const float *w, int 
     return wave_allreduce_sum(a);
 }
 
+// Arg-max over an LDS array of n floats for the whole wave (ties: the lowest index; NaN, -inf and taken entries never win: 0x7fffffff).
+// A lane scans entries lane, lane + 64, ...; the exchange is a chain of LDS latencies, so up to eight entries take three steps, not six.
+__device__ __forceinline__ void wave_argmax(const float *v, int n, int lane, float &best, int &besti) {
+    best = -INFINITY;
+    besti = 0x7fffffff;
+    for (int e = lane; e < n; e += 64) {
+        if (v[e] > best) {      // strict: keeps the lowest id among a lane's equals
+            best = v[e];
+            besti = e;
+        }
+    }
+    auto exchange = [&](int m) {
+        const float ob = __shfl_xor(best, m, 64);
+        const int oi = __shfl_xor(besti, m, 64);
+        if (ob > best || (ob == best && oi < besti)) {
+            best = ob;
+            besti = oi;
+        }
+    };
+    if (n > 8) {
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) exchange(m);
+        return;
+    }
+#pragma unroll
+    for (int m = 4; m >= 1; m >>= 1) exchange(m);
+    best = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(best)));
+    besti = __builtin_amdgcn_readfirstlane(besti);
+}
+
 // act 0: g' = min(g, limit), u' = clamp(u, +-limit), g' sigmoid(1.702 g') (u' + 1); act 1: silu(g) u; act 2: silu(u) g
 __device__ __forceinline__ float gated_unit(float g, float u, float limit, int act) {
     if (act == 1) return g / (1.0f + expf(-g)) * u;
@@ -127,39 +157,39 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_kernel(int32_t *idx_out
         all_den = wave_allreduce_sum(all_den);
     }
     // top-k by repeated arg-max over the wave (each lane scans experts lane, lane + 64, ...)
-    float chosen_max = 0.f, denom = 0.f;
+    // Latency bounds the choice. Lane j keeps the j-th one until the sum is known: a store to global memory in the loop is waited for at
+    // every fence. With the shorter exchange, 3663 tokens of 2048, two of eight experts, bf16: 12.8 to 11.3 us, in groups 15.4 to 13.3;
+    // six or eight of 64 or 128 experts: 1 to 4 % less.
+    float chosen_max = 0.f, denom = 0.f, mine = 0.f;
+    int mine_idx = 0;
     for (int j = 0; j < top; ++j) {
-        float best = -INFINITY;
-        int besti = 0x7fffffff;
-        for (int e = lane; e < experts; e += 64) {
-            const float v = logit[e];
-            if (v > best) {     // strict: keeps the lowest id among a lane's equals (NaN / taken entries never win)
-                best = v;
-                besti = e;
-            }
-        }
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) {
-            const float ob = __shfl_xor(best, m, 64);
-            const int oi = __shfl_xor(besti, m, 64);
-            if (ob > best || (ob == best && oi < besti)) {
-                best = ob;
-                besti = oi;
-            }
-        }
+        float best;
+        int besti;
+        wave_argmax(logit, experts, lane, best, besti);
         if (j == 0) chosen_max = all_scores ? all_max : best;
         const float pj = expf(best - chosen_max);
         denom += pj;
+        if (lane == j) {
+            mine = pj;
+            mine_idx = besti;
+        }
         if (lane == 0) {
-            idx_out[t * top + j] = besti;
-            w_out[t * top + j] = pj;
+            if (top > 64) {     // (more choices than lanes)
+                idx_out[t * top + j] = besti;
+                w_out[t * top + j] = pj;
+            }
             logit[besti] = -INFINITY;
         }
         __builtin_amdgcn_wave_barrier();
         __threadfence_block();
     }
-    if (lane == 0) {
-        const float mult = all_scores ? scale / all_den : 1.0f / denom;
+    const float mult = all_scores ? scale / all_den : 1.0f / denom;
+    if (top <= 64) {
+        if (lane < top) {
+            idx_out[t * top + lane] = mine_idx;
+            w_out[t * top + lane] = mine * mult;
+        }
+    } else if (lane == 0) {
         for (int j = 0; j < top; ++j) w_out[t * top + j] *= mult;
     }
 }
@@ -190,26 +220,6 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_grouped_kernel(int32_t 
     }
     __syncthreads();
     if (wave != 0) return;
-    // arg-max over an LDS array of n floats for the whole wave (ties: the lowest index; -inf never wins)
-    auto argmax = [&](const float *v, int n, float &best, int &besti) {
-        best = -INFINITY;
-        besti = 0x7fffffff;
-        for (int e = lane; e < n; e += 64) {
-            if (v[e] > best) {
-                best = v[e];
-                besti = e;
-            }
-        }
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) {
-            const float ob = __shfl_xor(best, m, 64);
-            const int oi = __shfl_xor(besti, m, 64);
-            if (ob > best || (ob == best && oi < besti)) {
-                best = ob;
-                besti = oi;
-            }
-        }
-    };
     if (count > 1 && keep < count) {
         const int per = experts / count;
         for (int g = lane; g < count; g += 64) {    // a group's score: its two largest choice scores (one, in groups of one)
@@ -233,7 +243,7 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_grouped_kernel(int32_t 
         for (int j = 0; j < keep; ++j) {
             float best;
             int besti;
-            argmax(gscore, count, best, besti);
+            wave_argmax(gscore, count, lane, best, besti);
             if (lane == 0 && besti < count) {
                 gscore[besti] = -INFINITY;      // (taken)
                 gkeep[besti] = 1.f;
@@ -246,24 +256,36 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_grouped_kernel(int32_t 
         __builtin_amdgcn_wave_barrier();
         __threadfence_block();
     }
-    float denom = 0.f;
+    float denom = 0.f, mine = 0.f;      // (lane j keeps the j-th choice, as above)
+    int mine_idx = 0;
     for (int j = 0; j < top; ++j) {
         float best;
         int besti;
-        argmax(choice, experts, best, besti);
+        wave_argmax(choice, experts, lane, best, besti);
         if (besti >= experts) besti = 0;        // (fewer eligible experts than `top`: cannot happen for keep * per >= top)
         const float sc = score[besti];
         denom += sc;
+        if (lane == j) {
+            mine = sc;
+            mine_idx = besti;
+        }
         if (lane == 0) {
-            idx_out[t * top + j] = besti;
-            w_out[t * top + j] = sc;
+            if (top > 64) {
+                idx_out[t * top + j] = besti;
+                w_out[t * top + j] = sc;
+            }
             choice[besti] = -INFINITY;
         }
         __builtin_amdgcn_wave_barrier();
         __threadfence_block();
     }
-    if (lane == 0) {
-        const float mult = normalize ? 1.0f / (denom + 1e-20f) : 1.0f;
+    const float mult = normalize ? 1.0f / (denom + 1e-20f) : 1.0f;
+    if (top <= 64) {
+        if (lane < top) {
+            idx_out[t * top + lane] = mine_idx;
+            w_out[t * top + lane] = mine * mult;
+        }
+    } else if (lane == 0) {
         for (int j = 0; j < top; ++j) w_out[t * top + j] *= mult;
     }
 }
