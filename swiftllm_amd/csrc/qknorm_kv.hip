@@ -21,7 +21,7 @@ __global__ __launch_bounds__(kQkThreads) void qknorm_store_kv_kernel(
     T *qkv, const float *q_w, const float *k_w, T *k_cache, T *v_cache, const int32_t *block_table,
     const int32_t *tok_seq, const int32_t *tok_pos, int H, int G, int d, int dv, int64_t tok_stride,
     int max_blocks_per_seq, int64_t block_stride, float eps, int store) {
-    const int64_t t = blockIdx.x;
+    const int64_t t = page_token();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     T *row = qkv + t * tok_stride;
     const int pos = tok_pos[t];
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(kQkThreads) void qknorm_full_store_kv_kernel(
     const int32_t *tok_seq, const int32_t *tok_pos, int H, int G, int d, int dv, int64_t tok_stride,
     int max_blocks_per_seq, int64_t block_stride, float eps, float temp_coef, int temp_every, int store) {
     __shared__ float red[2][kQkThreads / 64];
-    const int64_t t = blockIdx.x;
+    const int64_t t = page_token();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     T *row = qkv + t * tok_stride;
     const int pos = tok_pos[t];
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kQkThreads) void qkv_bias_norm_store_kernel(
     int64_t v_other_stride, float mix, T *k_cache, T *v_cache, const int32_t *block_table, const int32_t *tok_seq,
     const int32_t *tok_pos, int H, int G, int d, int dv, int64_t tok_stride, int max_blocks_per_seq, int64_t block_stride,
     float eps, int store) {
-    const int64_t t = blockIdx.x;
+    const int64_t t = page_token();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     T *row = qkv + t * tok_stride;
     const int pos = tok_pos[t];

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(kRkThreads) void rope_store_kv_kernel(
     const int32_t *tok_pos, int nq, int nk, int nv, int d, int dv, int rot_dims, int64_t tok_stride, int max_blocks_per_seq,
     int64_t block_stride) {
     __shared__ float cs[kRkMaxPairs], sn[kRkMaxPairs];
-    const int64_t t = blockIdx.x;
+    const int64_t t = page_token();
     const int pos = tok_pos[t];
     const int pairs = rot_dims >> 1;
     rk_angles(cs, sn, freq, pos, pairs);
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(kRkThreads) void qk_norm_rope_store_kv_kernel(
     int nk, int nv, int d, int dv, int rot_dims, int half, double rot_mult, int64_t tok_stride, int64_t q_out_stride, int k_dim,
     int v_dim, int keys_as_values, int max_blocks_per_seq, int64_t block_stride, float eps) {
     __shared__ float cs[kRkMaxPairs], sn[kRkMaxPairs];
-    const int64_t t = blockIdx.x;
+    const int64_t t = page_token();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int pos = tok_pos[t];
     const int pairs = rot_dims >> 1;
@@ -274,7 +274,7 @@ __global__ __launch_bounds__(kRkThreads) void qkv_conv_rope_store_kv_kernel(
     int64_t num_tokens, int nq, int nk, int d, int dv, int k_dim, int v_dim, float eps) {
     extern __shared__ float act[];      // [(nq + nk) d + nk dv] biased, convolved channels; then [nq + nk] the heads' 1 / rms
     __shared__ float cs[kRkMaxPairs], sn[kRkMaxPairs];
-    const int64_t t = blockIdx.x;
+    const int64_t t = page_token();
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int pos = tok_pos[t];
     const int pairs = rot_dims >> 1, heads = nq + nk, C = heads * d + nk * dv;
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(kRkThreads) void latent_rope_store_kv_kernel(
     int v_dim) {
     __shared__ float cs[kRkMaxPairs], sn[kRkMaxPairs];
     __shared__ float red[kRkThreads / 64];
-    const int64_t t = blockIdx.x;
+    const int64_t t = page_token();
     const int pos = tok_pos[t];
     const int pairs = dr >> 1;
     rk_angles(cs, sn, freq, pos, pairs, rot_mult);

@@ -1,0 +1,54 @@
+"""Stores into transposed pages whose workgroups take their tokens in groups of 128 (csrc/swl_common.h, page_token): a step around the
+edges of a group leaves the rows and the pool that the same tokens leave in steps below 128, which keep the grid's order."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+H, G, D = 3, 2, 64
+
+
+def _kernels():
+    from swiftllm_amd.worker.kernels import rope_kv, window_attn as wa
+    g = torch.Generator().manual_seed(5)
+    w = {n: torch.randn(n, generator=g).cuda() for n in (H * D, G * D, D)}
+    freq = (10000.0 ** (-torch.arange(0, D, 2, dtype=torch.float64) / D)).cuda()
+    mixer = SimpleNamespace(num_q_heads=H, num_kv_heads=G, head_dim=D, value_dim=D, q_size=H * D, k_size=G * D, v_size=G * D,
+                            q_temp_coef=0.1, q_temp_every=16)
+    rot = SimpleNamespace(dims=D, half=True, multiplier=1.0)
+    latent = SimpleNamespace(num_q_heads=1, head_dim=D, rot_dim=D, kv_rank=2 * D, rot=rot)
+
+    def from_latent(x, *to):
+        qa = torch.zeros(x.shape[0], 3 * D, dtype=x.dtype, device="cuda")
+        rope_kv.latent_rope_and_store_kv(x, qa, freq, w[G * D], *to, latent, 2 * D, 1e-6)
+        return qa
+
+    return {"qknorm": lambda x, *to: wa.qknorm_and_store_kv(x, w[D], w[D], *to, mixer, 1e-6),
+            "qknorm_full": lambda x, *to: wa.qknorm_full_and_store_kv(x, w[H * D], w[G * D], *to, mixer, 1e-6, True),
+            "bias_norm": lambda x, *to: wa.qkv_bias_norm_store(x, w[H * D], w[G * D], w[G * D], w[D], None, *to, mixer, 1e-6),
+            "rope": lambda x, *to: rope_kv.rope_and_store_kv(x, freq, D, *to, H, G, G, D, D),
+            "qk_norm_rope": lambda x, *to: rope_kv.qk_norm_rope_and_store_kv(x, None, None, w[D], w[D], None, freq, rot, *to, H, G, G, D, D, 1e-6),
+            "latent": from_latent}
+
+
+@pytest.mark.parametrize("tokens", [127, 128, 129, 255, 256, 300])
+@pytest.mark.parametrize("name", ["qknorm", "qknorm_full", "bias_norm", "rope", "qk_norm_rope", "latent"])
+def test_same_pool(name, tokens):
+    from swiftllm_amd.worker.kernels.window_attn import PoolSlice
+    run, g = _kernels()[name], torch.Generator().manual_seed(tokens)
+    rows = torch.randn(tokens, (H + 2 * G) * D, generator=g).to(torch.bfloat16).cuda()
+    first = tokens // 3                 # two sequences, the second from the middle of a page on
+    seq = torch.tensor([0] * first + [1] * (tokens - first), dtype=torch.int32, device="cuda")
+    pos = torch.cat([torch.arange(first), 7 + torch.arange(tokens - first)]).int().cuda()
+    table = torch.randperm(64, generator=g)[:2 * 21].view(2, 21).int().cuda()
+    results = []
+    for step in (tokens, 100):
+        x, pool, made = rows.clone(), torch.zeros(64, 2 * G * D * 16 + D * 16, dtype=torch.bfloat16, device="cuda"), []
+        for a in range(0, tokens, step):
+            part = x[a:a + step]
+            made.append(run(part, pool, PoolSlice(0, 3 * D * 16 if name == "latent" else G * D * 16), table, seq[a:a + step], pos[a:a + step]))
+        results.append([x, pool] + ([torch.cat(made)] if made[0] is not None else []))
+    assert results[0][1].any()
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
