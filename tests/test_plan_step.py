@@ -51,3 +51,21 @@ def test_the_first_bad_entry_is_reported():
                             (StepEntry(2, [1], 0, (1,)), ValueError, "wanted offset 1"), (StepEntry(2, [1], 0, (-1,)), ValueError, "wanted offset -1")):
         with pytest.raises(kind, match=text):
             plan_step([good, bad, StepEntry(5, [], -1)], 50, 10)
+
+
+@pytest.mark.parametrize("bad,kind,text", [
+    (StepEntry(2, [1], 1 << 40), RuntimeError, "would reach position"), (StepEntry(2, [1], -(1 << 40)), ValueError, "negative start"),
+    (StepEntry(2, [1 << 63], -1), ValueError, "negative start"), (StepEntry(2, [1 << 63], 0), OverflowError, ""),
+    (StepEntry(1 << 40, [1], 0, (3,)), OverflowError, ""), (StepEntry(2, [1 << 40], 0), ValueError, r"must be in \[0, 50\)")])
+def test_values_beyond_32_bits(bad, kind, text):
+    """What no int32 holds is refused with the error that the entry's other faults get, the first bad entry's."""
+    with pytest.raises(kind, match=text):
+        plan_step([StepEntry(1, [3, 4], 0, (1,)), bad, StepEntry(5, [], -1)], 50, 10)
+
+
+def test_positions_end_with_32_bits():
+    """Without a position table the last position is 2^31 - 1: a portion that passes it is refused, not wrapped round."""
+    assert plan_step([StepEntry(1, [3, 4], (1 << 31) - 2)]).tok_pos.tolist() == [(1 << 31) - 2, (1 << 31) - 1]
+    for start in ((1 << 31) - 1, 1 << 31):
+        with pytest.raises(OverflowError):
+            plan_step([StepEntry(1, [3, 4], start)])
