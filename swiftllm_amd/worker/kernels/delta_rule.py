@@ -15,6 +15,13 @@ TILES_MIN_PORTION = 48
 TILES_MAX_SCRATCH = 1 << 30
 
 
+def most_tiles_scratch(num_tokens: int, portions: int, mixer) -> int:
+    """The most scratch (bytes) that the walk by tiles takes for a step of these sizes, however the tokens are shared out."""
+    tiles = num_tokens // 16 + min(portions, num_tokens)        # (every portion may end in a part of one)
+    need = _hip.load().swl_delta_rule_tiles_scratch_bytes(tiles, mixer.num_heads, mixer.head_dim, mixer.value_dim)
+    return min(need, TILES_MAX_SCRATCH)
+
+
 def delta_rule_mixer(proj: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
                      norm_w: torch.Tensor, st: StateRef, tail_off: int, state_off: int, mixer, eps: float) -> torch.Tensor:
     """proj [T, q | k | v | gate | b | a] (one fused projection) -> [T, heads * vdim] in proj's dtype: short convolutions

@@ -40,7 +40,7 @@ def sigmoid_attention(q: torch.Tensor, pool: torch.Tensor, pool_slice: PoolSlice
     if tiles is not None and wide_ok and tiles_supported(mixer, q.dtype):
         row0, cnt = tiles
         splits = choose_key_splits(row0.shape[0], mixer, max_positions)
-        scratch = share_scratch(q.device, splits, n * H * mixer.value_dim)
+        splits, scratch = share_scratch(q.device, splits, n * H * mixer.value_dim)
         _hip.call("swl_sigmoid_attn_tiles", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq),
                   _hip.ptr(tok_pos), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(talk), _hip.ptr(r1), _hip.ptr(r2), _hip.ptr(pb),
                   row0.shape[0], H, mixer.num_kv_heads, mixer.head_dim, mixer.value_dim, q.stride(0), mixer.window,

@@ -131,7 +131,7 @@ def _span_launch(q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles, H, 
     groups = max(1, n * H // (128 * G)) * G
     pages = (min(window, tiles.longest) if window > 0 else tiles.longest) // 16 + 1
     splits = max(1, min(2 * _NUM_CUS // groups, pages // 8, 8))
-    scratch = share_scratch(q.device, splits, n * H * (vdim + 2))
+    splits, scratch = share_scratch(q.device, splits, n * H * (vdim + 2))
     _hip.call("swl_span_attn", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq), _hip.ptr(tok_pos),
               _hip.ptr(start), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(rel), rel.shape[1] if rel is not None else 0, row0.shape[0],
               H, G, GV, dim, vdim, q.stride(0), window, mask_kind, float(scale), float(softcap), block_table.shape[1], pool.shape[1],
@@ -147,11 +147,17 @@ TILES_MIN_TOKENS = 1
 _NUM_CUS = 256
 
 
+# A launch takes fewer shares rather than more scratch than this (which memory profiling sets aside: its step runs without a pool).
+# The rules ask for 137 MiB at 512 value columns and 34 MiB at 128; only per-token steps of more than 64k value columns a token meet it.
+SHARE_MAX_SCRATCH = 256 << 20
+
+
 def share_scratch(device, splits: int, floats: int):
-    """fp32 scratch of `floats` per key share (None for one share), of this call alone: the launch that fills it and the one that combines it
-    run on the caller's stream, where the allocator hands the memory on afterwards; a captured graph keeps it in its own pool. (A buffer
-    kept per device would be shared by the streams and threads that launch attention at the same time.)"""
-    return torch.empty(splits * floats, dtype=torch.float32, device=device) if splits > 1 else None
+    """-> (key shares, their fp32 scratch of `floats` each; None for one share), of this call alone: the launch that fills it and the one that
+    combines it run on the caller's stream, where the allocator hands the memory on afterwards; a captured graph keeps it in its own
+    pool. (A buffer kept per device would be shared by the streams and threads that launch attention at the same time.)"""
+    splits = max(1, min(splits, SHARE_MAX_SCRATCH // (4 * max(floats, 1))))
+    return splits, torch.empty(splits * floats, dtype=torch.float32, device=device) if splits > 1 else None
 
 
 def choose_key_splits(num_tiles: int, mixer, max_positions: int, slots: int = _NUM_CUS) -> int:
@@ -167,7 +173,7 @@ def token_key_splits(n: int, heads: int, vdim: int, mixer, max_positions: int, d
     """Key shares of the per-token kernels (and their scratch): up to 16 while they leave at most four workgroups a CU — a chunk of 64
     keys is a chain of some microseconds, and a step of few tokens has nothing else to fill the chip with."""
     splits = choose_key_splits(n, mixer, max_positions, slots=4 * _NUM_CUS)
-    return splits, share_scratch(device, splits, n * heads * (vdim + 2))
+    return share_scratch(device, splits, n * heads * (vdim + 2))
 
 
 def mix_launch(entry, q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles, mixer, vectors, extra, floats) -> bool:
@@ -185,7 +191,7 @@ def mix_launch(entry, q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles
     # the registers allow one workgroup a CU: with fewer tiles than CUs, every tile's keys are shared out (at 2 and 4 workgroups a CU a
     # step of 1.4 thousand tokens at 16 heads of 128 gets no faster and 9 % slower: each has its own prologue and partial results)
     splits = choose_key_splits(row0.shape[0], mixer, tiles.longest)
-    scratch = share_scratch(q.device, splits, n * H * floats)
+    splits, scratch = share_scratch(q.device, splits, n * H * floats)
     _hip.call(entry, _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq), _hip.ptr(tok_pos),
               _hip.ptr(row0), _hip.ptr(cnt), *[_hip.ptr(t) for t in vectors], row0.shape[0], H, mixer.num_kv_heads, mixer.head_dim,
               mixer.value_dim, q.stride(0), mixer.window, float(mixer.scale), *extra, block_table.shape[1], pool.shape[1], splits,
@@ -229,7 +235,7 @@ def window_attention(qkv: torch.Tensor, talk: torch.Tensor, pool: torch.Tensor, 
         row0, cnt = tiles
         heads = talk is None and head_rows(mixer, row0, n)
         splits = head_rows_splits(mixer, n, max_positions) if heads else choose_key_splits(row0.shape[0], mixer, max_positions)
-        scratch = share_scratch(qkv.device, splits, n * mixer.num_q_heads * (mixer.value_dim + 2))
+        splits, scratch = share_scratch(qkv.device, splits, n * mixer.num_q_heads * (mixer.value_dim + 2))
         _hip.call("swl_masked_attn_tiles", _hip.ptr(out), _hip.ptr(qkv), pool.data_ptr() + pool_slice.k_offset * esize,
                   pool.data_ptr() + pool_slice.v_offset * esize, _hip.ptr(block_table), _hip.ptr(tok_seq),
                   _hip.ptr(tok_pos), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(talk), _hip.ptr(rel), rel_len, row0.shape[0],
@@ -362,7 +368,7 @@ def masked_attention(q: torch.Tensor, pool: torch.Tensor, pool_slice: PoolSlice,
             hpg = choose_heads_per_group(spec)
             groups = -(-spec.num_q_heads // hpg)
             splits = choose_key_splits(row0.shape[0] * groups, spec, max_positions)
-        scratch = share_scratch(q.device, splits, n * spec.num_q_heads * (spec.value_dim + 2))
+        splits, scratch = share_scratch(q.device, splits, n * spec.num_q_heads * (spec.value_dim + 2))
         _hip.call("swl_masked_attn_tiles", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq),
                   _hip.ptr(tok_pos), _hip.ptr(row0), _hip.ptr(cnt), 0, 0, 0, row0.shape[0], spec.num_q_heads,
                   spec.num_kv_heads, spec.head_dim, spec.value_dim, q.stride(0), spec.window, float(spec.scale),

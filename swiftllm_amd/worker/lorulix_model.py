@@ -21,6 +21,7 @@ import torch
 from swiftllm_amd.engine_config import EngineConfig
 from swiftllm_amd.model_config import LorulixModelConfig
 
+from .kernels.delta_rule import most_tiles_scratch
 from .kernels.layernorm import embed_positions
 from .kernels.linear import pack_weight, packable
 from .kernels.rms_stream import StateRef, causal_conv_state, gated_add_rmsnorm
@@ -61,6 +62,10 @@ class LorulixModel(SteppedModel):
             if layer.type == "attention" and layer.mixer.kv_from >= 0:
                 self.pool_slices[i] = self.pool_slices[layer.mixer.kv_from]
         self.block_elems = max(off, 8)      # (a model without attention layers still has a block table)
+
+    def _scratch_bytes(self, num_tokens: int, batch: int) -> int:
+        return max([super()._scratch_bytes(num_tokens, batch)] +
+                   [most_tiles_scratch(num_tokens, batch, c.mixer) for c in self.model_config.layers if c.type == "delta"])
 
     def _build(self):
         cfg, ecfg = self.model_config, self.engine_config

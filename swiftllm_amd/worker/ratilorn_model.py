@@ -23,6 +23,7 @@ from swiftllm_amd.model_config import RatilornModelConfig
 
 from .kernels.layernorm import embed_positions
 from .kernels.linear import pack_weight, packable
+from .kernels.linear_scan import SEGMENT_MAX_SCRATCH
 from .kernels.rms_stream import StateRef, gated_add_rmsnorm, post_norm_add
 from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import _project
@@ -60,6 +61,9 @@ class RatilornModel(SteppedModel):
             off += mx.v_size * bs
             off += -off % 8         # every slice starts on a 16-byte boundary
         self.block_elems = max(off, 8)
+
+    def _scratch_bytes(self, num_tokens: int, batch: int) -> int:
+        return max(super()._scratch_bytes(num_tokens, batch), SEGMENT_MAX_SCRATCH)
 
     def _build(self):
         cfg, ecfg = self.model_config, self.engine_config

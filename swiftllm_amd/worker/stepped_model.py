@@ -29,6 +29,7 @@ from .batch_plan import StepEntry, StepPlan, plan_step
 from .block_manager import BlockManager
 from .kernels.block_swapping import swap_blocks
 from .kernels.sampling import argmax_rows
+from .kernels.window_attn import SHARE_MAX_SCRATCH
 
 DTYPES = {"float16": torch.float16, "bfloat16": torch.bfloat16, "float32": torch.float32}
 
@@ -105,8 +106,8 @@ class SteppedModel:
 
     @torch.inference_mode()
     def profile_num_blocks(self) -> int:
-        """How many blocks fit: one forged worst-case step without a pool, the allocator's high-water mark, and the rest
-        of the usable memory divided by a block's bytes."""
+        """How many blocks fit: one forged worst-case step without a pool, the allocator's high-water mark and the scratch that this
+        step may not show, and the rest of the usable memory divided by a block's bytes."""
         ecfg = self.engine_config
         torch.cuda.empty_cache()
         torch.cuda.reset_peak_memory_stats()
@@ -122,7 +123,7 @@ class SteppedModel:
         self.kv_pool = saved
         torch.cuda.synchronize()
         free_memory, total_memory = torch.cuda.mem_get_info()
-        peak = total_memory - free_memory
+        peak = total_memory - free_memory + self._scratch_bytes(num_tokens, batch)
         usable = total_memory * ecfg.gpu_mem_utilization
         print(f"[Model.profile] GPU total memory: {total_memory / GB:.2f} GB, runtime peak memory: {peak / GB:.2f} GB")
         if usable < peak:
@@ -131,6 +132,12 @@ class SteppedModel:
         table_bytes = 2 * ecfg.max_seqs_in_block_table * ecfg.max_blocks_per_seq * 4
         torch.cuda.empty_cache()
         return max(math.floor((usable - peak - table_bytes) / block_bytes), 0)
+
+    def _scratch_bytes(self, num_tokens: int, batch: int) -> int:
+        """The most scratch that a launch of a step of these sizes takes beside what the forged step shows: of attention, which it
+        leaves out without a pool. (Designs whose recurrences take some by the lengths of the portions add it: the forged ones are
+        equal, and may all be short.)"""
+        return SHARE_MAX_SCRATCH
 
     @torch.inference_mode()
     def init_kvcache_and_swap(self, num_blocks: int):

@@ -22,6 +22,7 @@ from swiftllm_amd.model_config import VafozenModelConfig
 from .kernels.hyper_stream import StreamWeights, hyper_step
 from .kernels.layernorm import embed_positions
 from .kernels.linear import pack_weight, packable
+from .kernels.linear_scan import SEGMENT_MAX_SCRATCH
 from .kernels.rms_stream import StateRef
 from .kernels.window_attn import PoolSlice, StepTiles, served_row_sizes
 from .layers.kekapel_layer import _project
@@ -61,6 +62,9 @@ class VafozenModel(SteppedModel):
             off += mx.num_kv_heads * vd * bs
             off += -off % 8         # every slice starts on a 16-byte boundary
         self.block_elems = max(off, 8)      # (a model without attention still has a block table)
+
+    def _scratch_bytes(self, num_tokens: int, batch: int) -> int:
+        return max(super()._scratch_bytes(num_tokens, batch), SEGMENT_MAX_SCRATCH)
 
     def _build(self):
         cfg, ecfg = self.model_config, self.engine_config

@@ -103,3 +103,19 @@ def test_growing_prompts_leave_no_memory():
     for n in range(200, most, 70):
         turn(n)
         assert torch.cuda.memory_allocated() == before, n
+
+
+def test_profile_sets_scratch_aside(tmp_path, monkeypatch):
+    import lorulix_oracle as O
+    from test_gpu_lorulix import make_model
+    cfg = O.make_config()
+    model = make_model(tmp_path / "m", cfg, O.make_weights(cfg, seed=1))
+    ecfg = model.engine_config
+    want = model._scratch_bytes(ecfg.max_tokens_in_batch, ecfg.max_batch_size)
+    model.profile_num_blocks()
+    with_it = model.profile_num_blocks()
+    monkeypatch.setattr(model, "_scratch_bytes", lambda tokens, batch: 0)
+    without = model.profile_num_blocks()
+    block = model.block_elems * model.dtype.itemsize
+    # (what the two runs' free memory may differ by)
+    assert abs((without - with_it) * block - want) <= block + (32 << 20)
