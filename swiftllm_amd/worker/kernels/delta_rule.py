@@ -7,12 +7,24 @@ from .rms_stream import StateRef
 
 
 # A step whose longest portion holds this many tokens walks by tiles. Walked token by token a portion costs 10 us and 0.3 to 0.37 us a token;
-# by tiles (heads of 128, 8 heads, the step's launches together): 1 portion of 24 / 64 / 1000 tokens 13 / 16 / 70 us against 16 / 29 / 390;
-# 16 of 32 / 64: 27 / 35 against 25 / 40; 30 decoded tokens beside one of 32 / 64 / 200: 31 / 32 / 36 against 33 / 44 / 88. Shorter portions
-# leave the tiles mostly empty: 64 of 8 tokens 60 us against 29.
+# by tiles (heads of 128, 8 heads, the step's launches together): 1 portion of 24 / 64 / 1000 tokens 14 / 16 / 82 us against 17 / 30 / 331;
+# 16 of 24 / 48 / 64: 26 / 34 / 37 against 26 / 39 / 50; 30 decoded tokens beside one of 32 / 64 / 200: 33 / 34 / 46 against 36 / 48 / 99.
 TILES_MIN_PORTION = 48
+# Decoded tokens and other short portions cost a nearly empty tile each (16 heads of 128: 1.2 us by tiles, 0.5 us by tokens), which the longest
+# portion has to make up for: one more token for every so many workgroups (heads x 16 columns) of portions beyond a portion per
+# TILES_FULL_TOKENS tokens. 16 heads of 128, 100 decoded tokens beside one portion of 48 / 80 / 150: 131 / 133 / 136 us by tiles, 109 / 133 /
+# 189 by tokens; 200 beside one of 100 / 150 / 200: 245 / 249 / 254 against 220 / 257 / 291; 32 heads, 50 portions of 64 alone 292 against 430,
+# beside 100 / 200 decoded tokens 551 / 798 against 561 / 708. Over 635 steps (4 to 32 heads of 64 and 128, up to 250 portions) a choice costs at
+# most 2 % more than by tokens (66 % without this rule).
+TILES_WORKGROUPS_A_TOKEN, TILES_FULL_TOKENS = 160, 24
 # Steps that would need more scratch than this (1.6 KiB a token and head of 128) walk token by token.
 TILES_MAX_SCRATCH = 1 << 30
+
+
+def worth_tiles(longest: int, portions: int, tokens: int, heads: int, vdim: int) -> bool:
+    """Whether a step of these portions is walked by tiles."""
+    short = portions - tokens / TILES_FULL_TOKENS
+    return longest >= max(TILES_MIN_PORTION, short * heads * vdim / 16 / TILES_WORKGROUPS_A_TOKEN)
 
 
 def most_tiles_scratch(num_tokens: int, portions: int, mixer) -> int:
@@ -59,7 +71,7 @@ def delta_rule_scan(o, qn, kn, kq, vv, beta, decay, st: StateRef, state_off: int
     """o [T, H * dv] and the states from what the prep left (all fp32)."""
     num_seqs = st.seq_row0.shape[0]
     scratch_bytes = 0
-    if st.tiles is not None and st.longest >= TILES_MIN_PORTION and _hip.load().swl_delta_rule_tiles_supported(H, G, d, dv):
+    if st.tiles is not None and worth_tiles(st.longest, num_seqs, o.shape[0], H, dv) and _hip.load().swl_delta_rule_tiles_supported(H, G, d, dv):
         scratch_bytes = _hip.load().swl_delta_rule_tiles_scratch_bytes(st.tiles[0].shape[0], H, d, dv)
     if 0 < scratch_bytes <= TILES_MAX_SCRATCH:
         row0, cnt, seq_tile0 = st.tiles
