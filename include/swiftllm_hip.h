@@ -891,11 +891,11 @@ int swl_qkv_conv_rope_store_kv(
  * update. q (times q_scale) and k (times k_scale[t][h], NULL: 1) have num_qk_heads heads of dim, shared by num_heads / num_qk_heads
  * heads each; decay fp32, one per channel ([t][heads * dim]) or per head ([t][heads]). States [heads, dim, vdim] fp32 at s_off
  * inside the slots.
- * swl_linear_chunks prepares tiles of up to 16 tokens, dp = dim rounded up to 16: qd [tiles, heads, 16, dp], kd [tiles, heads, dp,
- * 16], total [tiles, heads, dp], intra [tiles, heads, 4, 4, 16] (key % 4, key / 4,
- * query); swl_linear_scan walks every portion's tiles (the first is
- * seq_tile0[s]) and writes o fp32. dim <= 320. swl_linear_step: portions of one token: y fp32 (NULL: not wanted) and / or out =
- * mult * o / rms(o over vdim) * norm_w[h * norm_head_stride + c] * silu(gate) in dtype. dtype (of q, k, v, gate, out) may be SWL_F32. */
+ * swl_linear_chunks prepares tiles of up to 16 tokens for the walks below, dp = dim rounded up to 16, in the order in which their lanes read:
+ * qd [tiles, heads, dp / 16, 16 tokens, 16 channels], kd [tiles, heads, dp, 16 tokens], total [tiles, heads, dp], intra [tiles, heads, 4, 4,
+ * 16] (key % 4, key / 4, query); swl_linear_scan walks every portion's tiles (the first is seq_tile0[s]) and writes o fp32. dim <= 320.
+ * swl_linear_step: portions of one token: y fp32 (NULL: not wanted) and / or out = mult * o / rms(o over vdim) * norm_w[h *
+ * norm_head_stride + c] * silu(gate) in dtype. dtype (of q, k, v, gate, out) may be SWL_F32. */
 int swl_linear_chunks(float *qd, float *kd, float *total, float *intra, const void *q, int64_t q_stride, const void *k,
                       int64_t k_stride, const float *decay, int64_t decay_stride, int32_t per_channel, const float *k_scale,
                       const float *bonus, float q_scale, const int32_t *tile_row0, const int32_t *tile_cnt, int32_t num_tiles,

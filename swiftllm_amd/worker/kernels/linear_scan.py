@@ -89,7 +89,7 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
                   float(eps), float(mult), code, stream)
         return y if finish is None else out
     dp = -(-dim // 16) * 16
-    qd = torch.empty((num_tiles, H, 16, dp), dtype=f32, device=dev)
+    qd = torch.empty((num_tiles, H, dp // 16, 16, 16), dtype=f32, device=dev)
     kd = torch.empty((num_tiles, H, dp, 16), dtype=f32, device=dev)
     total = torch.empty((num_tiles, H, dp), dtype=f32, device=dev)
     intra = torch.empty((num_tiles, H, 4, 4, 16), dtype=f32, device=dev)
