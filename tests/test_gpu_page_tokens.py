@@ -52,3 +52,41 @@ def test_same_pool(name, tokens):
     assert results[0][1].any()
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("tokens", [128, 129, 300])
+@pytest.mark.parametrize("taps", [2, 4, 5])
+def test_same_pool_and_carried_inputs(taps, tokens):
+    """The kernel whose tokens also read their neighbours' rows and write the sequence's carried convolution inputs: what a whole step stores
+    and carries on to the next tokens is what steps below 128 do."""
+    from test_gpu_lorulix import Slots
+    from swiftllm_amd.worker.kernels.rope_kv import qkv_conv_rope_and_store_kv
+    from swiftllm_amd.worker.kernels.window_attn import PoolSlice
+    g = torch.Generator().manual_seed(tokens + taps)
+    C = (H + 2 * G) * D
+    rand = lambda *shape: torch.randn(*shape, generator=g)      # noqa: E731
+    bias, conv, norm = rand(C).cuda(), (rand(taps, C) / taps ** 0.5).cuda(), (1 + 0.3 * rand(D)).cuda()
+    freq = (10000.0 ** (-torch.arange(0, D, 2, dtype=torch.float64) / D)).cuda()
+    rot = SimpleNamespace(dims=D, half=True, multiplier=1.0)
+    rows = rand(7 + tokens + 10, C).to(torch.bfloat16).cuda()
+    table = torch.randperm(64, generator=g)[:2 * 21].view(2, 21).int().cuda()
+    first = tokens // 3         # of sequence 0; the rest goes on with sequence 1, which has 7 tokens already
+    order = [(0, i) for i in range(first)] + [(1, 7 + i) for i in range(tokens - first)]
+    results = []
+    for most in (tokens, 100):
+        slots, pool, made = Slots([2 * (taps - 1) * C], num_slots=2), torch.zeros(64, 2 * G * D * 16, dtype=torch.bfloat16, device="cuda"), []
+        at = 0
+        steps = [[(1, 0, 7)]]
+        for a in range(0, tokens, most):
+            part = order[a:a + most]
+            steps.append([(s, min(p for x, p in part if x == s), sum(x == s for x, _ in part)) for s in sorted({x for x, _ in part})])
+        steps.append([(0, first, 5), (1, 7 + tokens - first, 5)])       # (reads what was carried)
+        for portions in steps:
+            n = sum(c for _, _, c in portions)
+            made.append(qkv_conv_rope_and_store_kv(rows[at:at + n], bias, conv, norm, norm, freq, rot, pool, PoolSlice(0, G * D * 16), table,
+                                                   slots.ref(portions), slots.off[0], H, G, D, D, D, D, 1e-6))
+            at += n
+        results.append((torch.cat(made), pool))
+    assert bool(torch.isfinite(results[0][0].float()).all()) and results[0][1].any()
+    for a, b in zip(*results):
+        assert torch.equal(a, b)

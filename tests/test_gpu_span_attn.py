@@ -138,3 +138,20 @@ def test_span_attention(case, parts, dtype):
             err = (got[at:at + m, :cols] - want).abs().max()
             assert err <= 1.1 * eps * max(1.0, float(want.abs().max())), (splits, i, float(err))
             at += m
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shares", [2, 3, 8, 40])
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_key_shares(case, shares, dtype, monkeypatch):
+    """The same with the pages shared out, also over more workgroups than a row sees pages: windows, chunks and sinks whose shares hold no
+    visible key of a row, or none at all. (No element of the scratch counts that no share has written.)"""
+    from swiftllm_amd.worker.kernels import window_attn
+    used = []
+
+    def forced(device, splits, floats):
+        used.append(shares)
+        return shares, torch.full((shares * floats,), float("nan"), device=device)
+    monkeypatch.setattr(window_attn, "share_scratch", forced)
+    test_span_attention(case, [(1, 96, 31), (2, 0, 64), (3, 250, 1), (4, 15, 130)], dtype)
+    assert used == [shares, shares]
