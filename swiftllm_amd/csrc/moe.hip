@@ -166,6 +166,7 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_kernel(int32_t *idx_out
         float best;
         int besti;
         wave_argmax(logit, experts, lane, best, besti);
+        if (besti >= experts) besti = 0;        // (only NaN, -inf or taken scores are left: an expert that exists, its weight 0 or NaN)
         if (j == 0) chosen_max = all_scores ? all_max : best;
         const float pj = expf(best - chosen_max);
         denom += pj;
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_grouped_kernel(int32_t 
         float best;
         int besti;
         wave_argmax(choice, experts, lane, best, besti);
-        if (besti >= experts) besti = 0;        // (fewer eligible experts than `top`: cannot happen for keep * per >= top)
+        if (besti >= experts) besti = 0;        // (as above)
         const float sc = score[besti];
         denom += sc;
         if (lane == j) {

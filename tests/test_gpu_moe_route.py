@@ -48,3 +48,30 @@ def test_groups(count, per, keep, top):
     same = (idx.long() == order).all(dim=1)
     assert same.float().mean() > 0.95      # (scores closer than fp32 sums tell apart may choose either way)
     torch.testing.assert_close(weights[same].double(), (want / want.sum(1, keepdim=True))[same], rtol=1e-4, atol=1e-7)
+
+
+@pytest.mark.parametrize("experts,top", [(2, 2), (8, 2), (9, 3), (72, 66)])
+def test_scores_that_are_no_numbers(experts, top):
+    """Tokens whose scores are NaN or -inf name experts that exist (what reads the experts' weights takes the ids as they are), with a weight
+    of 0 or NaN, and leave the other tokens alone."""
+    from swiftllm_amd.worker.kernels.moe import moe_experts, moe_route, moe_route_grouped, moe_route_scores
+    g = torch.Generator().manual_seed(experts)
+    h, router = torch.randn(13, 64, generator=g), torch.randn(experts, 64, generator=g) / 8
+    bias = torch.zeros(experts)
+    bad = h.clone()
+    bad[3], bad[7, 5], bad[9, 0] = float("nan"), float("inf"), float("-inf")
+    fine = [t for t in range(13) if t not in (3, 7, 9)]
+    gate_up, down = torch.randn(experts, 2 * 32, 64, generator=g) / 8, torch.randn(experts, 64, 32, generator=g) / 6
+    for route in (lambda x, b: moe_route(x, router.cuda(), b, top), lambda x, b: moe_route_scores(x, router.cuda(), top, 1.5),
+                  lambda x, b: moe_route_grouped(x, router.cuda(), b, top)):
+        want, got = route(h.cuda(), bias.cuda()), route(bad.cuda(), bias.cuda())
+        assert int(got[0].min()) >= 0 and int(got[0].max()) < experts
+        for a, b in zip(want, got):
+            assert torch.equal(a[fine], b[fine])
+        out = [moe_experts(x.cuda(), i, w, gate_up.cuda(), down.cuda(), 7.0).cpu() for x, (i, w) in ((h, want), (bad, got))]
+        assert torch.equal(out[0][fine], out[1][fine]) and torch.isnan(out[1][3]).all()
+    closed = torch.full((experts,), float("-inf"))      # every expert but one is closed
+    closed[1] = 0.0
+    idx, weights = (x.cpu() for x in moe_route(h.cuda(), router.cuda(), closed.cuda(), top))
+    assert (idx[:, 0] == 1).all() and (weights[:, 0] == 1).all() and int(idx.min()) >= 0 and int(idx.max()) < experts
+    assert (weights[:, 1:] == 0).all()
