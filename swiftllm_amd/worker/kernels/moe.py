@@ -44,8 +44,9 @@ def relu_squared(z: torch.Tensor, ff: int) -> torch.Tensor:
 def moe_experts_relu2(h: torch.Tensor, idx: torch.Tensor, wts: torch.Tensor, up: torch.Tensor,
                       down: torch.Tensor) -> torch.Tensor:
     """-> [T, width]: sum_j wts[t, j] * down[e_j] relu(up[e_j] h[t])^2 for experts without a gate. up [experts, ff, width],
-    down [experts, width, ff]. Large steps: assignments sorted by expert, a library product per expert; decode-sized 16-bit
-    steps: the expert-stationary matrix-core kernel; otherwise the per-assignment kernels."""
+    down [experts, width, ff]. Large steps: assignments sorted by expert, one matrix-core launch per product (a library product
+    per expert where the sizes or the type need it); decode-sized 16-bit steps: the expert-stationary matrix-core kernel; otherwise the
+    per-assignment kernels."""
     n, width = h.shape
     experts, ff, _ = up.shape
     top_k = idx.shape[1]
@@ -229,7 +230,7 @@ def moe_experts(h: torch.Tensor, idx: torch.Tensor, wts: torch.Tensor, gate_up: 
     """-> [T, width]: sum_j wts[t, j] * expert idx[t, j] applied to h[t]. gate_up [experts, 2 ff, width], down
     [experts, width, ff]. act: the experts' gated unit (ACT_CLAMPED with `limit`, or ACT_SILU). weigh_inputs: the weights
     multiply the experts' inputs instead, sum_j expert(wts[t, j] * h[t]) — applied to the fp32 products of the gate and up rows
-    (to their rounded products in the sorted form), which are linear in the input. combine False (with weigh_inputs): a step that
+    (to the rounded products of a library GEMM where a large step takes one per expert), which are linear in the input. combine False (with weigh_inputs): a step that
     has the experts' results as rows [T * top_k, width] hands them over un-summed (the caller's next step adds them)."""
     n, width = h.shape
     experts, two_ff, _ = gate_up.shape
