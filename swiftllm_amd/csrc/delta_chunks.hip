@@ -17,9 +17,11 @@
 // What bounds the walk: the chain of tiles (two products of 16 x 16 x dim on four SIMDs and an exchange through LDS a tile: about 1400
 // cycles, 512 of them matrix core). Splitting off the outputs and reading blocks took a tile from 3100 to 2100 cycles.
 // The column shares of a (portion, head) pair read the same operands: consecutive numbers on one XCD.
-// Measured against the walk token by token (8 heads of 128 x 128): 4 prompts of 2048 tokens 746 -> 146 us (both launches, back to back), 2 of 1000
-// beside 30 decoded tokens 899 -> 73 us. Error of o against 64 bits: 1 to 2e-7 of the largest value (0.6 to 1.3e-7 token by token); of
+// Measured against the walk token by token (8 heads of 128 x 128): 4 prompts of 2048 tokens 756 -> 159 us (both launches, back to back), 2 of 1000
+// beside 30 decoded tokens 921 -> 94 us. Error of o against 64 bits: 1 to 2e-7 of the largest value (0.6 to 1.3e-7 token by token); of
 // a model's logits in fp32: 0.98e-6 against 1.0e-6.
+// A NaN or an infinity of a token reaches the outputs of its whole tile, the tokens before it included (a zero of a triangular factor times
+// it), as it does in linear_scan.hip; token by token it reaches the later ones only. Other sequences never see it.
 #include "swl_common.h"
 
 namespace swl {

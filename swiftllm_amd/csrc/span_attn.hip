@@ -14,6 +14,8 @@
 // (mfma 16x16x32, eight waves), whose query fragments and accumulators fit 256 registers, so that two waves share a SIMD.
 // Pages are staged by LDS-DMA (1 KiB per wave instruction, full lines) into two buffers with one barrier a stage; the swizzles that
 // keep the 16-byte fragment reads off each other's banks are applied to the source addresses.
+// A value that is NaN or infinite reaches every row of a workgroup that stages its page (a weight of 0 times it), as it does in the tiles
+// of window_attn_mfma.hip: rows of the same portion whose queries come before it, at most 127 of them; never another sequence's.
 // Measured against the 16-row kernel of window_attn_mfma.hip (bf16, one layer): 4 prompts of about 2000 tokens, 8 heads of 128 over 2 key
 // heads 489 -> 99 us, with a bias by distance 535 -> 104 us (330 TFLOP/s of useful 2 (D + DV), 490 with the second value term); 8 latent
 // heads of 576 + 512 over one, window 1024: 1115 -> 253 us; 11 prompts of 333 tokens, 16 heads of 128 over 4: 120 -> 28 us.
