@@ -120,7 +120,7 @@ def _moe_sorted(h, idx, wts, up, down, ff, mode, act, limit, weigh_inputs):
     order = torch.empty(total, dtype=torch.int32, device=dev)
     where = torch.empty(total, dtype=torch.int64, device=dev)
     offsets = torch.empty(experts + 1, dtype=torch.int32, device=dev)
-    idx = idx.contiguous()
+    idx, wts = idx.contiguous(), wts.contiguous()
     _hip.call("swl_moe_sort", _hip.ptr(order), _hip.ptr(where), _hip.ptr(offsets), _hip.ptr(idx), total, experts, stream)
     y = torch.empty((total, ff), dtype=h.dtype, device=dev)
     _hip.call("swl_moe_gemm", _hip.ptr(y), _hip.ptr(h), _hip.ptr(up), _hip.ptr(order), _hip.ptr(offsets),

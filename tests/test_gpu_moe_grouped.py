@@ -69,3 +69,21 @@ def test_sorted_experts(n, top, experts, width, ff, kind, form, dtype):
     # rounds the first products too), and one of each result: 2^-9 relative in bf16, 2^-12 in fp16
     eps = 2.0 ** (-9 if dtype == torch.bfloat16 else -12)
     assert ((got.double().cpu() - want).abs() <= 8 * eps * (size + want.abs())).all()
+
+
+@pytest.mark.parametrize("form", ["silu", "silu_in", "relu2"])
+def test_assignments_of_other_strides(form):
+    """Ids and weights stored choice by choice (columns of the [tokens, choices] view are contiguous) give what contiguous ones give."""
+    from swiftllm_amd.worker.kernels import moe
+    g = torch.Generator().manual_seed(3)
+    n, top, experts, width, ff = 150, 2, 5, 128, 64
+    h, down = torch.randn(n, width, generator=g).bfloat16().cuda(), (torch.randn(experts, width, ff, generator=g) / 8).bfloat16().cuda()
+    up = (torch.randn(experts, ff * (1 if form == "relu2" else 2), width, generator=g) / 11).bfloat16().cuda()
+    idx, wts = _assign(n, top, experts, "any", g).int().cuda(), (torch.rand(n, top, generator=g) + 0.1).cuda()
+    assert moe._sorted_served(h, up, down, ff)
+
+    def run(i, w):
+        if form == "relu2":
+            return moe.moe_experts_relu2(h, i, w, up, down)
+        return moe.moe_experts(h, i, w, up, down, 0.0, moe.ACT_SILU, weigh_inputs=form == "silu_in")
+    assert torch.equal(run(idx, wts), run(idx.t().contiguous().t(), wts.t().contiguous().t()))
