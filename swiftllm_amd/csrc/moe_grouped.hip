@@ -1,17 +1,18 @@
 // moe_grouped.hip — the expert products of prompt-sized steps: assignments sorted by expert on the device, then ONE matrix-core
 // launch per product for all experts (16-bit storage, fp32 accumulation).
 //
-// What bounds it: the matrix cores (2 N_assignments (2 ff + ff) width flops). A library product per expert leaves most of the chip
-// idle at these sizes (2048 x 1024 x 1024: 128 tiles for 256 CUs) and needs the experts' row counts on the host: a read-back and the
-// launches' gaps behind it in every layer. Here a tile of 128 assignments of one expert x 128 weight rows is a workgroup of four
-// waves, each a 64 x 64 piece (mfma 32x32x16, 2 x 2 accumulators); operands are staged by LDS-DMA in 64-deep slices of whole 128-byte
-// lines into two buffers, with the swizzle that keeps the 16-byte fragment reads off each other's banks on the source side. Token rows
-// are gathered by the staging itself (no sorted copy of the inputs), the gated unit or the squared ReLU runs on the fp32 products in
-// the epilogue, and results leave as whole lines through LDS. Tiles of one expert are consecutive in one XCD's share of the grid, so its
-// weights stay in that XCD's L2.
-// Measured (bf16): 16000 assignments over 8 experts, width 1024, ff 1024: gate/up with the unit 97 us (690 TFLOP/s), down 43 us (770);
-// 9000 assignments, width and ff 2048: 208 and 108 us (725, 700). The sorted library products they replace, gather, read-back and
-// activation included: 740 us of a layer at the first size, 570 at the second.
+// What bounds it: what a CU takes from L2 (a tile of 128 x 128 asks for 32 KiB per 64 columns of the reduction: 52 of 70 us when nothing
+// else is done, 8192 rows, width and ff 2048) next to the matrix cores (43 us), and what of the two does not overlap. A library product per
+// expert leaves most of the chip idle at these sizes (2048 x 1024 x 1024: 128 tiles for 256 CUs) and needs the experts' row counts on the
+// host: a read-back and the launches' gaps behind it in every layer. Here a tile of 128 assignments of one expert x 128 weight rows is a
+// workgroup of four waves, each a 64 x 64 piece (mfma 32x32x16, 2 x 2 accumulators); operands are staged by LDS-DMA in 64-deep slices of
+// whole 128-byte lines (half lines take 1.4 times as long), with the swizzle that keeps the 16-byte fragment reads off each other's banks on
+// the source side. Token rows are gathered by the staging itself (no sorted copy of the inputs), the gated unit or the squared ReLU runs
+// on the fp32 products in the epilogue, and results leave as whole lines through LDS.
+// Measured (bf16), two staged slices and column tiles fastest -> now: 9000 assignments over 8 experts, width and ff 2048: gate/up with the
+// unit 223 -> 159 us (950 TFLOP/s), down 101 -> 85; 16000 assignments, width and ff 1024: 98 -> 82, 54 -> 45; 1562, width and ff 2048:
+// 61 -> 37, 30 -> 26. Tiles of 256 x 256 or 128 x 256 with rings of up to five slices: 225 and 172 us at the first size (the chip's last
+// turn is half empty, and first slices and results wait alone), 150 and 100 at the second; faster only where the tiles fill whole turns.
 #include "swl_common.h"
 
 namespace swl {
@@ -83,46 +84,75 @@ struct MoeGemmParams {
     const void *x, *w;
     const int32_t *order, *offsets;     // order NULL: row i of x belongs to sorted position i
     const float *in_w;
-    int top, experts, K, N, act, n_tiles, per_xcd;
+    int top, experts, K, N, act, n_tiles;
     float limit;
 };
 
-// MODE 0: out[pos][N] = x w^T; 1: w rows [N gate | N up], out = gated unit; 2: out = relu(x w^T)^2
-template <typename T, int MODE>
-__global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeGemmParams p) {
-    constexpr int TILEB = kMgTile * kMgDepth * 2;       // bytes of a staged operand slice
-    constexpr int OUTC = MODE == 1 ? 64 : 128;          // output columns of a tile
-    __shared__ __attribute__((aligned(16))) char smem[4 * TILEB];       // [buffer][weights, tokens]; the output tile of the epilogue
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int l32 = lane & 31, hf = lane >> 5, wn = wave & 1, wm = wave >> 1;
-    // ---- which tile: id % 8 is the XCD; an XCD takes consecutive row tiles, all column tiles of one after the other ----------------
-    const int id = blockIdx.x, j = id >> 3, n_tile = j % p.n_tiles;
-    int m_tile = (id & 7) * p.per_xcd + j / p.n_tiles;
-    int expert = -1, row0 = 0, rows = 0;
-    for (int e0 = 0; e0 < p.experts; e0 += 64) {        // (64 experts at a time: their tiles counted by a scan over the wave)
+// The tile of this workgroup: every XCD (workgroup id % 8) takes an equal run of the tiles that there are, row tiles eight at a time with
+// all their column tiles, the row tile fastest: what an XCD works on at once is about as many rows as columns of weights.
+struct MgTile {
+    int expert, row0, rows, n_tile;     // expert < 0: no tile
+};
+__device__ __forceinline__ MgTile mg_tile(const MoeGemmParams &p) {
+    constexpr int GROUP = 8;
+    const int lane = threadIdx.x & 63;
+    int a = 0, b = 0;
+    // row tiles of 64 experts, counted by a scan over the wave
+    auto tiles_to = [&](int e0) {
         const int e = min(e0 + lane, p.experts - 1);
-        const int a = p.offsets[e], b = e0 + lane < p.experts ? p.offsets[e + 1] : a;
-        const int tiles = (b - a + kMgTile - 1) / kMgTile;
-        int scan = tiles;
+        a = p.offsets[e];
+        b = e0 + lane < p.experts ? p.offsets[e + 1] : a;
+        int scan = (b - a + kMgTile - 1) / kMgTile;
         for (int o = 1; o < 64; o <<= 1) {
             const int v = __shfl_up(scan, o, 64);
             if (lane >= o) scan += v;
         }
+        return scan;
+    };
+    int total = 0;
+    for (int e0 = 64; e0 < p.experts; e0 += 64) total += __builtin_amdgcn_readlane(tiles_to(e0), 63);
+    int scan = tiles_to(0);
+    total += __builtin_amdgcn_readlane(scan, 63);
+    const int64_t all = static_cast<int64_t>(total) * p.n_tiles;
+    const int xcd = blockIdx.x & 7;
+    const int64_t at = xcd * all / 8 + (blockIdx.x >> 3);
+    MgTile t = {-1, 0, 0, 0};
+    if (at >= (xcd + 1) * all / 8) return t;
+    const int group = static_cast<int>(at / (GROUP * static_cast<int64_t>(p.n_tiles)));
+    const int in_group = static_cast<int>(at - group * (GROUP * static_cast<int64_t>(p.n_tiles)));
+    const int wide = min(GROUP, total - GROUP * group);
+    t.n_tile = in_group / wide;
+    int m_tile = GROUP * group + in_group - t.n_tile * wide;
+    for (int e0 = 0; e0 < p.experts; e0 += 64) {
+        if (e0 > 0) scan = tiles_to(e0);
         const unsigned long long past = __ballot(scan > m_tile);
         if (past) {
             const int l = __builtin_ctzll(past);
-            expert = e0 + l;
-            const int first = __shfl(scan - tiles, l, 64), lo = __shfl(a, l, 64), hi = __shfl(b, l, 64);
-            row0 = lo + (m_tile - first) * kMgTile;
-            rows = min(kMgTile, hi - row0);
+            const int lo = __builtin_amdgcn_readlane(a, l), hi = __builtin_amdgcn_readlane(b, l);
+            t.expert = e0 + l;
+            t.row0 = lo + (m_tile - __builtin_amdgcn_readlane(scan, l) + (hi - lo + kMgTile - 1) / kMgTile) * kMgTile;
+            t.rows = min(kMgTile, hi - t.row0);
             break;
         }
-        m_tile -= __shfl(scan, 63, 64);
+        m_tile -= __builtin_amdgcn_readlane(scan, 63);
     }
-    if (expert < 0) return;
-    expert = __builtin_amdgcn_readfirstlane(expert);
-    row0 = __builtin_amdgcn_readfirstlane(row0);
-    rows = __builtin_amdgcn_readfirstlane(rows);
+    return t;
+}
+
+// MODE 0: out[pos][N] = x w^T; 1: w rows [N gate | N up], out = gated unit; 2: out = relu(x w^T)^2
+// BUFS staged slices: 2 with two workgroups a CU, a slice on its way while one is multiplied; 1 with four workgroups a CU, which hide
+// each other's waits, first and last slices too.
+template <typename T, int MODE, int BUFS>
+__global__ __launch_bounds__(256, BUFS == 1 ? 4 : 2) void moe_gemm_kernel(MoeGemmParams p) {
+    constexpr int TILEB = kMgTile * kMgDepth * 2;       // bytes of a staged operand slice
+    constexpr int OUTC = MODE == 1 ? 64 : 128, PITCH = OUTC + 8;          // output columns of a tile, elements between its rows in LDS
+    constexpr int STAGED = BUFS * 2 * TILEB, RESULT = kMgTile * PITCH * 2;
+    __shared__ __attribute__((aligned(16))) char smem[STAGED > RESULT ? STAGED : RESULT];      // [buffer][weights, tokens]; then the output tile
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hf = lane >> 5, wn = wave & 1, wm = wave >> 1;
+    const MgTile t = mg_tile(p);
+    if (t.expert < 0) return;
+    const int row0 = t.row0, rows = t.rows, n_tile = t.n_tile;
 
     // ---- staging: wave w loads rows 32 w .. 32 w + 31 of both operands, 8 rows of 128 bytes an instruction --------------------------
     const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem));
@@ -143,11 +173,11 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeGemmParams p) {
         const int xr = p.order ? p.order[pos] / p.top : pos;
         x_off[i] = static_cast<unsigned>(xr * kb + unit * 16);
     }
-    const char *wb = static_cast<const char *>(p.w) + static_cast<int64_t>(expert) * (MODE == 1 ? 2 : 1) * p.N * kb;
+    const char *wb = static_cast<const char *>(p.w) + static_cast<int64_t>(t.expert) * (MODE == 1 ? 2 : 1) * p.N * kb;
     const char *xb = static_cast<const char *>(p.x);
     auto issue = [&](int st) {
         const char *ws = wb + static_cast<int64_t>(st) * kMgDepth * 2, *xs = xb + static_cast<int64_t>(st) * kMgDepth * 2;
-        const unsigned to = lds0 + static_cast<unsigned>((st & 1) * 2 * TILEB + wave * 4096);
+        const unsigned to = lds0 + static_cast<unsigned>((st & (BUFS - 1)) * 2 * TILEB + wave * 4096);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             unsigned keep;
@@ -166,27 +196,67 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeGemmParams p) {
     for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (int b = 0; b < 2; ++b) acc[a][b] = float16_t{};
+    vec8_t<T> wf[2][2], xf[2][2];       // [set][piece]: the fragments of 16 columns are requested in front of the products of the 16 before
+    auto read = [&](int st, int e, int set) {
+        const char *ws = smem + (st & (BUFS - 1)) * 2 * TILEB + wn * 64 * 128, *xs = smem + (st & (BUFS - 1)) * 2 * TILEB + TILEB + wm * 64 * 128;
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            wf[set][a] = *reinterpret_cast<const vec8_t<T> *>(ws + a * 32 * 128 + frag[e]);
+            xf[set][a] = *reinterpret_cast<const vec8_t<T> *>(xs + a * 32 * 128 + frag[e]);
+        }
+    };
+    auto multiply = [&](int set) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) acc[a][b] = mg_mfma(wf[set][a], xf[set][b], acc[a][b]);
+    };
+    auto step = [&](int st, int e, int set) {       // products of a set, the reads of the next spread between them
+        __builtin_amdgcn_sched_barrier(0);
+        read(st, e, set ^ 1);
+        multiply(set);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
     const int stages = p.K / kMgDepth;
     issue(0);
-    for (int st = 0; st < stages; ++st) {
-        // this wave's pieces of the slice have landed, its reads of the other buffer have returned; then everyone's
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        if (st + 1 < stages) issue(st + 1);
-        const char *ws = smem + (st & 1) * 2 * TILEB + wn * 64 * 128, *xs = smem + (st & 1) * 2 * TILEB + TILEB + wm * 64 * 128;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            vec8_t<T> wf[2], xf[2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a) {
-                wf[a] = *reinterpret_cast<const vec8_t<T> *>(ws + a * 32 * 128 + frag[e]);
-                xf[a] = *reinterpret_cast<const vec8_t<T> *>(xs + a * 32 * 128 + frag[e]);
-            }
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b) acc[a][b] = mg_mfma(wf[a], xf[b], acc[a][b]);
+    if constexpr (BUFS == 1) {
+        for (int st = 0;; ++st) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // this wave's pieces of the slice have landed; then everyone's
+            __builtin_amdgcn_s_barrier();
+            read(st, 0, 0);
+            step(st, 1, 0);
+            step(st, 2, 1);
+            step(st, 3, 0);
+            multiply(1);        // (its operands were the last reads of the slice: all of them have returned; then everyone's)
+            if (st + 1 == stages) break;
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            issue(st + 1);
         }
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        if (stages > 1) issue(1);
+        read(0, 0, 0);
+        for (int st = 0; st + 1 < stages; ++st) {
+            step(st, 1, 0);
+            step(st, 2, 1);
+            step(st, 3, 0);
+            // this wave's pieces of the next slice have landed, its reads of this one have returned; then everyone's
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            if (st + 2 < stages) issue(st + 2);
+            step(st + 1, 0, 1);
+        }
+        step(stages - 1, 1, 0);
+        step(stages - 1, 2, 1);
+        step(stages - 1, 3, 0);
+        multiply(1);
     }
     // ---- epilogue: acc[a][b][4 q + r] = product (weight row 64 wn + 32 a + 8 q + 4 hf + r, token 64 wm + 32 b + l32) ----------------
 #pragma unroll
@@ -196,7 +266,6 @@ __global__ __launch_bounds__(256, 2) void moe_gemm_kernel(MoeGemmParams p) {
             if (a + b < 2) mfma_results_tie(acc[a][b]);
     mfma_results_ready<8>(acc[1][1]);
     __syncthreads();        // every wave is done with the staged slices
-    constexpr int PITCH = OUTC + 8;
     T *tile = reinterpret_cast<T *>(smem);
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
@@ -277,16 +346,20 @@ extern "C" int swl_moe_gemm(void *out, const void *x, const void *w, const int32
     p.n_tiles = (N + cols - 1) / cols;
     // as many row tiles as there can be (every expert may end in a part of one); surplus workgroups leave at once
     const int64_t m_tiles = (num_assignments + swl::kMgTile - 1) / swl::kMgTile + (experts < num_assignments ? experts : num_assignments);
-    p.per_xcd = static_cast<int>((m_tiles + 7) / 8);
-    const int64_t grid = 8LL * p.per_xcd * p.n_tiles;
+    const int64_t grid = (m_tiles * p.n_tiles + 7) / 8 * 8;
     if (grid > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
     hipStream_t s = static_cast<hipStream_t>(stream);
-#define SWL_MG(MODE) hipLaunchKernelGGL((swl::moe_gemm_kernel<T, MODE>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, p)
+    // One staged slice and four workgroups a CU where there are more tiles than two a CU (about: an expert's last row tile half full),
+    // else two slices: 31.3 and 35.7 us at 688 tiles (4950 rows, width and ff 1024, gate/up), 39.1 and 36.6 at 512, 20.7 and 19.3 at 344.
+    const bool many = (num_assignments + 64LL * experts) / swl::kMgTile * p.n_tiles > 512;
+#define SWL_MG(MODE, BUFS) hipLaunchKernelGGL((swl::moe_gemm_kernel<T, MODE, BUFS>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, p)
+#define SWL_MG2(MODE) do { if (many) SWL_MG(MODE, 1); else SWL_MG(MODE, 2); } while (0)
     SWL_DISPATCH_DTYPE(dtype, T, {
-        if (mode == 0) SWL_MG(0);
-        else if (mode == 1) SWL_MG(1);
-        else SWL_MG(2);
+        if (mode == 0) SWL_MG2(0);
+        else if (mode == 1) SWL_MG2(1);
+        else SWL_MG2(2);
     });
+#undef SWL_MG2
 #undef SWL_MG
     return swl::check_launch();
 }

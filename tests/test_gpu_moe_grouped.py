@@ -87,3 +87,37 @@ def test_assignments_of_other_strides(form):
             return moe.moe_experts_relu2(h, i, w, up, down)
         return moe.moe_experts(h, i, w, up, down, 0.0, moe.ACT_SILU, weigh_inputs=form == "silu_in")
     assert torch.equal(run(idx, wts), run(idx.t().contiguous().t(), wts.t().contiguous().t()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("n,top,experts,K,N,kind", [
+    (1500, 2, 8, 64, 4096 + 8, "any"),          # one slice, a last column tile of 8
+    (900, 2, 70, 128, 1600, "any"),             # more experts than lanes, tiles of a few rows, two slices
+    (640, 1, 5, 192, 16384, "runs"),            # tiles filled to the row, one over, one short
+    (300, 2, 3, 320, 16384, "one")])            # an empty expert
+def test_many_tiles(n, top, experts, K, N, kind, mode, dtype):
+    """More tiles than two a CU take the form with one staged slice: the bits of launches over parts of the columns, which stay below."""
+    from swiftllm_amd import _hip
+    g = torch.Generator().manual_seed(K)
+    total = n * top
+    idx = _assign(n, top, experts, kind, g).to(torch.int32).cuda()
+    order, where = torch.empty(total, dtype=torch.int32, device="cuda"), torch.empty(total, dtype=torch.int64, device="cuda")
+    offsets = torch.empty(experts + 1, dtype=torch.int32, device="cuda")
+    _hip.call("swl_moe_sort", _hip.ptr(order), _hip.ptr(where), _hip.ptr(offsets), _hip.ptr(idx), total, experts, _hip.stream())
+    x = torch.randn(n, K, generator=g).to(dtype).cuda()
+    w = (torch.randn(experts, 2 if mode == 1 else 1, N, K, generator=g) / K ** 0.5).to(dtype).cuda()
+    in_w = (torch.rand(total, generator=g) + 0.5).cuda() if mode == 1 else None
+
+    def product(w):
+        cols = w.shape[2]
+        out = torch.zeros(total, cols, dtype=dtype, device="cuda")
+        _hip.call("swl_moe_gemm", _hip.ptr(out), _hip.ptr(x), _hip.ptr(w), _hip.ptr(order), _hip.ptr(offsets), _hip.ptr(in_w), total, n,
+                  top, experts, K, cols, mode, 0, 1.5, _hip.dtype_code(dtype), _hip.stream())
+        return out
+    row_tiles, width = (total + 64 * experts) // 128, 64 if mode == 1 else 128
+    part = width * (512 // row_tiles)
+    assert row_tiles * -(-N // width) > 512 and part > 0
+    got = product(w)
+    assert torch.equal(got, torch.cat([product(w[:, :, c:c + part].contiguous()) for c in range(0, N, part)], 1))
+    assert got.abs().amax(1).min() > 0
