@@ -288,7 +288,7 @@ int swl_gemm_packed_mid_silu_gate(void *out, const void *x, const void *w_up_gat
 /* Large decode batches on a packed weight (csrc/gemm_wide.hip): out[M, N] = x . W^T for up to 256 tokens — the projections
  * of reference kernels/linear.py:3-12 (transformer_layer.py:54-56,117,126,128) at the batch sizes a 264 GB KV pool holds;
  * every weight fragment feeds ceil(M/32) <= 8 MFMAs, x^T shared by the workgroup through LDS. N % 32 == 0, K % 64 == 0.
- * waves_per_group: 0 = library's choice, 4 or 8; k_splits: 0 = library's choice, else a power of two <= 16 with
+ * waves_per_group: 0, 4 or 8 (one form serves all); k_splits: 0 = library's choice, else a power of two <= 16 with
  * K % (64 * k_splits) == 0; workspace >= k_splits * M * N * 4 bytes when K is split. */
 int swl_gemm_packed_wide(void *out, const void *x, const void *w_packed, void *workspace, size_t workspace_bytes,
                          int32_t M, int32_t N, int32_t K, int64_t x_row_stride, int64_t out_row_stride,

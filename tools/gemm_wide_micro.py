@@ -27,7 +27,7 @@ def time_us(fn, iters, warm=3):
 
 
 def sha(t):
-    """Digest of a result tensor's bits (runs with different SWL_WIDE_TS / variant libraries must agree on it)."""
+    """Digest of a result tensor's bits (runs with variant libraries must agree on it)."""
     return hashlib.sha1(t.contiguous().view(torch.uint8).cpu().numpy().tobytes()).hexdigest()[:12]
 
 
@@ -44,7 +44,7 @@ def main():
     dtype = getattr(torch, a.dtype)
     code = _hip.dtype_code(dtype)
     g = torch.Generator(device="cuda").manual_seed(0)
-    tag = dict(ts=os.environ.get("SWL_WIDE_TS", "auto"), lib=os.path.basename(os.environ.get("SWIFTLLM_HIP_LIB", "product")))
+    tag = dict(lib=os.path.basename(os.environ.get("SWIFTLLM_HIP_LIB", "product")))
     for name in a.shapes.split(","):
         N, K = SHAPES[name]
         # cycle through enough copies that a re-read never finds its lines in the 256 MiB Infinity Cache (r06d: with 6 copies
