@@ -285,6 +285,12 @@ int swl_gemm_packed_mid_choose_splits(int32_t M, int32_t N, int32_t K); /* its c
 int swl_gemm_packed_mid_silu_gate(void *out, const void *x, const void *w_up_gate_packed, int32_t M, int32_t I,
                                   int32_t K, int64_t x_row_stride, int64_t out_row_stride, int32_t dtype,
                                   swl_stream_t stream);
+/* Projections of up to 16 tokens in true fp32 (csrc/gemm_f32.hip): out[M, N] = x[M, K] w[N, K]^T, w row-major. K % 4 == 0, x rows of whole
+ * 16-byte pieces. k_waves: 0 = library's choice, else 1, 2 or 4 waves share the columns of a row.
+ * supported: 0 = no, 1 = yes, 2 = and faster than a library product of these sizes. */
+int swl_gemm_f32_supported(int32_t M, int32_t N, int32_t K);
+int swl_gemm_f32(float *out, const float *x, const float *w, int32_t M, int32_t N, int32_t K, int64_t x_row_stride, int64_t out_row_stride,
+                 int32_t k_waves, swl_stream_t stream);
 /* Large decode batches on a packed weight (csrc/gemm_wide.hip): out[M, N] = x . W^T for up to 256 tokens — the projections
  * of reference kernels/linear.py:3-12 (transformer_layer.py:54-56,117,126,128) at the batch sizes a 264 GB KV pool holds;
  * every weight fragment feeds ceil(M/32) <= 8 MFMAs, x^T shared by the workgroup through LDS. N % 32 == 0, K % 64 == 0.

@@ -258,6 +258,18 @@ def _blas_linear(a: torch.Tensor, w: torch.Tensor, row_blocks=None, plateau=None
     return out
 
 
+def linear_f32(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """a[T, in] @ w[out, in]^T in true fp32: a few tokens on the hand-written kernel (csrc/gemm_f32.hip), the BLAS otherwise."""
+    if (a.is_cuda and a.dim() == 2 and a.dtype == w.dtype == torch.float32 and w.is_contiguous() and a.stride(1) == 1
+            and (a.data_ptr() | w.data_ptr()) % 16 == 0 and a.stride(0) % 4 == 0):
+        m, (n, k) = a.shape[0], w.shape
+        if _hip.load().swl_gemm_f32_supported(m, n, k) == 2:
+            out = torch.empty((m, n), dtype=a.dtype, device=a.device)
+            _hip.call("swl_gemm_f32", _hip.ptr(out), _hip.ptr(a), _hip.ptr(w), m, n, k, _row_stride(a), n, 0, _hip.stream())
+            return out
+    return F.linear(a, w)
+
+
 def linear_grouped(x: torch.Tensor, w: torch.Tensor, skinny: bool = False) -> torch.Tensor:
     """x [groups, T, in], w [groups * out, in] -> [T, groups * out]: columns g * out .. are x[g] @ w[g * out : (g + 1) * out]^T. One
     launch for decode-sized steps on a packed weight, a product per group otherwise."""

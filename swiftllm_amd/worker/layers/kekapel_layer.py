@@ -4,7 +4,7 @@ import torch
 
 from swiftllm_amd import _hip
 
-from ..kernels.linear import linear, linear_silu_gate, linear_splitk
+from ..kernels.linear import linear, linear_f32, linear_silu_gate, linear_splitk
 from ..kernels.moe import ACT_SILU_UP_FIRST, gated_unit, moe_experts, moe_route
 from ..kernels.polynorm import polynorm
 from ..kernels.window_attn import qknorm_and_store_kv, window_attention
@@ -12,9 +12,9 @@ from ..kernels.window_attn import qknorm_and_store_kv, window_attention
 
 def _project(a: torch.Tensor, w: torch.Tensor, skinny: bool) -> torch.Tensor:
     """a [T, in] @ w[out, in]^T. bf16 / f16: the framework's projection routing (hand-written weight-streaming GEMMs for
-    decode-sized batches, the BLAS otherwise); fp32: the BLAS in true fp32."""
+    decode-sized batches, the BLAS otherwise); fp32: true fp32, with a kernel for a few tokens."""
     if a.dtype == torch.float32:
-        return torch.nn.functional.linear(a, w)
+        return linear_f32(a, w)
     if skinny and not getattr(w, "_swl_blas_only", False):
         try:
             return linear(a, w, True)

@@ -1,0 +1,48 @@
+"""Products of a few tokens in true fp32 (csrc/gemm_f32.hip) against float64: edges of the 256-column slices, of the four-row waves and of
+the token counts that have a form of their own."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(1, 4), (3, 252), (17, 256), (1025, 1028), (64, 4096), (2048, 512), (4097, 260), (8200, 1024)])
+def test_gemm_f32(M, N, K):
+    from swiftllm_amd import _hip
+    g = torch.Generator().manual_seed(M * N + K)
+    x = torch.full((M, K + 8), float("nan"))
+    x[:, :K] = torch.randn(M, K, generator=g)
+    x, w = x.cuda(), torch.randn(N, K, generator=g).cuda()
+    want = x[:, :K].double() @ w.double().t()
+    size = x[:, :K].double().abs() @ w.double().abs().t()
+    first = None
+    for ks in (0, 1, 2, 4):
+        out = torch.full((M + 1, N + 4), 7.0, device="cuda")
+        _hip.call("swl_gemm_f32", _hip.ptr(out), _hip.ptr(x), _hip.ptr(w), M, N, K, x.stride(0), out.stride(0), ks, _hip.stream())
+        # one rounding a term: K / 64 of a lane in a row and at most 24 additions of partial sums
+        assert ((out[:M, :N].double() - want).abs() <= (K / 64 + 24) * 2.0 ** -24 * size + 1e-30).all(), ks
+        assert (out[M] == 7.0).all() and (out[:, N:] == 7.0).all()
+        if ks == 0:
+            first = out
+    # a token's bits do not hang on its company
+    alone = torch.empty(1, N, device="cuda")
+    _hip.call("swl_gemm_f32", _hip.ptr(alone), _hip.ptr(x[M - 1]), _hip.ptr(w), 1, N, K, K, N, 0, _hip.stream())
+    assert torch.equal(alone[0], first[M - 1, :N])
+
+
+@pytest.mark.parametrize("M,N,K,form", [(8, 64, 64, "own"), (9, 2049, 64, "library"), (17, 64, 64, "library"), (3, 64, 62, "library"),
+                                        (3, 64, 64, "odd"), (3, 64, 64, "columns"), (0, 64, 64, "library")])
+def test_linear_f32_routes(M, N, K, form, monkeypatch):
+    """What the kernel does not take goes to the library as before: more tokens, odd rows, unaligned or strided columns, no tokens."""
+    from swiftllm_amd import _hip
+    from swiftllm_amd.worker.kernels.linear import linear_f32
+    calls = []
+    real = _hip.call
+    monkeypatch.setattr(_hip, "call", lambda name, *a: (calls.append(name), real(name, *a))[1])
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(M, 2 * K + 1, generator=g).cuda(), torch.randn(N, K, generator=g).cuda()
+    x = x[:, 1:K + 1] if form == "odd" else x[:, 0:2 * K:2] if form == "columns" else x[:, :K].contiguous()
+    got = linear_f32(x, w)
+    assert (calls == ["swl_gemm_f32"]) == (form == "own")
+    assert torch.allclose(got.double(), x.double() @ w.double().t(), rtol=0, atol=1e-4) and got.shape == (M, N)
