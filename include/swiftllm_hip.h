@@ -437,6 +437,10 @@ int swl_gemm_tiny_silu_gate_from_splitk(void *out, const float *slabs_in, int32_
 int swl_gemm_rows_supported(int32_t M, int32_t N, int32_t K);
 int swl_gemm_rows_add(void *residual, const void *x, const void *w_packed, int32_t M, int32_t N, int32_t K,
                       int64_t x_row_stride, int32_t dtype, swl_stream_t stream);
+/* The same kernel with a plain result: out[M, N] = round(x . W^T), or with relu2 = 1 relu(that)^2 rounded again (swl_relu_sq's
+ * rounding points). K % 1024 == 0; any N: the packed weight holds whole tiles of 32 rows, rows of zeros from N on. */
+int swl_gemm_rows_store(void *out, const void *x, const void *w_packed, int32_t M, int32_t N, int32_t K, int64_t x_row_stride,
+                        int64_t out_row_stride, int32_t relu2, int32_t dtype, swl_stream_t stream);
 int swl_gemm_skinny_packed_partial_nf(float *slabs, size_t slabs_bytes, float *ssq_out, const void *x, const void *norm_w,
                                       const void *w_packed, int32_t M, int32_t N, int32_t K, int64_t x_row_stride,
                                       int32_t k_splits, int32_t dtype, swl_stream_t stream);

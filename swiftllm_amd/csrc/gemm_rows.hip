@@ -33,6 +33,11 @@
 // 8 KiB LDS tile of its own: ds_write_b128 at piece ^ (token & 15), ds_read_b128 of lane (r, kq) at (4j + kq) ^ r —
 // conflict-free for the 8-lane write groups and for the irregular 16-lane groups of the b128 read.
 // One wave's LDS operations execute in order: no barrier in the stream. Same MFMAs in the same order: the same bits.
+// Plain results (swl_gemm_rows_store, optionally through a squared ReLU) serve the narrower matrices of the stepped designs, any
+// number of rows: what such a launch costs is its start, one round trip and the 16 rows' share of x, where shares of K paid a second
+// launch and 8 to 16 slabs. us at 32 tokens, cold bf16 weights, against the split ring kernel with its reduce launch (the
+// library for 3088 rows): 1024 x 1024 6.3 -> 3.8, 2048 x 2048 7.7 -> 5.5, 3088 x 2048 11.5 -> 6.0, 8192 x 2048 12.8 -> 10.4
+// (3.2 TB/s; 7.6 at one token: x is two thirds of what a CU reads). Where its line lies: kernels/linear.py, _rows_serves.
 // No slabs, no second launch, no atomics, no cross-workgroup hand-off. (r05 also built an epilogue that wrote
 // round(residual * w_norm) and one sum-of-squares partial per tile, with a SiLU-gate GEMM that added the 256 partials from
 // LDS-DMA'd copies: correct, +2 us on the up/gate kernel, removed — last revision that has it: ca4e9a9, numbers in
@@ -51,13 +56,21 @@ __device__ __forceinline__ float4_t rows_mfma(vec8_t<bf16> a, vec8_t<bf16> b, fl
 constexpr int kRowsWaves = 8;     // K splits = waves per workgroup
 constexpr int kRowsTile = 16;     // rows of W per workgroup
 constexpr int kRowsCh = 4;        // k-steps (of 32) per ring chunk
-constexpr int kRowsRing = 4;      // chunks in flight per wave: 16 k-steps = 192 VGPRs at two token blocks
+constexpr int kRowsRing = 4;      // chunks in flight per wave, at most: 16 k-steps = 192 VGPRs at two token blocks
+constexpr int kRowsKUnit = 32 * kRowsWaves * kRowsCh;
 constexpr int kRowsRedPitch = 20; // floats per token row of a wave's tile image in LDS (80 B: 16-byte stores spread)
+
+// What a workgroup does with its finished 16 columns:
+//   kRowsAdd    residual += round(product)
+//   kRowsStore  out = round(product)
+//   kRowsRelu2  out = round(relu(round(product))^2): swl_relu_sq behind the stored product
+constexpr int kRowsAdd = 0, kRowsStore = 1, kRowsRelu2 = 2;
 
 struct RowsArgs {
     const void *x;
     const void *wp;
-    void *residual;
+    void *residual;         // kRowsAdd: rows of N; otherwise the output, rows out_stride apart
+    int64_t out_stride;
     int M, N, K;
     int64_t x_stride;
     // optional (r06c): ssq_out[M][N / 16] = sum of squares of the NEW residual values of (token, 16-column tile) — what an
@@ -65,25 +78,34 @@ struct RowsArgs {
     float *ssq_out;
 };
 
+constexpr int rows_waves_per_simd(int nch, int epi) { return epi != kRowsAdd && nch > 0 && nch <= 2 ? 4 : 2; }
+
 // NCH > 0: the chunk count per wave is a compile-time constant <= kRowsRing — every load is issued up front, straight-line
 // code with exact counted waits. NCH == 0: run-time chunk count, the ring refilled behind guards.
-template <typename T, int NCH, int MB, bool XLDS>
-__global__ __launch_bounds__(kRowsWaves * 64, 2) void gemm_rows_kernel(RowsArgs a) {
-    __shared__ __attribute__((aligned(16))) float red[kRowsWaves][32 * kRowsRedPitch];
+// Stores (EPI != kRowsAdd) take any N: the packed copy of a weight whose rows are no multiple of 32 ends with rows of zeros, and
+// columns from N on are not stored. With one or two chunks a wave needs half the registers, and two workgroups share a CU.
+template <typename T, int NCH, int MB, bool XLDS, int EPI>
+__global__ __launch_bounds__(kRowsWaves * 64, rows_waves_per_simd(NCH, EPI)) void gemm_rows_kernel(RowsArgs a) {
+    constexpr int kRing = NCH > 0 && NCH < kRowsRing ? NCH : kRowsRing;
     constexpr int XCK = 32 * kRowsCh;          // k per chunk (128): one 256-byte run per token
     constexpr int NXL = XLDS ? 4 * MB : kRowsCh * MB;   // x loads per chunk and lane (XLDS: 4 token rows each)
-    __shared__ __attribute__((aligned(16))) T xt[XLDS ? kRowsWaves : 1][XLDS ? 16 * MB * XCK : 8];
+    // a wave's x tile; its tile image takes the same place once the wave has multiplied (its LDS operations run in order)
+    constexpr int kXBytes = XLDS ? 16 * MB * XCK * 2 : 0, kRedBytes = 16 * MB * kRowsRedPitch * 4;
+    constexpr int kWaveBytes = kXBytes > kRedBytes ? kXBytes : kRedBytes;
+    __shared__ __attribute__((aligned(16))) char wave_lds[kRowsWaves][kWaveBytes];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int M = a.M, N = a.N, K = a.K;
     const int tile16 = blockIdx.x;
     const int n0 = tile16 * kRowsTile;
+    const auto red = [&](int w) { return reinterpret_cast<float *>(&wave_lds[w][0]); };
 
     // ---- epilogue operands first: the oldest requests of the wave, no wait of the stream ever includes them ----
     const int et = threadIdx.x >> 4, en = threadIdx.x & 15; // (token, column n0 + en)
-    const bool e_ok = et < M;
-    T *res_p = static_cast<T *>(a.residual) + static_cast<int64_t>(e_ok ? et : 0) * N + n0 + en;
-    const T rv = *res_p;
+    const bool e_ok = et < M && (EPI == kRowsAdd || n0 + en < N);
+    T *res_p = static_cast<T *>(a.residual) + static_cast<int64_t>(e_ok ? et : 0) * (EPI == kRowsAdd ? N : a.out_stride) + n0 + en;
+    T rv{};
+    if constexpr (EPI == kRowsAdd) rv = *res_p;
 
     // ---- the stream ----
     const int r = lane & 15, kq = lane >> 4;
@@ -114,9 +136,9 @@ __global__ __launch_bounds__(kRowsWaves * 64, 2) void gemm_rows_kernel(RowsArgs 
         for (int mb = 0; mb < MB; ++mb)
             xsrc[mb] = static_cast<const T *>(a.x) + static_cast<int64_t>(min(r + 16 * mb, M - 1)) * a.x_stride + 32 * s0 + 8 * kq;
     }
-    T *xtw = &xt[XLDS ? wave : 0][0];
+    T *xtw = reinterpret_cast<T *>(&wave_lds[wave][0]);
 
-    vec8_t<T> wr[kRowsRing][kRowsCh], xr[kRowsRing][NXL];
+    vec8_t<T> wr[kRing][kRowsCh], xr[kRing][NXL];
     float4_t acc[MB];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) acc[mb] = float4_t{0.f, 0.f, 0.f, 0.f};
@@ -151,28 +173,28 @@ __global__ __launch_bounds__(kRowsWaves * 64, 2) void gemm_rows_kernel(RowsArgs 
         // straight-line schedule, exact counted waits: the first min(NCH, ring) chunks are requested up front (K = 4096:
         // the whole K range of the wave), longer K (down_proj: 14 chunks) refills a slot as soon as it is multiplied
 #pragma unroll
-        for (int c = 0; c < (NCH < kRowsRing ? NCH : kRowsRing); ++c) SWL_ROWS_ISSUE(c, c);
+        for (int c = 0; c < kRing; ++c) SWL_ROWS_ISSUE(c, c);
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             // pinned: left alone the scheduler sinks requests between the MFMAs of earlier chunks (fewer live registers,
             // and nothing in flight while the wave multiplies)
             __builtin_amdgcn_sched_barrier(0);
-            SWL_ROWS_PROCESS(c % kRowsRing);
+            SWL_ROWS_PROCESS(c % kRing);
             __builtin_amdgcn_sched_barrier(0);
-            if (c + kRowsRing < NCH) SWL_ROWS_ISSUE(c % kRowsRing, c + kRowsRing);
+            if (c + kRing < NCH) SWL_ROWS_ISSUE(c % kRing, c + kRing);
         }
     } else {
 #pragma unroll
-        for (int c = 0; c < kRowsRing; ++c)
+        for (int c = 0; c < kRing; ++c)
             if (c < nch) SWL_ROWS_ISSUE(c, c);
-        for (int c0 = 0; c0 < nch; c0 += kRowsRing) {
+        for (int c0 = 0; c0 < nch; c0 += kRing) {
 #pragma unroll
-            for (int d = 0; d < kRowsRing; ++d) {
+            for (int d = 0; d < kRing; ++d) {
                 if (c0 + d < nch) {
                     __builtin_amdgcn_sched_barrier(0);
                     SWL_ROWS_PROCESS(d);
                     __builtin_amdgcn_sched_barrier(0);
-                    if (c0 + d + kRowsRing < nch) SWL_ROWS_ISSUE(d, c0 + d + kRowsRing);
+                    if (c0 + d + kRing < nch) SWL_ROWS_ISSUE(d, c0 + d + kRing);
                 }
             }
         }
@@ -186,12 +208,21 @@ __global__ __launch_bounds__(kRowsWaves * 64, 2) void gemm_rows_kernel(RowsArgs 
     mfma_results_ready<4>(acc[MB - 1]); // stored by DS instructions next (swl_common.h)
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
-        *reinterpret_cast<float4_t *>(&red[wave][(r + 16 * mb) * kRowsRedPitch + 4 * kq]) = acc[mb];
+        *reinterpret_cast<float4_t *>(red(wave) + (r + 16 * mb) * kRowsRedPitch + 4 * kq) = acc[mb];
     __syncthreads();
     float s = 0.f;
     if (MB == 2 || et < 16) {
 #pragma unroll
-        for (int w = 0; w < kRowsWaves; ++w) s += red[w][et * kRowsRedPitch + en]; // wave order = K order
+        for (int w = 0; w < kRowsWaves; ++w) s += red(w)[et * kRowsRedPitch + en]; // wave order = K order
+    }
+    if constexpr (EPI == kRowsStore) {
+        if (e_ok) *res_p = to_t<T>(s);
+        return;
+    }
+    if constexpr (EPI == kRowsRelu2) {
+        const float v = fmaxf(to_f(to_t<T>(s)), 0.f);
+        if (e_ok) *res_p = to_t<T>(v * v);
+        return;
     }
     // splitk_add_scale_kernel's arithmetic (rmsnorm.hip) on this thread's element
     const T xn = add_t<T>(to_t<T>(s), rv); // the projection is rounded, then the sum (rmsnorm.py:54-57)
@@ -204,18 +235,23 @@ __global__ __launch_bounds__(kRowsWaves * 64, 2) void gemm_rows_kernel(RowsArgs 
 }
 
 static bool rows_shape_ok(int M, int N, int K) {
-    return M > 0 && M <= 32 && N > 0 && N % 32 == 0 && K > 0 && K % (32 * kRowsWaves * kRowsCh) == 0;
+    return M > 0 && M <= 32 && N > 0 && N % 32 == 0 && K > 0 && K % kRowsKUnit == 0;
 }
 
-template <typename T, int MB, bool XLDS>
+template <typename T, int MB, bool XLDS, int EPI>
 static int launch_rows(const RowsArgs &a, hipStream_t stream) {
-    const dim3 grid(a.N / kRowsTile), block(kRowsWaves * 64);
+    const dim3 grid((a.N + kRowsTile - 1) / kRowsTile), block(kRowsWaves * 64);
     const int nch = a.K / (32 * kRowsWaves * kRowsCh);
     // K = 4096 (Llama-3-8B / Llama-2-7B hidden): 4 chunks, all in flight; 14336 (Llama-3-8B FFN): 14; 8192: 8
-    if (nch == 4) hipLaunchKernelGGL((gemm_rows_kernel<T, 4, MB, XLDS>), grid, block, 0, stream, a);
-    else if (nch == 14) hipLaunchKernelGGL((gemm_rows_kernel<T, 14, MB, XLDS>), grid, block, 0, stream, a);
-    else if (nch == 8) hipLaunchKernelGGL((gemm_rows_kernel<T, 8, MB, XLDS>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((gemm_rows_kernel<T, 0, MB, XLDS>), grid, block, 0, stream, a);
+    if constexpr (EPI != kRowsAdd) {
+        if (nch == 1) { hipLaunchKernelGGL((gemm_rows_kernel<T, 1, MB, XLDS, EPI>), grid, block, 0, stream, a); return check_launch(); }
+        if (nch == 2) { hipLaunchKernelGGL((gemm_rows_kernel<T, 2, MB, XLDS, EPI>), grid, block, 0, stream, a); return check_launch(); }
+    } else {
+        if (nch == 14) { hipLaunchKernelGGL((gemm_rows_kernel<T, 14, MB, XLDS, EPI>), grid, block, 0, stream, a); return check_launch(); }
+    }
+    if (nch == 4) hipLaunchKernelGGL((gemm_rows_kernel<T, 4, MB, XLDS, EPI>), grid, block, 0, stream, a);
+    else if (nch == 8) hipLaunchKernelGGL((gemm_rows_kernel<T, 8, MB, XLDS, EPI>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((gemm_rows_kernel<T, 0, MB, XLDS, EPI>), grid, block, 0, stream, a);
     return check_launch();
 }
 
@@ -225,6 +261,12 @@ static int launch_rows(const RowsArgs &a, hipStream_t stream) {
 static bool rows_x_through_lds(int M) {
     static const int forced = [] { const char *e = getenv("SWL_ROWS_X"); return !e ? 0 : e[0] == 'f' ? 1 : e[0] == 'l' ? 2 : 0; }();
     return forced ? forced == 2 : M > 8;
+}
+
+template <typename T, int EPI>
+static int launch_rows_m(const RowsArgs &a, hipStream_t s) {
+    if (rows_x_through_lds(a.M)) return a.M <= 16 ? launch_rows<T, 1, true, EPI>(a, s) : launch_rows<T, 2, true, EPI>(a, s);
+    return a.M <= 16 ? launch_rows<T, 1, false, EPI>(a, s) : launch_rows<T, 2, false, EPI>(a, s);
 }
 
 } // namespace swl
@@ -259,8 +301,24 @@ static int rows_add_impl(void *residual, float *ssq_out, const void *x, const vo
     a.M = M; a.N = N; a.K = K; a.x_stride = x_row_stride; a.ssq_out = ssq_out;
     SWL_DISPATCH_DTYPE(dtype, T, {
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        if (swl::rows_x_through_lds(M))
-            return M <= 16 ? swl::launch_rows<T, 1, true>(a, s) : swl::launch_rows<T, 2, true>(a, s);
-        return M <= 16 ? swl::launch_rows<T, 1, false>(a, s) : swl::launch_rows<T, 2, false>(a, s);
+        return swl::launch_rows_m<T, swl::kRowsAdd>(a, s);
+    });
+}
+
+/* out[M, N] = round(x . W^T), or relu(that)^2 rounded again (relu2 = 1): any N, the packed copy holding whole tiles of 32 rows. */
+extern "C" int swl_gemm_rows_store(void *out, const void *x, const void *w_packed, int32_t M, int32_t N, int32_t K,
+                                   int64_t x_row_stride, int64_t out_row_stride, int32_t relu2, int32_t dtype, swl_stream_t stream) {
+    if (M < 0 || N <= 0 || K <= 0 || relu2 < 0 || relu2 > 1) return SWL_ERR_BAD_ARG;
+    if (M == 0) return SWL_OK;
+    if (!out || !x || !w_packed) return SWL_ERR_BAD_ARG;
+    if (M > 32 || K % swl::kRowsKUnit != 0) return SWL_ERR_UNSUPPORTED;
+    if (x_row_stride < K || (x_row_stride & 7) || out_row_stride < N) return SWL_ERR_BAD_ARG;
+    if (!swl::aligned16(x) || !swl::aligned16(w_packed) || (reinterpret_cast<uintptr_t>(out) & 1u)) return SWL_ERR_BAD_ARG;
+    swl::RowsArgs a = {};
+    a.x = x; a.wp = w_packed; a.residual = out; a.out_stride = out_row_stride;
+    a.M = M; a.N = N; a.K = K; a.x_stride = x_row_stride;
+    SWL_DISPATCH_DTYPE(dtype, T, {
+        const hipStream_t s = static_cast<hipStream_t>(stream);
+        return relu2 ? swl::launch_rows_m<T, swl::kRowsRelu2>(a, s) : swl::launch_rows_m<T, swl::kRowsStore>(a, s);
     });
 }

@@ -16,7 +16,7 @@ from swiftllm_amd.model_config import KekapelModelConfig
 
 from .kekapel_weight import load_kekapel_weights
 from .kernels.layernorm import add_layernorm, embed_positions, layernorm
-from .kernels.linear import pack_weight, packable
+from .kernels.linear import pack_weight, packable_rows
 from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import KekapelAttention, KekapelFeedForward, _project
 from .stepped_model import SteppedModel
@@ -55,7 +55,7 @@ class KekapelModel(SteppedModel):
         skinny = bool(getattr(ecfg, "use_skinny_gemm", False)) and self.dtype != torch.float32
         if skinny and getattr(ecfg, "pack_decode_weights", False):
             for t in self.weight.projection_tensors():
-                if packable(t):
+                if packable_rows(t):
                     pack_weight(t)
         self._skinny = skinny
         eps = cfg.norm_eps

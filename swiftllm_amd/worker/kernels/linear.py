@@ -26,7 +26,7 @@ import torch.nn.functional as F
 from swiftllm_amd import _hip
 from . import route_tune
 
-_SKINNY_MAX_M = 32
+_SKINNY_MAX_M = ROWS_MAX_TOKENS = 32
 _workspaces = {}    # device -> persistent fp32 split-K scratch (fixed address: hipGraph replays use it)
 
 
@@ -58,10 +58,12 @@ def _row_stride(a: torch.Tensor) -> int:
 def pack_weight(w: torch.Tensor) -> torch.Tensor:
     """A copy of w[N, K] in MFMA-fragment order (csrc/gemm_skinny.hip, PACKED ring kernel), attached to `w` as
     `w._swl_packed` so that `linear(..., skinny=True)` and its split-K / SiLU-gate variants stream the packed copy
-    for decode-sized calls. Done once per weight at load time; call again after changing `w` in place."""
-    assert w.is_cuda and w.dim() == 2 and w.is_contiguous() and w.shape[0] % 32 == 0 and w.shape[1] % 128 == 0
-    wp = torch.empty_like(w)
-    _hip.call("swl_gemm_pack_weight", _hip.ptr(wp), _hip.ptr(w), w.shape[0], w.shape[1], _hip.dtype_code(w.dtype),
+    for decode-sized calls. Done once per weight at load time; call again after changing `w` in place. The copy holds whole
+    tiles of 32 rows, rows of zeros from N on (`linear_rows` alone reads such a copy)."""
+    assert w.is_cuda and w.dim() == 2 and w.is_contiguous() and w.shape[1] % 128 == 0
+    src = w if w.shape[0] % 32 == 0 else F.pad(w, (0, 0, 0, -w.shape[0] % 32))
+    wp = torch.empty_like(src)
+    _hip.call("swl_gemm_pack_weight", _hip.ptr(wp), _hip.ptr(src), src.shape[0], src.shape[1], _hip.dtype_code(w.dtype),
               _hip.stream())
     w._swl_packed = wp
     return wp
@@ -70,6 +72,38 @@ def pack_weight(w: torch.Tensor) -> torch.Tensor:
 def packable(w) -> bool:
     return (isinstance(w, torch.Tensor) and w.is_cuda and w.dim() == 2 and w.is_contiguous()
             and w.dtype in (torch.float16, torch.bfloat16) and w.shape[0] % 32 == 0 and w.shape[1] % 128 == 0)
+
+
+def _rows_serves(n: int, k: int) -> bool:
+    """The products of up to 32 tokens that the row-owned kernel (swl_gemm_rows_store) takes. us at 1 / 32 tokens, cold bf16
+    weights in a captured graph, against the packed ring kernel with its reduce launch (L: the library's, for rows that are no
+    multiple of 32): 1024 x 1024 2.7 / 3.8 (5.5 / 6.3), 4096 x 1024 3.4 / 4.3 (6.2 / 7.3), 3088 x 2048 4.1 / 6.0 (L 11.4 / 11.5),
+    8192 x 2048 7.6 / 10.4 (11.6 / 12.8), 16384 x 2048 13.2 / 18.6 (19.2 / 19.8), 4096 x 4096 7.3 / 10.3 (10.8 / 12.8). A workgroup
+    reads all of x for its 16 rows: beyond one workgroup a CU at K = 4096 (6144 rows: 12.1 / 17.9 against 12.6 / 14.3) and at
+    K = 8192 (2048 rows: 9.7 / 15.3 against 11.6 / 13.5) shares of K win."""
+    return k % 1024 == 0 and ((k <= 2048 and n <= 16384) or (k <= 4096 and n <= 4096))
+
+
+def packable_rows(w) -> bool:
+    """A weight that a packed copy serves in some decode step of the stepped designs: `packable`, or of any number of rows
+    that `linear_rows` takes."""
+    return packable(w) or (isinstance(w, torch.Tensor) and w.is_cuda and w.dim() == 2 and w.is_contiguous()
+                           and w.dtype in (torch.float16, torch.bfloat16) and _rows_serves(*w.shape))
+
+
+def linear_rows(a: torch.Tensor, w: torch.Tensor, relu2: bool = False):
+    """a[T, in] @ w[out, in]^T for up to 32 tokens in one launch without shares of K (csrc/gemm_rows.hip), `relu2`: squared ReLU of
+    the rounded product in the same launch; None where the kernel does not serve the call (`_rows_serves`)."""
+    wp = _packed_of(w)
+    if wp is None or not (a.is_cuda and a.dim() == 2 and 0 < a.shape[0] <= _SKINNY_MAX_M and a.dtype == w.dtype):
+        return None
+    m, (n, k) = a.shape[0], w.shape
+    if not _rows_serves(n, k) or a.shape[1] != k or a.stride(1) != 1 or (m > 1 and a.stride(0) % 8) or a.data_ptr() % 16:
+        return None
+    out = torch.empty((m, n), dtype=a.dtype, device=a.device)
+    _hip.call("swl_gemm_rows_store", _hip.ptr(out), _hip.ptr(a), _hip.ptr(wp), m, n, k, k if m == 1 else a.stride(0), n,
+              1 if relu2 else 0, _hip.dtype_code(a.dtype), _hip.stream())
+    return out
 
 
 def _packed_of(w: torch.Tensor):
@@ -106,12 +140,12 @@ def _mid_ok(a: torch.Tensor, w: torch.Tensor) -> bool:
     (swl_gemm_packed_mid). Measured against hipBLASLt (tools/gemm_micro.py --m 48/64): 20-30 % faster over a layer.
     (65..256 tokens: `_wide_ok`, csrc/gemm_wide.hip.)"""
     m = a.shape[0] if a.dim() == 2 else 0
-    if not (_SKINNY_MAX_M < m <= _MID_MAX_M) or _packed_of(w) is None:
+    if not (_SKINNY_MAX_M < m <= _MID_MAX_M) or _packed_of(w) is None or w.shape[0] % 32:
         return False
     return a.is_cuda and a.dtype == w.dtype and a.stride(1) == 1 and a.stride(0) % 8 == 0
 
 
-_WIDE_MAX_M = 256
+_WIDE_MAX_M = DECODE_MAX_TOKENS = 256
 
 
 def _launch_wide(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
@@ -256,6 +290,9 @@ def _blas_linear(a: torch.Tensor, w: torch.Tensor, row_blocks=None, plateau=None
     if start < m:
         torch.mm(a[start:], wt, out=out[start:])
     return out
+
+
+F32_MAX_TOKENS = 16     # (swl_gemm_f32_supported)
 
 
 def linear_f32(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

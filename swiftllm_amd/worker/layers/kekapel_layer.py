@@ -4,7 +4,8 @@ import torch
 
 from swiftllm_amd import _hip
 
-from ..kernels.linear import linear, linear_f32, linear_silu_gate, linear_splitk
+from ..kernels.linear import (DECODE_MAX_TOKENS, F32_MAX_TOKENS, ROWS_MAX_TOKENS, linear, linear_f32, linear_rows, linear_silu_gate,
+                              linear_splitk)
 from ..kernels.moe import ACT_SILU_UP_FIRST, gated_unit, moe_experts, moe_route
 from ..kernels.polynorm import polynorm
 from ..kernels.window_attn import qknorm_and_store_kv, window_attention
@@ -13,29 +14,39 @@ from ..kernels.window_attn import qknorm_and_store_kv, window_attention
 def _project(a: torch.Tensor, w: torch.Tensor, skinny: bool) -> torch.Tensor:
     """a [T, in] @ w[out, in]^T. bf16 / f16: the framework's projection routing (hand-written weight-streaming GEMMs for
     decode-sized batches, the BLAS otherwise); fp32: true fp32, with a kernel for a few tokens."""
+    m = a.shape[0]      # (asked for before anything else: the steps that nothing below serves pay for one comparison)
     if a.dtype == torch.float32:
-        return linear_f32(a, w)
-    if skinny and not getattr(w, "_swl_blas_only", False):
-        try:
-            return linear(a, w, True)
-        except _hip.HipLibraryError as exc:
-            # a projection shape the hand-written decode GEMMs are not specialised for (they say so with the "not supported"
-            # code): this weight goes through the BLAS from here on; any other failure is a real one
-            if "code -2" not in str(exc):
-                raise
-            w._swl_blas_only = True
+        return linear_f32(a, w) if m <= F32_MAX_TOKENS else torch.nn.functional.linear(a, w)
+    if not skinny or m > DECODE_MAX_TOKENS or getattr(w, "_swl_blas_only", False):
+        return linear(a, w, False)
+    y = linear_rows(a, w) if m <= ROWS_MAX_TOKENS else None
+    if y is not None:
+        return y
+    try:
+        return linear(a, w, True)
+    except _hip.HipLibraryError as exc:
+        # a projection shape the hand-written decode GEMMs are not specialised for (they say so with the "not supported"
+        # code): this weight goes through the BLAS from here on; any other failure is a real one
+        if "code -2" not in str(exc):
+            raise
+        w._swl_blas_only = True
     return linear(a, w, False)
 
 
 def _project_partials(a: torch.Tensor, w: torch.Tensor, skinny: bool):
     """_project for a consumer that takes a product's K shares too: SplitKPartials where the decode GEMM splits K, rows otherwise."""
-    if skinny and a.dtype != torch.float32 and not getattr(w, "_swl_blas_only", False):
-        try:
-            return linear_splitk(a, w)
-        except _hip.HipLibraryError as exc:
-            if "code -2" not in str(exc):       # (see _project)
-                raise
-            w._swl_blas_only = True
+    m = a.shape[0]
+    if not skinny or m > DECODE_MAX_TOKENS or a.dtype == torch.float32 or getattr(w, "_swl_blas_only", False):
+        return _project(a, w, skinny)
+    y = linear_rows(a, w) if m <= ROWS_MAX_TOKENS else None
+    if y is not None:
+        return y
+    try:
+        return linear_splitk(a, w)
+    except _hip.HipLibraryError as exc:
+        if "code -2" not in str(exc):       # (see _project)
+            raise
+        w._swl_blas_only = True
     return _project(a, w, skinny)
 
 

@@ -2,6 +2,7 @@
 stream and the next input norm are the model's fused step (kernels/rms_stream.py)."""
 import torch
 
+from ..kernels.linear import ROWS_MAX_TOKENS, linear_rows
 from ..kernels.moe import relu_squared
 from ..kernels.rope_kv import diff_head_combine, head_gate_, latent_rope_and_store_kv, rope_and_store_kv
 from ..kernels.window_attn import MASK_CHUNK, MASK_WINDOW, AttentionSpec, masked_attention
@@ -75,5 +76,7 @@ class RosilixFeedForward:
         self.mlp, self.w, self.skinny = layer_config.mlp, weight, skinny
 
     def forward(self, h: torch.Tensor, ctx: StepContext) -> torch.Tensor:
-        z = _project(h, self.w.up, self.skinny)
-        return _project_partials(relu_squared(z, self.mlp.ffn_inter_dim), self.w.down, self.skinny)
+        y = linear_rows(h, self.w.up, relu2=True) if self.skinny and h.shape[0] <= ROWS_MAX_TOKENS else None
+        if y is None:
+            y = relu_squared(_project(h, self.w.up, self.skinny), self.mlp.ffn_inter_dim)
+        return _project_partials(y, self.w.down, self.skinny)

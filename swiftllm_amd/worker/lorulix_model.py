@@ -23,7 +23,7 @@ from swiftllm_amd.model_config import LorulixModelConfig
 
 from .kernels.delta_rule import most_tiles_scratch
 from .kernels.layernorm import embed_positions
-from .kernels.linear import pack_weight, packable
+from .kernels.linear import pack_weight, packable_rows
 from .kernels.rms_stream import StateRef, causal_conv_state, gated_add_rmsnorm
 from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import _project
@@ -73,7 +73,7 @@ class LorulixModel(SteppedModel):
         skinny = bool(getattr(ecfg, "use_skinny_gemm", False)) and self.dtype != torch.float32
         if skinny and getattr(ecfg, "pack_decode_weights", False):
             for t in self.weight.projection_tensors():
-                if packable(t):
+                if packable_rows(t):
                     pack_weight(t)
         self._skinny = skinny
         eps, w, taps = cfg.norm_eps, cfg.hidden_size, cfg.canon_taps

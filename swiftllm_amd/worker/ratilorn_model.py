@@ -22,7 +22,7 @@ from swiftllm_amd.engine_config import EngineConfig
 from swiftllm_amd.model_config import RatilornModelConfig
 
 from .kernels.layernorm import embed_positions
-from .kernels.linear import pack_weight, packable
+from .kernels.linear import pack_weight, packable_rows
 from .kernels.linear_scan import SEGMENT_MAX_SCRATCH
 from .kernels.rms_stream import StateRef, gated_add_rmsnorm, post_norm_add
 from .kernels.window_attn import PoolSlice, StepTiles
@@ -71,7 +71,7 @@ class RatilornModel(SteppedModel):
         skinny = bool(getattr(ecfg, "use_skinny_gemm", False)) and self.dtype != torch.float32
         if skinny and getattr(ecfg, "pack_decode_weights", False):
             for t in self.weight.projection_tensors():
-                if packable(t):
+                if packable_rows(t):
                     pack_weight(t)
         self._skinny = skinny
         eps = cfg.norm_eps

@@ -22,7 +22,7 @@ from swiftllm_amd.engine_config import EngineConfig
 from swiftllm_amd.model_config import RokevikModelConfig
 
 from .kernels.hyper_stream import embed_streams, hyper_step
-from .kernels.linear import pack_weight, packable
+from .kernels.linear import pack_weight, packable_rows
 from .kernels.rms_stream import StateRef
 from .kernels.sampling import softcap_logits
 from .kernels.window_attn import PoolSlice, StepTiles, served_row_sizes
@@ -79,7 +79,7 @@ class RokevikModel(SteppedModel):
         skinny = bool(getattr(ecfg, "use_skinny_gemm", False)) and self.dtype != torch.float32
         if skinny and getattr(ecfg, "pack_decode_weights", False):
             for t in self.weight.projection_tensors():
-                if packable(t):
+                if packable_rows(t):
                     pack_weight(t)
         self._skinny = skinny
         # one slot per sequence that runs: as many as a batch holds

@@ -19,7 +19,7 @@ from swiftllm_amd.engine_config import EngineConfig
 from swiftllm_amd.model_config import RosilixModelConfig
 
 from .kernels.layernorm import embed_positions
-from .kernels.linear import pack_weight, packable
+from .kernels.linear import pack_weight, packable_rows
 from .kernels.rms_stream import gated_add_rmsnorm
 from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import _project
@@ -69,7 +69,7 @@ class RosilixModel(SteppedModel):
         skinny = bool(getattr(ecfg, "use_skinny_gemm", False)) and self.dtype != torch.float32
         if skinny and getattr(ecfg, "pack_decode_weights", False):
             for t in self.weight.projection_tensors():
-                if packable(t):
+                if packable_rows(t):
                     pack_weight(t)
         self._skinny = skinny
         eps = cfg.norm_eps

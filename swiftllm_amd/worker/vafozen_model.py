@@ -21,7 +21,7 @@ from swiftllm_amd.model_config import VafozenModelConfig
 
 from .kernels.hyper_stream import StreamWeights, hyper_step
 from .kernels.layernorm import embed_positions
-from .kernels.linear import pack_weight, packable
+from .kernels.linear import pack_weight, packable_rows
 from .kernels.linear_scan import SEGMENT_MAX_SCRATCH
 from .kernels.rms_stream import StateRef
 from .kernels.window_attn import PoolSlice, StepTiles, served_row_sizes
@@ -72,7 +72,7 @@ class VafozenModel(SteppedModel):
         skinny = bool(getattr(ecfg, "use_skinny_gemm", False)) and self.dtype != torch.float32
         if skinny and getattr(ecfg, "pack_decode_weights", False):
             for t in self.weight.projection_tensors():
-                if packable(t):
+                if packable_rows(t):
                     pack_weight(t)
         self._skinny = skinny
         self._plain = StreamWeights.plain(self.device)

@@ -49,6 +49,37 @@ def test_rows_add_is_one_rounding_of_the_product_plus_residual(dtype, M, N, K):
     assert torch.equal(res[M:], want_guard)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(8, 1024), (1000, 1024), (1, 2048), (3088, 2048), (545, 3072), (64, 4096), (40, 8192)])
+def test_rows_store_is_one_rounding_of_the_product(dtype, M, N, K):
+    """out = round(x . W^T), and relu(that)^2 rounded, for row counts that end inside a tile of 16 and of 32, every schedule (1, 2, 4,
+    8 chunks, the run-time ring) and both x paths; rows and columns beyond the result keep what they held. Bound: half an ulp of the
+    value in T and fp32 sums of K products (each partial sum rounds by 2^-24 of the magnitudes' sum, in any order)."""
+    from swiftllm_amd import _hip
+    from swiftllm_amd.worker.kernels.linear import _packed_of, linear_rows, pack_weight, packable_rows
+    g = gen(M + N + K)
+    x = torch.randn(M, K + 8, generator=g).to(dtype).cuda()[:, :K]
+    w = (torch.randn(N, K, generator=g) * 0.03).to(dtype).cuda()
+    pack_weight(w)
+    out = torch.full((M + 1, N + 3), 7.0, dtype=dtype, device="cuda")
+    z = out.clone()
+    for o, relu2 in ((out, 0), (z, 1)):
+        _hip.call("swl_gemm_rows_store", _hip.ptr(o), _hip.ptr(x), _hip.ptr(_packed_of(w)), M, N, K, K + 8, N + 3, relu2,
+                  _hip.dtype_code(dtype), _hip.stream())
+    want = x.double() @ w.double().T
+    bound = want.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) + K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 2.0 ** -24
+    assert ((out[:M, :N].double() - want).abs() <= bound).all()
+    assert torch.equal(z[:M, :N], (torch.relu(out[:M, :N].float()) ** 2).to(dtype))
+    for o in (out, z):
+        assert (o[M:] == 7).all() and (o[:, N:] == 7).all()
+    if packable_rows(w) and K <= 4096 and K != 3072:
+        assert torch.equal(linear_rows(x, w), out[:M, :N]) and torch.equal(linear_rows(x, w, relu2=True), z[:M, :N])
+        assert linear_rows(torch.zeros(33, K, dtype=dtype, device="cuda"), w) is None
+        odd = torch.zeros(M * K + 1, dtype=dtype, device="cuda")[1:].view(M, K)
+        assert linear_rows(odd, w) is None          # (rows that do not begin on 16 bytes stay with the general paths)
+
+
 @pytest.mark.parametrize("M", [1, 8, 32])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (4096, 14336)])
 def test_rows_add_carries_the_bits_of_splitk_plus_consumer(M, N, K):
