@@ -619,6 +619,16 @@ int swl_span_attn(void *out, const void *q, const void *k_cache, const void *v_c
                   int32_t mask_kind, float scale, float softcap, int32_t max_blocks_per_seq, int64_t block_stride,
                   int32_t key_splits, float *scratch, int64_t num_tokens, const float *sink, int32_t out_f32, const float *slopes,
                   int32_t out_dim, int64_t out_stride, const void *gate, int64_t gate_stride, int32_t dtype, swl_stream_t stream);
+/* The same with the order in which workgroups take the spans up (a permutation of them on the device; NULL: last to first). The spans that
+ * see the most keys belong first, four neighbours of a portion together. Results do not depend on it.
+ * longest: tokens of the step's longest sequence (0: not known), for the choice of rows a workgroup. */
+int swl_span_attn_ordered(const int32_t *span_order, int32_t longest, void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
+                  const int32_t *tok_seq, const int32_t *tok_pos, const int32_t *tok_start, const int32_t *span_row0,
+                  const int32_t *span_cnt, const float *rel, int32_t rel_len, int32_t num_spans, int32_t num_q_heads,
+                  int32_t num_kv_heads, int32_t num_v_heads, int32_t dim, int32_t vdim, int64_t q_tok_stride, int32_t window,
+                  int32_t mask_kind, float scale, float softcap, int32_t max_blocks_per_seq, int64_t block_stride,
+                  int32_t key_splits, float *scratch, int64_t num_tokens, const float *sink, int32_t out_f32, const float *slopes,
+                  int32_t out_dim, int64_t out_stride, const void *gate, int64_t gate_stride, int32_t dtype, swl_stream_t stream);
 
 /* swl_window_attn_tiles / swl_sigmoid_attn_tiles with a mixing matrix (csrc/mix_attn.hip) for steps that bring prompt portions: at most
  * 16 query heads; the same tiles, masks and scratch ([splits][tokens][heads] x (vdim + 2) floats, sigmoid: x vdim). q, k_cache and

@@ -115,6 +115,8 @@ SIGNATURES = {
                               _I32, _P],
     "swl_span_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _I32,
                       _F32, _F32, _I32, _I64, _I32, _P, _I64, _P, _I32, _P, _I32, _I64, _P, _I64, _I32, _P],
+    "swl_span_attn_ordered": [_P, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _I32,
+                              _F32, _F32, _I32, _I64, _I32, _P, _I64, _P, _I32, _P, _I32, _I64, _P, _I64, _I32, _P],
     "swl_mix_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _F32, _F32, _I32, _I64, _I32,
                      _P, _I64, _I32, _P],
     "swl_mix_sigmoid_attn": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _F32, _I32,

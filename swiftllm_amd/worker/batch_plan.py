@@ -178,6 +178,17 @@ class StepPlan:
     SEGMENTS = ("input_ids", "tok_pos", "tok_seq", "want_rows", "tile_row0", "tile_cnt", "seq_row0", "seq_cnt", "tok_start",
                 "tok_state", "chunk_row0", "chunk_cnt", "seq_chunk0", "seq_tile0")
 
+    def span_order(self):
+        """The chunks in the order in which attention takes them up, int32: runs of four of a portion (128 tokens, nearly the same
+        keys) together, the runs at the highest positions first. None for steps so small that all are taken up at once."""
+        n = self.chunk_row0.size
+        if n <= 64:
+            return None
+        portion = np.repeat(np.arange(self.num_seqs), np.diff(self.seq_chunk0, append=n))
+        first = self.tok_pos[self.chunk_row0] - ((np.arange(n) - self.seq_chunk0[portion]) & 3) * self.CHUNK      # position of the run
+        key = first.astype(np.int64) * self.num_seqs + portion
+        return (n - 1 - np.argsort(-key[::-1], kind="stable")).astype(np.int32)
+
     def packed_layout(self):
         out, off = [], 0
         for name in self.SEGMENTS:

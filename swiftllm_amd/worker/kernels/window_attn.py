@@ -98,16 +98,18 @@ def qkv_bias_norm_store(qkv: torch.Tensor, q_b: torch.Tensor, k_b: torch.Tensor,
 
 class StepTiles(tuple):
     """(tile_row0, tile_cnt) of a step, and its spans: runs of up to 32 consecutive tokens of one portion (row0, cnt, and per token
-    the position where its portion starts). longest: the longest sequence of the step (spans only: never under graph replay)."""
+    the position where its portion starts). longest: the longest sequence of the step (spans only: never under graph replay).
+    span_order: the spans in the order to take them up (StepPlan.span_order; None: last to first)."""
 
-    def __new__(cls, tile_row0, tile_cnt, spans=None, longest=0):
+    def __new__(cls, tile_row0, tile_cnt, spans=None, longest=0, span_order=None):
         self = super().__new__(cls, (tile_row0, tile_cnt))
-        self.spans, self.longest = spans, longest
+        self.spans, self.longest, self.span_order = spans, longest, span_order
         return self
 
     @classmethod
     def of(cls, dev):
-        return cls(dev["tile_row0"], dev["tile_cnt"], (dev["chunk_row0"], dev["chunk_cnt"], dev["tok_start"]), dev.get("longest", 0))
+        return cls(dev["tile_row0"], dev["tile_cnt"], (dev["chunk_row0"], dev["chunk_cnt"], dev["tok_start"]), dev.get("longest", 0),
+                   dev.get("span_order"))
 
 
 # A step whose spans hold this many tokens on average or more is a prompt step (a span of one token fills one of a workgroup's 128 rows a
@@ -130,13 +132,15 @@ def _span_launch(q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles, H, 
     if (q.data_ptr() | kp | vp) % 16 or q.stride(0) % 8 or pool.shape[1] % 8:      # 16-byte operand loads
         return False
     row0, cnt, start = spans
-    # workgroups of 128 rows (queries x heads of a key head); with fewer than fill the chip, every tile's keys are shared out
-    groups = max(1, n * H // (128 * G)) * G
+    # workgroups of 64 rows (queries x heads of a key head; wide rows: 128). Few of them: every tile's keys are shared out, many only where
+    # the walk is long, as partial results cost a launch and their bytes. us by shares, 8 heads of 128 over 2: 57 tokens at 17 to 692
+    # 18.5 (1), 15.2 (3), 14.4 (8); 500 tokens 15.5 (1), 17.7 (2), 16.0 (4); 1500 33.9 (1), 36.5 (2); 2000 beside 30 decoded 29 (1), 39 (2), 42 (4)
+    groups = max(1, n * H // ((64 if dim + vdim <= 320 else 128) * G)) * G
     pages = (min(window, tiles.longest) if window > 0 else tiles.longest) // 16 + 1
-    splits = max(1, min(2 * _NUM_CUS // groups, pages // 8, 8))
+    splits = max(1, min(_NUM_CUS // groups, pages // (8 if groups <= 32 else 32), 8))
     splits, scratch = share_scratch(q.device, splits, n * H * (vdim + 2))
-    _hip.call("swl_span_attn", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq), _hip.ptr(tok_pos),
-              _hip.ptr(start), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(rel), rel.shape[1] if rel is not None else 0, row0.shape[0],
+    _hip.call("swl_span_attn_ordered", _hip.ptr(tiles.span_order), tiles.longest, _hip.ptr(out), _hip.ptr(q), kp, vp,
+              _hip.ptr(block_table), _hip.ptr(tok_seq), _hip.ptr(tok_pos), _hip.ptr(start), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(rel), rel.shape[1] if rel is not None else 0, row0.shape[0],
               H, G, GV, dim, vdim, q.stride(0), window, mask_kind, float(scale), float(softcap), block_table.shape[1], pool.shape[1],
               splits, _hip.ptr(scratch), n, _hip.ptr(sink), int(out_f32), _hip.ptr(slopes), vdim if out_dim is None else out_dim,
               out.stride(0), _hip.ptr(gate), gate.stride(0) if gate is not None else 0, _hip.dtype_code(q.dtype), _hip.stream())

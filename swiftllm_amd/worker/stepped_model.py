@@ -161,6 +161,8 @@ class SteppedModel:
     def _upload_plan(self, plan: StepPlan):
         """The plan's int32 arrays through ONE pinned buffer and ONE async copy; returns device views."""
         layout, total = plan.packed_layout()
+        order = plan.span_order()
+        order_at, total = total, total + (order.size if order is not None else 0)
         if self._meta_done is not None:
             self._meta_done.synchronize()
         if self._meta_host is None or self._meta_host.numel() < total:
@@ -174,9 +176,14 @@ class SteppedModel:
             self._decode_graphs.clear()
             self._graph_pool = None
         plan.pack_into(self._meta_host_np)
+        if order is not None:
+            self._meta_host_np[order_at:total] = order
         self._meta_dev[:total].copy_(self._meta_host[:total], non_blocking=True)
         self._meta_done.record()
-        return _PlanViews(self._meta_dev, layout)
+        dev = _PlanViews(self._meta_dev, layout)
+        if order is not None:
+            dev["span_order"] = self._meta_dev[order_at:total]
+        return dev
 
     def _begin_state_step(self, plan: StepPlan):
         """Per-sequence state: slots for the sequences of this step, their codes into the plan."""

@@ -155,3 +155,27 @@ def test_key_shares(case, shares, dtype, monkeypatch):
     monkeypatch.setattr(window_attn, "share_scratch", forced)
     test_span_attention(case, [(1, 96, 31), (2, 0, 64), (3, 250, 1), (4, 15, 130)], dtype)
     assert used == [shares, shares]
+
+
+@pytest.mark.parametrize("H,G,d,dv,window", [(8, 2, 128, 128, 0), (4, 4, 64, 64, 100), (6, 2, 192, 128, 0), (8, 1, 576, 512, 300),
+                                             (2, 1, 320, 256, 0), (3, 1, 64, 128, 0)])
+def test_spans_in_any_order(H, G, d, dv, window):
+    """Steps of more than 64 spans take them up in the plan's order: the same bits as last to first (which the oracle checks above), for
+    fewer workgroups than CUs, up to two a CU (taken from both ends) and more, whole and broken runs of spans and all key heads."""
+    from swiftllm_amd.worker.batch_plan import StepEntry, plan_step
+    from swiftllm_amd.worker.kernels import window_attn
+    g = torch.Generator().manual_seed(H)
+    for parts in ([(1, 0, 1500), (2, 33, 700), (3, 77, 1)], [(1, 0, 2000), (2, 0, 1999), (3, 5, 1), (4, 100, 1234)],
+                  [(i, 16 * i, 1700 - 100 * i) for i in range(8)]):
+        pool, sl, table, _, _ = _pool([a + n for _, a, n in parts], G, G, d, dv, torch.bfloat16, g)
+        seq, pos, tiles = _spans(parts)
+        order = plan_step([StepEntry(i, [1] * n, a) for i, a, n in parts]).span_order()
+        assert sorted(order) == list(range(tiles.spans[0].shape[0]))
+        q = torch.randn(seq.shape[0], H * d, generator=g).to(torch.bfloat16).cuda()
+        tiles.longest = 0           # (no key shares)
+        out = []
+        for tiles.span_order in (None, torch.from_numpy(order).cuda()):
+            out.append(torch.full((seq.shape[0], H * dv), 7.0, dtype=torch.bfloat16, device="cuda"))
+            assert window_attn._span_launch(q, out[-1], pool.data_ptr() + sl.k_offset * 2, pool.data_ptr() + sl.v_offset * 2, pool, table, seq,
+                                            pos, tiles, H, G, G, d, dv, window, 0, d ** -0.5, 0.0)
+        assert torch.equal(out[0], out[1]) and not bool((out[0] == 7.0).all(1).any())

@@ -69,3 +69,20 @@ def test_positions_end_with_32_bits():
     for start in ((1 << 31) - 1, 1 << 31):
         with pytest.raises(OverflowError):
             plan_step([StepEntry(1, [3, 4], start)])
+
+
+def test_span_order_takes_runs_of_four_from_the_highest_positions():
+    """A permutation; runs of four chunks of a portion stay together, last chunk first; runs come in descending position; small steps have
+    none."""
+    assert plan_step([StepEntry(0, [1] * 2048, 0)]).span_order() is None        # (64 chunks)
+    parts = [(0, 0, 1000), (1, 77, 1), (2, 40, 900), (3, 0, 31), (4, 5, 385)]
+    plan = plan_step([StepEntry(i, [1] * n, a) for i, a, n in parts])
+    order = plan.span_order()
+    assert order.dtype == np.int32 and sorted(order) == list(range(plan.chunk_row0.size))
+    runs, at = [], 0
+    for i, a, n in parts:
+        chunks = -(-n // 32)
+        runs += [(a + 128 * k, i, [at + c for c in range(min(4 * k + 4, chunks) - 1, 4 * k - 1, -1)]) for k in range(-(-chunks // 4))]
+        at += chunks
+    runs.sort(key=lambda r: (-r[0], -r[1]))
+    assert order.tolist() == [c for r in runs for c in r[2]]
