@@ -6,6 +6,30 @@
 
 namespace swl {
 
+// Eight fp32 weights as two 16-bit terms each. bf16 in pairs: one conversion for two, and the first term as fp32 is a shift or a mask.
+__device__ __forceinline__ void split_weights(const float (&x)[8], vec8_t<bf16> &hi, vec8_t<bf16> &lo) {
+    typedef float float2_t __attribute__((ext_vector_type(2)));
+    typedef bf16 bf2_t __attribute__((ext_vector_type(2)));
+    typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+    uint4v h, l;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{x[2 * j], x[2 * j + 1]}), bf2_t));
+        const float2_t r = {x[2 * j] - __uint_as_float(u << 16), x[2 * j + 1] - __uint_as_float(u & 0xffff0000u)};
+        h[j] = u;
+        l[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf2_t));
+    }
+    hi = __builtin_bit_cast(vec8_t<bf16>, h);
+    lo = __builtin_bit_cast(vec8_t<bf16>, l);
+}
+__device__ __forceinline__ void split_weights(const float (&x)[8], vec8_t<f16> &hi, vec8_t<f16> &lo) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        hi[j] = to_t<f16>(x[j]);
+        lo[j] = to_t<f16>(x[j] - to_f(hi[j]));
+    }
+}
+
 // out[t][h][:] = sum_s e^{m_s - M} O_s / sum_s e^{m_s - M} l_s over the key shares s (a share without keys has l = 0).
 // The first wave evaluates the shares' weights once (one share per lane, at most 64) and leaves them in LDS.
 // NATURAL: the maxima are in natural units (the per-token kernel, whose arithmetic is full-precision throughout).

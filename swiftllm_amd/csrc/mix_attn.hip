@@ -11,10 +11,13 @@
 // blocks of pairs a wave; its result goes back the same way. The VALU mix it replaces read every head's scores from LDS in every wave
 // and spent H FMAs per score. A pair's place in a row is (lane of its owner) x 8 + key % 8: owners write and read 32 bytes a lane, and
 // the row pitches (528 and 516 floats) keep the transposed accesses on different banks. The key that A row m of a score product takes
-// is chosen as in span_attn.hip, so that a lane's eight scores are eight consecutive keys, the B operand of the value product.
-// Tiles are taken from the back: the long ones start first.
+// is chosen as in span_attn.hip, so that a lane's eight scores are eight consecutive keys, the B operand of the value product. The score products of a stage are
+// made where the weights of the one before are: one uses the matrix core, the other the vector units. Tiles are taken from the back: the long ones start first.
 // Measured, 16 heads of 128 over 4, bf16, against the 16-query tiles with the mix on the VALU: softmax, 3 prompts of 1500 tokens, window 1024
-// 697 -> 143 us; sigmoid, 11 prompts of 333 tokens 231 -> 61 us.
+// 697 -> 143 us; sigmoid, 11 prompts of 333 tokens 231 -> 61 us. With the score products of a stage beside the weights of the one before, the
+// reads of the mix together and no load that only some paths make (each is waited for on all of them, with what was asked for before it):
+// softmax 139 -> 130 us, sigmoid 71 us both (the same prompts, in a step). Vector instructions, 3500 cycles a stage, and matrix steps, 2600,
+// still run mostly one after the other.
 #include "attn_combine.h"
 #include "swl_common.h"
 
@@ -74,14 +77,15 @@ __global__ __launch_bounds__(kMxThreads, 2) void mix_attn_kernel(MixParams p) {
     // rows of the mix that belong to no head: zero once, so that their products with a zero of talk are zero
     for (int i = H * kMxIn + tid; i < HM * kMxIn; i += kMxThreads) s_in[i] = 0.f;
     // A operand of the mix: talk[h = li][g = 4 s + lq]; softmax scores come out in base-2 exponent units
-    const int steps = (H + 3) / 4;
-    float mixw[4];
+    constexpr int STEPS = 2 * HPW;              // (eight heads or fewer: one a wave, two steps; rows of no head are zero on both sides)
+    float mixw[STEPS];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < STEPS; ++s) {
         const int g = 4 * s + lq;
         mixw[s] = li < H && g < H ? p.talk[li * H + g] * (SIG ? 1.0f : kLog2e) : 0.f;
     }
-    vec8_t<T> qf[HPW][KS], kf[2][KS];
+    vec8_t<T> qf[HPW][KS], kf[2][KS], vf[CT];
+    const T *v_now = nullptr, *v_next = nullptr;        // values of the stage at hand and of the one whose keys were asked for last
     float4_t acc[HPW][CT];
     float mrun[HPW], lrun[HPW], hr1[HPW], hr2[HPW], hpb[HPW];
 #pragma unroll
@@ -106,49 +110,50 @@ __global__ __launch_bounds__(kMxThreads, 2) void mix_attn_kernel(MixParams p) {
     const T *kc = static_cast<const T *>(p.k_cache) + (static_cast<int64_t>(kv) * 16 + (8 * (li >> 2) & 15) + (li & 3)) * D + 8 * lq;
     const T *vc = static_cast<const T *>(p.v_cache) + (static_cast<int64_t>(kv) * DV + li) * 16 + 8 * (lq & 1);
     const int nstages = kb1 >= kb0 ? (kb1 - kb0) / 2 + 1 : 0;
-    auto block_of = [&](int st, int half) { return bt[min(kb0 + 2 * st + half, kb1)]; };     // (past the last page: that page again)
-    auto fetch_k = [&](int b0, int b1) {
+    // (scalar loads: a vector load of the ids inside the walk would be waited for with all keys and values that are on their way)
+    const auto *ids = (const __attribute__((address_space(4))) int32_t *)bt;
+    int b0 = 0, b1 = 0;
+    auto fetch_ids = [&](int st) {      // past the last page: that page again
+        b0 = ids[min(kb0 + 2 * st, kb1)];
+        b1 = ids[min(kb0 + 2 * st + 1, kb1)];
+    };
+    auto fetch_k = [&]() {
         const T *kp = kc + static_cast<int64_t>(li >> 3 ? b1 : b0) * p.block_stride;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int e = 0; e < KS; ++e) kf[t][e] = load8(kp + 4 * t * D + 32 * e);
+        v_next = vc + static_cast<int64_t>(lq >> 1 ? b1 : b0) * p.block_stride;
     };
-    int b0 = 0, b1 = 0, n0 = 0, n1 = 0;
-    if (nstages > 0) {
-        b0 = block_of(0, 0);
-        b1 = block_of(0, 1);
-        fetch_k(b0, b1);
-        n0 = block_of(min(1, nstages - 1), 0);
-        n1 = block_of(min(1, nstages - 1), 1);
-    }
-    __syncthreads();        // (the zero rows)
-    for (int st = 0; st < nstages; ++st) {
-        const int k0 = (kb0 + 2 * st) * 16, kd = qpos - k0 - 8 * lq, lo = qlo - k0 - 8 * lq;     // visible: lo <= key - (k0 + 8 lq) <= kd
-        // ---- 1. scores of this wave's heads -> LDS ------------------------------------------------------------------------------
-        vec8_t<T> vf[CT];
-        {
-            const T *vp = vc + static_cast<int64_t>(lq >> 1 ? b1 : b0) * p.block_stride;
+    auto fetch_v = [&]() {
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct) vf[ct] = load8(vp + ct * 256);
-        }
+        for (int ct = 0; ct < CT; ++ct) vf[ct] = load8(v_now + ct * 256);
+    };
+    // scores of a stage: the products of this wave's heads, and what is done to them on their way to LDS
+    float4_t sc[HPW][2];
+    auto products = [&]() {     // (a wave without heads goes along: what it makes is not stored)
 #pragma unroll
         for (int hh = 0; hh < HPW; ++hh) {
+            sc[hh][0] = sc[hh][1] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < KS; ++e)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) sc[hh][t] = mx_mfma(kf[t][e], qf[hh][e], sc[hh][t]);
+        }
+    };
+    auto hand_in = [&](int st) {
+        const int k0 = (kb0 + 2 * st) * 16, kd = qpos - k0 - 8 * lq, lo = qlo - k0 - 8 * lq;     // visible: lo <= key - (k0 + 8 lq) <= kd
+#pragma unroll
+        for (int hh = 0; hh < HPW; ++hh) {
+            mfma_results_tie(sc[hh][0]);
+            mfma_results_ready<8>(sc[hh][1]);
             if (hh < nh) {
-                float4_t s[2];
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    s[t] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int e = 0; e < KS; ++e) s[t] = mx_mfma(kf[t][e], qf[hh][e], s[t]);
-                }
-                mfma_results_tie(s[0]);
-                mfma_results_ready<8>(s[1]);
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
+                    float4_t s = sc[hh][t];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {       // key 8 lq + 4 t + r of the stage
-                        float x = s[t][r];
+                        float x = s[r];
                         if constexpr (SIG) {
                             const int at = 4 * t + r;
                             float z = fmaf(x, c_mul, hpb[hh]);
@@ -159,97 +164,111 @@ __global__ __launch_bounds__(kMxThreads, 2) void mix_attn_kernel(MixParams p) {
                         } else {
                             x *= c_mul;
                         }
-                        s[t][r] = x;
+                        s[r] = x;
                     }
-                    *reinterpret_cast<float4_t *>(s_in + (h0 + hh) * kMxIn + lane * 8 + 4 * t) = s[t];
+                    *reinterpret_cast<float4_t *>(s_in + (h0 + hh) * kMxIn + lane * 8 + 4 * t) = s;
                 }
             }
         }
+    };
+    if (nstages > 0) {
+        fetch_ids(0);
+        fetch_k();
+        v_now = v_next;
+        products();
+        fetch_ids(1);
+        fetch_k();
+        __builtin_amdgcn_sched_barrier(0);      // (the order of the walk: keys, then values)
+        fetch_v();
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();        // (the zero rows)
+    if (nstages > 0) hand_in(0);
+    for (int st = 0; st < nstages; ++st) {
+        const int k0 = (kb0 + 2 * st) * 16, kd = qpos - k0 - 8 * lq, lo = qlo - k0 - 8 * lq;     // visible: lo <= key - (k0 + 8 lq) <= kd
         __syncthreads();
-        b0 = n0;
-        b1 = n1;
-        if (st + 1 < nstages) {
-            fetch_k(b0, b1);
-            n0 = block_of(min(st + 2, nstages - 1), 0);
-            n1 = block_of(min(st + 2, nstages - 1), 1);
-        }
-        // ---- 2. the mix: blocks 4 wave .. 4 wave + 3 of 16 pairs -------------------------------------------------------------------
+        fetch_ids(st + 2);      // (past the last stage: its keys again. A load that only some paths make is waited for on all of them)
+        // ---- 1. the mix: blocks 4 wave .. 4 wave + 3 of 16 pairs -------------------------------------------------------------------
         {
             float4_t m[4];
-            float b[4][4];
+            float b[4][STEPS];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 m[u] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int s = 0; s < 4; ++s) b[u][s] = s < steps ? s_in[(4 * s + lq) * kMxIn + (4 * wave + u) * 16 + li] : 0.f;
+                for (int s = 0; s < STEPS; ++s) b[u][s] = s_in[(4 * s + lq) * kMxIn + (4 * wave + u) * 16 + li];
             }
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                if (s < steps) {        // (uniform)
+            for (int s = 0; s < STEPS; ++s)
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) m[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(mixw[s], b[u][s], m[u], 0, 0, 0);
-                }
-            }
+                for (int u = 0; u < 4; ++u) m[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(mixw[s], b[u][s], m[u], 0, 0, 0);
 #pragma unroll
             for (int u = 0; u < 3; ++u) mfma_results_tie(m[u]);
             mfma_results_ready<8>(m[3]);
+            __builtin_amdgcn_sched_group_barrier(0x100, 2 * STEPS, 0);     // (the LDS reads together, before the first matrix step)
+            __builtin_amdgcn_sched_group_barrier(0x008, 4 * STEPS, 0);
 #pragma unroll
             for (int u = 0; u < 4; ++u)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) s_out[(4 * lq + r) * kMxOut + (4 * wave + u) * 16 + li] = m[u][r];
         }
         __syncthreads();
+        // ---- 2. score products of the next stage, which the matrix core works off beside the weights of this one -------------------
+        const T *v_after = v_next;
+        products();
+        fetch_k();
         // ---- 3. weights and value products of this wave's heads ---------------------------------------------------------------------
 #pragma unroll
         for (int hh = 0; hh < HPW; ++hh) {
-            if (hh < nh) {
-                float x[8];
+            float x[8];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const float4_t v = *reinterpret_cast<const float4_t *>(s_out + (h0 + hh) * kMxOut + lane * 8 + 4 * t);
+            for (int t = 0; t < 2; ++t) {
+                const float4_t v = *reinterpret_cast<const float4_t *>(s_out + (h0 + hh) * kMxOut + lane * 8 + 4 * t);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) x[4 * t + r] = v[r];
-                }
-                if constexpr (!SIG) {
-                    float mx = kNegBig;
+                for (int r = 0; r < 4; ++r) x[4 * t + r] = v[r];
+            }
+            if constexpr (!SIG) {
+                if (k0 + kMxKeys - 1 > p0 || (p.window > 0 && k0 < p0 + cnt - p.window)) {        // (uniform) the keys cross a query's limits
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) {
+                    for (int j = 0; j < 8; ++j)
                         if (j > kd || j < lo) x[j] = kNegBig;
-                        mx = fmaxf(mx, x[j]);
-                    }
-                    mx = mx_rows_max(mx);
-                    // lazy running maximum: a row moves its reference only when a stage raises it by more than kLazy
-                    const float mnew = mx - mrun[hh] > kLazy ? mx : mrun[hh];
-                    const float alpha = fast_exp2(mrun[hh] - mnew);
-                    mrun[hh] = mnew;
-                    const float mref = mnew < 0.5f * kNegBig ? 0.f : mnew;
-                    float psum = 0.f;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        x[j] = fast_exp2(x[j] - mref);
-                        psum += x[j];
-                    }
-                    lrun[hh] = fmaf(lrun[hh], alpha, psum);
-                    if (!__all(alpha == 1.0f)) {
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) acc[hh][ct][r] *= alpha;
-                    }
                 }
-                vec8_t<T> phi, plo;
+                float mx = x[0];
+#pragma unroll
+                for (int j = 1; j < 8; ++j) mx = fmaxf(mx, x[j]);
+                mx = mx_rows_max(mx);
+                // lazy running maximum: a row moves its reference only when a stage raises it by more than kLazy
+                const float mnew = mx - mrun[hh] > kLazy ? mx : mrun[hh];
+                const float alpha = fast_exp2(mrun[hh] - mnew);
+                mrun[hh] = mnew;
+                const float mref = mnew < 0.5f * kNegBig ? 0.f : mnew;
+                float psum = 0.f;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    phi[j] = to_t<T>(x[j]);
-                    plo[j] = to_t<T>(x[j] - to_f(phi[j]));
+                    x[j] = fast_exp2(x[j] - mref);
+                    psum += x[j];
                 }
+                lrun[hh] = fmaf(lrun[hh], alpha, psum);
+                if (!__all(alpha == 1.0f)) {
 #pragma unroll
-                for (int ct = 0; ct < CT; ++ct) {
-                    acc[hh][ct] = mx_mfma(vf[ct], phi, acc[hh][ct]);
-                    acc[hh][ct] = mx_mfma(vf[ct], plo, acc[hh][ct]);
+                    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[hh][ct][r] *= alpha;
                 }
             }
+            vec8_t<T> phi, plo;
+            split_weights(x, phi, plo);
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                acc[hh][ct] = mx_mfma(vf[ct], phi, acc[hh][ct]);
+                acc[hh][ct] = mx_mfma(vf[ct], plo, acc[hh][ct]);
+            }
         }
+        __builtin_amdgcn_sched_barrier(0);
+        v_now = v_after;
+        fetch_v();
+        __builtin_amdgcn_sched_barrier(0);
+        if (st + 1 < nstages) hand_in(st + 1);
     }
     // ---- epilogue: acc[hh][ct][r] = O[query li][head][ct * 16 + 4 lq + r] --------------------------------------------------------
 #pragma unroll

@@ -75,30 +75,6 @@ __device__ __forceinline__ float span_row_sum(float v) {
     return v + __shfl_xor(v, 32, 64);
 }
 
-// Eight fp32 weights as two 16-bit terms each. bf16 in pairs: one conversion for two, and the first term as fp32 is a shift or a mask.
-__device__ __forceinline__ void span_split(const float (&x)[8], vec8_t<bf16> &hi, vec8_t<bf16> &lo) {
-    typedef float float2_t __attribute__((ext_vector_type(2)));
-    typedef bf16 bf2_t __attribute__((ext_vector_type(2)));
-    typedef unsigned uint4v __attribute__((ext_vector_type(4)));
-    uint4v h, l;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{x[2 * j], x[2 * j + 1]}), bf2_t));
-        const float2_t r = {x[2 * j] - __uint_as_float(u << 16), x[2 * j + 1] - __uint_as_float(u & 0xffff0000u)};
-        h[j] = u;
-        l[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf2_t));
-    }
-    hi = __builtin_bit_cast(vec8_t<bf16>, h);
-    lo = __builtin_bit_cast(vec8_t<bf16>, l);
-}
-__device__ __forceinline__ void span_split(const float (&x)[8], vec8_t<f16> &hi, vec8_t<f16> &lo) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        hi[j] = to_t<f16>(x[j]);
-        lo[j] = to_t<f16>(x[j] - to_f(hi[j]));
-    }
-}
-
 // N matrix steps whose operand comes from LDS, AHEAD of them on their way. (Left alone, the compiler reads every fragment right in
 // front of its step: a latency of LDS for each.)
 template <int AHEAD, int N, int MFMAS, typename V, typename Load, typename Step>
@@ -381,7 +357,7 @@ __global__ __launch_bounds__(kSpanWaves * 64, 2) void span_attn_kernel(SpanParam
                 for (int i = 0; i < 4; ++i) acc[ct][i] *= alpha;
         }
         vec8_t<T> hi, lo;
-        span_split(x, hi, lo);
+        split_weights(x, hi, lo);
         const char *vp = vbuf + v_frag;
         span_steps<AHEAD, CT, 2, vec8_t<T>>([&](int ct) { return *reinterpret_cast<const vec8_t<T> *>(vp + ct * 512); },
                                             [&](int ct, vec8_t<T> vf) {
