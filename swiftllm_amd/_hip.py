@@ -270,7 +270,7 @@ def is_available() -> bool:
 
 def call(name: str, *args) -> None:
     """Invoke `name`; map a non-zero return code to HipLibraryError (a RuntimeError)."""
-    fn = getattr(load(), name, None)
+    fn = getattr(_lib or load(), name, None)
     if fn is None:
         raise HipLibraryError(f"{library_path()} was built without {name}: run `python -m swiftllm_amd.csrc.build`")
     rc = fn(*args)

@@ -197,8 +197,8 @@ class StepPlan:
             off += (n + 3) // 4 * 4
         return out, off
 
-    def pack_into(self, buf: np.ndarray) -> int:
-        layout, total = self.packed_layout()
+    def pack_into(self, buf: np.ndarray, packed_layout=None) -> int:
+        layout, total = self.packed_layout() if packed_layout is None else packed_layout
         for name, off, n in layout:
             buf[off:off + n] = getattr(self, name)
         return total
@@ -238,6 +238,28 @@ def plan_step(entries: Sequence[StepEntry], vocab_size: int = None, max_position
     except (OverflowError, ValueError, TypeError):
         _check_entries(entries, vocab_size, max_positions)
         raise
+
+
+def plan_tokens(tokens: Sequence[int], seq_ids: Sequence[int], starts: Sequence[int], vocab_size: int = None, max_positions: int = None):
+    """plan_step of one wanted token for each sequence (StepEntry(seq_id, [token], start, (0,)) in order), or None where anything is out of
+    range: plan_step says what. A decode step waits for this with an idle device; 32 sequences 58 -> 15 us with the entries that it does
+    without, 3 sequences 23 -> 10."""
+    i32, n = np.int32, len(seq_ids)
+    try:
+        toks = np.asarray(tokens, dtype=np.int64)
+        ids, first, known = [int(s) for s in seq_ids], [int(a) for a in starts], toks.tolist()
+        targets = [a + 1 for a in first]
+        if not (n and toks.shape == (n,) and len(first) == n and min(first) >= 0 and len(set(ids)) == n
+                and max(targets) <= (1 << 31 if max_positions is None else min(max_positions, 1 << 31))
+                and (vocab_size is None or (min(known) >= 0 and max(known) < vocab_size))):
+            return None
+        pos, seq, toks = np.asarray(first, dtype=i32), np.asarray(ids, dtype=i32), toks.astype(i32)
+    except (OverflowError, ValueError, TypeError):
+        return None
+    rows, ones = np.arange(n, dtype=i32), np.ones(n, dtype=i32)
+    return StepPlan(num_tokens=n, num_seqs=n, seq_ids_list=ids, target_lens_list=targets, input_ids=toks, tok_pos=pos, tok_seq=seq,
+                    want_rows=rows, tile_row0=rows, tile_cnt=ones, seq_row0=rows, seq_cnt=ones, tok_start=pos,
+                    tok_state=np.zeros(n, dtype=i32), chunk_row0=rows, chunk_cnt=ones, seq_chunk0=rows, seq_tile0=rows)
 
 
 def _plan_whole(entries: Sequence[StepEntry], vocab_size, max_positions) -> StepPlan:

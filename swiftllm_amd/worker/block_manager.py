@@ -48,13 +48,13 @@ class BlockAllocatorHost:
     def plan_allocation(self, seq_ids: Sequence[int], target_lens: Sequence[int]):
         """Decide the blocks each sequence gains so that it owns ceil(len / block_size) blocks.
         Returns (block_needed int32[B], new_block_ids int32[sum]) and commits the decision."""
-        bs = self.block_size
-        needed = np.empty(len(seq_ids), dtype=np.int32)
-        for i, (sid, tlen) in enumerate(zip(seq_ids, target_lens)):
+        bs, owned = self.block_size, self.seq_blocks
+        needed = []
+        for sid, tlen in zip(seq_ids, target_lens):
             if not 0 <= sid < self.max_seqs:
                 raise RuntimeError(f"sequence id {sid} outside the block table (0..{self.max_seqs - 1})")
             target = -(-int(tlen) // bs)
-            have = self.num_allocated(sid)
+            have = len(owned.get(sid) or ())
             if have > target:
                 raise AssertionError(
                     f"(On {self.device_name}) Logic error: sequence {sid} already owns {have} blocks, "
@@ -62,8 +62,9 @@ class BlockAllocatorHost:
             if target > self.max_blocks_per_seq:
                 raise RuntimeError(f"sequence {sid} needs {target} blocks > max_blocks_per_seq "
                                    f"{self.max_blocks_per_seq}")
-            needed[i] = target - have
-        total = int(needed.sum())
+            needed.append(target - have)
+        total = sum(needed)
+        needed = np.asarray(needed, dtype=np.int32)
         if total > self.num_free_blocks:
             raise RuntimeError(
                 f"No enough free blocks available on {self.device_name} ({self.num_blocks} in total, "

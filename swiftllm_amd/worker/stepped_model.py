@@ -25,7 +25,7 @@ from swiftllm_amd import _hip
 from swiftllm_amd.engine_config import EngineConfig
 from swiftllm_amd.utils import GB
 
-from .batch_plan import StepEntry, StepPlan, plan_step
+from .batch_plan import StepEntry, StepPlan, plan_step, plan_tokens
 from .block_manager import BlockManager
 from .kernels.block_swapping import swap_blocks
 from .kernels.sampling import argmax_rows
@@ -175,7 +175,7 @@ class SteppedModel:
             # gone is refused by the caching allocator)
             self._decode_graphs.clear()
             self._graph_pool = None
-        plan.pack_into(self._meta_host_np)
+        plan.pack_into(self._meta_host_np, (layout, order_at))
         if order is not None:
             self._meta_host_np[order_at:total] = order
         self._meta_dev[:total].copy_(self._meta_host[:total], non_blocking=True)
@@ -189,23 +189,27 @@ class SteppedModel:
         """Per-sequence state: slots for the sequences of this step, their codes into the plan."""
         if self.state is None:
             return
-        starts = [int(plan.tok_pos[r]) for r in plan.seq_row0]
-        codes = self.state.begin_step(plan.seq_ids_list, starts)
-        plan.tok_state = np.repeat(codes, plan.seq_cnt).astype(np.int32)
+        codes = self.state.begin_step(plan.seq_ids_list, plan.tok_pos[plan.seq_row0].tolist())
+        plan.tok_state = codes if plan.num_tokens == plan.num_seqs else np.repeat(codes, plan.seq_cnt).astype(np.int32)
 
     @torch.inference_mode()
     def step(self, entries: Sequence[StepEntry], ignore_kvcache: bool = False) -> torch.Tensor:
         """Run one batch of portions. Returns the logits of the wanted places, [wanted, vocab] (device tensor in the compute
         dtype; fp32 from a design that caps them), in the order of the entries and of each entry's `want`."""
         cfg = self.model_config
-        plan = plan_step(entries, cfg.vocab_size, cfg.max_position_embeddings)
+        return self._run_plan(plan_step(entries, cfg.vocab_size, cfg.max_position_embeddings), ignore_kvcache)
+
+    @torch.inference_mode()
+    def _run_plan(self, plan: StepPlan, ignore_kvcache: bool) -> torch.Tensor:
+        cfg = self.model_config
         if plan.num_tokens == 0:
             return torch.empty((0, cfg.vocab_size), dtype=self.dtype, device=self.device)
         if not ignore_kvcache:
             self.gpu_block_manager.allocate_blocks_for_seqs(plan.seq_ids_list, plan.target_lens_list)
         self._begin_state_step(plan)
         dev = self._upload_plan(plan)
-        dev["longest"], dev["longest_portion"] = int(max(plan.target_lens_list)), int(plan.seq_cnt.max())
+        dev["longest"] = int(max(plan.target_lens_list))
+        dev["longest_portion"] = 1 if plan.num_tokens == plan.num_seqs else int(plan.seq_cnt.max())
         if (getattr(self.engine_config, "use_hip_graph", False) and not ignore_kvcache and self.layer_tap is None
                 and plan.num_tokens == plan.num_seqs == plan.want_rows.size):
             logits = self._step_decode_graph(plan, dev)
@@ -261,15 +265,19 @@ class SteppedModel:
         num_prefill = len(input_ids_list) - len(decoding_seq_lens_list)
         if num_prefill < 0 or len(seq_ids_list) != len(input_ids_list):
             raise ValueError("inconsistent batch: need len(seq_ids) == len(input_ids) >= len(decoding_seq_lens)")
+        plan = None
+        if num_prefill == 0 and all(len(ids) == 1 for ids in input_ids_list):
+            plan = plan_tokens([ids[0] for ids in input_ids_list], seq_ids_list, [n - 1 for n in decoding_seq_lens_list],
+                               self.model_config.vocab_size, self.model_config.max_position_embeddings)
         entries = []
-        for i, (ids, sid) in enumerate(zip(input_ids_list, seq_ids_list)):
+        for i, (ids, sid) in enumerate(zip(input_ids_list, seq_ids_list) if plan is None else ()):
             if i < num_prefill:
                 entries.append(StepEntry(sid, ids, 0, (len(ids) - 1,)))
             else:
                 if len(ids) != 1:
                     raise ValueError("every decoding sequence must contribute exactly one token")
                 entries.append(StepEntry(sid, ids, decoding_seq_lens_list[i - num_prefill] - 1, (0,)))
-        logits = self.step(entries, ignore_kvcache)
+        logits = self.step(entries, ignore_kvcache) if plan is None else self._run_plan(plan, ignore_kvcache)
         tokens = argmax_rows(logits)
         if self.after_launch_hook is not None:
             self.after_launch_hook()

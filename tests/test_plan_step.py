@@ -4,7 +4,7 @@ import random
 import numpy as np
 import pytest
 
-from swiftllm_amd.worker.batch_plan import StepEntry, StepPlan, plan_step
+from swiftllm_amd.worker.batch_plan import StepEntry, StepPlan, plan_step, plan_tokens
 
 
 def _by_entry(entries):
@@ -86,3 +86,28 @@ def test_span_order_takes_runs_of_four_from_the_highest_positions():
         at += chunks
     runs.sort(key=lambda r: (-r[0], -r[1]))
     assert order.tolist() == [c for r in runs for c in r[2]]
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 33])
+def test_plan_of_one_token_each(n):
+    """plan_tokens is plan_step of the same entries, array for array, and gives none where plan_step refuses."""
+    rng = random.Random(n)
+    toks, ids, starts = [rng.randrange(50) for _ in range(n)], rng.sample(range(100), n), [rng.randrange(300) for _ in range(n)]
+    for given in (toks, [np.int64(t) for t in toks]):
+        plan = plan_tokens(given, ids, starts, 50, 300)
+        want = plan_step([StepEntry(i, [t], a, (0,)) for i, t, a in zip(ids, toks, starts)], 50, 300)
+        for name in StepPlan.SEGMENTS:
+            got = getattr(plan, name)
+            assert got.dtype == np.int32 and got.tolist() == getattr(want, name).tolist(), name
+        assert (plan.num_tokens, plan.num_seqs, plan.seq_ids_list, plan.target_lens_list) == (n, n, want.seq_ids_list, want.target_lens_list)
+        assert plan.span_order() is None
+    at = rng.randrange(n)
+    for which, bad in ((0, 50), (0, -1), (0, 1 << 63), (1, 1 << 40), (2, -1), (2, 300), (2, 1 << 40)):
+        lists = [list(toks), list(ids), list(starts)]
+        lists[which][at] = bad
+        assert plan_tokens(*lists, 50, 300) is None
+        with pytest.raises((ValueError, RuntimeError, OverflowError)):
+            plan_step([StepEntry(i, [t], a, (0,)) for t, i, a in zip(*lists)], 50, 300)
+    if n > 1:
+        assert plan_tokens(toks, ids[:-1] + ids[:1], starts, 50, 300) is None
+    assert plan_tokens([], [], [], 50, 300) is None
