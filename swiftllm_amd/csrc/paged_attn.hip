@@ -214,7 +214,7 @@ template <typename T, int D, int G, int NW, bool QKV = false>
 // stores into the pools before its main loop, and without the no-alias guarantee the compiler must assume those
 // stores clobber the block table — it then fetches bt[b] with a VECTOR load and waits vmcnt(0) for it, draining
 // the whole K/V ring on every refill (seen in the ISA; the plain variant has no stores and got s_load all along).
-__global__ __launch_bounds__(NW * 64) void paged_attn_phase1_kernel(PagedAttnParams p,
+__global__ __launch_bounds__(NW * 64, 2) void paged_attn_phase1_kernel(PagedAttnParams p,
                                                                     const int *__restrict__ block_table,
                                                                     const int *__restrict__ seq_lens_r,
                                                                     const int *__restrict__ seq_ids_r) {
@@ -662,7 +662,12 @@ static int launch_phase1(const PagedAttnParams &p, int Bd, hipStream_t stream) {
     const dim3 grid(p.KVH, Bd, p.num_seq_blocks);
     // >= 32 KV blocks per sequence block: 8-wave workgroups (>= 4 blocks per wave); else 4 waves.
     // (the VALU variant of G = 8 would need > 256 registers per lane; the matrix-core one, G >= 2, does not.)
-    if (p.seq_block_size >= 32 * kBlk)
+    // With the new token's rotary and store in the prologue (QKV) a CU has registers for eight waves. In more than one round of workgroups,
+    // two of four waves hide each other's prologue and merge: 120 requests of about 600 tokens, 8 kv heads of 128, 64.1 -> 59.2 us (5.0 TB/s),
+    // 32 of about 1100 in two blocks 34.5 -> 30.3. (Without it three waves a SIMD fit either way: 37 us by eight waves, 41 by four.) Longest
+    // sequences first: the same for one block a sequence, 1 us for two.
+    const bool rounds = QKV && static_cast<int64_t>(p.KVH) * Bd * p.num_seq_blocks > 256;
+    if (p.seq_block_size >= 32 * kBlk && !rounds)
         hipLaunchKernelGGL((paged_attn_phase1_kernel<T, D, G, 8, QKV>), grid, dim3(512), 0, stream, p, p.block_table,
                            p.seq_lens, p.seq_ids);
     else
