@@ -88,7 +88,7 @@ def test_span_order_takes_runs_of_four_from_the_highest_positions():
     assert order.tolist() == [c for r in runs for c in r[2]]
 
 
-@pytest.mark.parametrize("n", [1, 2, 3, 33])
+@pytest.mark.parametrize("n", [1, 2, 3, 33, 65])
 def test_plan_of_one_token_each(n):
     """plan_tokens is plan_step of the same entries, array for array, and gives none where plan_step refuses."""
     rng = random.Random(n)
