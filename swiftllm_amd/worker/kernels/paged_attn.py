@@ -47,8 +47,10 @@ def paged_attention_from_qkv_splitk(partials, k_cache: torch.Tensor, v_cache: to
                                     cur_layer: int, o: torch.Tensor, row_scale=None, merge: bool = True):
     """Pure-decode batches: rotary + KV-store + paged attention in one launch, fed by the split-K partial slabs
     of the fused qkv projection (kernels/linear.py: SplitKPartials). Same bits as
-    rotary_embedding_and_store_kvcache_decode_from_splitk followed by paged_attention; q/k/v never exist as
-    tensors (the rotated k and the v go to the pools, q stays in the kernel)."""
+    rotary_embedding_and_store_kvcache_decode_from_splitk followed by paged_attention, except that in sequence blocks
+    of 512 tokens and more beyond 256 workgroups four waves share a block's keys where that has eight (the outputs'
+    partial sums meet in another order); q/k/v never exist as tensors (the rotated k and the v go to the pools, q stays in the
+    kernel)."""
     nd = infer_state.num_decoding_seqs
     if nd == 0:
         return

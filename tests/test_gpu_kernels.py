@@ -681,6 +681,43 @@ def test_paged_attention_from_qkv_slabs_equals_three_kernels(dtype, sbs, H, KVH,
     assert not torch.equal(kc2.cpu(), kc)                      # the new token really went into the pool
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nd,sbs", [(32, 512), (33, 512), (33, 1024)])      # 256 workgroups a block of the sequence, and more
+def test_paged_attention_from_qkv_slabs_in_several_rounds(dtype, nd, sbs):
+    """More than 256 workgroups: four waves instead of eight share a sequence's blocks. Pools are the same to the bit; outputs differ from
+    the three kernels' (eight waves) by what rounding gives: either side rounds weights and results to the type, half an ulp each
+    (2^-9 or 2^-12 of a term), so rows differ by at most twice the sum of both, 2^-7 or 2^-10 (2-norm)."""
+    from swiftllm_amd.worker.kernels.linear import SplitKPartials
+    from swiftllm_amd.worker.kernels.paged_attn import paged_attention_from_qkv_splitk
+    from swiftllm_amd.worker.kernels.rotary_emb import rotary_embedding_and_store_kvcache_decode_from_splitk
+    H, KVH, D, L, layer = 32, 8, 128, 1, 0
+    g = gen(nd + sbs)
+    lens = [1, 16, 17, 64, 65, 511, 512] + [(37 * i) % 512 + 1 for i in range(nd - 7)]
+    _, kc, vc, bt, seq_ids = _paged_case(g, H, KVH, D, L, lens, dtype, layer)
+    n = (H + 2 * KVH) * D
+    part = SplitKPartials(torch.randn(nd, n, generator=g).cuda(), 1, nd, n, dtype)
+    ang = torch.rand(512, D // 2, generator=g) * 6.28
+    st = _paged_state(lens, seq_ids, sbs, D, "cuda")
+    st.position_cos, st.position_sin = torch.cos(ang).to(dtype).cuda(), torch.sin(ang).to(dtype).cuda()
+    st.position_indices = torch.tensor([v - 1 for v in lens], dtype=torch.int32, device="cuda")
+    mc, ec = NS(num_q_heads=H, num_kv_heads=KVH, head_dim=D, num_layers=L), NS(block_size=16)
+    outs = []
+    for fused in (False, True):
+        kc1, vc1, btc = kc.cuda(), vc.cuda(), bt.cuda()
+        o = torch.zeros(nd, H, D, dtype=dtype, device="cuda")
+        if fused:
+            paged_attention_from_qkv_splitk(part, kc1, vc1, btc, mc, ec, st, layer, o)
+        else:
+            q1, _, _ = rotary_embedding_and_store_kvcache_decode_from_splitk(part, kc1, vc1, btc, mc, ec, st, layer)
+            K().paged_attention(q1, kc1, vc1, btc, mc, ec, st, layer, o)
+        outs.append((o.float().view(nd, -1), kc1, vc1))
+    (o1, k1, v1), (o2, k2, v2) = outs
+    assert torch.equal(k2, k1) and torch.equal(v2, v1)
+    if nd * KVH <= 256:
+        assert torch.equal(o2, o1)
+    assert ((o2 - o1).norm(dim=1) <= (2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10) * o1.norm(dim=1)).all()
+
+
 # ---- pre-packed weights ---------------------------------------------------------------------------------------
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M", [1, 7, 32])

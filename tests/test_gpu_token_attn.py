@@ -44,6 +44,23 @@ def test_softmax_attention(H, G, d, dv, window, kind, dtype):
             at += m
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,d,dv", [(8, 2, 128, 128), (6, 3, 36, 33), (40, 20, 24, 100)])
+def test_few_tokens_have_the_bits_of_many(H, G, d, dv, dtype):
+    """Up to 256 workgroups one serves the heads of a key head, beyond them as many heads as it holds: the same sums."""
+    from swiftllm_amd.worker.kernels import window_attn as wa
+    g = torch.Generator().manual_seed(H)
+    pool, sl, table, _, _ = _pool([a + n for _, a, n in PARTS], G, G, d, dv, dtype, g)
+    seq, pos, _ = _spans(PARTS)
+    n = seq.shape[0]
+    q = torch.randn(n, H * d, generator=g).to(dtype).cuda()
+    spec = wa.AttentionSpec(H, G, d, dv, d ** -0.5)
+    few = wa.masked_attention(q, pool, sl, table, seq, pos, spec, None, 64)
+    times = 256 // n + 1        # (the first count past 256 tokens)
+    many = wa.masked_attention(q.repeat(times, 1), pool, sl, table, seq.repeat(times), pos.repeat(times), spec, None, 64)
+    assert torch.equal(many.view(times, n, -1), few.expand(times, n, few.shape[1]))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("H,G,d,dv,window,mixed", [(8, 2, 128, 128, 0, True), (6, 3, 18, 5, 37, True), (40, 20, 24, 100, 0, False)])
 def test_sigmoid_attention(H, G, d, dv, window, mixed, dtype):
