@@ -31,6 +31,21 @@ def test_sort_by_expert(n, top, experts, kind):
     assert torch.equal(offsets.long().cpu(), torch.cat((torch.zeros(1, dtype=torch.long), torch.bincount(flat, minlength=experts).cumsum(0))))
 
 
+@pytest.mark.parametrize("shift", [0, 1])       # ids on and off the 16-byte boundaries
+@pytest.mark.parametrize("n,experts", [(3, 2), (4095, 9), (4096, 9), (4097, 9), (16384, 3), (16387, 3), (40001, 130)])
+def test_sort_at_the_ends_of_pieces(n, experts, shift):
+    """4096 ids in one piece of four a thread, pieces of 16384 beyond; ids that name no expert count as the nearest."""
+    from swiftllm_amd import _hip
+    ids = torch.randint(-1, experts + 1, (n + shift,), generator=torch.Generator().manual_seed(n)).to(torch.int32)
+    idx, flat = ids.cuda()[shift:], ids[shift:].long().clamp(0, experts - 1)
+    order, where = torch.full((n,), -1, dtype=torch.int32, device="cuda"), torch.full((n,), -1, dtype=torch.int64, device="cuda")
+    offsets = torch.empty(experts + 1, dtype=torch.int32, device="cuda")
+    _hip.call("swl_moe_sort", _hip.ptr(order), _hip.ptr(where), _hip.ptr(offsets), _hip.ptr(idx), n, experts, _hip.stream())
+    want = torch.argsort(flat, stable=True)
+    assert torch.equal(order.long().cpu(), want) and torch.equal(where.cpu()[want], torch.arange(n))
+    assert torch.equal(offsets.long().cpu(), torch.cat((torch.zeros(1, dtype=torch.long), torch.bincount(flat, minlength=experts).cumsum(0))))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("n,top,experts,width,ff,kind,form", [
     (300, 2, 5, 128, 64, "any", "silu"), (129, 1, 3, 64, 72 * 8, "any", "clamped"), (256, 3, 6, 192, 128, "runs", "silu_in"),
