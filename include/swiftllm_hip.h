@@ -441,6 +441,9 @@ int swl_gemm_rows_add(void *residual, const void *x, const void *w_packed, int32
  * rounding points). K % 1024 == 0; any N: the packed weight holds whole tiles of 32 rows, rows of zeros from N on. */
 int swl_gemm_rows_store(void *out, const void *x, const void *w_packed, int32_t M, int32_t N, int32_t K, int64_t x_row_stride,
                         int64_t out_row_stride, int32_t relu2, int32_t dtype, swl_stream_t stream);
+/* ... and with the fp32 sums themselves, one slab for the consumers of K shares (swl_gated_add_rmsnorm_parts, swl_hyper_step). */
+int swl_gemm_rows_partial(float *slab, const void *x, const void *w_packed, int32_t M, int32_t N, int32_t K, int64_t x_row_stride,
+                          int64_t slab_row_stride, int32_t dtype, swl_stream_t stream);
 int swl_gemm_skinny_packed_partial_nf(float *slabs, size_t slabs_bytes, float *ssq_out, const void *x, const void *norm_w,
                                       const void *w_packed, int32_t M, int32_t N, int32_t K, int64_t x_row_stride,
                                       int32_t k_splits, int32_t dtype, swl_stream_t stream);

@@ -42,6 +42,8 @@
 // round(residual * w_norm) and one sum-of-squares partial per tile, with a SiLU-gate GEMM that added the 256 partials from
 // LDS-DMA'd copies: correct, +2 us on the up/gate kernel, removed — last revision that has it: ca4e9a9, numbers in
 // profiles/r05a_gemm_rows_micro_o_proj_pair.jsonl.)
+#include <type_traits>
+
 #include "swl_common.h"
 
 namespace swl {
@@ -64,7 +66,8 @@ constexpr int kRowsRedPitch = 20; // floats per token row of a wave's tile image
 //   kRowsAdd    residual += round(product)
 //   kRowsStore  out = round(product)
 //   kRowsRelu2  out = round(relu(round(product))^2): swl_relu_sq behind the stored product
-constexpr int kRowsAdd = 0, kRowsStore = 1, kRowsRelu2 = 2;
+//   kRowsSlab   out = product, fp32: one slab for a consumer that adds slabs into an fp32 stream (nothing is rounded on the way)
+constexpr int kRowsAdd = 0, kRowsStore = 1, kRowsRelu2 = 2, kRowsSlab = 3;
 
 struct RowsArgs {
     const void *x;
@@ -103,7 +106,8 @@ __global__ __launch_bounds__(kRowsWaves * 64, rows_waves_per_simd(NCH, EPI)) voi
     // ---- epilogue operands first: the oldest requests of the wave, no wait of the stream ever includes them ----
     const int et = threadIdx.x >> 4, en = threadIdx.x & 15; // (token, column n0 + en)
     const bool e_ok = et < M && (EPI == kRowsAdd || n0 + en < N);
-    T *res_p = static_cast<T *>(a.residual) + static_cast<int64_t>(e_ok ? et : 0) * (EPI == kRowsAdd ? N : a.out_stride) + n0 + en;
+    using O = std::conditional_t<EPI == kRowsSlab, float, T>;
+    O *res_p = static_cast<O *>(a.residual) + static_cast<int64_t>(e_ok ? et : 0) * (EPI == kRowsAdd ? N : a.out_stride) + n0 + en;
     T rv{};
     if constexpr (EPI == kRowsAdd) rv = *res_p;
 
@@ -215,22 +219,22 @@ __global__ __launch_bounds__(kRowsWaves * 64, rows_waves_per_simd(NCH, EPI)) voi
 #pragma unroll
         for (int w = 0; w < kRowsWaves; ++w) s += red(w)[et * kRowsRedPitch + en]; // wave order = K order
     }
-    if constexpr (EPI == kRowsStore) {
+    if constexpr (EPI == kRowsSlab) {
+        if (e_ok) *res_p = s;
+    } else if constexpr (EPI == kRowsStore) {
         if (e_ok) *res_p = to_t<T>(s);
-        return;
-    }
-    if constexpr (EPI == kRowsRelu2) {
+    } else if constexpr (EPI == kRowsRelu2) {
         const float v = fmaxf(to_f(to_t<T>(s)), 0.f);
         if (e_ok) *res_p = to_t<T>(v * v);
-        return;
-    }
-    // splitk_add_scale_kernel's arithmetic (rmsnorm.hip) on this thread's element
-    const T xn = add_t<T>(to_t<T>(s), rv); // the projection is rounded, then the sum (rmsnorm.py:54-57)
-    if (e_ok) *res_p = xn;
-    if (a.ssq_out != nullptr) {             // (wave-uniform) the 16 column lanes of a token: one DPP row reduction
-        const float v = e_ok ? to_f(xn) : 0.f;
-        const float t = group_allreduce_sum<16>(v * v);
-        if (e_ok && en == 0) a.ssq_out[static_cast<int64_t>(et) * (N / kRowsTile) + tile16] = t;
+    } else {
+        // splitk_add_scale_kernel's arithmetic (rmsnorm.hip) on this thread's element
+        const T xn = add_t<T>(to_t<T>(s), rv); // the projection is rounded, then the sum (rmsnorm.py:54-57)
+        if (e_ok) *res_p = xn;
+        if (a.ssq_out != nullptr) {             // (wave-uniform) the 16 column lanes of a token: one DPP row reduction
+            const float v = e_ok ? to_f(xn) : 0.f;
+            const float t = group_allreduce_sum<16>(v * v);
+            if (e_ok && en == 0) a.ssq_out[static_cast<int64_t>(et) * (N / kRowsTile) + tile16] = t;
+        }
     }
 }
 
@@ -248,9 +252,9 @@ static int launch_rows(const RowsArgs &a, hipStream_t stream) {
         if (nch == 2) { hipLaunchKernelGGL((gemm_rows_kernel<T, 2, MB, XLDS, EPI>), grid, block, 0, stream, a); return check_launch(); }
     } else {
         if (nch == 14) { hipLaunchKernelGGL((gemm_rows_kernel<T, 14, MB, XLDS, EPI>), grid, block, 0, stream, a); return check_launch(); }
+        if (nch == 8) { hipLaunchKernelGGL((gemm_rows_kernel<T, 8, MB, XLDS, EPI>), grid, block, 0, stream, a); return check_launch(); }
     }
     if (nch == 4) hipLaunchKernelGGL((gemm_rows_kernel<T, 4, MB, XLDS, EPI>), grid, block, 0, stream, a);
-    else if (nch == 8) hipLaunchKernelGGL((gemm_rows_kernel<T, 8, MB, XLDS, EPI>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((gemm_rows_kernel<T, 0, MB, XLDS, EPI>), grid, block, 0, stream, a);
     return check_launch();
 }
@@ -305,20 +309,34 @@ static int rows_add_impl(void *residual, float *ssq_out, const void *x, const vo
     });
 }
 
-/* out[M, N] = round(x . W^T), or relu(that)^2 rounded again (relu2 = 1): any N, the packed copy holding whole tiles of 32 rows. */
-extern "C" int swl_gemm_rows_store(void *out, const void *x, const void *w_packed, int32_t M, int32_t N, int32_t K,
-                                   int64_t x_row_stride, int64_t out_row_stride, int32_t relu2, int32_t dtype, swl_stream_t stream) {
-    if (M < 0 || N <= 0 || K <= 0 || relu2 < 0 || relu2 > 1) return SWL_ERR_BAD_ARG;
+template <bool SLAB>
+static int rows_store_impl(void *out, const void *x, const void *w_packed, int32_t M, int32_t N, int32_t K, int64_t x_row_stride,
+                           int64_t out_row_stride, bool relu2, int32_t dtype, swl_stream_t stream) {
+    if (M < 0 || N <= 0 || K <= 0) return SWL_ERR_BAD_ARG;
     if (M == 0) return SWL_OK;
     if (!out || !x || !w_packed) return SWL_ERR_BAD_ARG;
     if (M > 32 || K % swl::kRowsKUnit != 0) return SWL_ERR_UNSUPPORTED;
     if (x_row_stride < K || (x_row_stride & 7) || out_row_stride < N) return SWL_ERR_BAD_ARG;
-    if (!swl::aligned16(x) || !swl::aligned16(w_packed) || (reinterpret_cast<uintptr_t>(out) & 1u)) return SWL_ERR_BAD_ARG;
+    if (!swl::aligned16(x) || !swl::aligned16(w_packed) || (reinterpret_cast<uintptr_t>(out) & (SLAB ? 3u : 1u))) return SWL_ERR_BAD_ARG;
     swl::RowsArgs a = {};
     a.x = x; a.wp = w_packed; a.residual = out; a.out_stride = out_row_stride;
     a.M = M; a.N = N; a.K = K; a.x_stride = x_row_stride;
     SWL_DISPATCH_DTYPE(dtype, T, {
         const hipStream_t s = static_cast<hipStream_t>(stream);
-        return relu2 ? swl::launch_rows_m<T, swl::kRowsRelu2>(a, s) : swl::launch_rows_m<T, swl::kRowsStore>(a, s);
+        if constexpr (SLAB) return swl::launch_rows_m<T, swl::kRowsSlab>(a, s);
+        else return relu2 ? swl::launch_rows_m<T, swl::kRowsRelu2>(a, s) : swl::launch_rows_m<T, swl::kRowsStore>(a, s);
     });
+}
+
+/* out[M, N] = round(x . W^T), or relu(that)^2 rounded again (relu2 = 1): any N, the packed copy holding whole tiles of 32 rows. */
+extern "C" int swl_gemm_rows_store(void *out, const void *x, const void *w_packed, int32_t M, int32_t N, int32_t K,
+                                   int64_t x_row_stride, int64_t out_row_stride, int32_t relu2, int32_t dtype, swl_stream_t stream) {
+    if (relu2 < 0 || relu2 > 1) return SWL_ERR_BAD_ARG;
+    return rows_store_impl<false>(out, x, w_packed, M, N, K, x_row_stride, out_row_stride, relu2 != 0, dtype, stream);
+}
+
+/* slab[M, N] = x . W^T, fp32: the sums that swl_gemm_rows_store rounds, for consumers of K shares (one slab). */
+extern "C" int swl_gemm_rows_partial(float *slab, const void *x, const void *w_packed, int32_t M, int32_t N, int32_t K,
+                                     int64_t x_row_stride, int64_t slab_row_stride, int32_t dtype, swl_stream_t stream) {
+    return rows_store_impl<true>(slab, x, w_packed, M, N, K, x_row_stride, slab_row_stride, false, dtype, stream);
 }

@@ -91,19 +91,40 @@ def packable_rows(w) -> bool:
                            and w.dtype in (torch.float16, torch.bfloat16) and _rows_serves(*w.shape))
 
 
-def linear_rows(a: torch.Tensor, w: torch.Tensor, relu2: bool = False):
-    """a[T, in] @ w[out, in]^T for up to 32 tokens in one launch without shares of K (csrc/gemm_rows.hip), `relu2`: squared ReLU of
-    the rounded product in the same launch; None where the kernel does not serve the call (`_rows_serves`)."""
-    wp = _packed_of(w)
-    if wp is None or not (a.is_cuda and a.dim() == 2 and 0 < a.shape[0] <= _SKINNY_MAX_M and a.dtype == w.dtype):
+def _rows_call(a: torch.Tensor, w: torch.Tensor):
+    """(tokens, rows of w, columns, row stride of a) of a product that the row-owned kernel takes, None where it does not serve the call."""
+    if _packed_of(w) is None or not (a.is_cuda and a.dim() == 2 and 0 < a.shape[0] <= _SKINNY_MAX_M and a.dtype == w.dtype):
         return None
     m, (n, k) = a.shape[0], w.shape
     if not _rows_serves(n, k) or a.shape[1] != k or a.stride(1) != 1 or (m > 1 and a.stride(0) % 8) or a.data_ptr() % 16:
         return None
+    return m, n, k, k if m == 1 else a.stride(0)
+
+
+def linear_rows(a: torch.Tensor, w: torch.Tensor, relu2: bool = False):
+    """a[T, in] @ w[out, in]^T for up to 32 tokens in one launch without shares of K (csrc/gemm_rows.hip), `relu2`: squared ReLU of
+    the rounded product in the same launch; None where the kernel does not serve the call (`_rows_serves`)."""
+    call = _rows_call(a, w)
+    if call is None:
+        return None
+    m, n, k, stride = call
     out = torch.empty((m, n), dtype=a.dtype, device=a.device)
-    _hip.call("swl_gemm_rows_store", _hip.ptr(out), _hip.ptr(a), _hip.ptr(wp), m, n, k, k if m == 1 else a.stride(0), n,
-              1 if relu2 else 0, _hip.dtype_code(a.dtype), _hip.stream())
+    _hip.call("swl_gemm_rows_store", _hip.ptr(out), _hip.ptr(a), _hip.ptr(_packed_of(w)), m, n, k, stride, n, 1 if relu2 else 0,
+              _hip.dtype_code(a.dtype), _hip.stream())
     return out
+
+
+def linear_rows_partial(a: torch.Tensor, w: torch.Tensor):
+    """linear_rows for a consumer that adds the product into an fp32 stream: its fp32 sums as one slab, not rounded to a's dtype (as the
+    K shares of linear_splitk are not). None where linear_rows would be, and for rows that do not divide into the consumers' loads of four."""
+    call = _rows_call(a, w)
+    if call is None or call[1] % 4:
+        return None
+    m, n, k, stride = call
+    slab = torch.empty((m, n), dtype=torch.float32, device=a.device)
+    _hip.call("swl_gemm_rows_partial", _hip.ptr(slab), _hip.ptr(a), _hip.ptr(_packed_of(w)), m, n, k, stride, n,
+              _hip.dtype_code(a.dtype), _hip.stream())
+    return SplitKPartials(slab, 1, m, n, a.dtype)
 
 
 def _packed_of(w: torch.Tensor):
@@ -113,7 +134,8 @@ def _packed_of(w: torch.Tensor):
 class SplitKPartials:
     """fp32 partial slabs [k_splits][M][N] of a projection whose K was split across workgroups.
     Lives in the shared split-K workspace: it must be consumed (or materialised) before the next
-    split projection is launched on the same stream — the layer code does exactly that."""
+    split projection is launched on the same stream — the layer code does exactly that. (A slab of
+    linear_rows_partial is a tensor of its own.)"""
     __slots__ = ("slabs", "k_splits", "shape", "dtype")
 
     def __init__(self, slabs: torch.Tensor, k_splits: int, m: int, n: int, dtype: torch.dtype):

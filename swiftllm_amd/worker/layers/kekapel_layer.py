@@ -4,8 +4,8 @@ import torch
 
 from swiftllm_amd import _hip
 
-from ..kernels.linear import (DECODE_MAX_TOKENS, F32_MAX_TOKENS, ROWS_MAX_TOKENS, linear, linear_f32, linear_rows, linear_silu_gate,
-                              linear_splitk)
+from ..kernels.linear import (DECODE_MAX_TOKENS, F32_MAX_TOKENS, ROWS_MAX_TOKENS, linear, linear_f32, linear_rows,
+                              linear_rows_partial, linear_silu_gate, linear_splitk)
 from ..kernels.moe import ACT_SILU_UP_FIRST, gated_unit, moe_experts, moe_route
 from ..kernels.polynorm import polynorm
 from ..kernels.window_attn import qknorm_and_store_kv, window_attention
@@ -34,11 +34,12 @@ def _project(a: torch.Tensor, w: torch.Tensor, skinny: bool) -> torch.Tensor:
 
 
 def _project_partials(a: torch.Tensor, w: torch.Tensor, skinny: bool):
-    """_project for a consumer that takes a product's K shares too: SplitKPartials where the decode GEMM splits K, rows otherwise."""
+    """_project for a consumer that takes a product's fp32 sums too (it adds them into an fp32 stream, so that they are rounded nowhere):
+    SplitKPartials from the decode GEMMs, rows otherwise."""
     m = a.shape[0]
     if not skinny or m > DECODE_MAX_TOKENS or a.dtype == torch.float32 or getattr(w, "_swl_blas_only", False):
         return _project(a, w, skinny)
-    y = linear_rows(a, w) if m <= ROWS_MAX_TOKENS else None
+    y = linear_rows_partial(a, w) if m <= ROWS_MAX_TOKENS else None
     if y is not None:
         return y
     try:

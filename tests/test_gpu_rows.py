@@ -80,6 +80,40 @@ def test_rows_store_is_one_rounding_of_the_product(dtype, M, N, K):
         assert linear_rows(odd, w) is None          # (rows that do not begin on 16 bytes stay with the general paths)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 9, 17, 32])
+@pytest.mark.parametrize("N,K", [(1024, 1024), (36, 2048), (3088, 2048), (68, 3072), (64, 4096), (512, 8192), (1025, 1024)])
+def test_products_for_the_fp32_stream_keep_their_fp32_sums(dtype, M, N, K):
+    """_project_partials, whose consumers add into an fp32 stream: where a decode kernel of up to 32 tokens serves the product, its sums are not
+    rounded to the compute dtype. Bound: fp32 sums of K products (2^-24 of the magnitudes' sum each, in any order). linear_rows rounds
+    the same sums."""
+    from swiftllm_amd import _hip
+    from swiftllm_amd.worker.kernels.linear import SplitKPartials, linear_rows, pack_weight, packable_rows
+    from swiftllm_amd.worker.layers.kekapel_layer import _project_partials
+    g = gen(M + N + K)
+    x = torch.randn(M, K + 8, generator=g).to(dtype).cuda()[:, :K]
+    w = (torch.randn(N, K, generator=g) * 0.03).to(dtype).cuda()
+    if packable_rows(w):
+        pack_weight(w)
+    y = _project_partials(x, w, True)
+    want = x.double() @ w.double().T
+    size = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    if N == 1025:       # (the consumers load four floats at a time)
+        assert isinstance(y, torch.Tensor)
+        assert ((y.double() - want).abs() <= want.abs() * (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) + size + 2.0 ** -24).all()
+        return
+    assert isinstance(y, SplitKPartials) and y.shape == (M, N)
+    sums = y.slabs.view(-1)[:y.k_splits * M * N].view(y.k_splits, M, N).double().sum(0)
+    assert ((sums - want).abs() <= size).all()
+    rows = linear_rows(x, w)
+    if rows is not None:
+        assert y.k_splits == 1 and torch.equal(y.materialize(), rows)
+        out = torch.full((M + 1, N + 3), 7.0, device="cuda")        # nothing outside the result is written
+        _hip.call("swl_gemm_rows_partial", _hip.ptr(out), _hip.ptr(x), _hip.ptr(w._swl_packed), M, N, K, K + 8, N + 3,
+                  _hip.dtype_code(dtype), _hip.stream())
+        assert torch.equal(out[:M, :N], y.slabs) and (out[M:] == 7).all() and (out[:, N:] == 7).all()
+
+
 @pytest.mark.parametrize("M", [1, 8, 32])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (4096, 14336)])
 def test_rows_add_carries_the_bits_of_splitk_plus_consumer(M, N, K):
