@@ -319,8 +319,8 @@ F32_MAX_TOKENS = 16     # (swl_gemm_f32_supported)
 
 def linear_f32(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """a[T, in] @ w[out, in]^T in true fp32: a few tokens on the hand-written kernel (csrc/gemm_f32.hip), the BLAS otherwise."""
-    if (a.is_cuda and a.dim() == 2 and a.dtype == w.dtype == torch.float32 and w.is_contiguous() and a.stride(1) == 1
-            and (a.data_ptr() | w.data_ptr()) % 16 == 0 and a.stride(0) % 4 == 0):
+    if (a.is_cuda and a.dim() == w.dim() == 2 and a.shape[1] == w.shape[1] and a.dtype == w.dtype == torch.float32 and w.is_contiguous()
+            and a.stride(1) == 1 and (a.data_ptr() | w.data_ptr()) % 16 == 0 and a.stride(0) % 4 == 0):
         m, (n, k) = a.shape[0], w.shape
         if _hip.load().swl_gemm_f32_supported(m, n, k) == 2:
             out = torch.empty((m, n), dtype=a.dtype, device=a.device)

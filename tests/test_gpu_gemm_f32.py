@@ -46,3 +46,13 @@ def test_linear_f32_routes(M, N, K, form, monkeypatch):
     got = linear_f32(x, w)
     assert (calls == ["swl_gemm_f32"]) == (form == "own")
     assert torch.allclose(got.double(), x.double() @ w.double().t(), rtol=0, atol=1e-4) and got.shape == (M, N)
+
+
+@pytest.mark.parametrize("columns", [60, 68, 128])
+def test_linear_f32_refuses_rows_of_another_length(columns):
+    """A product whose sides have different columns is the library's to refuse: contiguous rows and column slices of wider ones."""
+    from swiftllm_amd.worker.kernels.linear import linear_f32
+    x, w = torch.randn(3, 128, device="cuda"), torch.randn(64, 64, device="cuda")
+    for a in (x[:, :columns], x[:, :columns].contiguous()):
+        with pytest.raises(RuntimeError):
+            linear_f32(a, w)
