@@ -55,7 +55,7 @@ SOURCES = [
 # What a model family's worker calls (the shared pieces included): `build(only=MODEL_SOURCES[...])` compiles just these, so
 # that the first use from a fresh checkout does not pay for kernels the model never launches. A later full build compiles
 # the rest and links everything.
-_SHARED = ["swap_blocks.hip", "block_table.hip", "argmax.hip", "gemm_skinny.hip", "gemm_wide.hip", "gemm_f32.hip"]
+_SHARED = ["swap_blocks.hip", "block_table.hip", "argmax.hip", "gemm_skinny.hip", "gemm_wide.hip", "gemm_rows.hip", "gemm_f32.hip"]
 MODEL_SOURCES = {
     "llama": list(SOURCES[:14]),
     "Kekapel": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip",
