@@ -30,6 +30,10 @@ _TOKEN_BUCKET = 32
 BUCKETS = tuple(range(96, 257, _TOKEN_BUCKET))      # 65..96, ..128, ... ..256 tokens
 _WIN_MARGIN = 1.03
 _LOCK_WAIT_S = 120.0
+# Part of the key under which answers are saved. Raised whenever the hand-written kernel or the way of timing changes, so that answers of
+# others are not read any more: 1 both sides timed back to back on one weight, x alone through LDS; 2 cold weights, LDS rings of both
+# operands.
+_REVISION = 2
 
 _table = {}             # "N,K,dtype,bucket,silu" -> bool: this process's deployment table
 _device_key_cache = {}
@@ -95,7 +99,7 @@ def device_key(device) -> str:
             name = torch.cuda.get_device_name(device)
         except Exception:     # noqa: BLE001
             name = "unknown"
-        _device_key_cache[key] = f"{name}|hip {getattr(torch.version, 'hip', None)}|torch {torch.__version__}"
+        _device_key_cache[key] = f"{name}|hip {getattr(torch.version, 'hip', None)}|torch {torch.__version__}|routes {_REVISION}"
     return _device_key_cache[key]
 
 
@@ -210,11 +214,13 @@ def prepare(classes, dtype, device, model_path: str, measure) -> dict:
         for n, k, s, b in want:
             try:
                 fresh[_key(n, k, dtype, b, s)] = bool(measure(n, k, s, b))
+            except torch.cuda.OutOfMemoryError:     # says nothing about the shape: the library for this process, no answer for others
+                continue
             except Exception:     # noqa: BLE001 — a shape our kernel refuses: the library serves it
                 fresh[_key(n, k, dtype, b, s)] = False
         _table.update(fresh)
-        stats.update(measured=len(want))
-        if path is not None:
+        stats.update(measured=len(fresh))
+        if path is not None and fresh:
             data = _read(path)
             data.setdefault(dkey, {}).update(fresh)
             if _write(path, data):

@@ -469,6 +469,38 @@ def test_wide_kernel_routing_is_decided_once_per_deployment(tmp_path, monkeypatc
     assert R.decide(100, 4096, 11008, f16, False) is True          # K >= 2N by the table
 
 
+def test_saved_routes_of_another_kernel_or_method_are_not_read(tmp_path, monkeypatch):
+    """kernels/route_tune.py: answers are saved under device, software and the revision of what was measured; a file without the revision, or
+    of another one, is measured again and kept beside. A measurement that ran out of memory is no answer: not taken, not saved."""
+    import torch
+    from swiftllm_amd.worker.kernels import route_tune as R
+    monkeypatch.delenv("SWIFTLLM_ROUTE_TUNE", raising=False)
+    path = tmp_path / "routes.json"
+    monkeypatch.setenv("SWIFTLLM_ROUTE_CACHE", str(path))
+    monkeypatch.setattr(R, "_table", {})
+    monkeypatch.setattr(R, "_device_key_cache", {})
+    bf16, n, k = torch.bfloat16, 5120, 5120
+    current = R.device_key("cpu")
+    assert current.endswith(f"|routes {R._REVISION}")
+    answers = {R._key(n, k, bf16, b, False): True for b in R.BUCKETS}
+    older = current.rsplit("|routes", 1)[0]
+    path.write_text(json.dumps({older: answers, f"{older}|routes {R._REVISION - 1}": answers}))
+    st = R.prepare([(n, k, False)], bf16, "cpu", "", lambda *a: False)
+    assert st["measured"] == len(R.BUCKETS) and st["read"] == 0 and not R.decide(100, n, k, bf16, False)
+    disk = json.loads(path.read_text())
+    assert disk[older] == answers and not any(disk[current].values()) and len(disk[current]) == len(R.BUCKETS)
+
+    def short_of_memory(n, k, silu, bucket):
+        if bucket != 128:
+            raise torch.cuda.OutOfMemoryError("no memory")
+        return True
+    st = R.prepare([(7168, 7168, False)], bf16, "cpu", "", short_of_memory)
+    assert st["measured"] == 1 and R.decide(128, 7168, 7168, bf16, False) and not R.decide(160, 7168, 7168, bf16, False)
+    assert len(json.loads(path.read_text())[current]) == len(R.BUCKETS) + 1
+    st = R.prepare([(7168, 7168, False)], bf16, "cpu", "", lambda *a: True)
+    assert st["measured"] == len(R.BUCKETS) and R.decide(160, 7168, 7168, bf16, False)
+
+
 def test_tiny_batch_projection_policy():
     """kernels/linear.py: when may a projection consume the previous projection's slabs / the attention partials itself?
     (pure host logic: shapes, packed twin, K-chunk that fits LDS; the layer additionally limits the batch to 2)."""
