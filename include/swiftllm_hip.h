@@ -32,7 +32,7 @@ extern "C" {
 #endif
 
 /* raised whenever the parameters of an existing entry point change */
-#define SWL_ABI_VERSION 2
+#define SWL_ABI_VERSION 3
 
 #define SWL_F16 0
 #define SWL_BF16 1
@@ -119,14 +119,16 @@ int swl_silu_mul(void *x, int64_t num_tokens, int32_t ffn_inter_dim, int32_t dty
  * k_splits >= 1): the rotary embedding and the KV-cache store of the new token (reference rotary_emb.py:7-42 +
  * kvcache_mgmt.py:50-79, separate launches at transformer_layer.py:62-77) run in the attention kernel's
  * prologue; results are bit-identical to swl_splitk_rotary_store_kv_decode + swl_paged_attn_decode.
- * qkv_slabs: [k_splits][Bd][(H + 2*KVH) * D] fp32. Other arguments as swl_paged_attn_decode. */
+ * qkv_slabs: [k_splits][Bd][(H + 2*KVH) * D] fp32. Other arguments as swl_paged_attn_decode. waves: 4 or 8 waves share a sequence block of
+ * 512 tokens or more (4 serve shorter ones); 0: chosen from the grid, in which inert sequences and blocks past a sequence's end count. The
+ * order of a row's partial sums depends on it. */
 int swl_paged_attn_decode_qkv(void *o, const float *qkv_slabs, int32_t k_splits, const void *cos_table,
                               const void *sin_table, const int32_t *pos_idx, void *k_cache, void *v_cache,
                               const int32_t *block_table, const int32_t *seq_ids, const int32_t *seq_lens,
                               void *scratch, float softmax_scale, int32_t num_decoding_seqs,
                               int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t num_layers,
                               int32_t block_size, int32_t cur_layer, int32_t max_blocks_per_seq,
-                              int32_t seq_block_size, int32_t num_seq_blocks, int64_t o_tok_stride,
+                              int32_t seq_block_size, int32_t num_seq_blocks, int64_t o_tok_stride, int32_t waves,
                               int32_t dtype, swl_stream_t stream);
 
 /* ---- Greedy sampling --------------------------------------------------------------------------
@@ -375,7 +377,7 @@ int swl_paged_attn_decode_qkv_rs(void *o, const float *qkv_slabs, int32_t k_spli
                                  void *scratch, float softmax_scale, int32_t num_decoding_seqs, int32_t num_q_heads,
                                  int32_t num_kv_heads, int32_t head_dim, int32_t num_layers, int32_t block_size,
                                  int32_t cur_layer, int32_t max_blocks_per_seq, int32_t seq_block_size,
-                                 int32_t num_seq_blocks, int64_t o_tok_stride, int32_t dtype, swl_stream_t stream);
+                                 int32_t num_seq_blocks, int64_t o_tok_stride, int32_t waves, int32_t dtype, swl_stream_t stream);
 
 /* ---- decode projections for very small batches that consume the previous projection's slabs (csrc/gemm_tiny.hip) ----
  * M <= swl_gemm_tiny_max_tokens() (4). At batch 1 the two split-K consumers of a decode layer (swl_splitk_add_scale:
@@ -405,7 +407,7 @@ int swl_paged_attn_decode_qkv_rs_partials(void *o, const float *qkv_slabs, int32
                                           int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                                           int32_t num_layers, int32_t block_size, int32_t cur_layer,
                                           int32_t max_blocks_per_seq, int32_t seq_block_size, int32_t num_seq_blocks,
-                                          int64_t o_tok_stride, int32_t dtype, swl_stream_t stream);
+                                          int64_t o_tok_stride, int32_t waves, int32_t dtype, swl_stream_t stream);
 int swl_gemm_tiny_partial_from_attn(float *slabs_out, size_t slabs_out_bytes, int32_t k_splits_out,
                                     const float *attn_scratch, const int32_t *seq_lens, int32_t num_q_heads,
                                     int32_t head_dim, int32_t seq_block_size, int32_t num_seq_blocks,

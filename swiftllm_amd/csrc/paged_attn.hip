@@ -60,6 +60,7 @@ struct PagedAttnParams {
     const float *row_ssq; // [ssq_parts][Bd], NULL = the slabs are final
     int ssq_parts, hidden;
     float eps;
+    int waves;                 // QKV: waves of a workgroup, 4 or 8; 0 = by the launch's own grid
 };
 
 // ---- matrix-core variant of attend_block (G >= 2) --------------------------------------------------------------------
@@ -665,9 +666,10 @@ static int launch_phase1(const PagedAttnParams &p, int Bd, hipStream_t stream) {
     // With the new token's rotary and store in the prologue (QKV) a CU has registers for eight waves. In more than one round of workgroups,
     // two of four waves hide each other's prologue and merge: 120 requests of about 600 tokens, 8 kv heads of 128, 64.1 -> 59.2 us (5.0 TB/s),
     // 32 of about 1100 in two blocks 34.5 -> 30.3. (Without it three waves a SIMD fit either way: 37 us by eight waves, 41 by four.) Longest
-    // sequences first: the same for one block a sequence, 1 us for two.
-    const bool rounds = QKV && static_cast<int64_t>(p.KVH) * Bd * p.num_seq_blocks > 256;
-    if (p.seq_block_size >= 32 * kBlk && !rounds)
+    // sequences first: the same for one block a sequence, 1 us for two. A caller whose grid is padded says what the launch of its sequences
+    // alone would take (`waves`); otherwise the grid decides.
+    const bool four = p.waves ? p.waves == 4 : QKV && static_cast<int64_t>(p.KVH) * Bd * p.num_seq_blocks > 256;
+    if (p.seq_block_size >= 32 * kBlk && !four)
         hipLaunchKernelGGL((paged_attn_phase1_kernel<T, D, G, 8, QKV>), grid, dim3(512), 0, stream, p, p.block_table,
                            p.seq_lens, p.seq_ids);
     else
@@ -831,7 +833,7 @@ static int paged_attn_decode_qkv_impl(void *o, const float *qkv_slabs, int32_t k
                                       void *scratch, float softmax_scale, int32_t num_decoding_seqs,
                                       int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32_t num_layers,
                                       int32_t block_size, int32_t cur_layer, int32_t max_blocks_per_seq,
-                                      int32_t seq_block_size, int32_t num_seq_blocks, int64_t o_tok_stride, int32_t dtype,
+                                      int32_t seq_block_size, int32_t num_seq_blocks, int64_t o_tok_stride, int32_t waves, int32_t dtype,
                                       swl_stream_t stream, const float *row_ssq, int32_t ssq_parts, int32_t hidden,
                                       float eps, bool merge = true);
 
@@ -842,12 +844,12 @@ extern "C" int swl_paged_attn_decode_qkv(void *o, const float *qkv_slabs, int32_
                                          int32_t num_decoding_seqs, int32_t num_q_heads, int32_t num_kv_heads,
                                          int32_t head_dim, int32_t num_layers, int32_t block_size,
                                          int32_t cur_layer, int32_t max_blocks_per_seq, int32_t seq_block_size,
-                                         int32_t num_seq_blocks, int64_t o_tok_stride, int32_t dtype,
+                                         int32_t num_seq_blocks, int64_t o_tok_stride, int32_t waves, int32_t dtype,
                                          swl_stream_t stream) {
     return paged_attn_decode_qkv_impl(o, qkv_slabs, k_splits, cos_table, sin_table, pos_idx, k_cache, v_cache, block_table,
                                       seq_ids, seq_lens, scratch, softmax_scale, num_decoding_seqs, num_q_heads,
                                       num_kv_heads, head_dim, num_layers, block_size, cur_layer, max_blocks_per_seq,
-                                      seq_block_size, num_seq_blocks, o_tok_stride, dtype, stream, nullptr, 0, 0, 0.f);
+                                      seq_block_size, num_seq_blocks, o_tok_stride, waves, dtype, stream, nullptr, 0, 0, 0.f);
 }
 
 /* swl_paged_attn_decode_qkv on the slabs of a qkv projection whose input had its RMSNorm scale deferred
@@ -862,7 +864,7 @@ extern "C" int swl_paged_attn_decode_qkv_rs(void *o, const float *qkv_slabs, int
                                             int32_t num_decoding_seqs, int32_t num_q_heads, int32_t num_kv_heads,
                                             int32_t head_dim, int32_t num_layers, int32_t block_size,
                                             int32_t cur_layer, int32_t max_blocks_per_seq, int32_t seq_block_size,
-                                            int32_t num_seq_blocks, int64_t o_tok_stride, int32_t dtype,
+                                            int32_t num_seq_blocks, int64_t o_tok_stride, int32_t waves, int32_t dtype,
                                             swl_stream_t stream) {
     if (num_decoding_seqs == 0 || num_seq_blocks == 0) return num_decoding_seqs < 0 ? SWL_ERR_BAD_ARG : SWL_OK;
     if (!row_ssq || ssq_parts <= 0 || hidden <= 0) return SWL_ERR_BAD_ARG;
@@ -870,7 +872,7 @@ extern "C" int swl_paged_attn_decode_qkv_rs(void *o, const float *qkv_slabs, int
     return paged_attn_decode_qkv_impl(o, qkv_slabs, k_splits, cos_table, sin_table, pos_idx, k_cache, v_cache, block_table,
                                       seq_ids, seq_lens, scratch, softmax_scale, num_decoding_seqs, num_q_heads,
                                       num_kv_heads, head_dim, num_layers, block_size, cur_layer, max_blocks_per_seq,
-                                      seq_block_size, num_seq_blocks, o_tok_stride, dtype, stream, row_ssq, ssq_parts,
+                                      seq_block_size, num_seq_blocks, o_tok_stride, waves, dtype, stream, row_ssq, ssq_parts,
                                       hidden, eps);
 }
 
@@ -881,7 +883,7 @@ static int paged_attn_decode_qkv_impl(void *o, const float *qkv_slabs, int32_t k
                                          int32_t num_decoding_seqs, int32_t num_q_heads, int32_t num_kv_heads,
                                          int32_t head_dim, int32_t num_layers, int32_t block_size,
                                          int32_t cur_layer, int32_t max_blocks_per_seq, int32_t seq_block_size,
-                                         int32_t num_seq_blocks, int64_t o_tok_stride, int32_t dtype,
+                                         int32_t num_seq_blocks, int64_t o_tok_stride, int32_t waves, int32_t dtype,
                                          swl_stream_t stream, const float *row_ssq, int32_t ssq_parts, int32_t hidden,
                                          float eps, bool merge) {
     if (num_decoding_seqs < 0) return SWL_ERR_BAD_ARG;
@@ -898,6 +900,7 @@ static int paged_attn_decode_qkv_impl(void *o, const float *qkv_slabs, int32_t k
         !swl::aligned16(cos_table) || !swl::aligned16(sin_table))
         return SWL_ERR_BAD_ARG;
     if (num_decoding_seqs > 65535 || num_kv_heads > 65535) return SWL_ERR_UNSUPPORTED;
+    if (!(waves == 0 || waves == 4 || waves == 8)) return SWL_ERR_BAD_ARG;
     float *mid_o = nullptr, *mid_lse = nullptr;
     if (num_seq_blocks > 1) {
         if (!scratch || !swl::aligned16(scratch)) return SWL_ERR_BAD_ARG;
@@ -931,6 +934,7 @@ static int paged_attn_decode_qkv_impl(void *o, const float *qkv_slabs, int32_t k
     p.ssq_parts = ssq_parts;
     p.hidden = hidden;
     p.eps = eps;
+    p.waves = waves;
     const int G = num_q_heads / num_kv_heads;
     int rc;
     SWL_DISPATCH_DTYPE(dtype, T, {
@@ -955,13 +959,13 @@ extern "C" int swl_paged_attn_decode_qkv_rs_partials(void *o, const float *qkv_s
                                                      int32_t num_kv_heads, int32_t head_dim, int32_t num_layers,
                                                      int32_t block_size, int32_t cur_layer, int32_t max_blocks_per_seq,
                                                      int32_t seq_block_size, int32_t num_seq_blocks,
-                                                     int64_t o_tok_stride, int32_t dtype, swl_stream_t stream) {
+                                                     int64_t o_tok_stride, int32_t waves, int32_t dtype, swl_stream_t stream) {
     if (num_decoding_seqs == 0 || num_seq_blocks == 0) return num_decoding_seqs < 0 ? SWL_ERR_BAD_ARG : SWL_OK;
     if (!row_ssq || ssq_parts <= 0 || hidden <= 0) return SWL_ERR_BAD_ARG;
     if (ssq_parts > 8 || !(k_splits == 1 || k_splits == 2 || k_splits == 4)) return SWL_ERR_UNSUPPORTED;
     return paged_attn_decode_qkv_impl(o, qkv_slabs, k_splits, cos_table, sin_table, pos_idx, k_cache, v_cache, block_table,
                                       seq_ids, seq_lens, scratch, softmax_scale, num_decoding_seqs, num_q_heads,
                                       num_kv_heads, head_dim, num_layers, block_size, cur_layer, max_blocks_per_seq,
-                                      seq_block_size, num_seq_blocks, o_tok_stride, dtype, stream, row_ssq, ssq_parts,
+                                      seq_block_size, num_seq_blocks, o_tok_stride, waves, dtype, stream, row_ssq, ssq_parts,
                                       hidden, eps, false);
 }

@@ -45,3 +45,5 @@ class LlamaInferState:
     last_token_indices: Optional[torch.Tensor] = None   # [batch_size] int32
     # Preallocated fp32 scratch for the flash-decoding partials.
     paged_attn_scratch: Optional[torch.Tensor] = None
+    # Waves of a workgroup of the slab-fed decode attention: 4 or 8 (batch_plan.decode_attention_waves), 0: by the launch's own grid.
+    paged_attn_waves: int = 0

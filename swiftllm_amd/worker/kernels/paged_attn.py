@@ -47,16 +47,16 @@ def paged_attention_from_qkv_splitk(partials, k_cache: torch.Tensor, v_cache: to
                                     cur_layer: int, o: torch.Tensor, row_scale=None, merge: bool = True):
     """Pure-decode batches: rotary + KV-store + paged attention in one launch, fed by the split-K partial slabs
     of the fused qkv projection (kernels/linear.py: SplitKPartials). Same bits as
-    rotary_embedding_and_store_kvcache_decode_from_splitk followed by paged_attention, except that in sequence blocks
-    of 512 tokens and more beyond 256 workgroups four waves share a block's keys where that has eight (the outputs'
-    partial sums meet in another order); q/k/v never exist as tensors (the rotated k and the v go to the pools, q stays in the
-    kernel)."""
+    rotary_embedding_and_store_kvcache_decode_from_splitk followed by paged_attention, except that four waves may share the keys of a
+    sequence block of 512 tokens and more where that has eight (`infer_state.paged_attn_waves`, batch_plan.decode_attention_waves: the
+    outputs' partial sums then meet in another order); q/k/v never exist as tensors (the rotated k and the v go to the pools, q stays in
+    the kernel)."""
     nd = infer_state.num_decoding_seqs
     if nd == 0:
         return
     h, kvh, d = model_config.num_q_heads, model_config.num_kv_heads, model_config.head_dim
     assert infer_state.num_prefill_seqs == 0 and infer_state.position_indices is not None
-    nsb = infer_state.num_seq_blocks
+    nsb, waves = infer_state.num_seq_blocks, getattr(infer_state, "paged_attn_waves", 0)
     assert o is not None or (not merge and nsb > 1), "no output tensor: only for split sequences with merge=False"
     assert partials.shape == (nd, (h + 2 * kvh) * d) and partials.dtype == k_cache.dtype
     assert k_cache.is_contiguous() and v_cache.is_contiguous() and block_table.is_contiguous()
@@ -85,7 +85,7 @@ def paged_attention_from_qkv_splitk(partials, k_cache: torch.Tensor, v_cache: to
                   _hip.ptr(infer_state.position_indices), _hip.ptr(k_cache), _hip.ptr(v_cache), _hip.ptr(block_table),
                   _hip.ptr(infer_state.seq_ids), _hip.ptr(infer_state.decoding_seq_lens), _hip.ptr(scratch),
                   infer_state.softmax_scale, nd, h, kvh, d, model_config.num_layers, engine_config.block_size,
-                  cur_layer, block_table.shape[1], infer_state.seq_block_size, nsb, o_stride,
+                  cur_layer, block_table.shape[1], infer_state.seq_block_size, nsb, o_stride, waves,
                   _hip.dtype_code(o_dtype), _hip.stream())
         return scratch if not merge and nsb > 1 else None
     assert merge, "phase-1-only attention needs the deferred-norm entry point"
@@ -94,5 +94,5 @@ def paged_attention_from_qkv_splitk(partials, k_cache: torch.Tensor, v_cache: to
               _hip.ptr(infer_state.position_indices), _hip.ptr(k_cache), _hip.ptr(v_cache), _hip.ptr(block_table),
               _hip.ptr(infer_state.seq_ids), _hip.ptr(infer_state.decoding_seq_lens), _hip.ptr(scratch),
               infer_state.softmax_scale, nd, h, kvh, d, model_config.num_layers, engine_config.block_size,
-              cur_layer, block_table.shape[1], infer_state.seq_block_size, nsb, token_stride(o, "o"),
+              cur_layer, block_table.shape[1], infer_state.seq_block_size, nsb, token_stride(o, "o"), waves,
               _hip.dtype_code(o.dtype), _hip.stream())

@@ -31,7 +31,7 @@ from swiftllm_amd.engine_config import EngineConfig
 from swiftllm_amd.model_config import LlamaModelConfig
 from swiftllm_amd.utils import GB
 
-from .batch_plan import BatchPlan, plan_batch
+from .batch_plan import BatchPlan, decode_attention_waves, plan_batch
 from .block_manager import BlockManager
 from . import decode_engine as _decode_engine
 from .infer_state import LlamaInferState
@@ -367,7 +367,11 @@ class LlamaModel:
             position_cos=self._cos_cached, position_sin=self._sin_cached,
             ignore_kvcache=ignore_kvcache,
             position_indices=dev["position_indices"], last_token_indices=dev["last_token_indices"],
-            paged_attn_scratch=self._scratch if nsb > 1 else None)
+            paged_attn_scratch=self._scratch if nsb > 1 else None, paged_attn_waves=self._attention_waves(plan))
+
+    def _attention_waves(self, plan: BatchPlan) -> int:
+        return decode_attention_waves(plan.real_seqs, plan.max_decoding_len, self.model_config.num_kv_heads, plan.seq_block_size,
+                                      self._num_slots)
 
     @torch.inference_mode()
     def _forward(self, input_ids: torch.Tensor, infer_state: LlamaInferState) -> torch.Tensor:
@@ -493,9 +497,9 @@ class LlamaModel:
         tap_len = len(tap) if tap is not None else 0
         # (the engine has one launch geometry; a graph captured while a test taps the logits keeps its [B, vocab] tensor
         # alive in the shared pool, one captured without the tap does not — up to 65 MB per graph at 256 sequences)
-        key = ((1, 0, 0) if use_engine else (plan.batch_size, sbs, nsb_cap)) + (tap is not None,)
-        entry = self._decode_graphs.pop(key, None)
         plan.seq_block_size, plan.num_seq_blocks = sbs, nsb_cap
+        key = ((1, 0, 0, 0) if use_engine else (plan.batch_size, sbs, nsb_cap, self._attention_waves(plan))) + (tap is not None,)
+        entry = self._decode_graphs.pop(key, None)
         if entry is None:
             self.graph_captures += 1
             t_cap = time.perf_counter()

@@ -611,6 +611,29 @@ def test_large_decode_batches_take_the_wide_kernels_and_match_the_oracle(tmp_pat
     assert ("swl_gemm_packed_wide_silu_gate" in wide) == (batch <= 128), sorted(set(wide))
 
 
+def test_a_batch_rounded_up_to_its_bucket_keeps_the_bits_of_its_exact_size(tmp_path):
+    """Six sequences of more than 512 tokens over 40 kv heads: 240 workgroups of attention, 320 in the bucket of eight that a replay runs. The
+    inert ones are no second round: tokens and logits of a replayed step are those of an eager step of six, bit for bit."""
+    cfg = synth.make_config(num_hidden_layers=2, hidden_size=1280, num_attention_heads=40, num_key_value_heads=40,
+                            intermediate_size=1024, vocab_size=512, max_position_embeddings=1024)
+    sd = synth.make_state_dict(cfg, seed=12, dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(4)
+    prompts = [torch.randint(0, cfg["vocab_size"], (600 + 17 * i,), generator=g).tolist() for i in range(6)]
+    runs = {}
+    for graph in (False, True):
+        model = _make_model(tmp_path / f"g{int(graph)}", cfg, sd, 6 * 48 + 8, max_blocks_per_seq=64, max_tokens_in_batch=8192,
+                            max_batch_size=8, max_seqs_in_block_table=16, dtype="bfloat16", use_hip_graph=graph)
+        toks = _run_script(model, prompts, 4)
+        runs[graph] = (toks, [t.clone() for t in model.post_layer.logits_tap])
+        if graph:
+            assert {k[0] for k in model._decode_graphs} == {8}
+        del model
+        torch.cuda.empty_cache()
+    assert runs[True][0] == runs[False][0]
+    for a, b in zip(runs[True][1], runs[False][1]):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("batch", [100, 200])
 def test_large_decode_batches_replay_their_hip_graph_bit_for_bit(tmp_path, batch, monkeypatch):
     """The product default (hipGraph replay) at decode batches beyond 64: the captured graph — wide GEMMs, their slabs into

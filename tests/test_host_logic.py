@@ -501,6 +501,24 @@ def test_saved_routes_of_another_kernel_or_method_are_not_read(tmp_path, monkeyp
     assert st["measured"] == len(R.BUCKETS) and R.decide(160, 7168, 7168, bf16, False)
 
 
+def test_attention_waves_follow_the_sequences_as_they_are():
+    """batch_plan.decode_attention_waves: rounding a decode batch up to its replay bucket, or its splits up to a power of two, does not change
+    the form of the attention launch, and with the form the order of the sums."""
+    from types import SimpleNamespace
+    from swiftllm_amd.worker.model import LlamaModel
+    for kvh, lens, sbs, want in [(40, [600] * 6, 1024, 8),           # 240 workgroups; padded to 8 sequences 320
+                                 (10, [700] * 25, 1024, 8),          # 250; padded to 32 320
+                                 (8, [4000] * 4, 512, 8),            # 256; padded to 8 sequences 512
+                                 (8, [5500, 3000, 2000, 5000, 4000], 640, 4),
+                                 (8, [1100] * 32, 640, 4), (8, [600] * 120, 1024, 4), (8, [5500], 448, 4), (8, [512], 512, 8)]:
+        model = SimpleNamespace(model_config=SimpleNamespace(num_kv_heads=kvh), _num_slots=256,
+                                _decode_batch_bucket=lambda b: LlamaModel._decode_batch_bucket(None, b))
+        for pad in (False, True):
+            plan = LlamaModel._plan_decode(model, list(range(len(lens))), lens, None, pad)
+            plan.seq_block_size, plan.num_seq_blocks = sbs, 1 << (-(-max(lens) // sbs) - 1).bit_length()
+            assert LlamaModel._attention_waves(model, plan) == want, (kvh, len(lens), pad)
+
+
 def test_tiny_batch_projection_policy():
     """kernels/linear.py: when may a projection consume the previous projection's slabs / the attention partials itself?
     (pure host logic: shapes, packed twin, K-chunk that fits LDS; the layer additionally limits the batch to 2)."""
