@@ -2,6 +2,7 @@
 the KV store, then sliding-window attention with tanh soft-capping and an [H, H] head-mixing matrix. Prompt portions (with
 or without a cached prefix) and decoded tokens go through the same two launches: every token carries its block-table row
 and its position. csrc/qknorm_kv.hip, csrc/window_attn.hip."""
+import numpy as np
 import torch
 
 from swiftllm_amd import _hip
@@ -99,17 +100,30 @@ def qkv_bias_norm_store(qkv: torch.Tensor, q_b: torch.Tensor, k_b: torch.Tensor,
 class StepTiles(tuple):
     """(tile_row0, tile_cnt) of a step, and its spans: runs of up to 32 consecutive tokens of one portion (row0, cnt, and per token
     the position where its portion starts). longest: the longest sequence of the step (spans only: never under graph replay).
-    span_order: the spans in the order to take them up (StepPlan.span_order; None: last to first)."""
+    span_order: the spans in the order to take them up (StepPlan.span_order; None: last to first). portions: (lengths after the step, tokens)
+    of the sequences, on the host."""
 
-    def __new__(cls, tile_row0, tile_cnt, spans=None, longest=0, span_order=None):
+    def __new__(cls, tile_row0, tile_cnt, spans=None, longest=0, span_order=None, portions=None):
         self = super().__new__(cls, (tile_row0, tile_cnt))
         self.spans, self.longest, self.span_order = spans, longest, span_order
+        self._portions, self._keys = portions, None
         return self
 
     @classmethod
     def of(cls, dev):
         return cls(dev["tile_row0"], dev["tile_cnt"], (dev["chunk_row0"], dev["chunk_cnt"], dev["tok_start"]), dev.get("longest", 0),
-                   dev.get("span_order"))
+                   dev.get("span_order"), dev.get("portions"))
+
+    def keys(self, tokens: int):
+        """(keys that the step's tokens see, summed; lengths of the sequences that bring fewer than eight tokens, summed). Made when first asked
+        for, where the device is already at work on the step."""
+        if self._keys is None:
+            if self._portions is None:
+                self._keys = tokens * self.longest, 0
+            else:
+                lens, cnt = np.asarray(self._portions[0], dtype=np.int64), np.asarray(self._portions[1], dtype=np.int64)
+                self._keys = int((cnt * (2 * lens - cnt + 1)).sum()) // 2, int(lens[cnt < 8].sum())
+        return self._keys
 
 
 # A step whose spans hold this many tokens on average or more is a prompt step (a span of one token fills one of a workgroup's 128 rows a
@@ -118,6 +132,31 @@ class StepTiles(tuple):
 # 18 / 32; 64 portions of 4 at 2000 keys 51 / 118, 115 / 179, 53 / 157; 200 decoded tokens at 1000 keys beside one portion of 930 92 / 299,
 # 359 / 755, 205 / 717; 30 at 3900 keys beside one of 200 56 / 157, 71 / 178, 44 / 123.
 SPAN_MIN_TOKENS = 4
+
+
+def span_shares(n: int, spans: int, H: int, G: int, dim: int, vdim: int, window: int, longest: int, row_keys: int, lone_keys: int) -> int:
+    """Over how many workgroups the keys of every tile of a prompt step are shared out: 1, 2, 4, or 8 where all of them are on the chip at
+    once. The longest walk of a workgroup and what a CU has to walk in all (us a page of 16 keys, the slower of the two is the launch's time)
+    shrink and stay; shares cost a launch and, each, the partial results written and read. Measured at 196 steps of 200 to 8000 tokens,
+    prompts alone and beside 1 to 30 decoded tokens at 0.8k to 8k keys, 4 to 40 heads of 64 to 576 columns over 1 to 8, windows of 256 to
+    1024: 3 % above the best of 1, 2, 4 and 8 on average (by workgroups and the longest sequence alone: 12 %). us by
+    shares, 8 heads of 128 over 2: 2000 tokens 40.7 (1), 43.6 (2), 43.4 (4), beside 30 at 3900 keys 74.0, 70.8, 62.7; 4 x 500 beside 8 at
+    8000 keys 140, 115, 91; 8 x 200 11.0, 24.4, 29.3, beside one at 2000 keys 40.4, 36.0, 31.9."""
+    narrow = dim + vdim <= 320      # (two workgroups of 64 rows a CU; wide rows: one of 128)
+    rows, slots = (64, 2 * _NUM_CUS) if narrow else (128, _NUM_CUS)
+    wide = (dim + 2 * vdim) / 1600
+    walk_us, load_us = (0.2, 0.3) if narrow else (1.07 * wide, 1.9 * wide)
+    queries = max(1, rows >> (H // G - 1).bit_length())     # of a workgroup
+    if window > 0:
+        longest, row_keys, lone_keys = min(longest, window), min(row_keys, n * window), min(lone_keys, spans * window)
+    walk, load = walk_us * (longest // 16 + 1), load_us * (row_keys / queries + lone_keys) * G / 16 / slots
+    share = n * H * (vdim + 2) * 8 / 6e6        # (6 TB/s)
+    best, best_us = 1, max(walk, load)
+    for splits in (2, 4, 8):
+        us = max(walk / splits, load) + 9 + splits * share
+        if us < best_us and (splits < 8 or 8 * G * max(n / queries, spans) <= slots):
+            best, best_us = splits, us
+    return best
 
 
 def _span_launch(q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles, H, G, GV, dim, vdim, window, mask_kind, scale, softcap,
@@ -132,12 +171,7 @@ def _span_launch(q, out, kp, vp, pool, block_table, tok_seq, tok_pos, tiles, H, 
     if (q.data_ptr() | kp | vp) % 16 or q.stride(0) % 8 or pool.shape[1] % 8:      # 16-byte operand loads
         return False
     row0, cnt, start = spans
-    # workgroups of 64 rows (queries x heads of a key head; wide rows: 128). Few of them: every tile's keys are shared out, many only where
-    # the walk is long, as partial results cost a launch and their bytes. us by shares, 8 heads of 128 over 2: 57 tokens at 17 to 692
-    # 18.5 (1), 15.2 (3), 14.4 (8); 500 tokens 15.5 (1), 17.7 (2), 16.0 (4); 1500 33.9 (1), 36.5 (2); 2000 beside 30 decoded 29 (1), 39 (2), 42 (4)
-    groups = max(1, n * H // ((64 if dim + vdim <= 320 else 128) * G)) * G
-    pages = (min(window, tiles.longest) if window > 0 else tiles.longest) // 16 + 1
-    splits = max(1, min(_NUM_CUS // groups, pages // (8 if groups <= 32 else 32), 8))
+    splits = span_shares(n, row0.shape[0], H, G, dim, vdim, window, tiles.longest, *tiles.keys(n))
     splits, scratch = share_scratch(q.device, splits, n * H * (vdim + 2))
     _hip.call("swl_span_attn_ordered", _hip.ptr(tiles.span_order), tiles.longest, _hip.ptr(out), _hip.ptr(q), kp, vp,
               _hip.ptr(block_table), _hip.ptr(tok_seq), _hip.ptr(tok_pos), _hip.ptr(start), _hip.ptr(row0), _hip.ptr(cnt), _hip.ptr(rel), rel.shape[1] if rel is not None else 0, row0.shape[0],

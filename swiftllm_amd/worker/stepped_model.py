@@ -208,7 +208,7 @@ class SteppedModel:
             self.gpu_block_manager.allocate_blocks_for_seqs(plan.seq_ids_list, plan.target_lens_list)
         self._begin_state_step(plan)
         dev = self._upload_plan(plan)
-        dev["longest"] = int(max(plan.target_lens_list))
+        dev["longest"], dev["portions"] = int(max(plan.target_lens_list)), (plan.target_lens_list, plan.seq_cnt)
         dev["longest_portion"] = 1 if plan.num_tokens == plan.num_seqs else int(plan.seq_cnt.max())
         if (getattr(self.engine_config, "use_hip_graph", False) and not ignore_kvcache and self.layer_tap is None
                 and plan.num_tokens == plan.num_seqs == plan.want_rows.size):
