@@ -161,7 +161,7 @@ class SteppedModel:
     def _upload_plan(self, plan: StepPlan):
         """The plan's int32 arrays through ONE pinned buffer and ONE async copy; returns device views."""
         layout, total = plan.packed_layout()
-        order = plan.span_order()
+        order = plan.upload_order()
         order_at, total = total, total + (order.size if order is not None else 0)
         if self._meta_done is not None:
             self._meta_done.synchronize()

@@ -88,6 +88,16 @@ def test_span_order_takes_runs_of_four_from_the_highest_positions():
     assert order.tolist() == [c for r in runs for c in r[2]]
 
 
+@pytest.mark.parametrize("parts,ordered", [([(0, 2000)] + [(800, 1)] * 30, False), ([(0, 4096)], False), ([(0, 4097)], True),
+                                           ([(0, 333)] * 12, True), ([(0, 333)] * 11, False), ([(5, 1)] * 200, False)])
+def test_small_steps_go_without_an_order(parts, ordered):
+    """Up to 128 spans (and in steps of one token each) the order costs the host more than it gives the launches."""
+    plan = plan_step([StepEntry(i, [1] * n, a) for i, (a, n) in enumerate(parts)])
+    order = plan.upload_order()
+    assert (order is not None) == ordered
+    assert order is None or order.tolist() == plan.span_order().tolist()
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 33, 65])
 def test_plan_of_one_token_each(n):
     """plan_tokens is plan_step of the same entries, array for array, and gives none where plan_step refuses."""
