@@ -7,7 +7,11 @@
 // than the library's, and the same whatever M is.
 // Measured (us, w cycled through 600 MB; library product -> here) at 1 / 3 / 8 / 16 tokens: 1024 x 1024 10.8 -> 2.8 / 11.0 -> 3.1 / 11.0 -> 4.0 /
 // 11.0 -> 5.5; 3200 x 1024 11.5 -> 4.4 / 4.9 / 6.4 / 11.8; 1024 x 4096 12.3 -> 5.8 / 6.5 / 10.3 / 12.1; 8192 x 1024 14.4 -> 7.6 / 8.0 / 11.0 / 21;
-// 32000 x 1024 36 -> 21.7 / 22.5 / 33.6 / 66. So: up to 8 tokens always, up to 16 where w has at most 2048 rows. Error against 64 bits 1.0e-7
+// 32000 x 1024 36 -> 21.7 / 22.5 / 33.6 / 66. Beyond a few tokens their share of x, read for every four rows, is what costs, and a library that
+// shares K over workgroups wins where there are many rows and columns. Library / here, at 4 tokens: 4096 x 4096 16.7 / 16.1, 4096 x 14336 47.9 /
+// 46.4, 28672 x 4096 113 / 78; at 8: 1024 x 16384 37.5 / 28.4, 1536 x 8192 22.1 / 20.5, 4096 x 3072 18.4 / 15.1, 2048 x 4096 13.6 / 14.3,
+// 4096 x 4096 16.6 / 20.1, 8192 x 2048 17.9 / 21.4; at 16: 1024 x 16384 38.1 / 34.6, 1536 x 2048 11.8 / 9.6, 1280 x 4096 12.8 / 16.1, 2048 x 1536
+// 10.0 / 11.2, 2048 x 8192 24 / 34. Hence the lines of swl_gemm_f32_supported. Error against 64 bits 1.0e-7
 // (relative, 2-norm) where the library's is 2.9e-7, at K 4096 1.2e-7 and 5.8e-7. Waves that share K (1 / 2 / 4): 4.9 / 3.6 / 3.1 us at
 // 1024 x 1024, 5.9 / 4.9 / 4.9 at 3200 rows, 26.1 / 22.5 / 22.4 at 32000.
 #include "swl_common.h"
@@ -98,7 +102,9 @@ static void launch_f32(int ks, hipStream_t s, float *out, const float *x, const 
  * product too. */
 extern "C" int swl_gemm_f32_supported(int32_t M, int32_t N, int32_t K) {
     if (M <= 0 || M > swl::kF32MaxTokens || N <= 0 || K <= 0 || K % 4) return 0;
-    return M <= 8 || N <= 2048 ? 2 : 1;
+    if (M <= 4) return 2;
+    if (M <= 8) return N <= 1536 || K <= 1024 || (N <= 4096 && K <= 3072) ? 2 : 1;
+    return N <= 1024 || (N <= 1536 && K <= 2048) || (N <= 2048 && K <= 1024) ? 2 : 1;
 }
 
 extern "C" int swl_gemm_f32(float *out, const float *x, const float *w, int32_t M, int32_t N, int32_t K, int64_t x_row_stride,

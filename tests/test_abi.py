@@ -117,3 +117,13 @@ def test_split_choosers_are_host_functions_with_the_documented_values():
                 assert kt // p >= 8
     assert even(100, 4096) == 0 and packed(4096, 100) == 0          # N % 32, K % 128
     assert lib.swl_gemm_tiny_max_tokens() == 4
+
+
+@pytest.mark.parametrize("M,N,K,faster", [
+    (4, 28672, 4096, True), (4, 4096, 14336, True), (8, 1024, 16384, True), (8, 1536, 8192, True), (8, 4096, 3072, True), (8, 32000, 1024, True),
+    (8, 2048, 4096, False), (8, 4096, 4096, False), (8, 8192, 2048, False), (8, 4096, 14336, False), (16, 1024, 16384, True),
+    (16, 1536, 2048, True), (16, 2048, 1024, True), (16, 1280, 4096, False), (16, 2048, 1536, False), (16, 2048, 8192, False), (16, 3200, 512, False)])
+def test_fp32_products_of_a_few_tokens_know_where_the_library_is_faster(M, N, K, faster):
+    """swl_gemm_f32_supported: 2 only where the kernel was measured ahead of a library product (csrc/gemm_f32.hip); 1 where it can run."""
+    from swiftllm_amd import _hip
+    assert _hip.load().swl_gemm_f32_supported(M, N, K) == (2 if faster else 1)
