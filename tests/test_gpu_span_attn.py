@@ -1,6 +1,7 @@
 """The prompt form of the paged attention (csrc/span_attn.hip) against the same attention in float64: edges of the 32-token spans and
 32-key stages, every kind of row grouping (query heads a key head), masks, bias, slopes, cap, sink, gate, narrow outputs, key shares."""
 import math
+import random
 
 import pytest
 import torch
@@ -155,6 +156,25 @@ def test_key_shares(case, shares, dtype, monkeypatch):
     monkeypatch.setattr(window_attn, "share_scratch", forced)
     test_span_attention(case, [(1, 96, 31), (2, 0, 64), (3, 250, 1), (4, 15, 130)], dtype)
     assert used == [shares, shares]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shares", [1, 3])
+@pytest.mark.parametrize("case", [i for i, c in enumerate(CASES) if c[3] + c[4] <= 320])
+def test_steps_of_many_workgroups(case, shares, dtype, monkeypatch):
+    """The same at more than 640 workgroups of 64 rows, where rows of up to 320 elements take the form of one wave a row group (128 rows):
+    portions of 1 to 70 tokens, with and without keys before them."""
+    from swiftllm_amd.worker.kernels import window_attn
+    H, G = CASES[case][:2]
+    queries, pick, parts, spans = 64 >> (H // G - 1).bit_length(), random.Random(case), [], 0
+    while spans * G * 32 <= 640 * queries:
+        n = pick.choice([1, 15, 31, 32, 33, 47, 64, 70])
+        parts.append((len(parts) + 1, pick.choice([0, 0, 16, 37, 100]), n))
+        spans += -(-n // 32)
+    if shares > 1:
+        monkeypatch.setattr(window_attn, "share_scratch", lambda device, splits, floats: (
+            shares, torch.full((shares * floats,), float("nan"), device=device)))
+    test_span_attention(case, parts, dtype)
 
 
 @pytest.mark.parametrize("H,G,d,dv,window", [(8, 2, 128, 128, 0), (4, 4, 64, 64, 100), (6, 2, 192, 128, 0), (8, 1, 576, 512, 300),
