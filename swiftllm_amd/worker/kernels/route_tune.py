@@ -31,9 +31,9 @@ BUCKETS = tuple(range(96, 257, _TOKEN_BUCKET))      # 65..96, ..128, ... ..256 t
 _WIN_MARGIN = 1.03
 _LOCK_WAIT_S = 120.0
 # Part of the key under which answers are saved. Raised whenever the hand-written kernel or the way of timing changes, so that answers of
-# others are not read any more: 1 both sides timed back to back on one weight, x alone through LDS; 2 cold weights, LDS rings of both
-# operands.
-_REVISION = 2
+# others are not read any more: 1 both sides timed back to back on one weight, x alone through LDS; 2 behind a written buffer, LDS rings of
+# both operands; 3 behind a buffer that was read.
+_REVISION = 3
 
 _table = {}             # "N,K,dtype,bucket,silu" -> bool: this process's deployment table
 _device_key_cache = {}
@@ -140,15 +140,18 @@ _COLD_BYTES = 512 << 20     # twice the Infinity Cache
 
 
 def time_us(fn, iters: int = 8, warm: int = 2) -> float:
-    """Median of `iters` calls, each after a buffer past the Infinity Cache was rewritten: a decode step finds a projection's weights in
-    HBM. (Called back to back on one weight, a side without non-temporal loads gets most of it from the cache: the head of 32000 x 4096 at
-    128 tokens took 64 us from the library cold and less than the 47 of the hand-written kernel warm.)"""
-    cold = torch.empty(_COLD_BYTES, dtype=torch.uint8, device="cuda")
+    """Median of `iters` calls, each after a buffer past the Infinity Cache was read: a decode step finds a projection's weights in HBM. (Called
+    back to back on one weight, a side without non-temporal loads gets most of it from the cache: the head of 32000 x 4096 at 128 tokens
+    took 64 us from the library cold and less than the 47 of the hand-written kernel warm. A buffer that was WRITTEN leaves its lines to be
+    put back by whoever needs their place: the library's loads then take up to twice as long, 94.8 for 52.8 us at 28672 x 4096 and 96 tokens,
+    and the hand-written kernel, whose weights pass the caches by, was chosen wherever it was allowed: o at 224 tokens 28.5 for 30.3 us
+    there, 28.4 for 25.1 behind a read buffer, 26.3 for 22.7 with the weights cycled through 1.2 GB.)"""
+    cold = torch.empty(_COLD_BYTES // 4, dtype=torch.int32, device="cuda")
     for _ in range(warm):
         fn()
     pairs = []
     for _ in range(iters):
-        cold.zero_()
+        cold.amax()
         s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         s.record()
         fn()

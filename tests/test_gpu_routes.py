@@ -72,3 +72,23 @@ def test_two_replicas_of_one_deployment_route_alike_and_return_identical_logits(
     measured = sum("classes measured" in e and " 0 (shape" not in e for _, e in outs)
     print("\n[routes] replicas that measured:", measured, "table entries:", len(a["table"]),
           "hand-written kernel chosen for:", sorted(k for k, v in a["table"].items() if v))
+
+
+def test_cold_timing_costs_neither_side_more_than_a_stream_of_other_weights():
+    """route_tune.time_us stands for a step that comes to each weight with clean caches full of others: a library product behind its buffer
+    takes what it takes with the weights cycled through 1.2 GB (a buffer that was written instead of read: 1.6 times that)."""
+    import torch
+    import torch.nn.functional as F
+    from swiftllm_amd.worker.kernels import route_tune
+    a = torch.randn(96, 4096, device="cuda").bfloat16()
+    ws = [torch.randn(28672, 4096, device="cuda").bfloat16() for _ in range(6)]
+    for w in ws:
+        F.linear(a, w)
+    s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    s.record()
+    for i in range(30):
+        F.linear(a, ws[i % 6])
+    e.record()
+    e.synchronize()
+    cycled = s.elapsed_time(e) * 1e3 / 30
+    assert route_tune.time_us(lambda: F.linear(a, ws[0])) <= 1.3 * cycled
