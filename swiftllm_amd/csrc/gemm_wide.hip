@@ -23,7 +23,8 @@
 //     as linear -> silu_and_mul_inplace (silu_and_mul.py:16-23).
 // Bits: every output is the fp32 sum over k in ascending 16-element steps inside a K-chunk, chunks added in slab
 // order — the summation order of the M <= 64 kernels at the same split count.
-// Measured (us, bf16, W cycled through 1.2 GB; W through registers -> now), at 120 / 192 / 256 tokens: qkv 6144 x 4096 19.7 -> 17.1 /
+// Measured (us, bf16, W cycled through 1.2 GB, this kernel alone: adding up K shares takes another 4 to 7; W through registers -> now; on other cards and
+// in long runs up to a fifth more: 18.0 / 21.2 / 25.2, 15.6 / 17.6 / 20.9, 56 / 67 / 81, 31.5 / 38.9 / 46.7, 57 / 74 / 87), at 120 / 192 / 256 tokens: qkv 6144 x 4096 19.7 -> 17.1 /
 // 24.0 -> 20.2 / 29.8 -> 25.1; o 4096 x 4096 17.5 -> 15.0 / 17.8 -> 16.5 / 22.2 -> 19.8; up/gate + SiLU 51.9 -> 47.3 / 65.4 -> 53.7 /
 // 83.6 -> 67.6; down 4096 x 14336 28.6 -> 27.4 / 37.7 -> 32.7 / 45.2 -> 40.6; head 32000 x 4096 51.7 -> 47.5 / 66.7 -> 57.1 / 82.3 -> 73.6.
 #include "swl_common.h"

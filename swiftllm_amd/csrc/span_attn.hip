@@ -488,7 +488,9 @@ int launch_span(SpanParams &p, int key_splits, hipStream_t s) {
 
 // Two waves a row group halve a workgroup's walk, one halves the workgroups, the pages they stage and what each spends before its first
 // stage. us by workgroups of 64 rows, 128 + 128 columns, two / one: 11 x 333 tokens, 458: 16.8 / 18.4; 3 x 1500, 562: 39 / 54; 32 x 100, 800: 21.5 /
-// 15.3; 22 x 333, 916: 28.8 / 23.0; 8 x 920, 920: 44 / 41; 4 x 1841, 920: 73 / 73, with a bias 72 / 79; 4 x 1841, 1840: 120 / 115.
+// 15.3; 22 x 333, 916: 28.8 / 23.0; 8 x 920, 920: 44 / 41; 5 x 1472, 920: 54 / 53; 4 x 1841, 920: 73 / 73, with a bias 72 / 79; 3 x 2450, 924:
+// 79 / 82; 7200, 900: 193 / 221; 4 x 1841, 1840: 120 / 115. The longest walk may be a decoded token's: 22 x 333 beside one at 2000 keys 43.6 / 66.9,
+// beside one at 8000 141 / 240 (972).
 template <typename T, int D, int DV>
 int launch_span_any(SpanParams &p, int key_splits, int longest, hipStream_t s) {
     if constexpr (span_halves(D, DV) == 2) {
@@ -518,14 +520,16 @@ extern "C" int swl_span_attn_supported(int32_t num_q_heads, int32_t num_kv_heads
     return 0;
 }
 
-static int span_attn(const int32_t *span_order, int32_t longest, void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
-                             const int32_t *tok_seq, const int32_t *tok_pos, const int32_t *tok_start, const int32_t *span_row0,
-                             const int32_t *span_cnt, const float *rel, int32_t rel_len, int32_t num_spans, int32_t num_q_heads,
-                             int32_t num_kv_heads, int32_t num_v_heads, int32_t dim, int32_t vdim, int64_t q_tok_stride,
-                             int32_t window, int32_t mask_kind, float scale, float softcap, int32_t max_blocks_per_seq,
-                             int64_t block_stride, int32_t key_splits, float *scratch, int64_t num_tokens, const float *sink,
-                             int32_t out_f32, const float *slopes, int32_t out_dim, int64_t out_stride, const void *gate,
-                             int64_t gate_stride, int32_t dtype, swl_stream_t stream) {
+/* span_order: the spans in the order in which workgroups take them up (a permutation, or NULL); longest: tokens of the longest sequence
+ * (0: not known). */
+extern "C" int swl_span_attn_ordered(const int32_t *span_order, int32_t longest, void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
+                                     const int32_t *tok_seq, const int32_t *tok_pos, const int32_t *tok_start, const int32_t *span_row0,
+                                     const int32_t *span_cnt, const float *rel, int32_t rel_len, int32_t num_spans, int32_t num_q_heads,
+                                     int32_t num_kv_heads, int32_t num_v_heads, int32_t dim, int32_t vdim, int64_t q_tok_stride,
+                                     int32_t window, int32_t mask_kind, float scale, float softcap, int32_t max_blocks_per_seq,
+                                     int64_t block_stride, int32_t key_splits, float *scratch, int64_t num_tokens, const float *sink,
+                                     int32_t out_f32, const float *slopes, int32_t out_dim, int64_t out_stride, const void *gate,
+                                     int64_t gate_stride, int32_t dtype, swl_stream_t stream) {
     if (num_spans < 0 || window < 0 || mask_kind < 0 || mask_kind > 1 || key_splits < 1 || key_splits > 64) return SWL_ERR_BAD_ARG;
     if (key_splits > 1 && (!scratch || num_tokens <= 0 || !swl::aligned16(scratch))) return SWL_ERR_BAD_ARG;
     if (out_dim <= 0 || out_dim > vdim || out_stride < static_cast<int64_t>(num_q_heads) * out_dim) return SWL_ERR_BAD_ARG;
@@ -550,7 +554,6 @@ static int span_attn(const int32_t *span_order, int32_t longest, void *out, cons
     p.part_ml = scratch ? scratch + static_cast<int64_t>(key_splits) * num_tokens * num_q_heads * vdim : nullptr;
     p.rel_len = rel_len; p.num_spans = num_spans; p.H = num_q_heads; p.G = num_kv_heads; p.GV = num_v_heads;
     p.window = window; p.mask_kind = mask_kind; p.max_blocks = max_blocks_per_seq; p.out_f32 = out_f32; p.out_dim = out_dim;
-    
     p.scale = scale; p.softcap = softcap;
     p.q_stride = q_tok_stride; p.block_stride = block_stride; p.out_stride = out_stride; p.gate_stride = gate_stride;
     p.num_tokens = num_tokens;
@@ -569,18 +572,8 @@ extern "C" int swl_span_attn(void *out, const void *q, const void *k_cache, cons
                              int64_t block_stride, int32_t key_splits, float *scratch, int64_t num_tokens, const float *sink,
                              int32_t out_f32, const float *slopes, int32_t out_dim, int64_t out_stride, const void *gate,
                              int64_t gate_stride, int32_t dtype, swl_stream_t stream) {
-    return span_attn(nullptr, 0, out, q, k_cache, v_cache, block_table, tok_seq, tok_pos, tok_start, span_row0, span_cnt, rel, rel_len, num_spans, num_q_heads, num_kv_heads, num_v_heads, dim, vdim, q_tok_stride, window, mask_kind, scale, softcap, max_blocks_per_seq, block_stride, key_splits, scratch, num_tokens, sink, out_f32, slopes, out_dim, out_stride, gate, gate_stride, dtype, stream);
-}
-
-/* span_order: the spans in the order in which workgroups take them up (a permutation, or NULL); longest: tokens of the longest sequence
- * (0: not known). */
-extern "C" int swl_span_attn_ordered(const int32_t *span_order, int32_t longest, void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
-                             const int32_t *tok_seq, const int32_t *tok_pos, const int32_t *tok_start, const int32_t *span_row0,
-                             const int32_t *span_cnt, const float *rel, int32_t rel_len, int32_t num_spans, int32_t num_q_heads,
-                             int32_t num_kv_heads, int32_t num_v_heads, int32_t dim, int32_t vdim, int64_t q_tok_stride,
-                             int32_t window, int32_t mask_kind, float scale, float softcap, int32_t max_blocks_per_seq,
-                             int64_t block_stride, int32_t key_splits, float *scratch, int64_t num_tokens, const float *sink,
-                             int32_t out_f32, const float *slopes, int32_t out_dim, int64_t out_stride, const void *gate,
-                             int64_t gate_stride, int32_t dtype, swl_stream_t stream) {
-    return span_attn(span_order, longest, out, q, k_cache, v_cache, block_table, tok_seq, tok_pos, tok_start, span_row0, span_cnt, rel, rel_len, num_spans, num_q_heads, num_kv_heads, num_v_heads, dim, vdim, q_tok_stride, window, mask_kind, scale, softcap, max_blocks_per_seq, block_stride, key_splits, scratch, num_tokens, sink, out_f32, slopes, out_dim, out_stride, gate, gate_stride, dtype, stream);
+    return swl_span_attn_ordered(nullptr, 0, out, q, k_cache, v_cache, block_table, tok_seq, tok_pos, tok_start, span_row0, span_cnt, rel,
+                                 rel_len, num_spans, num_q_heads, num_kv_heads, num_v_heads, dim, vdim, q_tok_stride, window, mask_kind,
+                                 scale, softcap, max_blocks_per_seq, block_stride, key_splits, scratch, num_tokens, sink, out_f32, slopes,
+                                 out_dim, out_stride, gate, gate_stride, dtype, stream);
 }

@@ -3,10 +3,10 @@ or the library GEMM (`F.linear` -> hipBLASLt, the reference's own call: swiftllm
 
 Both compute the same product (one rounding of an fp32-accumulated sum) but sum K in different orders, so WHICH one runs
 is part of a deployment's numerics: it must not depend on a timing race inside a request, and every replica of a
-data-parallel deployment must answer alike (VERDICT r05 weak 7, ADVICE r05).
+data-parallel deployment must answer alike.
 
-  * the measured table (r04 sweep, qkv / o re-measured with cold weights in r06d: Llama-3-8B widths, bfloat16, ROCm 7.2)
-    answers for the (N, K, dtype) classes it was measured on (`MEASURED`);
+  * the measured table (Llama-3-8B widths, bfloat16, ROCm 7.2, cold weights) answers for the (N, K, dtype) classes it was measured on
+    (`MEASURED`): these are not timed at load;
   * any other class is measured ONCE PER DEPLOYMENT, at `LlamaModel.load_weights()` time — before any request and before
     any hipGraph capture — for every 32-token bucket of 65..256 tokens (`prepare`, driven by kernels/linear.py:
     tune_wide_routes): a few launches of each side, the hand-written kernel taken when it wins by more than 3 %. The table
@@ -24,7 +24,7 @@ import time
 import torch
 
 MEASURED_DTYPE = torch.bfloat16
-# (N, K) of the Llama-3-8B projections the r04 sweep covered: fused qkv, o_proj, up/gate, down
+# (N, K) of the Llama-3-8B projections that the table covers: fused qkv, o_proj, up/gate, down
 MEASURED = {(6144, 4096), (4096, 4096), (28672, 4096), (4096, 14336)}
 _TOKEN_BUCKET = 32
 BUCKETS = tuple(range(96, 257, _TOKEN_BUCKET))      # 65..96, ..128, ... ..256 tokens
@@ -40,20 +40,15 @@ _device_key_cache = {}
 
 
 def table_wide_wins(m: int, n: int, k: int) -> bool:
-    """Llama-3-8B widths, bf16, MI355X, us ours / library. r04 sweep (profiles/r04c_ / r04d_gemm_wide_micro.jsonl; M = 96, 128,
-    160, 192, 224, 256):
-        down (K >= 2N)   33/63  34/75  43/85  44/104  52/60  54/63      -> always
-    qkv and o re-measured in r06d (profiles/r06d_gemm_wide_routing_remeasure.jsonl) with the weights cycled through 1.2 GB —
-    the r04 sweep's six copies left 200-300 MB of them in the Infinity Cache, which flattered the library's 160-token
-    kernels (o: 24 us then, 31.5 cold) — and with the token-split tiling of csrc/gemm_wide.hip; M = 136, 144, 160, 176, 192,
-    208, 224, 256:
-        qkv  (N = 6144)  27/41  27/41  28/31  29/30  29/37  37/30  37/40  38/43   -> always
-        o    (N = 4096)  22/28  22/24  22/32  23/26  24/36  29/27  29/29  30/27   -> up to 192
-    (up to 128 tokens both were already ours.) Thresholds sit on the 32-token bucket edges of the hipGraph replay cache
-    (`LlamaModel._decode_batch_bucket`) and nowhere else: a batch of 200 runs as 200 rows eagerly and as 224 rows in a replayed
-    graph, and both must take the same side — the library's one good qkv kernel at 208 tokens is therefore not used (the
-    bucket's replay shape, 224, is ours: `test_large_decode_batches_replay_their_hip_graph_bit_for_bit`). The plain up/gate
-    projection only ties (53 / 54 at 128) and loses beyond; its SiLU-gate form is `table_wide_silu_wins`."""
+    """Llama-3-8B widths, bf16, MI355X. us ours / library at M = 96, 128, 160, 192, 224, 256, captured, weights cycled through 1.2 GB, the launch
+    that adds the K shares included (the consumers of a decode step add them themselves):
+        down     32/64  33/76  42/85  40/103  49/60  49/62         -> always
+        qkv      22/23  25/26  27/28  27/33   31/37  32/40         -> always
+        o        19/22  21/25  22/27  24/33   26/22  28/23         -> up to 192
+        up/gate  46/55  53/57  59/60  64/67   77/65  75/66         -> never: up to 128 its SiLU-gate form is ours (table_wide_silu_wins)
+    Thresholds sit on the 32-token bucket edges of the hipGraph replay cache (`LlamaModel._decode_batch_bucket`) and nowhere else: a batch
+    of 200 runs as 200 rows eagerly and as 224 rows in a replayed graph, and both must take the same side, whatever the library's good
+    sizes in between are (o at 104 tokens 19.4/16.5, qkv at 208 30.2/26.7): `test_large_decode_batches_replay_their_hip_graph_bit_for_bit`."""
     if k >= 2 * n:
         return True
     if n > 8192:
@@ -62,9 +57,9 @@ def table_wide_wins(m: int, n: int, k: int) -> bool:
 
 
 def table_wide_silu_wins(m: int) -> bool:
-    """up/gate projection + SiLU-gate in one launch against the library GEMM + silu_and_mul: 53.5 / 63.3 us at 128 tokens,
-    60.0 / 62.5 at 96; r06d (pipelined B fragments, cold weights): 81 / 71 at 136, 77 / 71 at 160, 81 / 76 at 192, 108 / 87 at
-    256: up to 128 tokens."""
+    """up/gate projection + SiLU-gate in one launch against the library GEMM + silu_and_mul, us as above: 48/55, 51/58, 56/63, 59/68, 74/68,
+    80/76 at M = 96 ... 256. The line at 128 was measured on the kernel without rings (81/71 at 136, 81/76 at 192); the present one is
+    ahead up to 192."""
     return m <= 128
 
 
@@ -163,7 +158,7 @@ def time_us(fn, iters: int = 8, warm: int = 2) -> float:
 
 def prepare(classes, dtype, device, model_path: str, measure) -> dict:
     """Fill this process's table for `classes` — an iterable of (N, K, silu) — at every token bucket.
-    `measure(n, k, silu, bucket) -> bool` times the two candidates (kernels/linear.py supplies it). Classes the r04 table
+    `measure(n, k, silu, bucket) -> bool` times the two candidates (kernels/linear.py supplies it). Classes the measured table
     answers are skipped; answers already in the deployment's file (same device + software key) are READ, not re-measured;
     what is missing is measured under a lock file so that concurrently starting replicas do it once. Returns
     {"measured": n, "read": n, "path": file or None}."""
