@@ -33,6 +33,12 @@ __device__ __forceinline__ void row_store(T *p, const float (&v)[4]) {
 template <int TPR, int NV>
 __device__ __forceinline__ void row_load_parts(float (&v)[NV][4], const float *p, int c0, int width, int parts, int64_t stride) {
     constexpr int DEEP = NV <= 2 ? 4 : 2;
+    if (parts == 1) {       // (the last slab stands in for the missing ones below: one slab would be read DEEP times)
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+            if (c0 + 4 * TPR * j < width) row_load<float>(v[j], p + c0 + 4 * TPR * j);
+        return;
+    }
     for (int k = 0; k < parts; k += DEEP) {
         float4_t b[DEEP][NV];
 #pragma unroll

@@ -85,3 +85,10 @@ def test_slabs_of_a_split_product(rows, width, parts, dtype):
         else:       # one rounding of m to its type first
             eps = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
             assert (gpu.double().cpu() - want).abs().max() <= 4 * eps * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,width", [(3, 1028), (32, 2048), (6, 4096), (2, 8192), (1030, 1000), (1030, 1544)])
+def test_one_slab(rows, width, dtype):
+    """A product that was not split, for every number of columns that a thread holds."""
+    test_slabs_of_a_split_product(rows, width, 1, dtype)
