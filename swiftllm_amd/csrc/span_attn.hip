@@ -264,8 +264,8 @@ __global__ __launch_bounds__(kSpanWaves * 64, 2) void span_attn_kernel(SpanParam
     const unsigned v_frag = static_cast<unsigned>(kh * KW * DV * 2 + (lk >> 1) * 16 * DV * 2 + (lr * 2 + (lk & 1)) * 16);
 
     // ---- scores as they are compared and their unit in powers of two: products of queries and keys where nothing is done to them but
-    // the scale, the model's logits otherwise (capped ones in base-2 units already)
-    const bool capped = p.softcap > 0.f, plain = !REL && !capped && !p.slopes && p.scale > 0.f;
+    // the scale, the model's logits otherwise (capped ones in base-2 units already). A scale that leaves kNegBig no mask is applied first.
+    const bool capped = p.softcap > 0.f, plain = !REL && !capped && !p.slopes && p.scale > 1e-20f;
     const float c_mul = capped ? 2.0f * kLog2e * p.scale / p.softcap : p.scale;
     const float unit = plain ? p.scale * kLog2e : capped ? 1.0f : kLog2e;
     const float cap = p.softcap * kLog2e, cap2 = -2.0f * p.softcap * kLog2e, rel_mul = capped ? kLog2e : 1.0f;

@@ -177,6 +177,24 @@ def test_steps_of_many_workgroups(case, shares, dtype, monkeypatch):
     test_span_attention(case, parts, dtype)
 
 
+@pytest.mark.parametrize("scale", [1e-38, 1e-30, 1e-19, -0.05, 0.0])
+def test_scales_of_any_size(scale):
+    """Masked keys weigh nothing whatever the scale: next to none at all, the visible values' mean, and negative ones."""
+    from swiftllm_amd.worker.kernels import window_attn
+    from swiftllm_amd.worker.kernels.window_attn import AttentionSpec
+    parts, g = [(1, 0, 40), (2, 21, 77)], torch.Generator().manual_seed(2)
+    pool, sl, table, ks, vs = _pool([a + n for _, a, n in parts], 2, 2, 64, 64, torch.bfloat16, g)
+    seq, pos, tiles = _spans(parts)
+    q = torch.randn(seq.shape[0], 4 * 64, generator=g).to(torch.bfloat16)
+    spec = AttentionSpec(4, 2, 64, 64, scale, window=50)
+    out = window_attn.masked_attention(q.cuda(), pool, sl, table, seq, pos, spec, tiles)
+    at = 0
+    for k, v, (_, a, n) in zip(ks, vs, parts):
+        want = _want(q[at:at + n].double().view(n, 4, 64), k, v, a, spec, None, None)
+        assert (out[at:at + n].double().cpu() - want).abs().max() <= 1.1 * 2.0 ** -8 * max(1.0, float(want.abs().max()))
+        at += n
+
+
 @pytest.mark.parametrize("H,G,d,dv,window", [(8, 2, 128, 128, 0), (4, 4, 64, 64, 100), (6, 2, 192, 128, 0), (8, 1, 576, 512, 300),
                                              (2, 1, 320, 256, 0), (3, 1, 64, 128, 0)])
 def test_spans_in_any_order(H, G, d, dv, window):
