@@ -202,9 +202,10 @@ class StepPlan:
         key = first.astype(np.int64) * self.num_seqs + portion
         return (n - 1 - np.argsort(-key[::-1], kind="stable")).astype(np.int32)
 
-    # Steps of up to so many spans go without: the order takes 10 us of the host, with the device idle, and gives a launch at most 3 us there
-    # (8 or 4 heads of 128 over 2 or 4, 66 to 128 spans; 16 heads over 4 up to 7, 8 latent heads over one none), against 1 to 22 us at 220 and
-    # more. A step of 2030 tokens (94 spans, three such launches) 1322 -> 1315 us without it, one of 3663 (121) 3010 -> 2995.
+    # Steps of up to so many spans go without: making and packing the order takes a step 25 us of the host (10 in a loop of nothing else), with
+    # the device idle, and it gives a launch at most 3 us there (8 or 4 heads of 128 over 2 or 4, 66 to 128 spans; 16 heads over 4 up to 7, 8
+    # latent heads over one none), against 1 to 22 us at 220 and more. A step of 2030 tokens (94 spans, three such launches) 1322 -> 1315 us
+    # without it, one of 3663 (121) 3010 -> 2995.
     ORDER_MIN_SPANS = 128
 
     def upload_order(self):
