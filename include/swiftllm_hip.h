@@ -665,6 +665,12 @@ int swl_mix_sigmoid_attn(void *out, const void *q, const void *k_cache, const vo
  *   again, transposed, as one value head of kv_rank. half = 0: interleaved pairs, 1: dimension i turns with i + rot_dim / 2;
  *   cosines and sines are multiplied by rot_mult. Query heads and key rows are k_dim (>= kv_rank + rot_dim) elements wide in qa
  *   and in the pool, value rows v_dim (>= kv_rank): the columns beyond are zeroed.
+ * swl_latent_rope_store_kv_rows: the same where the query heads of the first `in_place` rows are rotated where they are, in proj
+ *   (their unrotated parts stay), and the rotated parts of row in_place + i go to row i of qa (which may be NULL for none).
+ * swl_latent_expand: pages of the latent key cache expanded to the keys and values of every head. Page i of the call is page page_no[i]
+ *   of block-table row page_row[i] and goes to out + page_dst[i] pages of num_heads * 16 * (dim + rot_dim + vdim) elements: keys
+ *   [heads, 16, dim + rot_dim] = (uk[h] c | rotated part), uk [heads, dim, kv_rank], then values [heads, vdim, 16] = uv[h] c, uv [heads, vdim,
+ *   kv_rank]; products are rounded once. k_dim: elements of a cached row (kv_rank | rot_dim first). Ask swl_latent_expand_supported.
  * swl_diff_head_combine: maps fp32 [T, 2, H, vdim] -> out[T, H, vdim] = unit_rms(a1 - lambda a2; eps) * mult *
  *   sigmoid(gate[t * gate_stride + h]) (gate NULL: no gate).
  * swl_head_gate: y[T, H, vdim] *= sigmoid(gate[t * gate_stride + h]) in place. */
@@ -679,6 +685,17 @@ int swl_latent_rope_store_kv(const void *proj, void *qa, const double *freq, con
                              int64_t proj_stride, int64_t dkv_col, int64_t qa_stride, int32_t max_blocks_per_seq,
                              int64_t block_stride, float eps, int32_t half, double rot_mult, int32_t k_dim, int32_t v_dim,
                              int32_t dtype, swl_stream_t stream);
+int swl_latent_rope_store_kv_rows(void *proj, void *qa, int64_t in_place, const double *freq, const float *c_norm, void *k_cache,
+                                  void *v_cache, const int32_t *block_table, const int32_t *tok_seq, const int32_t *tok_pos,
+                                  int64_t num_tokens, int32_t num_heads, int32_t dim, int32_t rot_dim, int32_t kv_rank,
+                                  int64_t proj_stride, int64_t dkv_col, int64_t qa_stride, int32_t max_blocks_per_seq,
+                                  int64_t block_stride, float eps, int32_t half, double rot_mult, int32_t k_dim, int32_t v_dim,
+                                  int32_t dtype, swl_stream_t stream);
+int swl_latent_expand_supported(int32_t dim, int32_t vdim, int32_t rot_dim, int32_t kv_rank, int32_t k_dim, int32_t dtype);
+int swl_latent_expand(void *out, const void *k_cache, const void *uk, const void *uv, const int32_t *block_table,
+                      const int32_t *page_row, const int32_t *page_no, const int32_t *page_dst, int64_t num_pages,
+                      int32_t num_heads, int32_t dim, int32_t vdim, int32_t rot_dim, int32_t kv_rank, int32_t k_dim,
+                      int32_t max_blocks_per_seq, int64_t block_stride, int32_t dtype, swl_stream_t stream);
 int swl_diff_head_combine(void *out, const float *maps, const void *gate, int64_t gate_stride, float lambda, float mult,
                           float eps, int64_t num_tokens, int32_t num_heads, int32_t vdim, int32_t dtype,
                           swl_stream_t stream);

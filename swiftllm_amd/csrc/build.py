@@ -51,6 +51,7 @@ SOURCES = [
     "mix_attn.hip",
     "delta_chunks.hip",
     "gemm_f32.hip",
+    "latent_expand.hip",
 ]
 # What a model family's worker calls (the shared pieces included): `build(only=MODEL_SOURCES[...])` compiles just these, so
 # that the first use from a fresh checkout does not pay for kernels the model never launches. A later full build compiles
@@ -63,14 +64,14 @@ MODEL_SOURCES = {
     "Lorulix": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip",
                           "rms_stream.hip", "delta_rule.hip", "delta_chunks.hip"],
     "Rosilix": _SHARED + ["layernorm.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rms_stream.hip",
-                          "rope_kv.hip"],
+                          "rope_kv.hip", "latent_expand.hip"],
     "Ratilorn": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip",
                            "rms_stream.hip", "sigmoid_attn.hip", "mix_attn.hip", "ssd.hip", "linear_scan.hip", "delta_rule.hip"],
-    "Rokevik": _SHARED + ["window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rope_kv.hip", "hyper_stream.hip", "min_gru.hip"],
+    "Rokevik": _SHARED + ["window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rope_kv.hip", "hyper_stream.hip", "min_gru.hip", "latent_expand.hip"],
     "Vafozen": _SHARED + ["layernorm.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rms_stream.hip", "rope_kv.hip",
                           "hyper_stream.hip", "delta_rule.hip", "ssd.hip", "linear_scan.hip", "low_rank_decay.hip"],
 }
-HEADERS = ["swl_common.h", "attend_block.h", "attn_combine.h", "token_attn.h", "conv_tail.h", "row_wide.h", os.path.join(ROOT, "include", "swiftllm_hip.h")]
+HEADERS = ["swl_common.h", "attend_block.h", "attn_combine.h", "token_attn.h", "conv_tail.h", "row_wide.h", "tile_product.h", os.path.join(ROOT, "include", "swiftllm_hip.h")]
 LIB = os.path.join(HERE, "libswiftllm_hip.so")
 OBJ_DIR = os.path.join(HERE, "build")
 ARCH = "gfx950"

@@ -13,18 +13,11 @@
 // unit 223 -> 159 us (950 TFLOP/s), down 101 -> 85; 16000 assignments, width and ff 1024: 98 -> 82, 54 -> 45; 1562, width and ff 2048:
 // 61 -> 37, 30 -> 26. Tiles of 256 x 256 or 128 x 256 with rings of up to five slices: 225 and 172 us at the first size (the chip's last
 // turn is half empty, and first slices and results wait alone), 150 and 100 at the second; faster only where the tiles fill whole turns.
-#include "swl_common.h"
+#include "tile_product.h"
 
 namespace swl {
 
-constexpr int kMgTile = 128, kMgDepth = 64, kSortThreads = 1024;
-
-__device__ __forceinline__ float16_t mg_mfma(vec8_t<f16> a, vec8_t<f16> b, float16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ float16_t mg_mfma(vec8_t<bf16> a, vec8_t<bf16> b, float16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
+constexpr int kSortThreads = 1024;
 
 // One workgroup per expert: how many assignments go to lower experts, then a stable list of its own. Bound by latency: a thread asks for its
 // I consecutive ids at once (16 bytes a load) and counts, scans and places from registers, one barrier for 1024 I assignments.
@@ -129,7 +122,7 @@ __device__ __forceinline__ MgTile mg_tile(const MoeGemmParams &p) {
         const int e = min(e0 + lane, p.experts - 1);
         a = p.offsets[e];
         b = e0 + lane < p.experts ? p.offsets[e + 1] : a;
-        int scan = (b - a + kMgTile - 1) / kMgTile;
+        int scan = (b - a + kTile - 1) / kTile;
         for (int o = 1; o < 64; o <<= 1) {
             const int v = __shfl_up(scan, o, 64);
             if (lane >= o) scan += v;
@@ -157,8 +150,8 @@ __device__ __forceinline__ MgTile mg_tile(const MoeGemmParams &p) {
             const int l = __builtin_ctzll(past);
             const int lo = __builtin_amdgcn_readlane(a, l), hi = __builtin_amdgcn_readlane(b, l);
             t.expert = e0 + l;
-            t.row0 = lo + (m_tile - __builtin_amdgcn_readlane(scan, l) + (hi - lo + kMgTile - 1) / kMgTile) * kMgTile;
-            t.rows = min(kMgTile, hi - t.row0);
+            t.row0 = lo + (m_tile - __builtin_amdgcn_readlane(scan, l) + (hi - lo + kTile - 1) / kTile) * kTile;
+            t.rows = min(kTile, hi - t.row0);
             break;
         }
         m_tile -= __builtin_amdgcn_readlane(scan, 63);
@@ -171,9 +164,8 @@ __device__ __forceinline__ MgTile mg_tile(const MoeGemmParams &p) {
 // each other's waits, first and last slices too.
 template <typename T, int MODE, int BUFS>
 __global__ __launch_bounds__(256, BUFS == 1 ? 4 : 2) void moe_gemm_kernel(MoeGemmParams p) {
-    constexpr int TILEB = kMgTile * kMgDepth * 2;       // bytes of a staged operand slice
     constexpr int OUTC = MODE == 1 ? 64 : 128, PITCH = OUTC + 8;          // output columns of a tile, elements between its rows in LDS
-    constexpr int STAGED = BUFS * 2 * TILEB, RESULT = kMgTile * PITCH * 2;
+    constexpr int STAGED = BUFS * 2 * kTileSliceB, RESULT = kTile * PITCH * 2;
     __shared__ __attribute__((aligned(16))) char smem[STAGED > RESULT ? STAGED : RESULT];      // [buffer][weights, tokens]; then the output tile
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hf = lane >> 5, wn = wave & 1, wm = wave >> 1;
@@ -181,13 +173,13 @@ __global__ __launch_bounds__(256, BUFS == 1 ? 4 : 2) void moe_gemm_kernel(MoeGem
     if (t.expert < 0) return;
     const int row0 = t.row0, rows = t.rows, n_tile = t.n_tile;
 
-    // ---- staging: wave w loads rows 32 w .. 32 w + 31 of both operands, 8 rows of 128 bytes an instruction --------------------------
+    // ---- staging --------------------------------------------------------------------------------------------------------------------
     const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem));
     unsigned w_off[4], x_off[4];
     const int64_t kb = static_cast<int64_t>(p.K) * 2;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int r = wave * 32 + i * 8 + (lane >> 3), unit = (lane & 7) ^ ((r >> 1) & 7);
+        const int r = tile_row(wave, i, lane), unit = tile_unit(r, lane);
         int wr;
         if (MODE == 1) {        // a wave's 64 weight rows: 32 gate rows, then the up rows of the same columns
             const int c = min(n_tile * 64 + (r >> 6) * 32 + (r & 31), p.N - 1);
@@ -202,96 +194,17 @@ __global__ __launch_bounds__(256, BUFS == 1 ? 4 : 2) void moe_gemm_kernel(MoeGem
     }
     const char *wb = static_cast<const char *>(p.w) + static_cast<int64_t>(t.expert) * (MODE == 1 ? 2 : 1) * p.N * kb;
     const char *xb = static_cast<const char *>(p.x);
-    auto issue = [&](int st) {
-        const char *ws = wb + static_cast<int64_t>(st) * kMgDepth * 2, *xs = xb + static_cast<int64_t>(st) * kMgDepth * 2;
-        const unsigned to = lds0 + static_cast<unsigned>((st & (BUFS - 1)) * 2 * TILEB + wave * 4096);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            unsigned keep;
-            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                         : "=&s"(keep) : "v"(w_off[i]), "s"(ws), "s"(to + i * 1024) : "memory");
-            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                         : "=&s"(keep) : "v"(x_off[i]), "s"(xs), "s"(to + TILEB + i * 1024) : "memory");
-        }
-    };
-    // fragments: row l32 of a 32-row piece, 16-byte unit 2 e + hf (swizzled as staged; rows 32 apart share the swizzle)
-    unsigned frag[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) frag[e] = static_cast<unsigned>(l32 * 128 + (((2 * e + hf) ^ ((l32 >> 1) & 7)) * 16));
     float16_t acc[2][2];        // [weight piece][token piece]
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = float16_t{};
-    vec8_t<T> wf[2][2], xf[2][2];       // [set][piece]: the fragments of 16 columns are requested in front of the products of the 16 before
-    auto read = [&](int st, int e, int set) {
-        const char *ws = smem + (st & (BUFS - 1)) * 2 * TILEB + wn * 64 * 128, *xs = smem + (st & (BUFS - 1)) * 2 * TILEB + TILEB + wm * 64 * 128;
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            wf[set][a] = *reinterpret_cast<const vec8_t<T> *>(ws + a * 32 * 128 + frag[e]);
-            xf[set][a] = *reinterpret_cast<const vec8_t<T> *>(xs + a * 32 * 128 + frag[e]);
-        }
-    };
-    auto multiply = [&](int set) {
-#pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc[a][b] = mg_mfma(wf[set][a], xf[set][b], acc[a][b]);
-    };
-    auto step = [&](int st, int e, int set) {       // products of a set, the reads of the next spread between them
-        __builtin_amdgcn_sched_barrier(0);
-        read(st, e, set ^ 1);
-        multiply(set);
+    tile_product<T, BUFS, false>(smem, p.K / kTileDepth, wn, wm, lane, acc, [&](int st) {
+        const char *ws = wb + static_cast<int64_t>(st) * kTileDepth * 2, *xs = xb + static_cast<int64_t>(st) * kTileDepth * 2;
+        const unsigned to = lds0 + static_cast<unsigned>((st & (BUFS - 1)) * 2 * kTileSliceB + wave * 4096);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            tile_ask(ws, w_off[i], to + i * 1024);
+            tile_ask(xs, x_off[i], to + kTileSliceB + i * 1024);
         }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    const int stages = p.K / kMgDepth;
-    issue(0);
-    if constexpr (BUFS == 1) {
-        for (int st = 0;; ++st) {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // this wave's pieces of the slice have landed; then everyone's
-            __builtin_amdgcn_s_barrier();
-            read(st, 0, 0);
-            step(st, 1, 0);
-            step(st, 2, 1);
-            step(st, 3, 0);
-            multiply(1);        // (its operands were the last reads of the slice: all of them have returned; then everyone's)
-            if (st + 1 == stages) break;
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            issue(st + 1);
-        }
-    } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        if (stages > 1) issue(1);
-        read(0, 0, 0);
-        for (int st = 0; st + 1 < stages; ++st) {
-            step(st, 1, 0);
-            step(st, 2, 1);
-            step(st, 3, 0);
-            // this wave's pieces of the next slice have landed, its reads of this one have returned; then everyone's
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            if (st + 2 < stages) issue(st + 2);
-            step(st + 1, 0, 1);
-        }
-        step(stages - 1, 1, 0);
-        step(stages - 1, 2, 1);
-        step(stages - 1, 3, 0);
-        multiply(1);
-    }
+    });
     // ---- epilogue: acc[a][b][4 q + r] = product (weight row 64 wn + 32 a + 8 q + 4 hf + r, token 64 wm + 32 b + l32) ----------------
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-            if (a + b < 2) mfma_results_tie(acc[a][b]);
-    mfma_results_ready<8>(acc[1][1]);
     __syncthreads();        // every wave is done with the staged slices
     T *tile = reinterpret_cast<T *>(smem);
 #pragma unroll
@@ -328,7 +241,7 @@ __global__ __launch_bounds__(256, BUFS == 1 ? 4 : 2) void moe_gemm_kernel(MoeGem
     __syncthreads();
     T *out = static_cast<T *>(p.out);
     constexpr int CPR = OUTC / 8;       // 16-byte pieces of a row
-    for (int i = tid; i < kMgTile * CPR; i += 256) {
+    for (int i = tid; i < kTile * CPR; i += 256) {
         const int r = i / CPR, c = (i - r * CPR) * 8;
         if (r < rows && n_tile * OUTC + c < p.N)
             store8(out + static_cast<int64_t>(row0 + r) * p.N + n_tile * OUTC + c, *reinterpret_cast<const vec8_t<T> *>(tile + r * PITCH + c));
@@ -352,7 +265,7 @@ extern "C" int swl_moe_sort(int32_t *order, int64_t *where, int32_t *offsets, co
  * operand rows within 4 GiB of their matrix's start. */
 extern "C" int swl_moe_gemm_supported(int64_t x_rows, int32_t K, int32_t N, int32_t dtype) {
     if (dtype != SWL_F16 && dtype != SWL_BF16) return 0;
-    if (x_rows <= 0 || K <= 0 || N <= 0 || K % swl::kMgDepth || N % 8) return 0;
+    if (x_rows <= 0 || K <= 0 || N <= 0 || K % swl::kTileDepth || N % 8) return 0;
     const int64_t row = static_cast<int64_t>(K) * 2;
     return x_rows * row < (1LL << 32) && 2LL * N * row < (1LL << 32);
 }
@@ -373,13 +286,13 @@ extern "C" int swl_moe_gemm(void *out, const void *x, const void *w, const int32
     const int cols = mode == 1 ? 64 : 128;
     p.n_tiles = (N + cols - 1) / cols;
     // as many row tiles as there can be (every expert may end in a part of one); surplus workgroups leave at once
-    const int64_t m_tiles = (num_assignments + swl::kMgTile - 1) / swl::kMgTile + (experts < num_assignments ? experts : num_assignments);
+    const int64_t m_tiles = (num_assignments + swl::kTile - 1) / swl::kTile + (experts < num_assignments ? experts : num_assignments);
     const int64_t grid = (m_tiles * p.n_tiles + 7) / 8 * 8;
     if (grid > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
     hipStream_t s = static_cast<hipStream_t>(stream);
     // One staged slice and four workgroups a CU where there are more tiles than two a CU (about: an expert's last row tile half full),
     // else two slices: 31.3 and 35.7 us at 688 tiles (4950 rows, width and ff 1024, gate/up), 39.1 and 36.6 at 512, 20.7 and 19.3 at 344.
-    const bool many = (num_assignments + 64LL * experts) / swl::kMgTile * p.n_tiles > 512;
+    const bool many = (num_assignments + 64LL * experts) / swl::kTile * p.n_tiles > 512;
 #define SWL_MG(MODE, BUFS) hipLaunchKernelGGL((swl::moe_gemm_kernel<T, MODE, BUFS>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, s, p)
 #define SWL_MG2(MODE) do { if (many) SWL_MG(MODE, 1); else SWL_MG(MODE, 2); } while (0)
     SWL_DISPATCH_DTYPE(dtype, T, {

@@ -391,7 +391,7 @@ __global__ __launch_bounds__(kRkThreads) void qkv_conv_rope_store_kv_kernel(
 
 template <typename T>
 __global__ __launch_bounds__(kRkThreads) void latent_rope_store_kv_kernel(
-    const T *proj, T *qa, const double *freq, const float *c_w, T *k_cache, T *v_cache, const int32_t *block_table,
+    T *proj, T *qa, int64_t in_place, const double *freq, const float *c_w, T *k_cache, T *v_cache, const int32_t *block_table,
     const int32_t *tok_seq, const int32_t *tok_pos, int H, int d, int dr, int r, int64_t proj_stride, int64_t dkv_col,
     int64_t qa_stride, int max_blocks_per_seq, int64_t block_stride, float eps, int half, double rot_mult, int k_dim,
     int v_dim) {
@@ -402,22 +402,24 @@ __global__ __launch_bounds__(kRkThreads) void latent_rope_store_kv_kernel(
     const int pairs = dr >> 1;
     rk_angles(cs, sn, freq, pos, pairs, rot_mult);
     __syncthreads();
-    const T *row = proj + t * proj_stride;
-    T *qrow = qa + t * qa_stride;
+    T *row = proj + t * proj_stride;
+    const bool here = t < in_place;     // (the query heads stay where they are)
+    T *qrow = here ? row + d : qa + (t - in_place) * qa_stride + r;
+    const int qhead = here ? d + dr : k_dim;
     // pair j of a rotated part: elements (2j, 2j + 1), or (j, j + pairs)
     const int step = half ? 1 : 2, gap = half ? pairs : 1;
     for (int i = threadIdx.x; i < H * pairs; i += kRkThreads) {
         const int h = i / pairs, j = i - h * pairs;
         const T *p = row + static_cast<int64_t>(h) * (d + dr) + d + step * j;
-        T *o = qrow + static_cast<int64_t>(h) * k_dim + r + step * j;
+        T *o = qrow + static_cast<int64_t>(h) * qhead + step * j;
         const float u = to_f(p[0]), v = to_f(p[gap]);
         o[0] = to_t<T>(u * cs[j] - v * sn[j]);
         o[gap] = to_t<T>(v * cs[j] + u * sn[j]);
     }
     const int kpad = k_dim - r - dr, vpad = v_dim - r;
-    for (int i = threadIdx.x; i < H * kpad; i += kRkThreads) {
+    for (int i = threadIdx.x; i < (here ? 0 : H * kpad); i += kRkThreads) {
         const int h = i / kpad;
-        qrow[static_cast<int64_t>(h) * k_dim + r + dr + i - h * kpad] = to_t<T>(0.f);
+        qrow[static_cast<int64_t>(h) * k_dim + dr + i - h * kpad] = to_t<T>(0.f);
     }
     if (dkv_col < 0 || k_cache == nullptr) return;
     const T *z = row + dkv_col;
@@ -572,6 +574,34 @@ extern "C" int swl_qkv_conv_rope_store_kv(
     return swl::check_launch();
 }
 
+extern "C" int swl_latent_rope_store_kv_rows(void *proj, void *qa, int64_t in_place, const double *freq, const float *c_norm,
+                                        void *k_cache, void *v_cache, const int32_t *block_table, const int32_t *tok_seq,
+                                        const int32_t *tok_pos, int64_t num_tokens, int32_t num_heads, int32_t dim,
+                                        int32_t rot_dim, int32_t kv_rank, int64_t proj_stride, int64_t dkv_col,
+                                        int64_t qa_stride, int32_t max_blocks_per_seq, int64_t block_stride, float eps,
+                                        int32_t half, double rot_mult, int32_t k_dim, int32_t v_dim, int32_t dtype,
+                                        swl_stream_t stream) {
+    if (in_place < 0) return SWL_ERR_BAD_ARG;
+    if (num_tokens < 0 || num_heads <= 0 || dim <= 0 || rot_dim <= 0 || (rot_dim & 1) || kv_rank <= 0) return SWL_ERR_BAD_ARG;
+    if (k_dim < kv_rank + rot_dim || v_dim < kv_rank) return SWL_ERR_BAD_ARG;
+    if (proj_stride < static_cast<int64_t>(num_heads) * (dim + rot_dim) || qa_stride < static_cast<int64_t>(num_heads) * k_dim)
+        return SWL_ERR_BAD_ARG;
+    if (dkv_col >= 0 && dkv_col + kv_rank + rot_dim > proj_stride) return SWL_ERR_BAD_ARG;
+    if (num_tokens == 0) return SWL_OK;
+    if (!proj || (!qa && in_place < num_tokens) || !freq || !tok_pos) return SWL_ERR_BAD_ARG;
+    if (dkv_col >= 0 && k_cache && (!v_cache || !c_norm || !block_table || !tok_seq || max_blocks_per_seq <= 0))
+        return SWL_ERR_BAD_ARG;
+    if (num_tokens > 0x7fffffffLL || rot_dim > 2 * swl::kRkMaxPairs) return SWL_ERR_UNSUPPORTED;
+    SWL_DISPATCH_DTYPE3(dtype, T, {
+        hipLaunchKernelGGL((swl::latent_rope_store_kv_kernel<T>), dim3(static_cast<unsigned>(num_tokens)),
+                           dim3(swl::kRkThreads), 0, static_cast<hipStream_t>(stream), static_cast<T *>(proj),
+                           static_cast<T *>(qa), in_place, freq, c_norm, static_cast<T *>(k_cache), static_cast<T *>(v_cache),
+                           block_table, tok_seq, tok_pos, num_heads, dim, rot_dim, kv_rank, proj_stride, dkv_col, qa_stride,
+                           max_blocks_per_seq, block_stride, eps, half, rot_mult, k_dim, v_dim);
+    });
+    return swl::check_launch();
+}
+
 extern "C" int swl_latent_rope_store_kv(const void *proj, void *qa, const double *freq, const float *c_norm, void *k_cache,
                                         void *v_cache, const int32_t *block_table, const int32_t *tok_seq,
                                         const int32_t *tok_pos, int64_t num_tokens, int32_t num_heads, int32_t dim,
@@ -579,24 +609,9 @@ extern "C" int swl_latent_rope_store_kv(const void *proj, void *qa, const double
                                         int64_t qa_stride, int32_t max_blocks_per_seq, int64_t block_stride, float eps,
                                         int32_t half, double rot_mult, int32_t k_dim, int32_t v_dim, int32_t dtype,
                                         swl_stream_t stream) {
-    if (num_tokens < 0 || num_heads <= 0 || dim <= 0 || rot_dim <= 0 || (rot_dim & 1) || kv_rank <= 0) return SWL_ERR_BAD_ARG;
-    if (k_dim < kv_rank + rot_dim || v_dim < kv_rank) return SWL_ERR_BAD_ARG;
-    if (proj_stride < static_cast<int64_t>(num_heads) * (dim + rot_dim) || qa_stride < static_cast<int64_t>(num_heads) * k_dim)
-        return SWL_ERR_BAD_ARG;
-    if (dkv_col >= 0 && dkv_col + kv_rank + rot_dim > proj_stride) return SWL_ERR_BAD_ARG;
-    if (num_tokens == 0) return SWL_OK;
-    if (!proj || !qa || !freq || !tok_pos) return SWL_ERR_BAD_ARG;
-    if (dkv_col >= 0 && k_cache && (!v_cache || !c_norm || !block_table || !tok_seq || max_blocks_per_seq <= 0))
-        return SWL_ERR_BAD_ARG;
-    if (num_tokens > 0x7fffffffLL || rot_dim > 2 * swl::kRkMaxPairs) return SWL_ERR_UNSUPPORTED;
-    SWL_DISPATCH_DTYPE3(dtype, T, {
-        hipLaunchKernelGGL((swl::latent_rope_store_kv_kernel<T>), dim3(static_cast<unsigned>(num_tokens)),
-                           dim3(swl::kRkThreads), 0, static_cast<hipStream_t>(stream), static_cast<const T *>(proj),
-                           static_cast<T *>(qa), freq, c_norm, static_cast<T *>(k_cache), static_cast<T *>(v_cache),
-                           block_table, tok_seq, tok_pos, num_heads, dim, rot_dim, kv_rank, proj_stride, dkv_col, qa_stride,
-                           max_blocks_per_seq, block_stride, eps, half, rot_mult, k_dim, v_dim);
-    });
-    return swl::check_launch();
+    return swl_latent_rope_store_kv_rows(const_cast<void *>(proj), qa, 0, freq, c_norm, k_cache, v_cache, block_table, tok_seq, tok_pos,
+                                         num_tokens, num_heads, dim, rot_dim, kv_rank, proj_stride, dkv_col, qa_stride,
+                                         max_blocks_per_seq, block_stride, eps, half, rot_mult, k_dim, v_dim, dtype, stream);
 }
 
 extern "C" int swl_diff_head_combine(void *out, const float *maps, const void *gate, int64_t gate_stride, float lambda,

@@ -490,12 +490,13 @@ int launch_span(SpanParams &p, int key_splits, hipStream_t s) {
 // stage. us by workgroups of 64 rows, 128 + 128 columns, two / one: 11 x 333 tokens, 458: 16.8 / 18.4; 3 x 1500, 562: 39 / 54; 32 x 100, 800: 21.5 /
 // 15.3; 22 x 333, 916: 28.8 / 23.0; 8 x 920, 920: 44 / 41; 5 x 1472, 920: 54 / 53; 4 x 1841, 920: 73 / 73, with a bias 72 / 79; 3 x 2450, 924:
 // 79 / 82; 7200, 900: 193 / 221; 4 x 1841, 1840: 120 / 115. The longest walk may be a decoded token's: 22 x 333 beside one at 2000 keys 43.6 / 66.9,
-// beside one at 8000 141 / 240 (972).
+// beside one at 8000 141 / 240 (972). Rows of 192 + 128, a key head for each query head: two are never the slower ones (expansion and rotary of
+// latent rows included, 16 heads: 4 x 2000 tokens 350 / 474, 40 x 100 98 / 110, 11 x 333 81 / 79).
 template <typename T, int D, int DV>
 int launch_span_any(SpanParams &p, int key_splits, int longest, hipStream_t s) {
     if constexpr (span_halves(D, DV) == 2) {
         const int64_t workgroups = static_cast<int64_t>(p.num_spans) * p.G * kSpan / span_queries(p.H / p.G, 64);
-        if (workgroups <= 640 || (workgroups <= 1024 && longest >= 1536)) return launch_span<T, D, DV, 2>(p, key_splits, s);
+        if (D + DV > 256 || workgroups <= 640 || (workgroups <= 1024 && longest >= 1536)) return launch_span<T, D, DV, 2>(p, key_splits, s);
     }
     return launch_span<T, D, DV, 1>(p, key_splits, s);
 }

@@ -157,6 +157,40 @@ class StepEntry:
     want: Sequence[int] = ()
 
 
+class LatentExpansion:
+    """What decides whether the latent attention of a portion runs on the heads' own keys and values, expanded from the cached rows
+    (csrc/latent_expand.hip), or on queries folded through the key up-projection: the matrix steps of both, by the sizes of the layers.
+    window: of the layers' the largest, 0 if one sees every key; max_pages: pages that the expansion may take."""
+    MIN_TOKENS = 16
+
+    def __init__(self, dim: int, rot_dim: int, vdim: int, rank: int, window: int, max_pages: int):
+        self.window, self.max_pages = window, max_pages
+        # columns a visible (query, key) pair costs more when folded (values count twice), and what expanding one more key costs
+        self.pair_gain = (3 * rank + rot_dim) - (dim + rot_dim + 2 * vdim)
+        self.key_cost = (dim + vdim) * rank
+
+    def pays(self, start: np.ndarray, count: np.ndarray) -> np.ndarray:
+        """By portion: its own keys take as long to expand as its queries to fold; keys before it are extra. A column of the expansion takes
+        half as long as one of attention. Measured, us from the projection to the heads' results, 8 heads of 128 + 64 over rank 512 in a window
+        of 1024, folded and expanded: 16 tokens 34.9, 21.4; 11 x 333 94.7, 57.0; 4 x 2000 276, 165; 64 behind 1000 50.2, 33.1; 8 x 64 behind
+        1000 67.6, 66.2; 8 x 128 98.5, 69.4. 16 heads, no window: 4 x 2000 566, 350; 8 x 64 behind 1000 97.8, 88.6; 8 x 128 behind 3000 277, 269."""
+        before, seen = start, count * (2 * start + count + 1) // 2      # (seen: pairs)
+        if self.window > 0:
+            before, seen = np.minimum(start, self.window - 1), np.minimum(seen, count * self.window)
+        return (count >= self.MIN_TOKENS) & (2 * seen * self.pair_gain > before * self.key_cost)
+
+
+class ExpandedPortions:
+    """The first `seqs` portions of a step (`rows` tokens, `chunks` chunks, `tiles` tiles) on `pages` expanded pages. arrays: int32, for the
+    device: the pages to expand (block-table row, page, its number), ex_tok_row: what ex_table's entry of a token's page is the page's
+    number less (attention finds page i of a portion at ex_table[ex_tok_row + i]), ex_order: the order of the portions' spans, and the
+    first rows of the other portions' chunks and tiles counted from theirs."""
+    __slots__ = ("seqs", "rows", "chunks", "tiles", "pages", "arrays")
+
+    def __init__(self, seqs, rows, chunks, tiles, pages, arrays):
+        self.seqs, self.rows, self.chunks, self.tiles, self.pages, self.arrays = seqs, rows, chunks, tiles, pages, arrays
+
+
 @dataclasses.dataclass
 class StepPlan:
     """Flat per-token metadata of a step. Kernels that serve portions and decoded tokens alike need nothing else: a token's
@@ -212,6 +246,39 @@ class StepPlan:
         """span_order where it pays, or None."""
         return self.span_order() if self.chunk_row0.size > self.ORDER_MIN_SPANS else None
 
+    def latent_expansion(self, spec: "LatentExpansion"):
+        """The portions at the head of the step whose latent attention runs on expanded pages (spec.pays says which gain by it): ->
+        ExpandedPortions, or None where there is none."""
+        count = np.asarray(self.seq_cnt, dtype=np.int64)
+        if count.size == 0 or count[0] < LatentExpansion.MIN_TOKENS:
+            return None
+        start = self.tok_pos[self.seq_row0].astype(np.int64)
+        first = np.maximum(start - spec.window + 1, 0) // 16 if spec.window > 0 else np.zeros_like(start)    # first page with a visible key
+        pages = -(-(start + count) // 16)
+        # a portion's pages are numbered from `at` on, those before the first visible one too: `at` tells portions apart
+        at = np.cumsum(pages) - pages
+        ok = spec.pays(start, count) & (at + pages <= spec.max_pages)
+        k = ok.size if ok.all() else int(np.argmin(ok))
+        if k == 0:
+            return None
+        rest = k < ok.size
+        row0, chunk0, tile0 = ((int(self.seq_row0[k]), int(self.seq_chunk0[k]), int(self.seq_tile0[k])) if rest else
+                               (self.num_tokens, self.chunk_row0.size, self.tile_row0.size))
+        first, pages, at, count = first[:k], pages[:k], at[:k], count[:k]
+        each = pages - first
+        page_no = np.arange(int(each.sum())) - np.repeat(np.cumsum(each) - each - first, each)
+        i32, numbers = np.int32, int(at[-1] + pages[-1])
+        arrays = {"ex_page_row": np.repeat(self.tok_seq[self.seq_row0[:k]], each), "ex_page_no": page_no.astype(i32),
+                  "ex_page_dst": (page_no + np.repeat(at, each)).astype(i32), "ex_tok_row": np.repeat(at, count).astype(i32),
+                  "ex_table": np.arange(numbers, dtype=i32)}
+        order = self.upload_order()
+        if order is not None:
+            arrays["ex_order"] = order[order < chunk0]
+        if rest:
+            arrays["ex_rest_chunk_row0"] = self.chunk_row0[chunk0:] - i32(row0)
+            arrays["ex_rest_tile_row0"] = self.tile_row0[tile0:] - i32(row0)
+        return ExpandedPortions(k, row0, chunk0, tile0, numbers, arrays)
+
     def packed_layout(self):
         out, off = [], 0
         for name in self.SEGMENTS:
@@ -220,8 +287,8 @@ class StepPlan:
             off += (n + 3) // 4 * 4
         return out, off
 
-    def pack_into(self, buf: np.ndarray, packed_layout=None) -> int:
-        layout, total = self.packed_layout() if packed_layout is None else packed_layout
+    def pack_into(self, buf: np.ndarray) -> int:
+        layout, total = self.packed_layout()
         for name, off, n in layout:
             buf[off:off + n] = getattr(self, name)
         return total

@@ -1,0 +1,109 @@
+"""Latent attention of a step: which rows run on the heads' own keys and values, expanded from the cached rows
+(csrc/latent_expand.hip), and which on queries folded through the key up-projection."""
+import torch
+
+from swiftllm_amd import _hip
+
+from ..batch_plan import LatentExpansion
+from .rope_kv import latent_rope_and_store_kv
+from .window_attn import MASK_WINDOW, AttentionSpec, PoolSlice, StepTiles, masked_attention
+
+# A layer's expanded pages take at most this much (which memory profiling sets aside: its step runs without a pool); portions past it stay
+# folded. 8192 tokens of 16 heads of 128 + 64 and 128 columns take 80 MiB.
+EXPAND_MAX_SCRATCH = 256 << 20
+
+
+class ExpandedStep:
+    """The device's side of a step's ExpandedPortions: `rows` leading rows on expanded pages, the rest folded."""
+    __slots__ = ("rows", "pages", "page_row", "page_no", "page_dst", "tok_row", "table", "tiles", "rest")
+
+    @classmethod
+    def of(cls, dev):
+        """From a step's views; None where every row stays folded."""
+        ex = dev.get("expanded")
+        if ex is None:
+            return None
+        self = cls()
+        self.rows, self.pages = ex.rows, ex.pages
+        self.page_row, self.page_no, self.page_dst = dev["ex_page_row"], dev["ex_page_no"], dev["ex_page_dst"]
+        self.tok_row, self.table = dev["ex_tok_row"], dev["ex_table"].view(-1, 1)
+        lens, cnt = dev["portions"]
+        c0, t0, k = ex.chunks, ex.tiles, ex.seqs
+        self.tiles = StepTiles(dev["tile_row0"][:t0], dev["tile_cnt"][:t0],
+                               (dev["chunk_row0"][:c0], dev["chunk_cnt"][:c0], dev["tok_start"][:ex.rows]), int(max(lens[:k])),
+                               dev["ex_order"] if "ex_order" in ex.arrays else None, (lens[:k], cnt[:k]))
+        self.rest = None
+        if k < len(lens):
+            self.rest = StepTiles(dev["ex_rest_tile_row0"], dev["tile_cnt"][t0:],
+                                  (dev["ex_rest_chunk_row0"], dev["chunk_cnt"][c0:], dev["tok_start"][ex.rows:]), int(max(lens[k:])),
+                                  None, (lens[k:], cnt[k:]))
+        return self
+
+
+def latent_expansion(mixers, row_sizes, dtype: torch.dtype):
+    """What decides for the steps of a model with these latent layers (LatentExpansion; None where no layer is served). row_sizes: of
+    each layer's cached keys and values."""
+    served = [mx for mx, (k_dim, _) in zip(mixers, row_sizes) if expansion_served(mx, k_dim, dtype)]
+    if not served:
+        return None
+    page_bytes = max(2 * 16 * mx.num_q_heads * (mx.head_dim + mx.rot_dim + mx.value_dim) for mx in served)
+    windows = [getattr(mx, "window", 0) for mx in served]
+    mx = served[0]
+    return LatentExpansion(mx.head_dim, mx.rot_dim, mx.value_dim, mx.kv_rank, 0 if 0 in windows else max(windows),
+                           EXPAND_MAX_SCRATCH // page_bytes)
+
+
+def expansion_served(mx, k_dim: int, dtype: torch.dtype) -> bool:
+    if dtype not in (torch.float16, torch.bfloat16):
+        return False
+    lib, code, H = _hip.load(), _hip.dtype_code(dtype), mx.num_q_heads
+    return bool(lib.swl_latent_expand_supported(mx.head_dim, mx.value_dim, mx.rot_dim, mx.kv_rank, k_dim, code)
+                and lib.swl_span_attn_supported(H, H, H, mx.head_dim + mx.rot_dim, mx.value_dim, 0, code))
+
+
+class LatentAttention:
+    """The attention of a latent layer from its projected rows [query heads (dim | rot_dim) | ...] to the heads' results. spec: the folded
+    attention (one key row of kv_rank + rot_dim and one value row of kv_rank for all heads)."""
+
+    def __init__(self, mixer, weight, spec: AttentionSpec, eps: float, pool_slice, max_positions: int, dkv_col: int):
+        self.mixer, self.w, self.spec, self.eps, self.pool_slice, self.max_positions = mixer, weight, spec, eps, pool_slice, max_positions
+        self.dkv_col = dkv_col
+        H = mixer.num_q_heads
+        self.heads_spec = AttentionSpec(H, H, mixer.head_dim + mixer.rot_dim, mixer.value_dim, spec.scale, window=spec.window,
+                                        mask_kind=MASK_WINDOW, sink=spec.sink)
+        self.served = expansion_served(mixer, spec.head_dim, weight.uk.dtype)
+
+    def __call__(self, proj: torch.Tensor, ctx) -> torch.Tensor:
+        mx, w, sp = self.mixer, self.w, self.spec
+        n, H, d, dr, r, e = proj.shape[0], mx.num_q_heads, mx.head_dim, mx.rot_dim, mx.kv_rank, mx.value_dim
+        ex = ctx.expanded if self.served and ctx.pool is not None and ctx.pool.shape[1] % 8 == 0 and self.pool_slice.k_offset % 8 == 0 else None
+        m = ex.rows if ex is not None else 0
+        qa = torch.empty((n - m, H * sp.head_dim), dtype=proj.dtype, device=proj.device)
+        latent_rope_and_store_kv(proj, qa, w.freq, w.c_norm, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq,
+                                 ctx.tok_pos, mx, self.dkv_col, self.eps, sp.head_dim, sp.value_dim, in_place=m)
+        y = torch.empty((n, H * e), dtype=proj.dtype, device=proj.device)
+        if m:
+            self._expanded(proj, y[:m], ctx, ex)
+        if m < n:
+            rows = slice(m, n)
+            # q_abs[t, h, :] = W_uk,h^T q_unrotated[t, h, :]  -> the first kv_rank columns of every head of qa
+            qn = proj[rows, :H * (d + dr)].view(n - m, H, d + dr)[:, :, :d].transpose(0, 1)       # [H, T, d]
+            torch.bmm(qn, w.uk, out=qa.view(n - m, H, sp.head_dim)[:, :, :r].transpose(0, 1))   # (a strided batched product: no copy)
+            if ctx.pool is None:    # memory profiling: the attention's output buffer without its reads
+                att = torch.zeros((n - m, H * sp.value_dim), dtype=proj.dtype, device=proj.device)
+            else:
+                att = masked_attention(qa, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq[rows], ctx.tok_pos[rows], sp,
+                                       ex.rest if m else ctx.tiles, self.max_positions)
+            torch.bmm(att.view(n - m, H, sp.value_dim)[:, :, :r].transpose(0, 1), w.uv_t, out=y[rows].view(n - m, H, e).transpose(0, 1))
+        return y
+
+    def _expanded(self, proj, out, ctx, ex: ExpandedStep):
+        mx, w, sp, hs = self.mixer, self.w, self.spec, self.heads_spec
+        H, m, esize = mx.num_q_heads, ex.rows, proj.element_size()
+        keys, values = 16 * H * hs.head_dim, 16 * H * mx.value_dim      # (elements of a page)
+        pages = torch.empty((ex.pages, keys + values), dtype=proj.dtype, device=proj.device)
+        _hip.call("swl_latent_expand", _hip.ptr(pages), ctx.pool.data_ptr() + self.pool_slice.k_offset * esize, _hip.ptr(w.uk),
+                  _hip.ptr(w.uv), _hip.ptr(ctx.block_table), _hip.ptr(ex.page_row), _hip.ptr(ex.page_no), _hip.ptr(ex.page_dst),
+                  ex.page_no.shape[0], H, mx.head_dim, mx.value_dim, mx.rot_dim, mx.kv_rank, sp.head_dim, ctx.block_table.shape[1],
+                  ctx.pool.shape[1], _hip.dtype_code(proj.dtype), _hip.stream())
+        masked_attention(proj[:m], pages, PoolSlice(0, keys), ex.table, ex.tok_row, ctx.tok_pos[:m], hs, ex.tiles, self.max_positions, out=out)

@@ -108,23 +108,24 @@ def qkv_conv_rope_and_store_kv(rows: torch.Tensor, bias: torch.Tensor, conv_w: t
 
 def latent_rope_and_store_kv(proj: torch.Tensor, qa: torch.Tensor, freq: torch.Tensor, c_norm: torch.Tensor,
                              pool: torch.Tensor, pool_slice: PoolSlice, block_table: torch.Tensor, tok_seq: torch.Tensor,
-                             tok_pos: torch.Tensor, mixer, dkv_col: int, eps: float, k_dim: int = 0, v_dim: int = 0):
+                             tok_pos: torch.Tensor, mixer, dkv_col: int, eps: float, k_dim: int = 0, v_dim: int = 0,
+                             in_place: int = 0):
     """proj rows: the query heads [dim | rot_dim] and, at column dkv_col (< 0: the layer reads another layer's cache), the
     compressed row [kv_rank | rot_dim]. Writes the rotated query parts into qa [T, heads, k_dim] (columns kv_rank .. kv_rank +
     rot_dim) and the normed latent + rotated shared key part into the pool. The layout of the pairs and the multiplier of the
     rotation are mixer.rot's. k_dim / v_dim: row sizes in qa and in the pool (default kv_rank + rot_dim / kv_rank), columns beyond
-    zeroed."""
+    zeroed. in_place: this many leading rows have their query heads rotated where they are; qa has the rows after them."""
     _hip.require_gpu_tensor(proj, "proj")
     n = proj.shape[0]
     k_dim, v_dim = k_dim or mixer.kv_rank + mixer.rot_dim, v_dim or mixer.kv_rank
     assert proj.dim() == 2 and proj.stride(1) == 1 and qa.is_contiguous() and qa.dtype == proj.dtype
-    assert qa.shape == (n, mixer.num_q_heads * k_dim)
+    assert 0 <= in_place <= n and qa.shape == (n - in_place, mixer.num_q_heads * k_dim)
     assert freq.dtype == torch.float64 and freq.numel() == mixer.rot_dim // 2
     assert tok_pos.dtype == torch.int32 and tok_pos.shape[0] == n
     kp, vp, stride = _pool_ptrs(pool if dkv_col >= 0 else None, pool_slice)
     if kp:
         assert pool.dtype == proj.dtype and c_norm.dtype == torch.float32 and c_norm.numel() == mixer.kv_rank
-    _hip.call("swl_latent_rope_store_kv", _hip.ptr(proj), _hip.ptr(qa), _hip.ptr(freq), _hip.ptr(c_norm), kp, vp,
+    _hip.call("swl_latent_rope_store_kv_rows", _hip.ptr(proj), _hip.ptr(qa), in_place, _hip.ptr(freq), _hip.ptr(c_norm), kp, vp,
               _hip.ptr(block_table), _hip.ptr(tok_seq), _hip.ptr(tok_pos), n, mixer.num_q_heads, mixer.head_dim,
               mixer.rot_dim, mixer.kv_rank, proj.stride(0), dkv_col if kp else -1, qa.stride(0),
               block_table.shape[1] if block_table is not None else 0, stride, float(eps), 1 if mixer.rot.half else 0,

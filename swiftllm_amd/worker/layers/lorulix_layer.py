@@ -11,12 +11,13 @@ from swiftllm_amd import _hip
 
 class StepContext:
     """What the sublayers of one step share: the block pool and table, the per-token plan arrays, the state slots, the portions'
-    chunks (chunk_row0, chunk_cnt, seq_chunk0: designs whose recurrence runs in parallel over them)."""
-    __slots__ = ("pool", "block_table", "tok_seq", "tok_pos", "tiles", "state", "chunks")
+    chunks (chunk_row0, chunk_cnt, seq_chunk0: designs whose recurrence runs in parallel over them), the rows whose latent attention
+    runs on expanded pages (kernels/latent.py)."""
+    __slots__ = ("pool", "block_table", "tok_seq", "tok_pos", "tiles", "state", "chunks", "expanded")
 
-    def __init__(self, pool, block_table, tok_seq, tok_pos, tiles, state, chunks=None):
-        self.pool, self.block_table, self.tok_seq, self.tok_pos, self.tiles, self.state, self.chunks = \
-            pool, block_table, tok_seq, tok_pos, tiles, state, chunks
+    def __init__(self, pool, block_table, tok_seq, tok_pos, tiles, state, chunks=None, expanded=None):
+        self.pool, self.block_table, self.tok_seq, self.tok_pos, self.tiles, self.state, self.chunks, self.expanded = \
+            pool, block_table, tok_seq, tok_pos, tiles, state, chunks, expanded
 
 
 class LorulixAttention:

@@ -2,9 +2,10 @@
 mixing the result into the streams and the next input's norm are the model's fused step (kernels/hyper_stream.py)."""
 import torch
 
+from ..kernels.latent import LatentAttention
 from ..kernels.min_gru import min_gru
 from ..kernels.moe import ACT_SILU, moe_experts, moe_route_grouped
-from ..kernels.rope_kv import head_gate_, latent_rope_and_store_kv, qk_norm_rope_and_store_kv
+from ..kernels.rope_kv import head_gate_, qk_norm_rope_and_store_kv
 from ..kernels.window_attn import MASK_WINDOW, AttentionSpec, masked_attention
 from .kekapel_layer import _project, _silu_unit
 from .lorulix_layer import StepContext
@@ -42,35 +43,21 @@ class RokevikAttention:
 
 
 class RokevikLatentAttention:
-    """(q | compressed kv | gate) projection -> rotary, latent norm and cache store -> queries folded through the key
-    up-projection -> attention of all heads over the one cached row per token (key: latent | rotated part, value: latent) inside
-    the window -> value up-projection per head -> head gate -> output projection."""
+    """(q | compressed kv | gate) projection -> rotary, latent norm and cache store -> attention over the cached rows inside the
+    window, expanded or folded (kernels/latent.py) -> head gate -> output projection."""
 
     def __init__(self, layer_config, weight, eps: float, skinny: bool, pool_slice, max_positions: int, row_sizes):
         mx = self.mixer = layer_config.mixer
-        self.w, self.eps, self.skinny, self.pool_slice, self.max_positions = weight, eps, skinny, pool_slice, max_positions
+        self.w, self.skinny = weight, skinny
         self.y_bias = None
-        self.spec = AttentionSpec(mx.num_q_heads, 1, row_sizes[0], row_sizes[1], mx.scale, window=mx.window,
-                                  mask_kind=MASK_WINDOW)
+        spec = AttentionSpec(mx.num_q_heads, 1, row_sizes[0], row_sizes[1], mx.scale, window=mx.window, mask_kind=MASK_WINDOW)
+        self.attend = LatentAttention(mx, weight, spec, eps, pool_slice, max_positions, mx.q_size)
 
     def forward(self, h: torch.Tensor, ctx: StepContext):
-        mx, w, sp = self.mixer, self.w, self.spec
-        n, H, d, dr, r, e = h.shape[0], mx.num_q_heads, mx.head_dim, mx.rot_dim, mx.kv_rank, mx.value_dim
+        mx, w = self.mixer, self.w
         proj = _project(h, w.proj, self.skinny)
-        qa = torch.empty((n, H * sp.head_dim), dtype=h.dtype, device=h.device)
-        latent_rope_and_store_kv(proj, qa, w.freq, w.c_norm, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq,
-                                 ctx.tok_pos, mx, mx.q_size, self.eps, sp.head_dim, sp.value_dim)
-        # q_abs[t, h, :] = W_uk,h^T q_unrotated[t, h, :]  -> the first kv_rank columns of every head of qa
-        qn = proj[:, :mx.q_size].view(n, H, d + dr)[:, :, :d].transpose(0, 1)           # [H, T, d]
-        torch.bmm(qn, w.uk, out=qa.view(n, H, sp.head_dim)[:, :, :r].transpose(0, 1))   # (a strided batched product: no copy)
-        if ctx.pool is None:
-            att = torch.zeros((n, H * sp.value_dim), dtype=h.dtype, device=h.device)
-        else:
-            att = masked_attention(qa, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq, ctx.tok_pos, sp, ctx.tiles,
-                                   self.max_positions)
-        y = torch.empty((n, H * e), dtype=h.dtype, device=h.device)
-        torch.bmm(att.view(n, H, sp.value_dim)[:, :, :r].transpose(0, 1), w.uv_t, out=y.view(n, H, e).transpose(0, 1))
-        head_gate_(y, proj[:, w.gate_col:w.gate_col + H], H, e)
+        y = self.attend(proj, ctx)
+        head_gate_(y, proj[:, w.gate_col:w.gate_col + mx.num_q_heads], mx.num_q_heads, mx.value_dim)
         return _project(y, w.o, self.skinny), None
 
 

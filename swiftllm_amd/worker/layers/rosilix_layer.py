@@ -2,9 +2,10 @@
 stream and the next input norm are the model's fused step (kernels/rms_stream.py)."""
 import torch
 
+from ..kernels.latent import LatentAttention
 from ..kernels.linear import ROWS_MAX_TOKENS, linear_rows
 from ..kernels.moe import relu_squared
-from ..kernels.rope_kv import diff_head_combine, head_gate_, latent_rope_and_store_kv, rope_and_store_kv
+from ..kernels.rope_kv import diff_head_combine, head_gate_, rope_and_store_kv
 from ..kernels.window_attn import MASK_CHUNK, MASK_WINDOW, AttentionSpec, masked_attention
 from .kekapel_layer import _project, _project_partials
 from .lorulix_layer import StepContext
@@ -37,35 +38,22 @@ class RosilixDiffAttention:
 
 
 class RosilixLatentAttention:
-    """(q | compressed kv | gate) projection -> rotary, latent norm and cache store -> queries folded through the key
-    up-projection -> attention of all heads over the one cached row per token (key: latent | rotated part, value: latent)
-    with the heads' sinks -> value up-projection per head -> head gate -> output projection. A layer that reads another
-    layer's cache projects queries and gates only."""
+    """(q | compressed kv | gate) projection -> rotary, latent norm and cache store -> attention over the cached rows with the heads'
+    sinks, expanded or folded (kernels/latent.py) -> head gate -> output projection. A layer that reads another layer's cache
+    projects queries and gates only."""
 
     def __init__(self, layer_config, weight, eps: float, skinny: bool, pool_slice, max_positions: int):
         mx = self.mixer = layer_config.mixer
-        self.w, self.eps, self.skinny, self.pool_slice, self.max_positions = weight, eps, skinny, pool_slice, max_positions
-        self.spec = AttentionSpec(mx.num_q_heads, 1, mx.kv_rank + mx.rot_dim, mx.kv_rank, mx.scale, window=0,
-                                  mask_kind=MASK_WINDOW, sink=weight.sink)
+        self.w, self.skinny = weight, skinny
+        spec = AttentionSpec(mx.num_q_heads, 1, mx.kv_rank + mx.rot_dim, mx.kv_rank, mx.scale, window=0, mask_kind=MASK_WINDOW,
+                             sink=weight.sink)
+        self.attend = LatentAttention(mx, weight, spec, eps, pool_slice, max_positions, weight.dkv_col)
 
     def forward(self, h: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         mx, w = self.mixer, self.w
-        n, H, d, dr, r, e = h.shape[0], mx.num_q_heads, mx.head_dim, mx.rot_dim, mx.kv_rank, mx.value_dim
         proj = _project(h, w.proj, self.skinny)
-        qa = torch.empty((n, H * (r + dr)), dtype=h.dtype, device=h.device)
-        latent_rope_and_store_kv(proj, qa, w.freq, w.c_norm, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq,
-                                 ctx.tok_pos, mx, w.dkv_col, self.eps)
-        # q_abs[t, h, :] = W_uk,h^T q_unrotated[t, h, :]  -> the first kv_rank columns of every head of qa
-        qn = proj[:, :H * (d + dr)].view(n, H, d + dr)[:, :, :d].transpose(0, 1)        # [H, T, d]
-        torch.bmm(qn, w.uk, out=qa.view(n, H, r + dr)[:, :, :r].transpose(0, 1))      # (a strided batched product: no copy)
-        if ctx.pool is None:
-            att = torch.zeros((n, H * r), dtype=h.dtype, device=h.device)
-        else:
-            att = masked_attention(qa, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq, ctx.tok_pos, self.spec,
-                                   ctx.tiles, self.max_positions)
-        y = torch.empty((n, H * e), dtype=h.dtype, device=h.device)
-        torch.bmm(att.view(n, H, r).transpose(0, 1), w.uv_t, out=y.view(n, H, e).transpose(0, 1))
-        head_gate_(y, proj[:, w.gate_col:w.gate_col + H], H, e)
+        y = self.attend(proj, ctx)
+        head_gate_(y, proj[:, w.gate_col:w.gate_col + mx.num_q_heads], mx.num_q_heads, mx.value_dim)
         return _project_partials(y, w.o, self.skinny)
 
 

@@ -22,6 +22,7 @@ from swiftllm_amd.engine_config import EngineConfig
 from swiftllm_amd.model_config import RokevikModelConfig
 
 from .kernels.hyper_stream import embed_streams, hyper_step
+from .kernels.latent import EXPAND_MAX_SCRATCH, ExpandedStep, latent_expansion
 from .kernels.linear import pack_weight, packable_rows
 from .kernels.rms_stream import StateRef
 from .kernels.sampling import softcap_logits
@@ -98,6 +99,12 @@ class RokevikModel(SteppedModel):
                 self.sublayers.append(_Sublayer(RokevikFeedForward(lcfg, lw, skinny), lw.norm2, lw.streams2, True))
         if self.state is not None:
             self.state.allocate()
+        latent = [(cfg.layers[run.layer].mixer, self.row_sizes[run.index]) for run in cfg.layer_runs
+                  if cfg.layers[run.layer].type == "latent_attention"]
+        self.latent_expansion = latent_expansion([mx for mx, _ in latent], [sizes for _, sizes in latent], self.dtype)
+
+    def _scratch_bytes(self, num_tokens: int, batch: int) -> int:
+        return super()._scratch_bytes(num_tokens, batch) + (EXPAND_MAX_SCRATCH if self.latent_expansion is not None else 0)
 
     @torch.inference_mode()
     def _run_stack(self, dev: dict, use_pool: bool) -> torch.Tensor:
@@ -110,7 +117,7 @@ class RokevikModel(SteppedModel):
                           dev["seq_row0"], dev["seq_cnt"])
         ctx = StepContext(self.kv_pool if use_pool else None, self.gpu_block_manager.block_table if use_pool else None,
                           dev["tok_seq"], dev["tok_pos"], StepTiles.of(dev), st,
-                          (dev["chunk_row0"], dev["chunk_cnt"], dev["seq_chunk0"]))
+                          (dev["chunk_row0"], dev["chunk_cnt"], dev["seq_chunk0"]), ExpandedStep.of(dev))
         x = embed_streams(dev["input_ids"], w.embed, max(cfg.num_streams, 1))
         tap = self.layer_tap
         subs = self.sublayers

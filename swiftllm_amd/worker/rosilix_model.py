@@ -19,6 +19,7 @@ from swiftllm_amd.engine_config import EngineConfig
 from swiftllm_amd.model_config import RosilixModelConfig
 
 from .kernels.layernorm import embed_positions
+from .kernels.latent import EXPAND_MAX_SCRATCH, ExpandedStep, latent_expansion
 from .kernels.linear import pack_weight, packable_rows
 from .kernels.rms_stream import gated_add_rmsnorm
 from .kernels.window_attn import PoolSlice, StepTiles
@@ -85,6 +86,11 @@ class RosilixModel(SteppedModel):
                 f.op = RosilixFeedForward(lcfg, lw, skinny)
                 f.pre, f.post, f.ends_layer = lw.norm2, lw.norm2b, True
                 self.sublayers.append(f)
+        latent = [layer.mixer for layer in cfg.layers if layer.type != "attention"]
+        self.latent_expansion = latent_expansion(latent, [(mx.kv_rank + mx.rot_dim, mx.kv_rank) for mx in latent], self.dtype)
+
+    def _scratch_bytes(self, num_tokens: int, batch: int) -> int:
+        return super()._scratch_bytes(num_tokens, batch) + (EXPAND_MAX_SCRATCH if self.latent_expansion is not None else 0)
 
     @torch.inference_mode()
     def _run_stack(self, dev: dict, use_pool: bool) -> torch.Tensor:
@@ -92,7 +98,7 @@ class RosilixModel(SteppedModel):
         cfg, w = self.model_config, self.weight
         eps = cfg.norm_eps
         ctx = StepContext(self.kv_pool if use_pool else None, self.gpu_block_manager.block_table if use_pool else None,
-                          dev["tok_seq"], dev["tok_pos"], StepTiles.of(dev), None)
+                          dev["tok_seq"], dev["tok_pos"], StepTiles.of(dev), None, expanded=ExpandedStep.of(dev))
         x, _ = embed_positions(dev["input_ids"], dev["tok_pos"], w.embed, None, cfg.embedding_scale, keep_copy=False)
         tap = self.layer_tap
         subs = self.sublayers

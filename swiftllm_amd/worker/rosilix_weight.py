@@ -71,8 +71,8 @@ class RosilixLayerWeight:
             parts.append(mat("mix.g", (H, w)))
             self.proj = _pad_rows(torch.cat(parts, dim=0))
             self.uk = mat("mix.uk", (H * mx.head_dim, mx.kv_rank)).view(H, mx.head_dim, mx.kv_rank).contiguous()
-            self.uv_t = mat("mix.uv", (H * mx.value_dim, mx.kv_rank)).view(H, mx.value_dim, mx.kv_rank) \
-                .transpose(1, 2).contiguous()
+            self.uv = mat("mix.uv", (H * mx.value_dim, mx.kv_rank)).view(H, mx.value_dim, mx.kv_rank).contiguous()
+            self.uv_t = self.uv.transpose(1, 2).contiguous()
             self.sink = f32("mix.sink", (H,))
         self.o = mat("mix.o", (w, mx.o_size))
         if lcfg.mlp is not None:

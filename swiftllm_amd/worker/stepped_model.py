@@ -66,6 +66,7 @@ class SteppedModel:
         self._layout_pool()
         self._meta_host = self._meta_host_np = self._meta_dev = self._meta_done = None
         self.after_launch_hook = None
+        self.latent_expansion = None        # LatentExpansion of designs with latent attention (worker/kernels/latent.py)
         # pure-decode steps (every sequence brings one token and asks for its logits) replay a captured hipGraph, one per
         # batch size: the step's launch geometry depends on the token count only, never on positions, block ids or slots
         self._decode_graphs = {}
@@ -158,15 +159,23 @@ class SteppedModel:
                                               ecfg.max_blocks_per_seq, ecfg.block_size, self.device)
 
     # ---- one step ----------------------------------------------------------------------------------------------------
-    def _upload_plan(self, plan: StepPlan):
+    def _upload_plan(self, plan: StepPlan, use_pool: bool = True):
         """The plan's int32 arrays through ONE pinned buffer and ONE async copy; returns device views."""
         layout, total = plan.packed_layout()
         order = plan.upload_order()
-        order_at, total = total, total + (order.size if order is not None else 0)
+        extra = [] if order is None else [("span_order", order)]
+        expanded = plan.latent_expansion(self.latent_expansion) if self.latent_expansion is not None and use_pool else None
+        if expanded is not None:
+            extra += expanded.arrays.items()
+        places = [(at, getattr(plan, name)) for name, at, _ in layout]
+        for name, values in extra:
+            layout.append((name, total, values.size))
+            places.append((total, values))
+            total += (values.size + 3) // 4 * 4
         if self._meta_done is not None:
             self._meta_done.synchronize()
         if self._meta_host is None or self._meta_host.numel() < total:
-            cap = max(total, 4 * self.engine_config.max_tokens_in_batch + 64)
+            cap = max(total, 8 * self.engine_config.max_tokens_in_batch + 64)
             self._meta_host = torch.empty(cap, dtype=torch.int32, pin_memory=True)
             self._meta_host_np = self._meta_host.numpy()
             self._meta_dev = torch.empty(cap, dtype=torch.int32, device=self.device)
@@ -175,14 +184,13 @@ class SteppedModel:
             # gone is refused by the caching allocator)
             self._decode_graphs.clear()
             self._graph_pool = None
-        plan.pack_into(self._meta_host_np, (layout, order_at))
-        if order is not None:
-            self._meta_host_np[order_at:total] = order
+        for at, values in places:
+            self._meta_host_np[at:at + values.size] = values
         self._meta_dev[:total].copy_(self._meta_host[:total], non_blocking=True)
         self._meta_done.record()
         dev = _PlanViews(self._meta_dev, layout)
-        if order is not None:
-            dev["span_order"] = self._meta_dev[order_at:total]
+        dev["span_order"] = dev["span_order"] if order is not None else None
+        dev["expanded"] = expanded
         return dev
 
     def _begin_state_step(self, plan: StepPlan):
@@ -207,7 +215,7 @@ class SteppedModel:
         if not ignore_kvcache:
             self.gpu_block_manager.allocate_blocks_for_seqs(plan.seq_ids_list, plan.target_lens_list)
         self._begin_state_step(plan)
-        dev = self._upload_plan(plan)
+        dev = self._upload_plan(plan, not ignore_kvcache)
         dev["longest"], dev["portions"] = int(max(plan.target_lens_list)), (plan.target_lens_list, plan.seq_cnt)
         dev["longest_portion"] = 1 if plan.num_tokens == plan.num_seqs else int(plan.seq_cnt.max())
         if (getattr(self.engine_config, "use_hip_graph", False) and not ignore_kvcache and self.layer_tap is None

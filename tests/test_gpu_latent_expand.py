@@ -1,0 +1,136 @@
+"""Latent attention on expanded pages (csrc/latent_expand.hip, kernels/latent.py): the pages against float64 products of the cached rows, and the
+attention of whole steps (portions with and without earlier tokens, beside decoded ones) against the folded form's oracle."""
+import math
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+UNIT = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}      # half a unit in the last place, relative
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,d,dr,e,r,pad,pages", [(2, 128, 64, 128, 512, 0, 21), (3, 64, 64, 64, 64, 0, 8), (1, 136, 8, 200, 128, 8, 1),
+                                                  (2, 8, 56, 128, 192, 40, 9), (5, 256, 64, 256, 64, 0, 17)])
+def test_pages(H, d, dr, e, r, pad, pages, dtype):
+    from swiftllm_amd import _hip
+    g = torch.Generator().manual_seed(pages)
+    k_dim, off = r + dr + pad, 24
+    blocks = pages + 5
+    pool = torch.randn(blocks, off + 16 * k_dim + 16, generator=g).to(dtype)
+    uk, uv = (torch.randn(H, n, r, generator=g).div(math.sqrt(r)).to(dtype) for n in (d, e))
+    table = torch.randperm(blocks, generator=g)[:2 * ((pages + 1) // 2)].view(2, -1).int()
+    row = torch.tensor([i % 2 for i in range(pages)]).int()
+    no = torch.tensor([i // 2 for i in range(pages)]).int()
+    dst = (torch.randperm(pages + 2, generator=g)[:pages]).int()
+    page = 16 * H * (d + dr + e)
+    out = torch.full((pages + 2, page), 3.0, dtype=dtype, device="cuda")
+    dev = [t.cuda() for t in (pool, uk, uv, table, row, no, dst)]
+    _hip.call("swl_latent_expand", out.data_ptr(), dev[0].data_ptr() + off * 2, *[t.data_ptr() for t in dev[1:]], pages, H, d, e, dr, r, k_dim,
+              table.shape[1], pool.shape[1], _hip.dtype_code(dtype), _hip.stream())
+    out = out.cpu()
+    for i in range(pages):
+        c = pool[int(table[int(row[i]), int(no[i])]), off:off + 16 * k_dim].view(16, k_dim)
+        lat = c[:, :r].double()
+        got_k = out[int(dst[i]), :16 * H * (d + dr)].view(H, 16, d + dr)
+        got_v = out[int(dst[i]), 16 * H * (d + dr):].view(H, e, 16)
+        for got, want, mag in ((got_k[:, :, :d], torch.einsum("tr,hdr->htd", lat, uk.double()), torch.einsum("tr,hdr->htd", lat.abs(), uk.double().abs())),
+                               (got_v, torch.einsum("tr,her->het", lat, uv.double()), torch.einsum("tr,her->het", lat.abs(), uv.double().abs()))):
+            # one rounding of a sum of r fp32 terms
+            assert bool(((got.double() - want).abs() <= UNIT[dtype] * want.abs() + r * 2.0 ** -23 * mag + 1e-7).all())
+        assert torch.equal(got_k[:, :, d:], c[None, :, r:r + dr].expand(H, 16, dr))
+    untouched = [i for i in range(pages + 2) if i not in dst.tolist()]
+    assert bool((out[untouched] == 3.0).all())
+
+
+def _step(parts, window, max_pages=1 << 20):
+    """-> (plan, device views) of portions (sequence, start, tokens)."""
+    from swiftllm_amd.worker.batch_plan import LatentExpansion, StepEntry, plan_step
+    plan = plan_step([StepEntry(s, [1] * n, a, ()) for s, a, n in parts])
+    expanded = plan.latent_expansion(LatentExpansion(128, 64, 128, 512, window, max_pages))
+    dev = {n: torch.from_numpy(np.ascontiguousarray(getattr(plan, n))).cuda() for n in plan.SEGMENTS}
+    dev["portions"], dev["longest"], dev["expanded"] = (plan.target_lens_list, plan.seq_cnt), max(plan.target_lens_list), expanded
+    if expanded is not None:
+        dev.update({n: torch.from_numpy(np.ascontiguousarray(v)).cuda() for n, v in expanded.arrays.items()})
+    return plan, dev
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("window,sink,half", [(0, True, False), (70, False, True)])
+@pytest.mark.parametrize("parts,rows", [([(1, 0, 200), (2, 0, 16), (0, 0, 33)], 249), ([(2, 0, 40), (1, 130, 190), (0, 99, 1), (3, 16, 1)], 230),
+                                        ([(0, 0, 128), (1, 40, 5), (2, 0, 64)], 128), ([(0, 60, 1), (1, 0, 64)], 0)])
+def test_steps(parts, rows, window, sink, half, dtype):
+    """Whatever rows are expanded, the results are those of 64-bit attention on the cached rows."""
+    from swiftllm_amd.worker.kernels.latent import ExpandedStep, LatentAttention
+    from swiftllm_amd.worker.kernels.window_attn import AttentionSpec, PoolSlice, StepTiles
+    g = torch.Generator().manual_seed(rows + window)
+    H, d, dr, e, r = 4, 128, 64, 128, 512
+    mx = SimpleNamespace(num_q_heads=H, head_dim=d, rot_dim=dr, value_dim=e, kv_rank=r, window=window,
+                         rot=SimpleNamespace(dims=dr, half=half, multiplier=1.0))
+    uk, uv = (torch.randn(H, n, r, generator=g).div(math.sqrt(r)).to(dtype) for n in (d, e))
+    freq = 10000.0 ** (-torch.arange(0, dr, 2, dtype=torch.float64) / dr)
+    w = SimpleNamespace(uk=uk.cuda(), uv=uv.cuda(), uv_t=uv.transpose(1, 2).contiguous().cuda(), freq=freq.cuda(),
+                        c_norm=torch.ones(r, device="cuda"))
+    sinks = torch.randn(H, generator=g) if sink else None
+    spec = AttentionSpec(H, 1, r + dr, r, (d + dr) ** -0.5, window=window, sink=sinks.cuda() if sink else None)
+    plan, dev = _step(parts, window)
+    ex = ExpandedStep.of(dev)
+    assert (ex.rows if ex else 0) == rows
+    # earlier tokens' rows in shuffled blocks, stale rows behind the ends
+    blocks, block = torch.randperm(64, generator=g), 16 * (2 * r + dr)
+    pool = torch.randn(64, block, generator=g).to(dtype)
+    pool[:, 16 * (r + dr):] = pool[:, :16 * (r + dr)].view(64, 16, r + dr)[:, :, :r].transpose(1, 2).reshape(64, -1)
+    table = torch.zeros(4, 22, dtype=torch.int32)
+    at = 0
+    for s, a, n in parts:
+        pages = -(-(a + n) // 16)
+        table[s, :pages] = blocks[at:at + pages]
+        at += pages
+    n = plan.num_tokens
+    rows_in = torch.randn(n, H * (d + dr) + r + dr + 16, generator=g).to(dtype)
+    pool_dev, proj = pool.cuda(), rows_in.cuda()
+    ctx = SimpleNamespace(pool=pool_dev, block_table=table.cuda(), tok_seq=dev["tok_seq"], tok_pos=dev["tok_pos"], tiles=StepTiles.of(dev),
+                          expanded=ex)
+    attend = LatentAttention(mx, w, spec, 1e-6, PoolSlice(0, 16 * (r + dr)), 4096, H * (d + dr))
+    got = attend(proj, ctx).cpu().double()
+    pool = pool_dev.cpu()
+    folded_rows = SimpleNamespace(**{**ctx.__dict__, "expanded": None})
+    folded = attend(rows_in.cuda(), folded_rows).cpu().double()
+    row = 0
+    worst, worst_folded = 0.0, 0.0
+    for s, a, cnt in parts:
+        cached = torch.cat([pool[int(table[s, b]), :16 * (r + dr)].view(16, r + dr) for b in range(-(-(a + cnt) // 16))])[:a + cnt].double()
+        k = torch.cat((torch.einsum("tr,hdr->htd", cached[:, :r], uk.double()), cached[None, :, r:].expand(H, -1, -1)), 2)
+        v = torch.einsum("tr,her->hte", cached[:, :r], uv.double())
+        q = rows_in[row:row + cnt, :H * (d + dr)].view(cnt, H, d + dr).double()
+        ang = torch.arange(a, a + cnt, dtype=torch.float64)[:, None] * freq
+        cs, sn = torch.cos(ang)[:, None].float().double(), torch.sin(ang)[:, None].float().double()
+        x, y = (q[..., d:d + dr // 2], q[..., d + dr // 2:]) if half else (q[..., d::2], q[..., d + 1::2])
+        u, z = x * cs - y * sn, y * cs + x * sn
+        rot = torch.cat((u, z), -1) if half else torch.stack((u, z), -1).flatten(-2)
+        q = torch.cat((q[..., :d], rot.to(dtype).double()), -1)
+        sc = torch.einsum("qhd,hkd->hqk", q, k) * spec.scale
+        pos, key = torch.arange(a, a + cnt)[:, None], torch.arange(a + cnt)[None]
+        see = (key <= pos) & ((pos - key < window) if window else torch.ones_like(key <= pos))
+        sc = sc.masked_fill(~see, -math.inf)
+        if sink:
+            sc = torch.cat((sc, sinks.double()[:, None, None].expand(H, cnt, 1)), 2)
+        want = torch.einsum("hqk,hke->qhe", torch.softmax(sc, 2)[:, :, :a + cnt], v).reshape(cnt, -1)
+        # a key's and a value's products are rounded once (as folded queries and latent results are): scores move by sqrt(d) of such
+        # roundings of |q| |k| ~ 1, results by one of the largest |v| ~ 4, and by what the scores' weights move
+        bound = 24 * UNIT[dtype]
+        err = (got[row:row + cnt] - want).abs().max().item()
+        worst += float(((got[row:row + cnt] - want) ** 2).sum())
+        worst_folded += float(((folded[row:row + cnt] - want) ** 2).sum())
+        assert err <= bound, (s, a, cnt, err, bound)
+        row += cnt
+    print(f"largest error {math.sqrt(worst):.4e}, folded {math.sqrt(worst_folded):.4e}")
+
+
+def test_portions_past_the_scratch_limit_stay_folded():
+    parts = [(0, 0, 64), (1, 0, 64), (2, 0, 64)]
+    for pages, rows in ((12, 192), (11, 128), (4, 64), (3, 0)):
+        ex = _step(parts, 0, pages)[1]["expanded"]
+        assert (ex.rows if ex else 0) == rows

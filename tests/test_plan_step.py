@@ -121,3 +121,40 @@ def test_plan_of_one_token_each(n):
     if n > 1:
         assert plan_tokens(toks, ids[:-1] + ids[:1], starts, 50, 300) is None
     assert plan_tokens([], [], [], 50, 300) is None
+
+
+@pytest.mark.parametrize("window", [0, 48])
+def test_latent_expansion_covers_what_its_portions_see(window):
+    """Every page that a query of an expanded portion sees is expanded once, under the number that the attention's table gives it; what is
+    left keeps its chunks and tiles."""
+    from swiftllm_amd.worker.batch_plan import LatentExpansion
+    rng = random.Random(window)
+    spec = LatentExpansion(128, 64, 128, 512, window, 4096)
+    for _ in range(60):
+        parts = [(s, rng.choice((0, 0, rng.randint(0, 300))), rng.choice((1, 17, rng.randint(16, 260)))) for s in rng.sample(range(40), rng.randint(1, 6))]
+        plan = plan_step([StepEntry(s, [1] * n, a, ()) for s, a, n in parts])
+        ex = plan.latent_expansion(spec)
+        pays = spec.pays(np.array([a for _, a, _ in parts]), np.array([n for _, _, n in parts])).tolist()
+        k = (pays + [False]).index(False)
+        if k == 0:
+            assert ex is None
+            continue
+        A = ex.arrays
+        assert ex.seqs == k and ex.rows == sum(n for _, _, n in parts[:k])
+        made = {int(d): (int(r), int(p)) for r, p, d in zip(A["ex_page_row"], A["ex_page_no"], A["ex_page_dst"])}
+        assert len(made) == A["ex_page_dst"].size and max(made) < ex.pages == A["ex_table"].size
+        row, first = 0, []
+        for s, a, n in parts[:k]:
+            rows = A["ex_tok_row"][row:row + n]
+            assert (rows == rows[0]).all()
+            first.append(int(rows[0]))
+            for page in range((max(a - window + 1, 0) if window else 0) // 16, (a + n - 1) // 16 + 1):
+                assert made.pop(int(A["ex_table"][rows[0] + page])) == (s, page)
+            row += n
+        assert not made and len(set(first)) == k
+        if k < len(parts):
+            assert np.array_equal(A["ex_rest_chunk_row0"] + row, plan.chunk_row0[ex.chunks:]) and plan.chunk_row0[ex.chunks] == row
+            assert np.array_equal(A["ex_rest_tile_row0"] + row, plan.tile_row0[ex.tiles:]) and plan.tile_row0[ex.tiles] == row
+        order = plan.upload_order()
+        if order is not None:
+            assert sorted(A["ex_order"]) == list(range(ex.chunks))
