@@ -24,6 +24,7 @@ from .kernels.block_mgmt import (
     unset_block_table_and_num_seq_alloc_blocks,
     gather_allocated_blocks_and_unset,
 )
+from .pinned_ring import PinnedRing
 
 
 class BlockAllocatorHost:
@@ -135,8 +136,7 @@ class BlockManager:
         self.block_table = torch.empty((max_seqs_in_block_table, max_blocks_per_seq),
                                        dtype=torch.int32, device=self.device)
         self.is_block_free = torch.ones((num_blocks,), dtype=torch.bool, device=self.device)
-        self._staging = None        # pinned int32 staging buffer, grown on demand
-        self._staging_done = None   # event recorded after the last copy out of it
+        self._staging = PinnedRing(4)       # (a step allocates and frees: two steps' worth)
 
     @property
     def num_free_blocks(self) -> int:
@@ -144,25 +144,15 @@ class BlockManager:
 
     # ---- host -> device metadata upload -------------------------------------------------------------
     def _upload(self, *arrays: np.ndarray):
-        """Pack int32 arrays into the pinned staging buffer, issue one async H2D copy, return device
-        views. The staging buffer is reused; an event guards it against being overwritten while the
-        previous copy is still queued (normally long complete: one cheap event query)."""
-        total = sum(a.size for a in arrays)
-        if self._staging_done is not None:
-            self._staging_done.synchronize()    # previous copy out of the staging buffer finished
-        if self._staging is None or self._staging.numel() < total:
-            cap = max(1024, 1 << (max(total, 1) - 1).bit_length())
-            self._staging = torch.empty(cap, dtype=torch.int32, pin_memory=True)
-            self._staging_np = self._staging.numpy()
-        off = 0
+        """Pack int32 arrays into a pinned staging buffer, issue one async H2D copy, return device views."""
+        total, places = 0, []
         for a in arrays:
-            self._staging_np[off:off + a.size] = a
-            off += a.size
+            places.append((total, a))
+            total += a.size
+        staged, enqueued = self._staging.fill(total, places)
         dev = torch.empty(total, dtype=torch.int32, device=self.device)
-        dev.copy_(self._staging[:total], non_blocking=True)
-        if self._staging_done is None:
-            self._staging_done = torch.cuda.Event()
-        self._staging_done.record()
+        dev.copy_(staged, non_blocking=True)
+        enqueued()
         views, off = [], 0
         for a in arrays:
             views.append(dev[off:off + a.size])

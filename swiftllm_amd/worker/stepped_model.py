@@ -30,6 +30,7 @@ from .block_manager import BlockManager
 from .kernels.block_swapping import swap_blocks
 from .kernels.sampling import argmax_rows
 from .kernels.window_attn import SHARE_MAX_SCRATCH
+from .pinned_ring import PinnedRing
 
 DTYPES = {"float16": torch.float16, "bfloat16": torch.bfloat16, "float32": torch.float32}
 
@@ -64,7 +65,7 @@ class SteppedModel:
         self.state = None           # StateSlotManager of designs with per-sequence recurrent state
         self.block_elems = 0
         self._layout_pool()
-        self._meta_host = self._meta_host_np = self._meta_dev = self._meta_done = None
+        self._meta_staging, self._meta_dev = PinnedRing(2), None
         self.after_launch_hook = None
         self.latent_expansion = None        # LatentExpansion of designs with latent attention (worker/kernels/latent.py)
         # pure-decode steps (every sequence brings one token and asks for its logits) replay a captured hipGraph, one per
@@ -160,7 +161,7 @@ class SteppedModel:
 
     # ---- one step ----------------------------------------------------------------------------------------------------
     def _upload_plan(self, plan: StepPlan, use_pool: bool = True):
-        """The plan's int32 arrays through ONE pinned buffer and ONE async copy; returns device views."""
+        """The plan's int32 arrays through one pinned buffer and ONE async copy; returns device views."""
         layout, total = plan.packed_layout()
         order = plan.upload_order()
         extra = [] if order is None else [("span_order", order)]
@@ -172,22 +173,15 @@ class SteppedModel:
             layout.append((name, total, values.size))
             places.append((total, values))
             total += (values.size + 3) // 4 * 4
-        if self._meta_done is not None:
-            self._meta_done.synchronize()
-        if self._meta_host is None or self._meta_host.numel() < total:
-            cap = max(total, 8 * self.engine_config.max_tokens_in_batch + 64)
-            self._meta_host = torch.empty(cap, dtype=torch.int32, pin_memory=True)
-            self._meta_host_np = self._meta_host.numpy()
-            self._meta_dev = torch.empty(cap, dtype=torch.int32, device=self.device)
-            self._meta_done = torch.cuda.Event()
+        staged, enqueued = self._meta_staging.fill(total, places)
+        if self._meta_dev is None or self._meta_dev.numel() < total:
+            self._meta_dev = torch.empty(max(total, 4 * self.engine_config.max_tokens_in_batch + 64), dtype=torch.int32, device=self.device)
             # captured graphs read the old buffer; their shared memory pool goes with them (a capture into a pool whose last graph is
             # gone is refused by the caching allocator)
             self._decode_graphs.clear()
             self._graph_pool = None
-        for at, values in places:
-            self._meta_host_np[at:at + values.size] = values
-        self._meta_dev[:total].copy_(self._meta_host[:total], non_blocking=True)
-        self._meta_done.record()
+        self._meta_dev[:total].copy_(staged, non_blocking=True)
+        enqueued()
         dev = _PlanViews(self._meta_dev, layout)
         dev["span_order"] = dev["span_order"] if order is not None else None
         dev["expanded"] = expanded
