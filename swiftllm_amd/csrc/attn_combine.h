@@ -6,28 +6,39 @@
 
 namespace swl {
 
-// Eight fp32 weights as two 16-bit terms each. bf16 in pairs: one conversion for two, and the first term as fp32 is a shift or a mask.
-__device__ __forceinline__ void split_weights(const float (&x)[8], vec8_t<bf16> &hi, vec8_t<bf16> &lo) {
+// Two fp32 weights as two 16-bit terms each, in the halves of a register. bf16: one conversion for two, and the first term as fp32 is a shift
+// or a mask.
+template <typename T>
+__device__ __forceinline__ void split_pair(float x0, float x1, unsigned &h, unsigned &l);
+template <>
+__device__ __forceinline__ void split_pair<bf16>(float x0, float x1, unsigned &h, unsigned &l) {
     typedef float float2_t __attribute__((ext_vector_type(2)));
     typedef bf16 bf2_t __attribute__((ext_vector_type(2)));
+    h = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{x0, x1}), bf2_t));
+    const float2_t r = {x0 - __uint_as_float(h << 16), x1 - __uint_as_float(h & 0xffff0000u)};
+    l = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf2_t));
+}
+template <>
+__device__ __forceinline__ void split_pair<f16>(float x0, float x1, unsigned &h, unsigned &l) {
+    const vec2_t<f16> a = {to_t<f16>(x0), to_t<f16>(x1)};
+    const vec2_t<f16> b = {to_t<f16>(x0 - to_f(a[0])), to_t<f16>(x1 - to_f(a[1]))};
+    h = __builtin_bit_cast(unsigned, a);
+    l = __builtin_bit_cast(unsigned, b);
+}
+// ... eight
+template <typename T>
+__device__ __forceinline__ void split_weights(const float (&x)[8], vec8_t<T> &hi, vec8_t<T> &lo) {
     typedef unsigned uint4v __attribute__((ext_vector_type(4)));
     uint4v h, l;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{x[2 * j], x[2 * j + 1]}), bf2_t));
-        const float2_t r = {x[2 * j] - __uint_as_float(u << 16), x[2 * j + 1] - __uint_as_float(u & 0xffff0000u)};
-        h[j] = u;
-        l[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf2_t));
+        unsigned a, b;
+        split_pair<T>(x[2 * j], x[2 * j + 1], a, b);
+        h[j] = a;
+        l[j] = b;
     }
-    hi = __builtin_bit_cast(vec8_t<bf16>, h);
-    lo = __builtin_bit_cast(vec8_t<bf16>, l);
-}
-__device__ __forceinline__ void split_weights(const float (&x)[8], vec8_t<f16> &hi, vec8_t<f16> &lo) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        hi[j] = to_t<f16>(x[j]);
-        lo[j] = to_t<f16>(x[j] - to_f(hi[j]));
-    }
+    hi = __builtin_bit_cast(vec8_t<T>, h);
+    lo = __builtin_bit_cast(vec8_t<T>, l);
 }
 
 // out[t][h][:] = sum_s e^{m_s - M} O_s / sum_s e^{m_s - M} l_s over the key shares s (a share without keys has l = 0).

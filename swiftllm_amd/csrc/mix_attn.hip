@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kMxThreads, 2) void mix_attn_kernel(MixParams p) {
                 }
             }
             vec8_t<T> phi, plo;
-            split_weights(x, phi, plo);
+            split_weights<T>(x, phi, plo);
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
                 acc[hh][ct] = mx_mfma(vf[ct], phi, acc[hh][ct]);

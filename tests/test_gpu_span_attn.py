@@ -93,6 +93,9 @@ CASES = [       # H, G, GV, d, dv, features
     (8, 1, 1, 576, 512, dict(window=70)),
     (40, 1, 1, 320, 256, dict(sink=True)),
     (3, 1, 1, 576, 512, {}),
+    (8, 2, 2, 64, 64, dict(rel=True)),          # (a wave's 32 rows: 16 queries of two heads)
+    (6, 2, 2, 64, 128, dict(rel=True, window=45, softcap=7.0)),
+    (5, 1, 1, 128, 64, dict(sink=True, slopes=True)),
 ]
 
 
@@ -175,6 +178,12 @@ def test_steps_of_many_workgroups(case, shares, dtype, monkeypatch):
         monkeypatch.setattr(window_attn, "share_scratch", lambda device, splits, floats: (
             shares, torch.full((shares * floats,), float("nan"), device=device)))
     test_span_attention(case, parts, dtype)
+
+
+@pytest.mark.parametrize("case", [i for i, c in enumerate(CASES) if c[3] + c[4] <= 320])
+def test_portions_of_many_pages(case):
+    """More pages than one load of block ids holds (64), from the first page on and behind cached tokens."""
+    test_span_attention(case, [(1, 0, 1300), (2, 1037, 40)], torch.bfloat16)
 
 
 @pytest.mark.parametrize("scale", [1e-38, 1e-30, 1e-19, -0.05, 0.0])
