@@ -671,6 +671,13 @@ int swl_mix_sigmoid_attn(void *out, const void *q, const void *k_cache, const vo
  *   of block-table row page_row[i] and goes to out + page_dst[i] pages of num_heads * 16 * (dim + rot_dim + vdim) elements: keys
  *   [heads, 16, dim + rot_dim] = (uk[h] c | rotated part), uk [heads, dim, kv_rank], then values [heads, vdim, 16] = uv[h] c, uv [heads, vdim,
  *   kv_rank]; products are rounded once. k_dim: elements of a cached row (kv_rank | rot_dim first). Ask swl_latent_expand_supported.
+ * swl_latent_fold: swl_latent_rope_store_kv beside the queries folded through the key up-projection: qa[t][h][:kv_rank] = uk[h]^T
+ *   (unrotated part of the query), uk_t [heads, kv_rank, dim]; rounded once. Ask swl_latent_fold_supported.
+ * swl_latent_decode: attention of single tokens over the latent key cache, all heads over the one row of each earlier token (its first kv_rank
+ *   columns are the value): rows qa as swl_latent_fold leaves them. Every token's pages are shared out over `shares` workgroups a 16 heads;
+ *   scratch: fp32 [shares, tokens, heads, kv_rank] unnormalised results, then [shares, tokens, heads, 2] (maximum in base-2 units, sum).
+ *   swl_latent_unfold: y[t][h] = sigmoid(gate[t * gate_stride + h]) uv[h] (sum of the shares over their sums and sink[h], rounded), uv
+ *   [heads, vdim, kv_rank]; sink, gate may be NULL. Ask swl_latent_decode_supported.
  * swl_diff_head_combine: maps fp32 [T, 2, H, vdim] -> out[T, H, vdim] = unit_rms(a1 - lambda a2; eps) * mult *
  *   sigmoid(gate[t * gate_stride + h]) (gate NULL: no gate).
  * swl_head_gate: y[T, H, vdim] *= sigmoid(gate[t * gate_stride + h]) in place. */
@@ -691,6 +698,18 @@ int swl_latent_rope_store_kv_rows(void *proj, void *qa, int64_t in_place, const 
                                   int64_t proj_stride, int64_t dkv_col, int64_t qa_stride, int32_t max_blocks_per_seq,
                                   int64_t block_stride, float eps, int32_t half, double rot_mult, int32_t k_dim, int32_t v_dim,
                                   int32_t dtype, swl_stream_t stream);
+int swl_latent_fold_supported(int32_t dim, int32_t rot_dim, int32_t kv_rank, int32_t k_dim, int32_t dtype);
+int swl_latent_fold(const void *proj, void *qa, const void *uk_t, const double *freq, const float *c_norm, void *k_cache, void *v_cache,
+                    const int32_t *block_table, const int32_t *tok_seq, const int32_t *tok_pos, int64_t num_tokens, int32_t num_heads,
+                    int32_t dim, int32_t rot_dim, int32_t kv_rank, int64_t proj_stride, int64_t dkv_col, int64_t qa_stride,
+                    int32_t max_blocks_per_seq, int64_t block_stride, float eps, int32_t half, double rot_mult, int32_t k_dim,
+                    int32_t v_dim, int32_t dtype, swl_stream_t stream);
+int swl_latent_decode_supported(int32_t kv_rank, int32_t rot_dim, int32_t k_dim, int32_t vdim, int32_t dtype);
+int swl_latent_decode(float *scratch, const void *q, const void *k_cache, const int32_t *block_table, const int32_t *tok_seq,
+                      const int32_t *tok_pos, int64_t num_tokens, int32_t num_heads, int64_t q_stride, int32_t window, float scale,
+                      int32_t max_blocks_per_seq, int64_t block_stride, int32_t shares, int32_t dtype, swl_stream_t stream);
+int swl_latent_unfold(void *y, const float *scratch, const void *uv, const float *sink, const void *gate, int64_t gate_stride, int64_t num_tokens,
+                      int32_t num_heads, int32_t vdim, int32_t shares, int32_t dtype, swl_stream_t stream);
 int swl_latent_expand_supported(int32_t dim, int32_t vdim, int32_t rot_dim, int32_t kv_rank, int32_t k_dim, int32_t dtype);
 int swl_latent_expand(void *out, const void *k_cache, const void *uk, const void *uv, const int32_t *block_table,
                       const int32_t *page_row, const int32_t *page_no, const int32_t *page_dst, int64_t num_pages,

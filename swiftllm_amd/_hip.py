@@ -128,6 +128,10 @@ SIGNATURES = {
     "swl_latent_rope_store_kv_rows": [_P, _P, _I64, _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I64, _I64, _I64, _I32,
                                       _I64, _F32, _I32, _F64, _I32, _I32, _I32, _P],
     "swl_latent_expand": [_P, _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I64, _I32, _P],
+    "swl_latent_fold": [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I64, _I64, _I64, _I32, _I64, _F32, _I32,
+                        _F64, _I32, _I32, _I32, _P],
+    "swl_latent_decode": [_P, _P, _P, _P, _P, _P, _I64, _I32, _I64, _I32, _F32, _I32, _I64, _I32, _I32, _P],
+    "swl_latent_unfold": [_P, _P, _P, _P, _P, _I64, _I64, _I32, _I32, _I32, _I32, _P],
     "swl_diff_head_combine": [_P, _P, _P, _I64, _F32, _F32, _F32, _I64, _I32, _I32, _I32, _P],
     "swl_head_gate": [_P, _P, _I64, _I64, _I32, _I32, _I32, _P],
     "swl_polynorm": [_P, _P, _F32, _F32, _F32, _F32, _F32, _I64, _I32, _I32, _P],
@@ -208,6 +212,8 @@ _SPECIAL = {
     "swl_window_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_masked_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_moe_gemm_supported": ([_I64, _I32, _I32, _I32], _I32),
+    "swl_latent_fold_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
+    "swl_latent_decode_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_latent_expand_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_span_attn_supported": ([_I32, _I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_delta_rule_tiles_supported": ([_I32, _I32, _I32, _I32], _I32),

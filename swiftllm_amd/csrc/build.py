@@ -52,6 +52,7 @@ SOURCES = [
     "delta_chunks.hip",
     "gemm_f32.hip",
     "latent_expand.hip",
+    "latent_decode.hip",
 ]
 # What a model family's worker calls (the shared pieces included): `build(only=MODEL_SOURCES[...])` compiles just these, so
 # that the first use from a fresh checkout does not pay for kernels the model never launches. A later full build compiles
@@ -64,10 +65,10 @@ MODEL_SOURCES = {
     "Lorulix": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip",
                           "rms_stream.hip", "delta_rule.hip", "delta_chunks.hip"],
     "Rosilix": _SHARED + ["layernorm.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rms_stream.hip",
-                          "rope_kv.hip", "latent_expand.hip"],
+                          "rope_kv.hip", "latent_expand.hip", "latent_decode.hip"],
     "Ratilorn": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip",
                            "rms_stream.hip", "sigmoid_attn.hip", "mix_attn.hip", "ssd.hip", "linear_scan.hip", "delta_rule.hip"],
-    "Rokevik": _SHARED + ["window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rope_kv.hip", "hyper_stream.hip", "min_gru.hip", "latent_expand.hip"],
+    "Rokevik": _SHARED + ["window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rope_kv.hip", "hyper_stream.hip", "min_gru.hip", "latent_expand.hip", "latent_decode.hip"],
     "Vafozen": _SHARED + ["layernorm.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rms_stream.hip", "rope_kv.hip",
                           "hyper_stream.hip", "delta_rule.hip", "ssd.hip", "linear_scan.hip", "low_rank_decay.hip"],
 }

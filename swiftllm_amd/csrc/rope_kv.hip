@@ -390,14 +390,13 @@ __global__ __launch_bounds__(kRkThreads) void qkv_conv_rope_store_kv_kernel(
 }
 
 template <typename T>
-__global__ __launch_bounds__(kRkThreads) void latent_rope_store_kv_kernel(
+__device__ __forceinline__ void latent_rope_store_token(int64_t t,
     T *proj, T *qa, int64_t in_place, const double *freq, const float *c_w, T *k_cache, T *v_cache, const int32_t *block_table,
     const int32_t *tok_seq, const int32_t *tok_pos, int H, int d, int dr, int r, int64_t proj_stride, int64_t dkv_col,
     int64_t qa_stride, int max_blocks_per_seq, int64_t block_stride, float eps, int half, double rot_mult, int k_dim,
     int v_dim) {
     __shared__ float cs[kRkMaxPairs], sn[kRkMaxPairs];
     __shared__ float red[kRkThreads / 64];
-    const int64_t t = page_token();
     const int pos = tok_pos[t];
     const int pairs = dr >> 1;
     rk_angles(cs, sn, freq, pos, pairs, rot_mult);
@@ -451,6 +450,64 @@ __global__ __launch_bounds__(kRkThreads) void latent_rope_store_kv_kernel(
     }
     for (int i = threadIdx.x; i < kpad; i += kRkThreads) kdst[r + dr + i] = to_t<T>(0.f);
     for (int i = threadIdx.x; i < vpad; i += kRkThreads) vdst[static_cast<int64_t>(r + i) * kRkBlock] = to_t<T>(0.f);
+}
+
+template <typename T>
+__global__ __launch_bounds__(kRkThreads) void latent_rope_store_kv_kernel(
+    T *proj, T *qa, int64_t in_place, const double *freq, const float *c_w, T *k_cache, T *v_cache, const int32_t *block_table,
+    const int32_t *tok_seq, const int32_t *tok_pos, int H, int d, int dr, int r, int64_t proj_stride, int64_t dkv_col,
+    int64_t qa_stride, int max_blocks_per_seq, int64_t block_stride, float eps, int half, double rot_mult, int k_dim,
+    int v_dim) {
+    latent_rope_store_token<T>(page_token(), proj, qa, in_place, freq, c_w, k_cache, v_cache, block_table, tok_seq, tok_pos, H, d, dr, r, proj_stride,
+                               dkv_col, qa_stride, max_blocks_per_seq, block_stride, eps, half, rot_mult, k_dim, v_dim);
+}
+
+// The same for a few tokens (the first workgroups, one a token) beside the queries folded through the key up-projection (the others): qa[t][h][:r]
+// = W_uk,h^T q_th, W_uk transposed [H, r, d]. The two write different columns and read nothing of each other: one launch instead of two. A workgroup
+// folds 64 columns of a head for all tokens, a wave 16 (16x16x32, columns as A, tokens as B): 2 MB of matrices over 128 workgroups at 16 heads of 128.
+template <typename T>
+__device__ __forceinline__ float4_t rk_mfma(vec8_t<T> a, vec8_t<T> b, float4_t c);
+template <>
+__device__ __forceinline__ float4_t rk_mfma<f16>(vec8_t<f16> a, vec8_t<f16> b, float4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+template <>
+__device__ __forceinline__ float4_t rk_mfma<bf16>(vec8_t<bf16> a, vec8_t<bf16> b, float4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+constexpr int kFoldMaxDim = 256;
+
+template <typename T>
+__global__ __launch_bounds__(kRkThreads) void latent_fold_kernel(
+    T *proj, T *qa, int n, const T *uk_t, const double *freq, const float *c_w, T *k_cache, T *v_cache, const int32_t *block_table,
+    const int32_t *tok_seq, const int32_t *tok_pos, int H, int d, int dr, int r, int64_t proj_stride, int64_t dkv_col,
+    int64_t qa_stride, int max_blocks_per_seq, int64_t block_stride, float eps, int half, double rot_mult, int k_dim,
+    int v_dim) {
+    if (blockIdx.x < static_cast<unsigned>(n)) {
+        latent_rope_store_token<T>(blockIdx.x, proj, qa, 0, freq, c_w, k_cache, v_cache, block_table, tok_seq, tok_pos, H, d, dr, r, proj_stride,
+                                   dkv_col, qa_stride, max_blocks_per_seq, block_stride, eps, half, rot_mult, k_dim, v_dim);
+        return;
+    }
+    const int tiles = r / 64, at = static_cast<int>(blockIdx.x) - n, h = at / tiles, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int lr = lane & 15, lk = lane >> 4, r0 = (at - h * tiles) * 64 + wave * 16, steps = d / 32;
+    vec8_t<T> wf[kFoldMaxDim / 32];
+    const T *wp = uk_t + (static_cast<int64_t>(h) * r + r0 + lr) * d + lk * 8;
+#pragma unroll
+    for (int e = 0; e < kFoldMaxDim / 32; ++e)
+        if (e < steps) wf[e] = load8(wp + e * 32);
+    for (int t0 = 0; t0 < n; t0 += 16) {
+        const T *qp = proj + min(t0 + lr, n - 1) * proj_stride + static_cast<int64_t>(h) * (d + dr) + lk * 8;
+        float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < kFoldMaxDim / 32; ++e)
+            if (e < steps) acc = rk_mfma<T>(wf[e], load8(qp + e * 32), acc);
+        mfma_results_ready<8>(acc);
+        // acc[k]: column r0 + 4 lk + k of token t0 + lr
+        vec4_t<T> v;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = to_t<T>(acc[k]);
+        if (t0 + lr < n) *reinterpret_cast<vec4_t<T> *>(qa + (t0 + lr) * qa_stride + static_cast<int64_t>(h) * k_dim + r0 + 4 * lk) = v;
+    }
 }
 
 template <typename T>
@@ -612,6 +669,39 @@ extern "C" int swl_latent_rope_store_kv(const void *proj, void *qa, const double
     return swl_latent_rope_store_kv_rows(const_cast<void *>(proj), qa, 0, freq, c_norm, k_cache, v_cache, block_table, tok_seq, tok_pos,
                                          num_tokens, num_heads, dim, rot_dim, kv_rank, proj_stride, dkv_col, qa_stride,
                                          max_blocks_per_seq, block_stride, eps, half, rot_mult, k_dim, v_dim, dtype, stream);
+}
+
+/* 1 when swl_latent_fold serves these sizes. */
+extern "C" int swl_latent_fold_supported(int32_t dim, int32_t rot_dim, int32_t kv_rank, int32_t k_dim, int32_t dtype) {
+    if (dtype != SWL_F16 && dtype != SWL_BF16) return 0;
+    return dim > 0 && dim % 32 == 0 && dim <= swl::kFoldMaxDim && rot_dim > 0 && rot_dim % 8 == 0 && rot_dim <= 2 * swl::kRkMaxPairs && kv_rank > 0 &&
+           kv_rank % 64 == 0 && k_dim >= kv_rank + rot_dim && k_dim % 4 == 0;
+}
+
+extern "C" int swl_latent_fold(const void *proj, void *qa, const void *uk_t, const double *freq, const float *c_norm, void *k_cache, void *v_cache,
+                               const int32_t *block_table, const int32_t *tok_seq, const int32_t *tok_pos, int64_t num_tokens, int32_t num_heads,
+                               int32_t dim, int32_t rot_dim, int32_t kv_rank, int64_t proj_stride, int64_t dkv_col, int64_t qa_stride,
+                               int32_t max_blocks_per_seq, int64_t block_stride, float eps, int32_t half, double rot_mult, int32_t k_dim,
+                               int32_t v_dim, int32_t dtype, swl_stream_t stream) {
+    if (num_tokens < 0 || num_heads <= 0 || v_dim < kv_rank) return SWL_ERR_BAD_ARG;
+    if (!swl_latent_fold_supported(dim, rot_dim, kv_rank, k_dim, dtype)) return SWL_ERR_UNSUPPORTED;
+    if (proj_stride < static_cast<int64_t>(num_heads) * (dim + rot_dim) || qa_stride < static_cast<int64_t>(num_heads) * k_dim)
+        return SWL_ERR_BAD_ARG;
+    if (dkv_col >= 0 && dkv_col + kv_rank + rot_dim > proj_stride) return SWL_ERR_BAD_ARG;
+    if (num_tokens == 0) return SWL_OK;
+    if (!proj || !qa || !uk_t || !freq || !tok_pos) return SWL_ERR_BAD_ARG;
+    if (dkv_col >= 0 && k_cache && (!v_cache || !c_norm || !block_table || !tok_seq || max_blocks_per_seq <= 0)) return SWL_ERR_BAD_ARG;
+    // 16-byte loads of queries and matrices, 8-byte stores
+    if (!swl::aligned16(proj) || (proj_stride & 7) || !swl::aligned16(uk_t) || (reinterpret_cast<uintptr_t>(qa) & 7) || (qa_stride & 3)) return SWL_ERR_BAD_ARG;
+    const int64_t grid = num_tokens + static_cast<int64_t>(num_heads) * (kv_rank / 64);
+    if (grid > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
+    SWL_DISPATCH_DTYPE(dtype, T, {
+        hipLaunchKernelGGL((swl::latent_fold_kernel<T>), dim3(static_cast<unsigned>(grid)), dim3(swl::kRkThreads), 0, static_cast<hipStream_t>(stream),
+                           static_cast<T *>(const_cast<void *>(proj)), static_cast<T *>(qa), static_cast<int>(num_tokens), static_cast<const T *>(uk_t), freq,
+                           c_norm, static_cast<T *>(k_cache), static_cast<T *>(v_cache), block_table, tok_seq, tok_pos, num_heads, dim, rot_dim, kv_rank,
+                           proj_stride, dkv_col, qa_stride, max_blocks_per_seq, block_stride, eps, half, rot_mult, k_dim, v_dim);
+    });
+    return swl::check_launch();
 }
 
 extern "C" int swl_diff_head_combine(void *out, const float *maps, const void *gate, int64_t gate_stride, float lambda,

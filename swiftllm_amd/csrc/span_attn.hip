@@ -87,26 +87,6 @@ __device__ __forceinline__ float span_row_sum(float v) {
     return v + __shfl_xor(v, 32, 64);
 }
 
-// N matrix steps whose operand comes from LDS, AHEAD of them on their way. (Left alone, the compiler reads every fragment right in
-// front of its step: a latency of LDS for each.)
-template <int AHEAD, int N, int MFMAS, typename V, typename Load, typename Step>
-__device__ __forceinline__ void span_steps(Load &&load, Step &&step) {
-    constexpr int R = AHEAD < N ? AHEAD : N;
-    V ring[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) ring[i] = load(i);
-    __builtin_amdgcn_sched_group_barrier(0x100, R, 0);      // LDS reads
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        step(i, ring[i % R]);
-        __builtin_amdgcn_sched_group_barrier(0x008, MFMAS, 0);      // matrix steps
-        if (i + R < N) {
-            ring[i % R] = load(i + R);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-    }
-}
-
 // The workgroup's place (at: along the spans, heaviest first; g: key head) from its number.
 //   * Runs of `run` workgroups, the queries of four neighbouring spans, see the same keys but for 128. Workgroups go round the eight XCDs
 //     by their number, so a run takes every eighth number: one XCD's L2 holds its keys once.
@@ -252,40 +232,7 @@ __device__ __forceinline__ void span_store(const __attribute__((address_space(4)
     }
 }
 
-// 1 KiB (16 bytes a lane) or 256 bytes (4 a lane) of `base` + the lane's `off` to the LDS address `to`
-__device__ __forceinline__ void span_ask16(const char *base, unsigned off, unsigned to) {
-    unsigned keep;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(off), "s"(base), "s"(to) : "memory");
-}
-// N KiB: lane offsets off[j] from `base`, LDS addresses `to` + 1024 j
-template <int N, int M>
-__device__ __forceinline__ void span_ask16s(const char *base, const unsigned (&off)[M], unsigned to) {
-    unsigned keep;
-#define SWL_ASK_FIRST "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %3, %2\n\t"
-#define SWL_ASK_NEXT(K) "s_add_u32 m0, m0, 0x400\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %" #K ", %2\n\t"
-#define SWL_ASK_LAST "s_mov_b32 m0, %0"
-    static_assert(N >= 1 && N <= 6 && N <= M, "");
-    if constexpr (N == 1)
-        asm volatile(SWL_ASK_FIRST SWL_ASK_LAST : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]) : "memory", "scc");
-    else if constexpr (N == 2)
-        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_LAST : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]) : "memory", "scc");
-    else if constexpr (N == 3)
-        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_NEXT(5) SWL_ASK_LAST
-                     : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]) : "memory", "scc");
-    else if constexpr (N == 4)
-        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_NEXT(5) SWL_ASK_NEXT(6) SWL_ASK_LAST
-                     : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]) : "memory", "scc");
-    else if constexpr (N == 5)
-        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_NEXT(5) SWL_ASK_NEXT(6) SWL_ASK_NEXT(7) SWL_ASK_LAST
-                     : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]) : "memory", "scc");
-    else
-        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_NEXT(5) SWL_ASK_NEXT(6) SWL_ASK_NEXT(7) SWL_ASK_NEXT(8) SWL_ASK_LAST
-                     : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]), "v"(off[5]) : "memory", "scc");
-#undef SWL_ASK_FIRST
-#undef SWL_ASK_NEXT
-#undef SWL_ASK_LAST
-}
+// 256 bytes (4 a lane) of `base` + the lane's `off` to the LDS address `to`
 __device__ __forceinline__ void span_ask4(const void *base, unsigned off, unsigned to) {
     unsigned keep;
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 4\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
@@ -416,12 +363,12 @@ __global__ __launch_bounds__(kSpanNarrowWaves * 64, 2) void span_attn_narrow_ker
     const unsigned to_keys = lds0 + static_cast<unsigned>(my_page * 16 * D * 2 + my_part * KA * 1024);
     const unsigned to_values = lds0 + 2 * KB + static_cast<unsigned>(my_page * 16 * DV * 2 + my_part * VA * 1024);
     auto ask_keys = [&](int stage) {
-        span_ask16s<KA>(kc + block(stage), src, to_keys + static_cast<unsigned>(stage & 1) * KB);
+        lds_ask<KA>(kc + block(stage), src, to_keys + static_cast<unsigned>(stage & 1) * KB);
     };
     // (REL) the wave's windows of its heads' bias, entry i: distance wp0 - (its first key of the stage) - (KW - 1) + i
     float *const rel_lds = reinterpret_cast<float *>(smem + 2 * BUF) + wave * HW * 64;       // [2][NW][HW][64]
     auto ask_values = [&](int stage) {
-        span_ask16s<VA>(vc + block(stage), vsrc, to_values + static_cast<unsigned>(stage & 1) * VB);
+        lds_ask<VA>(vc + block(stage), vsrc, to_values + static_cast<unsigned>(stage & 1) * VB);
         if constexpr (REL) {
             const int d = wp0 - (w.kb0 + stage * NP) * 16 - kh * KW - (KW - 1) + lane, head = (rg * 32) / qt;
             const unsigned off = static_cast<unsigned>(min(max(d, 0), p.rel_len - 1)) * 4,
@@ -467,7 +414,7 @@ __global__ __launch_bounds__(kSpanNarrowWaves * 64, 2) void span_attn_narrow_ker
     for (int e = 0; e < KS; ++e) asm volatile("" : "+v"(qf[e]));
     auto score = [&](int stage) {
         s = float16_t{};
-        span_steps<AHEAD, KS, 1, vec8_t<T>>([&](int e) { return key_at(stage, e); }, [&](int e, vec8_t<T> kf) { s = span_mfma(kf, qf[e], s); });
+        lds_steps<AHEAD, KS, 1, vec8_t<T>>([&](int e) { return key_at(stage, e); }, [&](int e, vec8_t<T> kf) { s = span_mfma(kf, qf[e], s); });
     };
     auto turn = [&](int st) {
         // this wave's pieces of the next keys and of these values have landed, its reads of what is overwritten now have returned
@@ -563,7 +510,7 @@ __global__ __launch_bounds__(kSpanNarrowWaves * 64, 2) void span_attn_narrow_ker
         }
         // (step i: keys 16 (i % 2) .., value tile i / 2)
         const char *vp = smem + 2 * KB + (st & 1) * VB + v_frag;
-        span_steps<AHEAD, 2 * CT, 2, vec8_t<T>>(
+        lds_steps<AHEAD, 2 * CT, 2, vec8_t<T>>(
             [&](int i) { return *reinterpret_cast<const vec8_t<T> *>(vp + (i & 1) * 16 * DV * 2 + (i >> 1) * 1024); },
             [&](int i, vec8_t<T> vf) {
                 acc[i >> 1] = span_mfma(vf, __builtin_bit_cast(vec8_t<T>, hi[i & 1]), acc[i >> 1]);
@@ -691,8 +638,8 @@ __global__ __launch_bounds__(kSpanWaves * 64, 2) void span_attn_kernel(SpanParam
         if constexpr (PARTS) {
             const int64_t blk = static_cast<int64_t>(__builtin_amdgcn_readlane(id_lane, stage * NP - id_base + my_page)) * bstride;
             const unsigned dst = my_dst + static_cast<unsigned>(stage & 1) * BUF;
-            if (PK == PV || my_keys) span_ask16s<PK>(my_base + blk, src, dst);
-            else span_ask16s<PV>(my_base + blk, src, dst);
+            if (PK == PV || my_keys) lds_ask<PK>(my_base + blk, src, dst);
+            else lds_ask<PV>(my_base + blk, src, dst);
         } else {
             const unsigned dst = lds0 + static_cast<unsigned>(stage & 1) * BUF;
 #pragma unroll
@@ -706,7 +653,7 @@ __global__ __launch_bounds__(kSpanWaves * 64, 2) void span_attn_kernel(SpanParam
                     const char *base = (key ? kc : vc + (u - KI) * 1024) + blk;
                     const unsigned off = page & 1 ? src[j] ^ (key ? kOddFlip * 16 : 0) : src[j];
                     const unsigned to = dst + static_cast<unsigned>(key ? page * 16 * D * 2 + u * 1024 : KB + page * 16 * DV * 2 + (u - KI) * 1024);
-                    span_ask16(base, off, to);
+                    lds_ask<1>(base, {off}, to);
                 }
             }
         }
@@ -757,7 +704,7 @@ __global__ __launch_bounds__(kSpanWaves * 64, 2) void span_attn_kernel(SpanParam
 #pragma unroll
         for (int t = 0; t < NT; ++t) s[t] = float4_t{0.f, 0.f, 0.f, 0.f};
         // (step i: score tile i % NT, elements 32 (i / NT) ..)
-        span_steps<AHEAD, NT * KS, 1, vec8_t<T>>(
+        lds_steps<AHEAD, NT * KS, 1, vec8_t<T>>(
             [&](int i) { return *reinterpret_cast<const vec8_t<T> *>(kbuf + k_frag[i % NT][(i / NT) % KF] + (i / NT) / KF * KF * 64); },
             [&](int i, vec8_t<T> kf) { s[i % NT] = mfma_step(kf, qf[i / NT], s[i % NT]); });
         mfma_results_tie(s[0]);
@@ -801,7 +748,7 @@ __global__ __launch_bounds__(kSpanWaves * 64, 2) void span_attn_kernel(SpanParam
         vec8_t<T> hi, lo;
         split_weights<T>(x, hi, lo);
         const char *vp = vbuf + v_frag;
-        span_steps<AHEAD, CT, 2, vec8_t<T>>([&](int ct) { return *reinterpret_cast<const vec8_t<T> *>(vp + ct * 512); },
+        lds_steps<AHEAD, CT, 2, vec8_t<T>>([&](int ct) { return *reinterpret_cast<const vec8_t<T> *>(vp + ct * 512); },
                                             [&](int ct, vec8_t<T> vf) {
                                                 acc[ct] = mfma_step(vf, hi, acc[ct]);
                                                 acc[ct] = mfma_step(vf, lo, acc[ct]);

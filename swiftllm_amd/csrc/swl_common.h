@@ -299,6 +299,55 @@ __device__ __forceinline__ void load4(vec4_t<T> &dst, const T *p) {    // 8-byte
 }
 
 
+// LDS-DMA of N KiB, 16 bytes a lane: lane offsets off[j] from `base`, LDS addresses `to` + 1024 j. Not waited for: the compiler knows nothing of it
+// (s_waitcnt vmcnt in asm). One asm for all of them, so that M0 is set aside once and goes on by additions.
+template <int N, int M>
+__device__ __forceinline__ void lds_ask(const char *base, const unsigned (&off)[M], unsigned to) {
+    unsigned keep;
+#define SWL_ASK_FIRST "s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %3, %2\n\t"
+#define SWL_ASK_NEXT(K) "s_add_u32 m0, m0, 0x400\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %" #K ", %2\n\t"
+#define SWL_ASK_LAST "s_mov_b32 m0, %0"
+    static_assert(N >= 1 && N <= 6 && N <= M, "");
+    if constexpr (N == 1)
+        asm volatile(SWL_ASK_FIRST SWL_ASK_LAST : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]) : "memory", "scc");
+    else if constexpr (N == 2)
+        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_LAST : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]) : "memory", "scc");
+    else if constexpr (N == 3)
+        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_NEXT(5) SWL_ASK_LAST
+                     : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]) : "memory", "scc");
+    else if constexpr (N == 4)
+        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_NEXT(5) SWL_ASK_NEXT(6) SWL_ASK_LAST
+                     : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]) : "memory", "scc");
+    else if constexpr (N == 5)
+        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_NEXT(5) SWL_ASK_NEXT(6) SWL_ASK_NEXT(7) SWL_ASK_LAST
+                     : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]) : "memory", "scc");
+    else
+        asm volatile(SWL_ASK_FIRST SWL_ASK_NEXT(4) SWL_ASK_NEXT(5) SWL_ASK_NEXT(6) SWL_ASK_NEXT(7) SWL_ASK_NEXT(8) SWL_ASK_LAST
+                     : "=&s"(keep) : "s"(to), "s"(base), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "v"(off[4]), "v"(off[5]) : "memory", "scc");
+#undef SWL_ASK_FIRST
+#undef SWL_ASK_NEXT
+#undef SWL_ASK_LAST
+}
+// N matrix steps whose operand comes from LDS, AHEAD of them on their way. (Left alone, the compiler reads every fragment right in
+// front of its step: a latency of LDS for each.)
+template <int AHEAD, int N, int MFMAS, typename V, typename Load, typename Step>
+__device__ __forceinline__ void lds_steps(Load &&load, Step &&step) {
+    constexpr int R = AHEAD < N ? AHEAD : N;
+    V ring[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) ring[i] = load(i);
+    __builtin_amdgcn_sched_group_barrier(0x100, R, 0);      // LDS reads
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        step(i, ring[i % R]);
+        __builtin_amdgcn_sched_group_barrier(0x008, MFMAS, 0);      // matrix steps
+        if (i + R < N) {
+            ring[i % R] = load(i + R);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+    }
+}
+
 // exp2 on the hardware transcendental unit (v_exp_f32 IS 2^x).
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }

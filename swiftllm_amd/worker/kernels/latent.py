@@ -1,12 +1,13 @@
 """Latent attention of a step: which rows run on the heads' own keys and values, expanded from the cached rows
-(csrc/latent_expand.hip), and which on queries folded through the key up-projection."""
+(csrc/latent_expand.hip), and which on queries folded through the key up-projection — single tokens in three launches of their own
+(csrc/latent_decode.hip)."""
 import torch
 
 from swiftllm_amd import _hip
 
 from ..batch_plan import LatentExpansion
-from .rope_kv import latent_rope_and_store_kv
-from .window_attn import MASK_WINDOW, AttentionSpec, PoolSlice, StepTiles, masked_attention
+from .rope_kv import head_gate_, latent_rope_and_store_kv
+from .window_attn import MASK_WINDOW, SHARE_MAX_SCRATCH, AttentionSpec, PoolSlice, StepTiles, choose_key_splits, masked_attention
 
 # A layer's expanded pages take at most this much (which memory profiling sets aside: its step runs without a pool); portions past it stay
 # folded. 8192 tokens of 16 heads of 128 + 64 and 128 columns take 80 MiB.
@@ -61,41 +62,93 @@ def expansion_served(mx, k_dim: int, dtype: torch.dtype) -> bool:
                 and lib.swl_span_attn_supported(H, H, H, mx.head_dim + mx.rot_dim, mx.value_dim, 0, code))
 
 
+# Steps of up to this many tokens fold their queries beside the rotary and the store (one launch; the matrices are read once, a wave walks over
+# the tokens); more go through a batched library product.
+FOLD_MAX_TOKENS = 64
+
+
 class LatentAttention:
-    """The attention of a latent layer from its projected rows [query heads (dim | rot_dim) | ...] to the heads' results. spec: the folded
-    attention (one key row of kv_rank + rot_dim and one value row of kv_rank for all heads)."""
+    """The attention of a latent layer from its projected rows [query heads (dim | rot_dim) | ...] to the heads' gated results. spec: the
+    folded attention (one key row of kv_rank + rot_dim and one value row of kv_rank for all heads).
+
+    Single tokens, us of 32 at 1024 keys, 16 heads of 128 over rank 512 + 64, from the projection to the gated results: rotary and store 5.5, two
+    batched products 4.2 and 9.2, attention of csrc/window_attn_mfma.hip 26, its combining launch 6.3, gate 4.7: 56; by csrc/latent_decode.hip
+    6.6, 15.8 and 7.8: 30."""
 
     def __init__(self, mixer, weight, spec: AttentionSpec, eps: float, pool_slice, max_positions: int, dkv_col: int):
         self.mixer, self.w, self.spec, self.eps, self.pool_slice, self.max_positions = mixer, weight, spec, eps, pool_slice, max_positions
         self.dkv_col = dkv_col
-        H = mixer.num_q_heads
+        H, dtype = mixer.num_q_heads, weight.uk.dtype
         self.heads_spec = AttentionSpec(H, H, mixer.head_dim + mixer.rot_dim, mixer.value_dim, spec.scale, window=spec.window,
                                         mask_kind=MASK_WINDOW, sink=spec.sink)
-        self.served = expansion_served(mixer, spec.head_dim, weight.uk.dtype)
+        self.expands = expansion_served(mixer, spec.head_dim, dtype)
+        self.decodes = self.folds = False
+        if dtype != torch.float32:
+            lib, code = _hip.load(), _hip.dtype_code(dtype)
+            self.decodes = bool(lib.swl_latent_decode_supported(mixer.kv_rank, mixer.rot_dim, spec.head_dim, mixer.value_dim, code))
+            self.folds = bool(lib.swl_latent_fold_supported(mixer.head_dim, mixer.rot_dim, mixer.kv_rank, spec.head_dim, code))
 
-    def __call__(self, proj: torch.Tensor, ctx) -> torch.Tensor:
+    def __call__(self, proj: torch.Tensor, gate: torch.Tensor, ctx) -> torch.Tensor:
+        """gate: [T, heads] logits, a column slice of the projected rows."""
         mx, w, sp = self.mixer, self.w, self.spec
         n, H, d, dr, r, e = proj.shape[0], mx.num_q_heads, mx.head_dim, mx.rot_dim, mx.kv_rank, mx.value_dim
-        ex = ctx.expanded if self.served and ctx.pool is not None and ctx.pool.shape[1] % 8 == 0 and self.pool_slice.k_offset % 8 == 0 else None
+        aligned = ctx.pool is not None and ctx.pool.shape[1] % 8 == 0 and self.pool_slice.k_offset % 8 == 0      # 16-byte loads of cached rows
+        ex = ctx.expanded if self.expands and aligned else None
         m = ex.rows if ex is not None else 0
+        tiles = ex.rest if m else ctx.tiles
+        single = self.decodes and aligned and m < n and tiles is not None and tiles[0].shape[0] == n - m and \
+            (n - m) * H * (r + 2) * 4 <= SHARE_MAX_SCRATCH
         qa = torch.empty((n - m, H * sp.head_dim), dtype=proj.dtype, device=proj.device)
-        latent_rope_and_store_kv(proj, qa, w.freq, w.c_norm, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq,
-                                 ctx.tok_pos, mx, self.dkv_col, self.eps, sp.head_dim, sp.value_dim, in_place=m)
+        folded = single and m == 0 and self.folds and n <= FOLD_MAX_TOKENS and proj.data_ptr() % 16 == 0 and proj.stride(0) % 8 == 0
+        if folded:
+            self._fold(proj, qa, ctx)
+        else:
+            latent_rope_and_store_kv(proj, qa, w.freq, w.c_norm, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq,
+                                     ctx.tok_pos, mx, self.dkv_col, self.eps, sp.head_dim, sp.value_dim, in_place=m)
         y = torch.empty((n, H * e), dtype=proj.dtype, device=proj.device)
         if m:
             self._expanded(proj, y[:m], ctx, ex)
         if m < n:
             rows = slice(m, n)
-            # q_abs[t, h, :] = W_uk,h^T q_unrotated[t, h, :]  -> the first kv_rank columns of every head of qa
-            qn = proj[rows, :H * (d + dr)].view(n - m, H, d + dr)[:, :, :d].transpose(0, 1)       # [H, T, d]
-            torch.bmm(qn, w.uk, out=qa.view(n - m, H, sp.head_dim)[:, :, :r].transpose(0, 1))   # (a strided batched product: no copy)
+            if not folded:
+                # q_abs[t, h, :] = W_uk,h^T q_unrotated[t, h, :]  -> the first kv_rank columns of every head of qa
+                qn = proj[rows, :H * (d + dr)].view(n - m, H, d + dr)[:, :, :d].transpose(0, 1)       # [H, T, d]
+                torch.bmm(qn, w.uk, out=qa.view(n - m, H, sp.head_dim)[:, :, :r].transpose(0, 1))   # (a strided batched product: no copy)
+            if single:
+                self._single(qa, y[rows], gate[rows], ctx, rows)
+                if m:
+                    head_gate_(y[:m], gate[:m], H, e)
+                return y
             if ctx.pool is None:    # memory profiling: the attention's output buffer without its reads
                 att = torch.zeros((n - m, H * sp.value_dim), dtype=proj.dtype, device=proj.device)
             else:
                 att = masked_attention(qa, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq[rows], ctx.tok_pos[rows], sp,
-                                       ex.rest if m else ctx.tiles, self.max_positions)
+                                       tiles, self.max_positions)
             torch.bmm(att.view(n - m, H, sp.value_dim)[:, :, :r].transpose(0, 1), w.uv_t, out=y[rows].view(n - m, H, e).transpose(0, 1))
-        return y
+        return head_gate_(y, gate, H, e)
+
+    def _fold(self, proj, qa, ctx):
+        mx, w, sp, esize = self.mixer, self.w, self.spec, proj.element_size()
+        own = self.dkv_col >= 0
+        kp, vp = (ctx.pool.data_ptr() + off * esize if own else 0 for off in (self.pool_slice.k_offset, self.pool_slice.v_offset))
+        _hip.call("swl_latent_fold", _hip.ptr(proj), _hip.ptr(qa), _hip.ptr(w.uk_t), _hip.ptr(w.freq), _hip.ptr(w.c_norm), kp, vp,
+                  _hip.ptr(ctx.block_table), _hip.ptr(ctx.tok_seq), _hip.ptr(ctx.tok_pos), proj.shape[0], mx.num_q_heads, mx.head_dim,
+                  mx.rot_dim, mx.kv_rank, proj.stride(0), self.dkv_col if own else -1, qa.stride(0), ctx.block_table.shape[1],
+                  ctx.pool.shape[1], float(self.eps), 1 if mx.rot.half else 0, float(mx.rot.multiplier), sp.head_dim, sp.value_dim,
+                  _hip.dtype_code(proj.dtype), _hip.stream())
+
+    def _single(self, qa, y, gate, ctx, rows):
+        mx, w, sp = self.mixer, self.w, self.spec
+        n, H, code = qa.shape[0], mx.num_q_heads, _hip.dtype_code(qa.dtype)
+        # (of the counts and the model alone: a captured step stays valid)
+        floats = n * H * (mx.kv_rank + 2)
+        shares = max(1, min(choose_key_splits(n * -(-H // 16), sp, self.max_positions), SHARE_MAX_SCRATCH // (4 * floats)))
+        scratch = torch.empty(shares * floats, dtype=torch.float32, device=qa.device)
+        _hip.call("swl_latent_decode", _hip.ptr(scratch), _hip.ptr(qa), ctx.pool.data_ptr() + self.pool_slice.k_offset * qa.element_size(),
+                  _hip.ptr(ctx.block_table), _hip.ptr(ctx.tok_seq[rows]), _hip.ptr(ctx.tok_pos[rows]), n, H, qa.stride(0), sp.window,
+                  float(sp.scale), ctx.block_table.shape[1], ctx.pool.shape[1], shares, code, _hip.stream())
+        _hip.call("swl_latent_unfold", _hip.ptr(y), _hip.ptr(scratch), _hip.ptr(w.uv), _hip.ptr(sp.sink), _hip.ptr(gate), gate.stride(0), n, H,
+                  mx.value_dim, shares, code, _hip.stream())
 
     def _expanded(self, proj, out, ctx, ex: ExpandedStep):
         mx, w, sp, hs = self.mixer, self.w, self.spec, self.heads_spec

@@ -44,7 +44,7 @@ class RokevikAttention:
 
 class RokevikLatentAttention:
     """(q | compressed kv | gate) projection -> rotary, latent norm and cache store -> attention over the cached rows inside the
-    window, expanded or folded (kernels/latent.py) -> head gate -> output projection."""
+    window, expanded or folded, and head gate (kernels/latent.py) -> output projection."""
 
     def __init__(self, layer_config, weight, eps: float, skinny: bool, pool_slice, max_positions: int, row_sizes):
         mx = self.mixer = layer_config.mixer
@@ -56,8 +56,7 @@ class RokevikLatentAttention:
     def forward(self, h: torch.Tensor, ctx: StepContext):
         mx, w = self.mixer, self.w
         proj = _project(h, w.proj, self.skinny)
-        y = self.attend(proj, ctx)
-        head_gate_(y, proj[:, w.gate_col:w.gate_col + mx.num_q_heads], mx.num_q_heads, mx.value_dim)
+        y = self.attend(proj, proj[:, w.gate_col:w.gate_col + mx.num_q_heads], ctx)
         return _project(y, w.o, self.skinny), None
 
 

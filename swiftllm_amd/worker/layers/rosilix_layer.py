@@ -5,7 +5,7 @@ import torch
 from ..kernels.latent import LatentAttention
 from ..kernels.linear import ROWS_MAX_TOKENS, linear_rows
 from ..kernels.moe import relu_squared
-from ..kernels.rope_kv import diff_head_combine, head_gate_, rope_and_store_kv
+from ..kernels.rope_kv import diff_head_combine, rope_and_store_kv
 from ..kernels.window_attn import MASK_CHUNK, MASK_WINDOW, AttentionSpec, masked_attention
 from .kekapel_layer import _project, _project_partials
 from .lorulix_layer import StepContext
@@ -39,7 +39,7 @@ class RosilixDiffAttention:
 
 class RosilixLatentAttention:
     """(q | compressed kv | gate) projection -> rotary, latent norm and cache store -> attention over the cached rows with the heads'
-    sinks, expanded or folded (kernels/latent.py) -> head gate -> output projection. A layer that reads another layer's cache
+    sinks, expanded or folded, and head gate (kernels/latent.py) -> output projection. A layer that reads another layer's cache
     projects queries and gates only."""
 
     def __init__(self, layer_config, weight, eps: float, skinny: bool, pool_slice, max_positions: int):
@@ -52,8 +52,7 @@ class RosilixLatentAttention:
     def forward(self, h: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         mx, w = self.mixer, self.w
         proj = _project(h, w.proj, self.skinny)
-        y = self.attend(proj, ctx)
-        head_gate_(y, proj[:, w.gate_col:w.gate_col + mx.num_q_heads], mx.num_q_heads, mx.value_dim)
+        y = self.attend(proj, proj[:, w.gate_col:w.gate_col + mx.num_q_heads], ctx)
         return _project_partials(y, w.o, self.skinny)
 
 

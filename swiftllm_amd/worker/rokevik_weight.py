@@ -64,6 +64,7 @@ class RokevikLayerWeight:
             self.gate_col = mx.q_size + mx.dkv_size
             self.c_norm = f32("mix.dkv.norm", (mx.kv_rank,))
             self.uk = mat("mix.uk", (H * mx.head_dim, mx.kv_rank)).view(H, mx.head_dim, mx.kv_rank).contiguous()
+            self.uk_t = self.uk.transpose(1, 2).contiguous()
             self.uv = mat("mix.uv", (H * mx.value_dim, mx.kv_rank)).view(H, mx.value_dim, mx.kv_rank).contiguous()
             self.uv_t = self.uv.transpose(1, 2).contiguous()
             self.o = mat("mix.o", (w, mx.o_size))

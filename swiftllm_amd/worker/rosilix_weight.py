@@ -71,6 +71,7 @@ class RosilixLayerWeight:
             parts.append(mat("mix.g", (H, w)))
             self.proj = _pad_rows(torch.cat(parts, dim=0))
             self.uk = mat("mix.uk", (H * mx.head_dim, mx.kv_rank)).view(H, mx.head_dim, mx.kv_rank).contiguous()
+            self.uk_t = self.uk.transpose(1, 2).contiguous()
             self.uv = mat("mix.uv", (H * mx.value_dim, mx.kv_rank)).view(H, mx.value_dim, mx.kv_rank).contiguous()
             self.uv_t = self.uv.transpose(1, 2).contiguous()
             self.sink = f32("mix.sink", (H,))

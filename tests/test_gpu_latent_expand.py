@@ -63,15 +63,30 @@ def _step(parts, window, max_pages=1 << 20):
                                         ([(0, 0, 128), (1, 40, 5), (2, 0, 64)], 128), ([(0, 60, 1), (1, 0, 64)], 0)])
 def test_steps(parts, rows, window, sink, half, dtype):
     """Whatever rows are expanded, the results are those of 64-bit attention on the cached rows."""
+    check_step(parts, rows, window, sink, half, dtype, 4, 128)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("window,sink,half,H,e", [(0, True, False, 16, 128), (70, False, True, 8, 128), (0, False, True, 20, 64), (33, True, True, 3, 272)])
+@pytest.mark.parametrize("parts", [[(2, 0, 1)], [(1, 15, 1), (0, 16, 1), (3, 17, 1)], [(s, (37 * s) % 300, 1) for s in range(20)],
+                                   [(s, 5 + 9 * s, 1) for s in range(33)], [(0, 4500, 1), (1, 3000, 1)], [(0, 0, 40), (1, 99, 1), (2, 250, 1)],
+                                   [(s, s, 1) for s in range(70)]])
+def test_single_tokens(parts, window, sink, half, H, e, dtype):
+    """Steps of single tokens, and behind expanded portions (csrc/latent_decode.hip): shares with and without keys, one page and more than one
+    load of page ids holds, tokens and heads around the kernels' groups of 8 and 16, and more tokens than are folded beside the rotary."""
+    check_step(parts, sum(n for _, _, n in parts if n > 1), window, sink, half, dtype, H, e)
+
+
+def check_step(parts, rows, window, sink, half, dtype, H, e):
     from swiftllm_amd.worker.kernels.latent import ExpandedStep, LatentAttention
     from swiftllm_amd.worker.kernels.window_attn import AttentionSpec, PoolSlice, StepTiles
     g = torch.Generator().manual_seed(rows + window)
-    H, d, dr, e, r = 4, 128, 64, 128, 512
+    d, dr, r = 128, 64, 512
     mx = SimpleNamespace(num_q_heads=H, head_dim=d, rot_dim=dr, value_dim=e, kv_rank=r, window=window,
                          rot=SimpleNamespace(dims=dr, half=half, multiplier=1.0))
     uk, uv = (torch.randn(H, n, r, generator=g).div(math.sqrt(r)).to(dtype) for n in (d, e))
     freq = 10000.0 ** (-torch.arange(0, dr, 2, dtype=torch.float64) / dr)
-    w = SimpleNamespace(uk=uk.cuda(), uv=uv.cuda(), uv_t=uv.transpose(1, 2).contiguous().cuda(), freq=freq.cuda(),
+    w = SimpleNamespace(uk=uk.cuda(), uk_t=uk.transpose(1, 2).contiguous().cuda(), uv=uv.cuda(), uv_t=uv.transpose(1, 2).contiguous().cuda(), freq=freq.cuda(),
                         c_norm=torch.ones(r, device="cuda"))
     sinks = torch.randn(H, generator=g) if sink else None
     spec = AttentionSpec(H, 1, r + dr, r, (d + dr) ** -0.5, window=window, sink=sinks.cuda() if sink else None)
@@ -79,25 +94,30 @@ def test_steps(parts, rows, window, sink, half, dtype):
     ex = ExpandedStep.of(dev)
     assert (ex.rows if ex else 0) == rows
     # earlier tokens' rows in shuffled blocks, stale rows behind the ends
-    blocks, block = torch.randperm(64, generator=g), 16 * (2 * r + dr)
-    pool = torch.randn(64, block, generator=g).to(dtype)
-    pool[:, 16 * (r + dr):] = pool[:, :16 * (r + dr)].view(64, 16, r + dr)[:, :, :r].transpose(1, 2).reshape(64, -1)
-    table = torch.zeros(4, 22, dtype=torch.int32)
+    total = sum(-(-(a + n) // 16) for _, a, n in parts) + 2
+    blocks, block = torch.randperm(total, generator=g), 16 * (2 * r + dr)
+    pool = torch.randn(total, block, generator=g).to(dtype)
+    pool[:, 16 * (r + dr):] = pool[:, :16 * (r + dr)].view(total, 16, r + dr)[:, :, :r].transpose(1, 2).reshape(total, -1)
+    table = torch.zeros(max(s for s, _, _ in parts) + 1, max(-(-(a + n) // 16) for _, a, n in parts) + 1, dtype=torch.int32)
     at = 0
     for s, a, n in parts:
         pages = -(-(a + n) // 16)
         table[s, :pages] = blocks[at:at + pages]
         at += pages
     n = plan.num_tokens
-    rows_in = torch.randn(n, H * (d + dr) + r + dr + 16, generator=g).to(dtype)
+    gate_col = H * (d + dr) + r + dr
+    rows_in = torch.randn(n, -(-(gate_col + H) // 8) * 8, generator=g).to(dtype)
     pool_dev, proj = pool.cuda(), rows_in.cuda()
     ctx = SimpleNamespace(pool=pool_dev, block_table=table.cuda(), tok_seq=dev["tok_seq"], tok_pos=dev["tok_pos"], tiles=StepTiles.of(dev),
                           expanded=ex)
-    attend = LatentAttention(mx, w, spec, 1e-6, PoolSlice(0, 16 * (r + dr)), 4096, H * (d + dr))
-    got = attend(proj, ctx).cpu().double()
+    attend = LatentAttention(mx, w, spec, 1e-6, PoolSlice(0, 16 * (r + dr)), 8192, H * (d + dr))
+    got = attend(proj, proj[:, gate_col:gate_col + H], ctx).cpu().double()
     pool = pool_dev.cpu()
     folded_rows = SimpleNamespace(**{**ctx.__dict__, "expanded": None})
-    folded = attend(rows_in.cuda(), folded_rows).cpu().double()
+    other = LatentAttention(mx, w, spec, 1e-6, PoolSlice(0, 16 * (r + dr)), 8192, H * (d + dr))
+    other.decodes = False
+    proj = rows_in.cuda()
+    folded = other(proj, proj[:, gate_col:gate_col + H], folded_rows).cpu().double()
     row = 0
     worst, worst_folded = 0.0, 0.0
     for s, a, cnt in parts:
@@ -117,7 +137,8 @@ def test_steps(parts, rows, window, sink, half, dtype):
         sc = sc.masked_fill(~see, -math.inf)
         if sink:
             sc = torch.cat((sc, sinks.double()[:, None, None].expand(H, cnt, 1)), 2)
-        want = torch.einsum("hqk,hke->qhe", torch.softmax(sc, 2)[:, :, :a + cnt], v).reshape(cnt, -1)
+        want = torch.einsum("hqk,hke->qhe", torch.softmax(sc, 2)[:, :, :a + cnt], v)
+        want = (want * torch.sigmoid(rows_in[row:row + cnt, gate_col:gate_col + H].double())[:, :, None]).reshape(cnt, -1)
         # a key's and a value's products are rounded once (as folded queries and latent results are): scores move by sqrt(d) of such
         # roundings of |q| |k| ~ 1, results by one of the largest |v| ~ 4, and by what the scores' weights move
         bound = 24 * UNIT[dtype]
