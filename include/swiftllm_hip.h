@@ -806,6 +806,14 @@ int swl_gated_add_rmsnorm(float *x, const void *m, const void *m2, const void *m
 int swl_gated_add_rmsnorm_parts(float *x, const float *slabs, int32_t parts, const void *m2, const void *m2_gate, int64_t m2_gate_stride,
                                 const void *r, int64_t r_stride, const float *r_bias, const float *w1, void *out, const float *w2,
                                 float eps, int64_t num_rows, int32_t width, int32_t dtype, swl_stream_t stream);
+/* Either of the two (m or slabs, or neither) for a step of one token a sequence, which also leaves sum = out + the causal convolution of out
+ * (swl_causal_conv_state with add_input) and the carried inputs. At most 4 taps and 4096 columns, width % 4 == 0, 16-byte aligned rows and
+ * state (slot_stride, tail_off % 4 == 0); anything else is SWL_ERR_UNSUPPORTED. */
+int swl_gated_add_rmsnorm_conv(float *x, const void *m, const float *slabs, int32_t parts, const void *m2, const void *m2_gate,
+                               int64_t m2_gate_stride, const void *r, int64_t r_stride, const float *r_bias, const float *w1, void *out,
+                               const float *w2, void *sum, const float *conv_w, int32_t taps, float *state, int64_t slot_stride,
+                               int64_t tail_off, const int32_t *tok_pos, const int32_t *tok_state, float eps, int64_t num_rows,
+                               int32_t width, int32_t dtype, swl_stream_t stream);
 int swl_causal_conv_state(void *out, int64_t out_stride, const void *h, int64_t h_stride, const float *w, float *state,
                           int64_t slot_stride, int64_t tail_off, const int32_t *tok_pos, const int32_t *tok_start,
                           const int32_t *tok_state, const int32_t *tok_seq, int64_t num_tokens, int32_t channels,

@@ -150,6 +150,8 @@ SIGNATURES = {
                                  _F32, _I32, _I32, _P],
     "swl_gated_add_rmsnorm": [_P, _P, _P, _P, _I64, _P, _I64, _P, _P, _P, _P, _P, _F32, _I64, _I32, _I32, _P],
     "swl_gated_add_rmsnorm_parts": [_P, _P, _I32, _P, _P, _I64, _P, _I64, _P, _P, _P, _P, _F32, _I64, _I32, _I32, _P],
+    "swl_gated_add_rmsnorm_conv": [_P, _P, _P, _I32, _P, _P, _I64, _P, _I64, _P, _P, _P, _P, _P, _P, _I32, _P, _I64, _I64, _P, _P, _F32, _I64,
+                                   _I32, _I32, _P],
     "swl_causal_conv_state": [_P, _I64, _P, _I64, _P, _P, _I64, _I64, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _P],
     "swl_delta_prep": [_P, _P, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P, _I64, _I32, _I32, _I32,
                        _I32, _I32, _I32, _P],

@@ -10,6 +10,9 @@
 //     add them up is saved, and their rounding to the compute dtype with it.
 //     Statistics, gates and the sum are fp32; m, m2, s, r and out are the compute dtype. Weights arrive as the factor itself
 //     (a loader that stores "weight around zero" adds the one).
+//     swl_gated_add_rmsnorm_conv, for steps of one token a sequence: the next sublayer's input convolution in the same launch. The row it
+//     convolves is in registers, what came before it in the state slot, asked for with the stream's. A step's latency is a chain of
+//     launches: 3 tokens x 1024 columns of 3 taps in fp32, the two launches of each of 8 sublayers 64 -> 46 us a step of 402 -> 384.
 //   swl_post_norm_add: the same step for models whose sublayers read the stream itself (norm on the sublayer's RESULT only):
 //       y   = c * (a' + b')      a' = a / rms(a) * wa when wa is given, else a; b' likewise (b optional)
 //       x  += y / rms(y) * w1
@@ -82,10 +85,22 @@ __global__ __launch_bounds__(kRsThreads) void gated_add_rmsnorm_kernel(
     for (int i = threadIdx.x; i < width; i += kRsThreads) out[o * width + i] = to_t<T>(row[i] * rstd * w2[i]);
 }
 
-template <typename T, int TPR, int NV>
+// What a step of one token a sequence needs to convolve its rows where they are normed: tails and taps as swl_causal_conv_state's.
+struct ConvStep {
+    float *state;
+    int64_t slot_stride, tail_off;
+    const float *w;
+    const int32_t *tok_pos, *tok_state;
+    int taps;
+};
+constexpr int kConvStepTaps = 4;
+
+// NC: 0, or kConvStepTaps: `sum` receives out + its causal convolution. The earlier inputs and the taps are asked for first, so that they
+// come while the row is normed.
+template <typename T, int TPR, int NV, int NC>
 __global__ __launch_bounds__(kRowThreads) void gated_add_rmsnorm_wide_kernel(
     float *x, const T *m, const float *slabs, int parts, int64_t slab_stride, const T *m2, const T *m2_gate, int64_t m2_gate_stride, const T *r, int64_t r_stride,
-    const float *r_bias, const float *w1, T *out, const float *w2, const int32_t *row_idx, float eps, int64_t rows, int width) {
+    const float *r_bias, const float *w1, T *out, const float *w2, const int32_t *row_idx, float eps, int64_t rows, int width, T *sum, ConvStep conv) {
     __shared__ float red[2][kRowThreads / 64];
     const int64_t id = static_cast<int64_t>(blockIdx.x) * (kRowThreads / TPR) + threadIdx.x / TPR, o = min(id, rows - 1);
     const bool live = id < rows;
@@ -98,6 +113,36 @@ __global__ __launch_bounds__(kRowThreads) void gated_add_rmsnorm_wide_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[j][e] = 0.f;
         if (c0 + 4 * TPR * j < width) row_load<float>(v[j], xr + c0 + 4 * TPR * j);
+    }
+    constexpr int MOST = NC > 0 ? NC - 1 : 1;
+    float past[MOST][NV][4], taps[MOST + 1][NV][4];     // past[k - 1], taps[k]: the input k tokens back and its weights
+    const int R = NC > 0 ? conv.taps - 1 : 0;
+    float *new_tail = nullptr;
+    int pos = 0;
+    if constexpr (NC > 0) {
+        pos = conv.tok_pos[o];
+        const float *old_tail = nullptr;
+        if (R > 0) {
+            const int code = conv.tok_state[o];
+            float *base = conv.state + static_cast<int64_t>(code >> 1) * conv.slot_stride + conv.tail_off;
+            old_tail = base + static_cast<int64_t>(code & 1) * R * width;
+            new_tail = base + static_cast<int64_t>(1 - (code & 1)) * R * width;
+        }
+#pragma unroll
+        for (int k = 0; k <= MOST; ++k)
+#pragma unroll
+            for (int j = 0; j < NV; ++j) {
+                const int c = c0 + 4 * TPR * j;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    taps[k][j][e] = 0.f;
+                    if (k > 0) past[k > 0 ? k - 1 : 0][j][e] = 0.f;
+                }
+                if (k <= R && c < width) {
+                    row_load<float>(taps[k][j], conv.w + static_cast<int64_t>(R - k) * width + c);
+                    if (k > 0 && pos >= k) row_load<float>(past[k > 0 ? k - 1 : 0][j], old_tail + static_cast<int64_t>(R - k) * width + c);
+                }
+            }
     }
     if (m || slabs) {
         float y[NV][4], a2[NV][4], rv[NV][4];
@@ -155,7 +200,42 @@ __global__ __launch_bounds__(kRowThreads) void gated_add_rmsnorm_wide_kernel(
             row_load<float>(w, w2 + c);
 #pragma unroll
             for (int e = 0; e < 4; ++e) w[e] = v[j][e] * rstd * w[e];
-            row_store<T>(out + o * width + c, w);
+            if constexpr (NC == 0) {
+                row_store<T>(out + o * width + c, w);
+            } else {
+                // (one rounding for the row, the sum and the tail: left alone the compiler rounds the product to fp16 in one step for one
+                // of them and in two for the others)
+                typedef int Bits __attribute__((ext_vector_type(sizeof(T))));
+                vec4_t<T> x;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = to_t<T>(w[e]);
+                Bits bits = __builtin_bit_cast(Bits, x);
+                asm volatile("" : "+v"(bits));
+                x = __builtin_bit_cast(vec4_t<T>, bits);
+                *reinterpret_cast<vec4_t<T> *>(out + o * width + c) = x;
+                float cur[4], y[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    cur[e] = to_f(x[e]);
+                    y[e] = 0.f;
+                }
+#pragma unroll
+                for (int k = MOST; k >= 1; --k) {
+                    if (k <= R) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) y[e] += taps[k][j][e] * past[k - 1][j][e];
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    y[e] += taps[0][j][e] * cur[e];
+                    y[e] += cur[e];
+                }
+                row_store<T>(sum + o * width + c, y);
+#pragma unroll
+                for (int k = 0; k < MOST; ++k)      // (the input k tokens back becomes entry R - 1 - k)
+                    if (k < R && pos >= k) row_store<float>(new_tail + static_cast<int64_t>(R - 1 - k) * width + c, k == 0 ? cur : past[k > 0 ? k - 1 : 0][j]);
+            }
         }
     }
 }
@@ -369,7 +449,7 @@ inline size_t rs_lds_bytes(int width) { return (static_cast<size_t>(width) + kRs
 static int gated_add_rmsnorm(float *x, const void *m, const float *slabs, int parts, const void *m2, const void *m2_gate, int64_t m2_gate_stride,
                                      const void *r, int64_t r_stride, const float *r_bias, const float *w1, void *out,
                                      const float *w2, const int32_t *row_idx, float eps, int64_t num_rows, int32_t width,
-                                     int32_t dtype, swl_stream_t stream) {
+                                     int32_t dtype, swl_stream_t stream, void *sum = nullptr, const swl::ConvStep &conv = {}) {
     if (num_rows < 0 || width <= 0) return SWL_ERR_BAD_ARG;
     if (num_rows == 0) return SWL_OK;
     if (!x || ((m || slabs) && !w1) || (m2 && ((!m && !slabs) || !m2_gate)) || (r && ((!m && !slabs) || !r_bias)) || (out && !w2) ||
@@ -377,16 +457,26 @@ static int gated_add_rmsnorm(float *x, const void *m, const float *slabs, int pa
         return SWL_ERR_BAD_ARG;
     if (!m && !slabs && !out) return SWL_OK;
     if (num_rows > 0x7fffffffLL || swl::rs_lds_bytes(width) > 64 * 1024) return SWL_ERR_UNSUPPORTED;
-#define SWL_GO(TPR, NV)                                                                                                                \
-    hipLaunchKernelGGL((swl::gated_add_rmsnorm_wide_kernel<T, TPR, NV>), dim3(static_cast<unsigned>((num_rows * TPR + 255) / 256)),    \
+#define SWL_GO_NC(TPR, NV, NC)                                                                                                         \
+    hipLaunchKernelGGL((swl::gated_add_rmsnorm_wide_kernel<T, TPR, NV, NC>), dim3(static_cast<unsigned>((num_rows * TPR + 255) / 256)),    \
                        dim3(swl::kRowThreads), 0, static_cast<hipStream_t>(stream), x, static_cast<const T *>(m), slabs, parts,        \
                        num_rows * width, static_cast<const T *>(m2), static_cast<const T *>(m2_gate), m2_gate_stride, static_cast<const T *>(r),         \
-                       r_stride, r_bias, w1, static_cast<T *>(out), w2, row_idx, eps, num_rows, width)
+                       r_stride, r_bias, w1, static_cast<T *>(out), w2, row_idx, eps, num_rows, width, static_cast<T *>(sum), conv)
+#define SWL_GO(TPR, NV) SWL_GO_NC(TPR, NV, 0)
     SWL_DISPATCH_DTYPE3(dtype, T, {
         const bool wide = width % 4 == 0 && width <= swl::kRowMaxWidth && r_stride % 4 == 0 && swl::row_aligned<float>(x) &&
                           swl::row_aligned<T>(m) && swl::row_aligned<T>(m2) && swl::row_aligned<T>(r) && swl::row_aligned<T>(out) &&
                           swl::row_aligned<float>(r_bias) && swl::row_aligned<float>(w1) && swl::row_aligned<float>(w2) && swl::row_aligned<float>(slabs);
-        if (slabs && !wide) return SWL_ERR_UNSUPPORTED;
+        if ((slabs || sum) && !wide) return SWL_ERR_UNSUPPORTED;
+        if (sum) {
+            if (!swl::row_aligned<T>(sum) || !swl::row_aligned<float>(conv.w) || !swl::row_aligned<float>(conv.state) || conv.slot_stride % 4 ||
+                conv.tail_off % 4)
+                return SWL_ERR_UNSUPPORTED;
+            if (width <= 1024) SWL_GO_NC(256, 1, swl::kConvStepTaps);
+            else if (width <= 2048) SWL_GO_NC(256, 2, swl::kConvStepTaps);
+            else SWL_GO_NC(256, 4, swl::kConvStepTaps);
+            return swl::check_launch();
+        }
         if (wide) {
             SWL_ROW_SHAPE(num_rows, width, SWL_GO);
             return swl::check_launch();
@@ -397,6 +487,7 @@ static int gated_add_rmsnorm(float *x, const void *m, const float *slabs, int pa
                            static_cast<const T *>(r), r_stride, r_bias, w1, static_cast<T *>(out), w2, row_idx, eps, width);
     });
 #undef SWL_GO
+#undef SWL_GO_NC
     return swl::check_launch();
 }
 
@@ -415,6 +506,18 @@ extern "C" int swl_gated_add_rmsnorm_parts(float *x, const float *slabs, int32_t
     if (!slabs || parts < 1) return SWL_ERR_BAD_ARG;
     return gated_add_rmsnorm(x, nullptr, slabs, parts, m2, m2_gate, m2_gate_stride, r, r_stride, r_bias, w1, out, w2, nullptr, eps, num_rows,
                              width, dtype, stream);
+}
+
+extern "C" int swl_gated_add_rmsnorm_conv(float *x, const void *m, const float *slabs, int32_t parts, const void *m2, const void *m2_gate,
+                                          int64_t m2_gate_stride, const void *r, int64_t r_stride, const float *r_bias, const float *w1,
+                                          void *out, const float *w2, void *sum, const float *conv_w, int32_t taps, float *state,
+                                          int64_t slot_stride, int64_t tail_off, const int32_t *tok_pos, const int32_t *tok_state,
+                                          float eps, int64_t num_rows, int32_t width, int32_t dtype, swl_stream_t stream) {
+    if (taps < 1 || (m && slabs) || (slabs && parts < 1)) return SWL_ERR_BAD_ARG;
+    if (num_rows > 0 && (!out || !sum || !conv_w || !tok_pos || (taps > 1 && (!state || !tok_state)))) return SWL_ERR_BAD_ARG;
+    if (taps > swl::kConvStepTaps || width > 4096) return SWL_ERR_UNSUPPORTED;
+    return gated_add_rmsnorm(x, m, slabs, parts, m2, m2_gate, m2_gate_stride, r, r_stride, r_bias, w1, out, w2, nullptr, eps, num_rows, width,
+                             dtype, stream, sum, swl::ConvStep{state, slot_stride, tail_off, conv_w, tok_pos, tok_state, taps});
 }
 
 extern "C" int swl_causal_conv_state(void *out, int64_t out_stride, const void *h, int64_t h_stride, const float *w,

@@ -10,19 +10,20 @@ from .linear import SplitKPartials
 def gated_add_rmsnorm(x: torch.Tensor, m: torch.Tensor = None, post: torch.Tensor = None, gate: torch.Tensor = None,
                       gate_bias: torch.Tensor = None, m2: torch.Tensor = None, m2_gate: torch.Tensor = None,
                       pre: torch.Tensor = None, eps: float = 1e-6, out_dtype: torch.dtype = None,
-                      row_idx: torch.Tensor = None):
+                      row_idx: torch.Tensor = None, conv=None):
     """In place on the fp32 stream x [T, width]:
         y = m (+ sigmoid(m2_gate[t]) * m2);  y *= sigmoid(gate + gate_bias);  x += y / rms(y) * post
     and returns x / rms(x) * pre in out_dtype when `pre` is given (of rows row_idx only, when given; then m must be None).
     `gate` and `m2_gate` may be column slices of wider matrices (row stride taken from the tensor). m may be a product's SplitKPartials, whose
-    fp32 slabs are summed here."""
+    fp32 slabs are summed here. With `conv` (ConvInput; only where conv.fits(x), without row_idx) -> (that, its
+    causal_conv_state with add_input), the convolution in the same launch where the rows' addresses allow it."""
     _hip.require_gpu_tensor(x, "x")
     n, width = x.shape
     assert x.dtype == torch.float32 and x.is_contiguous()
     dtype = m.dtype if m is not None else out_dtype
     if isinstance(m, SplitKPartials):
         assert m.shape == (n, width)
-        quads = all(t is None or t.data_ptr() % (4 * t.element_size()) == 0 for t in (x, m.slabs, m2, gate, gate_bias, post, pre))
+        quads = _quads(x, m.slabs, m2, gate, gate_bias, post, pre)
         if width % 4 or width > 8192 or not quads or (gate is not None and gate.stride(0) % 4):
             m = m.materialize()
     parts = m if isinstance(m, SplitKPartials) else None
@@ -37,15 +38,30 @@ def gated_add_rmsnorm(x: torch.Tensor, m: torch.Tensor = None, post: torch.Tenso
     out = torch.empty((rows, width), dtype=dtype, device=x.device) if pre is not None else None
     if m is None and pre is None:
         return None
+    fused = conv is not None and (gate is None or gate.stride(0) % 4 == 0) and _quads(x, None if m is None else m.slabs if parts is not None else m,
+                                                                                      m2, gate, gate_bias, post, pre)
+    if conv is not None:
+        assert row_idx is None and pre is not None and conv.fits(x)
     rest = (_hip.ptr(m2), _hip.ptr(m2_gate), m2_gate.stride(0) if m2_gate is not None else 0, _hip.ptr(gate),
             gate.stride(0) if gate is not None else 0, _hip.ptr(gate_bias), _hip.ptr(post), _hip.ptr(out), _hip.ptr(pre))
     tail = (float(eps), rows, width, _hip.dtype_code3(dtype), _hip.stream())
+    if fused:
+        st, total = conv.st, torch.empty_like(out)
+        _hip.call("swl_gated_add_rmsnorm_conv", _hip.ptr(x), 0 if parts is not None else _hip.ptr(m), 0 if parts is None else _hip.ptr(parts.slabs),
+                  0 if parts is None else parts.k_splits, *rest, _hip.ptr(total), _hip.ptr(conv.w), conv.w.shape[0], _hip.ptr(st.pool),
+                  st.pool.stride(0), int(conv.tail_off), _hip.ptr(st.tok_pos), _hip.ptr(st.tok_state), *tail)
+        return out, total
     if parts is not None:
         assert row_idx is None
         _hip.call("swl_gated_add_rmsnorm_parts", _hip.ptr(x), _hip.ptr(parts.slabs), parts.k_splits, *rest, *tail)
     else:
         _hip.call("swl_gated_add_rmsnorm", _hip.ptr(x), _hip.ptr(m), *rest, _hip.ptr(row_idx), *tail)
-    return out
+    return out if conv is None else (out, causal_conv_state(out, conv.w, conv.st, conv.tail_off, add_input=True))
+
+
+def _quads(*tensors) -> bool:
+    """Whether each starts on four of its elements (None: no such operand)."""
+    return all(t is None or t.data_ptr() % (4 * t.element_size()) == 0 for t in tensors)
 
 
 def post_norm_add(x: torch.Tensor, a: torch.Tensor, post: torch.Tensor, b: torch.Tensor = None, a_norm: torch.Tensor = None,
@@ -78,6 +94,23 @@ class StateRef:
         self.tiles, self.longest = tiles, longest
         self.pool, self.tok_pos, self.tok_start, self.tok_state = pool, tok_pos, tok_start, tok_state
         self.tok_seq, self.seq_row0, self.seq_cnt = tok_seq, seq_row0, seq_cnt
+
+
+class ConvInput:
+    """The input convolution of the next sublayer: what causal_conv_state takes beside the rows."""
+    __slots__ = ("w", "st", "tail_off")
+    MAX_TAPS, MAX_WIDTH = 4, 4096       # (swl_gated_add_rmsnorm_conv)
+
+    def __init__(self, w: torch.Tensor, st: StateRef, tail_off: int):
+        self.w, self.st, self.tail_off = w, st, tail_off
+
+    def fits(self, x: torch.Tensor) -> bool:
+        """Whether rows like x's may be convolved in the launch that norms them: every portion a single token, whose earlier inputs are
+        all in the state slot."""
+        w, st = self.w, self.st
+        return (st.longest == 1 and w.dtype == torch.float32 and w.is_contiguous() and w.shape[0] <= self.MAX_TAPS and w.shape[1] == x.shape[1]
+                and w.shape[1] <= self.MAX_WIDTH and w.shape[1] % 4 == 0 and st.pool.stride(0) % 4 == 0 and self.tail_off % 4 == 0
+                and _quads(w, st.pool))
 
 
 def token_shift_mix(h: torch.Tensor, mu: torch.Tensor, st: StateRef, tail_off: int) -> torch.Tensor:

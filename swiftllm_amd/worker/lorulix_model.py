@@ -24,7 +24,7 @@ from swiftllm_amd.model_config import LorulixModelConfig
 from .kernels.delta_rule import most_tiles_scratch
 from .kernels.layernorm import embed_positions
 from .kernels.linear import pack_weight, packable_rows
-from .kernels.rms_stream import StateRef, causal_conv_state, gated_add_rmsnorm
+from .kernels.rms_stream import ConvInput, StateRef, causal_conv_state, gated_add_rmsnorm
 from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import _project
 from .layers.lorulix_layer import LorulixAttention, LorulixDelta, LorulixFeedForward, StepContext
@@ -114,13 +114,18 @@ class LorulixModel(SteppedModel):
         x, _ = embed_positions(dev["input_ids"], dev["tok_pos"], w.embed, w.pos, 1.0, keep_copy=False)
         tap = self.layer_tap
         subs = self.sublayers
-        h = gated_add_rmsnorm(x, pre=subs[0].pre, eps=eps, out_dtype=self.dtype)
+        inputs = [ConvInput(s.canon, st, s.canon_off) for s in subs]
+        fused = all(c.fits(x) for c in inputs)      # (one token a sequence: the convolution is part of the norm's launch)
+        h = gated_add_rmsnorm(x, pre=subs[0].pre, eps=eps, out_dtype=self.dtype, conv=inputs[0] if fused else None)
         for i, s in enumerate(subs):
+            h, hc = h if fused else (h, None)
             r = _project(h, s.rg, self._skinny)
-            hc = causal_conv_state(h, s.canon, st, s.canon_off, add_input=True)
+            if hc is None:
+                hc = causal_conv_state(h, s.canon, st, s.canon_off, add_input=True)
             m, m2, m2_gate = s.op.forward(hc, ctx)
-            nxt = subs[i + 1].pre if i + 1 < len(subs) else None
-            h = gated_add_rmsnorm(x, m, s.post, r, s.rg_b, m2, m2_gate, pre=nxt, eps=eps)
+            last = i + 1 == len(subs)
+            h = gated_add_rmsnorm(x, m, s.post, r, s.rg_b, m2, m2_gate, pre=None if last else subs[i + 1].pre, eps=eps,
+                                  conv=inputs[i + 1] if fused and not last else None)
             if tap is not None and s.ends_layer:
                 tap.append(x.clone())
         return x

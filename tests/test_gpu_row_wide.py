@@ -92,3 +92,46 @@ def test_slabs_of_a_split_product(rows, width, parts, dtype):
 def test_one_slab(rows, width, dtype):
     """A product that was not split, for every number of columns that a thread holds."""
     test_slabs_of_a_split_product(rows, width, 1, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,width,taps,form", [(1, 4, 4, "m"), (3, 1024, 3, "gated"), (5, 1028, 2, "parts"), (4, 2048, 4, "none"), (7, 2052, 1, "m"),
+                                                  (1100, 1020, 3, "gated"), (2, 4096, 4, "parts"), (3, 1022, 3, "m"), (3, 4096, 5, "none")])
+def test_gated_add_rmsnorm_conv(rows, width, taps, form, dtype):
+    """The convolution in the norm's launch: the stream and the normed rows as the norm alone leaves them, the sum and the carried inputs
+    (bit by bit) as the convolution of these rows does. Rows and taps the kernel does not take are refused by `fits`."""
+    from swiftllm_amd.worker.kernels.rms_stream import ConvInput, StateRef, causal_conv_state, gated_add_rmsnorm
+    from swiftllm_amd.worker.kernels.linear import SplitKPartials
+    g = torch.Generator().manual_seed(rows * width + taps)
+    rand = lambda *shape, dt=torch.float32: torch.randn(*shape, generator=g).to(dt).cuda()
+    off, slots = 12, rows + 2
+    pool = rand(slots, off + 2 * (taps - 1) * width + 4)
+    pos = torch.tensor([(0, 1, 2, 3, 9)[i % 5] for i in range(rows)], dtype=torch.int32).cuda()
+    code = (2 * torch.randperm(slots, generator=g)[:rows] + torch.arange(rows) % 2).to(torch.int32).cuda()
+    seq = torch.arange(rows, dtype=torch.int32).cuda()
+    x, w, post, pre, bias = rand(rows, width), rand(taps, width), rand(width), rand(width), rand(width)
+    kw = {"eps": EPS, "pre": pre, "out_dtype": dtype}
+    if form == "parts":
+        kw["m"] = SplitKPartials(rand(3, rows, width), 3, rows, width, dtype)
+    elif form != "none":
+        kw["m"] = rand(rows, width, dt=dtype)
+    if form == "gated":
+        kw |= {"gate": rand(rows, width, dt=dtype), "gate_bias": bias, "m2": rand(rows, width, dt=dtype), "m2_gate": rand(rows, 3, dt=dtype)[:, 1:2]}
+    kw["post"] = post
+    st = StateRef(pool.clone(), pos, pos, code, seq, seq, torch.ones_like(seq), longest=1)
+    conv, x1 = ConvInput(w, st, off), x.clone()
+    if width % 4 or taps > 4:
+        assert not conv.fits(x1)
+        return
+    assert conv.fits(x1)
+    h, total = gated_add_rmsnorm(x1, conv=conv, **kw)
+    x2 = x.clone()
+    gated_add_rmsnorm(x2, **kw)
+    _close(x1, h, x2.double().cpu(), _rms(x2.double().cpu()) * pre.double().cpu(), dtype)
+    ref = StateRef(pool.clone(), pos, pos, code, seq, seq, torch.ones_like(seq), longest=1)
+    want = causal_conv_state(h, w, ref, off, add_input=True).double()
+    assert torch.equal(st.pool, ref.pool)
+    # up to five fp32 terms, whose products a compiler may or may not round before they are added, then one rounding to the type
+    size = 5 * (w.double().abs().sum(0) + 1) * max(float(pool.abs().max()), float(h.abs().max()))
+    eps = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+    assert ((total.double() - want).abs() <= eps * want.abs() + 2.0 ** -24 * size).all()
