@@ -293,6 +293,11 @@ int swl_gemm_packed_mid_silu_gate(void *out, const void *x, const void *w_up_gat
 int swl_gemm_f32_supported(int32_t M, int32_t N, int32_t K);
 int swl_gemm_f32(float *out, const float *x, const float *w, int32_t M, int32_t N, int32_t K, int64_t x_row_stride, int64_t out_row_stride,
                  int32_t k_waves, swl_stream_t stream);
+/* Two such products of the same M and K in one launch, each with the sums of its own; N1 at most 4096. glu: w2 is [gate; up] and out2 [M, N2 / 2]
+ * the clamped gated unit of the two (swl_glu_clamp, act 0). relu2_columns: so many of out2's first columns are max(0, product)^2. */
+int swl_gemm_f32_pair(float *out1, const float *x1, const float *w1, int32_t N1, int64_t x1_row_stride, int64_t out1_row_stride, float *out2,
+                      const float *x2, const float *w2, int32_t N2, int64_t x2_row_stride, int64_t out2_row_stride, int32_t M, int32_t K,
+                      int32_t glu, int32_t relu2_columns, float limit, swl_stream_t stream);
 /* Large decode batches on a packed weight (csrc/gemm_wide.hip): out[M, N] = x . W^T for up to 256 tokens — the projections
  * of reference kernels/linear.py:3-12 (transformer_layer.py:54-56,117,126,128) at the batch sizes a 264 GB KV pool holds;
  * every weight fragment feeds ceil(M/32) <= 8 MFMAs, x^T shared by the workgroup through LDS. N % 32 == 0, K % 64 == 0.

@@ -21,13 +21,16 @@ namespace swl {
 constexpr int kF32MaxTokens = 16;
 
 // KS waves share the columns of the same rows, 4 / KS groups of rows a workgroup
-template <int M, int R, int KS>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(float *__restrict__ out, const float *__restrict__ x, const float *__restrict__ w, int rows,
-                                                       int N, int K, int64_t x_stride, int64_t out_stride) {
-    constexpr int V = M * R;
-    __shared__ float part[4][4][V];         // [wave][16-lane row]
+// GLU: rows [gate; up] of w, a wave takes R / 2 of each; out[c] = gated_unit of the two products. relu2: the first so many columns of out are
+// max(0, product)^2.
+template <int M, int R, int KS, bool GLU>
+__device__ __forceinline__ void gemm_f32_block(float (*part)[4][M * R], int block, float *__restrict__ out, const float *__restrict__ x,
+                                               const float *__restrict__ w, int rows, int N, int K, int64_t x_stride, int64_t out_stride,
+                                               int relu2, float limit) {
+    constexpr int V = M * R, OUT = GLU ? R / 2 : R;
+    const int columns = GLU ? N / 2 : N;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int n0 = (blockIdx.x * (4 / KS) + wave / KS) * R;
+    const int n0 = (block * (4 / KS) + wave / KS) * OUT;
     const int chunks = (K + 255) / 256, per = (chunks + KS - 1) / KS;
     const int k_end = min(K, (wave % KS + 1) * per * 256);
     float acc[R][M];
@@ -37,7 +40,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(float *__restrict__ out, 
         for (int m = 0; m < M; ++m) acc[r][m] = 0.f;
     const float *wr[R], *xr[M];
 #pragma unroll
-    for (int r = 0; r < R; ++r) wr[r] = w + static_cast<int64_t>(min(n0 + r, N - 1)) * K;
+    for (int r = 0; r < R; ++r) wr[r] = w + static_cast<int64_t>(min(n0 + r % OUT, columns - 1) + r / OUT * columns) * K;
 #pragma unroll
     for (int m = 0; m < M; ++m) xr[m] = x + min(m, rows - 1) * x_stride;
     auto slice = [&](int k) {
@@ -75,16 +78,53 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(float *__restrict__ out, 
     for (int j = 0; j < (V + 15) / 16; ++j)
         if (16 * j + (lane & 15) < V) part[wave][lane >> 4][16 * j + (lane & 15)] = keep[j];
     __syncthreads();
-    for (int t = threadIdx.x; t < V * (4 / KS); t += 256) {
-        const int g = t / V, v = t - g * V, r = v / M, m = v - r * M;
+    auto sum = [&](int g, int v) {
         float s = 0.f;
 #pragma unroll
         for (int i = 0; i < KS; ++i)
 #pragma unroll
             for (int q = 0; q < 4; ++q) s += part[g * KS + i][q][v];
-        const int n = (blockIdx.x * (4 / KS) + g) * R + r;
-        if (n < N && m < rows) out[m * out_stride + n] = s;
+        return s;
+    };
+    for (int t = threadIdx.x; t < OUT * M * (4 / KS); t += 256) {
+        const int g = t / (OUT * M), v = t - g * OUT * M, r = v / M, m = v - r * M;
+        const int n = (block * (4 / KS) + g) * OUT + r;
+        float s = sum(g, v);
+        if constexpr (GLU) {
+            s = gated_unit(s, sum(g, v + OUT * M), limit, 0);
+        } else if (n < relu2) {
+            s = fmaxf(s, 0.f);
+            s *= s;
+        }
+        if (n < columns && m < rows) out[m * out_stride + n] = s;
     }
+}
+
+template <int M, int R, int KS>
+__global__ __launch_bounds__(256) void gemm_f32_kernel(float *__restrict__ out, const float *__restrict__ x, const float *__restrict__ w, int rows,
+                                                       int N, int K, int64_t x_stride, int64_t out_stride) {
+    __shared__ float part[4][4][M * R];         // [wave][16-lane row]
+    gemm_f32_block<M, R, KS, false>(part, blockIdx.x, out, x, w, rows, N, K, x_stride, out_stride, 0, 0.f);
+}
+
+struct F32Product {
+    float *out;
+    const float *x, *w;
+    int64_t x_stride, out_stride;
+    int N;
+};
+
+// Two products of the same tokens and columns in one launch, the first in the first `blocks` workgroups (four waves share K in it).
+// A decode step is a chain of launches of 3 to 5 us each, and a product of a few MiB does not fill the chip: 3 tokens of width 1024 through 8
+// sublayers, the gate's 1024 rows beside the sublayer's first product and its activation in the same launch (12 launches less), 396 -> 363 us
+// a step. Every sum is that of a launch of its own.
+template <int M, int R, int KS, bool GLU>
+__global__ __launch_bounds__(256) void gemm_f32_pair_kernel(F32Product a, F32Product b, int blocks, int rows, int K, int relu2, float limit) {
+    __shared__ float part[4][4][M * R];
+    if (static_cast<int>(blockIdx.x) < blocks)
+        gemm_f32_block<M, R, 4, false>(part, blockIdx.x, a.out, a.x, a.w, rows, a.N, K, a.x_stride, a.out_stride, 0, 0.f);
+    else
+        gemm_f32_block<M, R, KS, GLU>(part, blockIdx.x - blocks, b.out, b.x, b.w, rows, b.N, K, b.x_stride, b.out_stride, relu2, limit);
 }
 
 template <int M, int R>
@@ -95,6 +135,21 @@ static void launch_f32(int ks, hipStream_t s, float *out, const float *x, const 
     else if (ks == 2) hipLaunchKernelGGL((gemm_f32_kernel<M, R, 2>), grid, dim3(256), 0, s, out, x, w, rows, N, K, xs, os);
     else hipLaunchKernelGGL((gemm_f32_kernel<M, R, 1>), grid, dim3(256), 0, s, out, x, w, rows, N, K, xs, os);
 }
+
+template <int M, int R>
+static void launch_f32_pair(int ks, hipStream_t s, const F32Product &a, const F32Product &b, int rows, int K, bool glu, int relu2, float limit) {
+    const int first = (a.N + R - 1) / R, per = (glu ? R / 2 : R) * (4 / ks), columns = glu ? b.N / 2 : b.N;
+    const dim3 grid(static_cast<unsigned>(first + (columns + per - 1) / per));
+#define SWL_F32_PAIR(KS, GLU) hipLaunchKernelGGL((gemm_f32_pair_kernel<M, R, KS, GLU>), grid, dim3(256), 0, s, a, b, first, rows, K, relu2, limit)
+    if (ks == 4 && glu) SWL_F32_PAIR(4, true);
+    else if (ks == 4) SWL_F32_PAIR(4, false);
+    else if (glu) SWL_F32_PAIR(2, true);
+    else SWL_F32_PAIR(2, false);
+#undef SWL_F32_PAIR
+}
+
+// (the rows of w alone decide: a token's bits do not hang on its company)
+static int f32_k_waves(int N) { return N <= 4096 ? 4 : 2; }
 
 } // namespace swl
 
@@ -115,9 +170,36 @@ extern "C" int swl_gemm_f32(float *out, const float *x, const float *w, int32_t 
     if (!swl_gemm_f32_supported(M, N, K)) return SWL_ERR_UNSUPPORTED;
     if (x_row_stride < K || out_row_stride < N || x_row_stride % 4 || !swl::aligned16(x) || !swl::aligned16(w)) return SWL_ERR_BAD_ARG;
     if (!(k_waves == 0 || k_waves == 1 || k_waves == 2 || k_waves == 4)) return SWL_ERR_BAD_ARG;
-    const int ks = k_waves ? k_waves : N <= 4096 ? 4 : 2;     // (the rows of w alone decide: a token's bits do not hang on its company)
+    const int ks = k_waves ? k_waves : swl::f32_k_waves(N);
     hipStream_t s = static_cast<hipStream_t>(stream);
 #define SWL_F32_CASE(MM, R) swl::launch_f32<MM, R>(ks, s, out, x, w, M, N, K, x_row_stride, out_row_stride)
+    switch (M) {
+        case 1: SWL_F32_CASE(1, 4); break;
+        case 2: SWL_F32_CASE(2, 4); break;
+        case 3: SWL_F32_CASE(3, 4); break;
+        case 4: SWL_F32_CASE(4, 4); break;
+        default:
+            if (M <= 8) SWL_F32_CASE(8, 4);
+            else SWL_F32_CASE(16, 2);
+    }
+#undef SWL_F32_CASE
+    return swl::check_launch();
+}
+
+extern "C" int swl_gemm_f32_pair(float *out1, const float *x1, const float *w1, int32_t N1, int64_t x1_row_stride, int64_t out1_row_stride,
+                                 float *out2, const float *x2, const float *w2, int32_t N2, int64_t x2_row_stride, int64_t out2_row_stride,
+                                 int32_t M, int32_t K, int32_t glu, int32_t relu2_columns, float limit, swl_stream_t stream) {
+    if (M < 0 || N1 <= 0 || N2 <= 0 || K <= 0 || relu2_columns < 0 || relu2_columns > N2 || (glu && (relu2_columns || N2 % 2))) return SWL_ERR_BAD_ARG;
+    if (M == 0) return SWL_OK;
+    if (!out1 || !x1 || !w1 || !out2 || !x2 || !w2) return SWL_ERR_BAD_ARG;
+    if (!swl_gemm_f32_supported(M, N1, K) || !swl_gemm_f32_supported(M, N2, K) || swl::f32_k_waves(N1) != 4) return SWL_ERR_UNSUPPORTED;
+    if (x1_row_stride < K || out1_row_stride < N1 || x1_row_stride % 4 || x2_row_stride < K || out2_row_stride < (glu ? N2 / 2 : N2) ||
+        x2_row_stride % 4 || !swl::aligned16(x1) || !swl::aligned16(w1) || !swl::aligned16(x2) || !swl::aligned16(w2))
+        return SWL_ERR_BAD_ARG;
+    const swl::F32Product a{out1, x1, w1, x1_row_stride, out1_row_stride, N1}, b{out2, x2, w2, x2_row_stride, out2_row_stride, N2};
+    const int ks = swl::f32_k_waves(N2);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+#define SWL_F32_CASE(MM, R) swl::launch_f32_pair<MM, R>(ks, s, a, b, M, K, glu != 0, relu2_columns, limit)
     switch (M) {
         case 1: SWL_F32_CASE(1, 4); break;
         case 2: SWL_F32_CASE(2, 4); break;

@@ -122,15 +122,6 @@ __device__ __forceinline__ void wave_argmax(const float *v, int n, int lane, flo
     besti = __builtin_amdgcn_readfirstlane(besti);
 }
 
-// act 0: g' = min(g, limit), u' = clamp(u, +-limit), g' sigmoid(1.702 g') (u' + 1); act 1: silu(g) u; act 2: silu(u) g
-__device__ __forceinline__ float gated_unit(float g, float u, float limit, int act) {
-    if (act == 1) return g / (1.0f + expf(-g)) * u;
-    if (act == 2) return u / (1.0f + expf(-u)) * g;
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-    return g * (1.0f / (1.0f + expf(-1.702f * g))) * (u + 1.0f);
-}
-
 template <typename T>
 __global__ __launch_bounds__(kMoeThreads) void moe_route_kernel(int32_t *idx_out, float *w_out, const T *h,
                                                                 const float *router, const float *bias, int width,

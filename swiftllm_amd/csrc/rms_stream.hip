@@ -12,7 +12,7 @@
 //     (a loader that stores "weight around zero" adds the one).
 //     swl_gated_add_rmsnorm_conv, for steps of one token a sequence: the next sublayer's input convolution in the same launch. The row it
 //     convolves is in registers, what came before it in the state slot, asked for with the stream's. A step's latency is a chain of
-//     launches: 3 tokens x 1024 columns of 3 taps in fp32, the two launches of each of 8 sublayers 64 -> 46 us a step of 402 -> 384.
+//     launches: 3 tokens x 1024 columns of 3 taps in fp32, 8 sublayers, 414 -> 396 us a step.
 //   swl_post_norm_add: the same step for models whose sublayers read the stream itself (norm on the sublayer's RESULT only):
 //       y   = c * (a' + b')      a' = a / rms(a) * wa when wa is given, else a; b' likewise (b optional)
 //       x  += y / rms(y) * w1

@@ -356,6 +356,15 @@ inline int check_launch() { return hipGetLastError() == hipSuccess ? SWL_OK : SW
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// act 0: g' = min(g, limit), u' = clamp(u, +-limit), g' sigmoid(1.702 g') (u' + 1); act 1: silu(g) u; act 2: silu(u) g
+__device__ __forceinline__ float gated_unit(float g, float u, float limit, int act) {
+    if (act == 1) return g / (1.0f + expf(-g)) * u;
+    if (act == 2) return u / (1.0f + expf(-u)) * g;
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return g * (1.0f / (1.0f + expf(-1.702f * g))) * (u + 1.0f);
+}
+
 } // namespace swl
 
 // Dispatch a templated launcher on the runtime dtype code.

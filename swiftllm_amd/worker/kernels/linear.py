@@ -317,16 +317,40 @@ def _blas_linear(a: torch.Tensor, w: torch.Tensor, row_blocks=None, plateau=None
 F32_MAX_TOKENS = 16     # (swl_gemm_f32_supported)
 
 
+F32_PAIR_MAX_ROWS = 4096    # (swl_gemm_f32_pair: of the first matrix)
+
+
+def _f32_takes(a: torch.Tensor, w: torch.Tensor) -> bool:
+    return (a.is_cuda and a.dim() == w.dim() == 2 and a.shape[1] == w.shape[1] and a.dtype == w.dtype == torch.float32 and w.is_contiguous()
+            and a.stride(1) == 1 and (a.data_ptr() | w.data_ptr()) % 16 == 0 and a.stride(0) % 4 == 0
+            and _hip.load().swl_gemm_f32_supported(a.shape[0], w.shape[0], w.shape[1]) == 2)
+
+
 def linear_f32(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """a[T, in] @ w[out, in]^T in true fp32: a few tokens on the hand-written kernel (csrc/gemm_f32.hip), the BLAS otherwise."""
-    if (a.is_cuda and a.dim() == w.dim() == 2 and a.shape[1] == w.shape[1] and a.dtype == w.dtype == torch.float32 and w.is_contiguous()
-            and a.stride(1) == 1 and (a.data_ptr() | w.data_ptr()) % 16 == 0 and a.stride(0) % 4 == 0):
+    if _f32_takes(a, w):
         m, (n, k) = a.shape[0], w.shape
-        if _hip.load().swl_gemm_f32_supported(m, n, k) == 2:
-            out = torch.empty((m, n), dtype=a.dtype, device=a.device)
-            _hip.call("swl_gemm_f32", _hip.ptr(out), _hip.ptr(a), _hip.ptr(w), m, n, k, _row_stride(a), n, 0, _hip.stream())
-            return out
+        out = torch.empty((m, n), dtype=a.dtype, device=a.device)
+        _hip.call("swl_gemm_f32", _hip.ptr(out), _hip.ptr(a), _hip.ptr(w), m, n, k, _row_stride(a), n, 0, _hip.stream())
+        return out
     return F.linear(a, w)
+
+
+def linear_f32_pair(a1: torch.Tensor, w1: torch.Tensor, a2: torch.Tensor, w2: torch.Tensor, glu_limit: float = None, relu2_columns: int = 0):
+    """-> (a1 w1^T, a2 w2^T) of the same few tokens in true fp32, in one launch; None where that launch does not serve them. The second with an
+    activation: glu_limit: w2 = [gate; up] and the clamped gated unit of the two products; relu2_columns: relu(.)^2 of its first columns."""
+    if not (w1.shape == (w1.shape[0], a2.shape[1]) and a1.shape == a2.shape and _f32_takes(a1, w1) and _f32_takes(a2, w2)
+            and w1.shape[0] <= F32_PAIR_MAX_ROWS and a1.device == a2.device):
+        return None
+    m, k = a1.shape
+    n1, n2 = w1.shape[0], w2.shape[0]
+    n_out = n2 // 2 if glu_limit is not None else n2
+    y1 = torch.empty((m, n1), dtype=a1.dtype, device=a1.device)
+    # (columns that feed another product: rows on 16 bytes)
+    y2 = torch.empty((m, (n_out + 3) // 4 * 4 if relu2_columns else n_out), dtype=a1.dtype, device=a1.device)
+    _hip.call("swl_gemm_f32_pair", _hip.ptr(y1), _hip.ptr(a1), _hip.ptr(w1), n1, _row_stride(a1), n1, _hip.ptr(y2), _hip.ptr(a2), _hip.ptr(w2), n2,
+              _row_stride(a2), y2.stride(0), m, k, 0 if glu_limit is None else 1, int(relu2_columns), float(glu_limit or 0.0), _hip.stream())
+    return y1, y2[:, :n_out]
 
 
 def linear_grouped(x: torch.Tensor, w: torch.Tensor, skinny: bool = False) -> torch.Tensor:

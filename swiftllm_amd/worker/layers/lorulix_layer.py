@@ -1,5 +1,8 @@
 """The sublayers of a Lorulix layer, each a function from its (normed, convolved) input to its raw result; the bookkeeping
-around them (result gate, post-norm into the fp32 stream, the next input norm and convolution) is the model's fused step."""
+around them (result gate, post-norm into the fp32 stream, the next input norm and convolution) is the model's fused step.
+
+`first` of a sublayer is the product its forward begins with: the matrix and the activation that linear_f32_pair may apply to it (None: no
+such product). A caller that already has that result passes it as forward's `done`."""
 import torch
 
 from ..kernels.delta_rule import delta_rule_mixer
@@ -29,10 +32,11 @@ class LorulixAttention:
         self.mixer, self.w, self.eps, self.skinny = layer_config.mixer, weight, eps, skinny
         self.pool_slice, self.max_positions = pool_slice, max_positions
         self.own_kv = self.mixer.kv_from < 0
+        self.first = (weight.qkv, {})
 
-    def forward(self, h: torch.Tensor, ctx: StepContext):
+    def forward(self, h: torch.Tensor, ctx: StepContext, done: torch.Tensor = None):
         mx = self.mixer
-        qkv = _project(h, self.w.qkv, self.skinny)
+        qkv = done if done is not None else _project(h, self.w.qkv, self.skinny)
         qknorm_full_and_store_kv(qkv, self.w.q_norm, self.w.k_norm, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq,
                                  ctx.tok_pos, mx, self.eps, self.own_kv)
         if ctx.pool is None:    # memory profiling: the attention's output buffer without its reads
@@ -50,9 +54,10 @@ class LorulixDelta:
     def __init__(self, layer_config, weight, eps: float, skinny: bool, tail_off: int, state_off: int):
         self.mixer, self.w, self.eps, self.skinny = layer_config.mixer, weight, eps, skinny
         self.tail_off, self.state_off = tail_off, state_off
+        self.first = (weight.proj, {})
 
-    def forward(self, h: torch.Tensor, ctx: StepContext):
-        proj = _project(h, self.w.proj, self.skinny)
+    def forward(self, h: torch.Tensor, ctx: StepContext, done: torch.Tensor = None):
+        proj = done if done is not None else _project(h, self.w.proj, self.skinny)
         y = delta_rule_mixer(proj, self.w.conv, self.w.a_log, self.w.dt_bias, self.w.out_norm, ctx.state, self.tail_off,
                              self.state_off, self.mixer, self.eps)
         return _project_partials(y, self.w.o, self.skinny), None, None
@@ -64,20 +69,26 @@ class LorulixFeedForward:
 
     def __init__(self, layer_config, weight, skinny: bool):
         self.mlp, self.w, self.skinny = layer_config.mlp, weight, skinny
+        if self.mlp.kind == "dense":
+            self.first = (weight.gate_up, {"glu_limit": float(self.mlp.limit)})
+        else:
+            self.first = (weight.shared_up, {"relu2_columns": self.mlp.shared_ffn_inter_dim}) if weight.shared_up is not None else None
 
-    def forward(self, h: torch.Tensor, ctx: StepContext):
+    def forward(self, h: torch.Tensor, ctx: StepContext, done: torch.Tensor = None):
         mlp, w = self.mlp, self.w
         if mlp.kind == "dense":
-            gu = _project(h, w.gate_up, self.skinny)
-            y = torch.empty((h.shape[0], mlp.ffn_inter_dim), dtype=h.dtype, device=h.device)
-            _hip.call("swl_glu_clamp", _hip.ptr(y), _hip.ptr(gu), 0, h.shape[0], mlp.ffn_inter_dim, float(mlp.limit), 0,
-                      _hip.dtype_code3(h.dtype), _hip.stream())
+            y = done
+            if y is None:
+                gu = _project(h, w.gate_up, self.skinny)
+                y = torch.empty((h.shape[0], mlp.ffn_inter_dim), dtype=h.dtype, device=h.device)
+                _hip.call("swl_glu_clamp", _hip.ptr(y), _hip.ptr(gu), 0, h.shape[0], mlp.ffn_inter_dim, float(mlp.limit), 0,
+                          _hip.dtype_code3(h.dtype), _hip.stream())
             return _project_partials(y, w.down, self.skinny), None, None
         idx, wts = moe_route_scores(h, w.router, mlp.top_k, mlp.router_scale)
         out = moe_experts_relu2(h, idx, wts, w.up, w.down)
         if w.shared_up is None:
             return out, None, None
         fs = mlp.shared_ffn_inter_dim
-        z = _project(h, w.shared_up, self.skinny)           # [T, fs + 1]: the shared expert's up rows, then its gate logit
-        shared = _project(relu_squared(z, fs), w.shared_down, self.skinny)
+        z = done if done is not None else _project(h, w.shared_up, self.skinny)     # [T, fs + 1]: the shared expert's up rows, then its gate logit
+        shared = _project(z[:, :fs] if done is not None else relu_squared(z, fs), w.shared_down, self.skinny)
         return out, shared, z[:, fs:fs + 1]

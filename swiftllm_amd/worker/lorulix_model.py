@@ -23,7 +23,7 @@ from swiftllm_amd.model_config import LorulixModelConfig
 
 from .kernels.delta_rule import most_tiles_scratch
 from .kernels.layernorm import embed_positions
-from .kernels.linear import pack_weight, packable_rows
+from .kernels.linear import F32_MAX_TOKENS, linear_f32_pair, pack_weight, packable_rows
 from .kernels.rms_stream import ConvInput, StateRef, causal_conv_state, gated_add_rmsnorm
 from .kernels.window_attn import PoolSlice, StepTiles
 from .layers.kekapel_layer import _project
@@ -115,14 +115,18 @@ class LorulixModel(SteppedModel):
         tap = self.layer_tap
         subs = self.sublayers
         inputs = [ConvInput(s.canon, st, s.canon_off) for s in subs]
+        few = self.dtype == torch.float32 and x.shape[0] <= F32_MAX_TOKENS
         fused = all(c.fits(x) for c in inputs)      # (one token a sequence: the convolution is part of the norm's launch)
         h = gated_add_rmsnorm(x, pre=subs[0].pre, eps=eps, out_dtype=self.dtype, conv=inputs[0] if fused else None)
         for i, s in enumerate(subs):
             h, hc = h if fused else (h, None)
-            r = _project(h, s.rg, self._skinny)
             if hc is None:
                 hc = causal_conv_state(h, s.canon, st, s.canon_off, add_input=True)
-            m, m2, m2_gate = s.op.forward(hc, ctx)
+            both = None
+            if few and s.op.first is not None:
+                both = linear_f32_pair(h, s.rg, hc, s.op.first[0], **s.op.first[1])
+            r, done = both if both is not None else (_project(h, s.rg, self._skinny), None)
+            m, m2, m2_gate = s.op.forward(hc, ctx, done)
             last = i + 1 == len(subs)
             h = gated_add_rmsnorm(x, m, s.post, r, s.rg_b, m2, m2_gate, pre=None if last else subs[i + 1].pre, eps=eps,
                                   conv=inputs[i + 1] if fused and not last else None)

@@ -56,3 +56,35 @@ def test_linear_f32_refuses_rows_of_another_length(columns):
     for a in (x[:, :columns], x[:, :columns].contiguous()):
         with pytest.raises(RuntimeError):
             linear_f32(a, w)
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 7, 16])
+@pytest.mark.parametrize("N1,N2,K,form", [(1, 2, 4, "glu"), (64, 17, 252, ""), (1024, 3200, 1024, ""), (257, 513, 516, "relu2"), (255, 2 * 131, 1028, "glu"),
+                                          (4096, 8194, 256, "glu"), (33, 4100, 260, "relu2"), (4097, 64, 64, "refused")])
+def test_gemm_f32_pair(M, N1, N2, K, form):
+    """Two products in one launch: the bits of the two launches, and of the activation's where the second has one."""
+    from swiftllm_amd import _hip
+    from swiftllm_amd.worker.kernels.linear import linear_f32_pair
+    from swiftllm_amd.worker.kernels.moe import relu_squared
+    g = torch.Generator().manual_seed(M + N1 * N2 + K)
+    x1, x2, w1, w2 = (torch.randn(n, K, generator=g).cuda() for n in (M, M, N1, N2))
+
+    def alone(x, w):
+        out = torch.empty(M, w.shape[0], device="cuda")
+        _hip.call("swl_gemm_f32", _hip.ptr(out), _hip.ptr(x), _hip.ptr(w), M, w.shape[0], K, K, w.shape[0], 0, _hip.stream())
+        return out
+
+    kw = {"glu": {"glu_limit": 0.75}, "relu2": {"relu2_columns": N2 - 1}}.get(form, {})
+    got = linear_f32_pair(x1, w1, x2, w2, **kw)
+    served = [_hip.load().swl_gemm_f32_supported(M, n, K) == 2 for n in (N1, N2)]
+    if form == "refused" or not all(served):
+        assert got is None
+        return
+    want = alone(x2, w2)
+    if form == "glu":
+        want, both = torch.empty(M, N2 // 2, device="cuda"), want
+        _hip.call("swl_glu_clamp", _hip.ptr(want), _hip.ptr(both), 0, M, N2 // 2, 0.75, 0, _hip.dtype_code3(torch.float32), _hip.stream())
+    elif form == "relu2":
+        want = torch.cat((relu_squared(want, N2 - 1), want[:, N2 - 1:]), dim=1)
+        assert got[1].stride(0) % 4 == 0
+    assert torch.equal(got[0], alone(x1, w1)) and torch.equal(got[1], want)
