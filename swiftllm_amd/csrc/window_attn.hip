@@ -206,6 +206,230 @@ inline size_t wa_lds_bytes(int H, int d) {
     return wa_float_count(H, d) * 4 + 4 * sizeof(int64_t);
 }
 
+// The same loop in fp32 for the H heads of one key head, D columns a key and DV a value, nothing mixed. What bounds a share of 64 keys is the
+// chain of its memory round trips: above they are the blocks' ids, the queries, two rounds of keys, the distance bias and the values, one
+// behind the other. Here the ids are scalar loads and a chunk's keys, bias and values are all asked for before the first score (the next
+// chunk's as soon as the registers are free); a lane has its queries in registers, and where a value row has 64 or 128 columns two or four
+// groups of threads share the pages. 90 to 145 registers: a sum left alone sinks below the next chunk's loads and takes 256.
+// us with the launch that adds up the shares, above -> here (heads of 128, 8 over 2, fp32; other sizes named): 3 tokens at 513 keys 18.0 ->
+// 10.7, one at 100 14.1 -> 10.5, 3 at 4000 50 -> 19.8, 12 at 500 18.2 -> 13.0, 32 at 1000 32 -> 20; prompts of 100 23 -> 16, 500 120 -> 39, 4 x 125
+// 48 -> 21, 500 with 8 key heads 365 -> 74, 500 of 64 / 128 columns 73 -> 31. Nothing measured was slower, so whatever it takes goes to it. Error
+// against 64 bits 2.0 to 3.7e-7 (2-norm) where it is 2.1 to 3.8e-7 above.
+struct HeadsParams {
+    void *out;
+    const float *q, *k, *v;
+    const int32_t *block_table, *tok_seq, *tok_pos;
+    const float *rel, *sink, *slopes, *gate;
+    float *part_o, *part_ml;
+    int64_t q_stride, block_stride, out_stride, gate_stride;
+    int rel_len, window, mask_kind, max_blocks, G, GV, out_dim;
+    float scale, softcap;
+};
+
+template <int D, int DV, int H>
+__global__ __launch_bounds__(kTaThreads, 2) void window_attn_heads_kernel(HeadsParams a) {
+    constexpr int LPR = D / 4, ROWS = 64 / LPR, KU = kTaChunk / (4 * ROWS);     // lanes of a key row, keys a wave loads at once, loads a chunk
+    constexpr int VP = kTaThreads / DV, PV = kTaChunk / kTaPage / VP;           // groups of threads that share the pages, pages of each
+    constexpr int HW = (H + 3) / 4;                                             // heads a wave
+    __shared__ __attribute__((aligned(16))) float s[H][kTaChunk], p[H][kTaChunk], red[VP > 1 ? VP - 1 : 1][H][DV], alpha[H];
+    const int64_t t = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kv = blockIdx.y, hb = kv * H, gv = kv % a.GV, Hall = a.G * H;
+    const int pos = a.tok_pos[t];
+    const int32_t *bt = a.block_table + static_cast<int64_t>(a.tok_seq[t]) * a.max_blocks;
+    const int lo = a.window <= 0 ? 0 : a.mask_kind == 1 ? (pos / a.window) * a.window : max(pos - a.window + 1, 0);
+    int kb0 = lo / kTaPage, kb1 = pos / kTaPage;
+    if (gridDim.z > 1) {        // a contiguous share of the pages (possibly none)
+        const int per = (kb1 - kb0 + static_cast<int>(gridDim.z)) / static_cast<int>(gridDim.z);
+        kb0 += per * static_cast<int>(blockIdx.z);
+        kb1 = min(kb1, kb0 + per - 1);
+    }
+    const int sub = lane % LPR, row = lane / LPR;
+    const int col = tid % DV, grp = __builtin_amdgcn_readfirstlane(tid / DV);
+    float4_t qv[H], x[KU];
+    float v[PV][kTaPage], relv[HW], acc[H], mrun[HW], lrun[HW];
+#pragma unroll
+    for (int h = 0; h < H; ++h) acc[h] = 0.f;
+#pragma unroll
+    for (int i = 0; i < HW; ++i) {
+        mrun[i] = kNegBig;
+        lrun[i] = relv[i] = 0.f;
+    }
+    auto ask_keys = [&](int kb) {
+#pragma unroll
+        for (int i = 0; i < HW; ++i) {
+            const int h = wave + 4 * i, dist = pos - (kb * kTaPage + lane);
+            if (a.rel && h < H) relv[i] = a.rel[static_cast<int64_t>(hb + h) * a.rel_len + max(min(dist, a.rel_len - 1), 0)];
+        }
+#pragma unroll
+        for (int u = 0; u < KU; ++u) {
+            const int pg = u * 4 * ROWS / kTaPage, in = u * 4 * ROWS % kTaPage;
+            const float *page = a.k + bt[min(kb + pg, kb1)] * a.block_stride + (static_cast<int64_t>(kv) * kTaPage + in) * D;
+            x[u] = *reinterpret_cast<const float4_t *>(page + (wave * ROWS + row) * D + 4 * sub);
+        }
+    };
+    auto ask_values = [&](int kb) {
+#pragma unroll
+        for (int i = 0; i < PV; ++i) {
+            const float *page = a.v + bt[min(kb + grp + VP * i, kb1)] * a.block_stride + static_cast<int64_t>(gv) * DV * kTaPage;
+#pragma unroll
+            for (int k = 0; k < kTaPage; k += 4) {
+                const float4_t w = *reinterpret_cast<const float4_t *>(page + col * kTaPage + k);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[i][k + c] = w[c];
+            }
+        }
+    };
+    if (kb0 <= kb1) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) qv[h] = *reinterpret_cast<const float4_t *>(a.q + t * a.q_stride + (hb + h) * D + 4 * sub);
+        ask_keys(kb0);
+        ask_values(kb0);
+    }
+    for (int kb = kb0; kb <= kb1; kb += 4) {
+        const int first = max(lo - kb * kTaPage, 0), last = min(min(pos, kb1 * kTaPage + kTaPage - 1) - kb * kTaPage, kTaChunk - 1);
+        // 1. scores (what a key outside first .. last gives is not looked at)
+#pragma unroll
+        for (int u = 0; u < KU; ++u) {
+            float mine = 0.f;
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                float d = 0.f;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) d = fmaf(qv[h][c], x[u][c], d);
+                d = ta_lane_sum(d, LPR);
+                mine = sub == h ? d : mine;
+            }
+            if (sub < H) s[sub][(u * 4 + wave) * ROWS + row] = mine;
+            if ((u + 1) * H % 16 == 0) __builtin_amdgcn_sched_barrier(0);
+        }
+        float bias[HW];
+#pragma unroll
+        for (int i = 0; i < HW; ++i) bias[i] = relv[i];
+        if (kb + 4 <= kb1) ask_keys(kb + 4);
+        __syncthreads();
+        // 2. online softmax: wave w owns heads w and w + 4, a lane a key
+        const bool ok = lane >= first && lane <= last;
+#pragma unroll
+        for (int i = 0; i < HW; ++i) {
+            const int h = wave + 4 * i;
+            if (h < H) {
+                float m = kNegBig;
+                if (ok) {
+                    m = s[h][lane] * a.scale;
+                    if (a.softcap > 0.f) m = a.softcap * tanhf(m / a.softcap);
+                    if (a.rel) m += bias[i];
+                    if (a.slopes) m -= a.slopes[hb + h] * static_cast<float>(pos - (kb * kTaPage + lane));
+                }
+                const float mnew = fmaxf(mrun[i], wave_allreduce_max(m));
+                const float pj = ok ? expf(m - mnew) : 0.f;
+                const float csum = wave_allreduce_sum(pj);
+                const float al = expf(mrun[i] - mnew);      // first chunk: exp(-1e30 - m) = 0
+                lrun[i] = lrun[i] * al + csum;
+                mrun[i] = mnew;
+                p[h][lane] = pj;
+                if (lane == 0) alpha[h] = al;
+            }
+        }
+        __syncthreads();
+        // 3. weighted values (those outside first .. last do not count, whatever they hold)
+#pragma unroll
+        for (int h = 0; h < H; ++h) acc[h] *= alpha[h];
+#pragma unroll
+        for (int i = 0; i < PV; ++i) {
+            const int j0 = (grp + VP * i) * kTaPage;
+            if (j0 < first || j0 + kTaPage - 1 > last) {
+#pragma unroll
+                for (int k = 0; k < kTaPage; ++k)
+                    if (j0 + k < first || j0 + k > last) v[i][k] = 0.f;
+            }
+#pragma unroll
+            for (int k = 0; k < kTaPage; k += 4) {
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    const float4_t w = *reinterpret_cast<const float4_t *>(&p[h][j0 + k]);
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) acc[h] = fmaf(w[c], v[i][k + c], acc[h]);
+                }
+                if ((k / 4 + 1) * H % (H > 1 ? 8 : 4) == 0) {     // (else the sums sink below the next loads, and all the weights stay in registers)
+#pragma unroll
+                    for (int h = 0; h < H; ++h) asm volatile("" : "+v"(acc[h]));
+                }
+            }
+        }
+        if (kb + 4 <= kb1) ask_values(kb + 4);
+    }
+    if constexpr (VP > 1) {
+        if (grp > 0) {
+#pragma unroll
+            for (int h = 0; h < H; ++h) red[grp - 1][h][col] = acc[h];
+        }
+        __syncthreads();
+        if (grp == 0) {
+#pragma unroll
+            for (int g = 0; g < VP - 1; ++g)
+#pragma unroll
+                for (int h = 0; h < H; ++h) acc[h] += red[g][h][col];
+        }
+    }
+    if (gridDim.z > 1) {
+        const int64_t slot = (static_cast<int64_t>(blockIdx.z) * gridDim.x + t) * Hall + hb;
+#pragma unroll
+        for (int i = 0; i < HW; ++i) {
+            const int h = wave + 4 * i;
+            if (h < H && lane == 0) {
+                a.part_ml[(slot + h) * 2] = mrun[i];
+                a.part_ml[(slot + h) * 2 + 1] = lrun[i];
+            }
+        }
+        if (grp == 0) {
+#pragma unroll
+            for (int h = 0; h < H; ++h) a.part_o[(slot + h) * DV + col] = acc[h];
+        }
+        return;
+    }
+    __syncthreads();
+    // final scale of every head, as in window_attn_kernel
+#pragma unroll
+    for (int i = 0; i < HW; ++i) {
+        const int h = wave + 4 * i;
+        if (h < H) {
+            float al = 1.f, l = lrun[i];
+            if (a.sink) {
+                const float sk = a.sink[hb + h], big = fmaxf(mrun[i], sk);
+                al = expf(mrun[i] - big);
+                l = l * al + expf(sk - big);
+            }
+            if (lane == 0) alpha[h] = al / l;
+        }
+    }
+    __syncthreads();
+    if (grp > 0 || col >= a.out_dim) return;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+        float o = acc[h] * alpha[h];
+        const int64_t hc = static_cast<int64_t>(hb + h) * a.out_dim + col;
+        if (a.gate) o /= 1.0f + expf(-a.gate[t * a.gate_stride + hc]);
+        static_cast<float *>(a.out)[t * a.out_stride + hc] = o;
+    }
+}
+
+// Launches window_attn_heads_kernel where it serves the heads; false: nothing was launched.
+static bool launch_heads(const HeadsParams &a, int rep, int d, int dv, const dim3 &grid, hipStream_t st) {
+#define SWL_HEADS(D, DV, H)                                                                                         \
+    if (d == D && dv == DV && rep == H) {                                                                           \
+        hipLaunchKernelGGL((window_attn_heads_kernel<D, DV, H>), grid, dim3(kTaThreads), 0, st, a);                 \
+        return true;                                                                                                \
+    }
+#define SWL_HEADS_OF(D, DV) SWL_HEADS(D, DV, 1) SWL_HEADS(D, DV, 2) SWL_HEADS(D, DV, 4) SWL_HEADS(D, DV, 8)
+    SWL_HEADS_OF(128, 128)
+    SWL_HEADS_OF(64, 64)
+    SWL_HEADS_OF(64, 128)
+#undef SWL_HEADS_OF
+#undef SWL_HEADS
+    return false;
+}
+
 } // namespace swl
 
 extern "C" int swl_masked_attn_shares(void *out, const void *q, const void *k_cache, const void *v_cache,
@@ -255,6 +479,15 @@ extern "C" int swl_masked_attn_shares(void *out, const void *q, const void *k_ca
     float *part_ml = key_splits > 1 ? scratch + static_cast<int64_t>(key_splits) * num_tokens * num_q_heads * vdim : nullptr;
     const dim3 grid(static_cast<unsigned>(num_tokens), groups, static_cast<unsigned>(key_splits));
     hipStream_t st = static_cast<hipStream_t>(stream);
+    bool served = false;
+    if (!talk && dtype == SWL_F32 && k_wide && v_wide && q_tok_stride % 4 == 0 && swl::aligned16(q) && num_kv_heads <= 65535) {
+        const swl::HeadsParams a{out, static_cast<const float *>(q), static_cast<const float *>(k_cache), static_cast<const float *>(v_cache),
+                                 block_table, tok_seq, tok_pos, rel, sink, slopes, static_cast<const float *>(gate), part_o, part_ml, q_tok_stride,
+                                 block_stride, out_stride, gate_stride, rel_len, window, mask_kind, max_blocks_per_seq, num_kv_heads, num_v_heads,
+                                 out_dim, scale, softcap};
+        served = swl::launch_heads(a, num_q_heads / num_kv_heads, dim, vdim,
+                                   dim3(static_cast<unsigned>(num_tokens), static_cast<unsigned>(num_kv_heads), static_cast<unsigned>(key_splits)), st);
+    }
     SWL_DISPATCH_DTYPE3(dtype, T, {
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, grid, dim3(swl::kTaThreads), lds, st, static_cast<T *>(out), static_cast<const T *>(q),
@@ -263,7 +496,7 @@ extern "C" int swl_masked_attn_shares(void *out, const void *q, const void *k_ca
                                block_stride, mask_kind, sink, num_v_heads, out_f32, num_q_heads, slopes, out_dim, out_stride,
                                static_cast<const T *>(gate), gate_stride, part_o, part_ml, k_wide, v_wide);
         };
-        switch (swl::ta_share(num_q_heads / num_kv_heads, hpg)) {
+        if (!served) switch (swl::ta_share(num_q_heads / num_kv_heads, hpg)) {
         case 8: go(&swl::window_attn_kernel<T, 8>); break;
         case 4: go(&swl::window_attn_kernel<T, 4>); break;
         case 2: go(&swl::window_attn_kernel<T, 2>); break;

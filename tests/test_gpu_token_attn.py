@@ -122,3 +122,45 @@ def test_experts_by_assignment(width, ff, top, form):
         want += (1.0 if form == "clamped_in" else wts[:, j:j + 1].double()) * torch.einsum("tf,twf->tw", y, down.double()[idx[:, j]])
     # two fp32 sums of up to 1024 terms of order one, one behind the other
     assert (got.double().cpu() - want).abs().max() <= 2.0 ** -17 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("H,G,GV,d,dv,kind", [(4, 4, 2, 128, 128, "slopes"), (4, 2, 2, 128, 128, "gate"), (8, 2, 2, 128, 128, "rel"), (8, 1, 1, 128, 128, "chunk"),
+                                              (3, 3, 3, 64, 64, "rel"), (6, 3, 3, 64, 64, "window"), (4, 1, 1, 64, 64, "sink"), (16, 2, 1, 64, 64, "cap"),
+                                              (8, 8, 4, 64, 128, "window"), (8, 4, 2, 64, 128, "cap"), (8, 2, 1, 64, 128, "gate"), (8, 1, 1, 64, 128, "sink"),
+                                              (3, 1, 1, 128, 128, "odd")])
+def test_heads_of_a_key_head_in_fp32(H, G, GV, d, dv, kind):
+    """The kernel that takes the heads of one key head (1, 2, 4 or 8 of them; three stay with the other), in one and in many key shares;
+    what stands in a sequence's last page behind its keys does not count, whatever it is."""
+    from swiftllm_amd.worker.kernels import window_attn as wa
+    g = torch.Generator().manual_seed(H * d + dv)
+    lens = [a + n for _, a, n in PARTS]
+    pool, sl, table, ks, vs = _pool(lens, G, GV, d, dv, torch.float32, g)
+    for i, n in enumerate(lens):
+        if n % 16:
+            blk = int(table[i + 1, n // 16])
+            pool[blk, sl.k_offset:sl.k_offset + 16 * G * d].view(G, 16, d)[:, n % 16:] = float("nan")
+            pool[blk, sl.v_offset:sl.v_offset + 16 * GV * dv].view(GV, dv, 16)[:, :, n % 16:] = float("nan")
+    seq, pos, _ = _spans(PARTS)
+    n = seq.shape[0]
+    wide = torch.randn(n, H * d + 8, generator=g)
+    q = wide[:, 4:4 + H * d]
+    rel = torch.randn(H, 90, generator=g) if kind == "rel" else None
+    out_dim = dv - 5 if kind in ("gate", "slopes") else dv
+    gate = torch.randn(n, H * out_dim, generator=g) if kind == "gate" else None
+    spec = wa.AttentionSpec(H, G, d, dv, d ** -0.5, window={"window": 70, "chunk": 100}.get(kind, 0), num_v_heads=GV, softcap=1.5 if kind == "cap" else 0.0,
+                            mask_kind=wa.MASK_CHUNK if kind == "chunk" else wa.MASK_WINDOW, out_f32=kind == "cap", out_dim=out_dim,
+                            sink=torch.randn(H, generator=g).cuda() if kind == "sink" else None,
+                            slopes=(torch.rand(H, generator=g) * 0.1).cuda() if kind == "slopes" else None)
+    for reach in (4096, 64):        # (sixteen key shares; one)
+        if kind == "rel":
+            mixer = type("Mixer", (), dict(num_q_heads=H, num_kv_heads=G, head_dim=d, value_dim=dv, window=0, scale=d ** -0.5, softcap=0.0,
+                                           q_size=H * d, k_size=0, v_size=0))
+            o = wa.window_attention(q.cuda().contiguous(), None, pool, sl, table, seq, pos, mixer, None, reach, rel=rel.cuda())
+        else:
+            o = wa.masked_attention(wide.cuda()[:, 4:4 + H * d], pool, sl, table, seq, pos, spec, None, reach, gate=gate.cuda() if gate is not None else None)
+        at = 0
+        for b, (_, a, m) in enumerate(PARTS):
+            want = _want(q[at:at + m].double().reshape(m, H, d), ks[b], vs[b], a, spec, rel.double() if rel is not None else None,
+                         gate[at:at + m].double() if gate is not None else None)
+            assert (o[at:at + m].double().cpu() - want).abs().max() <= _bound(want, torch.float32), (reach, b)
+            at += m
