@@ -596,7 +596,10 @@ int swl_masked_attn(void *out, const void *q, const void *k_cache, const void *v
                     const float *slopes, int32_t out_dim, int64_t out_stride, const void *gate, int64_t gate_stride,
                     int32_t dtype, swl_stream_t stream);
 /* swl_masked_attn with every token's pages shared out over key_splits (at most 64) workgroups, whose partial results (scratch:
- * key_splits * num_tokens * num_q_heads * (vdim + 2) floats, 16-byte aligned) a second launch combines. */
+ * key_splits * num_tokens * num_q_heads * (vdim + 2) floats, 16-byte aligned) a second launch combines.
+ * out_f32 = SWL_OUT_SHARES (here and in the tiles form, key_splits > 1, without sink and gate): that launch is left to the caller, out may be
+ * NULL. */
+#define SWL_OUT_SHARES 2
 int swl_masked_attn_shares(void *out, const void *q, const void *k_cache, const void *v_cache, const int32_t *block_table,
                            const int32_t *tok_seq, const int32_t *tok_pos, const float *talk, const float *rel, int32_t rel_len,
                            int64_t num_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t dim, int32_t vdim,
@@ -723,6 +726,12 @@ int swl_latent_expand(void *out, const void *k_cache, const void *uk, const void
 int swl_diff_head_combine(void *out, const float *maps, const void *gate, int64_t gate_stride, float lambda, float mult,
                           float eps, int64_t num_tokens, int32_t num_heads, int32_t vdim, int32_t dtype,
                           swl_stream_t stream);
+/* The same from the key shares of both maps, as swl_masked_attn_tiles / _shares (natural: the latter) leave them with out_f32 =
+ * SWL_OUT_SHARES: fp32 [shares][tokens][2 heads][vdim] results, then [shares][tokens][2 heads][2] maxima and sums. vdim % 4 == 0, at most 256;
+ * at most 32 shares; 16-byte aligned. */
+int swl_diff_head_combine_shares(void *out, const float *shares, int32_t num_shares, int32_t natural, const void *gate, int64_t gate_stride,
+                                 float lambda, float mult, float eps, int64_t num_tokens, int32_t num_heads, int32_t vdim, int32_t dtype,
+                                 swl_stream_t stream);
 int swl_head_gate(void *y, const void *gate, int64_t gate_stride, int64_t num_tokens, int32_t num_heads, int32_t vdim,
                   int32_t dtype, swl_stream_t stream);
 

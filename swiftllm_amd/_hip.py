@@ -133,6 +133,7 @@ SIGNATURES = {
                         _F64, _I32, _I32, _I32, _P],
     "swl_latent_decode": [_P, _P, _P, _P, _P, _P, _I64, _I32, _I64, _I32, _F32, _I32, _I64, _I32, _I32, _P],
     "swl_latent_unfold": [_P, _P, _P, _P, _P, _I64, _I64, _I32, _I32, _I32, _I32, _P],
+    "swl_diff_head_combine_shares": [_P, _P, _I32, _I32, _P, _I64, _F32, _F32, _F32, _I64, _I32, _I32, _I32, _P],
     "swl_diff_head_combine": [_P, _P, _P, _I64, _F32, _F32, _F32, _I64, _I32, _I32, _I32, _P],
     "swl_head_gate": [_P, _P, _I64, _I64, _I32, _I32, _I32, _P],
     "swl_polynorm": [_P, _P, _F32, _F32, _F32, _F32, _F32, _I64, _I32, _I32, _P],

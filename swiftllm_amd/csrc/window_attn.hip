@@ -449,7 +449,8 @@ extern "C" int swl_masked_attn_shares(void *out, const void *q, const void *k_ca
     if (gate && gate_stride < static_cast<int64_t>(num_q_heads) * out_dim) return SWL_ERR_BAD_ARG;
     if (key_splits < 1 || key_splits > 64 || (key_splits > 1 && (!scratch || !swl::aligned16(scratch)))) return SWL_ERR_BAD_ARG;
     if (num_tokens == 0) return SWL_OK;
-    if (!out || !q || !k_cache || !v_cache || !block_table || !tok_seq || !tok_pos || (rel && rel_len <= 0))
+    if (out_f32 == SWL_OUT_SHARES && (key_splits < 2 || sink || gate)) return SWL_ERR_BAD_ARG;
+    if ((!out && out_f32 != SWL_OUT_SHARES) || !q || !k_cache || !v_cache || !block_table || !tok_seq || !tok_pos || (rel && rel_len <= 0))
         return SWL_ERR_BAD_ARG;
     // heads per workgroup: all of them when they are mixed, else as many as its accumulators and LDS hold
     int hpg = num_q_heads;
@@ -502,7 +503,7 @@ extern "C" int swl_masked_attn_shares(void *out, const void *q, const void *k_ca
         case 2: go(&swl::window_attn_kernel<T, 2>); break;
         default: go(&swl::window_attn_kernel<T, 1>); break;
         }
-        if (key_splits > 1) {
+        if (key_splits > 1 && out_f32 != SWL_OUT_SHARES) {
             const int64_t rows = num_tokens * num_q_heads;
             if (rows > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
             hipLaunchKernelGGL((swl::window_attn_combine_kernel<T, true>), dim3(static_cast<unsigned>(rows)), dim3(vdim < 256 ? 64 : 256), 0,

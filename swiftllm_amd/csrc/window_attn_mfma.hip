@@ -352,7 +352,7 @@ int launch_wm(int hpw, dim3 grid, size_t lds, hipStream_t s, T *out, const T *q,
         hipLaunchKernelGGL((window_attn_mfma_kernel<T, D, DV, 1, 1, false, true>), grid, dim3(64), 0, s, out, q, kc, vc, bt, ts,
                            tp, r0, cn, nullptr, rel, rel_len, H, G, qs, window, scale, softcap, mb, bs, po, pml, nt, nbuf,
                            mask_kind, sink, GV, out_f32, hpg, slopes, od, ostr, gate, gstr);
-        if (grid.y > 1) {
+        if (grid.y > 1 && out_f32 != SWL_OUT_SHARES) {
             const int64_t rows = nt * H;
             hipLaunchKernelGGL((window_attn_combine_kernel<T>), dim3(static_cast<unsigned>(rows)), dim3(DV < 256 ? 64 : 256), 0,
                                s, out, po, pml, rows, DV, static_cast<int>(grid.y), sink, H, out_f32, od, ostr, gate, gstr);
@@ -382,7 +382,7 @@ int launch_wm(int hpw, dim3 grid, size_t lds, hipStream_t s, T *out, const T *q,
     }
 #undef SWL_WM_LAUNCH
 #undef SWL_WM_LAUNCH1
-    if (grid.y > 1) {
+    if (grid.y > 1 && out_f32 != SWL_OUT_SHARES) {
         const int64_t rows = nt * H;
         hipLaunchKernelGGL((window_attn_combine_kernel<T>), dim3(static_cast<unsigned>(rows)), dim3(DV < 256 ? 64 : 256), 0, s,
                            out, po, pml, rows, DV, static_cast<int>(grid.y), sink, H, out_f32, od, ostr, gate, gstr);
@@ -461,7 +461,8 @@ extern "C" int swl_masked_attn_tiles(void *out, const void *q, const void *k_cac
         if (hpg > 4 * per_wave) hpg = 4 * per_wave;
     }
     if (num_tiles == 0) return SWL_OK;
-    if (!out || !q || !k_cache || !v_cache || !block_table || !tok_seq || !tok_pos || !tile_row0 || !tile_cnt ||
+    if (out_f32 == SWL_OUT_SHARES && (key_splits < 2 || sink || gate)) return SWL_ERR_BAD_ARG;
+    if ((!out && out_f32 != SWL_OUT_SHARES) || !q || !k_cache || !v_cache || !block_table || !tok_seq || !tok_pos || !tile_row0 || !tile_cnt ||
         (rel && rel_len <= 0))
         return SWL_ERR_BAD_ARG;
     if ((q_tok_stride & 3) || (block_stride & 3) || (reinterpret_cast<uintptr_t>(q) & 7) ||

@@ -4,7 +4,7 @@ import torch
 
 from swiftllm_amd import _hip
 
-from .window_attn import PoolSlice
+from .window_attn import KeyShares, PoolSlice
 
 
 def rotary_frequencies(rot, device) -> torch.Tensor:
@@ -132,17 +132,24 @@ def latent_rope_and_store_kv(proj: torch.Tensor, qa: torch.Tensor, freq: torch.T
               float(mixer.rot.multiplier), k_dim, v_dim, _hip.dtype_code3(proj.dtype), _hip.stream())
 
 
-def diff_head_combine(maps: torch.Tensor, gate: torch.Tensor, lam: float, mult: float, eps: float, num_heads: int,
-                      vdim: int, out_dtype: torch.dtype) -> torch.Tensor:
-    """maps fp32 [T, 2 * heads * vdim] (map-major) -> [T, heads * vdim]: unit_rms(a1 - lam * a2) * mult * sigmoid(gate[t, h]).
-    gate: [T, heads] logits, possibly a column slice of a wider matrix."""
-    _hip.require_gpu_tensor(maps, "maps")
-    n = maps.shape[0]
-    assert maps.dtype == torch.float32 and maps.is_contiguous() and maps.shape[1] == 2 * num_heads * vdim
+def diff_head_combine(maps, gate: torch.Tensor, lam: float, mult: float, eps: float, num_heads: int, vdim: int,
+                      out_dtype: torch.dtype) -> torch.Tensor:
+    """maps fp32 [T, 2 * heads * vdim] (map-major) or their KeyShares -> [T, heads * vdim]: unit_rms(a1 - lam * a2) * mult *
+    sigmoid(gate[t, h]). gate: [T, heads] logits (KeyShares: not None), possibly a column slice of a wider matrix."""
+    shares = maps if isinstance(maps, KeyShares) else None
+    data = maps if shares is None else shares.data
+    _hip.require_gpu_tensor(data, "maps")
+    n = data.shape[0] if shares is None else gate.shape[0]
+    assert data.dtype == torch.float32 and data.is_contiguous()
+    assert data.shape[1] == 2 * num_heads * vdim if shares is None else data.numel() == shares.shares * n * 2 * num_heads * (vdim + 2)
     assert gate is None or (gate.shape == (n, num_heads) and gate.stride(1) == 1 and gate.dtype == out_dtype)
-    out = torch.empty((n, num_heads * vdim), dtype=out_dtype, device=maps.device)
-    _hip.call("swl_diff_head_combine", _hip.ptr(out), _hip.ptr(maps), _hip.ptr(gate), gate.stride(0) if gate is not None else 0,
-              float(lam), float(mult), float(eps), n, num_heads, vdim, _hip.dtype_code3(out_dtype), _hip.stream())
+    out = torch.empty((n, num_heads * vdim), dtype=out_dtype, device=data.device)
+    rest = (_hip.ptr(gate), gate.stride(0) if gate is not None else 0, float(lam), float(mult), float(eps), n, num_heads, vdim,
+            _hip.dtype_code3(out_dtype), _hip.stream())
+    if shares is not None:
+        _hip.call("swl_diff_head_combine_shares", _hip.ptr(out), _hip.ptr(data), shares.shares, 1 if shares.natural else 0, *rest)
+    else:
+        _hip.call("swl_diff_head_combine", _hip.ptr(out), _hip.ptr(data), *rest)
     return out
 
 

@@ -373,14 +373,30 @@ def choose_heads_per_group(spec: AttentionSpec) -> int:
     return min(spec.num_q_heads, 4 * per_wave)
 
 
+class KeyShares:
+    """Results of attention whose keys were shared out over workgroups, not added up yet (csrc/attn_combine.h): fp32 [shares][tokens][heads]
+    [columns], then a maximum and a sum for every one; natural: the maxima are not in base-2 units."""
+    __slots__ = ("data", "shares", "natural")
+    MOST, MAX_DIM = 32, 256     # (swl_diff_head_combine_shares)
+
+    def __init__(self, data: torch.Tensor, shares: int, natural: bool):
+        self.data, self.shares, self.natural = data, shares, natural
+
+    @classmethod
+    def serve(cls, splits: int, value_dim: int) -> bool:
+        return 1 < splits <= cls.MOST and value_dim <= cls.MAX_DIM and value_dim % 4 == 0
+
+
 def masked_attention(q: torch.Tensor, pool: torch.Tensor, pool_slice: PoolSlice, block_table: torch.Tensor,
                      tok_seq: torch.Tensor, tok_pos: torch.Tensor, spec: AttentionSpec, tiles=None,
-                     max_positions: int = 1 << 20, out: torch.Tensor = None, gate: torch.Tensor = None) -> torch.Tensor:
+                     max_positions: int = 1 << 20, out: torch.Tensor = None, gate: torch.Tensor = None, leave_shares: bool = False):
     """-> [T, num_q_heads * out_dim] (fp32 when spec.out_f32, else q's dtype), written to `out` when given (a column slice of wider
     rows is fine), times sigmoid(gate) element by element when `gate` (likewise) is. q: rows whose first num_q_heads * head_dim
     columns are the queries (a column slice of a wider matrix is fine); keys and values come from the pool, which already
-    holds this step's tokens."""
+    holds this step's tokens. leave_shares (without sink, gate and out): a caller that adds up key shares itself takes them as KeyShares
+    where the keys are shared out."""
     _hip.require_gpu_tensor(q, "q")
+    assert not leave_shares or (spec.sink is None and gate is None and out is None and spec.out_dim == spec.value_dim)
     assert q.dim() == 2 and q.stride(1) == 1 and q.shape[1] >= spec.num_q_heads * spec.head_dim
     assert pool.is_contiguous() and pool.dtype == q.dtype and tok_pos.dtype == torch.int32 and tok_seq.dtype == torch.int32
     sink = spec.sink
@@ -410,17 +426,19 @@ def masked_attention(q: torch.Tensor, pool: torch.Tensor, pool_slice: PoolSlice,
             groups = -(-spec.num_q_heads // hpg)
             splits = choose_key_splits(row0.shape[0] * groups, spec, max_positions)
         splits, scratch = share_scratch(q.device, splits, n * spec.num_q_heads * (spec.value_dim + 2))
+        leave = leave_shares and KeyShares.serve(splits, spec.value_dim)
         _hip.call("swl_masked_attn_tiles", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq),
                   _hip.ptr(tok_pos), _hip.ptr(row0), _hip.ptr(cnt), 0, 0, 0, row0.shape[0], spec.num_q_heads,
                   spec.num_kv_heads, spec.head_dim, spec.value_dim, q.stride(0), spec.window, float(spec.scale),
                   float(spec.softcap), block_table.shape[1], pool.shape[1], splits, _hip.ptr(scratch), n, spec.mask_kind,
-                  _hip.ptr(sink), spec.num_v_heads, 1 if spec.out_f32 else 0, hpg, _hip.ptr(spec.slopes), spec.out_dim,
+                  _hip.ptr(sink), spec.num_v_heads, 2 if leave else 1 if spec.out_f32 else 0, hpg, _hip.ptr(spec.slopes), spec.out_dim,
                   out.stride(0), _hip.ptr(gate), gate_stride, _hip.dtype_code(q.dtype), _hip.stream())
-        return out
+        return KeyShares(scratch, splits, False) if leave else out
     splits, scratch = token_key_splits(n, spec.num_q_heads, spec.value_dim, spec, max_positions, q.device)
+    leave = leave_shares and KeyShares.serve(splits, spec.value_dim)
     _hip.call("swl_masked_attn_shares", _hip.ptr(out), _hip.ptr(q), kp, vp, _hip.ptr(block_table), _hip.ptr(tok_seq),
               _hip.ptr(tok_pos), 0, 0, 0, n, spec.num_q_heads, spec.num_kv_heads, spec.head_dim, spec.value_dim, q.stride(0),
               spec.window, float(spec.scale), float(spec.softcap), block_table.shape[1], pool.shape[1], spec.mask_kind,
-              _hip.ptr(sink), spec.num_v_heads, 1 if spec.out_f32 else 0, _hip.ptr(spec.slopes), spec.out_dim, out.stride(0),
+              _hip.ptr(sink), spec.num_v_heads, 2 if leave else 1 if spec.out_f32 else 0, _hip.ptr(spec.slopes), spec.out_dim, out.stride(0),
               _hip.ptr(gate), gate_stride, splits, _hip.ptr(scratch), _hip.dtype_code3(q.dtype), _hip.stream())
-    return out
+    return KeyShares(scratch, splits, True) if leave else out

@@ -31,7 +31,7 @@ class RosilixDiffAttention:
             maps = torch.zeros((h.shape[0], 2 * mx.o_size), dtype=torch.float32, device=h.device)
         else:
             maps = masked_attention(proj, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq, ctx.tok_pos, self.spec,
-                                    ctx.tiles, self.max_positions)
+                                    ctx.tiles, self.max_positions, leave_shares=True)
         gate = proj[:, w.gate_col:w.gate_col + mx.num_q_heads]
         y = diff_head_combine(maps, gate, w.lam, 1.0 - mx.diff, self.eps, mx.num_q_heads, mx.value_dim, h.dtype)
         return _project_partials(y, w.o, self.skinny)

@@ -686,3 +686,36 @@ def test_trace_runner_replays_a_mixed_schedule(tmp_path, dtype, tol):
             assert close(got[-1], want[-1], dtype, tol), f"step {n}"
     assert close(torch.cat(got), torch.cat(want), dtype, tol)
 
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,G,d,dv,reach", [(1, 16, 4, 64, 128, 4096), (33, 4, 2, 64, 128, 1024), (5, 3, 3, 32, 64, 256), (3, 2, 1, 320, 256, 4096)])
+def test_diff_combine_of_key_shares(T, H, G, d, dv, reach, dtype):
+    """Key shares of both maps added up where they are combined, against the maps added up first; the shares of short sequences are empty."""
+    from swiftllm_amd.worker.kernels import window_attn as wa
+    from swiftllm_amd.worker.kernels.rope_kv import diff_head_combine
+    g = torch.Generator().manual_seed(T * H + d)
+    lens = [(7, 16, 300, 129, 1)[i % 5] for i in range(T)]
+    blocks = [-(-n // 16) for n in lens]
+    pool = torch.randn(sum(blocks), 16 * (2 * G * d + G * dv), generator=g).to(dtype).cuda()
+    table, at = torch.zeros(T, max(blocks), dtype=torch.int32), 0
+    for i, b in enumerate(blocks):
+        table[i, :b] = torch.arange(at, at + b)
+        at += b
+    seq, pos = torch.arange(T, dtype=torch.int32).cuda(), (torch.tensor(lens, dtype=torch.int32) - 1).cuda()
+    q = torch.randn(T, 2 * H * d, generator=g).to(dtype).cuda()
+    gate = torch.randn(T, H + 2, generator=g).to(dtype).cuda()[:, 1:1 + H]
+    spec = wa.AttentionSpec(2 * H, 2 * G, d, dv, d ** -0.5, num_v_heads=G, out_f32=True)
+    tiles = (seq, torch.ones_like(seq))
+    args = (q, pool, wa.PoolSlice(0, 32 * G * d), table.cuda(), seq, pos, spec, tiles, reach)
+    shares, maps = wa.masked_attention(*args, leave_shares=True), wa.masked_attention(*args)
+    assert isinstance(shares, wa.KeyShares) and shares.natural == (dtype == torch.float32) and shares.shares > 1
+    got = diff_head_combine(shares, gate, 0.3, 0.7, 1e-6, H, dv, dtype).double()
+    m = maps.double().view(T, 2, H, dv)
+    o = m[:, 0] - 0.3 * m[:, 1]
+    want = (o / torch.sqrt((o * o).mean(-1, keepdim=True) + 1e-6) * 0.7 * torch.sigmoid(gate.double())[:, :, None]).view(T, H * dv)
+    # one rounding to the type; the difference of two fp32 sums of up to 32 terms each, over its own root mean square
+    eps = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    cancel = float((m.abs().amax(-1).sum(1) / torch.sqrt((o * o).mean(-1) + 1e-6)).max())
+    assert ((got - want).abs() <= 1.01 * eps * want.abs() + 64 * 2.0 ** -24 * cancel + 2.0 ** -24).all()
+    assert torch.isfinite(got).all()
