@@ -389,6 +389,198 @@ __global__ __launch_bounds__(kRkThreads) void qkv_conv_rope_store_kv_kernel(
     }
 }
 
+// The same for heads of 8 LPH columns (16, 32, 64 or 128), up to four taps and rows of whole aligned pieces of eight: a lane's eight channels
+// stay in registers, a head's sum and its rotation are exchanges between neighbouring lanes. What bounds it is the chain of a token's
+// workgroup, which above is a round trip for every earlier input and the norm's and the rotation's passes over LDS: here the row, up to
+// three earlier ones, taps, bias and norm weights are asked for together. From kRkManyTokens tokens a workgroup takes four in a row, for which
+// the taps (8 to 16 KiB a row of 2 KiB) are read once and whose earlier inputs move on by one in registers; below, its longer chain costs more (10 us
+// at any count).
+// us, above -> one token / four, heads of 128, bf16: 8 over 2 with 4 taps and norm 128 tokens 9.6 -> 6.0 / 10.3, 1000 12.8 -> 7.9 / 10.8, 1500 15.9 -> 12.3 /
+// 11.7, 2030 20.9 -> 16.1 / 15.2, 3000 27.0 -> 20.7 / 14.8; without norm 2030 14.6 -> 15.6 / 14.7, 5000 26.3 -> 30.2 / 23.4; 16 over 4 with norm, no taps 500
+// 14.1 -> 7.2 / 10.7, 1500 24.2 -> 13.2 / 14.5, 2030 31.6 -> 18.1 / 15.7; fp32, 3 tokens 13.2 -> 5.9, 500 14.1 -> 7.4.
+constexpr int kRkManyTokens = 1536;
+template <typename T, int LPH, int TOK>
+__global__ __launch_bounds__(kRkThreads, 3) void qkv_conv_rope_rows_kernel(
+    const T *rows, int64_t tok_stride, T *q_out, int64_t q_out_stride, const float *bias, const float *conv_w, int taps,
+    const float *q_w, const float *k_w, const double *freq, int rot_dims, int half, double rot_mult, float v_mult, T *k_cache,
+    T *v_cache, const int32_t *block_table, int max_blocks_per_seq, int64_t block_stride, float *state, int64_t slot_stride,
+    int64_t tail_off, const int32_t *tok_pos, const int32_t *tok_start, const int32_t *tok_state, const int32_t *tok_seq,
+    int64_t num_tokens, int nq, int nk, int dv, int k_dim, int v_dim, float eps) {
+    constexpr int d = 8 * LPH, MOST = 3;
+    __shared__ float cs[TOK][d / 2], sn[TOK][d / 2];
+    __shared__ int meta[TOK][5];        // position, first position of the portion, state slot and parity, ends its portion, block
+    // workgroup -> its tokens; those of a page on one XCD (page_token)
+    int64_t t0;
+    if constexpr (TOK == 1) {
+        t0 = page_token();
+    } else {
+        constexpr int RUN = 128 / TOK;
+        const unsigned b = blockIdx.x, first = b & ~(RUN - 1u);
+        t0 = (gridDim.x - first < RUN ? b : first + (b & 7) * (16 / TOK) + ((b >> 3) & (16 / TOK - 1))) * TOK;
+    }
+    const int n = static_cast<int>(min<int64_t>(TOK, num_tokens - t0));
+    const int lane = threadIdx.x & 63, pairs = rot_dims >> 1, heads = nq + nk, C = heads * d + nk * dv;
+    const int step = blockDim.x * 8, R = conv_w ? taps - 1 : 0;
+    const bool store = k_cache != nullptr;
+    float past[MOST][8], wk[MOST + 1][8], b[8], wn[8];      // past[k - 1], wk[k]: the input k tokens back and its weights
+    T raw[TOK][8];
+    auto earlier = [&](int64_t t, int code, int pos, int start, int c) {        // the inputs before token t, from rows of its portion or the tail
+        const float *old_tail = state + static_cast<int64_t>(code >> 1) * slot_stride + tail_off + static_cast<int64_t>(code & 1) * R * C;
+#pragma unroll
+        for (int k = 1; k <= MOST; ++k)
+            if (k <= R && pos >= k) {       // (uniform)
+                if (pos - k >= start) ConvTail::row8(rows + (t - k) * tok_stride + c, past[k - 1]);
+                else ConvTail::row8(old_tail + static_cast<int64_t>(R - (start - (pos - k))) * C + c, past[k - 1]);
+            }
+    };
+    auto ask = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < TOK; ++i) {
+            const T *p = rows + (t0 + min(i, n - 1)) * tok_stride + c;
+            if constexpr (sizeof(T) == 2) {
+                const vec8_t<T> x = load8(p);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) raw[i][j] = x[j];
+            } else {
+                ConvTail::row8(p, raw[i]);
+            }
+        }
+        if (R > 0) earlier(t0, tok_state[t0], tok_pos[t0], tok_start[t0], c);
+        if (conv_w) {
+#pragma unroll
+            for (int k = 0; k <= MOST; ++k)
+                if (k <= R) ConvTail::row8(conv_w + static_cast<int64_t>(R - k) * C + c, wk[k]);
+        }
+        if (bias) ConvTail::row8(bias + c, b);
+        if (q_w && c < heads * d) ConvTail::row8((c < nq * d ? q_w : k_w) + c % d, wn);
+    };
+#pragma unroll
+    for (int j = 0; j < 8; ++j) b[j] = wn[j] = 0.f;
+    if (threadIdx.x * 8 < C) ask(threadIdx.x * 8);
+    if (static_cast<int>(threadIdx.x) < n) {
+        const int64_t t = t0 + threadIdx.x;
+        const int pos = tok_pos[t], seq = tok_seq[t];
+        int *m = meta[threadIdx.x];
+        m[0] = pos;
+        m[1] = R > 0 ? tok_start[t] : 0;
+        m[2] = R > 0 ? tok_state[t] : 0;
+        m[3] = t + 1 == num_tokens || tok_seq[t + 1] != seq;
+        m[4] = store ? block_table[static_cast<int64_t>(seq) * max_blocks_per_seq + pos / kRkBlock] : 0;
+    }
+    for (int i = threadIdx.x; i < n * pairs; i += blockDim.x) {
+        const int u = i / pairs, p = i - u * pairs;
+        const double a = static_cast<double>(tok_pos[t0 + u]) * freq[p];
+        cs[u][p] = static_cast<float>(cos(a) * rot_mult);
+        sn[u][p] = static_cast<float>(sin(a) * rot_mult);
+    }
+    __syncthreads();
+    for (int c = threadIdx.x * 8; c < C; c += step) {
+        if (c >= step) ask(c);
+#pragma unroll
+        for (int i = 0; i < TOK; ++i) {
+            if (i >= n) break;      // (uniform)
+            const int64_t t = t0 + i;
+            auto of = [&](int what) { return __builtin_amdgcn_readfirstlane(meta[i][what]); };
+            const int pos = of(0), off = pos % kRkBlock;
+            const int64_t blk = of(4);
+            T *qrow = q_out + t * q_out_stride, *kpage = k_cache + blk * block_stride, *vpage = v_cache + blk * block_stride;
+            float a[8], cur[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) cur[j] = to_f(raw[i][j]);
+            if (conv_w) {
+                // (a token whose portion begins with it finds its earlier inputs in the tail; else they moved on by one)
+                if (i > 0 && R > 0 && of(1) == pos) earlier(t, of(2), pos, pos, c);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) a[j] = 0.f;
+#pragma unroll
+                for (int k = MOST; k >= 1; --k) {
+                    if (k <= R && pos >= k) {       // inputs before the sequence are zero, biases included
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) a[j] += wk[k][j] * (past[k - 1][j] + b[j]);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j) a[j] = a[j] + wk[0][j] * (cur[j] + b[j]);
+                if (R > 0 && of(3)) {
+                    const int code = of(2);     // (the layout of conv_tail.h; the input k tokens back becomes entry R - 1 - k)
+                    float *new_tail = state + static_cast<int64_t>(code >> 1) * slot_stride + tail_off + static_cast<int64_t>(1 - (code & 1)) * R * C;
+#pragma unroll
+                    for (int k = 0; k < MOST; ++k)
+                        if (k < R && pos >= k)
+                            ConvTail::put8<float>(new_tail + static_cast<int64_t>(R - 1 - k) * C + c, k == 0 ? cur : past[k > 0 ? k - 1 : 0]);
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+#pragma unroll
+                    for (int k = MOST - 1; k > 0; --k) past[k][j] = past[k - 1][j];
+                    past[0][j] = cur[j];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) a[j] = cur[j] + b[j];
+            }
+            if (c >= heads * d) {       // values: 16 tokens of a column together
+                if (store) {
+                    const int x = c - heads * d, g = x / dv;
+                    T *dst = vpage + (static_cast<int64_t>(g) * v_dim + (x - g * dv)) * kRkBlock + off;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) dst[j * kRkBlock] = to_t<T>(a[j] * v_mult);
+                }
+                continue;
+            }
+            const int h = c / d, e0 = c - h * d;
+            if (q_w) {
+                float ss = 0.f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) ss += a[j] * a[j];
+                ss = group_allreduce_sum<LPH>(ss);
+                const float r = 1.0f / sqrtf(ss / static_cast<float>(d) + eps);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) a[j] = a[j] * r * wn[j];
+            }
+            const bool turns = e0 < rot_dims, first = e0 < pairs;
+            if (half) {     // (the partner's columns are another lane's of the head)
+                const int from = !turns ? lane : first ? lane + pairs / 8 : lane - pairs / 8;
+                float o[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) o[j] = __shfl(a[j], from, 64);
+                if (turns) {
+                    const int a0 = first ? e0 : e0 - pairs;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const float co = cs[i][a0 + j], si = sn[i][a0 + j];
+                        a[j] = first ? a[j] * co - o[j] * si : a[j] * co + o[j] * si;
+                    }
+                }
+            } else if (turns) {
+#pragma unroll
+                for (int j = 0; j < 8; j += 2) {
+                    const float co = cs[i][(e0 + j) >> 1], si = sn[i][(e0 + j) >> 1], u = a[j], v = a[j + 1];
+                    a[j] = u * co - v * si;
+                    a[j + 1] = v * co + u * si;
+                }
+            }
+            if (h < nq) ConvTail::put8(qrow + static_cast<int64_t>(h) * k_dim + e0, a);
+            else if (store) ConvTail::put8(kpage + (static_cast<int64_t>(h - nq) * kRkBlock + off) * k_dim + e0, a);
+        }
+    }
+    const int kpad = k_dim - d, vpad = v_dim - dv;      // the columns beyond the heads are zero
+    if (kpad == 0 && vpad == 0) return;
+    for (int i = 0; i < n; ++i) {
+        const int64_t t = t0 + i, blk = meta[i][4];
+        const int off = meta[i][0] % kRkBlock;
+        for (int x = threadIdx.x; x < (store ? heads : nq) * kpad; x += blockDim.x) {
+            const int h = x / kpad, e = d + x - h * kpad;
+            if (h < nq) q_out[t * q_out_stride + static_cast<int64_t>(h) * k_dim + e] = to_t<T>(0.f);
+            else k_cache[blk * block_stride + (static_cast<int64_t>(h - nq) * kRkBlock + off) * k_dim + e] = to_t<T>(0.f);
+        }
+        for (int x = threadIdx.x; x < (store ? nk * vpad : 0); x += blockDim.x) {
+            const int g = x / vpad, c = dv + x - g * vpad;
+            v_cache[blk * block_stride + (static_cast<int64_t>(g) * v_dim + c) * kRkBlock + off] = to_t<T>(0.f);
+        }
+    }
+}
+
 template <typename T>
 __device__ __forceinline__ void latent_rope_store_token(int64_t t,
     T *proj, T *qa, int64_t in_place, const double *freq, const float *c_w, T *k_cache, T *v_cache, const int32_t *block_table,
@@ -686,7 +878,31 @@ extern "C" int swl_qkv_conv_rope_store_kv(
     if (k_cache && (!v_cache || !block_table || max_blocks_per_seq <= 0)) return SWL_ERR_BAD_ARG;
     const size_t lds = (static_cast<size_t>(C) + num_q_heads + num_kv_heads) * sizeof(float);
     if (num_tokens > 0x7fffffffLL || rot_dims > 2 * swl::kRkMaxPairs || lds > 60 * 1024) return SWL_ERR_UNSUPPORTED;
+#define SWL_ROWS_TOK(LPH, TOK)                                                                                                            \
+    hipLaunchKernelGGL((swl::qkv_conv_rope_rows_kernel<T, LPH, TOK>), dim3(static_cast<unsigned>((num_tokens + TOK - 1) / TOK)), dim3(threads), 0, \
+                       static_cast<hipStream_t>(stream), static_cast<const T *>(rows), tok_stride, static_cast<T *>(q_out), q_out_stride, \
+                       bias, conv_w, taps, q_w, k_w, freq, rot_dims, half, rot_mult, v_mult, static_cast<T *>(k_cache),                   \
+                       static_cast<T *>(v_cache), block_table, max_blocks_per_seq, block_stride, state, slot_stride, tail_off, tok_pos,   \
+                       tok_start, tok_state, tok_seq, num_tokens, num_q_heads, num_kv_heads, vdim, k_dim, v_dim, eps)
+#define SWL_ROWS(LPH)                                                                                                                     \
+    if (rows8 && dim == 8 * LPH) {                                                                                                        \
+        if (num_tokens >= swl::kRkManyTokens) SWL_ROWS_TOK(LPH, 4);                                                                              \
+        else SWL_ROWS_TOK(LPH, 1);                                                                                                        \
+        return swl::check_launch();                                                                                                       \
+    }
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        constexpr int PIECE = 16 / static_cast<int>(sizeof(T));
+        const bool rows8 = swl::aligned16(rows) && swl::aligned16(q_out) && tok_stride % PIECE == 0 && q_out_stride % PIECE == 0 && k_dim % 8 == 0 &&
+                           vdim % 8 == 0 && (!bias || swl::aligned16(bias)) && (!q_w || (swl::aligned16(q_w) && swl::aligned16(k_w))) &&
+                           (half ? rot_dims % 16 == 0 : rot_dims % 8 == 0) && (!k_cache || (swl::aligned16(k_cache) && block_stride % PIECE == 0)) &&
+                           (!conv_w || (taps <= 4 && swl::aligned16(conv_w) &&
+                                        (taps == 1 || (swl::aligned16(state) && slot_stride % 4 == 0 && tail_off % 4 == 0))));
+        // (a thread takes eight channels: no more waves than have some)
+        const int threads = static_cast<int>(C < 8 * swl::kRkThreads ? (C / 8 + 63) / 64 * 64 : swl::kRkThreads);
+        SWL_ROWS(2)
+        SWL_ROWS(4)
+        SWL_ROWS(8)
+        SWL_ROWS(16)
         hipLaunchKernelGGL((swl::qkv_conv_rope_store_kv_kernel<T>), dim3(static_cast<unsigned>(num_tokens)), dim3(swl::kRkThreads),
                            lds, static_cast<hipStream_t>(stream), static_cast<const T *>(rows), tok_stride, static_cast<T *>(q_out),
                            q_out_stride, bias, conv_w, taps, q_w, k_w, freq, rot_dims, half, rot_mult, v_mult,
@@ -694,6 +910,8 @@ extern "C" int swl_qkv_conv_rope_store_kv(
                            state, slot_stride, tail_off, tok_pos, tok_start, tok_state, tok_seq, num_tokens, num_q_heads,
                            num_kv_heads, dim, vdim, k_dim, v_dim, eps);
     });
+#undef SWL_ROWS
+#undef SWL_ROWS_TOK
     return swl::check_launch();
 }
 

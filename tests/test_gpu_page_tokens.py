@@ -90,3 +90,44 @@ def test_same_pool_and_carried_inputs(taps, tokens):
     assert bool(torch.isfinite(results[0][0].float()).all()) and results[0][1].any()
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("taps,dim,vdim,rot_dims,half", [(4, 128, 64, 64, True), (1, 64, 128, 64, False), (3, 16, 24, 16, True), (2, 32, 32, 8, False),
+                                                         (0, 128, 128, 0, True)])
+def test_four_tokens_a_workgroup(taps, dim, vdim, rot_dims, half, dtype):
+    """From 1536 tokens a workgroup takes four in a row, whose portions may begin and end between them: the rows, pages and carried inputs of
+    steps of fewer."""
+    from test_gpu_lorulix import Slots
+    from swiftllm_amd.worker.kernels.rope_kv import qkv_conv_rope_and_store_kv
+    from swiftllm_amd.worker.kernels.window_attn import PoolSlice
+    g = torch.Generator().manual_seed(dim + taps)
+    heads, kv, kd, vd = 3, 2, dim + 8, vdim + 8
+    C = (heads + kv) * dim + kv * vdim
+    rand = lambda *shape: torch.randn(*shape, generator=g)      # noqa: E731
+    bias, conv, norm = rand(C).cuda(), (rand(taps, C) / taps ** 0.5).cuda() if taps else None, (1 + 0.3 * rand(dim)).cuda()
+    freq = (777.0 ** (-torch.arange(0, rot_dims, 2, dtype=torch.float64) / rot_dims)).cuda() if rot_dims else None
+    rot = SimpleNamespace(dims=rot_dims, half=half, multiplier=1.0)
+    lens = [1, 2, 1, 5, 3, 1000, 1, 1, 520, 3]
+    assert 1536 <= sum(lens) and sum(lens) % 4
+    ahead = [(s, 0, 3) for s in range(0, len(lens), 2)]         # (half of the sequences have tokens already)
+    begin = [3 if s % 2 == 0 else 0 for s in range(len(lens))]
+    total = sum(c for _, _, c in ahead) + sum(lens) + len(lens)
+    rows = rand(total, C).to(dtype).cuda()
+    table = torch.randperm(70 * len(lens), generator=g).view(len(lens), 70).int().cuda()
+    results = []
+    for whole in (True, False):
+        slots, made, at = Slots([2 * max(taps - 1, 0) * C], num_slots=len(lens)), [], 0
+        pool = torch.zeros(table.numel(), kv * (kd + vd) * 16, dtype=dtype, device="cuda")
+        main = [(s, begin[s], c) for s, c in enumerate(lens)]
+        steps = [ahead] + ([main] if whole else [main[:6], main[6:]]) + [[(s, begin[s] + c, 1) for s, c in enumerate(lens)]]
+        for portions in steps:
+            n = sum(c for _, _, c in portions)
+            made.append(qkv_conv_rope_and_store_kv(rows[at:at + n], bias, conv, norm, norm, freq, rot, pool, PoolSlice(0, kv * kd * 16), table,
+                                                   slots.ref(portions), slots.off[0], heads, kv, dim, vdim, kd, vd, 1e-6))
+            at += n
+        assert at == total
+        results.append((torch.cat(made), pool))
+    assert bool(torch.isfinite(results[0][0].float()).all()) and results[0][1].any()
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
