@@ -193,4 +193,98 @@ struct ConvTail {
     }
 };
 
+// The wide form for a workgroup that takes TOK tokens in a row (steps of many tokens): the taps, fp32 and four to eight times a 16-bit row, are
+// read once for them, and a token's earlier inputs move on by one in registers. Up to four taps. meta: TOK x 4 ints of LDS, which a barrier has to
+// stand behind before `walk`. us, a token a workgroup / four, bf16: 1024 channels of 3 taps 1024 tokens 4.5 / 5.1, 2030 5.5 / 5.6, 3663 7.7 / 6.4, 8192
+// 15.6 / 10.6; the delta rule's 1536 of 4 taps with their norms 1024 9.3 / 11.0, 2030 14.8 / 14.5, 3663 22.1 / 20.2, 8192 41.8 / 35.7 (the state space's
+// 2304, which end in fp32: 3663 26.4 / 24.6, too little to be seen in a pass). Hence kConvRunTokens.
+constexpr int64_t kConvRunTokens = 2048;
+template <int TOK>
+struct ConvRun {
+    static constexpr int MOST = 3;
+    int64_t t0;
+    int n, R, C, pos0, start0, code0;
+    float *region;
+    int64_t slot_stride;
+    const int (*meta)[4];       // position, first position of the portion, state slot and parity, ends its portion
+
+    __device__ ConvRun(int (*shared)[4], float *state, int64_t slot_stride_, int64_t tail_off, const int32_t *tok_pos, const int32_t *tok_start,
+                       const int32_t *tok_state, const int32_t *tok_seq, int64_t num_tokens, int channels, int taps, int64_t first)
+        : t0(first), R(taps - 1), C(channels), code0(0), region(state + tail_off), slot_stride(slot_stride_), meta(shared) {
+        n = static_cast<int>(min<int64_t>(TOK, num_tokens - t0));
+        pos0 = tok_pos[t0];
+        start0 = tok_start[t0];
+        if (R > 0) code0 = tok_state[t0];
+        if (static_cast<int>(threadIdx.x) < n) {
+            const int64_t t = t0 + threadIdx.x;
+            int *m = shared[threadIdx.x];
+            m[0] = tok_pos[t];
+            m[1] = tok_start[t];
+            m[2] = R > 0 ? tok_state[t] : 0;
+            m[3] = t + 1 == num_tokens || tok_seq[t + 1] != tok_seq[t];
+        }
+    }
+
+    __device__ __forceinline__ float *tail(int code, int parity) const {
+        return region + static_cast<int64_t>(code >> 1) * slot_stride + static_cast<int64_t>(parity) * R * C;
+    }
+
+    // each(i, input[8], sum[8]) for tokens t0 + i, i < n, of channels c .. c + 7; the sums of ConvTail::conv8, in its order
+    template <typename T, typename F>
+    __device__ __forceinline__ void walk(const T *h, int64_t h_stride, const float *w, int c, F &&each) const {
+        float past[MOST][8], wk[MOST + 1][8];
+        typedef T Raw __attribute__((ext_vector_type(8)));
+        Raw raw[TOK];
+#pragma unroll
+        for (int i = 0; i < TOK; ++i) raw[i] = *reinterpret_cast<const Raw *>(h + (t0 + min(i, n - 1)) * h_stride + c);
+        auto earlier = [&](int64_t t, int code, int pos, int start) {
+#pragma unroll
+            for (int k = 1; k <= MOST; ++k)
+                if (k <= R && pos >= k) {       // (uniform)
+                    if (pos - k >= start) ConvTail::row8(h + (t - k) * h_stride + c, past[k - 1]);
+                    else ConvTail::row8(tail(code, code & 1) + static_cast<int64_t>(R - (start - (pos - k))) * C + c, past[k - 1]);
+                }
+        };
+        earlier(t0, code0, pos0, start0);
+#pragma unroll
+        for (int k = 0; k <= MOST; ++k)
+            if (k <= R) ConvTail::row8(w + static_cast<int64_t>(R - k) * C + c, wk[k]);
+#pragma unroll
+        for (int i = 0; i < TOK; ++i) {
+            if (i >= n) break;      // (uniform)
+            auto of = [&](int what) { return __builtin_amdgcn_readfirstlane(meta[i][what]); };
+            const int pos = of(0);
+            if (i > 0 && R > 0 && of(1) == pos) earlier(t0 + i, of(2), pos, pos);      // (a portion begins)
+            float cur[8], a[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                cur[j] = to_f(raw[i][j]);
+                a[j] = 0.f;
+            }
+#pragma unroll
+            for (int k = MOST; k >= 1; --k) {
+                if (k <= R && pos >= k) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) a[j] += wk[k][j] * past[k - 1][j];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) a[j] += wk[0][j] * cur[j];
+            if (R > 0 && of(3)) {
+                float *next = tail(of(2), 1 - (of(2) & 1));
+#pragma unroll
+                for (int k = 0; k < MOST; ++k)
+                    if (k < R && pos >= k) ConvTail::put8<float>(next + static_cast<int64_t>(R - 1 - k) * C + c, k == 0 ? cur : past[k > 0 ? k - 1 : 0]);
+            }
+            each(i, cur, a);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+#pragma unroll
+                for (int k = MOST - 1; k > 0; --k) past[k][j] = past[k - 1][j];
+                past[0][j] = cur[j];
+            }
+        }
+    }
+};
+
 } // namespace swl

@@ -84,6 +84,60 @@ __global__ __launch_bounds__(kDpThreads) void delta_prep_kernel(
     }
 }
 
+template <typename T, int TOK>
+__global__ __launch_bounds__(kDpThreads) void delta_prep_run_kernel(
+    float *qn, float *kn, float *kq, float *vv, float *beta, float *decay, const T *proj, int64_t proj_stride,
+    const float *conv_w, const float *a_log, const float *dt_bias, float *state, int64_t slot_stride, int64_t tail_off, const int32_t *tok_pos,
+    const int32_t *tok_start, const int32_t *tok_state, const int32_t *tok_seq, int64_t num_tokens, int H, int G, int d,
+    int dv, int taps) {
+    extern __shared__ __attribute__((aligned(16))) float act[];      // [TOK][2 G d] convolved, activated channels of q and k
+    __shared__ int meta[TOK][4];
+    const int qk = G * d, C = 2 * qk + H * dv;
+    const ConvRun<TOK> run(meta, state, slot_stride, tail_off, tok_pos, tok_start, tok_state, tok_seq, num_tokens, C, taps,
+                           static_cast<int64_t>(blockIdx.x) * TOK);
+    __syncthreads();
+    for (int c = threadIdx.x * 8; c < C; c += kDpThreads * 8)
+        run.walk(proj, proj_stride, conv_w, c, [&](int i, const float (&)[8], float (&a)[8]) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) a[j] *= dr_sigmoid(a[j]);
+            ConvTail::put8<float>(c < 2 * qk ? act + i * 2 * qk + c : vv + (run.t0 + i) * H * dv + c - 2 * qk, a);
+        });
+    __syncthreads();
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const float qscale = 1.0f / sqrtf(static_cast<float>(d));
+    for (int x = wave; x < G * run.n; x += kDpThreads / 64) {       // q head g and k head g: unit norms and their dot product
+        const int i = x / G, g = x - i * G;
+        const int64_t t = run.t0 + i;
+        const float *qsrc = act + i * 2 * qk + g * d, *ksrc = qsrc + qk;
+        float sq = 0.f, sk = 0.f, dot = 0.f;
+        for (int e = lane; e < d; e += 64) {
+            sq += qsrc[e] * qsrc[e];
+            sk += ksrc[e] * ksrc[e];
+            dot += qsrc[e] * ksrc[e];
+        }
+        sq = wave_allreduce_sum(sq);
+        sk = wave_allreduce_sum(sk);
+        dot = wave_allreduce_sum(dot);
+        const float rq = qscale / sqrtf(sq + 1e-6f), rk = 1.0f / sqrtf(sk + 1e-6f);
+        float *qdst = qn + t * qk + g * d, *kdst = kn + t * qk + g * d;
+        for (int e = lane; e < d; e += 64) {
+            qdst[e] = qsrc[e] * rq;
+            kdst[e] = ksrc[e] * rk;
+        }
+        if (lane == 0) kq[t * G + g] = dot * rq * rk;
+    }
+    for (int x = threadIdx.x; x < H * run.n; x += kDpThreads) {
+        const int i = x / H, h = x - i * H;
+        const int64_t t = run.t0 + i;
+        const T *row = proj + t * proj_stride;
+        const float b = to_f(row[C + H * dv + h]), a = to_f(row[C + H * dv + H + h]);
+        beta[t * H + h] = dr_sigmoid(b);
+        const float z = a + dt_bias[h];
+        const float sp = z > 20.f ? z : log1pf(expf(z));
+        decay[t * H + h] = expf(-expf(a_log[h]) * sp);
+    }
+}
+
 template <int L>
 __device__ __forceinline__ float dr_group_sum(float v) {
     return group_allreduce_sum<L>(v);
@@ -305,6 +359,15 @@ extern "C" int swl_delta_prep(float *qn, float *kn, float *kq, float *vv, float 
     const size_t lds = static_cast<size_t>(C) * sizeof(float);
     if (num_tokens > 0x7fffffffLL || lds > 64 * 1024) return SWL_ERR_UNSUPPORTED;
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        const int64_t qk2 = 2LL * num_qk_heads * dim;
+        if (num_tokens >= swl::kConvRunTokens && taps <= 4 && qk2 % 8 == 0 && 4 * qk2 * sizeof(float) <= 32 * 1024 && swl::aligned16(vv) &&
+            swl::ConvTail::wide_ok(static_cast<const T *>(proj), proj_stride, conv_w, state, slot_stride, tail_off, static_cast<int>(C))) {
+            hipLaunchKernelGGL((swl::delta_prep_run_kernel<T, 4>), dim3(static_cast<unsigned>((num_tokens + 3) / 4)), dim3(swl::kDpThreads),
+                               4 * qk2 * sizeof(float), static_cast<hipStream_t>(stream), qn, kn, kq, vv, beta, decay, static_cast<const T *>(proj),
+                               proj_stride, conv_w, a_log, dt_bias, state, slot_stride, tail_off, tok_pos, tok_start, tok_state, tok_seq,
+                               num_tokens, num_heads, num_qk_heads, dim, vdim, taps);
+            return swl::check_launch();
+        }
         hipLaunchKernelGGL((swl::delta_prep_kernel<T>), dim3(static_cast<unsigned>(num_tokens)), dim3(swl::kDpThreads), lds,
                            static_cast<hipStream_t>(stream), qn, kn, kq, vv, beta, decay, static_cast<const T *>(proj),
                            proj_stride, conv_w, a_log, dt_bias, state, slot_stride, tail_off, tok_pos, tok_start,

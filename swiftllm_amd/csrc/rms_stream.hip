@@ -405,6 +405,25 @@ __global__ __launch_bounds__(kRsThreads) void causal_conv_state_kernel(
     }
 }
 
+template <typename T, int TOK>
+__global__ __launch_bounds__(kRsThreads) void causal_conv_run_kernel(
+    T *out, int64_t out_stride, const T *h, int64_t h_stride, const float *w, float *state, int64_t slot_stride,
+    int64_t tail_off, const int32_t *tok_pos, const int32_t *tok_start, const int32_t *tok_state, const int32_t *tok_seq,
+    int64_t num_tokens, int C, int taps, int add_input) {
+    __shared__ int meta[TOK][4];
+    const ConvRun<TOK> run(meta, state, slot_stride, tail_off, tok_pos, tok_start, tok_state, tok_seq, num_tokens, C, taps,
+                           static_cast<int64_t>(blockIdx.x) * TOK);
+    __syncthreads();
+    for (int c = threadIdx.x * 8; c < C; c += blockDim.x * 8)
+        run.walk(h, h_stride, w, c, [&](int i, const float (&cur)[8], float (&a)[8]) {
+            if (add_input) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) a[j] += cur[j];
+            }
+            ConvTail::put8(out + (run.t0 + i) * out_stride + c, a);
+        });
+}
+
 template <typename T>
 __global__ __launch_bounds__(kRsThreads) void token_shift_mix_kernel(
     T *out, int64_t plane, const T *h, int64_t h_stride, const float *mu, int mixes, float *state, int64_t slot_stride,
@@ -534,6 +553,12 @@ extern "C" int swl_causal_conv_state(void *out, int64_t out_stride, const void *
         // (a thread takes eight channels: no more waves than have some)
         const bool wide = swl::ConvTail::wide_ok(static_cast<const T *>(h), h_stride, w, state, slot_stride, tail_off, channels);
         const int threads = wide && channels < 8 * swl::kRsThreads ? (channels / 8 + 63) / 64 * 64 : swl::kRsThreads;
+        if (wide && taps <= 4 && out_stride % (16 / sizeof(T)) == 0 && swl::aligned16(out) && num_tokens >= swl::kConvRunTokens) {
+            hipLaunchKernelGGL((swl::causal_conv_run_kernel<T, 4>), dim3(static_cast<unsigned>((num_tokens + 3) / 4)), dim3(static_cast<unsigned>(threads)),
+                               0, static_cast<hipStream_t>(stream), static_cast<T *>(out), out_stride, static_cast<const T *>(h), h_stride, w, state,
+                               slot_stride, tail_off, tok_pos, tok_start, tok_state, tok_seq, num_tokens, channels, taps, add_input);
+            return swl::check_launch();
+        }
         hipLaunchKernelGGL((swl::causal_conv_state_kernel<T>), dim3(static_cast<unsigned>(num_tokens)),
                            dim3(static_cast<unsigned>(threads)), 0, static_cast<hipStream_t>(stream), static_cast<T *>(out), out_stride,
                            static_cast<const T *>(h), h_stride, w, state, slot_stride, tail_off, tok_pos, tok_start,
