@@ -317,8 +317,8 @@ int launch_mix(const MixParams &p, int key_splits, hipStream_t s) {
             hipLaunchKernelGGL((sigmoid_attn_sum_kernel<T>), dim3(static_cast<unsigned>((rows * DV / 4 + 255) / 256)), dim3(256), 0, s,
                                static_cast<T *>(p.out), p.part_o, rows * DV, key_splits);
         else
-            hipLaunchKernelGGL((window_attn_combine_kernel<T>), dim3(static_cast<unsigned>(rows)), dim3(64), 0, s, static_cast<T *>(p.out),
-                               p.part_o, p.part_ml, rows, DV, key_splits, nullptr, p.H, 0, DV, static_cast<int64_t>(p.H) * DV, nullptr, 0);
+            launch_attn_combine<T>(static_cast<T *>(p.out), p.part_o, p.part_ml, rows, DV, key_splits, nullptr, p.H, 0, DV,
+                                   static_cast<int64_t>(p.H) * DV, nullptr, 0, s);
     }
     return check_launch();
 }

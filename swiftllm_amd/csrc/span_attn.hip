@@ -822,9 +822,8 @@ int launch_span(SpanParams &p, int key_splits, hipStream_t s) {
     if (!ok) return SWL_ERR_LAUNCH;
     if (key_splits > 1) {
         const int64_t rows = p.num_tokens * p.H;
-        hipLaunchKernelGGL((window_attn_combine_kernel<T>), dim3(static_cast<unsigned>(rows)), dim3(DV < 256 ? 64 : 256), 0, s,
-                           static_cast<T *>(p.out), p.part_o, p.part_ml, rows, DV, key_splits, p.sink, p.H, p.out_f32, p.out_dim,
-                           p.out_stride, static_cast<const T *>(p.gate), p.gate_stride);
+        launch_attn_combine<T>(static_cast<T *>(p.out), p.part_o, p.part_ml, rows, DV, key_splits, p.sink, p.H, p.out_f32, p.out_dim,
+                               p.out_stride, static_cast<const T *>(p.gate), p.gate_stride, s);
     }
     return check_launch();
 }

@@ -15,7 +15,8 @@
 // What bounds it is latency: a step of a few tokens is a few workgroups, each a chain of chunks. Key rows are read by neighbouring lanes
 // (one 512-byte row of 128 fp32 by half a wave) and serve four heads, a page's values are read once for the heads that share them
 // (token_attn.h), and key_splits > 1 shares a token's pages out over workgroups whose partial results a second launch combines.
-// 3 tokens at 513 keys, 8 heads of 128 over 2, fp32: 685 us with a key per thread and no shares, 22 + 6 us (16 shares and their sum).
+// 3 tokens at 513 keys, 8 heads of 128 over 2, fp32: 685 us with a key per thread and no shares, 18 us (16 shares and their sum; 8.4 in the
+// form below).
 //
 // The general entry point (swl_masked_attn) adds what other designs need of the same loop:
 //   * mask_kind 1: chunked visibility — keys [floor(p / window) * window, p], chunks counted from position 0;
@@ -211,9 +212,9 @@ inline size_t wa_lds_bytes(int H, int d) {
 // behind the other. Here the ids are scalar loads and a chunk's keys, bias and values are all asked for before the first score (the next
 // chunk's as soon as the registers are free); a lane has its queries in registers, and where a value row has 64 or 128 columns two or four
 // groups of threads share the pages. 90 to 145 registers: a sum left alone sinks below the next chunk's loads and takes 256.
-// us with the launch that adds up the shares, above -> here (heads of 128, 8 over 2, fp32; other sizes named): 3 tokens at 513 keys 18.0 ->
-// 10.7, one at 100 14.1 -> 10.5, 3 at 4000 50 -> 19.8, 12 at 500 18.2 -> 13.0, 32 at 1000 32 -> 20; prompts of 100 23 -> 16, 500 120 -> 39, 4 x 125
-// 48 -> 21, 500 with 8 key heads 365 -> 74, 500 of 64 / 128 columns 73 -> 31. Nothing measured was slower, so whatever it takes goes to it. Error
+// us with the launch that adds up the shares, both as they were -> both as they are (heads of 128, 8 over 2, fp32; other sizes named): 3 tokens at 513 keys
+// 18.0 -> 8.4, one at 100 14.1 -> 8.1, 3 at 4000 50 -> 17.5, 12 at 500 18.2 -> 11.3, 32 at 1000 32 -> 18; prompts of 100 23 -> 14, 500 120 -> 39, 4 x 125
+// 48 -> 21, 500 with 8 key heads 365 -> 73, 500 of 64 / 128 columns 73 -> 30. Nothing measured was slower, so whatever it takes goes to it. Error
 // against 64 bits 2.0 to 3.7e-7 (2-norm) where it is 2.1 to 3.8e-7 above.
 struct HeadsParams {
     void *out;
@@ -506,9 +507,8 @@ extern "C" int swl_masked_attn_shares(void *out, const void *q, const void *k_ca
         if (key_splits > 1 && out_f32 != SWL_OUT_SHARES) {
             const int64_t rows = num_tokens * num_q_heads;
             if (rows > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
-            hipLaunchKernelGGL((swl::window_attn_combine_kernel<T, true>), dim3(static_cast<unsigned>(rows)), dim3(vdim < 256 ? 64 : 256), 0,
-                               st, static_cast<T *>(out), part_o, part_ml, rows, vdim, key_splits, sink, num_q_heads, out_f32, out_dim,
-                               out_stride, static_cast<const T *>(gate), gate_stride);
+            swl::launch_attn_combine<T, true>(static_cast<T *>(out), part_o, part_ml, rows, vdim, key_splits, sink, num_q_heads, out_f32, out_dim,
+                                              out_stride, static_cast<const T *>(gate), gate_stride, st);
         }
     });
     return swl::check_launch();

@@ -354,8 +354,7 @@ int launch_wm(int hpw, dim3 grid, size_t lds, hipStream_t s, T *out, const T *q,
                            mask_kind, sink, GV, out_f32, hpg, slopes, od, ostr, gate, gstr);
         if (grid.y > 1 && out_f32 != SWL_OUT_SHARES) {
             const int64_t rows = nt * H;
-            hipLaunchKernelGGL((window_attn_combine_kernel<T>), dim3(static_cast<unsigned>(rows)), dim3(DV < 256 ? 64 : 256), 0,
-                               s, out, po, pml, rows, DV, static_cast<int>(grid.y), sink, H, out_f32, od, ostr, gate, gstr);
+            launch_attn_combine<T>(out, po, pml, rows, DV, static_cast<int>(grid.y), sink, H, out_f32, od, ostr, gate, gstr, s);
         }
         return check_launch();
     }
@@ -384,8 +383,7 @@ int launch_wm(int hpw, dim3 grid, size_t lds, hipStream_t s, T *out, const T *q,
 #undef SWL_WM_LAUNCH1
     if (grid.y > 1 && out_f32 != SWL_OUT_SHARES) {
         const int64_t rows = nt * H;
-        hipLaunchKernelGGL((window_attn_combine_kernel<T>), dim3(static_cast<unsigned>(rows)), dim3(DV < 256 ? 64 : 256), 0, s,
-                           out, po, pml, rows, DV, static_cast<int>(grid.y), sink, H, out_f32, od, ostr, gate, gstr);
+        launch_attn_combine<T>(out, po, pml, rows, DV, static_cast<int>(grid.y), sink, H, out_f32, od, ostr, gate, gstr, s);
     }
     return check_launch();
 }

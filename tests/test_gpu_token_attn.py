@@ -164,3 +164,33 @@ def test_heads_of_a_key_head_in_fp32(H, G, GV, d, dv, kind):
                          gate[at:at + m].double() if gate is not None else None)
             assert (o[at:at + m].double().cpu() - want).abs().max() <= _bound(want, torch.float32), (reach, b)
             at += m
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("dv,cut,extra,kind", [(64, 0, 0, "sink"), (64, 5, 3, "gate"), (128, 0, 4, "gate"), (128, 2, 0, "f32"), (256, 0, 8, "sink"), (256, 1, 1, "f32"),
+                                               (100, 0, 0, "sink")])
+def test_sums_of_key_shares(dv, cut, extra, kind, dtype):
+    """Any number of key shares, most of them empty for short sequences, against one: rows of 64, 128 and 256 columns, and others; columns that do
+    not count, results in a column slice."""
+    from swiftllm_amd import _hip
+    g = torch.Generator().manual_seed(dv + extra)
+    H, G, d = 4, 2, 64
+    pool, sl, table, _, _ = _pool([a + n for _, a, n in PARTS], G, G, d, dv, dtype, g)
+    seq, pos, _ = _spans(PARTS)
+    n, out_dim = seq.shape[0], dv - cut
+    q = torch.randn(n, H * d, generator=g).to(dtype).cuda()
+    sink = torch.randn(H, generator=g).cuda() if kind == "sink" else None
+    gate = torch.randn(n, H * out_dim + extra, generator=g).to(dtype).cuda() if kind == "gate" else None
+    results = []
+    for shares in (1, 2, 7, 8, 9, 17, 32, 33, 64):
+        out = torch.full((n, H * out_dim + extra), 7.0, dtype=torch.float32 if kind == "f32" else dtype, device="cuda")
+        scratch = torch.full((shares * n * H * (dv + 2),), float("nan"), device="cuda")
+        at = pool.data_ptr()
+        _hip.call("swl_masked_attn_shares", _hip.ptr(out), _hip.ptr(q), at + sl.k_offset * pool.element_size(), at + sl.v_offset * pool.element_size(),
+                  _hip.ptr(table), _hip.ptr(seq), _hip.ptr(pos), 0, 0, 0, n, H, G, d, dv, H * d, 0, d ** -0.5, 0.0, table.shape[1], pool.shape[1], 0,
+                  _hip.ptr(sink), G, 1 if kind == "f32" else 0, 0, out_dim, out.stride(0), _hip.ptr(gate), gate.stride(0) if gate is not None else 0,
+                  shares, _hip.ptr(scratch), _hip.dtype_code3(dtype), _hip.stream())
+        assert bool((out[:, H * out_dim:] == 7.0).all())
+        results.append(out[:, :H * out_dim].double().cpu())
+    for got in results[1:]:     # two roundings of the type apart, or sums of some hundred fp32 terms
+        assert (got - results[0]).abs().max() <= 2 * _bound(results[0], torch.float32 if kind == "f32" else dtype)
