@@ -160,11 +160,12 @@ class StepEntry:
 class LatentExpansion:
     """What decides whether the latent attention of a portion runs on the heads' own keys and values, expanded from the cached rows
     (csrc/latent_expand.hip), or on queries folded through the key up-projection: the matrix steps of both, by the sizes of the layers.
-    window: of the layers' the largest, 0 if one sees every key; max_pages: pages that the expansion may take."""
+    window: of the layers' the largest, 0 if one sees every key; max_pages: pages that the expansion may take; min_beside: tokens it takes
+    beside portions that stay folded."""
     MIN_TOKENS = 16
 
-    def __init__(self, dim: int, rot_dim: int, vdim: int, rank: int, window: int, max_pages: int):
-        self.window, self.max_pages = window, max_pages
+    def __init__(self, dim: int, rot_dim: int, vdim: int, rank: int, window: int, max_pages: int, min_beside: int = 0):
+        self.window, self.max_pages, self.min_beside = window, max_pages, min_beside
         # columns a visible (query, key) pair costs more when folded (values count twice), and what expanding one more key costs
         self.pair_gain = (3 * rank + rot_dim) - (dim + rot_dim + 2 * vdim)
         self.key_cost = (dim + vdim) * rank
@@ -252,6 +253,8 @@ class StepPlan:
         count = np.asarray(self.seq_cnt, dtype=np.int64)
         if count.size == 0 or count[0] < LatentExpansion.MIN_TOKENS:
             return None
+        if self.num_tokens < spec.min_beside and count.min() < LatentExpansion.MIN_TOKENS:      # (one stays folded, the others are too few)
+            return None
         start = self.tok_pos[self.seq_row0].astype(np.int64)
         first = np.maximum(start - spec.window + 1, 0) // 16 if spec.window > 0 else np.zeros_like(start)    # first page with a visible key
         pages = -(-(start + count) // 16)
@@ -264,6 +267,8 @@ class StepPlan:
         rest = k < ok.size
         row0, chunk0, tile0 = ((int(self.seq_row0[k]), int(self.seq_chunk0[k]), int(self.seq_tile0[k])) if rest else
                                (self.num_tokens, self.chunk_row0.size, self.tile_row0.size))
+        if rest and row0 < spec.min_beside:
+            return None
         first, pages, at, count = first[:k], pages[:k], at[:k], count[:k]
         each = pages - first
         page_no = np.arange(int(each.sum())) - np.repeat(np.cumsum(each) - each - first, each)

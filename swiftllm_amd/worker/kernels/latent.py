@@ -12,6 +12,11 @@ from .window_attn import MASK_WINDOW, SHARE_MAX_SCRATCH, AttentionSpec, PoolSlic
 # A layer's expanded pages take at most this much (which memory profiling sets aside: its step runs without a pool); portions past it stay
 # folded. 8192 tokens of 16 heads of 128 + 64 and 128 columns take 80 MiB.
 EXPAND_MAX_SCRATCH = 256 << 20
+# (token, head) pairs that portions take beside others that stay folded. Two ways through attention are three launches more a layer, which the
+# host, not the device, has to find time for in steps below about a millisecond. Two prompts beside 16 decoded tokens, us a pass, all folded
+# and split: 2048 wide, 16 heads 2 x 16 924, 1057; 2 x 250 1038, 1098; 2 x 400 1060, 1120; 2 x 682 1242, 1173; 2 x 1000 1579, 1453; 1024 wide, 8 heads
+# 2 x 250 1042, 1085; 2 x 1000 1093, 1131.
+EXPAND_MIN_BESIDE = 18 * 1024
 
 
 class ExpandedStep:
@@ -51,7 +56,7 @@ def latent_expansion(mixers, row_sizes, dtype: torch.dtype):
     windows = [getattr(mx, "window", 0) for mx in served]
     mx = served[0]
     return LatentExpansion(mx.head_dim, mx.rot_dim, mx.value_dim, mx.kv_rank, 0 if 0 in windows else max(windows),
-                           EXPAND_MAX_SCRATCH // page_bytes)
+                           EXPAND_MAX_SCRATCH // page_bytes, EXPAND_MIN_BESIDE // mx.num_q_heads)
 
 
 def expansion_served(mx, k_dim: int, dtype: torch.dtype) -> bool:
@@ -109,22 +114,23 @@ class LatentAttention:
         if m:
             self._expanded(proj, y[:m], ctx, ex)
         if m < n:
-            rows = slice(m, n)
+            # (views cost the host as much as a launch: none where every row is folded)
+            part = (lambda t: t[m:]) if m else (lambda t: t)
+            seq, pos, yr = part(ctx.tok_seq), part(ctx.tok_pos), part(y)
             if not folded:
                 # q_abs[t, h, :] = W_uk,h^T q_unrotated[t, h, :]  -> the first kv_rank columns of every head of qa
-                qn = proj[rows, :H * (d + dr)].view(n - m, H, d + dr)[:, :, :d].transpose(0, 1)       # [H, T, d]
+                qn = part(proj)[:, :H * (d + dr)].view(n - m, H, d + dr)[:, :, :d].transpose(0, 1)       # [H, T, d]
                 torch.bmm(qn, w.uk, out=qa.view(n - m, H, sp.head_dim)[:, :, :r].transpose(0, 1))   # (a strided batched product: no copy)
             if single:
-                self._single(qa, y[rows], gate[rows], ctx, rows)
+                self._single(qa, yr, part(gate), ctx, seq, pos)
                 if m:
                     head_gate_(y[:m], gate[:m], H, e)
                 return y
             if ctx.pool is None:    # memory profiling: the attention's output buffer without its reads
                 att = torch.zeros((n - m, H * sp.value_dim), dtype=proj.dtype, device=proj.device)
             else:
-                att = masked_attention(qa, ctx.pool, self.pool_slice, ctx.block_table, ctx.tok_seq[rows], ctx.tok_pos[rows], sp,
-                                       tiles, self.max_positions)
-            torch.bmm(att.view(n - m, H, sp.value_dim)[:, :, :r].transpose(0, 1), w.uv_t, out=y[rows].view(n - m, H, e).transpose(0, 1))
+                att = masked_attention(qa, ctx.pool, self.pool_slice, ctx.block_table, seq, pos, sp, tiles, self.max_positions)
+            torch.bmm(att.view(n - m, H, sp.value_dim)[:, :, :r].transpose(0, 1), w.uv_t, out=yr.view(n - m, H, e).transpose(0, 1))
         return head_gate_(y, gate, H, e)
 
     def _fold(self, proj, qa, ctx):
@@ -137,7 +143,7 @@ class LatentAttention:
                   ctx.pool.shape[1], float(self.eps), 1 if mx.rot.half else 0, float(mx.rot.multiplier), sp.head_dim, sp.value_dim,
                   _hip.dtype_code(proj.dtype), _hip.stream())
 
-    def _single(self, qa, y, gate, ctx, rows):
+    def _single(self, qa, y, gate, ctx, seq, pos):
         mx, w, sp = self.mixer, self.w, self.spec
         n, H, code = qa.shape[0], mx.num_q_heads, _hip.dtype_code(qa.dtype)
         # (of the counts and the model alone: a captured step stays valid)
@@ -145,7 +151,7 @@ class LatentAttention:
         shares = max(1, min(choose_key_splits(n * -(-H // 16), sp, self.max_positions), SHARE_MAX_SCRATCH // (4 * floats)))
         scratch = torch.empty(shares * floats, dtype=torch.float32, device=qa.device)
         _hip.call("swl_latent_decode", _hip.ptr(scratch), _hip.ptr(qa), ctx.pool.data_ptr() + self.pool_slice.k_offset * qa.element_size(),
-                  _hip.ptr(ctx.block_table), _hip.ptr(ctx.tok_seq[rows]), _hip.ptr(ctx.tok_pos[rows]), n, H, qa.stride(0), sp.window,
+                  _hip.ptr(ctx.block_table), _hip.ptr(seq), _hip.ptr(pos), n, H, qa.stride(0), sp.window,
                   float(sp.scale), ctx.block_table.shape[1], ctx.pool.shape[1], shares, code, _hip.stream())
         _hip.call("swl_latent_unfold", _hip.ptr(y), _hip.ptr(scratch), _hip.ptr(w.uv), _hip.ptr(sp.sink), _hip.ptr(gate), gate.stride(0), n, H,
                   mx.value_dim, shares, code, _hip.stream())

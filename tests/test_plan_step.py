@@ -158,3 +158,13 @@ def test_latent_expansion_covers_what_its_portions_see(window):
         order = plan.upload_order()
         if order is not None:
             assert sorted(A["ex_order"]) == list(range(ex.chunks))
+
+
+@pytest.mark.parametrize("tokens,beside,expanded", [(100, 0, True), (63, 3, False), (64, 3, True), (200, 1, True), (16, 30, False)])
+def test_latent_expansion_beside_folded_portions(tokens, beside, expanded):
+    """Beside portions that stay folded a step expands from min_beside tokens on, alone always."""
+    from swiftllm_amd.worker.batch_plan import LatentExpansion
+    entries = [StepEntry(0, [1] * (tokens // 2), 0, ()), StepEntry(1, [1] * (tokens - tokens // 2), 0, ())] if tokens >= 32 else [StepEntry(0, [1] * tokens, 0, ())]
+    plan = plan_step(entries + [StepEntry(9 + i, [1], 20, (0,)) for i in range(beside)])
+    ex = plan.latent_expansion(LatentExpansion(128, 64, 128, 512, 0, 4096, 64))
+    assert (ex is not None and ex.rows == tokens) == expanded and (expanded or ex is None)
