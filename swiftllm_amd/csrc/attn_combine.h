@@ -91,6 +91,8 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel(T *out, const fl
                                                                 const float *sink, int H, int out_f32, int out_dim, int64_t out_stride,
                                                                 const T *gate, int64_t gate_stride) {
     constexpr int dv = 4 * LP, SIDE = 64 / LP, DEEP = 8;
+    // (a lane reads another's weight with all of them at work: inside a branch by its own share, the lane asked may have gone the other way)
+    static_assert(64 % (DEEP * SIDE) == 0, "shares named below are lanes of the wave");
     const int lane = threadIdx.x & 63, sub = lane % LP, side = lane / LP;
     const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // (token, head)
     if (row >= rows) return;
@@ -111,10 +113,7 @@ __global__ __launch_bounds__(256) void attn_combine_rows_kernel(T *out, const fl
             inv = 1.0f / (wave_allreduce_sum(w * l) + extra);
         }
 #pragma unroll
-        for (int u = 0; u < DEEP; ++u) {
-            const int s = s0 + u * SIDE + side;
-            a += (s < nsplit ? __shfl(w, min(s, 63), 64) : 0.f) * p[u];
-        }
+        for (int u = 0; u < DEEP; ++u) a += __shfl(w, s0 + u * SIDE + side, 64) * p[u];     // (lanes without a share have weight zero)
     }
 #pragma unroll
     for (int d = LP; d < 64; d *= 2)

@@ -170,27 +170,44 @@ def test_heads_of_a_key_head_in_fp32(H, G, GV, d, dv, kind):
 @pytest.mark.parametrize("dv,cut,extra,kind", [(64, 0, 0, "sink"), (64, 5, 3, "gate"), (128, 0, 4, "gate"), (128, 2, 0, "f32"), (256, 0, 8, "sink"), (256, 1, 1, "f32"),
                                                (100, 0, 0, "sink")])
 def test_sums_of_key_shares(dv, cut, extra, kind, dtype):
-    """Any number of key shares, most of them empty for short sequences, against one: rows of 64, 128 and 256 columns, and others; columns that do
-    not count, results in a column slice."""
+    """Every number of key shares against float64: there is a token that sees as many pages (all its shares hold keys), and for most tokens some are
+    empty; rows of 64, 128 and 256 columns, and others; columns that do not count, results in a column slice; the per-token entry and, where it
+    serves, the tiles'."""
     from swiftllm_amd import _hip
+    from swiftllm_amd.worker.kernels import window_attn as wa
     g = torch.Generator().manual_seed(dv + extra)
     H, G, d = 4, 2, 64
-    pool, sl, table, _, _ = _pool([a + n for _, a, n in PARTS], G, G, d, dv, dtype, g)
-    seq, pos, _ = _spans(PARTS)
+    parts = PARTS + [(6, 16 * s - 5, 1) for s in range(1, 65)]
+    pool, sl, table, ks, vs = _pool([a + n for _, a, n in PARTS] + [1024], G, G, d, dv, dtype, g)
+    seq, pos, (row0, cnt) = _spans(parts)
     n, out_dim = seq.shape[0], dv - cut
-    q = torch.randn(n, H * d, generator=g).to(dtype).cuda()
+    q = torch.randn(n, H * d, generator=g).to(dtype)
     sink = torch.randn(H, generator=g).cuda() if kind == "sink" else None
-    gate = torch.randn(n, H * out_dim + extra, generator=g).to(dtype).cuda() if kind == "gate" else None
-    results = []
-    for shares in (1, 2, 7, 8, 9, 17, 32, 33, 64):
-        out = torch.full((n, H * out_dim + extra), 7.0, dtype=torch.float32 if kind == "f32" else dtype, device="cuda")
-        scratch = torch.full((shares * n * H * (dv + 2),), float("nan"), device="cuda")
-        at = pool.data_ptr()
-        _hip.call("swl_masked_attn_shares", _hip.ptr(out), _hip.ptr(q), at + sl.k_offset * pool.element_size(), at + sl.v_offset * pool.element_size(),
-                  _hip.ptr(table), _hip.ptr(seq), _hip.ptr(pos), 0, 0, 0, n, H, G, d, dv, H * d, 0, d ** -0.5, 0.0, table.shape[1], pool.shape[1], 0,
-                  _hip.ptr(sink), G, 1 if kind == "f32" else 0, 0, out_dim, out.stride(0), _hip.ptr(gate), gate.stride(0) if gate is not None else 0,
-                  shares, _hip.ptr(scratch), _hip.dtype_code3(dtype), _hip.stream())
-        assert bool((out[:, H * out_dim:] == 7.0).all())
-        results.append(out[:, :H * out_dim].double().cpu())
-    for got in results[1:]:     # two roundings of the type apart, or sums of some hundred fp32 terms
-        assert (got - results[0]).abs().max() <= 2 * _bound(results[0], torch.float32 if kind == "f32" else dtype)
+    gate = torch.randn(n, H * out_dim + extra, generator=g).to(dtype) if kind == "gate" else None
+    spec = wa.AttentionSpec(H, G, d, dv, d ** -0.5, sink=sink, out_dim=out_dim)
+    rows = torch.cumsum(torch.tensor([0] + [m for _, _, m in parts]), 0).tolist()
+    want = torch.cat([_want(q[r:r + m].double().view(m, H, d), ks[b - 1], vs[b - 1], a, spec, None, gate[r:r + m, :H * out_dim].double() if gate is not None else None)
+                      for (b, a, m), r in zip(parts, rows)])
+    # sums of some hundred fp32 terms, the tiles' weights in two 16-bit terms (2^-17 of values of up to four); a 16-bit result's own rounding.
+    # (a share of 64 holds a sixty-fourth of the weights: without it a result moves by some 2^-8)
+    bound = 1.1 * (2.0 ** -18 * max(1.0, float(want.abs().max())) if dtype == torch.float32 else 2.0 ** -15 + (0 if kind == "f32" else 2.0 ** -8) * want.abs())
+    q, gate, at, size = q.cuda(), gate.cuda() if gate is not None else None, pool.data_ptr(), pool.element_size()
+    wide = gate is None and out_dim % 4 == 0 and (H * out_dim + extra) % 4      # (the tiles' stores of four elements)
+    tiled = dtype != torch.float32 and not wide and bool(_hip.load().swl_masked_attn_tiles_supported(H, G, G, d, dv, _hip.dtype_code(dtype)))
+    for shares in range(1, 65):
+        for entry in ("tokens", "tiles")[:1 + tiled]:
+            out = torch.full((n, H * out_dim + extra), 7.0, dtype=torch.float32 if kind == "f32" else dtype, device="cuda")
+            scratch = torch.full((shares * n * H * (dv + 2),), float("nan"), device="cuda")
+            head = (_hip.ptr(out), _hip.ptr(q), at + sl.k_offset * size, at + sl.v_offset * size, _hip.ptr(table), _hip.ptr(seq), _hip.ptr(pos))
+            tail = (out_dim, out.stride(0), _hip.ptr(gate), gate.stride(0) if gate is not None else 0)
+            f32 = 1 if kind == "f32" else 0
+            if entry == "tokens":
+                _hip.call("swl_masked_attn_shares", *head, 0, 0, 0, n, H, G, d, dv, H * d, 0, d ** -0.5, 0.0, table.shape[1], pool.shape[1], 0,
+                          _hip.ptr(sink), G, f32, 0, *tail, shares, _hip.ptr(scratch), _hip.dtype_code3(dtype), _hip.stream())
+            else:
+                _hip.call("swl_masked_attn_tiles", *head, _hip.ptr(row0), _hip.ptr(cnt), 0, 0, 0, row0.shape[0], H, G, d, dv, H * d, 0, d ** -0.5, 0.0,
+                          table.shape[1], pool.shape[1], shares, _hip.ptr(scratch), n, 0, _hip.ptr(sink), G, f32, 4, 0, *tail, _hip.dtype_code(dtype),
+                          _hip.stream())
+            assert bool((out[:, H * out_dim:] == 7.0).all())
+            err = (out[:, :H * out_dim].double().cpu() - want).abs()
+            assert bool((err <= bound).all()), (shares, entry, float(err.max()))
