@@ -208,7 +208,9 @@ __global__ __launch_bounds__(kQkThreads) void qkv_bias_norm_store_kernel(
 // stores into the transposed page; everything a piece needs (row, bias, weights, the other layer's values) is asked for together, where a
 // weight at a time after the norm's sum costs 15 us of 33. Before -> here, heads of 128: biased 3663 tokens 16 over 4 33.3 -> 16.4 us, 8 over 2
 // 18.6 -> 9.9, 32 tokens 6.5 -> 4.0, 5000 of 32 over 32 169 -> 82; whole projections 8192 of 8 over 2 24.7 -> 15.5, 4500 of 16 over 4 25.8 -> 19.4, 32 6.1 ->
-// 4.3, 3 in fp32 4.4 -> 3.8; per head in fp32 500 tokens 6.0 -> 4.8.
+// 4.3, 3 in fp32 4.4 -> 3.8; per head in fp32 500 tokens 6.0 -> 4.8. Values that are no whole pieces (or blend in another layer's
+// that are not) go one at a time behind heads normed one by one; in the kernel above / here, 3663 tokens: 8 over 2 heads of 64 with 33 columns of values
+// 12.7 / 7.0, 16 over 4 of 128 blended with values three columns into a row 32.7 / 19.5, 16 over 4 of 64 with 36 (whole pieces over the heads) 20.4 / 8.9.
 template <typename T>
 struct QkvRows {
     T *qkv;
@@ -222,8 +224,10 @@ struct QkvRows {
 };
 constexpr int kQkRowsThreads = 512;
 
-template <typename T, int LPH>
+// V_PIECES: values in pieces of eight too (LPH 0: always)
+template <typename T, int LPH, bool V_PIECES>
 __global__ __launch_bounds__(kQkRowsThreads) void qkv_rows_kernel(QkvRows<T> a) {
+    static_assert(LPH > 0 || V_PIECES, "");
     __shared__ float red[2][kQkRowsThreads / 64];
     extern __shared__ __attribute__((aligned(16))) char lds[];
     T *values = reinterpret_cast<T *>(lds);     // [G dv]
@@ -234,7 +238,7 @@ __global__ __launch_bounds__(kQkRowsThreads) void qkv_rows_kernel(QkvRows<T> a) 
     int64_t blk = 0;
     if (a.store) blk = a.block_table[static_cast<int64_t>(a.tok_seq[t]) * a.max_blocks + pos / kQkBlock];
     T *kpage = a.k_cache + blk * a.block_stride, *vpage = a.v_cache + blk * a.block_stride;
-    const int end = a.store || a.v_back ? C : nq;
+    const int end = !a.store && !a.v_back ? nq : V_PIECES ? C : nqk;
     float x[8], y[8], w[8], b[8];       // the row's piece, the other layer's values, weights, biases
     T raw[8];
     auto ask = [&](int c) {
@@ -333,6 +337,16 @@ __global__ __launch_bounds__(kQkRowsThreads) void qkv_rows_kernel(QkvRows<T> a) 
             put(c);
         }
     }
+    if constexpr (!V_PIECES) {
+        for (int i = threadIdx.x; i < (a.store || a.v_back ? a.G * a.dv : 0); i += blockDim.x) {
+            float v = to_f(row[nqk + i]) + (a.v_b ? a.v_b[i] : 0.f);
+            if (a.v_other) v = (1.0f - a.mix) * v + a.mix * to_f(a.v_other[t * a.v_other_stride + i]);
+            const T vt = to_t<T>(v);
+            if (a.v_back && (a.v_b || a.v_other)) row[nqk + i] = vt;
+            if (a.store) vpage[static_cast<int64_t>(i) * kQkBlock + off] = vt;
+        }
+        return;
+    }
     if (!a.store) return;
     __syncthreads();
     // the transposed page keeps the 16 tokens of a column together: neighbouring lanes take neighbouring columns, 32 bytes apart (a lane that
@@ -346,20 +360,24 @@ static bool launch_rows(const QkvRows<T> &a, bool whole, int64_t num_tokens, hip
     constexpr int PIECE = 16 / static_cast<int>(sizeof(T));
     const int64_t C = static_cast<int64_t>(a.H + a.G) * a.d + static_cast<int64_t>(a.G) * a.dv;
     auto ok = [](const void *p) { return aligned16(p); };       // (NULL is)
-    if (a.d % 8 || a.dv % 8 || a.tok_stride % PIECE || !ok(a.qkv) || !ok(a.q_b) || !ok(a.k_b) || !ok(a.v_b) || !ok(a.q_w) || !ok(a.k_w) ||
-        (a.v_other && (!ok(a.v_other) || a.v_other_stride % PIECE)) || (a.store && (!ok(a.k_cache) || a.block_stride % PIECE)))
+    if (a.d % 8 || a.tok_stride % PIECE || !ok(a.qkv) || !ok(a.q_b) || !ok(a.k_b) || !ok(a.q_w) || !ok(a.k_w) ||
+        (a.store && (!ok(a.k_cache) || a.block_stride % PIECE)))
         return false;
-    const size_t lds = sizeof(T) * a.G * a.dv;
-    if ((whole && C > 8 * kQkRowsThreads) || lds > 32 * 1024) return false;
+    const size_t values = sizeof(T) * a.G * a.dv;
+    const bool v_pieces = a.G * a.dv % 8 == 0 && ok(a.v_b) && (!a.v_other || (ok(a.v_other) && a.v_other_stride % PIECE == 0)) && values <= 32 * 1024;
+    if (whole && (!v_pieces || C > 8 * kQkRowsThreads)) return false;
+    const size_t lds = v_pieces ? values : 0;
     // (no more waves than have a piece)
-    const dim3 grid(static_cast<unsigned>(num_tokens)), block(static_cast<unsigned>(C < 8 * kQkRowsThreads ? (C / 8 + 63) / 64 * 64 : kQkRowsThreads));
-#define SWL_ROWS(LPH) hipLaunchKernelGGL((qkv_rows_kernel<T, LPH>), grid, block, lds, s, a)
-    if (whole) SWL_ROWS(0);
-    else if (a.d == 16) SWL_ROWS(2);
-    else if (a.d == 32) SWL_ROWS(4);
-    else if (a.d == 64) SWL_ROWS(8);
-    else if (a.d == 128) SWL_ROWS(16);
+    const dim3 grid(static_cast<unsigned>(num_tokens)), block(static_cast<unsigned>(C < 8 * kQkRowsThreads ? (C + 511) / 512 * 64 : kQkRowsThreads));
+#define SWL_ROWS(LPH, PIECES) hipLaunchKernelGGL((qkv_rows_kernel<T, LPH, PIECES>), grid, block, lds, s, a)
+#define SWL_ROWS_OF(LPH) do { if (v_pieces) SWL_ROWS(LPH, true); else SWL_ROWS(LPH, false); } while (0)
+    if (whole) SWL_ROWS(0, true);
+    else if (a.d == 16) SWL_ROWS_OF(2);
+    else if (a.d == 32) SWL_ROWS_OF(4);
+    else if (a.d == 64) SWL_ROWS_OF(8);
+    else if (a.d == 128) SWL_ROWS_OF(16);
     else return false;
+#undef SWL_ROWS_OF
 #undef SWL_ROWS
     return true;
 }

@@ -134,17 +134,20 @@ def test_four_tokens_a_workgroup(taps, dim, vdim, rot_dims, half, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("heads,kv,dim,vdim,n", [(3, 1, 128, 64, 33), (5, 2, 64, 8, 5), (1, 1, 16, 128, 17), (33, 3, 128, 128, 3), (4, 4, 32, 40, 150)])
-@pytest.mark.parametrize("kind", ["bias_norm", "bias", "mix", "full", "norm"])
+@pytest.mark.parametrize("heads,kv,dim,vdim,n", [(3, 1, 128, 64, 33), (5, 2, 64, 8, 5), (1, 1, 16, 128, 17), (33, 3, 128, 128, 3), (4, 4, 32, 40, 150),
+                                                  (4, 2, 64, 36, 33), (3, 1, 128, 20, 5), (3, 3, 64, 33, 150)])
+@pytest.mark.parametrize("kind", ["bias_norm", "bias", "mix", "mix_slice", "full", "norm"])
 def test_rows_of_aligned_eights(kind, heads, kv, dim, vdim, n, dtype):
     """Rows in registers against the kernel for any rows, which takes them where their stride is not a multiple of 16 bytes: one rounding of the
-    type apart, sums of up to 4224 squares in another order; with and without a pool."""
+    type apart, sums of up to 4224 squares in another order; values in whole pieces of eight over all heads or not, or beside another layer's that
+    start anywhere; with and without a pool."""
     from swiftllm_amd.worker.kernels import window_attn as wa
     g = torch.Generator().manual_seed(heads * dim + vdim)
     rand = lambda *shape: torch.randn(*shape, generator=g)      # noqa: E731
     nq, nk, nv = heads * dim, kv * dim, kv * vdim
     C = nq + nk + nv
-    rows, other = rand(n, C).to(dtype), rand(n, nv).to(dtype).cuda()
+    rows, other = rand(n, C).to(dtype), rand(n, nv + 3).to(dtype).cuda()
+    other = other[:, 3:] if kind == "mix_slice" else other[:, :nv].contiguous()
     w = {size: (1 + 0.3 * rand(size)).cuda() for size in {nq, nk, nv, dim}}
     mixer = SimpleNamespace(num_q_heads=heads, num_kv_heads=kv, head_dim=dim, value_dim=vdim, q_size=nq, k_size=nk, v_size=nv, q_temp_coef=0.1,
                             q_temp_every=3)
@@ -152,7 +155,7 @@ def test_rows_of_aligned_eights(kind, heads, kv, dim, vdim, n, dtype):
     table = torch.randperm(12, generator=g).view(1, 12).int().cuda()
     for with_pool in (True, False):
         results = []
-        for extra in (8, 1):
+        for extra in (8 + -C % 8, 1 + C % 2):
             wide = torch.zeros(n, C + extra, dtype=dtype)
             wide[:, :C] = rows
             wide = wide.cuda()
@@ -166,7 +169,7 @@ def test_rows_of_aligned_eights(kind, heads, kv, dim, vdim, n, dtype):
             elif kind == "bias":
                 wa.qkv_bias_norm_store(x, None, w[nk], w[nv], None, None, *to)
             else:
-                wa.qkv_bias_norm_store(x, w[nq], w[nk], w[nv], w[dim], None, *to, *((other, 0.3) if kind == "mix" else ()))
+                wa.qkv_bias_norm_store(x, w[nq], w[nk], w[nv], w[dim], None, *to, *((other, 0.3) if kind in ("mix", "mix_slice") else ()))
             assert bool((wide[:, C:] == 0).all())
             results.append((x.double(), pool.double() if with_pool else x.double()))
         eps = {torch.float32: 2.0 ** -20, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
