@@ -195,10 +195,12 @@ struct ConvTail {
 
 // The wide form for a workgroup that takes TOK tokens in a row (steps of many tokens): the taps, fp32 and four to eight times a 16-bit row, are
 // read once for them, and a token's earlier inputs move on by one in registers. Up to four taps. meta: TOK x 4 ints of LDS, which a barrier has to
-// stand behind before `walk`. us, a token a workgroup / four, bf16: 1024 channels of 3 taps 1024 tokens 4.5 / 5.1, 2030 5.5 / 5.6, 3663 7.7 / 6.4, 8192
-// 15.6 / 10.6; the delta rule's 1536 of 4 taps with their norms 1024 9.3 / 11.0, 2030 14.8 / 14.5, 3663 22.1 / 20.2, 8192 41.8 / 35.7 (the state space's
-// 2304, which end in fp32: 3663 26.4 / 24.6, too little to be seen in a pass). Hence kConvRunTokens.
-constexpr int64_t kConvRunTokens = 2048;
+// stand behind before `walk`.
+// When it pays: few tokens leave CUs idle, and a narrow row's workgroup is one wave, whose chain of four tokens takes its time. us of the causal convolution, a
+// token a workgroup / four, bf16, 4 taps (2 taps and fp32 alike): 64 channels 4096 tokens 5.7 / 6.7, 6144 6.4 / 5.7; 256 2048 4.7 / 5.3, 4096 5.7 / 5.6, 8192
+// 7.8 / 6.3; 512 2048 4.9 / 5.4, 3072 5.5 / 5.6, 4096 6.1 / 5.9, 8192 10.6 / 6.9; 1024 1024 4.7 / 5.4, 2048 6.2 / 6.1, 4096 10.5 / 7.0, 8192 18.1 / 11.4; 4096
+// 2048 17.6 / 14.0, 8192 51.1 / 35.7. (The state space's 2304 channels, which end in fp32: 3663 tokens 26.4 / 24.6, too little to be seen in a pass.)
+inline bool conv_run_pays(int64_t tokens, int64_t channels) { return tokens >= 6144 || (tokens >= 2048 && tokens * channels >= 1 << 21); }
 template <int TOK>
 struct ConvRun {
     static constexpr int MOST = 3;

@@ -360,7 +360,7 @@ extern "C" int swl_delta_prep(float *qn, float *kn, float *kq, float *vv, float 
     if (num_tokens > 0x7fffffffLL || lds > 64 * 1024) return SWL_ERR_UNSUPPORTED;
     SWL_DISPATCH_DTYPE3(dtype, T, {
         const int64_t qk2 = 2LL * num_qk_heads * dim;
-        if (num_tokens >= swl::kConvRunTokens && taps <= 4 && qk2 % 8 == 0 && 4 * qk2 * sizeof(float) <= 32 * 1024 && swl::aligned16(vv) &&
+        if (num_tokens >= 2048 && taps <= 4 && qk2 % 8 == 0 && 4 * qk2 * sizeof(float) <= 32 * 1024 && swl::aligned16(vv) &&
             swl::ConvTail::wide_ok(static_cast<const T *>(proj), proj_stride, conv_w, state, slot_stride, tail_off, static_cast<int>(C))) {
             hipLaunchKernelGGL((swl::delta_prep_run_kernel<T, 4>), dim3(static_cast<unsigned>((num_tokens + 3) / 4)), dim3(swl::kDpThreads),
                                4 * qk2 * sizeof(float), static_cast<hipStream_t>(stream), qn, kn, kq, vv, beta, decay, static_cast<const T *>(proj),

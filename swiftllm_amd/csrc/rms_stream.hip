@@ -553,7 +553,7 @@ extern "C" int swl_causal_conv_state(void *out, int64_t out_stride, const void *
         // (a thread takes eight channels: no more waves than have some)
         const bool wide = swl::ConvTail::wide_ok(static_cast<const T *>(h), h_stride, w, state, slot_stride, tail_off, channels);
         const int threads = wide && channels < 8 * swl::kRsThreads ? (channels / 8 + 63) / 64 * 64 : swl::kRsThreads;
-        if (wide && taps <= 4 && out_stride % (16 / sizeof(T)) == 0 && swl::aligned16(out) && num_tokens >= swl::kConvRunTokens) {
+        if (wide && taps <= 4 && out_stride % (16 / sizeof(T)) == 0 && swl::aligned16(out) && swl::conv_run_pays(num_tokens, channels)) {
             hipLaunchKernelGGL((swl::causal_conv_run_kernel<T, 4>), dim3(static_cast<unsigned>((num_tokens + 3) / 4)), dim3(static_cast<unsigned>(threads)),
                                0, static_cast<hipStream_t>(stream), static_cast<T *>(out), out_stride, static_cast<const T *>(h), h_stride, w, state,
                                slot_stride, tail_off, tok_pos, tok_start, tok_state, tok_seq, num_tokens, channels, taps, add_input);

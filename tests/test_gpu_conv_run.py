@@ -1,18 +1,19 @@
-"""Kernels whose workgroups take four tokens in a row from 2048 tokens on (csrc/conv_tail.h, ConvRun) against steps of fewer, a token a workgroup:
+"""Kernels whose workgroups take four tokens in a row in steps of many (csrc/conv_tail.h, ConvRun) against steps of fewer, a token a workgroup:
 the same bits of every result and of the carried inputs, with portions that begin and end between the four."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
-LENS = [1, 2, 1, 5, 3, 1500, 1, 1, 532, 3]      # (2049 tokens: the last workgroup has one)
+LENS = [1, 2, 1, 5, 3, 1500, 1, 1, 1532, 3, 1500, 2, 1598, 1, 3]    # (6153 tokens: rows of any width are many; the last workgroup has one)
+CUTS = [6, 10, 12]      # (1512, 1537, 1502 and 1602 tokens: few of any width)
 
 
 def _steps():
-    """(portions of every step) for a step of all LENS and for the same cut in two: a few tokens ahead of half the sequences, and one behind all."""
+    """(portions of every step) for a step of all LENS and for the same cut in four: a few tokens ahead of half the sequences, and one behind all."""
     ahead = [(s, 0, 3) for s in range(0, len(LENS), 2)]
     main = [(s, 3 if s % 2 == 0 else 0, c) for s, c in enumerate(LENS)]
     behind = [(s, a + c, 1) for s, a, c in main]
-    return [ahead, main, behind], [ahead, main[:6], main[6:], behind]
+    return [ahead, main, behind], [ahead] + [main[a:b] for a, b in zip([0] + CUTS, CUTS + [len(LENS)])] + [behind]
 
 
 def _same(run, channels, taps):
