@@ -84,6 +84,11 @@ __global__ __launch_bounds__(kDpThreads) void delta_prep_kernel(
     }
 }
 
+// The same for TOK tokens in a row (conv_tail.h, ConvRun). The norms of q and k heads are one behind the other in a workgroup's four waves: with many
+// of them, or few taps to read once instead of TOK times, it takes more tokens to gain, or never does. us, a token a workgroup / four, bf16, heads
+// x columns of q, k and taps: 4 x 64, 4 taps 2048 tokens 12.9 / 14.2, 3072 18.0 / 15.6, 8192 37.7 / 33.0, 2 taps 3072 14.8 / 14.6, 8192 32.4 / 29.8; 2 x 64 of
+// 128 value columns, 4 taps 3072 18.4 / 17.1; 8 x 64, 4 taps 3072 21.3 / 22.3, 4096 25.9 / 25.1, 8192 44.2 / 42.5, 2 taps 4096 22.8 / 23.7, 16384 70.3 / 71.6; 4 x
+// 128, 4 taps 4096 24.2 / 22.1, 8192 40.9 / 37.4.
 template <typename T, int TOK>
 __global__ __launch_bounds__(kDpThreads) void delta_prep_run_kernel(
     float *qn, float *kn, float *kq, float *vv, float *beta, float *decay, const T *proj, int64_t proj_stride,
@@ -360,7 +365,8 @@ extern "C" int swl_delta_prep(float *qn, float *kn, float *kq, float *vv, float 
     if (num_tokens > 0x7fffffffLL || lds > 64 * 1024) return SWL_ERR_UNSUPPORTED;
     SWL_DISPATCH_DTYPE3(dtype, T, {
         const int64_t qk2 = 2LL * num_qk_heads * dim;
-        if (num_tokens >= 2048 && taps <= 4 && qk2 % 8 == 0 && 4 * qk2 * sizeof(float) <= 32 * 1024 && swl::aligned16(vv) &&
+        const bool many = qk2 <= 512 ? num_tokens >= 3072 : num_tokens >= 4096 && taps >= 3;
+        if (many && taps <= 4 && qk2 % 8 == 0 && 4 * qk2 * sizeof(float) <= 32 * 1024 && swl::aligned16(vv) &&
             swl::ConvTail::wide_ok(static_cast<const T *>(proj), proj_stride, conv_w, state, slot_stride, tail_off, static_cast<int>(C))) {
             hipLaunchKernelGGL((swl::delta_prep_run_kernel<T, 4>), dim3(static_cast<unsigned>((num_tokens + 3) / 4)), dim3(swl::kDpThreads),
                                4 * qk2 * sizeof(float), static_cast<hipStream_t>(stream), qn, kn, kq, vv, beta, decay, static_cast<const T *>(proj),

@@ -44,7 +44,7 @@ def test_causal_conv(taps, channels, add, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("H,G,d,dv,taps", [(8, 2, 128, 128, 4), (3, 1, 24, 8, 2), (4, 4, 64, 40, 3), (2, 2, 20, 16, 1)])
+@pytest.mark.parametrize("H,G,d,dv,taps", [(8, 2, 128, 128, 4), (3, 1, 24, 8, 2), (4, 4, 64, 40, 3), (2, 2, 20, 16, 1), (8, 8, 64, 24, 3)])
 def test_delta_prep(H, G, d, dv, taps, dtype):
     from swiftllm_amd import _hip
     g = torch.Generator().manual_seed(d + taps)
