@@ -392,13 +392,15 @@ __global__ __launch_bounds__(kRkThreads) void qkv_conv_rope_store_kv_kernel(
 // The same for heads of 8 LPH columns (16, 32, 64 or 128), up to four taps and rows of whole aligned pieces of eight: a lane's eight channels
 // stay in registers, a head's sum and its rotation are exchanges between neighbouring lanes. What bounds it is the chain of a token's
 // workgroup, which above is a round trip for every earlier input and the norm's and the rotation's passes over LDS: here the row, up to
-// three earlier ones, taps, bias and norm weights are asked for together. From kRkManyTokens tokens a workgroup takes four in a row, for which
-// the taps (8 to 16 KiB a row of 2 KiB) are read once and whose earlier inputs move on by one in registers; below, its longer chain costs more (10 us
-// at any count).
-// us, above -> one token / four, heads of 128, bf16: 8 over 2 with 4 taps and norm 128 tokens 9.6 -> 6.0 / 10.3, 1000 12.8 -> 7.9 / 10.8, 1500 15.9 -> 12.3 /
-// 11.7, 2030 20.9 -> 16.1 / 15.2, 3000 27.0 -> 20.7 / 14.8; without norm 2030 14.6 -> 15.6 / 14.7, 5000 26.3 -> 30.2 / 23.4; 16 over 4 with norm, no taps 500
-// 14.1 -> 7.2 / 10.7, 1500 24.2 -> 13.2 / 14.5, 2030 31.6 -> 18.1 / 15.7; fp32, 3 tokens 13.2 -> 5.9, 500 14.1 -> 7.4.
-constexpr int kRkManyTokens = 1536;
+// three earlier ones, taps, bias and norm weights are asked for together. In steps of many tokens a workgroup takes four in a row, for which
+// the taps (8 to 16 KiB a row of 2 KiB) are read once and whose earlier inputs move on by one in registers; its longer chain costs more where the
+// workgroups of one token, few or of one wave each, are all on the chip at once (rk_four_pay).
+// us, above -> one token / four, heads of 128, bf16: 8 over 2 with 4 taps and norm 32 tokens 10.5 -> 5.8, 500 11.7 -> 6.9, 1536 19.6 -> 12.5 / 11.7, 2030 25.6 -> 16.3 /
+// 12.5, 5000 53.7 -> - / 24.8; without norm 3 7.6 -> 5.5, 500 9.1 -> 6.7, 1000 11.4 -> 7.8, 1500 14.3 -> 11.8, 2030 19.4 -> 15.7 / 11.7, 5000 36.8 -> - / 23.8; without
+// norm and taps 500 7.5 -> 5.4, 2030 15.8 -> 11.7 / 9.4; 16 over 4 without norm 1000 18.1 -> 15.0, 2030 33.7 -> - / 18.9; fp32 without norm 3 11.4 -> 5.7, 1000
+// 14.6 -> 9.1, 2030 25.0 -> 17.2 / 14.5. One / four by channels of q, k and v, 4 taps without norm: 96 3072 8.3 / 10.5, 4096 10.9 / 10.6, 8192 16.9 / 11.7; 384 1536 6.8 /
+// 9.6, 3072 8.2 / 10.0, 4096 11.3 / 10.3; 768 1536 8.0 / 10.0, 2048 11.2 / 10.3, 3072 13.6 / 10.7; 1024 1536 8.2 / 10.9, 2048 12.0 / 11.2; 1536 1024 7.6 / 10.4, 1536 12.1 / 11.1.
+inline bool rk_four_pay(int64_t tokens, int64_t channels) { return tokens >= 4096 || (tokens >= 1536 && tokens * channels >= 1 << 21); }
 template <typename T, int LPH, int TOK>
 __global__ __launch_bounds__(kRkThreads, 3) void qkv_conv_rope_rows_kernel(
     const T *rows, int64_t tok_stride, T *q_out, int64_t q_out_stride, const float *bias, const float *conv_w, int taps,
@@ -886,7 +888,7 @@ extern "C" int swl_qkv_conv_rope_store_kv(
                        tok_start, tok_state, tok_seq, num_tokens, num_q_heads, num_kv_heads, vdim, k_dim, v_dim, eps)
 #define SWL_ROWS(LPH)                                                                                                                     \
     if (rows8 && dim == 8 * LPH) {                                                                                                        \
-        if (num_tokens >= swl::kRkManyTokens) SWL_ROWS_TOK(LPH, 4);                                                                              \
+        if (swl::rk_four_pay(num_tokens, C)) SWL_ROWS_TOK(LPH, 4);                                                                         \
         else SWL_ROWS_TOK(LPH, 1);                                                                                                        \
         return swl::check_launch();                                                                                                       \
     }

@@ -96,8 +96,8 @@ def test_same_pool_and_carried_inputs(taps, tokens):
 @pytest.mark.parametrize("taps,dim,vdim,rot_dims,half", [(4, 128, 64, 64, True), (1, 64, 128, 64, False), (3, 16, 24, 16, True), (2, 32, 32, 8, False),
                                                          (0, 128, 128, 0, True)])
 def test_four_tokens_a_workgroup(taps, dim, vdim, rot_dims, half, dtype):
-    """From 1536 tokens a workgroup takes four in a row, whose portions may begin and end between them: the rows, pages and carried inputs of
-    steps of fewer."""
+    """From 4096 tokens of any width a workgroup takes four in a row, whose portions may begin and end between them: the rows, pages and carried
+    inputs of steps of fewer (below 1536: one)."""
     from test_gpu_lorulix import Slots
     from swiftllm_amd.worker.kernels.rope_kv import qkv_conv_rope_and_store_kv
     from swiftllm_amd.worker.kernels.window_attn import PoolSlice
@@ -108,19 +108,19 @@ def test_four_tokens_a_workgroup(taps, dim, vdim, rot_dims, half, dtype):
     bias, conv, norm = rand(C).cuda(), (rand(taps, C) / taps ** 0.5).cuda() if taps else None, (1 + 0.3 * rand(dim)).cuda()
     freq = (777.0 ** (-torch.arange(0, rot_dims, 2, dtype=torch.float64) / rot_dims)).cuda() if rot_dims else None
     rot = SimpleNamespace(dims=rot_dims, half=half, multiplier=1.0)
-    lens = [1, 2, 1, 5, 3, 1000, 1, 1, 520, 3]
-    assert 1536 <= sum(lens) and sum(lens) % 4
+    lens, cuts = [1, 2, 1, 5, 3, 1000, 1, 1, 520, 3, 1400, 2, 1161, 1], [0, 6, 10, 12, 14]
+    assert sum(lens) >= 4096 and sum(lens) % 4 and max(sum(lens[a:b]) for a, b in zip(cuts, cuts[1:])) < 1536
     ahead = [(s, 0, 3) for s in range(0, len(lens), 2)]         # (half of the sequences have tokens already)
     begin = [3 if s % 2 == 0 else 0 for s in range(len(lens))]
     total = sum(c for _, _, c in ahead) + sum(lens) + len(lens)
     rows = rand(total, C).to(dtype).cuda()
-    table = torch.randperm(70 * len(lens), generator=g).view(len(lens), 70).int().cuda()
+    table = torch.randperm(90 * len(lens), generator=g).view(len(lens), 90).int().cuda()
     results = []
     for whole in (True, False):
         slots, made, at = Slots([2 * max(taps - 1, 0) * C], num_slots=len(lens)), [], 0
         pool = torch.zeros(table.numel(), kv * (kd + vd) * 16, dtype=dtype, device="cuda")
         main = [(s, begin[s], c) for s, c in enumerate(lens)]
-        steps = [ahead] + ([main] if whole else [main[:6], main[6:]]) + [[(s, begin[s] + c, 1) for s, c in enumerate(lens)]]
+        steps = [ahead] + ([main] if whole else [main[a:b] for a, b in zip(cuts, cuts[1:])]) + [[(s, begin[s] + c, 1) for s, c in enumerate(lens)]]
         for portions in steps:
             n = sum(c for _, _, c in portions)
             made.append(qkv_conv_rope_and_store_kv(rows[at:at + n], bias, conv, norm, norm, freq, rot, pool, PoolSlice(0, kv * kd * 16), table,
