@@ -180,6 +180,13 @@ class LatentExpansion:
             before, seen = np.minimum(start, self.window - 1), np.minimum(seen, count * self.window)
         return (count >= self.MIN_TOKENS) & (2 * seen * self.pair_gain > before * self.key_cost)
 
+    def most_ints(self, tokens: int, portions: int, pages: int) -> int:
+        """Ints that a step's orders and the arrays of its expansion (ExpandedPortions, each on 16 bytes) take at most: so many tokens, portions,
+        and pages of a portion."""
+        pages = min(pages * portions, self.max_pages)
+        chunks, tiles = tokens // StepPlan.CHUNK + portions, tokens // StepPlan.TILE + portions
+        return 4 * pages + tokens + 3 * chunks + tiles + 9 * 4
+
 
 class ExpandedPortions:
     """The first `seqs` portions of a step (`rows` tokens, `chunks` chunks, `tiles` tiles) on `pages` expanded pages. arrays: int32, for the

@@ -163,7 +163,7 @@ class SteppedModel:
     def _upload_plan(self, plan: StepPlan, use_pool: bool = True):
         """The plan's int32 arrays through one pinned buffer and ONE async copy; returns device views."""
         layout, total = plan.packed_layout()
-        order = plan.upload_order()
+        order, room = plan.upload_order(), total
         extra = [] if order is None else [("span_order", order)]
         expanded = plan.latent_expansion(self.latent_expansion) if self.latent_expansion is not None and use_pool else None
         if expanded is not None:
@@ -175,7 +175,10 @@ class SteppedModel:
             total += (values.size + 3) // 4 * 4
         staged, enqueued = self._meta_staging.fill(total, places)
         if self._meta_dev is None or self._meta_dev.numel() < total:
-            self._meta_dev = torch.empty(max(total, 4 * self.engine_config.max_tokens_in_batch + 64), dtype=torch.int32, device=self.device)
+            ecfg = self.engine_config
+            if self.latent_expansion is not None:       # (the step of memory profiling, the largest, comes without their arrays)
+                room += self.latent_expansion.most_ints(ecfg.max_tokens_in_batch, ecfg.max_batch_size, ecfg.max_blocks_per_seq)
+            self._meta_dev = torch.empty(max(total, room, 4 * ecfg.max_tokens_in_batch + 64), dtype=torch.int32, device=self.device)
             # captured graphs read the old buffer; their shared memory pool goes with them (a capture into a pool whose last graph is
             # gone is refused by the caching allocator)
             self._decode_graphs.clear()

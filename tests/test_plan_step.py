@@ -140,6 +140,7 @@ def test_latent_expansion_covers_what_its_portions_see(window):
             assert ex is None
             continue
         A = ex.arrays
+        assert sum((v.size + 3) // 4 * 4 for v in A.values()) <= spec.most_ints(plan.num_tokens, len(parts), max(-(-(a + n) // 16) for _, a, n in parts))
         assert ex.seqs == k and ex.rows == sum(n for _, _, n in parts[:k])
         made = {int(d): (int(r), int(p)) for r, p, d in zip(A["ex_page_row"], A["ex_page_no"], A["ex_page_dst"])}
         assert len(made) == A["ex_page_dst"].size and max(made) < ex.pages == A["ex_table"].size
