@@ -8,7 +8,9 @@ class PinnedRing:
     prepares a step waits for the copy that the step before it enqueued, which on the device comes after everything enqueued in
     front of it; with several it prepares the next step while the device still works. Steps in a row that nobody waits for, one buffer
     and several: rokevik's prompts (4 x 2000 tokens) 2350 and 2166 us, vafozen's prompts beside decoded tokens 1345 and 1251, the prompts of
-    kekapel, lorulix and ratilorn 2635 and 2556, 2555 and 2436, 3041 and 2965. The number of buffers bounds how far it gets ahead."""
+    kekapel, lorulix and ratilorn 2635 and 2556, 2555 and 2436, 3041 and 2965. The number of buffers bounds how far it gets ahead. A caller
+    that reads a step's results before it prepares the next gains nothing by them. A buffer that is made is as large as the largest so far:
+    each is made anew only where the steps themselves grow."""
 
     def __init__(self, slots: int, floor: int = 1024):
         self._slots = [[None, None, None] for _ in range(slots)]        # tensor, its numpy view, event
@@ -22,8 +24,8 @@ class PinnedRing:
         if slot[2] is not None:
             slot[2].synchronize()
         if slot[0] is None or slot[0].numel() < total:
-            cap = max(self._floor, 1 << (max(total, 1) - 1).bit_length())
-            slot[0] = torch.empty(cap, dtype=torch.int32, pin_memory=True)
+            self._floor = max(self._floor, 1 << (max(total, 1) - 1).bit_length())
+            slot[0] = torch.empty(self._floor, dtype=torch.int32, pin_memory=True)
             slot[1] = slot[0].numpy()
         host: np.ndarray = slot[1]
         for at, values in arrays:

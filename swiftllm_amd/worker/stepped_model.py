@@ -65,7 +65,7 @@ class SteppedModel:
         self.state = None           # StateSlotManager of designs with per-sequence recurrent state
         self.block_elems = 0
         self._layout_pool()
-        self._meta_staging, self._meta_dev = PinnedRing(2), None
+        self._meta_staging, self._meta_dev = PinnedRing(2, 4 * engine_config.max_tokens_in_batch + 64), None
         self.after_launch_hook = None
         self.latent_expansion = None        # LatentExpansion of designs with latent attention (worker/kernels/latent.py)
         # pure-decode steps (every sequence brings one token and asks for its logits) replay a captured hipGraph, one per

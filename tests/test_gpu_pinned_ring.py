@@ -22,3 +22,15 @@ def test_copies_behind_a_busy_device(slots):
         out.append((i, n, dev))
     for i, n, dev in out:
         assert dev.tolist() == [1000 + i] * 2 + [i + k for k in range(n - 2)]
+
+
+def test_buffers_are_as_large_as_the_largest_so_far():
+    """One large step (memory profiling) sizes every buffer: those after it are not made anew as steps grow up to its size."""
+    from swiftllm_amd.worker.pinned_ring import PinnedRing
+    ring, made = PinnedRing(3, floor=4), set()
+    for n in [900] + list(range(3, 900, 40)):
+        staged, enqueued = ring.fill(n, [(0, np.arange(n, dtype=np.int32))])
+        assert staged.numel() == n and staged.tolist() == list(range(n))
+        enqueued()
+        made.add(staged.data_ptr())
+    assert len(made) == 3
