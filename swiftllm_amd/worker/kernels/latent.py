@@ -91,7 +91,12 @@ class LatentAttention:
         if dtype != torch.float32:
             lib, code = _hip.load(), _hip.dtype_code(dtype)
             self.decodes = bool(lib.swl_latent_decode_supported(mixer.kv_rank, mixer.rot_dim, spec.head_dim, mixer.value_dim, code))
-            self.folds = bool(lib.swl_latent_fold_supported(mixer.head_dim, mixer.rot_dim, mixer.kv_rank, spec.head_dim, code))
+            self.folds = self.decodes and bool(lib.swl_latent_fold_supported(mixer.head_dim, mixer.rot_dim, mixer.kv_rank, spec.head_dim, code))
+        # the up-projections the other way round, where a kernel reads them; kept with the weights, which several runs of a layer share
+        if self.folds and weight.uk_t is None:
+            weight.uk_t = weight.uk.transpose(1, 2).contiguous()
+        if (self.decodes or self.expands) and weight.uv is None:
+            weight.uv = weight.uv_t.transpose(1, 2).contiguous()
 
     def __call__(self, proj: torch.Tensor, gate: torch.Tensor, ctx) -> torch.Tensor:
         """gate: [T, heads] logits, a column slice of the projected rows."""

@@ -64,9 +64,9 @@ class RokevikLayerWeight:
             self.gate_col = mx.q_size + mx.dkv_size
             self.c_norm = f32("mix.dkv.norm", (mx.kv_rank,))
             self.uk = mat("mix.uk", (H * mx.head_dim, mx.kv_rank)).view(H, mx.head_dim, mx.kv_rank).contiguous()
-            self.uk_t = self.uk.transpose(1, 2).contiguous()
-            self.uv = mat("mix.uv", (H * mx.value_dim, mx.kv_rank)).view(H, mx.value_dim, mx.kv_rank).contiguous()
-            self.uv_t = self.uv.transpose(1, 2).contiguous()
+            self.uv_t = mat("mix.uv", (H * mx.value_dim, mx.kv_rank)).view(H, mx.value_dim, mx.kv_rank) \
+                .transpose(1, 2).contiguous()
+            self.uk_t = self.uv = None      # (the same the other way round: LatentAttention, where a kernel reads them)
             self.o = mat("mix.o", (w, mx.o_size))
         else:
             n = mx.width

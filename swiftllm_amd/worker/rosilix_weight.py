@@ -71,9 +71,9 @@ class RosilixLayerWeight:
             parts.append(mat("mix.g", (H, w)))
             self.proj = _pad_rows(torch.cat(parts, dim=0))
             self.uk = mat("mix.uk", (H * mx.head_dim, mx.kv_rank)).view(H, mx.head_dim, mx.kv_rank).contiguous()
-            self.uk_t = self.uk.transpose(1, 2).contiguous()
-            self.uv = mat("mix.uv", (H * mx.value_dim, mx.kv_rank)).view(H, mx.value_dim, mx.kv_rank).contiguous()
-            self.uv_t = self.uv.transpose(1, 2).contiguous()
+            self.uv_t = mat("mix.uv", (H * mx.value_dim, mx.kv_rank)).view(H, mx.value_dim, mx.kv_rank) \
+                .transpose(1, 2).contiguous()
+            self.uk_t = self.uv = None      # (the same the other way round: LatentAttention, where a kernel reads them)
             self.sink = f32("mix.sink", (H,))
         self.o = mat("mix.o", (w, mx.o_size))
         if lcfg.mlp is not None:

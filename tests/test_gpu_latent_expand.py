@@ -150,6 +150,37 @@ def check_step(parts, rows, window, sink, half, dtype, H, e):
     print(f"largest error {math.sqrt(worst):.4e}, folded {math.sqrt(worst_folded):.4e}")
 
 
+@pytest.mark.parametrize("r,dr,e,pad,dtype,held", [(512, 64, 128, 0, torch.bfloat16, "uk_t uv"), (512, 64, 128, 0, torch.float32, ""), (128, 64, 128, 0, torch.float16, "uv"),
+                                                   (96, 64, 128, 0, torch.bfloat16, ""), (512, 64, 24, 0, torch.bfloat16, ""),
+                                                   (512, 64, 128, 32, torch.bfloat16, "uv")])
+def test_up_projections_are_held_the_way_they_are_read(r, dr, e, pad, dtype, held):
+    """Beside the two of the folded form a layer keeps the matrices that its kernels read, once for all of its runs."""
+    from swiftllm_amd.worker.kernels.latent import LatentAttention
+    from swiftllm_amd.worker.kernels.window_attn import AttentionSpec, PoolSlice
+    H, d = 4, 128
+    mx = SimpleNamespace(num_q_heads=H, head_dim=d, rot_dim=dr, value_dim=e, kv_rank=r)
+    uk, uv = torch.randn(H, d, r).to(dtype).cuda(), torch.randn(H, e, r).to(dtype).cuda()
+    w = SimpleNamespace(uk=uk, uk_t=None, uv=None, uv_t=uv.transpose(1, 2).contiguous())
+    spec = AttentionSpec(H, 1, r + dr + pad, r + pad, 0.1)
+    kept = []
+    for _ in range(2):
+        LatentAttention(mx, w, spec, 1e-6, PoolSlice(0, 16 * (r + dr + pad)), 4096, 0)
+        assert " ".join(n for n in ("uk_t", "uv") if getattr(w, n) is not None) == held
+        assert w.uk_t is None or torch.equal(w.uk_t, uk.transpose(1, 2))
+        assert w.uv is None or torch.equal(w.uv, uv)
+        kept.append((w.uk_t, w.uv))
+    assert all(a is b for a, b in zip(*kept))
+
+
+def test_the_weights_of_a_layer_in_fp32_are_held_once(tmp_path):
+    import rosilix_oracle as O
+    from test_gpu_rosilix import make_model
+    cfg = O.make_config([O.latent_mixer(heads=2, dim=128, rot_dim=64, vdim=128, kv_rank=512)])
+    for dtype, held in (("float32", False), ("bfloat16", True)):
+        lw = make_model(tmp_path / dtype, cfg, O.make_weights(cfg), dtype).weight.layers[0]
+        assert (lw.uk_t is not None, lw.uv is not None) == (held, held)
+
+
 def test_portions_past_the_scratch_limit_stay_folded():
     parts = [(0, 0, 64), (1, 0, 64), (2, 0, 64)]
     for pages, rows in ((12, 192), (11, 128), (4, 64), (3, 0)):
