@@ -72,8 +72,8 @@ def test_steps(parts, rows, window, sink, half, dtype):
                                    [(s, 5 + 9 * s, 1) for s in range(33)], [(0, 4500, 1), (1, 3000, 1)], [(0, 0, 40), (1, 99, 1), (2, 250, 1)],
                                    [(s, s, 1) for s in range(70)]])
 def test_single_tokens(parts, window, sink, half, H, e, dtype):
-    """Steps of single tokens, and behind expanded portions (csrc/latent_decode.hip): shares with and without keys, one page and more than one
-    load of page ids holds, tokens and heads around the kernels' groups of 8 and 16, and more tokens than are folded beside the rotary."""
+    """Steps of single tokens, and behind expanded portions (csrc/latent_decode.hip): shares with and without keys, from one page a share on,
+    tokens and heads around the kernels' groups of 4 and 16, and more tokens than are folded beside the rotary."""
     check_step(parts, sum(n for _, _, n in parts if n > 1), window, sink, half, dtype, H, e)
 
 
@@ -137,17 +137,65 @@ def check_step(parts, rows, window, sink, half, dtype, H, e):
         sc = sc.masked_fill(~see, -math.inf)
         if sink:
             sc = torch.cat((sc, sinks.double()[:, None, None].expand(H, cnt, 1)), 2)
-        want = torch.einsum("hqk,hke->qhe", torch.softmax(sc, 2)[:, :, :a + cnt], v)
-        want = (want * torch.sigmoid(rows_in[row:row + cnt, gate_col:gate_col + H].double())[:, :, None]).reshape(cnt, -1)
+        results = []
+        for without in (slice(0), slice(max(a - a % 16 - 16, 0), a - a % 16)):     # (a whole page's keys left out: what a result that lost them would be)
+            x = sc.clone()
+            x[:, :, without] = -math.inf
+            o = torch.einsum("hqk,hke->qhe", torch.softmax(x, 2)[:, :, :a + cnt], v)
+            results.append((o * torch.sigmoid(rows_in[row:row + cnt, gate_col:gate_col + H].double())[:, :, None]).reshape(cnt, -1))
+        want, lost = results
         # a key's and a value's products are rounded once (as folded queries and latent results are): scores move by sqrt(d) of such
         # roundings of |q| |k| ~ 1, results by one of the largest |v| ~ 4, and by what the scores' weights move
         bound = 24 * UNIT[dtype]
         err = (got[row:row + cnt] - want).abs().max().item()
+        # averages over many keys are small: the 2-norm of a portion's error against its result's. Rounded are the keys or the queries (scores of order
+        # one move by 0.6 of a unit), the values, their sums and the result: some five times 0.6 of a unit, in squares
+        size = 4 * UNIT[dtype] * want.norm()
+        for name, o in (("got", got), ("folded", folded)):
+            assert (o[row:row + cnt] - want).norm() <= size, (name, s, a, cnt, float((o[row:row + cnt] - want).norm() / want.norm()))
+        if cnt == 1 and a >= 16 and not window:
+            assert (lost - want).norm() > 2 * size
         worst += float(((got[row:row + cnt] - want) ** 2).sum())
         worst_folded += float(((folded[row:row + cnt] - want) ** 2).sum())
         assert err <= bound, (s, a, cnt, err, bound)
         row += cnt
     print(f"largest error {math.sqrt(worst):.4e}, folded {math.sqrt(worst_folded):.4e}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("window", [0, 4999])
+@pytest.mark.parametrize("H,e,shares", [(16, 128, 1), (3, 64, 1), (20, 16, 1), (16, 128, 2)])
+def test_shares_of_many_pages(H, e, shares, window, dtype):
+    """A share whose pages are more than a wave loads the ids of at a time (64 of its every fourth one): 5000 and 9000 keys, windows that begin
+    inside a page, and a sequence of few beside them."""
+    from swiftllm_amd import _hip
+    g = torch.Generator().manual_seed(H + shares)
+    r, dr = 512, 64
+    lens = [5000, 37, 9011]
+    pages = [-(-n // 16) for n in lens]
+    pool = torch.randn(sum(pages) + 2, 16 * (r + dr), generator=g).to(dtype)
+    blocks, table = torch.randperm(sum(pages) + 2, generator=g).int(), torch.zeros(len(lens), max(pages), dtype=torch.int32)
+    for s, n in enumerate(pages):
+        table[s, :n] = blocks[sum(pages[:s]):sum(pages[:s]) + n]
+    q = torch.randn(len(lens), H * (r + dr), generator=g).to(dtype)
+    uv = torch.randn(H, e, r, generator=g).div(math.sqrt(r)).to(dtype)
+    scale = (r + dr) ** -0.5
+    dev = [t.cuda() for t in (q, pool, table, torch.arange(len(lens)).int(), torch.tensor(lens).int() - 1, uv)]
+    scratch = torch.full((shares * len(lens) * H * (r + 2),), float("nan"), device="cuda")
+    y = torch.empty(len(lens), H * e, dtype=dtype, device="cuda")
+    code, stream = _hip.dtype_code(dtype), _hip.stream()
+    _hip.call("swl_latent_decode", _hip.ptr(scratch), *[_hip.ptr(t) for t in dev[:5]], len(lens), H, q.shape[1], window, scale, table.shape[1], pool.shape[1],
+              shares, code, stream)
+    _hip.call("swl_latent_unfold", _hip.ptr(y), _hip.ptr(scratch), _hip.ptr(dev[5]), 0, 0, 0, len(lens), H, e, shares, code, stream)
+    for s, n in enumerate(lens):
+        c = torch.cat([pool[int(b)].view(16, r + dr) for b in table[s, :pages[s]]])[:n].double()
+        sc = q[s].view(H, -1).double() @ c.T * scale
+        if window:
+            sc[:, :max(n - window, 0)] = -math.inf
+        want = torch.einsum("hr,her->he", torch.softmax(sc, 1) @ c[:, :r], uv.double())
+        err = (y[s].cpu().double().view(H, e) - want).norm(dim=1) / want.norm(dim=1)
+        # the sum's and the result's rounding; a page of 16 keys of n is some sqrt(16 / n) of the result, 4 % and more
+        assert float(err.max()) <= 2 * UNIT[dtype], (s, float(err.max()))
 
 
 @pytest.mark.parametrize("r,dr,e,pad,dtype,held", [(512, 64, 128, 0, torch.bfloat16, "uk_t uv"), (512, 64, 128, 0, torch.float32, ""), (128, 64, 128, 0, torch.float16, "uv"),
