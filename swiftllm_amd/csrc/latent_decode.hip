@@ -4,6 +4,8 @@
 //   swl_latent_fold     qa[t][h] = (W_uk,h^T q_th | rotated part), and the token's own cached row (the work of swl_latent_rope_store_kv)
 //   swl_latent_decode   attention over shares of the keys, partial results
 //   swl_latent_unfold   y[t][h] = sigmoid(gate) W_uv,h (sum of the shares)
+// Made for one row, R = 512 and 64 rotated columns, whose fragments, LDS places and loads of a page are constants below: at any other a step takes the
+// folded chain (two batched library products around the attention of window_attn_mfma.hip).
 //
 // What bounds it: 32 tokens at 1000 keys are 38 MB of cached rows, 6 to 8 us; every launch of a step costs about 4 us whatever it does.
 // window_attn_mfma.hip reads the values' transposed copy beside the rows (71 MB) with one-wave workgroups, two a CU, and leaves 16 shares of 32 x 16

@@ -5,7 +5,7 @@
 // Why: a prompt's queries folded through W_uk attend to rows of rank + rot columns and sum values of `rank`; expanded, a (query, key, head)
 // takes dim + rot + 2 vdim column steps instead of 3 rank + rot (values count twice, in two 16-bit terms): 448 instead of 1600 at 128 + 64,
 // 128 and rank 512. The expansion is one product of the cached rows with both matrices, which is what folding the queries in and unfolding
-// the values took. Decoded tokens read few queries' worth of keys and stay folded (StepPlan.expand_prefix has the rule).
+// the values took. Decoded tokens read few queries' worth of keys and stay folded (worker/batch_plan.py, LatentExpansion.pays, has the rule).
 // What bounds it: as the expert products (moe_grouped.hip), a CU's share of L2: a workgroup takes 128 cached tokens x 128 columns
 // (tile_product.h), 8 pages whose rows the staging picks up one page an instruction; every XCD takes an equal run of the row tiles with all
 // their column tiles, so that its L2 holds a few of the rows and the matrices. Results leave as whole lines through LDS.

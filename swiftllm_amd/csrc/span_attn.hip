@@ -804,6 +804,7 @@ int launch_span(SpanParams &p, int key_splits, hipStream_t s) {
     constexpr bool narrow = D + DV < 256;
     constexpr int waves = narrow ? kSpanNarrowWaves : kSpanWaves, windows = narrow ? kSpanNarrowWaves * KH : kSpanWaves;
     p.qt = span_queries(p.H / p.G, 128 / KH);
+    if (p.rel && p.qt < (narrow && KH == 1 ? 32 : 16)) return SWL_ERR_UNSUPPORTED;      // (a wave's rows are of more heads than it has bias windows)
     const int per = p.qt < kSpan ? kSpan / p.qt : 1;
     const dim3 grid(static_cast<unsigned>(p.num_spans * per), static_cast<unsigned>(key_splits), static_cast<unsigned>(p.G));
     const size_t lds = 2 * (static_cast<size_t>(kSpanKeys * KH) * (D + DV) * 2 + (p.rel ? windows * 64 * sizeof(float) : 0));
@@ -858,7 +859,8 @@ extern "C" int swl_span_attn_supported(int32_t num_q_heads, int32_t num_kv_heads
     if (num_v_heads <= 0 || num_kv_heads % num_v_heads) return 0;
     const int rep = num_q_heads / num_kv_heads;
     if (rep > 64 || num_kv_heads > 65535) return 0;
-    // (a wave's bias window is one head's: its 16 rows are queries of one)
+    // (a wave holds the bias windows of one head, in the narrow kernel with two waves a row group of two: up to four heads a key head leave 16 or
+    // 32 queries of a head to a workgroup of 64 or 128 rows; launch_span checks it)
     if (has_rel && (rep > 4 || dim > 128 || vdim > 128)) return 0;
 #define SWL_SPAN_IS(DD, DDV) if (dim == DD && vdim == DDV) return 1;
     SWL_SPAN_SHAPES(SWL_SPAN_IS)

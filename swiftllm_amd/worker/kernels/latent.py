@@ -78,7 +78,11 @@ class LatentAttention:
 
     Single tokens, us of 32 at 1024 keys, 16 heads of 128 over rank 512 + 64, from the projection to the gated results: rotary and store 5.5, two
     batched products 4.2 and 9.2, attention of csrc/window_attn_mfma.hip 26, its combining launch 6.3, gate 4.7: 56; by csrc/latent_decode.hip
-    6.6, 15.8 and 7.8: 30."""
+    6.6, 15.8 and 7.8: 30. That is made for rank 512 + 64 (swl_latent_decode_supported); other rows take the chain. All of it by tokens, heads
+    and keys, chain / own launches: 1 x 16 x 1000 41 / 21; 64 x 8 x 300 46 / 28, x 4000 143 / 70; 64 x 40 x 1000 129 / 61; 256 x 16 x 300 93 / 57; 512 x
+    16 x 40 79 / 76, x 1000 287 / 182; 256 x 40 x 40 91 / 94, x 300 165 / 128; 512 x 40 x 40 98 / 164, x 300 282 / 226: the value product reads a
+    head's matrix for every four tokens, which only keys few enough not to matter let one see. (Counts alone decide, for captured steps, and cannot
+    tell these apart.)"""
 
     def __init__(self, mixer, weight, spec: AttentionSpec, eps: float, pool_slice, max_positions: int, dkv_col: int):
         self.mixer, self.w, self.spec, self.eps, self.pool_slice, self.max_positions = mixer, weight, spec, eps, pool_slice, max_positions
