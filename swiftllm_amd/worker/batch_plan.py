@@ -166,15 +166,18 @@ class LatentExpansion:
 
     def __init__(self, dim: int, rot_dim: int, vdim: int, rank: int, window: int, max_pages: int, min_beside: int = 0):
         self.window, self.max_pages, self.min_beside = window, max_pages, min_beside
-        # columns a visible (query, key) pair costs more when folded (values count twice), and what expanding one more key costs
-        self.pair_gain = (3 * rank + rot_dim) - (dim + rot_dim + 2 * vdim)
-        self.key_cost = (dim + vdim) * rank
+        # tenths of a column: what a visible (query, key) pair costs more when folded (values count twice; a column of the heads' own keys, which
+        # a workgroup stages for one head alone, 1.3 of one for all), and what expanding one more key costs
+        self.pair_gain = 10 * (3 * rank + rot_dim) - 13 * (dim + rot_dim + 2 * vdim)
+        self.key_cost = 10 * (dim + vdim) * rank
 
     def pays(self, start: np.ndarray, count: np.ndarray) -> np.ndarray:
         """By portion: its own keys take as long to expand as its queries to fold; keys before it are extra. A column of the expansion takes
         half as long as one of attention. Measured, us from the projection to the heads' results, 8 heads of 128 + 64 over rank 512 in a window
         of 1024, folded and expanded: 16 tokens 34.9, 21.4; 11 x 333 94.7, 57.0; 4 x 2000 276, 165; 64 behind 1000 50.2, 33.1; 8 x 64 behind
-        1000 67.6, 66.2; 8 x 128 98.5, 69.4. 16 heads, no window: 4 x 2000 566, 350; 8 x 64 behind 1000 97.8, 88.6; 8 x 128 behind 3000 277, 269."""
+        1000 67.6, 66.2; 8 x 128 98.5, 69.4. 16 heads, no window: 4 x 2000 566, 350; 8 x 64 behind 1000 97.8, 88.6; 8 x 128 behind 3000 277, 269.
+        By rank, no window: 40 heads of 64 + 64 and 128 over 128 (448 columns against 384, never expanded) 100 tokens 29, 24; 500 49, 46; 11 x 333 150, 164;
+        2000 181, 277; 4 x 500 behind 500 154, 248; 8 heads 2000 66, 62; 8 heads of 128 + 64 over 256 4 x 128 behind 3000 71, 74."""
         before, seen = start, count * (2 * start + count + 1) // 2      # (seen: pairs)
         if self.window > 0:
             before, seen = np.minimum(start, self.window - 1), np.minimum(seen, count * self.window)

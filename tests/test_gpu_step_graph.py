@@ -31,8 +31,9 @@ def test_a_step_on_expanded_pages_between_captured_decode_steps(tmp_path):
     """Memory profiling runs a step of the most tokens without a pool, and so without the arrays of the expansion: the buffer it sizes has
     room for them, and the largest step leaves the captures in place."""
     import rosilix_oracle
+    from swiftllm_amd.worker.batch_plan import plan_step
     from test_gpu_rosilix import make_model as make_rosilix
-    cfg = rosilix_oracle.make_config([rosilix_oracle.latent_mixer(heads=2, dim=64, rot_dim=64, vdim=64, kv_rank=64)])
+    cfg = rosilix_oracle.make_config([rosilix_oracle.latent_mixer(heads=2, dim=64, rot_dim=64, vdim=64, kv_rank=256)])
     W = rosilix_oracle.make_weights(cfg)
     model = make_rosilix(tmp_path / "m", cfg, W, "bfloat16", num_blocks=130, graph=True)
     model.profile_num_blocks()
@@ -43,7 +44,7 @@ def test_a_step_on_expanded_pages_between_captured_decode_steps(tmp_path):
     assert model.graph_captures == 1
     held = model._meta_dev
     prompts = [tokens_for(cfg, 341, s) for s in (1, 2, 3)]
-    assert model.latent_expansion is not None
+    assert plan_step([entry(s, prompts[s - 1], 0, (340,)) for s in (1, 2, 3)]).latent_expansion(model.latent_expansion).seqs == 3
     model.step([entry(s, prompts[s - 1], 0, (340,)) for s in (1, 2, 3)])                # 1023 tokens of 1024
     model.step([entry(s, tokens_for(cfg, 170, s), 341, (169,)) for s in (1, 2, 3)])     # (three times the pages of its tokens)
     model.free_seqs_resources([1, 2, 3])

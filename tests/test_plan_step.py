@@ -169,3 +169,12 @@ def test_latent_expansion_beside_folded_portions(tokens, beside, expanded):
     plan = plan_step(entries + [StepEntry(9 + i, [1], 20, (0,)) for i in range(beside)])
     ex = plan.latent_expansion(LatentExpansion(128, 64, 128, 512, 0, 4096, 64))
     assert (ex is not None and ex.rows == tokens) == expanded and (expanded or ex is None)
+
+
+@pytest.mark.parametrize("dim,rot,vdim,rank,start,count,pays", [(128, 64, 128, 512, 0, 16, True), (128, 64, 128, 512, 1000, 64, True), (128, 64, 128, 512, 3000, 17, False),
+                                                                (64, 64, 128, 128, 0, 2000, False), (64, 64, 128, 128, 0, 100, False),
+                                                                (128, 64, 128, 256, 0, 2000, True), (128, 64, 128, 256, 3000, 128, False)])
+def test_latent_expansion_by_the_rank(dim, rot, vdim, rank, start, count, pays):
+    """The heads' own keys have to be a good deal narrower than folded rows: they are staged for one head alone."""
+    from swiftllm_amd.worker.batch_plan import LatentExpansion
+    assert LatentExpansion(dim, rot, vdim, rank, 0, 4096).pays(np.array([start]), np.array([count])).tolist() == [pays]
