@@ -706,13 +706,38 @@ __global__ __launch_bounds__(kRkThreads) void latent_fold_kernel(
 
 constexpr int kDiffMaxDim = 256, kDiffMaxShares = 32;
 
-// A wave per (token, head). SHARES: a1 and a2 still are key shares (attn_combine.h; NATURAL: their maxima in natural units), which the wave
-// weighs and adds up itself: lane s weighs share s of a1, lane 32 + s of a2, and each half of the wave reads its map's columns, eight
-// shares in flight. Bound by latency: 32 tokens x 16 heads of 128, 8 shares: a launch that adds them up and this one after it (four heads a wave) 4.8 +
-// 6.6 us -> 4.7; with a lane on both maps' columns, a 4-byte load at a time, 8.8.
-template <typename T, bool SHARES, bool NATURAL>
-__global__ __launch_bounds__(256) void diff_head_combine_kernel(T *out, const float *a, const float *part_ml, int shares, const T *gate,
-                                                                int64_t gate_stride, float lambda, float mult, float eps, int64_t rows, int H, int dv) {
+// grid: (tokens, workgroups that share a token's heads), a wave takes every (4 grid.y)-th head.
+template <typename T>
+__global__ __launch_bounds__(256) void diff_head_combine_kernel(T *out, const float *a, const T *gate, int64_t gate_stride, float lambda, float mult,
+                                                                float eps, int H, int dv) {
+    const int64_t t = blockIdx.x;
+    const int lane = threadIdx.x & 63;
+    for (int h = blockIdx.y * 4 + (threadIdx.x >> 6); h < H; h += 4 * gridDim.y) {
+        const float *a1 = a + ((t * 2) * H + h) * dv, *a2 = a + ((t * 2 + 1) * H + h) * dv;
+        float ss = 0.f;
+        for (int e = lane; e < dv; e += 64) {
+            const float o = a1[e] - lambda * a2[e];
+            ss += o * o;
+        }
+        ss = wave_allreduce_sum(ss);
+        const float g = gate ? rk_sigmoid(to_f(gate[t * gate_stride + h])) : 1.0f;
+        const float f = mult * g / sqrtf(ss / static_cast<float>(dv) + eps);
+        for (int e = lane; e < dv; e += 64) out[(t * H + h) * dv + e] = to_t<T>((a1[e] - lambda * a2[e]) * f);
+    }
+}
+// Few tokens: a workgroup for every four heads, so that all are on the chip at once; many: one a token, whose rows lie together. us, one workgroup a token / one
+// for four heads: 32 tokens x 16 heads of 128 5.6 / 3.5, 500 6.4 / 4.8, 1000 7.6 / 6.9, 2000 12.5 / 13.4, 4000 21.9 / 22.5, 8000 39.8 / 43.0; 8 of 128 8000
+// 21.9 / 22.7.
+constexpr int64_t kDiffManyTokens = 1536;
+inline unsigned diff_groups(int H) { return static_cast<unsigned>(H < 4 * 65535 ? (H + 3) / 4 : 65535); }
+
+// The same where a1 and a2 still are key shares (attn_combine.h; NATURAL: their maxima in natural units), which a wave, of one (token, head), weighs and
+// adds up itself: lane s weighs share s of a1, lane 32 + s of a2, and each half of the wave reads its map's columns, eight shares in flight. Bound by
+// latency: 32 tokens x 16 heads of 128, 8 shares: a launch that adds them up and the one above after it (four heads a wave) 4.8 + 6.6 us -> 4.7; with a
+// lane on both maps' columns, a 4-byte load at a time, 8.8.
+template <typename T, bool NATURAL>
+__global__ __launch_bounds__(256) void diff_head_shares_kernel(T *out, const float *a, const float *part_ml, int shares, const T *gate, int64_t gate_stride,
+                                                               float lambda, float mult, float eps, int64_t rows, int H, int dv) {
     const int lane = threadIdx.x & 63;
     const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);     // t * H + h
     if (row >= rows) return;
@@ -720,71 +745,61 @@ __global__ __launch_bounds__(256) void diff_head_combine_kernel(T *out, const fl
     const float g = gate ? rk_sigmoid(to_f(gate[t * gate_stride + (row - t * H)])) : 1.0f;
     const float *a1 = a + r1 * dv, *a2 = a + r2 * dv;
     float ss = 0.f;
-    if constexpr (!SHARES) {
-        for (int e = lane; e < dv; e += 64) {
-            const float o = a1[e] - lambda * a2[e];
-            ss += o * o;
-        }
-        ss = wave_allreduce_sum(ss);
-        const float f = mult * g / sqrtf(ss / static_cast<float>(dv) + eps);
-        for (int e = lane; e < dv; e += 64) out[row * dv + e] = to_t<T>((a1[e] - lambda * a2[e]) * f);
-    } else {
-        constexpr int NE = kDiffMaxDim / 128;       // pieces of four columns of a lane, of its half's map
-        const int sub = lane & 31;
-        const bool live = sub < shares;
-        const float *ml = part_ml + ((live ? sub : 0) * 2 * rows + (lane < 32 ? r1 : r2)) * 2;
-        const float m = live ? ml[0] : kNegBig, l = live ? ml[1] : 0.f;
-        const float *mine = lane < 32 ? a1 : a2;
-        const int64_t plane = 2 * rows * dv;
-        float4_t x[NE];
-        float w = 0.f;
+    constexpr int NE = kDiffMaxDim / 128;       // pieces of four columns of a lane, of its half's map
+    const int sub = lane & 31;
+    const bool live = sub < shares;
+    const float *ml = part_ml + ((live ? sub : 0) * 2 * rows + (lane < 32 ? r1 : r2)) * 2;
+    const float m = live ? ml[0] : kNegBig, l = live ? ml[1] : 0.f;
+    const float *mine = lane < 32 ? a1 : a2;
+    const int64_t plane = 2 * rows * dv;
+    float4_t x[NE];
+    float w = 0.f;
 #pragma unroll
-        for (int j = 0; j < NE; ++j) x[j] = float4_t{0.f, 0.f, 0.f, 0.f};
-        for (int s0 = 0; s0 < shares; s0 += 8) {
-            float4_t p[8][NE];
+    for (int j = 0; j < NE; ++j) x[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < shares; s0 += 8) {
+        float4_t p[8][NE];
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
+        for (int u = 0; u < 8; ++u)
 #pragma unroll
-                for (int j = 0; j < NE; ++j)        // (the last share and piece stand in for the missing ones)
-                    if (j == 0 || dv > 128 * j)
-                        p[u][j] = *reinterpret_cast<const float4_t *>(mine + min(s0 + u, shares - 1) * plane + min(4 * sub + 128 * j, dv - 4));
-            if (s0 == 0) {
-                float mx = m;
+            for (int j = 0; j < NE; ++j)        // (the last share and piece stand in for the missing ones)
+                if (j == 0 || dv > 128 * j)
+                    p[u][j] = *reinterpret_cast<const float4_t *>(mine + min(s0 + u, shares - 1) * plane + min(4 * sub + 128 * j, dv - 4));
+        if (s0 == 0) {
+            float mx = m;
 #pragma unroll
-                for (int d = 1; d < 32; d *= 2) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
-                w = live ? (NATURAL ? expf(m - mx) : exp2f(m - mx)) : 0.f;
-                float den = w * l;
+            for (int d = 1; d < 32; d *= 2) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+            w = live ? (NATURAL ? expf(m - mx) : exp2f(m - mx)) : 0.f;
+            float den = w * l;
 #pragma unroll
-                for (int d = 1; d < 32; d *= 2) den += __shfl_xor(den, d, 64);
-                w *= 1.0f / den;
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const float ws = __shfl(w, (lane & 32) + min(s0 + u, 31), 64);       // (lanes without a share have weight zero)
-#pragma unroll
-                for (int j = 0; j < NE; ++j)
-                    if (j == 0 || dv > 128 * j) x[j] += ws * p[u][j];
-            }
+            for (int d = 1; d < 32; d *= 2) den += __shfl_xor(den, d, 64);
+            w *= 1.0f / den;
         }
 #pragma unroll
-        for (int j = 0; j < NE; ++j) {
+        for (int u = 0; u < 8; ++u) {
+            const float ws = __shfl(w, (lane & 32) + min(s0 + u, 31), 64);       // (lanes without a share have weight zero)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const float other = __shfl_xor(x[j][c], 32, 64);
-                x[j][c] = lane < 32 ? x[j][c] - lambda * other : 0.f;
-                if (4 * sub + 128 * j < dv) ss += x[j][c] * x[j][c];
-            }
+            for (int j = 0; j < NE; ++j)
+                if (j == 0 || dv > 128 * j) x[j] += ws * p[u][j];
         }
-        ss = wave_allreduce_sum(ss);
-        const float f = mult * g / sqrtf(ss / static_cast<float>(dv) + eps);
+    }
 #pragma unroll
-        for (int j = 0; j < NE; ++j) {
-            if (lane < 32 && 4 * sub + 128 * j < dv) {
-                vec4_t<T> o;
+    for (int j = 0; j < NE; ++j) {
 #pragma unroll
-                for (int c = 0; c < 4; ++c) o[c] = to_t<T>(x[j][c] * f);
-                *reinterpret_cast<vec4_t<T> *>(out + row * dv + 4 * sub + 128 * j) = o;
-            }
+        for (int c = 0; c < 4; ++c) {
+            const float other = __shfl_xor(x[j][c], 32, 64);
+            x[j][c] = lane < 32 ? x[j][c] - lambda * other : 0.f;
+            if (4 * sub + 128 * j < dv) ss += x[j][c] * x[j][c];
+        }
+    }
+    ss = wave_allreduce_sum(ss);
+    const float f = mult * g / sqrtf(ss / static_cast<float>(dv) + eps);
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+        if (lane < 32 && 4 * sub + 128 * j < dv) {
+            vec4_t<T> o;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) o[c] = to_t<T>(x[j][c] * f);
+            *reinterpret_cast<vec4_t<T> *>(out + row * dv + 4 * sub + 128 * j) = o;
         }
     }
 }
@@ -996,12 +1011,11 @@ extern "C" int swl_diff_head_combine(void *out, const float *maps, const void *g
     if (num_tokens < 0 || num_heads <= 0 || vdim <= 0 || (gate && gate_stride < num_heads)) return SWL_ERR_BAD_ARG;
     if (num_tokens == 0) return SWL_OK;
     if (!out || !maps) return SWL_ERR_BAD_ARG;
-    const int64_t rows = num_tokens * num_heads;
-    if (num_tokens > 0x7fffffffLL || rows / 4 >= 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
+    if (num_tokens > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
+    const dim3 grid(static_cast<unsigned>(num_tokens), num_tokens >= swl::kDiffManyTokens ? 1 : swl::diff_groups(num_heads));
     SWL_DISPATCH_DTYPE3(dtype, T, {
-        hipLaunchKernelGGL((swl::diff_head_combine_kernel<T, false, false>), dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0,
-                           static_cast<hipStream_t>(stream), static_cast<T *>(out), maps, nullptr, 0, static_cast<const T *>(gate),
-                           gate_stride, lambda, mult, eps, rows, num_heads, vdim);
+        hipLaunchKernelGGL((swl::diff_head_combine_kernel<T>), grid, dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<T *>(out), maps,
+                           static_cast<const T *>(gate), gate_stride, lambda, mult, eps, num_heads, vdim);
     });
     return swl::check_launch();
 }
@@ -1017,7 +1031,7 @@ extern "C" int swl_diff_head_combine_shares(void *out, const float *shares, int3
         !swl::aligned16(out) || !swl::aligned16(shares)) return SWL_ERR_UNSUPPORTED;
     const float *part_ml = shares + num_shares * 2 * rows * vdim;
 #define SWL_DIFF(NATURAL)                                                                                                                  \
-    hipLaunchKernelGGL((swl::diff_head_combine_kernel<T, true, NATURAL>), dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0,       \
+    hipLaunchKernelGGL((swl::diff_head_shares_kernel<T, NATURAL>), dim3(static_cast<unsigned>((rows + 3) / 4)), dim3(256), 0,              \
                        static_cast<hipStream_t>(stream), static_cast<T *>(out), shares, part_ml, num_shares, static_cast<const T *>(gate), \
                        gate_stride, lambda, mult, eps, rows, num_heads, vdim)
     SWL_DISPATCH_DTYPE3(dtype, T, {

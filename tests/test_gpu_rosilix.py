@@ -366,6 +366,18 @@ def test_map_combination_and_head_gate(dtype):
     assert (got.cpu().double().view(n, H, e) - y.double().view(n, H, e) * torch.sigmoid(gate.double())[:, :, None]).abs().max() < tol
 
 
+@pytest.mark.parametrize("tokens", [1535, 1536])
+@pytest.mark.parametrize("H,dv", [(1, 64), (5, 128), (8, 40)])
+def test_map_combination_of_few_and_many_tokens(tokens, H, dv):
+    """From 1536 tokens on a workgroup takes a token's heads, below that four of them."""
+    from swiftllm_amd.worker.kernels.rope_kv import diff_head_combine
+    g = torch.Generator().manual_seed(H)
+    maps, gate = torch.randn(tokens, 2, H, dv, generator=g), torch.randn(tokens, H, generator=g)
+    want = O.unit_rms(maps[:, 0].double() - 0.3 * maps[:, 1].double(), 1e-6) * 0.7 * torch.sigmoid(gate.double())[:, :, None]
+    got = diff_head_combine(maps.view(tokens, -1).cuda(), gate.cuda(), 0.3, 0.7, 1e-6, H, dv, torch.float32)
+    assert (got.cpu().double().view(tokens, H, dv) - want).abs().max() < 1e-5
+
+
 def test_embedding_without_positions_and_squared_relu():
     from swiftllm_amd.worker.kernels.layernorm import embed_positions
     from swiftllm_amd.worker.kernels.moe import relu_squared
