@@ -29,6 +29,7 @@ SOURCES = [
     "gemm_tiny.hip",
     "gemm_wide.hip",
     "gemm_rows.hip",
+    "gemm_tile.hip",
     "argmax.hip",
     "decode_engine.hip",
     "layernorm.hip",
@@ -57,9 +58,9 @@ SOURCES = [
 # What a model family's worker calls (the shared pieces included): `build(only=MODEL_SOURCES[...])` compiles just these, so
 # that the first use from a fresh checkout does not pay for kernels the model never launches. A later full build compiles
 # the rest and links everything.
-_SHARED = ["swap_blocks.hip", "block_table.hip", "argmax.hip", "gemm_skinny.hip", "gemm_wide.hip", "gemm_rows.hip", "gemm_f32.hip"]
+_SHARED = ["swap_blocks.hip", "block_table.hip", "argmax.hip", "gemm_skinny.hip", "gemm_wide.hip", "gemm_rows.hip", "gemm_tile.hip", "gemm_f32.hip"]
 MODEL_SOURCES = {
-    "llama": list(SOURCES[:14]),
+    "llama": list(SOURCES[:15]),
     "Kekapel": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip",
                           "mix_attn.hip", "polynorm.hip", "moe.hip", "moe_grouped.hip"],
     "Lorulix": _SHARED + ["layernorm.hip", "qknorm_kv.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip",

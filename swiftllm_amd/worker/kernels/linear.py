@@ -1,12 +1,13 @@
 """Dense projections. Reference: swiftllm/worker/kernels/linear.py:3-12.
 
-Default: `torch.nn.functional.linear`, which dispatches to hipBLASLt/rocBLAS on ROCm exactly as the
+Default (`skinny=False`): `torch.nn.functional.linear`, which dispatches to hipBLASLt/rocBLAS on ROCm exactly as the
 reference's call dispatches to cuBLAS — same GEMM kernels as the reference run on the same box.
 
 `skinny=True` (EngineConfig.use_skinny_gemm) routes decode-sized calls (M <= 32 tokens) to the
 hand-written weight-streaming MFMA kernel `swl_gemm_skinny` (csrc/gemm_skinny.hip): at that size the
-projection is pure HBM streaming of the weight matrix, 77 % of all bytes a decode step moves
-(SURVEY.md §8f rank 1). Larger M (prefill) stays on the BLAS, which is compute-bound territory.
+projection is pure HBM streaming of the weight matrix, 77 % of all bytes a decode step moves. Prompt-sized calls (more than 256
+tokens) go to the tiled kernel `swl_gemm_tile` (csrc/gemm_tile.hip), with their activation where there is one, as far as `_tile_pays`
+says; the rest stays on the BLAS.
 
 Weights that carry a packed twin (`pack_weight`: a copy in MFMA-fragment order made at load time,
 EngineConfig.pack_decode_weights) are streamed from that copy — same bits, 6-9 % faster (long sequential DRAM
@@ -274,7 +275,57 @@ def linear(a: torch.Tensor, w: torch.Tensor, skinny: bool = False) -> torch.Tens
                   ws.numel() * 4 if ws is not None else 0, m, n, k, _row_stride(a), n, 0,
                   _hip.dtype_code(a.dtype), _hip.stream())
         return out
-    return _blas_linear(a, w)
+    y = linear_tile(a, w) if skinny else None
+    return y if y is not None else _blas_linear(a, w)
+
+
+# Prompt-sized steps (csrc/gemm_tile.hip); up to here the decode GEMMs serve.
+TILE_MIN_TOKENS = DECODE_MAX_TOKENS + 1
+TILE_NONE, TILE_RELU2, TILE_GATED = 0, 1, 2
+TILE_SILU_ROUNDED = 3       # gated unit of rows [up | gate]: round(silu(gate)) up, what silu_and_mul_inplace makes of the product
+
+
+def _tile_pays(m: int, rows: int, k: int, gated: bool = False) -> bool:
+    """Whether the tiled kernel takes a product, `rows` rows of the matrix. Long sums of few tiles are the library's, which splits them (tiles of 64 x 128,
+    us, library's): 1024 x 4096, 409 tokens (56 tiles) 21.2 (13.9), 1110 (144) 21.8 (21.8), 2396 (304) 27 (32); 1024 x 6144, 572 (72) 31 (22), 1167 (152)
+    31.5 (30.5), 2036 (256) 33 (41); 2048 x 8192, 679 (176) 58 (45), 1260 (320) 70 (68), 1559 (400) 71 (73); 4096 x 14336, 360 (192) 107 (84), 741 (384)
+    129 (122), 1521 (768) 172 (188). Up to 2560 columns always (277 of 1024 x 1024 7.4, 8.7). So are very long ones of many tokens, which the
+    library takes in blocks of rows at its best rate: 5112 of 4096 x 14336 505 (458); 4010 tokens 353 (367). And beyond 8192 tokens what is not
+    small, where the library's rate is 5 % to 10 % higher: 12288 of 6144 x 4096 459 (424), 16384 of 8192 x 2048 381 (365), of 1024 x 4096 102 (93), but
+    12288 of 1024 x 4096 77 (102), 10000 of 3072 x 1024 55 (72) — unless the launch does an activation's work (28672 x 4096, 16384 2621 (2733))."""
+    if m > 8192 and m * rows * k > 6e10 and not gated:
+        return False
+    if k <= 2560:
+        return True
+    return -(-m // 64) * -(-rows // 128) * 16 >= min(k - 2048, 6400) and (k <= 8192 or m <= 4096)
+
+
+def linear_tile(a: torch.Tensor, w: torch.Tensor, act: int = TILE_NONE, act_columns: int = 0, limit: float = 0.0, out: torch.Tensor = None):
+    """a[T, in] @ w[out, in]^T of a prompt-sized step in one launch with its activation: TILE_RELU2, of the first act_columns columns;
+    TILE_GATED + ACT_CLAMPED (with `limit`), ACT_SILU, ACT_SILU_UP_FIRST (kernels/moe.py) or TILE_SILU_ROUNDED: of the halves of w's rows. out: rows to
+    write to (a column slice of wider ones, for one). None where the kernel does not serve the call. Rows that are no multiple of 8 long
+    are a column slice of longer ones."""
+    if not (a.is_cuda and a.dim() == w.dim() == 2 and a.shape[0] >= TILE_MIN_TOKENS and a.dtype == w.dtype and a.dtype in (torch.float16, torch.bfloat16)):
+        return None
+    m, k = a.shape
+    rows, n = w.shape[0], w.shape[0] // 2 if act >= TILE_GATED else w.shape[0]
+    if w.shape[1] != k or not w.is_contiguous() or a.stride(1) != 1 or (a.data_ptr() | w.data_ptr()) % 16 or not _tile_pays(m, rows, k, act != TILE_NONE) \
+            or (act == TILE_RELU2 and act_columns % 4) or (act >= TILE_GATED and rows % 2):
+        return None
+    lib, code, ldo = _hip.load(), _hip.dtype_code(a.dtype), -(-n // 8) * 8 if out is None else out.stride(0)
+    if not lib.swl_gemm_tile_supported(m, n, k, a.stride(0), ldo, act, code) or (out is not None and (out.data_ptr() % 16 or out.stride(1) != 1 or n % 8)):
+        return None
+    if out is None:
+        out = torch.empty((m, ldo), dtype=a.dtype, device=a.device)
+        out = out if ldo == n else out[:, :n]
+    _hip.call("swl_gemm_tile", _hip.ptr(out), _hip.ptr(a), _hip.ptr(w), m, n, k, a.stride(0), ldo, 0, 0, act, int(act_columns), float(limit), 0, code,
+              _hip.stream())
+    return out
+
+
+def linear_gated(a: torch.Tensor, w: torch.Tensor, act: int, limit: float = 0.0, out: torch.Tensor = None):
+    """The gated unit `act` (as in linear_tile, without TILE_GATED) of a[T, in] @ w[2 out, in]^T of a prompt-sized step, None where one launch does not serve it."""
+    return linear_tile(a, w, TILE_GATED + act, limit=limit, out=out) if a.shape[0] >= TILE_MIN_TOKENS else None
 
 
 # hipBLASLt's cost per token is far from flat in the token count M (Llama-3-8B widths, bf16, MI355X,
@@ -355,7 +406,7 @@ def linear_f32_pair(a1: torch.Tensor, w1: torch.Tensor, a2: torch.Tensor, w2: to
 
 def linear_grouped(x: torch.Tensor, w: torch.Tensor, skinny: bool = False) -> torch.Tensor:
     """x [groups, T, in], w [groups * out, in] -> [T, groups * out]: columns g * out .. are x[g] @ w[g * out : (g + 1) * out]^T. One
-    launch for decode-sized steps on a packed weight, a product per group otherwise."""
+    launch for decode-sized steps on a packed weight and for prompt-sized ones, a product per group otherwise."""
     groups, m, k = x.shape
     n = w.shape[0]
     out = torch.empty((m, n), dtype=x.dtype, device=x.device)
@@ -367,6 +418,12 @@ def linear_grouped(x: torch.Tensor, w: torch.Tensor, skinny: bool = False) -> to
                   ws.numel() * 4 if ws is not None else 0, m, n, k, k, n, _hip.dtype_code(x.dtype), _hip.stream())
         return out
     size = n // groups
+    if skinny and m >= TILE_MIN_TOKENS and size % 256 == 0 and w.shape[1] == k and x.is_contiguous() and w.is_contiguous() and x.dtype == w.dtype \
+            and x.dtype in (torch.float16, torch.bfloat16) and x.is_cuda and (x.data_ptr() | w.data_ptr()) % 16 == 0 and _tile_pays(m, n, k) \
+            and _hip.load().swl_gemm_tile_supported(m, n, k, k, n, TILE_NONE, _hip.dtype_code(x.dtype)):
+        _hip.call("swl_gemm_tile", _hip.ptr(out), _hip.ptr(x), _hip.ptr(w), m, n, k, k, n, size, m * k, TILE_NONE, 0, 0.0, 0, _hip.dtype_code(x.dtype),
+                  _hip.stream())
+        return out
     for g in range(groups):
         torch.mm(x[g], w[g * size:(g + 1) * size].t(), out=out[:, g * size:(g + 1) * size])
     return out

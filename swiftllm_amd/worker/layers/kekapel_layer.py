@@ -4,7 +4,7 @@ import torch
 
 from swiftllm_amd import _hip
 
-from ..kernels.linear import (DECODE_MAX_TOKENS, F32_MAX_TOKENS, ROWS_MAX_TOKENS, linear, linear_f32, linear_rows,
+from ..kernels.linear import (DECODE_MAX_TOKENS, F32_MAX_TOKENS, ROWS_MAX_TOKENS, linear, linear_f32, linear_gated, linear_rows,
                               linear_rows_partial, linear_silu_gate, linear_splitk)
 from ..kernels.moe import ACT_SILU_UP_FIRST, gated_unit, moe_experts, moe_route
 from ..kernels.polynorm import polynorm
@@ -13,11 +13,13 @@ from ..kernels.window_attn import qknorm_and_store_kv, window_attention
 
 def _project(a: torch.Tensor, w: torch.Tensor, skinny: bool) -> torch.Tensor:
     """a [T, in] @ w[out, in]^T. bf16 / f16: the framework's projection routing (hand-written weight-streaming GEMMs for
-    decode-sized batches, the BLAS otherwise); fp32: true fp32, with a kernel for a few tokens."""
+    decode-sized batches, tiled ones for prompt-sized steps, the BLAS otherwise); fp32: true fp32, with a kernel for a few tokens."""
     m = a.shape[0]      # (asked for before anything else: the steps that nothing below serves pay for one comparison)
     if a.dtype == torch.float32:
         return linear_f32(a, w) if m <= F32_MAX_TOKENS else torch.nn.functional.linear(a, w)
-    if not skinny or m > DECODE_MAX_TOKENS or getattr(w, "_swl_blas_only", False):
+    if m > DECODE_MAX_TOKENS:
+        return linear(a, w, skinny)
+    if not skinny or getattr(w, "_swl_blas_only", False):
         return linear(a, w, False)
     y = linear_rows(a, w) if m <= ROWS_MAX_TOKENS else None
     if y is not None:
@@ -63,7 +65,13 @@ def _silu_unit(a: torch.Tensor, up_gate: torch.Tensor, skinny: bool) -> torch.Te
             if "code -2" not in str(exc):       # (see _project)
                 raise
             up_gate._swl_no_silu = True
-    return gated_unit(_project(a, up_gate, skinny), up_gate.shape[0] // 2, ACT_SILU_UP_FIRST)
+    return _gated_project(a, up_gate, skinny, ACT_SILU_UP_FIRST)
+
+
+def _gated_project(a: torch.Tensor, w: torch.Tensor, skinny: bool, act: int, limit: float = 0.0) -> torch.Tensor:
+    """The gated unit `act` of the two halves of a's product with w's rows -> [T, ff]: in the product's launch for prompt-sized 16-bit steps."""
+    y = linear_gated(a, w, act, limit) if skinny else None
+    return y if y is not None else gated_unit(_project(a, w, skinny), w.shape[0] // 2, act, limit)
 
 
 class KekapelAttention:

@@ -6,10 +6,10 @@ such product). A caller that already has that result passes it as forward's `don
 import torch
 
 from ..kernels.delta_rule import delta_rule_mixer
-from ..kernels.moe import moe_experts_relu2, moe_route_scores, relu_squared
+from ..kernels.linear import TILE_RELU2, linear_tile
+from ..kernels.moe import ACT_CLAMPED, moe_experts_relu2, moe_route_scores, relu_squared
 from ..kernels.window_attn import qknorm_full_and_store_kv, window_attention
-from .kekapel_layer import _project, _project_partials
-from swiftllm_amd import _hip
+from .kekapel_layer import _gated_project, _project, _project_partials
 
 
 class StepContext:
@@ -77,18 +77,15 @@ class LorulixFeedForward:
     def forward(self, h: torch.Tensor, ctx: StepContext, done: torch.Tensor = None):
         mlp, w = self.mlp, self.w
         if mlp.kind == "dense":
-            y = done
-            if y is None:
-                gu = _project(h, w.gate_up, self.skinny)
-                y = torch.empty((h.shape[0], mlp.ffn_inter_dim), dtype=h.dtype, device=h.device)
-                _hip.call("swl_glu_clamp", _hip.ptr(y), _hip.ptr(gu), 0, h.shape[0], mlp.ffn_inter_dim, float(mlp.limit), 0,
-                          _hip.dtype_code3(h.dtype), _hip.stream())
+            y = done if done is not None else _gated_project(h, w.gate_up, self.skinny, ACT_CLAMPED, mlp.limit)
             return _project_partials(y, w.down, self.skinny), None, None
         idx, wts = moe_route_scores(h, w.router, mlp.top_k, mlp.router_scale)
         out = moe_experts_relu2(h, idx, wts, w.up, w.down)
         if w.shared_up is None:
             return out, None, None
         fs = mlp.shared_ffn_inter_dim
+        if done is None and self.skinny:
+            done = linear_tile(h, w.shared_up, TILE_RELU2, fs)
         z = done if done is not None else _project(h, w.shared_up, self.skinny)     # [T, fs + 1]: the shared expert's up rows, then its gate logit
         shared = _project(z[:, :fs] if done is not None else relu_squared(z, fs), w.shared_down, self.skinny)
         return out, shared, z[:, fs:fs + 1]

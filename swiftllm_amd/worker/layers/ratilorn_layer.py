@@ -2,11 +2,11 @@
 the result and its addition to the fp32 stream are the model's fused step (kernels/rms_stream.py: post_norm_add)."""
 import torch
 
-from ..kernels.moe import ACT_SILU, gated_unit, moe_experts, moe_route_grouped
+from ..kernels.moe import ACT_SILU, moe_experts, moe_route_grouped
 from ..kernels.sigmoid_attn import sigmoid_attention
 from ..kernels.ssd import state_space_mixer
 from ..kernels.window_attn import MASK_WINDOW, AttentionSpec, masked_attention, qkv_bias_norm_store
-from .kekapel_layer import _project
+from .kekapel_layer import _gated_project, _project
 from .lorulix_layer import StepContext
 
 
@@ -81,15 +81,15 @@ class RatilornFeedForward:
     def __init__(self, layer_config, weight, skinny: bool):
         self.mlp, self.w, self.skinny = layer_config.mlp, weight, skinny
 
-    def _unit(self, h, gate_up, down, ff):
-        return _project(gated_unit(_project(h, gate_up, self.skinny), ff, ACT_SILU), down, self.skinny)
+    def _unit(self, h, gate_up, down):
+        return _project(_gated_project(h, gate_up, self.skinny, ACT_SILU), down, self.skinny)
 
     def forward(self, h: torch.Tensor, ctx: StepContext, share: ValueShare):
         mlp, w = self.mlp, self.w
         if mlp.kind == "dense":
-            return self._unit(h, w.gate_up, w.down, mlp.ffn_inter_dim), None
+            return self._unit(h, w.gate_up, w.down), None
         idx, wts = moe_route_grouped(h, w.router, w.correction, mlp.top_k, mlp.group_count, mlp.group_keep)
         out = moe_experts(h, idx, wts, w.gate_up, w.down, 0.0, ACT_SILU)
         if w.shared_gate_up is None:
             return out, None
-        return out, self._unit(h, w.shared_gate_up, w.shared_down, mlp.shared_ffn_inter_dim)
+        return out, self._unit(h, w.shared_gate_up, w.shared_down)

@@ -3,7 +3,7 @@ stream and the next input norm are the model's fused step (kernels/rms_stream.py
 import torch
 
 from ..kernels.latent import LatentAttention
-from ..kernels.linear import ROWS_MAX_TOKENS, linear_rows
+from ..kernels.linear import ROWS_MAX_TOKENS, TILE_RELU2, linear_rows, linear_tile
 from ..kernels.moe import relu_squared
 from ..kernels.rope_kv import diff_head_combine, rope_and_store_kv
 from ..kernels.window_attn import MASK_CHUNK, MASK_WINDOW, AttentionSpec, masked_attention
@@ -64,6 +64,8 @@ class RosilixFeedForward:
 
     def forward(self, h: torch.Tensor, ctx: StepContext) -> torch.Tensor:
         y = linear_rows(h, self.w.up, relu2=True) if self.skinny and h.shape[0] <= ROWS_MAX_TOKENS else None
+        if y is None and self.skinny:
+            y = linear_tile(h, self.w.up, TILE_RELU2, self.mlp.ffn_inter_dim)
         if y is None:
             y = relu_squared(_project(h, self.w.up, self.skinny), self.mlp.ffn_inter_dim)
         return _project_partials(y, self.w.down, self.skinny)

@@ -43,6 +43,7 @@ from ..kernels.linear import (row_scaled_silu_gate_ok, alt_residual_like, linear
                               linear_splitk_from_splitk, tiny_from_splitk_ok)
 from ..kernels.linear import RawResidual, linear_rows_add, linear_silu_gate_nf, linear_splitk_nf, nf_ok, rows_add_ok
 from ..kernels.linear import linear_silu_gate_nx, linear_splitk_nx, nx_ok
+from ..kernels.linear import TILE_SILU_ROUNDED, linear_gated
 from ..kernels.rmsnorm import RowScalePending
 from ..kernels.rmsnorm import (add_scale_from_splitk, deferred_norm_ok, fused_add_rmsnorm_inplace,
                                fused_add_rmsnorm_from_splitk)
@@ -331,6 +332,8 @@ class LlamaTransformerLayer:
             attn_out = linear(input_embds, w.o_proj, self.skinny)
             fused_add_rmsnorm_inplace(attn_out, residual_buf, w.ffn_norm, cfg.rms_norm_eps)
         act = linear_silu_gate(attn_out, w.up_gate_proj) if self.skinny else None
+        if act is None and self.skinny:
+            act = linear_gated(attn_out, w.up_gate_proj, TILE_SILU_ROUNDED)
         if act is None:
             up_gate = linear(attn_out, w.up_gate_proj, self.skinny)
             silu_and_mul_inplace(up_gate)

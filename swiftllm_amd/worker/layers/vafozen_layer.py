@@ -4,8 +4,8 @@ next input's norm are the model's fused step (kernels/hyper_stream.py)."""
 import torch
 
 from ..kernels.linear_scan import DECAY_EXP_EXP, DECAY_SIGMOID_POWER, linear_recurrence, low_rank_decay
-from ..kernels.linear import linear_grouped
-from ..kernels.moe import gated_rows
+from ..kernels.linear import linear_gated, linear_grouped
+from ..kernels.moe import ACT_SILU, gated_rows
 from ..kernels.rms_stream import token_shift_mix
 from ..kernels.rope_kv import qkv_conv_rope_and_store_kv
 from ..kernels.ssd import state_space_mixer
@@ -107,12 +107,14 @@ class VafozenLayer:
     def forward(self, h: torch.Tensor, ctx: StepContext):
         """-> the layer's result, rows or SplitKPartials."""
         w = self.w
-        proj = _project(h, w.proj, self.skinny)
         make = torch.zeros if w.row_gaps else torch.empty       # (columns of no piece meet zero weights: they must be finite)
         row = make((h.shape[0], w.row_size), dtype=h.dtype, device=h.device)
+        # prompt-sized steps: the feed-forward's unit in a product of its own
+        gated = w.proj_ff is not None and self.skinny and linear_gated(h, w.proj_ff, ACT_SILU, out=row[:, w.ins["ff"]]) is not None
+        proj = _project(h, w.proj_mixer if gated else w.proj, self.skinny)
         if self.left is not None:
             self.left.forward(proj, row, ctx)
         self.right.forward(h, proj, row, ctx, self.skinny)
-        if self.mlp is not None:
+        if self.mlp is not None and not gated:
             gated_rows(row[:, w.ins["ff"]], proj[:, w.cols["ff_gate"]], proj[:, w.cols["ff_up"]])
         return _project_partials(row, w.out, self.skinny)

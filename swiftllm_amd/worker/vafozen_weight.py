@@ -134,6 +134,11 @@ class VafozenLayerWeight:
             outs.add("ff", mat("mlp.down", (w, ff)))
         self.proj, self.out = ins.cat(32), outs.cat()
         self.cols, self.ins = ins.at, outs.at
+        # the rows of `proj` in front of the feed-forward's and those, for steps that take them in two products
+        self.proj_mixer = self.proj_ff = None
+        if lcfg.mlp is not None and self.cols["ff_up"].start == self.cols["ff_gate"].stop:
+            at = self.cols["ff_gate"].start
+            self.proj_mixer, self.proj_ff = self.proj[:at], self.proj[at:self.cols["ff_up"].stop]
         self.row_size, self.row_gaps = outs.size, outs.has_gaps
 
 
