@@ -73,7 +73,7 @@ MODEL_SOURCES = {
     "Vafozen": _SHARED + ["layernorm.hip", "window_attn.hip", "window_attn_mfma.hip", "span_attn.hip", "moe.hip", "moe_grouped.hip", "rms_stream.hip", "rope_kv.hip",
                           "hyper_stream.hip", "delta_rule.hip", "ssd.hip", "linear_scan.hip", "low_rank_decay.hip"],
 }
-HEADERS = ["swl_common.h", "attend_block.h", "attn_combine.h", "token_attn.h", "conv_tail.h", "row_wide.h", "tile_product.h", os.path.join(ROOT, "include", "swiftllm_hip.h")]
+HEADERS = ["swl_common.h", "attend_block.h", "attn_combine.h", "token_attn.h", "conv_tail.h", "row_wide.h", "tile_product.h", "gemm_tile.h", os.path.join(ROOT, "include", "swiftllm_hip.h")]
 LIB = os.path.join(HERE, "libswiftllm_hip.so")
 OBJ_DIR = os.path.join(HERE, "build")
 ARCH = "gfx950"

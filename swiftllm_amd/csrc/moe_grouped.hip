@@ -1,18 +1,18 @@
 // moe_grouped.hip — the expert products of prompt-sized steps: assignments sorted by expert on the device, then ONE matrix-core
 // launch per product for all experts (16-bit storage, fp32 accumulation).
 //
-// What bounds it: what a CU takes from L2 (a tile of 128 x 128 asks for 32 KiB per 64 columns of the reduction: 52 of 70 us when nothing
-// else is done, 8192 rows, width and ff 2048) next to the matrix cores (43 us), and what of the two does not overlap. A library product per
-// expert leaves most of the chip idle at these sizes (2048 x 1024 x 1024: 128 tiles for 256 CUs) and needs the experts' row counts on the
-// host: a read-back and the launches' gaps behind it in every layer. Here a tile of 128 assignments of one expert x 128 weight rows is a
-// workgroup of four waves, each a 64 x 64 piece (mfma 32x32x16, 2 x 2 accumulators); operands are staged by LDS-DMA in 64-deep slices of
-// whole 128-byte lines (half lines take 1.4 times as long), with the swizzle that keeps the 16-byte fragment reads off each other's banks on
-// the source side. Token rows are gathered by the staging itself (no sorted copy of the inputs), the gated unit or the squared ReLU runs
-// on the fp32 products in the epilogue, and results leave as whole lines through LDS.
-// Measured (bf16), two staged slices and column tiles fastest -> now: 9000 assignments over 8 experts, width and ff 2048: gate/up with the
-// unit 223 -> 159 us (950 TFLOP/s), down 101 -> 85; 16000 assignments, width and ff 1024: 98 -> 82, 54 -> 45; 1562, width and ff 2048:
-// 61 -> 37, 30 -> 26. Tiles of 256 x 256 or 128 x 256 with rings of up to five slices: 225 and 172 us at the first size (the chip's last
-// turn is half empty, and first slices and results wait alone), 150 and 100 at the second; faster only where the tiles fill whole turns.
+// A library product per expert leaves most of the chip idle at these sizes (2048 x 1024 x 1024: 128 tiles for 256 CUs) and needs the experts' row
+// counts on the host: a read-back and the launches' gaps behind it in every layer. Here the tiles of all experts are one list. Token rows are
+// gathered by the staging itself (no sorted copy of the inputs), the gated unit or the squared ReLU runs on the fp32 products in the
+// epilogue, and results leave as whole lines through LDS.
+//   * Reductions of whole steps of 128 columns, up to 512 experts: the tiles of gemm_tile.h, which says what bounds them. Every workgroup counts the
+//     experts' tiles from the sorted assignments; a tile's assignments come to LDS while the tile before it is multiplied.
+//   * Others: a tile of 128 assignments of one expert x 128 weight rows a workgroup of four waves, each a 64 x 64 piece (mfma 32x32x16, 2 x 2
+//     accumulators), operands in 64-deep slices (tile_product.h). Bound by what a CU takes from L2 (32 KiB per 64 columns) beside the matrix steps.
+// Measured (us, bf16, by the second / by the first, gate/up with the unit, then down): 9000 assignments over 8 experts, width and ff 2048: 193 / 165, 89 / 73;
+// 7314: 147 / 113, 69 / 54; 15252, width and ff 1024: 75 / 60, 37 / 31; 1400, 2048: 40 / 33, 26 / 19; 200: 32 / 24, 22 / 16; 64000 over 64, width 2048, ff 1024: 637 /
+// 475, 320 / 255. Passes of 3 x 1500, 11 x 333 and 4 x 2000 tokens with experts in two of four layers or in all: 1.05, 1.04, 1.06.
+#include "gemm_tile.h"
 #include "tile_product.h"
 
 namespace swl {
@@ -248,6 +248,18 @@ __global__ __launch_bounds__(256, BUFS == 1 ? 4 : 2) void moe_gemm_kernel(MoeGem
     }
 }
 
+// Tiles of 256 x 256, 256 x 128 or 128 x 128: as gemm_tile_shape has it, an expert's last tile taken as half full (us by each, 9000 assignments,
+// 2048: 163, 167, 169; 7314 110, 127, 135; 1400 47, 33, 36; 600 of 1024 26, 17, 11; 12000 over 128 experts, ff 768 185, 207, 168).
+template <typename T, int ACT, int ROWS>
+int moe_gemm_dispatch(const GemmTileParams &p, int64_t w_rows, hipStream_t s) {
+    auto tiles = [&](int rows, int cols) { return (p.M / rows + (min(p.experts, p.M) + 1) / 2) * ((w_rows + cols - 1) / cols); };
+    switch (gemm_tile_shape(tiles, p.K, true)) {
+    case 1: return gemm_tile_launch<T, 16, 4, 4, 4, 4, 1, ACT, ROWS>(p, s);
+    case 6: return gemm_tile_launch<T, 16, 4, 4, 2, 2, 1, ACT, ROWS>(p, s);
+    default: return gemm_tile_launch<T, 16, 2, 2, 2, 2, 1, ACT, ROWS>(p, s);
+    }
+}
+
 } // namespace swl
 
 extern "C" int swl_moe_sort(int32_t *order, int64_t *where, int32_t *offsets, const int32_t *expert_idx, int64_t num_assignments,
@@ -280,6 +292,22 @@ extern "C" int swl_moe_gemm(void *out, const void *x, const void *w, const int32
     // (rows of x: assignments when sorted, else tokens)
     if (order ? x_rows * top < num_assignments : x_rows < num_assignments) return SWL_ERR_BAD_ARG;
     if (!out || !x || !w || !offsets || !swl::aligned16(out) || !swl::aligned16(x) || !swl::aligned16(w)) return SWL_ERR_BAD_ARG;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (K >= 256 && K % 128 == 0 && experts <= swl::kTileExperts && num_assignments <= (1 << 29) && 256LL * K * 2 < (1LL << 31) && 512LL * N < (1LL << 31)) {
+        swl::GemmTileParams p = {};
+        p.out = out; p.x = x; p.w = w; p.M = static_cast<int>(num_assignments); p.N = N; p.K = K; p.ldx = K; p.ldo = N; p.limit = limit;
+        p.order = order; p.offsets = offsets; p.in_w = in_w; p.experts = experts; p.top = swl::Divisor::of(static_cast<unsigned>(top));
+        p.x_bytes = static_cast<unsigned>(x_rows * K * 2); p.in_w_bytes = static_cast<unsigned>(num_assignments * 4);
+        const int64_t w_rows = mode == 1 ? 2LL * N : N;
+        SWL_DISPATCH_DTYPE(dtype, T, {
+            if (order) {
+                if (mode == 0) return swl::moe_gemm_dispatch<T, 0, swl::kTileGather>(p, w_rows, s);
+                if (mode == 2) return swl::moe_gemm_dispatch<T, 1, swl::kTileGather>(p, w_rows, s);
+                return act == 0 ? swl::moe_gemm_dispatch<T, 2, swl::kTileGather>(p, w_rows, s) : swl::moe_gemm_dispatch<T, 3, swl::kTileGather>(p, w_rows, s);
+            }
+            if (mode == 0) return swl::moe_gemm_dispatch<T, 0, swl::kTileExpert>(p, w_rows, s);
+        });
+    }
     swl::MoeGemmParams p;
     p.out = out; p.x = x; p.w = w; p.order = order; p.offsets = offsets; p.in_w = in_w;
     p.top = top; p.experts = experts; p.K = K; p.N = N; p.act = act; p.limit = limit;
@@ -289,7 +317,6 @@ extern "C" int swl_moe_gemm(void *out, const void *x, const void *w, const int32
     const int64_t m_tiles = (num_assignments + swl::kTile - 1) / swl::kTile + (experts < num_assignments ? experts : num_assignments);
     const int64_t grid = (m_tiles * p.n_tiles + 7) / 8 * 8;
     if (grid > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
-    hipStream_t s = static_cast<hipStream_t>(stream);
     // One staged slice and four workgroups a CU where there are more tiles than two a CU (about: an expert's last row tile half full),
     // else two slices: 31.3 and 35.7 us at 688 tiles (4950 rows, width and ff 1024, gate/up), 39.1 and 36.6 at 512, 20.7 and 19.3 at 344.
     const bool many = (num_assignments + 64LL * experts) / swl::kTile * p.n_tiles > 512;

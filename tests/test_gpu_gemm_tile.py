@@ -122,3 +122,60 @@ def test_replayed_from_a_graph_beside_other_launches():
         graph.replay()
         assert torch.equal(got, want)
         (x.float() @ w.float().T).sum().item()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,top,experts,K,N", [
+    (700, 2, 8, 256, 136),          # tiles of 128 x 128, a column tile of 8, experts that end anywhere in a tile
+    (300, 1, 70, 384, 264),         # more experts than lanes, most of them a few rows
+    (40, 3, 130, 512, 72),          # more experts than rows, no assignments for some
+    (4000, 2, 5, 256, 2048),        # several tiles a workgroup
+    (6000, 2, 3, 1024, 1024),       # tiles of 256 x 128 and 256 x 256
+    (9000, 2, 8, 512, 4096)])
+def test_products_of_experts(n, top, experts, K, N, dtype):
+    """Rows gathered through the sorted assignments (weights on the products or none), and rows by position, against products in 64 bits."""
+    from swiftllm_amd import _hip
+    g = torch.Generator(device="cuda").manual_seed(n + K)
+    total = n * top
+    idx = (torch.rand((n, top), generator=g, device="cuda") ** 2 * experts).int().clamp(max=experts - 1)      # (some experts take most)
+    idx[idx == 1] = 0
+    order, where = torch.empty(total, dtype=torch.int32, device="cuda"), torch.empty(total, dtype=torch.int64, device="cuda")
+    offsets = torch.empty(experts + 1, dtype=torch.int32, device="cuda")
+    _hip.call("swl_moe_sort", _hip.ptr(order), _hip.ptr(where), _hip.ptr(offsets), _hip.ptr(idx), total, experts, _hip.stream())
+    x = torch.randn((n, K), generator=g, device="cuda").to(dtype)
+    w = (torch.randn((experts, 2 * N, K), generator=g, device="cuda") / K ** 0.5).to(dtype)
+    in_w = torch.rand(total, generator=g, device="cuda") + 0.5
+    ulp, floor = (2.0 ** -10, 2.0 ** -24) if dtype == torch.float16 else (2.0 ** -7, 0.0)
+    flat, bounds = order.long(), offsets.tolist()
+    z = torch.empty((total, 2 * N), dtype=torch.float64, device="cuda")
+    size = torch.empty_like(z)
+    xs = x[flat // top].double()
+    for e in range(experts):
+        a, b = bounds[e], bounds[e + 1]
+        z[a:b], size[a:b] = xs[a:b] @ w[e].double().T, xs[a:b].abs() @ w[e].double().abs().T
+    off = 2.0 ** -24 * K * size        # (fp32 sums in any order)
+    limit = 0.7
+    for mode, act, weigh, ordered in ((0, 0, False, True), (1, 0, True, True), (1, 1, True, True), (1, 1, False, True), (2, 0, False, True), (0, 0, False, False)):
+        cols = 2 * N if mode == 1 else N
+        ww = w if mode == 1 else w[:, :N].contiguous()
+        rows = x if ordered else xs.to(dtype)
+        out = torch.full((total + 1, N), 7.0, dtype=dtype, device="cuda")
+        _hip.call("swl_moe_gemm", _hip.ptr(out), _hip.ptr(rows), _hip.ptr(ww), _hip.ptr(order) if ordered else 0, _hip.ptr(offsets),
+                  _hip.ptr(in_w) if weigh else 0, total, rows.shape[0], top, experts, K, N, mode, act, limit, _hip.dtype_code(dtype), _hip.stream())
+        torch.cuda.synchronize()
+        scale = in_w[flat].double()[:, None] if weigh else 1.0
+        p, d = z[:, :cols] * scale, off[:, :cols] * scale
+        if mode == 1:
+            f, s, df, ds = p[:, :N], p[:, N:], d[:, :N], d[:, N:]
+            if act == 0:
+                f, s = f.clamp(max=limit), s.clamp(-limit, limit)
+                want, slack = f * torch.sigmoid(1.702 * f) * (s + 1), 1.2 * df * (s.abs() + 1) + ds * f.abs()
+            else:
+                want, slack = torch.nn.functional.silu(f) * s, 1.1 * df * s.abs() + ds * f.abs()
+            slack = slack + df * ds + 2.0 ** -20 * want.abs()      # (the unit's own fp32 roundings)
+        elif mode == 2:
+            want, slack = torch.relu(p) ** 2, (2 * p.abs() + d) * d
+        else:
+            want, slack = p, d
+        assert bool(((out[:total].double() - want).abs() <= slack + ulp * want.abs() + floor).all()), (mode, act, weigh, ordered)
+        assert bool((out[total] == 7).all())
