@@ -776,7 +776,7 @@ int swl_moe_down_combine(void *out, const void *y, const void *down, const int32
  * the first act_cols columns (a multiple of four); 2 + a: w holds [N first | N second] rows and out their gated unit: a = 0 min(f, limit)
  * sigmoid(1.702 f) (clamp(s, +-limit) + 1), 1 silu(f) s, 2 silu(s) f, 3 round(silu(s)) f; all of the rounded products. x_cols (0: one matrix x;
  * a multiple of 256, acts 0 and 1): columns x_cols g .. of out are products of the matrix x_next * g elements behind x. shape 0: the
- * kernel's own choice of tile, 1 .. 6: that one. K a multiple of 128, at least 256; row strides multiples of 8, out rows with room for N rounded up
+ * kernel's own choice of tile, 1 .. 11: that one (acts: not 7 .. 9; x_cols: those whose columns divide it). K a multiple of 128, at least 256; row strides multiples of 8, out rows with room for N rounded up
  * to a multiple of 8 (columns from N on hold zeros' products); pointers on 16 bytes. */
 int swl_gemm_tile_supported(int64_t M, int32_t N, int32_t K, int64_t ldx, int64_t ldo, int32_t act, int32_t dtype);
 int swl_gemm_tile(void *out, const void *x, const void *w, int64_t M, int32_t N, int32_t K, int64_t ldx, int64_t ldo, int32_t x_cols,

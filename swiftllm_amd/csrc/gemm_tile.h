@@ -4,7 +4,7 @@
 // What bounds it: large products run the card at its power limit (8192^3 at 1.75 GHz: 1426 TFLOP/s, the library's 1338 on the same card),
 // whatever the tile; small ones wait for their first columns (5000 cycles from a cold start) and for their results to leave (128 KiB a CU at
 // the 32 bytes a cycle that an XCD's L2 takes of each of its CUs), and leave CUs idle in their last turn. So: one workgroup a CU that
-// takes tile after tile (two of 128 x 128 and less), the next tile's first columns asked for while one ends, and tiles of six sizes of
+// takes tile after tile (two of 128 x 128 and less), the next tile's first columns asked for while one ends, and tiles of eleven sizes of
 // which a model of turns and steps picks (gemm_tile_shape).
 //   * Four waves tile the result two by two. A step of 64 columns is four parts, the halves of the waves' rows of x and of w, four phases
 //     multiply half by half, in the order X0 W0, X0 W1, X1 W1, X1 W0 and then X0 W1, X0 W0, X1 W0, X1 W1: every phase needs one part
@@ -14,10 +14,11 @@
 //   * Fetches go through buffer descriptors of the tile's own rows: rows beyond the matrix are zeros without a memory access.
 //   * Results leave as whole lines through 4 KiB of LDS a wave, without a barrier, as stores that nobody waits for.
 // Measured (us, bf16, operands from a pool of 1.5 GB; in brackets the library, in one call and in the blocks of rows that it was called with
-// before): 7691 tokens: 1024 x 1024 19.0 (20.7, 27.1), 8192 x 1024 119 (130, 122), 1024 x 4096 60.5 (68, 87), 2576 x 1024 45 (60, 67); 4498: 2048 x 2048 37
-// (39, 48), 8192 x 2048 124 (147, 132), 3072 x 2048 54 (53, 62); 2029: 5696 x 1024 25 (35), 1024 x 1024 8.3 (11.1); 1828: 28672 x 4096 370 with its gated unit (342 to
-// 432 by card, and 32 for the unit); 5112: 6144 x 4096 191 to 209 (222, 238), 4096 x 4096 149 (155, 140). 340 products of 260 to 8192 tokens: 0.88 of the
-// library's time. From 16384 tokens on the library's rate is 5 % to 10 % higher (1.55 PFLOP/s).
+// before): 7691 tokens: 1024 x 1024 17.3 (20.7, 27.1), 8192 x 1024 106 (104, 104), 1024 x 4096 55 (62, 74), 2576 x 1024 40 (60, 63); 4498: 2048 x 2048 33
+// (38, 45), 2048 x 8192 117 (131, 141), 8192 x 2048 112 (125, 118), 3072 x 2048 45 (47, 59); 3657: 2048 x 8192 97 (105), 7440 x 2048 87 (104); 2029: 5696 x 1024 22
+// (34), 1024 x 1024 8.6 (11); 1828: 28672 x 4096 336 with its gated unit (342 to 430 by card, and 32 for the unit), 4096 x 14336 177 (185); 5112: 6144 x
+// 4096 182 (180, 207), 4096 x 4096 128 (135, 128). 270 products of 260 to 8192 tokens: 0.8 of the library's time where its calls are in blocks. From
+// 16384 tokens on the library's rate is 5 % to 10 % higher (1.55 PFLOP/s).
 #pragma once
 
 #include "swl_common.h"
@@ -473,26 +474,39 @@ int gemm_tile_launch(GemmTileParams p, hipStream_t s) {
     return check_launch();
 }
 
-// Which tile: the one whose time a model of turns and steps has as the least: us = start + steps of 128 columns x turns x a + turns x b + steps x
-// tiles / 256 x c (turns of whole and of half filled CUs apart where two tiles share one), fitted to 340 products (260 to 8192 tokens, 1024 to 28672
-// rows of w, 1024 to 14336 columns; bf16): 3 % to 8 % off, and the tile that it picks takes 1.002 times the best one's time. tiles(rows, rows of w): how many. experts:
-// of the three that the experts' products have.
+// The tiles that there are: rows and rows of w in 32s. The last two share a CU, the others take one each.
+struct TileShape {
+    int x, w;
+};
+constexpr TileShape kTileShapes[] = {{8, 8}, {6, 8}, {6, 6}, {5, 8}, {7, 8}, {8, 6}, {5, 4}, {5, 6}, {7, 6}, {4, 4}, {2, 4}};
+constexpr int kTileShapeCount = 11;
+constexpr unsigned kTilesPlain = 0x7ff, kTilesAct = 0x63f;      // with an activation: not 160 x 128, 160 x 192 and 224 x 192
+
+// Which tile of the set: the one whose time a model of turns and steps has as the least, us = 1.86 + turns (steps of 128 columns (0.0134 x w + 0.0667 (x +
+// w)) + 0.0666 x w) + 0.0123 x w steps tiles / 256, for two tiles a CU by turns of whole and of half filled CUs: fitted to 270 products (260 to 8192
+// tokens, 1024 to 28672 rows of w, 1024 to 14336 columns; bf16), 4 % to 8 % off; what it picks takes 1.004 times the best one's time.
+// tiles(rows, rows of w): how many. (Six tiles instead of eleven: 1.05 of the time, 1.08 to 1.14 for 1828 of 28672 x 4096, 4498 of 2048 x 2048, 3657 of
+// 2048 x 8192, 5112 of 4096 x 4096.)
 template <typename Tiles>
-int gemm_tile_shape(Tiles &&tiles, int64_t k, bool experts = false) {
+int gemm_tile_shape(Tiles &&tiles, int64_t k, unsigned set) {
     const double p = static_cast<double>(k) / 128;
-    auto one = [&](int bm, int bw, double start, double a, double b, double c) {
-        const int64_t t = tiles(bm, bw), turns = ((t + 7) / 8 + 31) / 32;
-        return start + turns * (p * a + b) + p * t / 256 * c;
+    auto one = [&](const TileShape &s) {
+        const int64_t t = tiles(32 * s.x, 32 * s.w), turns = ((t + 7) / 8 + 31) / 32;
+        const double area = s.x * s.w;
+        return 1.86 + turns * (p * (0.0134 * area + 0.0667 * (s.x + s.w)) + 0.0666 * area) + 0.0123 * area * p * t / 256;
     };
-    auto two = [&](int bm, int bw, double start, double a, double b, double half, double c) {
-        const int64_t t = tiles(bm, bw), each = (t + 7) / 8, rest = each % 64, full = each / 64 + (rest > 32), part = rest > 0 && rest <= 32;
+    auto two = [&](const TileShape &s, double start, double a, double b, double half, double c) {
+        const int64_t t = tiles(32 * s.x, 32 * s.w), each = (t + 7) / 8, rest = each % 64, full = each / 64 + (rest > 32), part = rest > 0 && rest <= 32;
         return start + full * p * a + (full + part) * b + part * p * half + p * t / 256 * c;
     };
-    const double us[6] = {one(256, 256, 2.14, 1.95, 4.57, 1.06), one(192, 256, 1.86, 1.37, 3.20, 0.99), one(192, 128, 1.63, 0.85, 1.34, 0.56),
-                          two(128, 128, 1.86, 1.20, 0.78, 0.64, 0.38), two(64, 128, 2.38, 0.86, 0.0, 0.54, 0.21), one(256, 128, 2.35, 1.14, 2.03, 0.56)};
-    int best = 0;
-    for (int i = 1; i < 6; ++i)
-        if (us[i] < us[best] && !(experts && (i == 1 || i == 2 || i == 4))) best = i;
+    int best = -1;
+    double least = 0;
+    for (int i = 0; i < kTileShapeCount; ++i) {
+        if (!(set >> i & 1)) continue;
+        const TileShape &s = kTileShapes[i];
+        const double us = i == 9 ? two(s, 1.81, 1.03, 0.78, 0.63, 0.42) : i == 10 ? two(s, 2.29, 0.85, 0.0, 0.55, 0.20) : one(s);
+        if (best < 0 || us < least) best = i, least = us;
+    }
     return best + 1;
 }
 

@@ -248,14 +248,16 @@ __global__ __launch_bounds__(256, BUFS == 1 ? 4 : 2) void moe_gemm_kernel(MoeGem
     }
 }
 
-// Tiles of 256 x 256, 256 x 128 or 128 x 128: as gemm_tile_shape has it, an expert's last tile taken as half full (us by each, 9000 assignments,
-// 2048: 163, 167, 169; 7314 110, 127, 135; 1400 47, 33, 36; 600 of 1024 26, 17, 11; 12000 over 128 experts, ff 768 185, 207, 168).
+// An expert's last row tile is taken as half full.
+constexpr unsigned kTilesExperts = 1u << 0 | 1u << 1 | 1u << 2 | 1u << 5 | 1u << 9;
 template <typename T, int ACT, int ROWS>
 int moe_gemm_dispatch(const GemmTileParams &p, int64_t w_rows, hipStream_t s) {
     auto tiles = [&](int rows, int cols) { return (p.M / rows + (min(p.experts, p.M) + 1) / 2) * ((w_rows + cols - 1) / cols); };
-    switch (gemm_tile_shape(tiles, p.K, true)) {
+    switch (gemm_tile_shape(tiles, p.K, kTilesExperts)) {
     case 1: return gemm_tile_launch<T, 16, 4, 4, 4, 4, 1, ACT, ROWS>(p, s);
-    case 6: return gemm_tile_launch<T, 16, 4, 4, 2, 2, 1, ACT, ROWS>(p, s);
+    case 2: return gemm_tile_launch<T, 16, 3, 3, 4, 4, 1, ACT, ROWS>(p, s);
+    case 3: return gemm_tile_launch<T, 16, 3, 3, 3, 3, 1, ACT, ROWS>(p, s);
+    case 6: return gemm_tile_launch<T, 16, 4, 4, 3, 3, 1, ACT, ROWS>(p, s);
     default: return gemm_tile_launch<T, 16, 2, 2, 2, 2, 1, ACT, ROWS>(p, s);
     }
 }

@@ -32,7 +32,7 @@ SIZES = [(1, 8, 256), (257, 136, 384), (300, 1032, 256), (129, 264, 640), (65, 1
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("shape", [0, 1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("shape", range(12))
 @pytest.mark.parametrize("m,n,k", SIZES + [(4500, 4352, 256)])
 def test_products_are_rounded_once(m, n, k, shape, dtype):
     x, w = _operands(m, n, k, dtype)
@@ -44,7 +44,7 @@ def test_products_are_rounded_once(m, n, k, shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("shape", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("shape", [1, 2, 3, 4, 5, 6, 10, 11])
 @pytest.mark.parametrize("m,n,k", SIZES)
 def test_gated_units_and_squared_relu(m, n, k, shape, dtype):
     """A unit f(a, b) of two rounded products that may be an ulp off each: |df/da| |a| + |df/db| |b| ulps, and an ulp of the result (two where it is
@@ -75,10 +75,10 @@ def test_gated_units_and_squared_relu(m, n, k, shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("shape", [0, 1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("shape", range(12))
 def test_columns_of_several_matrices(shape, dtype):
     from swiftllm_amd.worker.kernels.linear import linear_grouped
-    m, groups, size, k = 333, 3, 512, 384
+    m, groups, size, k = 333, 3, 768 if shape in (3, 6, 8, 9) else 512, 384      # (those are 192 columns wide)
     g = torch.Generator(device="cuda").manual_seed(5)
     x = torch.randn((groups, m, k), generator=g, device="cuda").to(dtype)
     w = (torch.randn((groups * size, k), generator=g, device="cuda") / k ** 0.5).to(dtype)
