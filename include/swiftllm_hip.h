@@ -776,11 +776,17 @@ int swl_moe_down_combine(void *out, const void *y, const void *down, const int32
  * the first act_cols columns (a multiple of four); 2 + a: w holds [N first | N second] rows and out their gated unit: a = 0 min(f, limit)
  * sigmoid(1.702 f) (clamp(s, +-limit) + 1), 1 silu(f) s, 2 silu(s) f, 3 round(silu(s)) f; all of the rounded products. x_cols (0: one matrix x;
  * a multiple of 256, acts 0 and 1): columns x_cols g .. of out are products of the matrix x_next * g elements behind x. shape 0: the
- * kernel's own choice of tile, 1 .. 11: that one (acts: not 7 .. 9; x_cols: those whose columns divide it). K a multiple of 128, at least 256; row strides multiples of 8, out rows with room for N rounded up
- * to a multiple of 8 (columns from N on hold zeros' products); pointers on 16 bytes. */
+ * kernel's own choice of tile, 1 .. 11: that one (acts: not 7 .. 9; x_cols: those whose columns divide it). K a multiple of 128, at least 256;
+ * row strides multiples of 8, out rows with room for N rounded up to a multiple of 8 (columns from N on hold zeros' products); pointers on 16
+ * bytes.
+ * swl_gemm_tile_partial: slabs[splits][M][N] fp32, the sums over equal shares of K (multiples of 128 columns, at least 256; N a multiple of 8), for
+ * consumers that add them up; swl_gemm_tile_choose_splits: how many shares pay for these sizes (1: none). */
 int swl_gemm_tile_supported(int64_t M, int32_t N, int32_t K, int64_t ldx, int64_t ldo, int32_t act, int32_t dtype);
 int swl_gemm_tile(void *out, const void *x, const void *w, int64_t M, int32_t N, int32_t K, int64_t ldx, int64_t ldo, int32_t x_cols,
                   int64_t x_next, int32_t act, int32_t act_cols, float limit, int32_t shape, int32_t dtype, swl_stream_t stream);
+int swl_gemm_tile_choose_splits(int64_t M, int32_t N, int32_t K);
+int swl_gemm_tile_partial(float *slabs, size_t slabs_bytes, const void *x, const void *w, int64_t M, int32_t N, int32_t K, int64_t ldx,
+                          int32_t splits, int32_t shape, int32_t dtype, swl_stream_t stream);
 
 /* The expert products of prompt-sized steps, 16-bit, on the matrix core. swl_moe_sort: assignments (expert_idx[n], ids clamped into
  * range) sorted stably by expert: order[pos] = assignment, where[assignment] = pos, offsets[experts + 1] = first position of every

@@ -143,6 +143,7 @@ SIGNATURES = {
     "swl_glu_clamp": [_P, _P, _P, _I64, _I32, _F32, _I32, _I32, _P],
     "swl_moe_sort": [_P, _P, _P, _P, _I64, _I32, _P],
     "swl_gemm_tile": [_P, _P, _P, _I64, _I32, _I32, _I64, _I64, _I32, _I64, _I32, _I32, _F32, _I32, _I32, _P],
+    "swl_gemm_tile_partial": [_P, ctypes.c_size_t, _P, _P, _I64, _I32, _I32, _I64, _I32, _I32, _I32, _P],
     "swl_moe_gemm": [_P, _P, _P, _P, _P, _P, _I64, _I64, _I32, _I32, _I32, _I32, _I32, _I32, _F32, _I32, _P],
     "swl_moe_combine": [_P, _P, _P, _P, _I64, _I32, _I32, _I32, _P],
     "swl_moe_down_combine": [_P, _P, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _P],
@@ -217,6 +218,7 @@ _SPECIAL = {
     "swl_window_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_masked_attn_tiles_supported": ([_I32, _I32, _I32, _I32, _I32, _I32], _I32),
     "swl_gemm_tile_supported": ([_I64, _I32, _I32, _I64, _I64, _I32, _I32], _I32),
+    "swl_gemm_tile_choose_splits": ([_I64, _I32, _I32], _I32),
     "swl_moe_gemm_supported": ([_I64, _I32, _I32, _I32], _I32),
     "swl_latent_fold_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),
     "swl_latent_decode_supported": ([_I32, _I32, _I32, _I32, _I32], _I32),

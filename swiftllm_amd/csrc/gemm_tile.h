@@ -96,24 +96,28 @@ struct GemmTileParams {
     Divisor top;
     unsigned x_bytes, in_w_bytes;
     Divisor group, wide, rest;      // tiles of a group, row tiles of one, of the last one
+    int splits;             // shares of K, each with an fp32 slab of out (one behind the other) of its own
+    Divisor share;          // tiles of a row of tiles in one of them
     float limit;
 };
 
 constexpr int kTileGroup = 8;       // row tiles that an XCD takes with all their column tiles
 constexpr int kTileExperts = 512;   // at most
+constexpr int kTileSlabs = -1;      // (for ACT)
 enum TileRows { kTileDense = 0, kTileExpert = 1, kTileGather = 2 };     // rows of x: all alike, an expert's a tile, and gathered through `order`
 
-// ACT 0: the product; 1: relu(.)^2 of the first act_cols columns; 2 + a: w rows [N first | N second], out = a gated unit of the two (a = 0 .. 2:
+// ACT kTileSlabs: fp32 sums over shares of K; 0: the product; 1: relu(.)^2 of the first act_cols columns; 2 + a: w rows [N first | N second], out = a gated unit of the two (a = 0 .. 2:
 // gated_unit, 3: round(silu(second)) first, rounded). Activations are of the rounded products.
 template <typename T, int U, int X0, int X1, int W0, int W1, int PAIRS, int ACT, int ROWS = kTileDense>
 __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS == 1 ? 2 : 1) void gemm_tile_kernel(GemmTileParams p) {
     constexpr int X = X0 + X1, W = W0 + W1, E = U == 32 ? 4 : 2;        // blocks of U rows a wave; matrix steps of 64 columns
-    constexpr bool GATED = ACT >= 2;
+    constexpr bool GATED = ACT >= 2, SLABS = ACT == kTileSlabs;
     constexpr int xn[2] = {X0, X1}, wn_[2] = {W0, W1};
     constexpr int BLOCK = 2 * U * 128, ASKS = U / 16;       // bytes of a block of both waves in LDS, fetches of a wave for it
     constexpr int STEP = (X + W) * BLOCK, PAIR = 2 * STEP;
     constexpr int BM = 2 * U * X, OUTW = GATED ? U * W0 : U * W, BN = 2 * OUTW;     // rows, columns of a wave, of the tile
-    constexpr int CB = 64 / U, PITCH = 128;     // blocks of columns that leave at once; a row of theirs in LDS
+    constexpr int SIZE = SLABS ? 4 : 2;         // bytes of a result
+    constexpr int CB = 128 / SIZE / U, PITCH = 128;     // blocks of columns that leave at once; a row of theirs in LDS
     constexpr bool ACC = U * U * X * W > 4096;
     using acc_t = std::conditional_t<U == 32, float16_t, float4_t>;
     static_assert(!GATED || W0 == W1, "");
@@ -155,10 +159,10 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
     int at = static_cast<int>(xcd * all / 8) + (blockIdx.x >> 3);
     if (at >= last) return;
     const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem));
-    const int64_t xb = p.ldx * 2, wb = static_cast<int64_t>(p.K) * 2, ob = p.ldo * 2;
-    const int steps = p.K / 64;
+    const int64_t xb = p.ldx * 2, wb = static_cast<int64_t>(p.K) * 2, ob = p.ldo * SIZE;
+    const int steps = p.K / 64 / (SLABS ? p.splits : 1);
     struct Place {
-        int row0, rows, col0, expert;
+        int row0, rows, col0, expert;       // (of slabs: the share of K in the expert's place)
     };
     auto place = [&](int t) {
         const unsigned group = divide(t, p.group), in_group = t - group * p.group.by;
@@ -182,23 +186,25 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
             to.rows = min(BM, hi - to.row0);
         } else {
             const Divisor wide = (group + 1) * p.wide.by > static_cast<unsigned>(p.m_tiles) ? p.rest : p.wide;
-            const unsigned n = divide(in_group, wide);
+            const unsigned n = divide(in_group, wide), share = SLABS ? divide(n, p.share) : 0;
             to.row0 = (group * p.wide.by + in_group - n * wide.by) * BM;
             to.rows = min(BM, p.M - to.row0);
-            to.col0 = n * BN;
-            to.expert = 0;
+            to.col0 = (SLABS ? n - share * p.share.by : n) * BN;
+            to.expert = share;
         }
         return to;
     };
     auto x_rsrc = [&](const Place &to) {
         if constexpr (GATHER) return tile_rsrc(static_cast<const char *>(p.x), p.x_bytes);
         const char *x = static_cast<const char *>(p.x) + (!EXPERT && p.x_cols ? to.col0 / p.x_cols * p.x_next : 0);
-        return tile_rsrc(x + to.row0 * xb, static_cast<unsigned>(to.rows * xb));
+        const int k0 = SLABS ? to.expert * steps * 128 : 0;
+        return tile_rsrc(x + to.row0 * xb + k0, static_cast<unsigned>(to.rows * xb - k0));
     };
     auto w_rsrc = [&](const Place &to) {
         const int64_t left = (GATED ? 2LL * p.N : static_cast<int64_t>(p.N)) - to.col0;
         const char *w = static_cast<const char *>(p.w) + (EXPERT ? static_cast<int64_t>(to.expert) * (GATED ? 2 : 1) * p.N * wb : 0);
-        return tile_rsrc(w + to.col0 * wb, static_cast<unsigned>((GATED ? left : min(static_cast<int64_t>(BN), left)) * wb));
+        const int k0 = SLABS ? to.expert * steps * 128 : 0;
+        return tile_rsrc(w + to.col0 * wb + k0, static_cast<unsigned>((GATED ? left : min(static_cast<int64_t>(BN), left)) * wb - k0));
     };
 
     // ---- staging: a step of 64 columns is four parts, the halves of the waves' rows of x and of w. A fetch is eight rows of 128 bytes, a
@@ -270,7 +276,7 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
     };
     constexpr int OW = GATED ? W0 : W;
     constexpr auto leaving = [](int left) { return left >= CB ? CB : left >= 2 ? 2 : 1; };     // blocks of columns at once, of those that are left
-    constexpr auto lines = [](int nb) { return U * U * nb >= 512 ? U * U * nb / 512 : 1; };     // stores of a wave for them
+    constexpr auto lines = [](int nb) { return U * U * nb * SIZE >= 1024 ? U * U * nb * SIZE / 1024 : 1; };     // stores of a wave for them
     constexpr int STORES = [=] { int n = 0; for (int b = 0; b < OW; b += leaving(OW - b)) n += lines(leaving(OW - b)); return X * n; }();   // for a tile
     // Phase P of eight: products of a half of x with a half of w. It reads part P + 2 and asks for part P + 8 PAIRS, whose place part P has left.
     // In front of every second phase: parts P + 2 and P + 3 have landed, everyone has read P and P + 1. (`stored`: the last tile's results, asked
@@ -386,9 +392,9 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
         // ---- results: U rows of 64 columns at a time through the wave's own piece of LDS, whole lines to memory. acc[a][b][4 q + k]: row U a
         // + lu, column U b + (256 / U) q + 4 lg + k. Stores beyond the rows or columns are dropped by the descriptor ----------------------
         char *mine = smem + PAIRS * PAIR + wave * U * PITCH;
-        char *base = static_cast<char *>(p.out) + here.row0 * ob + static_cast<int64_t>(here.col0) * 2;
-        const int bytes = static_cast<int>(here.rows * ob - static_cast<int64_t>(here.col0) * 2), cols = p.N - here.col0;
-        unsigned first = static_cast<unsigned>(wm * U * X * ob + wn * OUTW * 2);
+        char *base = static_cast<char *>(p.out) + ((SLABS ? static_cast<int64_t>(here.expert) * p.M : 0) + here.row0) * ob + static_cast<int64_t>(here.col0) * SIZE;
+        const int bytes = static_cast<int>(here.rows * ob - static_cast<int64_t>(here.col0) * SIZE), cols = p.N - here.col0;
+        unsigned first = static_cast<unsigned>(wm * U * X * ob + wn * OUTW * SIZE);
         asm volatile("" : "+s"(first));     // (addresses made anew for every tile: kept, they cost the loop its registers)
 #pragma unroll
         for (int a = 0; a < X; ++a) {
@@ -398,12 +404,18 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
             }
 #pragma unroll
             for (int b0 = 0; b0 < OW; b0 += leaving(OW - b0)) {
-                const int nb = leaving(OW - b0), pieces = nb * U / 8;       // 16-byte pieces of a row
+                const int nb = leaving(OW - b0), pieces = nb * U * SIZE / 16;       // 16-byte pieces of a row
 #pragma unroll
                 for (int b = b0; b < b0 + nb; ++b)
 #pragma unroll
                     for (int q = 0; q < U * U / 256; ++q) {
                         if constexpr (GATED) __builtin_amdgcn_sched_barrier(0);     // (one unit after the other: registers)
+                        const int col = (b - b0) * U + q * (256 / U) + 4 * lg;
+                        if constexpr (SLABS) {
+                            const float4_t v = {acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
+                            *reinterpret_cast<float4_t *>(mine + lu * PITCH + ((col >> 2) ^ (lu & 7)) * 16) = v;
+                            continue;
+                        }
                         vec4_t<T> v;
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
@@ -431,12 +443,11 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
                                 v[k] = y;
                             }
                         }
-                        const int col = (b - b0) * U + q * (256 / U) + 4 * lg;
                         *reinterpret_cast<vec4_t<T> *>(mine + lu * PITCH + (((col >> 3) ^ (lu & 7)) * 16 + (col & 4) * 2)) = v;
                     }
                 const int c = lane & (pieces - 1), r0 = lane / pieces;
                 unsigned off = static_cast<unsigned>(r0 * ob + c * 16) + first;
-                if (c * 8 >= cols - wn * OUTW - b0 * U || r0 >= U) off = 0x80000000u;
+                if (c * (16 / SIZE) >= cols - wn * OUTW - b0 * U || r0 >= U) off = 0x80000000u;
                 vec8_t<T> line[lines(CB)];
 #pragma unroll
                 for (int i = 0; i < lines(nb); ++i) {
@@ -444,7 +455,7 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
                     line[i] = *reinterpret_cast<const vec8_t<T> *>(mine + r * PITCH + ((c ^ (r & 7)) * 16));
                 }
                 const __amdgpu_buffer_rsrc_t rsrc =
-                    __builtin_amdgcn_make_buffer_rsrc(base + a * U * ob + b0 * U * 2, 0, max(0, bytes - static_cast<int>(a * U * ob) - b0 * U * 2), 0x00020000);
+                    __builtin_amdgcn_make_buffer_rsrc(base + a * U * ob + b0 * U * SIZE, 0, max(0, bytes - static_cast<int>(a * U * ob) - b0 * U * SIZE), 0x00020000);
 #pragma unroll
                 for (int i = 0; i < lines(nb); ++i)
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, line[i]), rsrc, static_cast<int>(off + i * static_cast<unsigned>(64 / pieces * ob)), 0, 0);
@@ -461,6 +472,7 @@ template <typename T, int U, int X0, int X1, int W0, int W1, int PAIRS, int ACT,
 int gemm_tile_launch(GemmTileParams p, hipStream_t s) {
     constexpr int BM = 2 * U * (X0 + X1), BN = 2 * U * (W0 + W1) / (ACT >= 2 ? 2 : 1), A_CU = U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS == 1 ? 2 : 1;
     p.n_tiles = (p.N + BN - 1) / BN;
+    if constexpr (ACT == kTileSlabs) p.share = Divisor::of(p.n_tiles), p.n_tiles *= p.splits;
     // (experts: as many row tiles as there can be, each of theirs may end in a part of one; how many there are is on the device)
     p.m_tiles = (p.M + BM - 1) / BM + (ROWS == kTileDense ? 0 : min(p.experts, p.M));
     const int64_t tiles = static_cast<int64_t>(p.m_tiles) * p.n_tiles;
@@ -488,7 +500,7 @@ constexpr unsigned kTilesPlain = 0x7ff, kTilesAct = 0x63f;      // with an activ
 // tiles(rows, rows of w): how many. (Six tiles instead of eleven: 1.05 of the time, 1.08 to 1.14 for 1828 of 28672 x 4096, 4498 of 2048 x 2048, 3657 of
 // 2048 x 8192, 5112 of 4096 x 4096.)
 template <typename Tiles>
-int gemm_tile_shape(Tiles &&tiles, int64_t k, unsigned set) {
+int gemm_tile_shape(Tiles &&tiles, int64_t k, unsigned set, double *us_out = nullptr) {
     const double p = static_cast<double>(k) / 128;
     auto one = [&](const TileShape &s) {
         const int64_t t = tiles(32 * s.x, 32 * s.w), turns = ((t + 7) / 8 + 31) / 32;
@@ -507,6 +519,7 @@ int gemm_tile_shape(Tiles &&tiles, int64_t k, unsigned set) {
         const double us = i == 9 ? two(s, 1.81, 1.03, 0.78, 0.63, 0.42) : i == 10 ? two(s, 2.29, 0.85, 0.0, 0.55, 0.20) : one(s);
         if (best < 0 || us < least) best = i, least = us;
     }
+    if (us_out) *us_out = least;
     return best + 1;
 }
 

@@ -281,6 +281,7 @@ def linear(a: torch.Tensor, w: torch.Tensor, skinny: bool = False) -> torch.Tens
 
 # Prompt-sized steps (csrc/gemm_tile.hip); up to here the decode GEMMs serve.
 TILE_MIN_TOKENS = DECODE_MAX_TOKENS + 1
+TILE_MAX_SLAB_BYTES = 64 << 20      # (as many tiles as CUs, of 256 x 256)
 TILE_NONE, TILE_RELU2, TILE_GATED = 0, 1, 2
 TILE_SILU_ROUNDED = 3       # gated unit of rows [up | gate]: round(silu(gate)) up, what silu_and_mul_inplace makes of the product
 
@@ -290,14 +291,15 @@ def _tile_pays(m: int, rows: int, k: int, gated: bool = False) -> bool:
     us, library's): 1024 x 4096, 409 tokens (56 tiles) 21.2 (13.9), 1110 (144) 21.8 (21.8), 2396 (304) 27 (32); 1024 x 6144, 572 (72) 31 (22), 1167 (152)
     31.5 (30.5), 2036 (256) 33 (41); 2048 x 8192, 679 (176) 58 (45), 1260 (320) 70 (68), 1559 (400) 71 (73); 4096 x 14336, 360 (192) 107 (84), 741 (384)
     129 (122), 1521 (768) 172 (188). Up to 2560 columns always (277 of 1024 x 1024 7.4, 8.7). So are very long ones of many tokens, which the
-    library takes in blocks of rows at its best rate: 5112 of 4096 x 14336 505 (458); 4010 tokens 353 (367). And beyond 8192 tokens what is not
+    library takes in blocks of rows at its best rate: 5112 of 4096 x 14336 505 (458); 4010 tokens 353 (367) (not with 2048 rows: 5000 of 2048 x 12288 205
+    (267), 7800 291 (374)). And beyond 8192 tokens what is not
     small, where the library's rate is 5 % to 10 % higher: 12288 of 6144 x 4096 459 (424), 16384 of 8192 x 2048 381 (365), of 1024 x 4096 102 (93), but
     12288 of 1024 x 4096 77 (102), 10000 of 3072 x 1024 55 (72) — unless the launch does an activation's work (28672 x 4096, 16384 2621 (2733))."""
     if m > 8192 and m * rows * k > 6e10 and not gated:
         return False
     if k <= 2560:
         return True
-    return -(-m // 64) * -(-rows // 128) * 16 >= min(k - 2048, 6400) and (k <= 8192 or m <= 4096)
+    return -(-m // 64) * -(-rows // 128) * 16 >= min(k - 2048, 6400) and (k <= 8192 or m <= 4096 or rows <= 2048)
 
 
 def linear_tile(a: torch.Tensor, w: torch.Tensor, act: int = TILE_NONE, act_columns: int = 0, limit: float = 0.0, out: torch.Tensor = None):
@@ -321,6 +323,26 @@ def linear_tile(a: torch.Tensor, w: torch.Tensor, act: int = TILE_NONE, act_colu
     _hip.call("swl_gemm_tile", _hip.ptr(out), _hip.ptr(a), _hip.ptr(w), m, n, k, a.stride(0), ldo, 0, 0, act, int(act_columns), float(limit), 0, code,
               _hip.stream())
     return out
+
+
+def linear_tile_partial(a: torch.Tensor, w: torch.Tensor):
+    """a[T, in] @ w[out, in]^T of a prompt-sized step as SplitKPartials, where few tiles of long sums leave the chip idle (swl_gemm_tile_choose_splits);
+    None otherwise."""
+    if not (a.is_cuda and a.dim() == w.dim() == 2 and a.shape[0] >= TILE_MIN_TOKENS and a.dtype == w.dtype and a.dtype in (torch.float16, torch.bfloat16)):
+        return None
+    m, k = a.shape
+    n = w.shape[0]
+    if w.shape[1] != k or not w.is_contiguous() or a.stride(1) != 1 or (a.data_ptr() | w.data_ptr()) % 16:
+        return None
+    lib, code = _hip.load(), _hip.dtype_code(a.dtype)
+    if not lib.swl_gemm_tile_supported(m, n, k, a.stride(0), -(-n // 8) * 8, TILE_NONE, code):
+        return None
+    splits = lib.swl_gemm_tile_choose_splits(m, n, k)
+    if splits < 2 or splits * m * n * 4 > TILE_MAX_SLAB_BYTES:
+        return None
+    slabs = torch.empty(splits * m * n, dtype=torch.float32, device=a.device)
+    _hip.call("swl_gemm_tile_partial", _hip.ptr(slabs), slabs.numel() * 4, _hip.ptr(a), _hip.ptr(w), m, n, k, a.stride(0), splits, 0, code, _hip.stream())
+    return SplitKPartials(slabs, splits, m, n, a.dtype)
 
 
 def linear_gated(a: torch.Tensor, w: torch.Tensor, act: int, limit: float = 0.0, out: torch.Tensor = None):

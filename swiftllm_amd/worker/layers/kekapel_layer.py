@@ -5,7 +5,7 @@ import torch
 from swiftllm_amd import _hip
 
 from ..kernels.linear import (DECODE_MAX_TOKENS, F32_MAX_TOKENS, ROWS_MAX_TOKENS, linear, linear_f32, linear_gated, linear_rows,
-                              linear_rows_partial, linear_silu_gate, linear_splitk)
+                              linear_rows_partial, linear_silu_gate, linear_splitk, linear_tile_partial)
 from ..kernels.moe import ACT_SILU_UP_FIRST, gated_unit, moe_experts, moe_route
 from ..kernels.polynorm import polynorm
 from ..kernels.window_attn import qknorm_and_store_kv, window_attention
@@ -37,10 +37,11 @@ def _project(a: torch.Tensor, w: torch.Tensor, skinny: bool) -> torch.Tensor:
 
 def _project_partials(a: torch.Tensor, w: torch.Tensor, skinny: bool):
     """_project for a consumer that takes a product's fp32 sums too (it adds them into an fp32 stream, so that they are rounded nowhere):
-    SplitKPartials from the decode GEMMs, rows otherwise."""
+    SplitKPartials from the decode GEMMs and from prompt-sized products of few tiles, rows otherwise."""
     m = a.shape[0]
     if not skinny or m > DECODE_MAX_TOKENS or a.dtype == torch.float32 or getattr(w, "_swl_blas_only", False):
-        return _project(a, w, skinny)
+        y = linear_tile_partial(a, w) if skinny and m > DECODE_MAX_TOKENS else None
+        return _project(a, w, skinny) if y is None else y
     y = linear_rows_partial(a, w) if m <= ROWS_MAX_TOKENS else None
     if y is not None:
         return y

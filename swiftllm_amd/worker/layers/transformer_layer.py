@@ -43,7 +43,7 @@ from ..kernels.linear import (row_scaled_silu_gate_ok, alt_residual_like, linear
                               linear_splitk_from_splitk, tiny_from_splitk_ok)
 from ..kernels.linear import RawResidual, linear_rows_add, linear_silu_gate_nf, linear_splitk_nf, nf_ok, rows_add_ok
 from ..kernels.linear import linear_silu_gate_nx, linear_splitk_nx, nx_ok
-from ..kernels.linear import TILE_SILU_ROUNDED, linear_gated
+from ..kernels.linear import TILE_SILU_ROUNDED, linear_gated, linear_tile_partial
 from ..kernels.rmsnorm import RowScalePending
 from ..kernels.rmsnorm import (add_scale_from_splitk, deferred_norm_ok, fused_add_rmsnorm_inplace,
                                fused_add_rmsnorm_from_splitk)
@@ -329,8 +329,12 @@ class LlamaTransformerLayer:
             else:
                 fused_add_rmsnorm_inplace(attn_out, residual_buf, w.ffn_norm, cfg.rms_norm_eps)
         else:
-            attn_out = linear(input_embds, w.o_proj, self.skinny)
-            fused_add_rmsnorm_inplace(attn_out, residual_buf, w.ffn_norm, cfg.rms_norm_eps)
+            partials = linear_tile_partial(input_embds, w.o_proj) if self.skinny else None
+            if partials is not None:    # (prompt-sized, few tiles)
+                attn_out = fused_add_rmsnorm_from_splitk(partials, residual_buf, w.ffn_norm, cfg.rms_norm_eps)
+            else:
+                attn_out = linear(input_embds, w.o_proj, self.skinny)
+                fused_add_rmsnorm_inplace(attn_out, residual_buf, w.ffn_norm, cfg.rms_norm_eps)
         act = linear_silu_gate(attn_out, w.up_gate_proj) if self.skinny else None
         if act is None and self.skinny:
             act = linear_gated(attn_out, w.up_gate_proj, TILE_SILU_ROUNDED)
@@ -338,4 +342,7 @@ class LlamaTransformerLayer:
             up_gate = linear(attn_out, w.up_gate_proj, self.skinny)
             silu_and_mul_inplace(up_gate)
             act = up_gate[:, :cfg.ffn_inter_dim]
-        return linear_splitk(act, w.down_proj) if fast else linear(act, w.down_proj, self.skinny)
+        if fast:
+            return linear_splitk(act, w.down_proj)
+        partials = linear_tile_partial(act, w.down_proj) if self.skinny else None
+        return linear(act, w.down_proj, self.skinny) if partials is None else partials

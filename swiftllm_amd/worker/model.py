@@ -36,7 +36,7 @@ from .block_manager import BlockManager
 from . import decode_engine as _decode_engine
 from .infer_state import LlamaInferState
 from .kernels.block_swapping import swap_blocks
-from .kernels.linear import RawResidual
+from .kernels.linear import TILE_MAX_SLAB_BYTES, RawResidual
 from .kernels.rmsnorm import fused_add_rmsnorm_from_splitk, rmsnorm_inplace
 from .layers.pre_layer import LlamaPreLayer
 from .layers.transformer_layer import LlamaTransformerLayer
@@ -226,7 +226,8 @@ class LlamaModel:
             graph_bytes = self._measure_decode_graph_bytes()
             free_memory, _ = torch.cuda.mem_get_info()      # (the measurement may have grown the regular pool as well)
             peak_memory = max(peak_memory, total_memory - free_memory)
-        num_blocks = math.floor((usable - peak_memory - table_bytes - graph_bytes) / block_bytes)
+        # (TILE_MAX_SLAB_BYTES: of a smaller prompt step, whose products' sums are split)
+        num_blocks = math.floor((usable - peak_memory - table_bytes - graph_bytes - TILE_MAX_SLAB_BYTES) / block_bytes)
         torch.cuda.empty_cache()
         return max(num_blocks, 0)
 

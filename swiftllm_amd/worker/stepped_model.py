@@ -28,6 +28,7 @@ from swiftllm_amd.utils import GB
 from .batch_plan import StepEntry, StepPlan, plan_step, plan_tokens
 from .block_manager import BlockManager
 from .kernels.block_swapping import swap_blocks
+from .kernels.linear import TILE_MAX_SLAB_BYTES
 from .kernels.sampling import argmax_rows
 from .kernels.window_attn import SHARE_MAX_SCRATCH
 from .pinned_ring import PinnedRing
@@ -137,9 +138,9 @@ class SteppedModel:
 
     def _scratch_bytes(self, num_tokens: int, batch: int) -> int:
         """The most scratch that a launch of a step of these sizes takes beside what the forged step shows: of attention, which it
-        leaves out without a pool. (Designs whose recurrences take some by the lengths of the portions add it: the forged ones are
+        leaves out without a pool, and of products whose sums a smaller step splits. (Designs whose recurrences take some by the lengths of the portions add it: the forged ones are
         equal, and may all be short.)"""
-        return SHARE_MAX_SCRATCH
+        return SHARE_MAX_SCRATCH + TILE_MAX_SLAB_BYTES
 
     @torch.inference_mode()
     def init_kvcache_and_swap(self, num_blocks: int):

@@ -179,3 +179,42 @@ def test_products_of_experts(n, top, experts, K, N, dtype):
             want, slack = p, d
         assert bool(((out[:total].double() - want).abs() <= slack + ulp * want.abs() + floor).all()), (mode, act, weigh, ordered)
         assert bool((out[total] == 7).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", range(12))
+@pytest.mark.parametrize("m,n,k,splits", [(1, 8, 512, 2), (257, 136, 768, 3), (300, 1032, 2048, 8), (129, 264, 1280, 5), (1025, 520, 1024, 2), (2500, 3080, 512, 2), (700, 72, 256, 1)])
+def test_slabs_of_k_shares(m, n, k, splits, shape, dtype):
+    """Every slab is the fp32 sum over its share, whatever the order of the additions; nothing is written behind the last."""
+    from swiftllm_amd import _hip
+    x, w = _operands(m, n, k, dtype)
+    slabs = torch.full((splits * m + 2, n), 7.0, device="cuda")
+    _hip.call("swl_gemm_tile_partial", _hip.ptr(slabs), splits * m * n * 4, _hip.ptr(x), _hip.ptr(w), m, n, k, x.stride(0), splits, shape,
+              _hip.dtype_code(dtype), _hip.stream())
+    xs, ws = x.double().reshape(m, splits, -1).transpose(0, 1), w.double().reshape(n, splits, -1).permute(1, 2, 0).contiguous()
+    bound = 2.0 ** -24 * (k // splits) * (xs.abs() @ ws.abs()).reshape(-1, n) + 2.0 ** -24 * (xs @ ws).reshape(-1, n).abs()
+    assert bool(((slabs[:splits * m].double() - (xs @ ws).reshape(-1, n)).abs() <= bound).all())
+    assert bool((slabs[splits * m:] == 7).all())
+
+
+@pytest.mark.parametrize("m,n,k,want", [(300, 1024, 4096, True), (2029, 1024, 6144, True), (600, 2048, 8192, True), (300, 4096, 14336, True),
+                                        (7691, 1024, 1024, False), (5112, 4096, 14336, False), (256, 1024, 4096, False), (300, 1026, 4096, False)])
+def test_slabs_where_tiles_are_few(m, n, k, want):
+    """What linear_tile_partial takes, and that its sums are those of the product's rows (whose one rounding is the difference)."""
+    from swiftllm_amd.worker.kernels import rms_stream
+    from swiftllm_amd.worker.kernels.linear import linear, linear_tile_partial
+    x, w = _operands(m, n, k, torch.bfloat16)
+    parts = linear_tile_partial(x, w)
+    assert (parts is not None) == want
+    if not want:
+        return
+    z = x.double() @ w.double().T
+    assert bool(((parts.materialize().double() - z).abs() <= _product_bound(z, x, w)).all())
+    # the fp32 stream's step on the slabs and on the rows: y / rms(y) of rows of about unit size, each rounded by half an ulp
+    g = torch.Generator(device="cuda").manual_seed(1)
+    stream, ones = torch.randn((m, n), generator=g, device="cuda"), torch.ones(n, device="cuda")
+    a, b = stream.clone(), stream.clone()
+    rms_stream.gated_add_rmsnorm(a, parts, post=ones, pre=ones)
+    rms_stream.gated_add_rmsnorm(b, linear(x, w, skinny=True), post=ones, pre=ones)
+    rms = z.pow(2).mean(-1, keepdim=True).sqrt()
+    assert bool(((a - b).double().abs() <= 2 * _product_bound(z, x, w) / rms + 2.0 ** -7 * (z / rms).abs()).all())
