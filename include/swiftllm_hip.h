@@ -1012,6 +1012,12 @@ int swl_linear_scan_segments(float *o, int64_t o_stride, const float *qd, const 
                              const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0, const int32_t *tok_pos,
                              const int32_t *tok_state, int32_t num_seqs, int32_t num_heads, int32_t dim, int32_t vdim,
                              int32_t segments, int32_t seg_tiles, float *scratch, int32_t dtype, swl_stream_t stream);
+/* ... of a step of num_tiles tiles, which bound the segments that there are (0: as many for every portion). */
+int swl_linear_scan_cut(float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra,
+                        const void *v, int64_t v_stride, const float *dskip, float *state, int64_t slot_stride, int64_t s_off,
+                        const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0, const int32_t *tok_pos,
+                        const int32_t *tok_state, int32_t num_seqs, int32_t num_heads, int32_t dim, int32_t vdim,
+                        int32_t segments, int32_t seg_tiles, int32_t num_tiles, float *scratch, int32_t dtype, swl_stream_t stream);
 int swl_linear_step(void *out, int64_t out_stride, float *y, int64_t y_stride, const void *q, int64_t q_stride, const void *k,
                     int64_t k_stride, const void *v, int64_t v_stride, const float *decay, int64_t decay_stride,
                     int32_t per_channel, const float *k_scale, const float *bonus, float q_scale, const float *dskip, float *state,

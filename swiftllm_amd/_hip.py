@@ -195,6 +195,8 @@ SIGNATURES = {
                         _I32, _P],
     "swl_linear_scan_segments": [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _I64, _I64,
                                  _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _P, _I32, _P],
+    "swl_linear_scan_cut": [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _I64, _I64,
+                            _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _P, _I32, _P],
     "swl_linear_step": [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _I64, _I32, _P, _P, _F32, _P, _P, _I64, _I64,
                         _P, _P, _P, _I32, _I32, _I32, _I32, _I32, _P, _I32, _P, _I64, _F32, _F32, _I32, _P],
     "swl_low_rank_decay": [_P, _P, _I64, _P, _P, _P, _I64, _I32, _I32, _I32, _I32, _I32, _F32, _I32, _P],

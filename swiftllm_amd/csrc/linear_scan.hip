@@ -30,7 +30,9 @@
 //   swl_linear_step:   steps whose portions are single tokens (decode): one workgroup per (sequence, head) streams the state once
 //                      and finishes the head — read-out, RMS norm over the head, weight, gate — in the same launch.
 // Everything after the loads of q, k, v is fp32.
-#include "swl_common.h"
+#include "gemm_tile.h"
+
+#include <algorithm>
 
 namespace swl {
 
@@ -41,7 +43,10 @@ constexpr int kLsMaxDim = 320;          // padded key channels: 3 * 16 * 320 flo
 
 __device__ __forceinline__ float ls_silu(float z) { return z / (1.0f + expf(-z)); }
 
-template <typename T, bool BONUS>
+// What bounds it: its rows and blocks are 30 MB for 2030 tokens and 8 heads of 128 channels (6 us); with one channel a load, each waited for behind
+// a division and a predicate, eight turns of that latency took 22 us. WIDE: a thread takes eight channels of a token, loaded without a
+// predicate and all at once, queries and keys are worked on by different waves, and the products read four channels at a time.
+template <typename T, bool BONUS, bool WIDE>
 __global__ __launch_bounds__(kLsThreads) void linear_chunks_kernel(
     float *qd, float *kd, float *total, float *intra, const T *q, int64_t q_stride, const T *k, int64_t k_stride, const float *decay,
     int64_t decay_stride, int per_channel, const float *k_scale, const float *bonus, float q_scale, const int32_t *tile_row0,
@@ -53,7 +58,40 @@ __global__ __launch_bounds__(kLsThreads) void linear_chunks_kernel(
     const int64_t at = static_cast<int64_t>(tile) * H + h;
     const int qk0 = (h / rep) * d;
     // tokens beyond the tile's and channels beyond the head: q = k = 0, decay 1
-    for (int i = threadIdx.x; i < kLsTile * dp; i += kLsThreads) {
+    if constexpr (WIDE) {       // (whole blocks of 64 channels, rows on 16 bytes)
+        const int per = d >> 3;
+        for (int i = threadIdx.x; i < kLsTile * per; i += kLsThreads) {
+            const int t = i / per, e = (i - t * per) * 8;
+            const int64_t row = row0 + min(t, cnt - 1);
+            const vec8_t<T> q8 = load8(q + row * q_stride + qk0 + e), k8 = load8(k + row * k_stride + qk0 + e);
+            const float *ap = decay + row * decay_stride;
+            float4_t a0, a1;
+            if (per_channel) {      // (uniform)
+                a0 = *reinterpret_cast<const float4_t *>(ap + h * d + e);
+                a1 = *reinterpret_cast<const float4_t *>(ap + h * d + e + 4);
+            } else {
+                const float a = ap[h];
+                a0 = a1 = float4_t{a, a, a, a};
+            }
+            const float scale = k_scale ? k_scale[row * H + h] : 1.f;
+            const bool ok = t < cnt;
+            float4_t o[6];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                o[c >> 2][c & 3] = ok ? to_f(q8[c]) * q_scale : 0.f;
+                const float kv = to_f(k8[c]);
+                o[2 + (c >> 2)][c & 3] = ok ? k_scale ? kv * scale : kv : 0.f;
+                o[4 + (c >> 2)][c & 3] = ok ? c < 4 ? a0[c & 3] : a1[c & 3] : 1.f;
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                *reinterpret_cast<float4_t *>(qs + t * dp + e + 4 * c) = o[c];
+                *reinterpret_cast<float4_t *>(ks + t * dp + e + 4 * c) = o[2 + c];
+                *reinterpret_cast<float4_t *>(as + t * dp + e + 4 * c) = o[4 + c];
+            }
+        }
+    }
+    for (int i = threadIdx.x; !WIDE && i < kLsTile * dp; i += kLsThreads) {
         const int t = i / dp, e = i - t * dp;
         float qv = 0.f, kv = 0.f, av = 1.f;
         if (t < cnt && e < d) {
@@ -68,31 +106,46 @@ __global__ __launch_bounds__(kLsThreads) void linear_chunks_kernel(
         as[i] = av;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < dp; e += kLsThreads) {
-        float p = 1.f;
-        float *qo = qd + at * kLsTile * dp + (e >> 4) * 256 + (e & 15);     // 16 x 16 blocks [channels / 16][token][channel]
+    // (WIDE: queries first, then keys: whole waves of either)
+    for (int at_e = threadIdx.x; at_e < (WIDE ? 2 : 1) * dp; at_e += kLsThreads) {
+        const bool of_q = !WIDE || at_e < dp, of_k = !WIDE || !of_q;
+        const int e = of_q ? at_e : at_e - dp;
+        const float *xs = of_q ? qs : ks;
+        float x[kLsTile], a[kLsTile];
 #pragma unroll
         for (int t = 0; t < kLsTile; ++t) {
-            const float a = as[t * dp + e];
-            if constexpr (BONUS) {
-                qo[t * 16] = qs[t * dp + e] * p;
-                p *= a;
-            } else {
-                p *= a;
-                qo[t * 16] = qs[t * dp + e] * p;
-            }
+            x[t] = xs[t * dp + e];
+            a[t] = as[t * dp + e];
         }
-        total[at * dp + e] = p;
-        float kk[kLsTile];
-        p = 1.f;
+        if (of_q) {
+            float *qo = qd + at * kLsTile * dp + (e >> 4) * 256 + (e & 15);     // 16 x 16 blocks [channels / 16][token][channel]
+            float p = 1.f;
+#pragma unroll
+            for (int t = 0; t < kLsTile; ++t) {
+                if constexpr (BONUS) {
+                    qo[t * 16] = x[t] * p;
+                    p *= a[t];
+                } else {
+                    p *= a[t];
+                    qo[t * 16] = x[t] * p;
+                }
+            }
+            total[at * dp + e] = p;
+        }
+        if (!of_k) continue;
+        if constexpr (!WIDE) {
+#pragma unroll
+            for (int t = 0; t < kLsTile; ++t) x[t] = ks[t * dp + e];
+        }
+        float p = 1.f;
 #pragma unroll
         for (int t = kLsTile - 1; t >= 0; --t) {
-            kk[t] = ks[t * dp + e] * p;
-            p *= as[t * dp + e];
+            x[t] *= p;
+            p *= a[t];
         }
         float *ko = kd + (at * dp + e) * kLsTile;
 #pragma unroll
-        for (int t = 0; t < kLsTile; t += 4) *reinterpret_cast<float4_t *>(ko + t) = float4_t{kk[t], kk[t + 1], kk[t + 2], kk[t + 3]};
+        for (int t = 0; t < kLsTile; t += 4) *reinterpret_cast<float4_t *>(ko + t) = float4_t{x[t], x[t + 1], x[t + 2], x[t + 3]};
     }
     // M: thread (s, g) takes key token s and the channels g, g + 16, ...; sixteen neighbouring lanes share an s
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -100,7 +153,40 @@ __global__ __launch_bounds__(kLsThreads) void linear_chunks_kernel(
     float acc[kLsTile];
 #pragma unroll
     for (int t = 0; t < kLsTile; ++t) acc[t] = 0.f;
-    for (int e = g; e < d; e += 16) {
+    auto products = [&](auto wc) {      // (a wave's key tokens are 4 wave .. 4 wave + 3)
+        constexpr int FIRST = 4 * decltype(wc)::value;
+        for (int e = 4 * g; e < d; e += 64) {
+            float4_t p = *reinterpret_cast<const float4_t *>(ks + s * dp + e), diag = {};
+            if constexpr (BONUS) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) diag[c] = p[c] * bonus[h * d + e + c];
+            }
+#pragma unroll
+            for (int t = FIRST; t < kLsTile; ++t) {
+                const float4_t a = *reinterpret_cast<const float4_t *>(as + t * dp + e), qv = *reinterpret_cast<const float4_t *>(qs + t * dp + e);
+                const bool past = t >= FIRST + 4 || t > s, now = t >= FIRST + 4 || t >= s;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    if constexpr (BONUS) {
+                        acc[t] = fmaf(qv[c], past ? p[c] : now ? diag[c] : 0.f, acc[t]);
+                        p[c] = past ? p[c] * a[c] : p[c];
+                    } else {
+                        p[c] = past ? p[c] * a[c] : p[c];
+                        acc[t] = fmaf(qv[c], now ? p[c] : 0.f, acc[t]);
+                    }
+                }
+            }
+        }
+    };
+    if constexpr (WIDE) {
+        switch (wave) {
+        case 0: products(std::integral_constant<int, 0>{}); break;
+        case 1: products(std::integral_constant<int, 1>{}); break;
+        case 2: products(std::integral_constant<int, 2>{}); break;
+        default: products(std::integral_constant<int, 3>{}); break;
+        }
+    }
+    for (int e = g; !WIDE && e < d; e += 16) {
         float p = ks[s * dp + e];
         float diag = 0.f;
         if constexpr (BONUS) diag = p * bonus[h * d + e];
@@ -370,6 +456,282 @@ __global__ __launch_bounds__(kLsThreads) void linear_segments_kernel(
     }
 }
 
+// ---- heads of 64 or 128 key channels: 64 columns a workgroup, 16 of all rows a wave ----------------------------------------------------
+// In the walks above four waves have a quarter of the rows each and add their partial outputs up through LDS once a tile, and every 16 columns read all
+// operands: 2.5 us a tile with two workgroups on a CU, a fifth of it matrix steps. Here a wave keeps all rows of its columns (NT accumulator
+// tiles), and a tile's operands come to LDS once for four of them, two tiles ahead. (Straight to every wave's registers they took a CU's
+// address units as long as the matrix steps: 1.6 us a tile.) The fp32 matrix core bounds it where every SIMD has a wave: 8 NT + 4 steps of 32 cycles.
+struct LwParams {
+    float *o;
+    const float *qd, *kd, *total, *intra;
+    const void *v;
+    const float *dskip;
+    float *state, *seg_states, *seg_decays;
+    const int32_t *seq_row0, *seq_cnt, *seq_tile0, *tok_pos, *tok_state;
+    int64_t o_stride, v_stride, slot_stride, s_off;
+    int H, dv, shares, num_seqs, segments, seg_tiles;       // shares: of 64 columns
+    Divisor span;           // tokens of a segment
+};
+
+// STATES false: the scan. true: the states that a cut portion's segments leave (linear_segments_kernel).
+template <typename T, int NT, bool STATES>
+__global__ __launch_bounds__(kLsThreads, 2) void linear_scan_wide_kernel(LwParams p) {
+    constexpr int D = 16 * NT, SZ = sizeof(T), VB = SZ;     // (a tile's values: 16 rows of 64 columns, a KiB each fetch)
+    constexpr int Q = 0, K = STATES ? 0 : NT, V = K + NT, A = V + VB, M = A + 1, FETCHES = M + (STATES ? 0 : 1), EACH = (FETCHES + 3) / 4;
+    constexpr int SLOT = FETCHES * 1024, SLOTS = 3;
+    __shared__ __attribute__((aligned(16))) char smem[SLOTS * SLOT];
+    // This workgroup's segment: those that there are, counted from the portions' lengths (a grid of as many for each portion as the longest has kept a step
+    // of 2 prompts beside 30 decoded tokens busy with workgroups that leave at once: 34 us instead of 27, 8 heads of 128 x 128), (segment, head) on the XCDs in turn,
+    // all columns of one on one XCD
+    const int id = static_cast<int>(blockIdx.x >> 3), rest = id / p.shares, at = rest * 8 + static_cast<int>(blockIdx.x & 7), piece = at / p.H, h = at - piece * p.H;
+    const int lane = threadIdx.x & 63, dv = p.dv;
+    int seq = piece, seg = 0, all, start, tile_0;       // (the three arrays asked for together: each wait is one for memory, the caches are cold)
+    if (p.segments > 1) {
+        int before = 0;
+        for (int s0 = 0;; s0 += 64) {
+            if (s0 >= p.num_seqs) return;
+            const int s = min(s0 + lane, p.num_seqs - 1), cnt_s = p.seq_cnt[s], row_s = p.seq_row0[s], tile_s = p.seq_tile0[s];
+            const int mine = s0 + lane < p.num_seqs ? min(p.segments, static_cast<int>(divide(static_cast<unsigned>(cnt_s) + p.span.by - 1, p.span))) : 0;
+            int scan = mine;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int x = __shfl_up(scan, o, 64);
+                if (lane >= o) scan += x;
+            }
+            const unsigned long long past = __ballot(before + scan > piece);
+            if (past) {
+                const int l = __builtin_ctzll(past);
+                seq = s0 + l;
+                seg = piece - before - __builtin_amdgcn_readlane(scan - mine, l);
+                all = __builtin_amdgcn_readlane(cnt_s, l), start = __builtin_amdgcn_readlane(row_s, l), tile_0 = __builtin_amdgcn_readlane(tile_s, l);
+                break;
+            }
+            before += __builtin_amdgcn_readlane(scan, 63);
+        }
+    } else {
+        if (piece >= p.num_seqs) return;
+        const int cnt_s = p.seq_cnt[seq], row_s = p.seq_row0[seq], tile_s = p.seq_tile0[seq];
+        all = __builtin_amdgcn_readfirstlane(cnt_s), start = __builtin_amdgcn_readfirstlane(row_s), tile_0 = __builtin_amdgcn_readfirstlane(tile_s);
+    }
+    const int unit = seq * p.H + h, first = seg * p.seg_tiles * kLsTile;
+    if (first >= all) return;
+    const bool last = all - first <= p.seg_tiles * kLsTile, cut = !(last && seg == 0);
+    if (STATES && last) return;     // a portion's last segment (an only one too) leaves its state to the scan
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lq = lane >> 4;
+    const int col0 = (id - rest * p.shares) * 64, cols = min(64, dv - col0), own = col0 + wave * 16 + li, col = min(own, dv - 1);
+    const bool okc = own < dv;
+    const int row0 = start + first, cnt = last ? all - first : p.seg_tiles * kLsTile, nt = (cnt + kLsTile - 1) / kLsTile;
+    const int64_t tile0 = (tile_0 + static_cast<int64_t>(seg) * p.seg_tiles) * p.H + h;
+    const int64_t states = static_cast<int64_t>(D) * dv;
+    float *S = p.state + static_cast<int64_t>(p.tok_state[start] >> 1) * p.slot_stride + p.s_off + h * states;
+    const bool fresh = p.tok_pos[start] == 0;       // a sequence starts from the zero state whatever the slot held
+    float *const from_seg = p.seg_states + static_cast<int64_t>(unit) * (p.segments + 1) * states;
+
+    // ---- fetches: KiB wave, wave + 4, ... of a tile's [queries | keys | values | decays | products] (as they are read: 16 bytes a lane); what is too
+    // many repeats the decays, rows beyond the portion and tiles beyond the last are zeros without a memory access --------------------
+    const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char *)smem));
+    const int64_t vb = p.v_stride * SZ;
+    int4v rsrc[EACH];       // (of the next tile that is asked for)
+    int64_t step[EACH];
+    int to[EACH], v_row[EACH];
+    unsigned off[EACH];
+    auto v_bytes = [&](int rows) { return rows > 0 ? static_cast<int>(min(rows, kLsTile) * vb - vb) + cols * SZ : 0; };
+#pragma unroll
+    for (int n = 0; n < EACH; ++n) {
+        const int f = wave + 4 * n < FETCHES ? wave + 4 * n : A;
+        to[n] = f * 1024;
+        v_row[n] = -1;
+        off[n] = lane * 16;
+        if (f < V) {
+            rsrc[n] = tile_rsrc(reinterpret_cast<const char *>(f < K ? p.qd : p.kd) + (tile0 * NT + (f < K ? f : f - K)) * 1024, 1024);
+            step[n] = static_cast<int64_t>(p.H) * NT * 1024;
+            off[n] = li * 64 + lq * 16;
+        } else if (f < A) {
+            constexpr int PER = 4 * SZ;     // lanes of a row
+            v_row[n] = (f - V) * (64 / PER);
+            rsrc[n] = tile_rsrc(static_cast<const char *>(p.v) + (row0 + v_row[n]) * vb + (static_cast<int64_t>(h) * dv + col0) * SZ, v_bytes(cnt - v_row[n]));
+            step[n] = kLsTile * vb;
+            off[n] = static_cast<unsigned>(lane / PER * vb) + lane % PER * 16;
+        } else if (f == A) {
+            rsrc[n] = tile_rsrc(reinterpret_cast<const char *>(p.total + tile0 * D), D * 4);
+            step[n] = static_cast<int64_t>(p.H) * D * 4;
+        } else {
+            rsrc[n] = tile_rsrc(reinterpret_cast<const char *>(p.intra + tile0 * 256), 1024);
+            step[n] = static_cast<int64_t>(p.H) * 1024;
+        }
+    }
+    int asked = 0;
+    unsigned slot_to = lds0;
+    auto ask = [&](int n) { tile_fetch(rsrc[n], off[n], 0, slot_to + to[n]); };
+    auto asked_all = [&]() {        // on to the next tile
+        ++asked;
+        slot_to = slot_to == lds0 + (SLOTS - 1) * SLOT ? lds0 : slot_to + SLOT;
+#pragma unroll
+        for (int n = 0; n < EACH; ++n) {
+            const uint64_t at = (static_cast<uint64_t>(static_cast<unsigned>(rsrc[n][1])) << 32 | static_cast<unsigned>(rsrc[n][0])) + step[n];
+            rsrc[n][0] = static_cast<int>(at), rsrc[n][1] = static_cast<int>(at >> 32);
+        }
+        if (asked >= nt - 1) {
+#pragma unroll
+            for (int n = 0; n < EACH; ++n) rsrc[n][2] = asked >= nt ? 0 : v_row[n] < 0 ? rsrc[n][2] : v_bytes(cnt - asked * kLsTile - v_row[n]);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < SLOTS - 1; ++i) {
+#pragma unroll
+        for (int n = 0; n < EACH; ++n) ask(n);
+        asked_all();
+    }
+
+    // ---- the state in front of the segment: st[j][r] = S[16 j + 4 lq + r][col] ---------------------------------------------------------
+    float4_t st[NT], decay[STATES ? NT : 1];
+    const int lane_at = 4 * lq * dv + col;
+    auto load = [&](const float *s, float4_t (&x)[NT]) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[j][r] = s[lane_at + (16 * j + r) * dv];
+    };
+    const float *begin = STATES || !cut ? S : seg == 0 ? from_seg : from_seg + states;
+    if (STATES ? seg > 0 || fresh : !cut && fresh) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) st[j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    } else {
+        load(begin, st);
+    }
+    if constexpr (STATES) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            decay[j] = float4_t{1.f, 1.f, 1.f, 1.f};
+            if (seg == 0 && okc) {      // (the last segment may be done with the slot before the first one's scan starts)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) from_seg[lane_at + (16 * j + r) * dv] = st[j][r];
+            }
+        }
+    } else {
+        // each segment's own state behind what came before it, the next one asked for beside it
+        const float *by = p.seg_decays + static_cast<int64_t>(unit) * p.segments * D + 4 * lq;
+        float4_t more[2][NT], b[2][NT];
+        auto load_segment = [&](int g, float4_t (&x)[NT], float4_t (&y)[NT]) {
+            load(from_seg + (g + 1) * states, x);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) y[j] = *reinterpret_cast<const float4_t *>(by + g * D + 16 * j);
+        };
+        auto behind = [&](const float4_t (&x)[NT], const float4_t (&y)[NT]) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) st[j][r] = fmaf(st[j][r], y[j][r], x[j][r]);
+        };
+        if (seg > 1) load_segment(1, more[0], b[0]);
+        for (int g = 1; g < seg; g += 2) {
+            load_segment(min(g + 1, seg - 1), more[1], b[1]);
+            behind(more[0], b[0]);
+            if (g + 1 >= seg) break;
+            load_segment(min(g + 2, seg - 1), more[0], b[0]);
+            behind(more[1], b[1]);
+        }
+    }
+    float dh = !STATES && p.dskip ? p.dskip[h] : 0.f;
+    // (arrived before the walk: a wait for them inside it is one for all fetches that are on their way)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) mfma_results_tie(st[j]);
+    mfma_results_tie(dh);
+
+    constexpr int STORES = STATES ? 0 : 4;
+    unsigned slot_at = 0;
+    for (int i = 0; i < nt; ++i) {
+        // this tile's fetches have landed (behind them: the next tile's and the last tile's stores), everyone is done with the slot before
+        __builtin_amdgcn_sched_barrier(0);
+        if (i == 0) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(EACH) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(EACH + STORES) : "memory");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        const char *slot = smem + slot_at;
+        float vv[4], m[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vv[r] = to_f(*reinterpret_cast<const T *>(slot + V * 1024 + ((4 * lq + r) * 64 + wave * 16 + li) * SZ));
+        if constexpr (!STATES) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) m[r] = *reinterpret_cast<const float *>(slot + M * 1024 + (r * 64 + lane) * 4);
+        }
+        float4_t q[2], k[2], a[2];
+        auto read = [&](int j) {
+            if constexpr (!STATES) q[j & 1] = *reinterpret_cast<const float4_t *>(slot + (Q + j) * 1024 + lane * 16);
+            k[j & 1] = *reinterpret_cast<const float4_t *>(slot + (K + j) * 1024 + lane * 16);
+            a[j & 1] = *reinterpret_cast<const float4_t *>(slot + A * 1024 + (16 * j + 4 * lq) * 4);
+        };
+        read(0);
+        // (sums of 16 rows each, added up in the order of linear_scan_kernel's: one long sum a register has 1.1 times the error)
+        float4_t part[NT], in_tile[4];
+        if constexpr (!STATES) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) in_tile[r] = mfma_f32_16x16x4(m[r], vv[r], float4_t{0.f, 0.f, 0.f, 0.f});
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {      // (operands are read while the rows before are multiplied)
+            if (j + 1 < NT) read(j + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (STATES) decay[j] *= a[j & 1];
+            float4_t next = st[j] * a[j & 1];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (!STATES) part[j] = mfma_f32_16x16x4(q[j & 1][r], st[j][r], r ? part[j] : float4_t{0.f, 0.f, 0.f, 0.f});
+                next = mfma_f32_16x16x4(k[j & 1][r], vv[r], next);
+                if (EACH <= NT ? r == 1 && j < EACH : r == 0 || r == 2) {       // (requests between the matrix steps)
+                    const int n = EACH <= NT ? j : 2 * j + (r >> 1);
+                    if (n < EACH) ask(n);
+                }
+            }
+            st[j] = next;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        asked_all();
+        slot_at = slot_at == (SLOTS - 1) * SLOT ? 0 : slot_at + SLOT;
+        if constexpr (STATES) {
+            mfma_results_ready<8>(st[NT - 1]);
+            continue;
+        }
+#pragma unroll
+        for (int j = 0; j < NT - 1; ++j) mfma_results_tie(part[j]);
+        mfma_results_ready<8>(part[NT - 1]);
+        float4_t out = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            float4_t sum = in_tile[c];
+#pragma unroll
+            for (int j = c * NT / 4; j < (c + 1) * NT / 4; ++j) sum += part[j];
+            out += sum;
+        }
+        if (p.dskip) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[r] = fmaf(dh, vv[r], out[r]);
+        }
+        // (stores that are always made, so that they can be counted; tokens beyond the portion's and columns beyond the head's are dropped)
+        const int rows = min(kLsTile, cnt - i * kLsTile);
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            p.o + (row0 + static_cast<int64_t>(i) * kLsTile) * p.o_stride + static_cast<int64_t>(h) * dv, 0, static_cast<int>((rows - 1) * p.o_stride + dv) * 4, 0x00020000);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(out[r]), rsrc, okc ? static_cast<int>((4 * lq + r) * p.o_stride + own) * 4 : 0x7fffffff, 0, 0);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");      // (fetches of no tile write zeros to LDS)
+    if (!STATES && !last) return;
+#pragma unroll
+    for (int j = 0; j < NT - 1; ++j) mfma_results_tie(st[j]);
+    mfma_results_ready<8>(st[NT - 1]);
+    float *const into = STATES ? from_seg + (seg + 1) * states : S;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        if (okc) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) into[lane_at + (16 * j + r) * dv] = st[j][r];
+        }
+        if constexpr (STATES) {
+            if (own == 0) *reinterpret_cast<float4_t *>(p.seg_decays + (static_cast<int64_t>(unit) * p.segments + seg) * D + 16 * j + 4 * lq) = decay[j];
+        }
+    }
+}
+
 // One token per sequence. Thread (rg, cg) owns columns V cg .. V cg + V - 1 and the state rows rg, rg + R, ...
 constexpr int kLsBatch = 8;     // state rows in flight per thread
 
@@ -499,7 +861,11 @@ extern "C" int swl_linear_chunks(float *qd, float *kd, float *total, float *intr
     const size_t lds = 3ull * swl::kLsTile * dp * sizeof(float);
     const dim3 grid(static_cast<unsigned>(num_tiles), static_cast<unsigned>(num_heads));
     SWL_DISPATCH_DTYPE3(dtype, T, {
-        auto kernel = bonus ? swl::linear_chunks_kernel<T, true> : swl::linear_chunks_kernel<T, false>;
+        // (eight channels of q and k a load, four of the decay)
+        const bool wide = dim % 64 == 0 && swl::aligned16(q) && swl::aligned16(k) && q_stride * sizeof(T) % 16 == 0 && k_stride * sizeof(T) % 16 == 0 &&
+                          (!per_channel || (swl::aligned16(decay) && decay_stride % 4 == 0));
+        auto kernel = wide ? (bonus ? swl::linear_chunks_kernel<T, true, true> : swl::linear_chunks_kernel<T, false, true>)
+                           : (bonus ? swl::linear_chunks_kernel<T, true, false> : swl::linear_chunks_kernel<T, false, false>);
         hipLaunchKernelGGL(kernel, grid, dim3(swl::kLsThreads), lds, static_cast<hipStream_t>(stream), qd, kd, total, intra,
                            static_cast<const T *>(q), q_stride, static_cast<const T *>(k), k_stride, decay, decay_stride,
                            per_channel, k_scale, bonus, q_scale, tile_row0, tile_cnt, num_heads, num_heads / num_qk_heads, dim, dp);
@@ -514,12 +880,13 @@ extern "C" size_t swl_linear_scan_scratch_bytes(int64_t num_seqs, int32_t num_he
     return sizeof(float) * static_cast<size_t>(num_seqs) * num_heads * (states + decays);
 }
 
-extern "C" int swl_linear_scan_segments(float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra,
-                               const void *v, int64_t v_stride, const float *dskip, float *state, int64_t slot_stride,
-                               int64_t s_off, const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0,
-                               const int32_t *tok_pos, const int32_t *tok_state, int32_t num_seqs, int32_t num_heads, int32_t dim,
-                               int32_t vdim, int32_t segments, int32_t seg_tiles, float *scratch, int32_t dtype,
-                                        swl_stream_t stream) {
+/* num_tiles: of the step (bounds the segments that there are; 0: as many for each portion) */
+extern "C" int swl_linear_scan_cut(float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra,
+                                   const void *v, int64_t v_stride, const float *dskip, float *state, int64_t slot_stride, int64_t s_off,
+                                   const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0, const int32_t *tok_pos,
+                                   const int32_t *tok_state, int32_t num_seqs, int32_t num_heads, int32_t dim, int32_t vdim, int32_t segments,
+                                   int32_t seg_tiles, int32_t num_tiles, float *scratch, int32_t dtype, swl_stream_t stream) {
+    if (num_tiles < 0) return SWL_ERR_BAD_ARG;
     if (num_seqs < 0 || num_heads <= 0 || dim <= 0 || vdim <= 0 || segments < 1 || segments > 64) return SWL_ERR_BAD_ARG;
     if (segments > 1 && (seg_tiles < 1 || !scratch)) return SWL_ERR_BAD_ARG;
     if (segments == 1) seg_tiles = 1 << 26;     // (one segment holds every portion)
@@ -532,9 +899,28 @@ extern "C" int swl_linear_scan_segments(float *o, int64_t o_stride, const float 
     const int dp = (dim + 15) / 16 * 16, shares = (vdim + 15) / 16;
     const int64_t units = static_cast<int64_t>(num_seqs) * num_heads, blocks = 8 * ((units + 7) / 8) * shares * segments;
     if (dp > swl::kLsMaxDim || num_heads > 65535 || shares > 65535 || blocks > 0x7fffffffLL) return SWL_ERR_UNSUPPORTED;
+    const hipStream_t on = static_cast<hipStream_t>(stream);
     const int tw = (dp / 16 + swl::kLsWaves - 1) / swl::kLsWaves;       // 1 .. 5
     const dim3 grid(static_cast<unsigned>(blocks));
     float *seg_states = scratch, *seg_decays = scratch ? scratch + units * (segments + 1) * dim * vdim : nullptr;
+    // Rows of values in whole aligned pieces of 16 bytes; states by 32-bit offsets, a tile's rows within 2 GiB
+    const int64_t size = dtype == SWL_F32 ? 4 : 2;
+    if ((dim == 64 || dim == 128) && swl::aligned16(v) && v_stride * size % 16 == 0 && vdim * size % 16 == 0 && static_cast<int64_t>(dim) * vdim < (1LL << 29) &&
+        16 * v_stride * size < (1LL << 31) && 16 * o_stride * 4 < (1LL << 31) && (segments == 1 || swl::aligned16(scratch))) {
+        const int wide = (vdim + 63) / 64;
+        swl::LwParams p = {o, qd, kd, total, intra, v, dskip, state, seg_states, seg_decays, seq_row0, seq_cnt, seq_tile0, tok_pos, tok_state,
+                           o_stride, v_stride, slot_stride, s_off, num_heads, vdim, wide, num_seqs, segments, seg_tiles,
+                           swl::Divisor::of(static_cast<unsigned>(seg_tiles) * swl::kLsTile)};
+        int64_t pieces = static_cast<int64_t>(num_seqs) * segments;
+        if (num_tiles > 0) pieces = std::min<int64_t>(pieces, num_seqs + static_cast<int64_t>(num_tiles) / seg_tiles);
+        const dim3 by_64(static_cast<unsigned>(8 * ((pieces * num_heads + 7) / 8) * wide));
+        SWL_DISPATCH_DTYPE3(dtype, T, {
+            if (segments > 1)
+                hipLaunchKernelGGL(dim == 64 ? (swl::linear_scan_wide_kernel<T, 4, true>) : (swl::linear_scan_wide_kernel<T, 8, true>), by_64, dim3(swl::kLsThreads), 0, on, p);
+            hipLaunchKernelGGL(dim == 64 ? (swl::linear_scan_wide_kernel<T, 4, false>) : (swl::linear_scan_wide_kernel<T, 8, false>), by_64, dim3(swl::kLsThreads), 0, on, p);
+        });
+        return swl::check_launch();
+    }
 #define SWL_LS(N)                                                                                                             \
     case N:                                                                                                                   \
         if (segments > 1)                                                                                                     \
@@ -561,6 +947,16 @@ extern "C" int swl_linear_scan_segments(float *o, int64_t o_stride, const float 
     });
 #undef SWL_LS
     return swl::check_launch();
+}
+
+extern "C" int swl_linear_scan_segments(float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra,
+                               const void *v, int64_t v_stride, const float *dskip, float *state, int64_t slot_stride,
+                               int64_t s_off, const int32_t *seq_row0, const int32_t *seq_cnt, const int32_t *seq_tile0,
+                               const int32_t *tok_pos, const int32_t *tok_state, int32_t num_seqs, int32_t num_heads, int32_t dim,
+                               int32_t vdim, int32_t segments, int32_t seg_tiles, float *scratch, int32_t dtype,
+                                        swl_stream_t stream) {
+    return swl_linear_scan_cut(o, o_stride, qd, kd, total, intra, v, v_stride, dskip, state, slot_stride, s_off, seq_row0, seq_cnt, seq_tile0,
+                               tok_pos, tok_state, num_seqs, num_heads, dim, vdim, segments, seg_tiles, 0, scratch, dtype, stream);
 }
 
 extern "C" int swl_linear_scan(float *o, int64_t o_stride, const float *qd, const float *kd, const float *total, const float *intra,

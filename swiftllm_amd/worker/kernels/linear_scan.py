@@ -29,27 +29,32 @@ def low_rank_decay(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, bias: to
     return out
 
 
-# Segments of a portion: as many as leave SEGMENT_MIN_TILES tiles each and SEGMENT_SLOTS workgroups on the chip, and three at least (two run
-# the first half's keys twice for little). A pass of 4 layers, 8 heads of 128, against whole portions: 1 prompt of 2000 tokens 1555 -> 1257 us (12
-# segments), 2 of 1000 beside 30 decoded tokens 1450 -> 1352 us (4), 4 of 1000 1870 -> 1854 us (3; 1893 with 2, 1900 with 4).
-SEGMENT_MIN_TILES, SEGMENT_SLOTS, SEGMENT_MAX_SCRATCH = 8, 768, 1 << 28
+# Segments of a portion: as many as leave a portion SEGMENT_MIN_TILES tiles each and the chip SEGMENT_SLOTS workgroups, three at least (two run
+# the first half's keys twice for little), and only portions of SEGMENT_PORTION_TILES and more. Heads of 64 and 128 key channels run 64 columns a
+# workgroup, one a CU: all launches of a recurrence, 8 heads of 128 x 128, us for 1, 4, 8 and 16 segments: 1 prompt of 2000 tokens 178, 92, 61, 49;
+# 2 of 1000 beside 30 decoded tokens 102, 62, 56, 66; 4 of 1000 104, 66, 67, 87; 1 of 400 43, 30, 26; 5 of 900 with 16 heads 109, 129, 139. The others
+# run 16 columns a workgroup, three a CU.
+SEGMENT_PORTION_TILES, SEGMENT_MAX_SCRATCH = 24, 1 << 28
+SEGMENT_MIN_TILES, SEGMENT_SLOTS = {True: 3, False: 8}, {True: 256, False: 768}
 
 
 def scan_segments(st: StateRef, heads: int, dim: int, vdim: int):
     """(segments, tiles of one, scratch) of a step's scan; (1, 0, None): portions run whole."""
-    tiles = -(-st.longest // 16)
-    if tiles < 3 * SEGMENT_MIN_TILES:
+    tiles, num_seqs = -(-st.longest // 16), st.seq_row0.shape[0]
+    if tiles < SEGMENT_PORTION_TILES:
         return 1, 0, None
-    long_portions = -(-st.tiles[0].shape[0] // tiles)       # (as if every tile belonged to a portion of the longest's length)
-    segments = min(SEGMENT_SLOTS // (long_portions * heads * -(-vdim // 16)), tiles // SEGMENT_MIN_TILES, 64)
-    if segments < 3:
-        return 1, 0, None
-    seg_tiles = -(-tiles // segments)
-    segments = -(-tiles // seg_tiles)
-    scratch_bytes = _hip.load().swl_linear_scan_scratch_bytes(st.seq_row0.shape[0], heads, dim, vdim, segments)
-    if scratch_bytes > SEGMENT_MAX_SCRATCH:
-        return 1, 0, None
-    return segments, seg_tiles, torch.empty(scratch_bytes // 4, dtype=torch.float32, device=st.pool.device)
+    wide = dim in (64, 128)
+    portions = -(-(st.tiles[0].shape[0] - num_seqs) // (tiles - 1))     # (as if every tile but the portions' first belonged to one of the longest's length)
+    segments = min(SEGMENT_SLOTS[wide] // (max(portions, 1) * heads * -(-vdim // (64 if wide else 16))), tiles // SEGMENT_MIN_TILES[wide], 64)
+    lib = _hip.load()
+    while segments >= 3:
+        seg_tiles = -(-tiles // segments)
+        segments = -(-tiles // seg_tiles)
+        scratch_bytes = lib.swl_linear_scan_scratch_bytes(num_seqs, heads, dim, vdim, segments)
+        if scratch_bytes <= SEGMENT_MAX_SCRATCH:
+            return segments, seg_tiles, torch.empty(scratch_bytes // 4, dtype=torch.float32, device=st.pool.device)
+        segments -= 1
+    return 1, 0, None
 
 
 def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: torch.Tensor, st: StateRef, state_off: int,
@@ -98,10 +103,10 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
               _hip.ptr(bonus), float(q_scale), _hip.ptr(row0), _hip.ptr(cnt), num_tiles, H, G, dim, code, stream)
     o = torch.empty((n, H * vdim), dtype=f32, device=dev)
     segments, seg_tiles, scratch = scan_segments(st, H, dim, vdim)
-    _hip.call("swl_linear_scan_segments", _hip.ptr(o), o.stride(0), _hip.ptr(qd), _hip.ptr(kd), _hip.ptr(total), _hip.ptr(intra),
+    _hip.call("swl_linear_scan_cut", _hip.ptr(o), o.stride(0), _hip.ptr(qd), _hip.ptr(kd), _hip.ptr(total), _hip.ptr(intra),
               _hip.ptr(v), v.stride(0), _hip.ptr(dskip), _hip.ptr(st.pool), st.pool.stride(0), int(state_off),
               _hip.ptr(st.seq_row0), _hip.ptr(st.seq_cnt), _hip.ptr(seq_tile0), _hip.ptr(st.tok_pos), _hip.ptr(st.tok_state),
-              num_seqs, H, dim, vdim, segments, seg_tiles, _hip.ptr(scratch), code, stream)
+              num_seqs, H, dim, vdim, segments, seg_tiles, num_tiles, _hip.ptr(scratch), code, stream)
     if finish is None:
         return o
     out, norm_w, gate, eps, mult = finish

@@ -1,0 +1,88 @@
+"""The linear recurrence of heads with 64 or 128 key channels, 64 columns a workgroup (csrc/linear_scan.hip), against float64: columns that fill no
+workgroup and no wave, portions around a tile's and a segment's end, more portions than a wave counts at once, carried states, operands that
+the wide kernels do not take."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def oracle(q, k, v, decay, s, u=None):
+    """One portion: [n, H, d], [n, H, d], [n, H, dv], [n, H, d], state [H, d, dv] (changed) -> [n, H, dv]; float64."""
+    out = torch.empty_like(v)
+    for t in range(q.shape[0]):
+        kv = k[t].unsqueeze(-1) * v[t].unsqueeze(-2)
+        if u is None:
+            s.mul_(decay[t].unsqueeze(-1)).add_(kv)
+            out[t] = (q[t].unsqueeze(-2) @ s).squeeze(-2)
+        else:
+            out[t] = (q[t].unsqueeze(-2) @ (s + u.unsqueeze(-1) * kv)).squeeze(-2)
+            s.mul_(decay[t].unsqueeze(-1)).add_(kv)
+    return out
+
+
+LONG = [401, 1, 16, 384, 17]
+MANY = [1] * 70 + [390, 2, 375]
+
+
+@pytest.mark.parametrize("lens,H,G,d,dv,bonus,scalar,aligned", [
+    (LONG, 2, 1, 128, 72, False, False, True), (LONG, 3, 3, 64, 8, True, False, True), (MANY, 1, 1, 64, 136, False, True, True), (MANY, 2, 2, 128, 64, True, False, True),
+    (LONG, 2, 2, 128, 72, False, False, False), (LONG, 1, 1, 128, 12, False, True, True), ([1, 15, 33, 16], 2, 1, 128, 128, False, False, True)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_wide_scan(lens, H, G, d, dv, bonus, scalar, aligned, dtype):
+    from swiftllm_amd.worker.kernels import linear_scan
+    from swiftllm_amd.worker.kernels.rms_stream import StateRef
+    g = torch.Generator().manual_seed(d + dv + len(lens))
+    n, off = sum(lens), 8
+    rows, counts, tile0, seq_row0, pos, slots = [], [], [], [], [], []
+    at = 0
+    for s, c in enumerate(lens):
+        seq_row0.append(at)
+        tile0.append(len(rows))
+        for o in range(0, c, 16):
+            rows.append(at + o)
+            counts.append(min(16, c - o))
+        first = 7 * (s % 2)         # (every other sequence has a state)
+        pos += range(first, first + c)
+        slots += [2 * (len(lens) - 1 - s)] * c
+        at += c
+    state = torch.randn(len(lens), H, d, dv, generator=g)
+    pool = torch.full((len(lens), off + H * d * dv), float("nan"))
+    for s in range(len(lens)):
+        if s % 2:
+            pool[len(lens) - 1 - s, off:] = state[s].flatten()
+    pool = pool.cuda()
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")      # noqa: E731
+    st = StateRef(pool, ints(pos), None, ints(slots), None, ints(seq_row0), ints(lens), (ints(rows), ints(counts), ints(tile0)), max(lens))
+    wide = torch.randn(n, 2 * G * d + H * dv + 1, generator=g).to(dtype)
+    if not aligned:
+        wide = wide[:, 1:]
+    elif wide.shape[1] % 8:
+        wide = torch.cat([wide, wide.new_zeros(n, -wide.shape[1] % 8)], dim=1)
+    q, k, v = (wide[:, a:b] for a, b in ((0, G * d), (G * d, 2 * G * d), (2 * G * d, 2 * G * d + H * dv)))
+    decay = torch.rand(n, H if scalar else H * d, generator=g) ** 0.02
+    decay[torch.rand(decay.shape, generator=g) < 0.002] = 0.0
+    scale = torch.rand(n, H, generator=g) if scalar else None
+    skip = torch.randn(H, generator=g) if scalar else None
+    u = torch.randn(H, d, generator=g) if bonus else None
+    dev = wide.cuda() if aligned else torch.cat([wide.new_zeros(n, 1), wide], dim=1).cuda()[:, 1:]
+    part = lambda a, b: dev[:, a:b]     # noqa: E731
+    y = linear_scan.linear_recurrence(part(0, G * d), part(G * d, 2 * G * d), part(2 * G * d, 2 * G * d + H * dv), decay.cuda(), st, off, H, d, dv, q_scale=0.3,
+                                      bonus=u.cuda() if bonus else None, k_scale=scale.cuda() if scalar else None,
+                                      dskip=skip.cuda() if scalar else None, num_qk_heads=G).cpu().double()
+    got_state = pool.cpu()[:, off:].double().view(len(lens), H, d, dv)
+    heads = lambda x: x.double().view(n, G, d).repeat_interleave(H // G, dim=1)     # noqa: E731
+    qq, kk, vv = 0.3 * heads(q), heads(k), v.double().reshape(n, H, dv)
+    if scalar:
+        kk = kk * scale.double().unsqueeze(-1)
+    dd = decay.double().view(n, H, -1).expand(n, H, d)
+    at = 0
+    for s, c in enumerate(lens):
+        S = state[s].double() if s % 2 else torch.zeros(H, d, dv, dtype=torch.float64)
+        want = oracle(qq[at:at + c], kk[at:at + c], vv[at:at + c], dd[at:at + c], S, u.double() if bonus else None)
+        if scalar:
+            want = want + skip.double().view(1, H, 1) * vv[at:at + c]
+        # fp32 products and sums: the bound of the walk without segments
+        assert (y[at:at + c] - want.reshape(c, -1)).abs().max() < 3e-5 * max(1.0, float(want.abs().max())), (s, c)
+        assert (got_state[len(lens) - 1 - s] - S).abs().max() < 3e-5 * max(1.0, float(S.abs().max())), (s, c)
+        at += c
