@@ -282,6 +282,193 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_grouped_kernel(int32_t 
     }
 }
 
+// Routers of up to eight experts for steps of many tokens: a wave takes two or four tokens, whose rows meet each load of the router's, and the choice is
+// made by a lane a token from registers. What bounds it is vector work (eight multiplies and adds a quad and expert, which stay apart) and the
+// chain of a choice; a workgroup a token, as above, also waits for its row, its two meetings and the router's rows (32 KiB of 1024 columns a token from
+// L2). The same sums in the same order, the same bits.
+// us, bf16, two of eight, before -> now: 7452 tokens of 1024 plain 13.6 -> 9.7, all scores 13.5 -> 11.3, in groups 17.5 -> 12.3; 3657 of 2048 12.0 -> 9.8, 11.9 ->
+// 11.3, 13.6 -> 11.9; 16000 of 2048 40 -> 22, 39 -> 23, 44 -> 25; fp32, 7452 of 2048 29 -> 13.
+constexpr int kRouteFew = 8;
+
+struct RouteParams {
+    int32_t *idx;
+    float *w;
+    const void *h;
+    const float *router, *bias;     // (or the correction)
+    int64_t num_tokens;
+    int width, experts, top, all_scores, count, keep, normalize;
+    float scale;
+};
+
+template <typename T, bool GROUPED, int N>
+__global__ __launch_bounds__(kMoeThreads) void moe_route_few_kernel(RouteParams p) {
+    constexpr int E = kRouteFew;
+    const int lane = threadIdx.x & 63, experts = p.experts;
+    const int64_t t0 = (static_cast<int64_t>(blockIdx.x) * kMoeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * N;
+    if (t0 >= p.num_tokens) return;
+    const T *x[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) x[n] = static_cast<const T *>(p.h) + min(t0 + n, p.num_tokens - 1) * p.width;
+    float a[N][E];
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int e = 0; e < E; ++e) a[n][e] = 0.f;
+    vec4_t<T> u[2][N];
+    float4_t r[2][E];
+    auto load = [&](int i, vec4_t<T> (&u)[N], float4_t (&r)[E]) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) u[n] = *reinterpret_cast<const vec4_t<T> *>(x[n] + i);
+#pragma unroll
+        for (int e = 0; e < E; ++e) r[e] = *reinterpret_cast<const float4_t *>(p.router + static_cast<int64_t>(min(e, experts - 1)) * p.width + i);
+    };
+    auto add = [&](const vec4_t<T> (&u)[N], const float4_t (&r)[E]) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const float u0 = to_f(u[n][0]), u1 = to_f(u[n][1]), u2 = to_f(u[n][2]), u3 = to_f(u[n][3]);
+#pragma unroll
+            for (int e = 0; e < E; ++e) a[n][e] += (u0 * r[e][0] + u1 * r[e][1]) + (u2 * r[e][2] + u3 * r[e][3]);
+        }
+    };
+    const int last = p.width - 4;       // (columns past the row: the last ones again, which nobody adds)
+    load(min(lane * 4, last), u[0], r[0]);
+    for (int i = lane * 4; i - lane * 4 < p.width; i += 512) {
+        load(min(i + 256, last), u[1], r[1]);
+        if (i < p.width) add(u[0], r[0]);
+        load(min(i + 512, last), u[0], r[0]);
+        if (i + 256 < p.width) add(u[1], r[1]);
+    }
+    // lane n: token n's logits
+    float v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        v[e] = 0.f;
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const float sum = wave_allreduce_sum(a[n][e]);
+            v[e] = lane == n ? sum : v[e];
+        }
+    }
+    const int64_t t = t0 + lane;
+    if (lane >= N || t >= p.num_tokens) return;
+    // the largest of eight, ties to the lowest (NaN and -inf never win: 0x7fffffff)
+    auto argmax = [](const float (&s)[E], float &best, int &besti) {
+        best = -INFINITY;
+        besti = 0x7fffffff;
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (s[e] > best) {
+                best = s[e];
+                besti = e;
+            }
+    };
+    auto take = [](float (&s)[E], int i) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) s[e] = e == i ? -INFINITY : s[e];
+    };
+    float c[E], mine[E], denom = 0.f;       // c: choice
+    int mine_idx[E];
+    float all_max = -INFINITY, all_den = 0.f, chosen_max = 0.f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        if constexpr (GROUPED) {
+            v[e] = 1.0f / (1.0f + expf(-v[e]));
+            c[e] = e < experts ? v[e] + (p.bias ? p.bias[e] : 0.f) : -INFINITY;
+        } else {
+            c[e] = e < experts ? v[e] + (p.bias ? p.bias[e] : 0.f) : -INFINITY;
+        }
+    }
+    if constexpr (GROUPED) {
+        if (p.count > 1 && p.keep < p.count) {
+            const int per = experts / p.count;
+            float g[E];
+            unsigned kept = 0;
+            auto scores = [&](int size) {       // a group's score: its two largest choice scores (one, in groups of one)
+#pragma unroll
+                for (int i = 0; i < E; ++i) {
+                    float a0 = -INFINITY, b0 = -INFINITY;
+#pragma unroll
+                    for (int e = 0; e < E; ++e) {
+                        if (e >= i * size && e < (i + 1) * size) {
+                            if (c[e] > a0) {
+                                b0 = a0;
+                                a0 = c[e];
+                            } else if (c[e] > b0) {
+                                b0 = c[e];
+                            }
+                        }
+                    }
+                    g[i] = i < p.count ? size > 1 ? a0 + b0 : a0 : -INFINITY;
+                }
+            };
+            auto leave = [&](int size) {
+#pragma unroll
+                for (int e = 0; e < E; ++e)
+                    if (!(kept >> e / size & 1)) c[e] = -INFINITY;
+            };
+            if (per == 2) scores(2);        // (sizes that are known leave few of the comparisons)
+            else if (per == 4) scores(4);
+            else scores(per);
+            for (int j = 0; j < p.keep; ++j) {
+                float best;
+                int besti;
+                argmax(g, best, besti);
+                take(g, besti);
+                if (besti < E) kept |= 1u << besti;
+            }
+            if (per == 2) leave(2);
+            else if (per == 4) leave(4);
+            else leave(per);
+        }
+    } else if (p.all_scores) {      // (sums in the order of a wave's exchange)
+        float q[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) all_max = e < experts ? fmaxf(all_max, c[e]) : all_max;
+#pragma unroll
+        for (int e = 0; e < E; ++e) q[e] = e < experts ? expf(c[e] - all_max) : 0.f;
+        all_den = ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+    }
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        if (j >= p.top) break;
+        float best;
+        int besti;
+        argmax(c, best, besti);
+        if (besti >= experts) besti = 0;        // (as above)
+        if constexpr (GROUPED) {
+            mine[j] = v[0];
+#pragma unroll
+            for (int e = 1; e < E; ++e) mine[j] = e == besti ? v[e] : mine[j];
+        } else {
+            if (j == 0) chosen_max = p.all_scores ? all_max : best;
+            mine[j] = expf(best - chosen_max);
+        }
+        denom += mine[j];
+        mine_idx[j] = besti;
+        take(c, besti);
+    }
+    const float mult = GROUPED ? p.normalize ? 1.0f / (denom + 1e-20f) : 1.0f : p.all_scores ? p.scale / all_den : 1.0f / denom;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        if (j >= p.top) break;
+        p.idx[t * p.top + j] = mine_idx[j];
+        p.w[t * p.top + j] = mine[j] * mult;
+    }
+}
+
+// From 3072 tokens on: 2048 of 1024 columns in groups 8.0 us a workgroup a token, 9.1 so; 3657 11.2 and 9.4. Four tokens a wave from 4609 on: 3657 of 1024
+// 7.4 with two and 8.0 with four, 4499 9.2 and 9.6, 7452 10.5 and 9.7.
+constexpr int64_t kRouteFewTokens = 3072, kRouteFourTokens = 4609;
+template <typename T, bool GROUPED>
+bool route_few(const RouteParams &p, hipStream_t s) {
+    if (p.num_tokens < kRouteFewTokens || p.experts > kRouteFew || p.width % 4 || !aligned16(p.router) || (reinterpret_cast<uintptr_t>(p.h) & (4 * sizeof(T) - 1))) return false;
+    const int each = p.num_tokens < kRouteFourTokens ? 2 : 4;
+    const dim3 grid(static_cast<unsigned>((p.num_tokens + each * kMoeWaves - 1) / (each * kMoeWaves)));
+    if (each == 2) hipLaunchKernelGGL((moe_route_few_kernel<T, GROUPED, 2>), grid, dim3(kMoeThreads), 0, s, p);
+    else hipLaunchKernelGGL((moe_route_few_kernel<T, GROUPED, 4>), grid, dim3(kMoeThreads), 0, s, p);
+    return true;
+}
+
 // The per-assignment kernels: every (token, chosen expert) streams its expert's rows. Bound by latency at decode sizes (3 tokens, two
 // experts of 1024 x 1024, fp32: 25 MB), so a workgroup owns sixteen outputs and a wave four rows at a time, whose loads are in flight
 // together. That shape: up 115 and down 228 us with 64 outputs a workgroup and one row
@@ -734,7 +921,9 @@ extern "C" int swl_moe_route(int32_t *idx_out, float *w_out, const void *h, cons
     if (!idx_out || !w_out || !h || !router || !bias) return SWL_ERR_BAD_ARG;
     const size_t lds = (static_cast<size_t>(width) + experts) * 4;
     if (num_tokens > 0x7fffffffLL || lds > 64 * 1024) return SWL_ERR_UNSUPPORTED;
+    const swl::RouteParams few = {idx_out, w_out, h, router, bias, num_tokens, width, experts, top, 0, 1, 1, 0, 1.0f};
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        if (swl::route_few<T, false>(few, static_cast<hipStream_t>(stream))) return swl::check_launch();
         hipLaunchKernelGGL((swl::moe_route_kernel<T>), dim3(static_cast<unsigned>(num_tokens)), dim3(swl::kMoeThreads),
                            lds, static_cast<hipStream_t>(stream), idx_out, w_out, static_cast<const T *>(h), router, bias,
                            width, experts, top, 0, 1.0f);
@@ -750,7 +939,9 @@ extern "C" int swl_moe_route_scores(int32_t *idx_out, float *w_out, const void *
     if (!idx_out || !w_out || !h || !router) return SWL_ERR_BAD_ARG;
     const size_t lds = (static_cast<size_t>(width) + experts) * 4;
     if (num_tokens > 0x7fffffffLL || lds > 64 * 1024) return SWL_ERR_UNSUPPORTED;
+    const swl::RouteParams few = {idx_out, w_out, h, router, bias, num_tokens, width, experts, top, 1, 1, 1, 0, scale};
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        if (swl::route_few<T, false>(few, static_cast<hipStream_t>(stream))) return swl::check_launch();
         hipLaunchKernelGGL((swl::moe_route_kernel<T>), dim3(static_cast<unsigned>(num_tokens)), dim3(swl::kMoeThreads),
                            lds, static_cast<hipStream_t>(stream), idx_out, w_out, static_cast<const T *>(h), router, bias,
                            width, experts, top, 1, scale);
@@ -848,7 +1039,9 @@ extern "C" int swl_moe_route_grouped(int32_t *idx_out, float *w_out, const void 
     if (!idx_out || !w_out || !h || !router) return SWL_ERR_BAD_ARG;
     const size_t lds = (static_cast<size_t>(width) + 2 * experts + 2 * group_count) * 4;
     if (num_tokens > 0x7fffffffLL || lds > 64 * 1024) return SWL_ERR_UNSUPPORTED;
+    const swl::RouteParams few = {idx_out, w_out, h, router, correction, num_tokens, width, experts, top, 0, group_count, group_keep, normalize, 1.0f};
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        if (swl::route_few<T, true>(few, static_cast<hipStream_t>(stream))) return swl::check_launch();
         hipLaunchKernelGGL((swl::moe_route_grouped_kernel<T>), dim3(static_cast<unsigned>(num_tokens)),
                            dim3(swl::kMoeThreads), lds, static_cast<hipStream_t>(stream), idx_out, w_out,
                            static_cast<const T *>(h), router, correction, width, experts, top, group_count, group_keep,
