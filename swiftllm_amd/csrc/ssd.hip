@@ -230,6 +230,53 @@ __global__ __launch_bounds__(kSsThreads) void gated_group_rmsnorm_kernel(T *out,
     }
 }
 
+// The same with eight columns a thread, N times, kept in registers between the sum and the result.
+// Bound by memory: 3657 tokens of 2048 columns, bf16 20.2 -> 12.8 us (4.7 TB/s; column by column the gate and y were read, and the sigmoid made, twice), by latency
+// in short steps: 32 tokens 5.1 -> 2.9.
+template <typename T, int N>
+__global__ __launch_bounds__(kSsThreads) void gated_group_rmsnorm_wide_kernel(T *out, const float *y, const T *gate, int64_t gate_stride, const float *w, float eps, int cols,
+                                                                              int part, int64_t out_stride) {
+    __shared__ float red[kSsThreads / 64];
+    const int64_t t = blockIdx.x;
+    const int c0 = blockIdx.y * part, step = blockDim.x * 8, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    float4_t x[N][2];
+    vec8_t<T> z[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) {       // (columns past the part: its last ones again, left out below)
+        const int c = c0 + min(static_cast<int>(threadIdx.x) * 8 + n * step, part - 8);
+        x[n][0] = *reinterpret_cast<const float4_t *>(y + t * cols + c);
+        x[n][1] = *reinterpret_cast<const float4_t *>(y + t * cols + c + 4);
+        z[n] = load8(gate + t * gate_stride + c);
+    }
+    float v[N][8], ss = 0.f;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        const bool in = static_cast<int>(threadIdx.x) * 8 + n * step < part;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float g = to_f(z[n][e]);
+            v[n][e] = x[n][e >> 2][e & 3] * (g * ss_sigmoid(g));
+            ss += in ? v[n][e] * v[n][e] : 0.f;
+        }
+    }
+    ss = wave_allreduce_sum(ss);
+    if (lane == 0) red[wave] = ss;
+    __syncthreads();
+    ss = 0.f;
+    for (int i = 0; i < static_cast<int>(blockDim.x) / 64; ++i) ss += red[i];
+    const float r = 1.0f / sqrtf(ss / static_cast<float>(part) + eps);
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+        const int c = static_cast<int>(threadIdx.x) * 8 + n * step;
+        if (c >= part) continue;
+        const float4_t w0 = *reinterpret_cast<const float4_t *>(w + c0 + c), w1 = *reinterpret_cast<const float4_t *>(w + c0 + c + 4);
+        vec8_t<T> o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = to_t<T>(v[n][e] * r * (e < 4 ? w0[e & 3] : w1[e & 3]));
+        store8(out + t * out_stride + c0 + c, o);
+    }
+}
+
 template <int L>
 int launch_ssd(int ds, dim3 grid, dim3 block, size_t lds, hipStream_t s, float *y, const float *xbc, const float *dt,
                const float *decay, const float *dskip, float *state, int64_t slot_stride, int64_t s_off,
@@ -326,6 +373,15 @@ extern "C" int swl_gated_group_rmsnorm(void *out, int64_t out_stride, const floa
     if (!out || !y || !gate || !w) return SWL_ERR_BAD_ARG;
     if (num_tokens > 0x7fffffffLL || groups > 65535) return SWL_ERR_UNSUPPORTED;
     SWL_DISPATCH_DTYPE3(dtype, T, {
+        // (parts of whole aligned pieces of eight columns, up to 8192)
+        const int part = cols / groups;
+        if (part % 8 == 0 && part <= 8192 && cols % 4 == 0 && swl::aligned16(out) && swl::aligned16(y) && swl::aligned16(gate) && swl::aligned16(w) &&
+            gate_stride * sizeof(T) % 16 == 0 && out_stride * sizeof(T) % 16 == 0) {
+            const auto kernel = part <= 2048 ? swl::gated_group_rmsnorm_wide_kernel<T, 1> : part <= 4096 ? swl::gated_group_rmsnorm_wide_kernel<T, 2> : swl::gated_group_rmsnorm_wide_kernel<T, 4>;
+            hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(num_tokens), groups), dim3(part < 2048 ? (part / 8 + 63) / 64 * 64 : swl::kSsThreads), 0,
+                               static_cast<hipStream_t>(stream), static_cast<T *>(out), y, static_cast<const T *>(gate), gate_stride, w, eps, cols, part, out_stride);
+            return swl::check_launch();
+        }
         hipLaunchKernelGGL((swl::gated_group_rmsnorm_kernel<T>), dim3(static_cast<unsigned>(num_tokens), groups),
                            dim3(swl::kSsThreads), 0, static_cast<hipStream_t>(stream), static_cast<T *>(out), y,
                            static_cast<const T *>(gate), gate_stride, w, eps, cols, cols / groups, out_stride);
