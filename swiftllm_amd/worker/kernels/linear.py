@@ -455,6 +455,14 @@ def linear_splitk(a: torch.Tensor, w: torch.Tensor, always: bool = False):
     """Like linear(a, w, skinny=True) but returns SplitKPartials when the kernel splits K (the caller
     hands them to a fused consumer); falls through to `linear` otherwise. `always`: also return the
     partial form (a single fp32 slab) when K is not split — for consumers that only take slabs."""
+    tile = _mid_tile(a, w) if a.dim() == 2 and 64 < a.shape[0] <= _WIDE_MAX_M else None
+    if tile is not None:
+        shape, ks = tile
+        (m, k), n = a.shape, w.shape[0]
+        ws = _workspace(a.device, ks * m * n * 4)
+        _hip.call("swl_gemm_tile_partial", _hip.ptr(ws), ws.numel() * 4, _hip.ptr(a), _hip.ptr(w), m, n, k, a.stride(0), ks, shape,
+                  _hip.dtype_code(a.dtype), _hip.stream())
+        return SplitKPartials(ws, ks, m, n, a.dtype)
     if _wide_ok(a, w):                          # large batch: slabs for the add+norm / slab-fed attention consumers
         m, k = a.shape
         n = w.shape[0]
@@ -488,6 +496,29 @@ def linear_splitk(a: torch.Tensor, w: torch.Tensor, always: bool = False):
                       _row_stride(a), ks, _hip.dtype_code(a.dtype), _hip.stream())
             return SplitKPartials(ws, ks, m, n, a.dtype)
     return linear(a, w, skinny=True)
+
+
+def _mid_tile(a: torch.Tensor, w: torch.Tensor):
+    """(tile of kTileShapes, shares of K) where the tiled kernel serves the slabs of 65 to 256 decoded tokens, else None: matrices of 16 million
+    elements and more with at most 8192 rows, which it brings to LDS in larger pieces, and earlier, than gemm_wide.hip. By the 32-token buckets of
+    the replay cache (a replay of 224 rows and an eager step of 200 have the same bits). us, bf16, cold weights, gemm_wide.hip with its
+    shares -> this with its: 6144 x 4096 96 tokens 16.1 (4) -> 15.0 (4), 120 17.3 -> 15.7, 160 20.9 -> 17.2, 200 25.1 -> 22.4 (2), 256 26.8 -> 24.3 (2);
+    4096 x 4096 14.7 (4) -> 12.6 (4), 15.6 -> 13.2, 16.4 (8) -> 14.3, 19.0 (8) -> 15.7, 20.6 (8) -> 16.6; 4096 x 14336 30.0 (8) -> 26.7 (8), 29.2 -> 27.9, 34.4 ->
+    29.1, then level (39.8 and 38.8): left where it is. Wider matrices are slower so: 32000 x 4096 51.8 and 61.7, 28672 x 4096 52.2 and 58.5. Smaller
+    ones gain too (2048 x 8192, 160 tokens 19.4 -> 14.5), in steps that wait for the host."""
+    (m, k), n = a.shape, w.shape[0]
+    if n > 8192 or n * k < 1 << 24 or w.shape[1] != k or a.dtype != w.dtype or a.dtype not in (torch.float16, torch.bfloat16):
+        return None
+    tokens, long = route_tune.bucket_of(m), k >= 2 * n
+    if long and tokens > 160:
+        return None
+    shares = 8 if long else 2 if tokens > 160 and n > 4096 else 4
+    if not (a.is_cuda and a.stride(1) == 1 and a.stride(0) % 8 == 0 and w.is_contiguous()) or n % 128 or k % (128 * shares) or (a.data_ptr() | w.data_ptr()) % 16 \
+            or not _hip.load().swl_gemm_tile_supported(m, n, k, a.stride(0), n, TILE_NONE, _hip.dtype_code(a.dtype)):
+        return None
+    # 128 x 128; 160 x 128 where that is one row of tiles instead of two; 64 x 128 where there are few
+    shape = 7 if tokens == 160 and (long or n > 4096) else 11 if tokens <= 128 and not long and n <= 4096 else 10
+    return shape, shares
 
 
 def row_scaled_silu_gate_ok(a: torch.Tensor, w_up_gate: torch.Tensor) -> bool:

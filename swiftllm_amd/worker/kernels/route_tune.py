@@ -40,7 +40,7 @@ _device_key_cache = {}
 
 
 def table_wide_wins(m: int, n: int, k: int) -> bool:
-    """Llama-3-8B widths, bf16, MI355X. us ours / library at M = 96, 128, 160, 192, 224, 256, captured, weights cycled through 1.2 GB, the launch
+    """Products whose slabs the tiled kernel serves (kernels/linear.py, _mid_tile) do not come here. Llama-3-8B widths, bf16, MI355X. us ours / library at M = 96, 128, 160, 192, 224, 256, captured, weights cycled through 1.2 GB, the launch
     that adds the K shares included (the consumers of a decode step add them themselves):
         down     32/64  33/76  42/85  40/103  49/60  49/62         -> always
         qkv      22/23  25/26  27/28  27/33   31/37  32/40         -> always
