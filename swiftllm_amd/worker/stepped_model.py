@@ -126,7 +126,8 @@ class SteppedModel:
         self.kv_pool = saved
         torch.cuda.synchronize()
         free_memory, total_memory = torch.cuda.mem_get_info()
-        peak = total_memory - free_memory + self._scratch_bytes(num_tokens, batch)
+        # (TILE_MAX_SLAB_BYTES: of a smaller step, whose products' sums are split)
+        peak = total_memory - free_memory + self._scratch_bytes(num_tokens, batch) + TILE_MAX_SLAB_BYTES
         usable = total_memory * ecfg.gpu_mem_utilization
         print(f"[Model.profile] GPU total memory: {total_memory / GB:.2f} GB, runtime peak memory: {peak / GB:.2f} GB")
         if usable < peak:
@@ -138,9 +139,9 @@ class SteppedModel:
 
     def _scratch_bytes(self, num_tokens: int, batch: int) -> int:
         """The most scratch that a launch of a step of these sizes takes beside what the forged step shows: of attention, which it
-        leaves out without a pool, and of products whose sums a smaller step splits. (Designs whose recurrences take some by the lengths of the portions add it: the forged ones are
+        leaves out without a pool. (Designs whose recurrences take some by the lengths of the portions add it: the forged ones are
         equal, and may all be short.)"""
-        return SHARE_MAX_SCRATCH + TILE_MAX_SLAB_BYTES
+        return SHARE_MAX_SCRATCH
 
     @torch.inference_mode()
     def init_kvcache_and_swap(self, num_blocks: int):
