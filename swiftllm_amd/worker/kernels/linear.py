@@ -251,7 +251,7 @@ _wide_silu_wins = route_tune.table_wide_silu_wins
 
 
 def linear(a: torch.Tensor, w: torch.Tensor, skinny: bool = False) -> torch.Tensor:
-    """a[T, in] @ w[out, in]^T -> [T, out] (fp32 accumulation, one rounding)."""
+    """a[T, in] @ w[out, in]^T -> [T, out], contiguous (fp32 accumulation, one rounding)."""
     if skinny and _wide_ok(a, w):
         return _launch_wide(a, w)
     if skinny and _mid_ok(a, w):
@@ -275,7 +275,8 @@ def linear(a: torch.Tensor, w: torch.Tensor, skinny: bool = False) -> torch.Tens
                   ws.numel() * 4 if ws is not None else 0, m, n, k, _row_stride(a), n, 0,
                   _hip.dtype_code(a.dtype), _hip.stream())
         return out
-    y = linear_tile(a, w) if skinny else None
+    # (rows of a result lie one behind the other, which many of its readers count on: linear_tile's would not, where they are no multiple of 8 long)
+    y = linear_tile(a, w) if skinny and w.shape[0] % 8 == 0 else None
     return y if y is not None else _blas_linear(a, w)
 
 
