@@ -500,22 +500,33 @@ def linear_splitk(a: torch.Tensor, w: torch.Tensor, always: bool = False):
 
 
 def _mid_tile(a: torch.Tensor, w: torch.Tensor):
-    """(tile of kTileShapes, shares of K) where the tiled kernel serves the slabs of 65 to 256 decoded tokens, else None: matrices of 16 million
-    elements and more with at most 8192 rows, which it brings to LDS in larger pieces, and earlier, than gemm_wide.hip. By the 32-token buckets of
-    the replay cache (a replay of 224 rows and an eager step of 200 have the same bits). us, bf16, cold weights, gemm_wide.hip with its
-    shares -> this with its: 6144 x 4096 96 tokens 16.1 (4) -> 15.0 (4), 120 17.3 -> 15.7, 160 20.9 -> 17.2, 200 25.1 -> 22.4 (2), 256 26.8 -> 24.3 (2);
-    4096 x 4096 14.7 (4) -> 12.6 (4), 15.6 -> 13.2, 16.4 (8) -> 14.3, 19.0 (8) -> 15.7, 20.6 (8) -> 16.6; 4096 x 14336 30.0 (8) -> 26.7 (8), 29.2 -> 27.9, 34.4 ->
-    29.1, then level (39.8 and 38.8): left where it is. Wider matrices are slower so: 32000 x 4096 51.8 and 61.7, 28672 x 4096 52.2 and 58.5. Smaller
-    ones gain too (2048 x 8192, 160 tokens 19.4 -> 14.5), in steps that wait for the host."""
+    """(tile of kTileShapes, shares of K) where the tiled kernel serves the slabs of 65 to 256 decoded tokens, else None: matrices of 2^24 elements and
+    more with at most 8192 rows, which it brings to LDS in larger pieces, and earlier, than gemm_wide.hip. By the 32-token buckets of
+    the replay cache (a replay of 224 rows and an eager step of 200 have the same bits).
+    Product and the residual step behind it, us, bf16 (fp16 within 2 %), cold weights, for 72 / 128 / 192 / 256 tokens: gemm_wide.hip, library -> this:
+        4096 x 4096    19.0 22.0 25.2 28.7, 19.6 28.0 36.5 26.4 -> 17.3 18.8 20.1 22.5      4096 x 6144  24.2 27.6 29.9 33.5, 26.8 39.2 51.9 33.3 -> 23.4 25.6 25.7 29.0
+        6144 x 4096    23.0 26.6 29.3 33.9, 27.3 30.1 38.8 45.0 -> 21.9 23.8 28.5 31.0      8192 x 4096  26.8 29.5 34.8 38.0, 30.6 33.2 41.7 47.3 -> 24.7 26.8 33.3 35.3
+        7168 x 3072    24.8 28.4 29.7 33.3, 24.6 27.2 33.8 38.6 -> 21.2 23.9 26.8 29.5      8192 x 2048  20.8 24.0 27.5 30.4, 20.3 21.6 28.5 30.8 -> 18.7 20.3 22.0 24.9
+    and of long sums for 72 / 128 / 160:
+        2048 x 8192    18.4 21.3 25.3, 23.6 23.6 28.9 -> 17.3 19.0 20.3                     4096 x 8192  25.1 28.4 31.2, 31.4 46.8 52.7 -> 23.1 25.8 28.1
+        4096 x 14336   33.1 36.0 45.1, 52.8 79.5 87.9 -> 31.7 35.7 40.4 (then level)        3072 x 12288 27.4 31.3 34.1, 60.8 69.2 47.2 -> 27.8 31.1 33.2
+    These take it whatever was measured at load for the other two (route_tune: rows of `linear`, and the slabs of what is not listed here). Where rows
+    and sums are both longer, and where long sums have fewer rows or more columns, gemm_wide.hip is as fast or faster, and this stands in for the library only,
+    below 2^26 elements:
+        5120 x 5120    25.1 29.6 31.8 38.7, 26.1 36.9 46.2 54.8 -> 25.4 27.5 33.0 37.6      7168 x 7168  32.9 36.9 43.1 50.4, 41.1 49.0 62.7 72.5 -> 32.4 37.4 45.6 50.6
+        5120 x 10240   37.1 42.7 45.4, 44.1 63.5 71.1 -> 39.8 46.5 50.3                     1024 x 16384 18.6 20.6 22.8, 24.6 29.3 36.8 -> 24.0 26.0 28.1
+        8192 x 8192    36.6 39.6 49.2 55.3, 43.2 55.7 72.5 83.4 -> 45.0 47.9 56.3 60.6      8192 x 16384 58.7 64.5 75.2, 75.2 101.6 113.0 -> 84.1 86.1 90.3
+    Wider matrices are slower so: 32000 x 4096 51.8 (product alone) and 61.7, 28672 x 4096 52.2 and 58.5. Smaller ones gain too, in steps that wait for the host."""
     (m, k), n = a.shape, w.shape[0]
-    if n > 8192 or n * k < 1 << 24 or w.shape[1] != k or a.dtype != w.dtype or a.dtype not in (torch.float16, torch.bfloat16):
+    if n > 8192 or not 1 << 24 <= n * k < 1 << 26 or w.shape[1] != k or a.dtype != w.dtype or a.dtype not in (torch.float16, torch.bfloat16):
         return None
     tokens, long = route_tune.bucket_of(m), k >= 2 * n
     if long and tokens > 160:
         return None
+    first = 2048 <= n <= 4096 and k <= 14336 if long else min(n, k) <= 4096
     shares = 8 if long else 2 if tokens > 160 and n > 4096 else 4
     if not (a.is_cuda and a.stride(1) == 1 and a.stride(0) % 8 == 0 and w.is_contiguous()) or n % 128 or k % (128 * shares) or (a.data_ptr() | w.data_ptr()) % 16 \
-            or not _hip.load().swl_gemm_tile_supported(m, n, k, a.stride(0), n, TILE_NONE, _hip.dtype_code(a.dtype)):
+            or not _hip.load().swl_gemm_tile_supported(m, n, k, a.stride(0), n, TILE_NONE, _hip.dtype_code(a.dtype)) or (not first and _wide_ok(a, w)):
         return None
     # 128 x 128; 160 x 128 where that is one row of tiles instead of two; 64 x 128 where there are few
     shape = 7 if tokens == 160 and (long or n > 4096) else 11 if tokens <= 128 and not long and n <= 4096 else 10

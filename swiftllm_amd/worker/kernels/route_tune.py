@@ -13,6 +13,8 @@ data-parallel deployment must answer alike.
     is written next to the checkpoint (`<model_path>/swiftllm_amd_routes.json`; `SWIFTLLM_ROUTE_CACHE` overrides, and a
     read-only model directory falls back to ~/.cache/swiftllm_amd/) under a lock file, so the first replica of a node
     measures and every other replica READS the same answer;
+  * slabs of some classes are neither's: kernels/linear.py's _mid_tile asks for sizes alone and comes first. The answers here still
+    serve these classes where rows are asked for;
   * `decide()` is a pure lookup: a class nobody measured goes to the library (deterministic), it never times anything,
     takes no lock and asks the driver for nothing;
   * `SWIFTLLM_ROUTE_TUNE=table` pins the measured table for every shape (tests that assert WHICH kernel ran), `=off` sends
@@ -40,8 +42,8 @@ _device_key_cache = {}
 
 
 def table_wide_wins(m: int, n: int, k: int) -> bool:
-    """Products whose slabs the tiled kernel serves (kernels/linear.py, _mid_tile) do not come here. Llama-3-8B widths, bf16, MI355X. us ours / library at M = 96, 128, 160, 192, 224, 256, captured, weights cycled through 1.2 GB, the launch
-    that adds the K shares included (the consumers of a decode step add them themselves):
+    """(For rows, and for slabs where kernels/linear.py's _mid_tile does not take them first.) Llama-3-8B widths, bf16, MI355X. us ours / library at
+    M = 96, 128, 160, 192, 224, 256, captured, weights cycled through 1.2 GB, the launch that adds the K shares included (the consumers of a decode step add them themselves):
         down     32/64  33/76  42/85  40/103  49/60  49/62         -> always
         qkv      22/23  25/26  27/28  27/33   31/37  32/40         -> always
         o        19/22  21/25  22/27  24/33   26/22  28/23         -> up to 192
