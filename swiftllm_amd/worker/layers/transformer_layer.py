@@ -295,6 +295,7 @@ class LlamaTransformerLayer:
 
     def _forward_after_attention(self, input_embds, residual_buf, fast: bool, st):
         cfg, w = self.model_config, self.weight
+        slabs = self.skinny and getattr(self.engine_config, "fuse_splitk_consumers", True)
         if (fast and st is not None and self._rows_applies(st, residual_buf, w.o_proj, input_embds, self.ROWS_O_MAX_M)
                 and nf_ok(residual_buf, w.up_gate_proj, w.ffn_norm) and w.up_gate_proj.shape[0] % 64 == 0):
             # o_proj adds itself into the residual; the SiLU-gate GEMM normalises the raw rows on the fly
@@ -329,7 +330,7 @@ class LlamaTransformerLayer:
             else:
                 fused_add_rmsnorm_inplace(attn_out, residual_buf, w.ffn_norm, cfg.rms_norm_eps)
         else:
-            partials = linear_tile_partial(input_embds, w.o_proj) if self.skinny else None
+            partials = linear_tile_partial(input_embds, w.o_proj) if slabs else None
             if partials is not None:    # (prompt-sized, few tiles)
                 attn_out = fused_add_rmsnorm_from_splitk(partials, residual_buf, w.ffn_norm, cfg.rms_norm_eps)
             else:
@@ -344,5 +345,5 @@ class LlamaTransformerLayer:
             act = up_gate[:, :cfg.ffn_inter_dim]
         if fast:
             return linear_splitk(act, w.down_proj)
-        partials = linear_tile_partial(act, w.down_proj) if self.skinny else None
+        partials = linear_tile_partial(act, w.down_proj) if slabs else None
         return linear(act, w.down_proj, self.skinny) if partials is None else partials
