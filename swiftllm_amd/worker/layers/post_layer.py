@@ -16,8 +16,8 @@ class LlamaPostLayer:
         self.logits_tap = None
         self.last_logits = None     # the logits tensor of the most recent (eager or captured) forward
 
-    def forward(self, input_embds: torch.Tensor, infer_state) -> torch.Tensor:
-        """[num_tokens, hidden] -> next-token ids int64 [batch_size] (argmax; ties -> lowest id)."""
+    def last_rows(self, input_embds: torch.Tensor, infer_state) -> torch.Tensor:
+        """[num_tokens, hidden] -> the rows of the sequences' last tokens, a fresh [batch, hidden] copy."""
         idx = infer_state.last_token_indices
         if idx is None:
             # the last token of each prefill sequence, then every decoding token
@@ -25,13 +25,17 @@ class LlamaPostLayer:
                 infer_state.prefill_seq_start_locs + infer_state.prefill_seq_lens - 1,
                 torch.arange(infer_state.num_prefill_tokens, infer_state.num_tokens,
                              device=input_embds.device, dtype=torch.int32)))
-        last_input = input_embds.index_select(0, idx)    # fresh [batch, hidden] copy
+        return input_embds.index_select(0, idx)
+
+    def forward(self, input_embds: torch.Tensor, infer_state) -> torch.Tensor:
+        """[num_tokens, hidden] -> next-token ids int64 [batch_size] (argmax; ties -> lowest id)."""
+        last_input = self.last_rows(input_embds, infer_state)
         rmsnorm_inplace(last_input, self.weights.final_norm, self.model_config.rms_norm_eps)
         return self.forward_normed(last_input)
 
     def forward_normed(self, last_input: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
-        """lm_head + greedy sampling on rows that already went through the final norm (a pure-decode batch whose
-        last add + norm ran fused on the split-K partials of the last down projection: every row is a last token)."""
+        """lm_head + greedy sampling on rows that already went through the final norm (steps whose
+        last add + norm ran fused on the split-K partials of the last down projection)."""
         logits = linear(last_input, self.weights.lm_head, self.skinny)   # [batch, vocab]
         self.last_logits = logits
         if self.logits_tap is not None:
