@@ -40,7 +40,8 @@ def _project_partials(a: torch.Tensor, w: torch.Tensor, skinny: bool):
     SplitKPartials from the decode GEMMs and from prompt-sized products of few tiles, rows otherwise."""
     m = a.shape[0]
     if not skinny or m > DECODE_MAX_TOKENS or a.dtype == torch.float32 or getattr(w, "_swl_blas_only", False):
-        y = linear_tile_partial(a, w) if skinny and m > DECODE_MAX_TOKENS else None
+        # (wider streams' steps take rows: gated_add_rmsnorm)
+        y = linear_tile_partial(a, w) if skinny and m > DECODE_MAX_TOKENS and w.shape[0] <= 8192 else None
         return _project(a, w, skinny) if y is None else y
     y = linear_rows_partial(a, w) if m <= ROWS_MAX_TOKENS else None
     if y is not None:

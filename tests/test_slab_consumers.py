@@ -22,3 +22,13 @@ def test_llama_layers(fuse, layer, monkeypatch):
     out = op._forward_after_attention(torch.zeros(300, 16), torch.zeros(300, 16), False, None)
     assert isinstance(out, torch.Tensor)
     assert asked == (["o", "down"] if fuse else [])
+
+
+@pytest.mark.parametrize("rows,asks", [(8192, True), (8448, False)])
+def test_stepped_designs(rows, asks, monkeypatch):
+    from swiftllm_amd.worker.layers import kekapel_layer as K
+    asked = []
+    monkeypatch.setattr(K, "linear_tile_partial", lambda a, w: asked.append(w))
+    monkeypatch.setattr(K, "linear", lambda a, w, skinny=False: torch.zeros(a.shape[0], w.shape[0]))
+    K._project_partials(torch.zeros(257, 8, dtype=torch.bfloat16), torch.zeros(rows, 8, dtype=torch.bfloat16), True)
+    assert bool(asked) == asks
