@@ -119,8 +119,8 @@ enum TileRows { kTileDense = 0, kTileExpert = 1, kTileGather = 2 };     // rows 
 
 // ACT kTileSlabs: fp32 sums over shares of K; 0: the product; 1: relu(.)^2 of the first act_cols columns; 2 + a: w rows [N first | N second], out = a gated unit of the two (a = 0 .. 2:
 // gated_unit, 3: round(silu(second)) first, rounded). Activations are of the rounded products.
-template <typename T, int U, int X0, int X1, int W0, int W1, int PAIRS, int ACT, int ROWS = kTileDense>
-__global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS == 1 ? 2 : 1) void gemm_tile_kernel(GemmTileParams p) {
+template <typename T, int U, int X0, int X1, int W0, int W1, int ACT, int ROWS = kTileDense>
+__global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 ? 2 : 1) void gemm_tile_kernel(GemmTileParams p) {
     constexpr int X = X0 + X1, W = W0 + W1, E = U == 32 ? 4 : 2;        // blocks of U rows a wave; matrix steps of 64 columns
     constexpr bool GATED = ACT >= 2, SLABS = ACT == kTileSlabs;
     constexpr int xn[2] = {X0, X1}, wn_[2] = {W0, W1};
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
     static_assert(!GATED || W0 == W1, "");
     constexpr bool GATHER = ROWS == kTileGather, EXPERT = ROWS != kTileDense;
     // the next tile's row of `order` and both tiles' weights; first positions of the experts, first row tiles behind them
-    constexpr int LISTS = PAIRS * PAIR + 4 * U * PITCH, TABLES = LISTS + (GATHER ? 3 * 1024 : 0);
+    constexpr int LISTS = PAIR + 4 * U * PITCH, TABLES = LISTS + (GATHER ? 3 * 1024 : 0);
     static_assert(!EXPERT || BM <= 256, "");
     __shared__ __attribute__((aligned(16))) char smem[TABLES + (EXPERT ? (2 * kTileExperts + 1) * 4 : 0)];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -257,16 +257,16 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
         __syncthreads();
     }
     x_offsets(here.rows, 0);
-    int4v ask_x = x_rsrc(here), ask_w = w_rsrc(here);       // the step that is asked for: its tile, its first column, its pair's place in LDS
-    unsigned ask_k = 0, ask_to = lds0;
+    int4v ask_x = x_rsrc(here), ask_w = w_rsrc(here);       // the step that is asked for: its tile, its first column
+    unsigned ask_k = 0;
 
     // Parts in the order of their use, eight for two steps: X0 W0 W1 X1, X0 W1 W0 X1
     auto fetch = [&](auto jc, int i) {
         constexpr int J = decltype(jc)::value & 7, odd = J >> 2, k = J & 3;
         constexpr bool of_x = k == 0 || k == 3;
         constexpr int h = k == 0 ? 0 : k == 3 ? 1 : ((k == 2) ^ odd);
-        if constexpr (of_x) tile_fetch(ask_x, xo[h * X0 * ASKS + i], ask_k, ask_to + odd * STEP + h * X0 * BLOCK + (wave * xn[h] * ASKS + i) * 1024);
-        else tile_fetch(ask_w, wo[h * W0 * ASKS + i], ask_k, ask_to + odd * STEP + (X + h * W0) * BLOCK + (wave * wn_[h] * ASKS + i) * 1024);
+        if constexpr (of_x) tile_fetch(ask_x, xo[h * X0 * ASKS + i], ask_k, lds0 + odd * STEP + h * X0 * BLOCK + (wave * xn[h] * ASKS + i) * 1024);
+        else tile_fetch(ask_w, wo[h * W0 * ASKS + i], ask_k, lds0 + odd * STEP + (X + h * W0) * BLOCK + (wave * wn_[h] * ASKS + i) * 1024);
     };
     constexpr auto blocks = [](int j) { const int k = j & 3, odd = (j >> 2) & 1; return k == 0 ? X0 : k == 3 ? X1 : ((k == 2) ^ odd) ? W1 : W0; };
     constexpr auto fetches = [=](int from, int to) { int n = 0; for (int j = from; j < to; ++j) n += blocks(j); return n * ASKS; };
@@ -289,15 +289,15 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
     constexpr auto leaving = [](int left) { return left >= CB ? CB : left >= 2 ? 2 : 1; };     // blocks of columns at once, of those that are left
     constexpr auto lines = [](int nb) { return U * U * nb * SIZE >= 1024 ? U * U * nb * SIZE / 1024 : 1; };     // stores of a wave for them
     constexpr int STORES = [=] { int n = 0; for (int b = 0; b < OW; b += leaving(OW - b)) n += lines(leaving(OW - b)); return X * n; }();   // for a tile
-    // Phase P of eight: products of a half of x with a half of w. It reads part P + 2 and asks for part P + 8 PAIRS, whose place part P has left.
+    // Phase P of eight: products of a half of x with a half of w. It reads part P + 2 and asks for part P + 8, whose place part P has left.
     // In front of every second phase: parts P + 2 and P + 3 have landed, everyone has read P and P + 1. (`stored`: the last tile's results, asked
-    // to be written behind the parts P + 2 .. 8 PAIRS - 1, need not be.)
+    // to be written behind the parts P + 2 .. 7, need not be.)
     auto phase = [&](auto pc, auto first_pair, int stored) {
         constexpr bool FIRST = decltype(first_pair)::value && decltype(pc)::value < 4;      // (its results are the first of its sums)
         constexpr int P = decltype(pc)::value, odd = P >> 2, k = P & 3;
         constexpr int xh = k >> 1, wh = ((k == 1 || k == 2) ? 1 : 0) ^ odd;
         if constexpr ((P & 1) == 0) {
-            constexpr int OUT = fetches(P + 4, P + 8 * PAIRS), LATE = decltype(first_pair)::value && P + 3 < 8 * PAIRS ? (OUT + STORES < 63 ? OUT + STORES : 63) : OUT;
+            constexpr int OUT = fetches(P + 4, P + 8), LATE = decltype(first_pair)::value && P + 3 < 8 ? (OUT + STORES < 63 ? OUT + STORES : 63) : OUT;
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (LATE > OUT)
                 asm volatile("s_cmp_eq_u32 %0, 0\n\ts_cbranch_scc1 .Lplain%=\n\ts_waitcnt vmcnt(%2) lgkmcnt(0)\n\ts_branch .Lgo%=\n"
@@ -333,20 +333,15 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
         }
     };
 
-    // ---- the first PAIRS pairs of steps of the first tile -----------------------------------------------------------------------------
+    // ---- the first pair of steps of the first tile ------------------------------------------------------------------------------------
     auto fetch_part = [&](auto jc) {
 #pragma unroll
         for (int i = 0; i < ASKS * blocks(decltype(jc)::value); ++i) fetch(jc, i);
     };
-#pragma unroll
-    for (int q = 0; q < PAIRS; ++q) {
-        fetch_part(Ic<0>{}); fetch_part(Ic<1>{}); fetch_part(Ic<2>{}); fetch_part(Ic<3>{});
-        ask_k += 128;
-        fetch_part(Ic<4>{}); fetch_part(Ic<5>{}); fetch_part(Ic<6>{}); fetch_part(Ic<7>{});
-        ask_k += 128, ask_to += PAIR;
-    }
-    ask_to = lds0;
-    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(fetches(2, 8 * PAIRS)) : "memory");
+    fetch_part(Ic<0>{}); fetch_part(Ic<1>{}); fetch_part(Ic<2>{}); fetch_part(Ic<3>{});
+    ask_k = 128;
+    fetch_part(Ic<4>{}); fetch_part(Ic<5>{}); fetch_part(Ic<6>{}); fetch_part(Ic<7>{});
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(fetches(2, 8)) : "memory");
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int i = 0; i < E * X0; ++i) read(Ic<0>{}, i);
@@ -370,20 +365,13 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
             }
         };
         auto pair = [&](int s, auto first_pair) {
-            ask_for(s + 2 * PAIRS);
+            ask_for(s + 2);
             if constexpr (GATHER && !decltype(first_pair)::value) {      // the next tile's first step: its rows, whose list came before this tile's second pair
-                if (s + 2 * PAIRS == steps && next < last) x_offsets(then.rows, slot ^ 1);
+                if (s + 2 == steps && next < last) x_offsets(then.rows, slot ^ 1);
             }
             phase(Ic<0>{}, first_pair, stored); phase(Ic<1>{}, first_pair, stored); phase(Ic<2>{}, first_pair, stored); phase(Ic<3>{}, first_pair, stored);
-            ask_for(s + 2 * PAIRS + 1);
-            phase(Ic<4>{}, first_pair, stored); phase(Ic<5>{}, first_pair, stored);
-            if constexpr (PAIRS > 1) {      // the pair that is read from here on
-                const unsigned from = ask_to - lds0, to = from + PAIR == PAIRS * PAIR ? 0 : from + PAIR;
-#pragma unroll
-                for (int e = 0; e < E; ++e) frag[e] += to - from;
-            }
-            phase(Ic<6>{}, first_pair, stored); phase(Ic<7>{}, first_pair, stored);
-            if constexpr (PAIRS > 1) ask_to = ask_to + PAIR == lds0 + PAIRS * PAIR ? lds0 : ask_to + PAIR;
+            ask_for(s + 3);
+            phase(Ic<4>{}, first_pair, stored); phase(Ic<5>{}, first_pair, stored); phase(Ic<6>{}, first_pair, stored); phase(Ic<7>{}, first_pair, stored);
         };
         pair(0, std::true_type{});
 #pragma nounroll
@@ -402,7 +390,7 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
 
         // ---- results: U rows of 64 columns at a time through the wave's own piece of LDS, whole lines to memory. acc[a][b][4 q + k]: row U a
         // + lu, column U b + (256 / U) q + 4 lg + k. Stores beyond the rows or columns are dropped by the descriptor ----------------------
-        char *mine = smem + PAIRS * PAIR + wave * U * PITCH;
+        char *mine = smem + PAIR + wave * U * PITCH;
         char *base = static_cast<char *>(p.out) + ((SLABS ? static_cast<int64_t>(here.expert) * p.M : 0) + here.row0) * ob + static_cast<int64_t>(here.col0) * SIZE;
         const int bytes = static_cast<int>(here.rows * ob - static_cast<int64_t>(here.col0) * SIZE), cols = p.N - here.col0;
         unsigned first = static_cast<unsigned>(wm * U * X * ob + wn * OUTW * SIZE);
@@ -479,9 +467,9 @@ __global__ __launch_bounds__(256, U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS
     asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
 }
 
-template <typename T, int U, int X0, int X1, int W0, int W1, int PAIRS, int ACT, int ROWS = kTileDense>
+template <typename T, int U, int X0, int X1, int W0, int W1, int ACT, int ROWS = kTileDense>
 int gemm_tile_launch(GemmTileParams p, hipStream_t s) {
-    constexpr int BM = 2 * U * (X0 + X1), BN = 2 * U * (W0 + W1) / (ACT >= 2 ? 2 : 1), A_CU = U * U * (X0 + X1) * (W0 + W1) <= 4096 && PAIRS == 1 ? 2 : 1;
+    constexpr int BM = 2 * U * (X0 + X1), BN = 2 * U * (W0 + W1) / (ACT >= 2 ? 2 : 1), A_CU = U * U * (X0 + X1) * (W0 + W1) <= 4096 ? 2 : 1;
     p.n_tiles = (p.N + BN - 1) / BN;
     if constexpr (ACT == kTileSlabs) p.share = Divisor::of(p.n_tiles), p.n_tiles *= p.splits;
     // (experts: as many row tiles as there can be, each of theirs may end in a part of one; how many there are is on the device)
@@ -493,7 +481,7 @@ int gemm_tile_launch(GemmTileParams p, hipStream_t s) {
     p.wide = Divisor::of(kTileGroup);
     p.rest = Divisor::of(rest ? rest : kTileGroup);
     const unsigned grid = static_cast<unsigned>(tiles < 256 * A_CU ? (tiles + 7) / 8 * 8 : 256 * A_CU);
-    hipLaunchKernelGGL((gemm_tile_kernel<T, U, X0, X1, W0, W1, PAIRS, ACT, ROWS>), dim3(grid), dim3(256), 0, s, p);
+    hipLaunchKernelGGL((gemm_tile_kernel<T, U, X0, X1, W0, W1, ACT, ROWS>), dim3(grid), dim3(256), 0, s, p);
     return check_launch();
 }
 

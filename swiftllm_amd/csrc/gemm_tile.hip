@@ -6,21 +6,21 @@ namespace swl {
 template <typename T, int ACT>
 int gemm_tile_dispatch(const GemmTileParams &p, int shape, hipStream_t s) {     // (in the order of kTileShapes)
     switch (shape) {
-    case 1: return gemm_tile_launch<T, 16, 4, 4, 4, 4, 1, ACT>(p, s);
-    case 2: return gemm_tile_launch<T, 16, 3, 3, 4, 4, 1, ACT>(p, s);
-    case 3: return gemm_tile_launch<T, 16, 3, 3, 3, 3, 1, ACT>(p, s);
-    case 4: return gemm_tile_launch<T, 16, 3, 2, 4, 4, 1, ACT>(p, s);
-    case 5: return gemm_tile_launch<T, 16, 4, 3, 4, 4, 1, ACT>(p, s);
-    case 6: return gemm_tile_launch<T, 16, 4, 4, 3, 3, 1, ACT>(p, s);
-    case 10: return gemm_tile_launch<T, 32, 1, 1, 1, 1, 1, ACT>(p, s);
-    case 11: return gemm_tile_launch<T, 16, 1, 1, 2, 2, 1, ACT>(p, s);
+    case 1: return gemm_tile_launch<T, 16, 4, 4, 4, 4, ACT>(p, s);
+    case 2: return gemm_tile_launch<T, 16, 3, 3, 4, 4, ACT>(p, s);
+    case 3: return gemm_tile_launch<T, 16, 3, 3, 3, 3, ACT>(p, s);
+    case 4: return gemm_tile_launch<T, 16, 3, 2, 4, 4, ACT>(p, s);
+    case 5: return gemm_tile_launch<T, 16, 4, 3, 4, 4, ACT>(p, s);
+    case 6: return gemm_tile_launch<T, 16, 4, 4, 3, 3, ACT>(p, s);
+    case 10: return gemm_tile_launch<T, 32, 1, 1, 1, 1, ACT>(p, s);
+    case 11: return gemm_tile_launch<T, 16, 1, 1, 2, 2, ACT>(p, s);
     default: break;
     }
     if constexpr (ACT <= 0) {
         switch (shape) {
-        case 7: return gemm_tile_launch<T, 16, 3, 2, 2, 2, 1, ACT>(p, s);
-        case 8: return gemm_tile_launch<T, 16, 3, 2, 3, 3, 1, ACT>(p, s);
-        case 9: return gemm_tile_launch<T, 16, 4, 3, 3, 3, 1, ACT>(p, s);
+        case 7: return gemm_tile_launch<T, 16, 3, 2, 2, 2, ACT>(p, s);
+        case 8: return gemm_tile_launch<T, 16, 3, 2, 3, 3, ACT>(p, s);
+        case 9: return gemm_tile_launch<T, 16, 4, 3, 3, 3, ACT>(p, s);
         default: break;
         }
     }

@@ -254,11 +254,11 @@ template <typename T, int ACT, int ROWS>
 int moe_gemm_dispatch(const GemmTileParams &p, int64_t w_rows, hipStream_t s) {
     auto tiles = [&](int rows, int cols) { return (p.M / rows + (min(p.experts, p.M) + 1) / 2) * ((w_rows + cols - 1) / cols); };
     switch (gemm_tile_shape(tiles, p.K, kTilesExperts)) {
-    case 1: return gemm_tile_launch<T, 16, 4, 4, 4, 4, 1, ACT, ROWS>(p, s);
-    case 2: return gemm_tile_launch<T, 16, 3, 3, 4, 4, 1, ACT, ROWS>(p, s);
-    case 3: return gemm_tile_launch<T, 16, 3, 3, 3, 3, 1, ACT, ROWS>(p, s);
-    case 6: return gemm_tile_launch<T, 16, 4, 4, 3, 3, 1, ACT, ROWS>(p, s);
-    default: return gemm_tile_launch<T, 16, 2, 2, 2, 2, 1, ACT, ROWS>(p, s);
+    case 1: return gemm_tile_launch<T, 16, 4, 4, 4, 4, ACT, ROWS>(p, s);
+    case 2: return gemm_tile_launch<T, 16, 3, 3, 4, 4, ACT, ROWS>(p, s);
+    case 3: return gemm_tile_launch<T, 16, 3, 3, 3, 3, ACT, ROWS>(p, s);
+    case 6: return gemm_tile_launch<T, 16, 4, 4, 3, 3, ACT, ROWS>(p, s);
+    default: return gemm_tile_launch<T, 16, 2, 2, 2, 2, ACT, ROWS>(p, s);
     }
 }
 
