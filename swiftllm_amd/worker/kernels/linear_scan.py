@@ -38,12 +38,13 @@ SEGMENT_PORTION_TILES, SEGMENT_MAX_SCRATCH = 24, 1 << 28
 SEGMENT_MIN_TILES, SEGMENT_SLOTS = {True: 3, False: 8}, {True: 256, False: 768}
 
 
-def scan_segments(st: StateRef, heads: int, dim: int, vdim: int):
-    """(segments, tiles of one, scratch) of a step's scan; (1, 0, None): portions run whole."""
+def scan_segments(st: StateRef, heads: int, dim: int, vdim: int, aligned: bool = True):
+    """(segments, tiles of one, scratch) of a step's scan; (1, 0, None): portions run whole. aligned: rows of values in whole pieces of 16 bytes, which the 64
+    columns a workgroup are for."""
     tiles, num_seqs = -(-st.longest // 16), st.seq_row0.shape[0]
     if tiles < SEGMENT_PORTION_TILES:
         return 1, 0, None
-    wide = dim in (64, 128)
+    wide = dim in (64, 128) and aligned
     portions = -(-(st.tiles[0].shape[0] - num_seqs) // (tiles - 1))     # (as if every tile but the portions' first belonged to one of the longest's length)
     segments = min(SEGMENT_SLOTS[wide] // (max(portions, 1) * heads * -(-vdim // (64 if wide else 16))), tiles // SEGMENT_MIN_TILES[wide], 64)
     lib = _hip.load()
@@ -102,7 +103,8 @@ def linear_recurrence(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, decay: 
               _hip.ptr(k), k.stride(0), _hip.ptr(decay), decay.stride(0), 1 if per_channel else 0, _hip.ptr(k_scale),
               _hip.ptr(bonus), float(q_scale), _hip.ptr(row0), _hip.ptr(cnt), num_tiles, H, G, dim, code, stream)
     o = torch.empty((n, H * vdim), dtype=f32, device=dev)
-    segments, seg_tiles, scratch = scan_segments(st, H, dim, vdim)
+    size = v.element_size()
+    segments, seg_tiles, scratch = scan_segments(st, H, dim, vdim, (v.data_ptr() | v.stride(0) * size | vdim * size) % 16 == 0)
     _hip.call("swl_linear_scan_cut", _hip.ptr(o), o.stride(0), _hip.ptr(qd), _hip.ptr(kd), _hip.ptr(total), _hip.ptr(intra),
               _hip.ptr(v), v.stride(0), _hip.ptr(dskip), _hip.ptr(st.pool), st.pool.stride(0), int(state_off),
               _hip.ptr(st.seq_row0), _hip.ptr(st.seq_cnt), _hip.ptr(seq_tile0), _hip.ptr(st.tok_pos), _hip.ptr(st.tok_state),

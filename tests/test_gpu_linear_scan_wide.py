@@ -86,3 +86,25 @@ def test_wide_scan(lens, H, G, d, dv, bonus, scalar, aligned, dtype):
         assert (y[at:at + c] - want.reshape(c, -1)).abs().max() < 3e-5 * max(1.0, float(want.abs().max())), (s, c)
         assert (got_state[len(lens) - 1 - s] - S).abs().max() < 3e-5 * max(1.0, float(S.abs().max())), (s, c)
         at += c
+
+
+@pytest.mark.parametrize("shift,dv,want", [(0, 64, (21, 3)), (1, 64, (7, 9)), (0, 60, (7, 9))])
+def test_segments_are_those_of_the_walk_that_runs(shift, dv, want, monkeypatch):
+    """Values that lie on no 16 bytes, or are no whole pieces of 16, take the walk of 16 columns a workgroup: portions are cut as its workgroups need it."""
+    from swiftllm_amd.worker.kernels import linear_scan
+    from swiftllm_amd.worker.kernels.rms_stream import StateRef
+    n, H, d = 1000, 4, 128
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")      # noqa: E731
+    starts = range(0, n, 16)
+    st = StateRef(torch.zeros(1, H * d * dv, device="cuda"), ints(range(n)), None, ints([0] * n), None, ints([0]), ints([n]),
+                  (ints(starts), ints([min(16, n - s) for s in starts]), ints([0])), n)
+    cut, got = linear_scan.scan_segments, []
+
+    def keep(*a):
+        got.append(cut(*a))
+        return got[-1]
+    monkeypatch.setattr(linear_scan, "scan_segments", keep)
+    v = torch.zeros(n, H * dv + 8, dtype=torch.bfloat16, device="cuda")[:, shift:shift + H * dv]
+    q = torch.zeros(n, H * d, dtype=torch.bfloat16, device="cuda")
+    linear_scan.linear_recurrence(q, q, v, torch.ones(n, H, device="cuda"), st, 0, H, d, dv)
+    assert got[0][:2] == want
