@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_grouped_kernel(int32_t 
     }
 }
 
-// Routers of up to eight experts for steps of many tokens: a wave takes two or four tokens, whose rows meet each load of the router's, and the choice is
+// Routers of five to eight experts for steps of many tokens: a wave takes two or four tokens, whose rows meet each load of the router's, and the choice is
 // made by a lane a token from registers. What bounds it is vector work (eight multiplies and adds a quad and expert, which stay apart) and the
 // chain of a choice; a workgroup a token, as above, also waits for its row, its two meetings and the router's rows (32 KiB of 1024 columns a token from
 // L2). The same sums in the same order, the same bits.
@@ -456,13 +456,19 @@ __global__ __launch_bounds__(kMoeThreads) void moe_route_few_kernel(RouteParams 
     }
 }
 
-// From 3072 tokens on: 2048 of 1024 columns in groups 8.0 us a workgroup a token, 9.1 so; 3657 11.2 and 9.4. Four tokens a wave from 4609 on: 3657 of 1024
-// 7.4 with two and 8.0 with four, 4499 9.2 and 9.6, 7452 10.5 and 9.7.
-constexpr int64_t kRouteFewTokens = 3072, kRouteFourTokens = 4609;
+// Where that pays, us by a workgroup a token -> so, bf16 (two tokens a wave). Seven and eight experts: from 3072 tokens on (2048 columns, 3000 tokens 10.8 -> 9.8
+// plain, 12.8 -> 11.7 in four groups; 1024 columns in groups 2000 tokens 1.13 times as long). All scores and one group, whose choice a workgroup makes
+// quickly, from 5632 on (1024 columns, 4500 tokens 10.0 -> 10.5, 6000 11.9 -> 10.5). Five and six, for which some of the eight sums are for nothing, from 6600 on (2048
+// columns, all scores 4500 tokens 11.9 -> 13.7, 7000 15.9 -> 13.7 by four). Fewer never (two, 2048 columns: 4700 tokens 8.8 -> 12.4 to 14.6, 9000 14.9 -> 17.0 to
+// 19.0). Four tokens a wave, not of fp32, from 6600 on: 2048 columns plain, two and four, 4500 tokens 12.4, 12.0, 7000 14.7, 12.5; 1024 6000 9.1, 9.5, 7000 10.3, 9.5.
+constexpr int64_t kRouteFewTokens = 3072, kRouteQuickTokens = 5632, kRouteFourTokens = 6600;
+constexpr int kRouteLeast = 5, kRouteMost = 7;
 template <typename T, bool GROUPED>
 bool route_few(const RouteParams &p, hipStream_t s) {
-    if (p.num_tokens < kRouteFewTokens || p.experts > kRouteFew || p.width % 4 || !aligned16(p.router) || (reinterpret_cast<uintptr_t>(p.h) & (4 * sizeof(T) - 1))) return false;
-    const int each = p.num_tokens < kRouteFourTokens ? 2 : 4;
+    const bool quick = GROUPED ? p.count <= 1 || p.keep >= p.count : p.all_scores != 0;
+    const int64_t least = p.experts < kRouteMost ? kRouteFourTokens : quick ? kRouteQuickTokens : kRouteFewTokens;
+    if (p.num_tokens < least || p.experts > kRouteFew || p.experts < kRouteLeast || p.width % 4 || !aligned16(p.router) || (reinterpret_cast<uintptr_t>(p.h) & (4 * sizeof(T) - 1))) return false;
+    const int each = sizeof(T) == 4 || p.num_tokens < kRouteFourTokens ? 2 : 4;
     const dim3 grid(static_cast<unsigned>((p.num_tokens + each * kMoeWaves - 1) / (each * kMoeWaves)));
     if (each == 2) hipLaunchKernelGGL((moe_route_few_kernel<T, GROUPED, 2>), grid, dim3(kMoeThreads), 0, s, p);
     else hipLaunchKernelGGL((moe_route_few_kernel<T, GROUPED, 4>), grid, dim3(kMoeThreads), 0, s, p);

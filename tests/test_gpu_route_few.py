@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [3073, 4609, 4614])
+@pytest.mark.parametrize("n", [3073, 4609, 4614, 5633, 6601, 6606])
 @pytest.mark.parametrize("experts,top,count,keep", [(8, 2, 4, 2), (6, 3, 3, 2), (6, 2, 2, 1), (8, 8, 2, 2), (5, 1, 1, 1), (8, 2, 8, 3), (4, 4, 2, 2), (1, 1, 1, 1)])
 @pytest.mark.parametrize("width,dtype", [(260, torch.bfloat16), (1024, torch.float16), (100, torch.float32)])
 def test_same_bits(n, experts, top, count, keep, width, dtype):
