@@ -108,3 +108,45 @@ def test_segments_are_those_of_the_walk_that_runs(shift, dv, want, monkeypatch):
     q = torch.zeros(n, H * d, dtype=torch.bfloat16, device="cuda")
     linear_scan.linear_recurrence(q, q, v, torch.ones(n, H, device="cuda"), st, 0, H, d, dv)
     assert got[0][:2] == want
+
+
+@pytest.mark.parametrize("lens", [[401, 1, 16, 384, 17], [33, 20, 50]])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_value_that_is_no_number_stays_in_its_column(lens, dtype):
+    """NaN and infinity among the values of one sequence, infinities in another's keys: other sequences, heads, columns and the tiles before have the bits that
+    they have without."""
+    from swiftllm_amd.worker.kernels import linear_scan
+    from swiftllm_amd.worker.kernels.rms_stream import StateRef
+    g = torch.Generator().manual_seed(1)
+    n, H, d, dv = sum(lens), 2, 64, 72
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")      # noqa: E731
+    rows, counts, tile0, seq_row0, at = [], [], [], [], 0
+    for c in lens:
+        seq_row0.append(at)
+        tile0.append(len(rows))
+        for o in range(0, c, 16):
+            rows.append(at + o)
+            counts.append(min(16, c - o))
+        at += c
+    q, k, v = (torch.randn(n, H * s, generator=g).to(dtype) for s in (d, d, dv))
+    decay = torch.rand(n, H * d, generator=g) ** 0.02
+    bad_v, bad_k = v.clone(), k.clone()
+    bad_v[20, dv + 70] = float("nan")          # the first sequence, second head, column 70, second tile
+    last = seq_row0[-1] + 16
+    bad_v[last, 3], bad_k[seq_row0[1], 5] = float("inf"), float("inf")
+    results = []
+    for vv, kk in ((v, k), (bad_v, bad_k)):
+        pool = torch.zeros(len(lens), H * d * dv, device="cuda")
+        st = StateRef(pool, ints([p for c in lens for p in range(c)]), None, ints([2 * s for s, c in enumerate(lens) for _ in range(c)]), None, ints(seq_row0), ints(lens),
+                      (ints(rows), ints(counts), ints(tile0)), max(lens))
+        y = linear_scan.linear_recurrence(q.cuda(), kk.cuda(), vv.cuda(), decay.cuda(), st, 0, H, d, dv)
+        results.append((y.cpu().view(n, H, dv), pool.cpu().view(len(lens), H, d, dv)))
+    (y, s), (bad_y, bad_s) = results
+    same, states = torch.ones_like(y, dtype=torch.bool), torch.ones_like(s, dtype=torch.bool)
+    same[16:lens[0], 1, 70], states[0, 1, :, 70] = False, False
+    same[last:, 0, 3], states[-1, 0, :, 3] = False, False
+    same[seq_row0[1]:seq_row0[1] + lens[1], 0], states[1, 0] = False, False
+    assert torch.equal(bad_y[same], y[same]) and torch.equal(bad_s[states], s[states])
+    assert not bool(bad_y[20:lens[0], 1, 70].isfinite().any()) and not bool(bad_s[0, 1, :, 70].isfinite().any())
+    assert not bool(bad_y[last:, 0, 3].isfinite().any()) and not bool(bad_s[-1, 0, :, 3].isfinite().any())
+    assert not bool(bad_y[seq_row0[1]:seq_row0[1] + lens[1], 0].isfinite().any())
