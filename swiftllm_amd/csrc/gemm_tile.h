@@ -16,7 +16,7 @@
 // Measured (us, bf16, operands from a pool of 1.5 GB; in brackets the library, in one call and in the blocks of rows that it was called with
 // before): 7691 tokens: 1024 x 1024 17.3 (20.7, 27.1), 8192 x 1024 106 (104, 104), 1024 x 4096 55 (62, 74), 2576 x 1024 40 (60, 63); 4498: 2048 x 2048 33
 // (38, 45), 2048 x 8192 117 (131, 141), 8192 x 2048 112 (125, 118), 3072 x 2048 45 (47, 59); 3657: 2048 x 8192 97 (105), 7440 x 2048 87 (104); 2029: 5696 x 1024 22
-// (34), 1024 x 1024 8.6 (11); 1828: 28672 x 4096 336 with its gated unit (342 to 430 by card, and 32 for the unit), 4096 x 14336 177 (185); 5112: 6144 x
+// (34), 1024 x 1024 8.6 (11); 1828: 28672 x 4096 355 with its gated unit (342 to 430 by card, and 32 for the unit), 4096 x 14336 177 (185); 5112: 6144 x
 // 4096 182 (180, 207), 4096 x 4096 128 (135, 128). 270 products of 260 to 8192 tokens: 0.8 of the library's time where its calls are in blocks. From
 // 16384 tokens on the library's rate is 5 % to 10 % higher (1.55 PFLOP/s).
 #pragma once

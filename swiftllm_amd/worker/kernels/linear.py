@@ -7,7 +7,7 @@ reference's call dispatches to cuBLAS — same GEMM kernels as the reference run
 hand-written weight-streaming MFMA kernel `swl_gemm_skinny` (csrc/gemm_skinny.hip): at that size the
 projection is pure HBM streaming of the weight matrix, 77 % of all bytes a decode step moves. Prompt-sized calls (more than 256
 tokens) go to the tiled kernel `swl_gemm_tile` (csrc/gemm_tile.hip), with their activation where there is one, as far as `_tile_pays`
-says; the rest stays on the BLAS.
+says and, without one, where the result's rows are whole eights; the rest stays on the BLAS.
 
 Weights that carry a packed twin (`pack_weight`: a copy in MFMA-fragment order made at load time,
 EngineConfig.pack_decode_weights) are streamed from that copy — same bits, 6-9 % faster (long sequential DRAM
@@ -300,7 +300,7 @@ def _tile_pays(m: int, rows: int, k: int, act: bool = False, groups: int = 1) ->
     Very long sums of many tokens are the library's, which takes them in blocks of rows at its best rate: 5112 of 4096 x 14336 505 (458); 4010 tokens 353 (367)
     (not with 2048 rows: 5000 of 2048 x 12288 205 (267), 7800 291 (374)). And beyond 8192 tokens what is not
     small, where the library's rate is 5 % to 10 % higher: 12288 of 6144 x 4096 459 (424), 16384 of 8192 x 2048 381 (365), of 1024 x 4096 102 (93), but
-    12288 of 1024 x 4096 77 (102), 10000 of 3072 x 1024 55 (72) — unless the launch does an activation's work (28672 x 4096, 16384 2621 (2733)).
+    12288 of 1024 x 4096 77 (102), 10000 of 3072 x 1024 55 (72) — unless the launch does an activation's work (28672 x 4096, 16384 2727 (2733)).
     groups: products in one launch that are one each otherwise: up to 2560 columns always."""
     if m > 8192 and m * rows * k > 6e10 and not act:
         return False
