@@ -287,31 +287,22 @@ TILE_NONE, TILE_RELU2, TILE_GATED = 0, 1, 2
 TILE_SILU_ROUNDED = 3       # gated unit of rows [up | gate]: round(silu(gate)) up, what silu_and_mul_inplace makes of the product
 
 
-def _tile_pays(m: int, rows: int, k: int, act: bool = False, groups: int = 1) -> bool:
-    """Whether the tiled kernel takes a product, `rows` rows of the matrix. Few tiles (of 64 x 128) are the library's, which splits their sums; the line is lower
-    where the launch does an activation's work too (`act`). Measured: 18000 products of 257 to 16384 tokens, 64 to 30000 rows and 256 to 14336 columns,
-    both types, cold weights: 0.865 of the library's time by these lines, 852 of 11771 more than 3 % slower, 1.31 the worst (with all up to 2560 columns: 0.876,
-    1989, 2.3); 12000 with their gated unit: 0.765, 575 of 9778. us (library), tokens x rows (tiles):
-        1024 columns   446 x 128 (7) 7.4 (6.2), 510 x 344 (24) 8.2 (8.0), 424 x 1024 (56) 7.7 (9.7)     with the unit   423 x 96 (7) 7.8 (9.1)
-        2048           402 x 1024 (56) 13.2 (10.4), 512 x 2048 (128) 13.4 (12.6), 1259 x 1152 (180) 13.6 (14.2)         294 x 512 (20) 13.0 (12.7), 654 x 640 (55) 13.4 (13.9)
-        2560           300 x 96 (5) 15.4 (9.0), 499 x 2048 (128) 15.6 (14.0), 668 x 2048 (176) 17.0 (17.5)              291 x 1408 (55) 16.0 (15.4), 375 x 2048 (96) 16.4 (17.6)
-        4096           470 x 2048 (128) 23.0 (19.9), 404 x 3064 (168) 23.7 (23.9), 1144 x 1024 (144) 23.6 (22.4)        643 x 1024 (88) 23.0 (22.3), 351 x 4096 (192) 29.8 (29.7)
-        8192           1367 x 1024 (176) 41.4 (37.6), 489 x 4096 (256) 60.3 (53.3), 1260 x 2048 (320) 70 (68)           497 x 4096 (256) 61.3 (58.8)
-    Very long sums of many tokens are the library's, which takes them in blocks of rows at its best rate: 5112 of 4096 x 14336 505 (458); 4010 tokens 353 (367)
-    (not with 2048 rows: 5000 of 2048 x 12288 205 (267), 7800 291 (374)). And beyond 8192 tokens what is not
+def _tile_pays(m: int, rows: int, k: int, gated: bool = False) -> bool:
+    """Whether the tiled kernel takes a product, `rows` rows of the matrix. Long sums of few tiles are the library's, which splits them (tiles of 64 x 128,
+    us, library's): 1024 x 4096, 409 tokens (56 tiles) 21.2 (13.9), 1110 (144) 21.8 (21.8), 2396 (304) 27 (32); 1024 x 6144, 572 (72) 31 (22), 1167 (152)
+    31.5 (30.5), 2036 (256) 33 (41); 2048 x 8192, 679 (176) 58 (45), 1260 (320) 70 (68), 1559 (400) 71 (73); 4096 x 14336, 360 (192) 107 (84), 741 (384)
+    129 (122), 1521 (768) 172 (188). Up to 2560 columns always (277 of 1024 x 1024 7.4, 8.7): the few tiles that take longer there (402 of 1024 x 2048 13.2, 10.4; 300 of 96 x
+    2560 15.4, 9.0) are of steps that wait for the host, which a library's call keeps 15 us longer than a launch (lines by device time alone: passes of 280 to 1341 tokens
+    on 1024 and 2048 columns 1.06 to 1.23 times as long, none shorter). So are very long ones of many tokens, which the
+    library takes in blocks of rows at its best rate: 5112 of 4096 x 14336 505 (458); 4010 tokens 353 (367) (not with 2048 rows: 5000 of 2048 x 12288 205
+    (267), 7800 291 (374)). And beyond 8192 tokens what is not
     small, where the library's rate is 5 % to 10 % higher: 12288 of 6144 x 4096 459 (424), 16384 of 8192 x 2048 381 (365), of 1024 x 4096 102 (93), but
-    12288 of 1024 x 4096 77 (102), 10000 of 3072 x 1024 55 (72) — unless the launch does an activation's work (28672 x 4096, 16384 2727 (2733)).
-    groups: products in one launch that are one each otherwise: up to 2560 columns always."""
-    if m > 8192 and m * rows * k > 6e10 and not act:
+    12288 of 1024 x 4096 77 (102), 10000 of 3072 x 1024 55 (72) — unless the launch does an activation's work (28672 x 4096, 16384 2727 (2733))."""
+    if m > 8192 and m * rows * k > 6e10 and not gated:
         return False
-    tiles = -(-m // 64) * -(-rows // 128)
-    if groups > 1:
-        enough = k <= 2560 or tiles * 16 >= min(k - 2048, 6400)
-    elif act:
-        enough = tiles * 28 >= k - 1024 or tiles * 36 >= k + 1024
-    else:
-        enough = tiles * 10 >= k - 512 or tiles * 36 >= k + 2048
-    return enough and (k <= 8192 or m <= 4096 or rows <= 2048)
+    if k <= 2560:
+        return True
+    return -(-m // 64) * -(-rows // 128) * 16 >= min(k - 2048, 6400) and (k <= 8192 or m <= 4096 or rows <= 2048)
 
 
 def linear_tile(a: torch.Tensor, w: torch.Tensor, act: int = TILE_NONE, act_columns: int = 0, limit: float = 0.0, out: torch.Tensor = None):
@@ -453,7 +444,7 @@ def linear_grouped(x: torch.Tensor, w: torch.Tensor, skinny: bool = False) -> to
         return out
     size = n // groups
     if skinny and m >= TILE_MIN_TOKENS and size % 256 == 0 and w.shape[1] == k and x.is_contiguous() and w.is_contiguous() and x.dtype == w.dtype \
-            and x.dtype in (torch.float16, torch.bfloat16) and x.is_cuda and (x.data_ptr() | w.data_ptr()) % 16 == 0 and _tile_pays(m, n, k, groups=groups) \
+            and x.dtype in (torch.float16, torch.bfloat16) and x.is_cuda and (x.data_ptr() | w.data_ptr()) % 16 == 0 and _tile_pays(m, n, k) \
             and _hip.load().swl_gemm_tile_supported(m, n, k, k, n, TILE_NONE, _hip.dtype_code(x.dtype)):
         _hip.call("swl_gemm_tile", _hip.ptr(out), _hip.ptr(x), _hip.ptr(w), m, n, k, k, n, size, m * k, TILE_NONE, 0, 0.0, 0, _hip.dtype_code(x.dtype),
                   _hip.stream())
