@@ -16,7 +16,7 @@
 // Measured (us, bf16, operands from a pool of 1.5 GB; in brackets the library, in one call and in the blocks of rows that it was called with
 // before): 7691 tokens: 1024 x 1024 17.3 (20.7, 27.1), 8192 x 1024 106 (104, 104), 1024 x 4096 55 (62, 74), 2576 x 1024 40 (60, 63); 4498: 2048 x 2048 33
 // (38, 45), 2048 x 8192 117 (131, 141), 8192 x 2048 112 (125, 118), 3072 x 2048 45 (47, 59); 3657: 2048 x 8192 97 (105), 7440 x 2048 87 (104); 2029: 5696 x 1024 22
-// (34), 1024 x 1024 8.6 (11); 1828: 28672 x 4096 355 with its gated unit (342 to 430 by card, and 32 for the unit), 4096 x 14336 177 (185); 5112: 6144 x
+// (34), 1024 x 1024 8.6 (11); 1828: 28672 x 4096 347 with its gated unit (342 to 430 by card, and 32 for the unit), 4096 x 14336 177 (185); 5112: 6144 x
 // 4096 182 (180, 207), 4096 x 4096 128 (135, 128). 270 products of 260 to 8192 tokens: 0.8 of the library's time where its calls are in blocks. From
 // 16384 tokens on the library's rate is 5 % to 10 % higher (1.55 PFLOP/s).
 #pragma once
@@ -76,16 +76,15 @@ __device__ __forceinline__ unsigned divide(unsigned n, Divisor d) {
 }
 
 // num / (1 + e^y) of the gated units below, with the error of the library's exponential and division (3.1 units of 2^-24 at most, 0.64 rms, from y = -87
-// to 88; infinities and NaN come out as theirs) for less of the time in which no matrix step runs: e^y as 2^n 2^f, y times log2 e in two parts; the quotient's
-// one correction, on a quarter of both, whose reciprocal is a normal number up to the largest. Results and products of 16 bits are the same ones
-// for every 16-bit y. us of 1828 tokens x 28672 x 4096, 3657 x 16384 x 2048, 7691 x 8192 x 1024: the library's two 348, 204, 125; so 336, 194, 114; with
-// the transcendental unit's as they are (its reciprocal and 2^(1.4427 y): 18 units at y = 20, 65 at 80, zero beyond 87.3) 329, 185, 104.
+// to 88; infinities and NaN come out as theirs) for less of the time in which no matrix step runs. 2^t of t = y log2 e, rounded, lacks a factor e^low, low = y - t
+// ln 2: it goes into the quotient's one correction. That is made on a quarter of both, whose reciprocal is a normal number up to the largest. Results and
+// products of 16 bits are the same ones for every 16-bit y. us of 1828 tokens x 28672 x 4096, 3657 x 16384 x 2048, 7691 x 8192 x 1024: the library's two 353, 207, 134;
+// so 345, 197, 120; with the transcendental unit's as they are (its reciprocal and 2^(1.4427 y): 18 units at y = 20, 65 at 80, zero beyond 87.3) 342, 187, 112.
 __device__ __forceinline__ float over_one_plus_exp(float num, float y) {
-    y = __builtin_amdgcn_fmed3f(y, -200.f, 200.f);
-    const float t = y * 0x1.715476p+0f, low = fmaf(y, 0x1.4ae0cp-26f, fmaf(y, 0x1.715476p+0f, -t)), n = __builtin_rintf(t);
-    const float d = fmaf(__builtin_amdgcn_ldexpf(fast_exp2((t - n) + low), static_cast<int>(n)), 0.25f, 0.25f);
-    const float a = num * 0.25f, r = __builtin_amdgcn_rcpf(d), q = a * r;
-    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, a), r, q), d, a);
+    y = fmaxf(y, -200.f);
+    const float t = y * 0x1.715476p+0f, low = fmaf(t, 0x1.05c61p-29f, fmaf(t, -0x1.62e43p-1f, y));      // (ln 2 in two parts)
+    const float e = fast_exp2(t) * 0.25f, d = e + 0.25f, a = num * 0.25f, r = __builtin_amdgcn_rcpf(d), q = a * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, e * low, fmaf(-d, q, a)), r, q), d, a);
 }
 // silu(z), and z sigmoid(1.702 z)
 __device__ __forceinline__ float tile_silu(float z) { return over_one_plus_exp(z, -z); }

@@ -12,7 +12,7 @@
 // Measured (us, bf16, by the second / by the first, gate/up with the unit, then down): 9000 assignments over 8 experts, width and ff 2048: 193 / 165, 89 / 73;
 // 7314: 147 / 113, 69 / 54; 15252, width and ff 1024: 75 / 60, 37 / 31; 1400, 2048: 40 / 33, 26 / 19; 200: 32 / 24, 22 / 16; 64000 over 64, width 2048, ff 1024: 637 /
 // 475, 320 / 255. (Before the exponential and the quotient of gemm_tile.h's units were as exact as the second's: with rows spread evenly over cold weights gate/up then
-// and now 151 / 158 at the first of these sizes, 113 / 117, 60 / 66, 46 / 47, 39 / 40, 474 / 492.) Passes of 3 x 1500, 11 x 333 and 4 x 2000 tokens with experts in two of four layers or in all: 1.05, 1.04, 1.06.
+// and now 151 / 156 at the first of these sizes, 113 / 115, 60 / 64, 46 / 47, 39 / 40, 474 / 483.) Passes of 3 x 1500, 11 x 333 and 4 x 2000 tokens with experts in two of four layers or in all: 1.05, 1.04, 1.06.
 #include "gemm_tile.h"
 #include "tile_product.h"
 

@@ -293,11 +293,11 @@ def _tile_pays(m: int, rows: int, k: int, gated: bool = False) -> bool:
     31.5 (30.5), 2036 (256) 33 (41); 2048 x 8192, 679 (176) 58 (45), 1260 (320) 70 (68), 1559 (400) 71 (73); 4096 x 14336, 360 (192) 107 (84), 741 (384)
     129 (122), 1521 (768) 172 (188). Up to 2560 columns always (277 of 1024 x 1024 7.4, 8.7): the few tiles that take longer there (402 of 1024 x 2048 13.2, 10.4; 300 of 96 x
     2560 15.4, 9.0) are of steps that wait for the host, which a library's call keeps 15 us longer than a launch (lines by device time alone: passes of 280 to 1341 tokens
-    on 1024 and 2048 columns 1.06 to 1.23 times as long, none shorter). So are very long ones of many tokens, which the
-    library takes in blocks of rows at its best rate: 5112 of 4096 x 14336 505 (458); 4010 tokens 353 (367) (not with 2048 rows: 5000 of 2048 x 12288 205
+    on 1024 and 2048 columns 1.06 to 1.23 times as long, none shorter). The library's are also very long sums of many tokens, which
+    it takes in blocks of rows at its best rate: 5112 of 4096 x 14336 505 (458); 4010 tokens 353 (367) (not with 2048 rows: 5000 of 2048 x 12288 205
     (267), 7800 291 (374)). And beyond 8192 tokens what is not
     small, where the library's rate is 5 % to 10 % higher: 12288 of 6144 x 4096 459 (424), 16384 of 8192 x 2048 381 (365), of 1024 x 4096 102 (93), but
-    12288 of 1024 x 4096 77 (102), 10000 of 3072 x 1024 55 (72) — unless the launch does an activation's work (28672 x 4096, 16384 2727 (2733))."""
+    12288 of 1024 x 4096 77 (102), 10000 of 3072 x 1024 55 (72) — unless the launch does an activation's work (28672 x 4096, 16384 2676 (2733))."""
     if m > 8192 and m * rows * k > 6e10 and not gated:
         return False
     if k <= 2560:
